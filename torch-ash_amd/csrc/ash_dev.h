@@ -30,11 +30,11 @@ void set_error(const std::string& msg);
 #define ASH_LAUNCH_CHECK() ASH_HIP(hipGetLastError())
 
 // ------------------------------------------------------- table geometry
-// One bucket is one 128-byte line read by a group of 8 lanes, 16 bytes each:
+// One bucket is one 128-byte line, eight pieces of 16 bytes:
 //   dwords [ 0,20)  ten 64-bit packed key codes
 //   dwords [20,30)  ten int32 indices (slot s -> dword 20+s)
 //   dwords [30,32)  unused
-constexpr int kGroup = 8;                       // lanes per bucket
+constexpr int kGroup = 8;                       // 16-byte pieces per bucket
 constexpr int kBucketDwords = kGroup * 4;       // 32
 constexpr int kBucketQwords = kGroup * 2;       // 16
 constexpr int kSlots = (kGroup * 16) / 12;      // 10

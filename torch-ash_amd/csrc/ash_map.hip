@@ -9,11 +9,11 @@
 // ("exotic" keys) live in a second, lock-based open-addressing region that is
 // only attached once such a key shows up.
 //
-// Probing.  A wavefront takes 64 keys.  Each group of 8 lanes owns 8 of them
-// and probes them one after the other: the 8 lanes read the 8 x 16 bytes of
-// the key's bucket in one coalesced request, compare, and agree through
-// ballots.  All 8 bucket reads of a group are issued before the first compare,
-// so a wavefront keeps 64 lines in flight.  If the bucket neither holds the key
+// Probing.  A wavefront takes 64 keys.  Each quad of lanes owns four of them
+// and probes them one after the other: the four lanes read the 128 bytes of
+// the key's bucket in two coalesced requests, compare, and agree through quad
+// permutations.  All reads of a quad are issued before the first compare, so a
+// wavefront keeps 64 lines in flight.  If the bucket neither holds the key
 // nor an empty slot the key moves on to the next bucket.
 //
 // Index allocation follows the reference's heap protocol
@@ -50,13 +50,6 @@ constexpr int kBlock = 256;
 constexpr int kHeapBlock = 256;
 constexpr uint32_t kSpinLimit = 1u << 22;
 
-__device__ __forceinline__ uint32_t spread8(uint32_t x) {
-    x = (x | (x << 4)) & 0x0F0Fu;
-    x = (x | (x << 2)) & 0x3333u;
-    x = (x | (x << 1)) & 0x5555u;
-    return x;
-}
-
 // -------------------------------------------------- cooperative probe pass
 enum { kProbeFound = 0, kProbeHasEmpty = 1, kProbeFull = 2 };
 
@@ -68,74 +61,69 @@ struct ProbeResult {
 };
 
 // Every lane of the wavefront calls this together.  Lane L owns key L; in
-// round r the 8 lanes of a group read the bucket `b` of the group's r-th key
-// (16 bytes per lane) and the result lands in that key's owner lane.  Keys
-// that are not pending cost no memory traffic.
+// round r the four lanes of a quad read the bucket `b` of the quad's r-th key
+// (two 16-byte pieces per lane: codes 0..7 with the first, codes 8, 9 and the
+// ten indices with the second) and the result lands in that key's owner lane.
+// Keys that are not pending cost no memory traffic.
+// A quad, because what its lanes tell each other -- whose key, which slot,
+// which index -- are quad permutations, modifiers of a vector instruction, where
+// groups of eight have to go through ballots and the LDS pipeline.
 __device__ __forceinline__ void probe_pass(const MapDev& m, uint64_t code,
                                            uint32_t b, bool pend, int lane,
                                            ProbeResult& out) {
-    const int j = lane & (kGroup - 1);
-    const int gbase = lane & ~(kGroup - 1);
-    const bool v0 = (2 * j) < kSlots;
-    const bool v1 = (2 * j + 1) < kSlots;
-
-    uint4 line[kGroup];
-#pragma unroll
-    for (int r = 0; r < kGroup; ++r) {
-        const int src = gbase | r;
-        const uint32_t br = __shfl(b, src);
-        const int pr = __shfl(static_cast<int>(pend), src);
-        line[r] = make_uint4(0u, 0u, 0u, 0u);
-        if (pr) {
-            line[r] = *(reinterpret_cast<const uint4*>(
-                                m.buckets +
-                                static_cast<size_t>(br) * kBucketQwords) +
-                        j);
+    static_assert(kSlots == 10 && kBucketDwords == 32, "two 16-byte pieces per lane");
+    const int j = lane & 3;
+    uint4 lo[4], hi[4];
+    auto fetch = [&](auto round) {
+        constexpr int r = decltype(round)::value;
+        const uint32_t br = quad_bcast<r>(b);
+        lo[r] = make_uint4(0u, 0u, 0u, 0u);
+        hi[r] = make_uint4(0u, 0u, 0u, 0u);
+        if (quad_bcast<r>(pend ? 1u : 0u)) {
+            const uint4* line = reinterpret_cast<const uint4*>(
+                    m.buckets + static_cast<size_t>(br) * kBucketQwords);
+            lo[r] = line[j];
+            hi[r] = line[4 + j];
         }
-    }
-
-#pragma unroll
-    for (int r = 0; r < kGroup; ++r) {
-        const int src = gbase | r;
-        const uint64_t cr = __shfl(code, src);
-        const uint64_t qa =
-                static_cast<uint64_t>(line[r].x) |
-                (static_cast<uint64_t>(line[r].y) << 32);
-        const uint64_t qb =
-                static_cast<uint64_t>(line[r].z) |
-                (static_cast<uint64_t>(line[r].w) << 32);
-        const uint32_t gm0 =
-                static_cast<uint32_t>(__ballot(v0 && qa == cr) >> gbase) & 0xFFu;
-        const uint32_t gm1 =
-                static_cast<uint32_t>(__ballot(v1 && qb == cr) >> gbase) & 0xFFu;
-        const uint32_t ge0 =
-                static_cast<uint32_t>(__ballot(v0 && qa == kEmpty) >> gbase) &
-                0xFFu;
-        const uint32_t ge1 =
-                static_cast<uint32_t>(__ballot(v1 && qb == kEmpty) >> gbase) &
-                0xFFu;
-        int slot = -1;
-        if (gm0) {
-            slot = 2 * __builtin_ctz(gm0);
-        } else if (gm1) {
-            slot = 2 * __builtin_ctz(gm1) + 1;
-        }
-        const uint32_t emask = spread8(ge0) | (spread8(ge1) << 1);
-        const int t = kValDword0 + (slot < 0 ? 0 : slot);
-        const int comp = t & 3;
-        const uint32_t sel = comp == 0   ? line[r].x
-                             : comp == 1 ? line[r].y
-                             : comp == 2 ? line[r].z
-                                         : line[r].w;
-        const int32_t val = __shfl(static_cast<int>(sel), gbase + (t >> 2));
+    };
+    auto compare = [&](auto round) {
+        constexpr int r = decltype(round)::value;
+        const uint64_t want = static_cast<uint64_t>(quad_bcast<r>(static_cast<uint32_t>(code))) |
+                              (static_cast<uint64_t>(quad_bcast<r>(static_cast<uint32_t>(code >> 32))) << 32);
+        const uint64_t q0 = lo[r].x | (static_cast<uint64_t>(lo[r].y) << 32);
+        const uint64_t q1 = lo[r].z | (static_cast<uint64_t>(lo[r].w) << 32);
+        // (codes 8 and 9, in the quad's first lane; indices in the others)
+        const uint64_t q8 = j == 0 ? hi[r].x | (static_cast<uint64_t>(hi[r].y) << 32) : 0ull;
+        const uint64_t q9 = j == 0 ? hi[r].z | (static_cast<uint64_t>(hi[r].w) << 32) : 0ull;
+        uint32_t v = 0;   // bits 0..3: slot + 1 of the match, bits 4..13: empty slots
+        if (j == 0 && q8 == want) v = 9;
+        if (j == 0 && q9 == want) v = 10;
+        if (q0 == want) v = 2 * j + 1;
+        if (q1 == want) v = 2 * j + 2;
+        if (q0 == kEmpty) v |= 16u << (2 * j);
+        if (q1 == kEmpty) v |= 32u << (2 * j);
+        if (q8 == kEmpty) v |= 16u << 8;
+        if (q9 == kEmpty) v |= 16u << 9;
+        v = quad_or(v);
+        const int slot = static_cast<int>(v & 15u) - 1;
+        const int comp = slot & 3;   // index of slot s: dword 20 + s of the bucket
+        const uint32_t word = comp == 0 ? hi[r].x : comp == 1 ? hi[r].y : comp == 2 ? hi[r].z : hi[r].w;
+        const uint32_t val = quad_or(j == ((4 + slot) >> 2) ? word : 0u);
         if (j == r) {
-            out.status = slot >= 0 ? kProbeFound
-                                   : (emask ? kProbeHasEmpty : kProbeFull);
+            out.emask = v >> 4;
+            out.status = slot >= 0 ? kProbeFound : (out.emask ? kProbeHasEmpty : kProbeFull);
             out.slot = slot;
-            out.val = val;
-            out.emask = emask;
+            out.val = static_cast<int32_t>(val);
         }
-    }
+    };
+    fetch(Round<0>());
+    fetch(Round<1>());
+    fetch(Round<2>());
+    fetch(Round<3>());
+    compare(Round<0>());
+    compare(Round<1>());
+    compare(Round<2>());
+    compare(Round<3>());
 }
 
 // ------------------------------------------------ general (exotic) region

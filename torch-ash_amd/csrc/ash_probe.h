@@ -19,6 +19,26 @@ __device__ __forceinline__ int32_t* value_ptr(const MapDev& m, uint32_t b,
            static_cast<size_t>(b) * kBucketDwords + kValDword0 + s;
 }
 
+// -------------------------------------------------- quads of lanes
+// Exchanges among the four lanes 4 q .. 4 q + 3 as modifiers of a vector
+// instruction (DPP quad permutation).  Every lane of the quad takes part.
+template <int R>
+__device__ __forceinline__ uint32_t quad_bcast(uint32_t v) {
+    return static_cast<uint32_t>(
+            __builtin_amdgcn_mov_dpp(static_cast<int>(v), R * 0x55, 0xF, 0xF, true));
+}
+
+__device__ __forceinline__ uint32_t quad_or(uint32_t v) {
+    v |= static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), 0xB1, 0xF, 0xF, true));
+    v |= static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), 0x4E, 0xF, 0xF, true));
+    return v;
+}
+
+template <int R>
+struct Round {
+    static constexpr int value = R;
+};
+
 // ------------------------------------------- general (exotic) region, reads
 template <int DIM>
 __device__ __forceinline__ uint32_t gen_home(const int32_t (&k)[DIM],

@@ -493,6 +493,25 @@ int ash_gather_rows(int n_values, const void* const* src, void* const* dst,
                     const int64_t* row_bytes, const int64_t* src_rows,
                     const int64_t* indices, int64_t n, void* stream);
 
+/* Look-up and gather in one launch: what `HashMap.find(return_values=True)`
+ * (ash/hashmap.py:82-95) and `HashEmbedding.forward` (ash/embedding.py:30-38) are
+ * made of.  As ash_map_find, and dst[v][i] = src[v][index of keys[i]] for up to
+ * four tensors (n_values may be 0); a key that is not stored reads row 0, as
+ * the reference's indexing does, or a row of zeros with zero_misses.  Rows of
+ * tensor v are row_bytes[v] bytes (a multiple of 4, at most 32764), the source
+ * has src_rows[v] rows.  indices and masks may be NULL when nobody wants them. */
+int ash_map_find_rows(ash_map_t* map, const int32_t* keys, int64_t n, int n_values,
+                      const void* const* src, void* const* dst, const int64_t* row_bytes,
+                      const int64_t* src_rows, int zero_misses, int64_t* indices,
+                      uint8_t* masks, void* stream);
+
+/* The gradient of that look-up with respect to a table (autograd of
+ * ash/embedding.py:38): out (out_rows x width, 16-byte aligned) is cleared and
+ * rows[i] (width elements of `dtype`) is added to out[indices[i]] where
+ * masks[i]; the order of the additions is not fixed. */
+int ash_add_rows(const void* rows, const int64_t* indices, const uint8_t* masks, int64_t n,
+                 int64_t width, int dtype, void* out, int64_t out_rows, void* stream);
+
 /* -------------------------------------------------------- trilinear queries */
 
 enum { ASH_INTERP_LINEAR = 0, ASH_INTERP_SMOOTH_STEP = 1 };

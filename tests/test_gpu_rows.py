@@ -1,0 +1,74 @@
+"""The look-up with rows (ash_map_find_rows) and its transpose (ash_add_rows)
+against torch's indexing on the indices that `find` returns: exact for the rows,
+to the rounding of a reordered sum for the gradient."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+def _engine(gpu_ash, dim, stored, seed):
+    g = torch.Generator().manual_seed(seed)
+    keys = torch.unique(torch.randint(-90, 90, (2 * stored, dim), generator=g, dtype=torch.int32), dim=0)
+    keys = keys[torch.randperm(len(keys), generator=g)][:stored]
+    engine = gpu_ash.ASHEngine(dim, stored + 50, DEV)
+    engine.insert_keys(keys.to(DEV))
+    return engine, keys
+
+
+def _queries(keys, n, seed):
+    g = torch.Generator().manual_seed(seed)
+    q = keys[torch.randint(len(keys), (n,), generator=g)].clone()
+    q[torch.rand(n, generator=g) < 0.3, 0] += 1000
+    if n > 2:
+        q[1, 0] = 1 << 29     # does not fit the packed code of dims 3 and 4
+    return q.to(DEV)
+
+
+@pytest.mark.parametrize("dim", [1, 2, 3, 4])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1023, 20_001])
+def test_rows_are_those_of_the_found_indices(gpu_ash, dim, n):
+    engine, keys = _engine(gpu_ash, dim, 100 if dim == 1 else 3000, seed=dim)
+    q = _queries(keys, n, seed=n)
+    indices, masks = engine.find(q)
+    rows = engine.capacity
+    tables = [torch.randn(rows, w, device=DEV) for w in (1, 3, 4, 67)]
+    tables[1] = torch.randint(-9, 9, (rows, 3, 5), device=DEV)           # 120 bytes
+    shifted = torch.randn(rows * 16 + 1, device=DEV)[1:].view(rows, 16)  # not 16-byte aligned
+    backend = gpu_ash.core.backend
+    for group in (tables, [shifted, torch.randn(rows, 8, device=DEV, dtype=torch.float64)]):
+        assert backend.finds_rows_of(group, DEV)
+        got_i, got_m, got = backend.find_rows(engine.backend, q, group)
+        assert torch.equal(got_i, indices) and torch.equal(got_m, masks)
+        for t, r in zip(group, got):
+            assert torch.equal(r, t[indices])
+        none, got_m, got = backend.find_rows(engine.backend, q, group, zero_misses=True, need_indices=False)
+        assert none is None and torch.equal(got_m, masks)
+        for t, r in zip(group, got):
+            assert torch.equal(r, t[indices] * masks.view(-1, *[1] * (t.dim() - 1)).to(t.dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("width,n", [(1, 1000), (3, 65), (16, 4097), (33, 300)])
+def test_gradient_of_embedding_rows(gpu_ash, dtype, width, n):
+    emb = gpu_ash.HashEmbedding(3, 701, width, DEV)
+    emb.embedding = torch.nn.Parameter(torch.randn(701, width, device=DEV, dtype=dtype))
+    g = torch.Generator().manual_seed(width)
+    keys = torch.unique(torch.randint(-30, 30, (650, 3), generator=g, dtype=torch.int32), dim=0)
+    emb.spatial_init_(keys.to(DEV))
+    q = _queries(keys, n, seed=width + n)
+    indices, masks = emb.engine.find(q)
+    z = torch.randn(n, width, device=DEV, dtype=dtype, requires_grad=True)
+    y = emb(q)
+    assert torch.equal(y, emb.embedding[indices] * masks.unsqueeze(1))
+    (got,) = torch.autograd.grad(y, emb.embedding, z, create_graph=True)
+    terms = z.detach().double() * masks.unsqueeze(1)
+    want = torch.zeros(701, width, device=DEV, dtype=torch.float64).index_add_(0, indices, terms)
+    sums = torch.zeros_like(want).index_add_(0, indices, terms.abs())
+    eps = 2.0**-24 if dtype == torch.float32 else 2.0**-53
+    assert bool(((got.double() - want).abs() <= 16 * eps * sums).all())
+    # and the gradient of the gradient: the look-up again
+    u = torch.randn(701, width, device=DEV, dtype=dtype)
+    (back,) = torch.autograd.grad(got, z, u)
+    assert torch.equal(back, u[indices] * masks.unsqueeze(1))

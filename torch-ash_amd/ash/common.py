@@ -199,6 +199,15 @@ _SIGNATURES = {
         [ctypes.c_int, ctypes.POINTER(_PTR), ctypes.POINTER(_PTR), ctypes.POINTER(_I64),
          ctypes.POINTER(_I64), _PTR, _I64, _PTR],
     ),
+    "ash_map_find_rows": (
+        ctypes.c_int,
+        [_PTR, _PTR, _I64, ctypes.c_int, ctypes.POINTER(_PTR), ctypes.POINTER(_PTR),
+         ctypes.POINTER(_I64), ctypes.POINTER(_I64), ctypes.c_int, _PTR, _PTR, _PTR],
+    ),
+    "ash_add_rows": (
+        ctypes.c_int,
+        [_PTR, _PTR, _PTR, _I64, _I64, ctypes.c_int, _PTR, _I64, _PTR],
+    ),
     "ash_isosurface_workspace_ints": (ctypes.c_int64, [_I64, _I64]),
     "ash_isosurface_classify": (
         ctypes.c_int,
@@ -270,6 +279,8 @@ COLLECT_MAX_BLOCKS = 1 << 20
 # Size of a second region that is attached before any key has asked for it
 # (2^16 slots of 20 bytes).
 GENERAL_JUST_IN_CASE_BYTES = 20 << 16
+# Longest row a look-up with rows gathers (the limit of ash_map_find_rows).
+MAX_ROW_BYTES = 32764
 # Which inserts (and erases) take the streaming path of the library (batch split
 # by bucket range, ranges handled in LDS) instead of the per-key kernel:
 # "auto" = when the library says the batch is large enough relative to the
@@ -698,6 +709,51 @@ class _Backend:
                     indices.data_ptr() if indices is not None else None, n, _stream_of(dev)))
         return {name: out[name] for name in tables}
 
+    # -- look-up with rows (ash/hashmap.py:82-95, ash/embedding.py:30-38) -----
+    @staticmethod
+    def finds_rows_of(tables, device) -> bool:
+        """Whether `find_rows` takes these tables (a list of tensors)."""
+        return 0 < len(tables) <= 4 and all(
+            t.device == device and t.is_contiguous() and t.numel() > 0 and t.shape[0] < 2**31
+            and _row_bytes(t) <= MAX_ROW_BYTES and _row_bytes(t) % 4 == 0
+            for t in tables
+        )
+
+    def find_rows(self, hashmap, keys, tables, zero_misses: bool = False,
+                  need_indices: bool = True):
+        """(indices or None, masks, [table[indices] for each table]) in one
+        launch; rows of keys that are not stored are row 0 of the table, or
+        zeros with `zero_misses`."""
+        keys = hashmap._keys(keys)
+        n, dev = keys.shape[0], hashmap.device()
+        indices = torch.empty(n, dtype=torch.int64, device=dev) if need_indices else None
+        masks = torch.empty(n, dtype=torch.bool, device=dev)
+        rows = [torch.empty((n,) + tuple(t.shape[1:]), dtype=t.dtype, device=dev) for t in tables]
+        k = len(tables)
+        with torch.cuda.device(dev):
+            self.check(self.lib.ash_map_find_rows(
+                hashmap._handle, keys.data_ptr(), n, k,
+                (_PTR * k)(*[t.data_ptr() for t in tables]),
+                (_PTR * k)(*[r.data_ptr() for r in rows]),
+                (_I64 * k)(*[_row_bytes(t) for t in tables]),
+                (_I64 * k)(*[t.shape[0] for t in tables]), int(zero_misses),
+                indices.data_ptr() if need_indices else None, masks.data_ptr(), _stream_of(dev)))
+        return indices, masks, rows
+
+    def add_rows(self, rows, indices, masks, out_rows: int) -> torch.Tensor:
+        """(out_rows, width) tensor of zeros with rows[i] added at indices[i]
+        where masks[i]."""
+        _require_hip(rows, "rows")
+        n, width = rows.shape
+        out = torch.empty((out_rows, width), dtype=rows.dtype, device=rows.device)
+        if rows.dtype not in _DTYPE or indices.shape[0] != n or masks.shape[0] != n:
+            raise RuntimeError("add_rows: rows must be float32/float64, one index and mask per row")
+        with torch.cuda.device(rows.device):
+            self.check(self.lib.ash_add_rows(
+                rows.data_ptr(), indices.data_ptr(), masks.data_ptr(), n, width,
+                _DTYPE[rows.dtype], out.data_ptr(), out_rows, _stream_of(rows.device)))
+        return out
+
     # -- trilinear queries (ash/src/pybind.cpp:25-29) ---------------------
     def _query_args(
         self,
@@ -1000,6 +1056,10 @@ def _accumulator(t: torch.Tensor, embeddings: torch.Tensor) -> torch.Tensor:
     ):
         raise RuntimeError("accumulate_into must be a contiguous tensor like the embeddings")
     return t
+
+
+def _row_bytes(t: torch.Tensor) -> int:
+    return t.numel() // t.shape[0] * t.element_size()
 
 
 def _numel(shape) -> int:

@@ -24,6 +24,8 @@
 
 #include "../../include/ash_hip.h"
 
+#include <hip/amd_detail/amd_hip_unsafe_atomics.h>
+
 #include <mutex>
 
 // Scratch of ash_grid_activate_static, the entry point that allocates nothing:
@@ -1468,6 +1470,128 @@ __global__ __launch_bounds__(kBlock) void gather_rows_kernel(
     }
 }
 
+// ----------------------------------------------- look-up with rows, and back
+// Row tables read by a look-up: row `index` of src[v] goes to row i of dst[v].
+// Rows are units[v] pieces of 4 bytes, or of 16 where `wide` has bit v set
+// (row size and both base addresses are multiples of 16).
+struct RowTables {
+    int n;
+    uint32_t wide;
+    const void* src[kMaxFusedValues];
+    void* dst[kMaxFusedValues];
+    uint32_t units[kMaxFusedValues];
+    uint32_t magic[kMaxFusedValues];   // t / units == umulhi(t, magic) for t < 64 * units
+    uint32_t src_rows[kMaxFusedValues];
+};
+
+// Longest row (in pieces) whose 64 * units numbers the multiplication above
+// divides exactly: t * (magic * units - 2^32) < 64 * units * units < 2^32.
+constexpr int64_t kMaxRowUnits = 8191;
+
+// The rows of the 64 keys of a wavefront: `from` is the row lane L's key reads
+// (negative: a row of zeros), `rows` how many of the 64 keys exist.  Lanes
+// walk the output in order, so it is written whole and a row is read by
+// neighbouring lanes; up to four pieces per lane are in flight.
+template <typename Unit>
+__device__ __forceinline__ void copy_found_rows(const Unit* __restrict__ src, Unit* __restrict__ dst,
+                                                uint32_t units, uint32_t magic, uint32_t src_rows,
+                                                int32_t from, int rows) {
+    constexpr int kAhead = 4;
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t total = static_cast<uint32_t>(rows) * units;
+    for (uint32_t t0 = 0; t0 < total; t0 += 64 * kAhead) {
+        Unit w[kAhead];
+#pragma unroll
+        for (int a = 0; a < kAhead; ++a) {
+            const uint32_t t = t0 + a * 64 + lane;
+            const uint32_t row = units == 1 ? t : __umulhi(t, magic);
+            const int32_t at = __shfl(from, static_cast<int>(row & 63u));
+            w[a] = Unit{};
+            if (t < total && static_cast<uint32_t>(at) < src_rows) {
+                w[a] = src[static_cast<size_t>(static_cast<uint32_t>(at)) * units + (t - row * units)];
+            }
+        }
+#pragma unroll
+        for (int a = 0; a < kAhead; ++a) {
+            const uint32_t t = t0 + a * 64 + lane;
+            if (t < total) __builtin_nontemporal_store(w[a], dst + t);
+        }
+    }
+}
+
+// find and the gather of the rows in one launch: the indices never travel
+// through memory unless the caller wants them, and the line of a key's bucket
+// and the lines of its rows are asked for by the same wavefront.  16 M keys
+// with rows of 12 and 4 bytes: see the table of the design notes.
+template <int DIM>
+__global__ __launch_bounds__(kBlock) void find_rows_kernel(
+        MapDev m, const int32_t* __restrict__ keys, int64_t n, RowTables tabs, int miss_row,
+        int64_t* __restrict__ idx_out, uint8_t* __restrict__ mask_out) {
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    const bool active = i < n;
+    int32_t k[DIM];
+    load_key<DIM>(keys, i, active, k);
+    int32_t res = 0;
+    const bool found = find_key<DIM>(m, k, active, res);
+    if (active) {
+        if (idx_out != nullptr) idx_out[i] = found ? static_cast<int64_t>(res) : 0;
+        if (mask_out != nullptr) mask_out[i] = found ? 1 : 0;
+    }
+    const int64_t first = i - (threadIdx.x & 63);
+    if (first >= n) return;   // whole wavefronts leave together
+    const int rows = n - first < 64 ? static_cast<int>(n - first) : 64;
+    const int32_t from = found ? res : miss_row;
+    for (int v = 0; v < tabs.n; ++v) {
+        const uint32_t units = tabs.units[v];
+        const size_t at = static_cast<size_t>(first) * units;
+        if ((tabs.wide >> v) & 1u) {
+            copy_found_rows<u4>(static_cast<const u4*>(tabs.src[v]), static_cast<u4*>(tabs.dst[v]) + at,
+                                units, tabs.magic[v], tabs.src_rows[v], from, rows);
+        } else {
+            copy_found_rows<uint32_t>(static_cast<const uint32_t*>(tabs.src[v]),
+                                      static_cast<uint32_t*>(tabs.dst[v]) + at, units,
+                                      tabs.magic[v], tabs.src_rows[v], from, rows);
+        }
+    }
+}
+
+// 16 bytes per thread, the words of a shorter tail one by one.
+__global__ __launch_bounds__(kBlock) void clear_rows_kernel(uint32_t* __restrict__ p, int64_t words) {
+    const int64_t t = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) * 4;
+    const int64_t stride = static_cast<int64_t>(gridDim.x) * kBlock * 4;
+    for (int64_t at = t; at < words; at += stride) {
+        if (at + 4 <= words) {
+            *reinterpret_cast<uint4*>(p + at) = make_uint4(0u, 0u, 0u, 0u);
+        } else {
+            for (int64_t w = at; w < words; ++w) p[w] = 0u;
+        }
+    }
+}
+
+// out[indices[i]] += rows[i] where masks[i]: the transpose of the look-up.  One
+// element per thread, so that the elements of a row leave in one atomic request
+// per 64-byte line whatever the row's width; the device executes such requests
+// at 15-20 G/s, which is what bounds this kernel (200 003 rows of 16 floats:
+// 13 us, where sorting the indices and adding the rows up in order took 8.8 ms).
+template <typename T>
+__global__ __launch_bounds__(kBlock) void add_rows_kernel(
+        const T* __restrict__ rows, const int64_t* __restrict__ indices,
+        const uint8_t* __restrict__ masks, int64_t n, int64_t width, T* __restrict__ out,
+        int64_t out_rows) {
+    const int64_t total = n * width;
+    const bool narrow = total <= 0xFFFFFFFFll;
+    const int64_t stride = static_cast<int64_t>(gridDim.x) * kBlock;
+    for (int64_t t = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; t < total; t += stride) {
+        const int64_t row = narrow ? static_cast<int64_t>(static_cast<uint32_t>(t) /
+                                                          static_cast<uint32_t>(width))
+                                   : t / width;
+        const int64_t to = indices[row];
+        if (masks[row] == 0 || to < 0 || to >= out_rows) continue;
+        unsafeAtomicAdd(out + to * width + (t - row * width), rows[t]);
+    }
+}
+
 // The rows whose flag an activation has set, in ascending order, with their
 // block coordinates; the flags are cleared on the way and the count goes to
 // the table's counters, where the read-back that follows an activation finds
@@ -2027,6 +2151,91 @@ int ash_map_find(ash_map_t* map, const int32_t* keys, int64_t n,
         default:
             find_kernel<4><<<g, kBlock, 0, s>>>(map->d, keys, n, indices, masks);
             break;
+    }
+    ASH_LAUNCH_CHECK();
+    return 0;
+}
+
+int ash_map_find_rows(ash_map_t* map, const int32_t* keys, int64_t n, int n_values,
+                      const void* const* src, void* const* dst, const int64_t* row_bytes,
+                      const int64_t* src_rows, int zero_misses, int64_t* indices,
+                      uint8_t* masks, void* stream) {
+    if (check_batch(map, keys, n)) return 1;
+    if (n_values < 0 || n_values > kMaxFusedValues) {
+        ASH_FAIL("find_rows takes up to " + std::to_string(kMaxFusedValues) + " tensors per call");
+    }
+    if (n_values > 0 && (src == nullptr || dst == nullptr || row_bytes == nullptr || src_rows == nullptr)) {
+        ASH_FAIL("null value tables");
+    }
+    RowTables tabs = {};
+    tabs.n = n_values;
+    for (int v = 0; v < n_values; ++v) {
+        if (n > 0 && (src[v] == nullptr || dst[v] == nullptr)) ASH_FAIL("null value tensor");
+        if (row_bytes[v] <= 0 || row_bytes[v] % 4 != 0) {
+            ASH_FAIL("find_rows: rows must be a positive multiple of 4 bytes");
+        }
+        if (src_rows[v] < 0 || src_rows[v] > 0x7FFFFFFFll) ASH_FAIL("find_rows: bad source row count");
+        const bool wide = (reinterpret_cast<uintptr_t>(src[v]) | reinterpret_cast<uintptr_t>(dst[v]) |
+                           static_cast<uintptr_t>(row_bytes[v])) % 16 == 0;
+        const int64_t units = row_bytes[v] / (wide ? 16 : 4);
+        if (units > kMaxRowUnits) ASH_FAIL("find_rows: rows of at most 32764 bytes");
+        if (wide) tabs.wide |= 1u << v;
+        tabs.src[v] = src[v];
+        tabs.dst[v] = dst[v];
+        tabs.units[v] = static_cast<uint32_t>(units);
+        tabs.magic[v] = static_cast<uint32_t>((0x100000000ull + units - 1) / units);
+        tabs.src_rows[v] = static_cast<uint32_t>(src_rows[v]);
+    }
+    if (n == 0) return 0;
+    DeviceGuard guard;
+    ASH_HIP(guard.enter(map->device));
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (settle_table(map, s)) return 1;
+    const unsigned g = grid_for(n);
+    const int miss = zero_misses ? -1 : 0;
+    switch (map->key_dim) {
+        case 1:
+            find_rows_kernel<1><<<g, kBlock, 0, s>>>(map->d, keys, n, tabs, miss, indices, masks);
+            break;
+        case 2:
+            find_rows_kernel<2><<<g, kBlock, 0, s>>>(map->d, keys, n, tabs, miss, indices, masks);
+            break;
+        case 3:
+            find_rows_kernel<3><<<g, kBlock, 0, s>>>(map->d, keys, n, tabs, miss, indices, masks);
+            break;
+        default:
+            find_rows_kernel<4><<<g, kBlock, 0, s>>>(map->d, keys, n, tabs, miss, indices, masks);
+            break;
+    }
+    ASH_LAUNCH_CHECK();
+    return 0;
+}
+
+int ash_add_rows(const void* rows, const int64_t* indices, const uint8_t* masks, int64_t n,
+                 int64_t width, int dtype, void* out, int64_t out_rows, void* stream) {
+    if (n < 0 || width < 1 || out_rows < 0) ASH_FAIL("add_rows: bad sizes");
+    if (dtype != ASH_F32 && dtype != ASH_F64) ASH_FAIL("add_rows: dtype must be float32 or float64");
+    if (out == nullptr && out_rows > 0) ASH_FAIL("null output pointer");
+    if (n > 0 && (rows == nullptr || indices == nullptr || masks == nullptr)) {
+        ASH_FAIL("null pointer in add_rows");
+    }
+    if (out_rows == 0) return 0;
+    if (reinterpret_cast<uintptr_t>(out) % 16 != 0) ASH_FAIL("add_rows: the output must be 16-byte aligned");
+    PointerGuard guard;
+    ASH_HIP(guard.enter_for(out));
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const int64_t bytes = out_rows * width * (dtype == ASH_F32 ? 4 : 8);
+    clear_rows_kernel<<<capped_grid((bytes + 15) / 16), kBlock, 0, s>>>(static_cast<uint32_t*>(out),
+                                                                       bytes / 4);
+    ASH_LAUNCH_CHECK();
+    if (n == 0) return 0;
+    const unsigned g = capped_grid(n * width);
+    if (dtype == ASH_F32) {
+        add_rows_kernel<float><<<g, kBlock, 0, s>>>(static_cast<const float*>(rows), indices, masks, n,
+                                                    width, static_cast<float*>(out), out_rows);
+    } else {
+        add_rows_kernel<double><<<g, kBlock, 0, s>>>(static_cast<const double*>(rows), indices, masks, n,
+                                                     width, static_cast<double*>(out), out_rows);
     }
     ASH_LAUNCH_CHECK();
     return 0;

@@ -971,6 +971,13 @@ class _Backend:
             )
         return grad_embeddings, grad_offsets
 
+    def query_backward_forward_onto(self, grad_embeddings, z, *operands, need_offsets: bool = True):
+        """query_backward_forward whose embedding gradient is added to
+        `grad_embeddings`, a tensor that no one else holds; returns
+        grad_offsets."""
+        return _Backend.query_backward_forward(self, z, *operands, need_offsets=need_offsets,
+                                               accumulate_into=grad_embeddings)[1]
+
     def query_backward_backward(
         self,
         grad_grad_embeddings,

@@ -3,6 +3,7 @@ backward.  Two chained Functions with the same operands and return
 conventions as the reference (ash/grid_query.py:10-283); each one is a single
 call into the HIP library.
 """
+import sys
 import weakref
 from typing import Literal
 
@@ -16,10 +17,12 @@ _N_TABLE_ARGS = 8  # grid_indices .. interpolation: operands without gradients
 
 # One backward pass can reach the same embeddings through several nodes: a
 # training step with a value loss and a gradient-norm loss runs both the first-
-# and the second-order backward, and each zero-fills a dense gradient of the
-# whole parameter and leaves the sum of the two to autograd (two fills and an
-# add over the parameter: about a third of such a step), as in the reference.
-# `dense_grad` below is the way around that.
+# and the second-order backward.  In the reference each zero-fills a dense
+# gradient of the whole parameter and leaves the sum of the two to autograd (two
+# fills and an add over the parameter: about a third of such a step).  The
+# module's forward hands the second one to the first inside the graph
+# (`grid._FusedGridForward`); `dense_grad` below also takes in what other nodes
+# and an existing `.grad` contribute.
 #
 # which way the embedding gradient of the latest backward node went: "own"
 # (a dense tensor of its own, handed to autograd), "contract" (added to the
@@ -121,19 +124,70 @@ def _record_path(path: str) -> None:
     LAST_GRADIENT_PATH = path
 
 
-def _grad_requested(ctx, index: int) -> bool:
+def _grad_requested(ctx, index: int, through: bool = False) -> bool:
     """Whether the running backward pass will consume the gradient of input
     `index`.  `ctx.needs_input_grad` only says that the input requires grad;
     in `autograd.grad(y, x)` the engine additionally knows which graph nodes it
     is going to execute, and the node behind an input it will not execute (the
-    dense embeddings parameter, typically) needs no gradient from us."""
+    dense embeddings parameter, typically) needs no gradient from us.
+    `through`: the input is the forward node's copy of the embeddings, and the
+    node asked about is the one behind that node's own embeddings."""
     if not ctx.needs_input_grad[index]:
         return False
     try:
         node = ctx.next_functions[index][0]
+        if through:
+            node = node.next_functions[0][0]
         return node is not None and torch._C._will_engine_execute_node(node)
     except Exception:  # outside an engine pass, or an older torch: be conservative
         return True
+
+
+def _holders(t: torch.Tensor):
+    """Who holds `t`: references to the Python object, to the tensor, to its
+    storage."""
+    return (sys.getrefcount(t), t._use_count(),
+            torch._C._storage_Use_Count(t.untyped_storage()._cdata))
+
+
+class _HoldersProbe(torch.autograd.Function):
+    """A node of the shape of `grid._FusedGridForward` that notes what
+    `_holders` says in its backward of a gradient that nobody else holds."""
+
+    seen = None
+
+    @staticmethod
+    def forward(ctx, t):
+        ctx.set_materialize_grads(False)
+        return t.clone(), t.new_zeros(1), t.detach()
+
+    @staticmethod
+    def backward(ctx, z, _unused, carried):
+        return _HoldersProbe.note(ctx, z, carried)
+
+    @staticmethod
+    def note(ctx, z, carried):
+        _HoldersProbe.seen = _holders(carried)
+        return carried
+
+
+_HOLDERS_ALONE = None
+
+
+def _learn_holders() -> None:
+    """What `_holders` says in a backward node, one call below its `backward`,
+    of a gradient that only the engine's call holds: learnt once from a node
+    that is made for it.  False where this torch cannot tell; gradients are then
+    never added in place."""
+    global _HOLDERS_ALONE
+    _HOLDERS_ALONE = False
+    try:
+        with torch.enable_grad():
+            y, _, again = _HoldersProbe.apply(torch.zeros(1, requires_grad=True))
+            (y.sum() + (2 * again).sum()).backward()
+        _HOLDERS_ALONE = _HoldersProbe.seen or False
+    except Exception:
+        pass
 
 
 class SparseDenseGridQuery(torch.autograd.Function):
@@ -181,15 +235,20 @@ class SparseDenseGridQuery(torch.autograd.Function):
         return first_order_backward(ctx, z, ctx.saved_tensors) + (None,) * _N_TABLE_ARGS
 
 
-def first_order_backward(ctx, z, operands, embeddings_input: int = 0, offsets_input: int = 1):
+def first_order_backward(ctx, z, operands, embeddings_input: int = 0, offsets_input: int = 1,
+                         again=None, carried=None):
     """(grad_embeddings, grad_offsets) of a forward node whose inputs number
     `embeddings_input` / `offsets_input` are the embeddings and (what the
     offsets depend on with unit Jacobian:) the offsets or positions; `operands`
-    = (embeddings, offsets, grid_indices, cell_indices, masks, three tables)."""
+    = (embeddings, offsets, grid_indices, cell_indices, masks, three tables).
+    `again`: the node's own copy of the embeddings, which a recorded backward is
+    to depend on instead; `carried`: the gradient that has arrived for it."""
     need_embeddings = _grad_requested(ctx, embeddings_input)
     need_offsets = _grad_requested(ctx, offsets_input)
     if not (need_embeddings or need_offsets):
         return None, None
+    if not need_embeddings:
+        carried = None
     # The reference always produces both gradients (ash/grid_query.py:104-116);
     # the dense embedding gradient (zero fill + atomics over the whole
     # parameter) is skipped when nobody asked for it, e.g. in
@@ -207,7 +266,24 @@ def first_order_backward(ctx, z, operands, embeddings_input: int = 0, offsets_in
             need_offsets=need_offsets,
             accumulate_into=target,
         )
-        return None, grad_offsets
+        return carried, grad_offsets
+    if (
+        carried is not None
+        and not torch.is_grad_enabled()
+        and _HOLDERS_ALONE
+        and _holders(carried) == _HOLDERS_ALONE
+        and carried.is_contiguous()
+        and hasattr(backend, "query_backward_forward_onto")
+    ):
+        # the tensor is this call's alone: the node's own contribution goes on top
+        grad_offsets = backend.query_backward_forward_onto(
+            carried, z.contiguous(), *operands, ctx.grid_dim, ctx.interpolation,
+            need_offsets=need_offsets)
+        return carried, grad_offsets
+    owner = None
+    if again is not None and torch.is_grad_enabled():
+        owner = weakref.ref(operands[0])
+        operands = (again, *operands[1:])
     grad_embeddings, grad_offsets = SparseDenseGridQueryBackward.apply(
         z.contiguous(),
         *operands,
@@ -215,7 +291,10 @@ def first_order_backward(ctx, z, operands, embeddings_input: int = 0, offsets_in
         ctx.interpolation,
         need_embeddings,
         need_offsets,
+        owner,
     )
+    if carried is not None:
+        grad_embeddings = grad_embeddings + carried
     return grad_embeddings, grad_offsets
 
 
@@ -244,10 +323,12 @@ class SparseDenseGridQueryBackward(torch.autograd.Function):
         interpolation,
         need_grad_embeddings: bool = True,
         need_grad_offsets: bool = True,
+        owner=None,
     ):
         """With both `need_*` flags at their default this is the reference's
         signature and result; an output that is not needed is returned as None
-        and its work is skipped."""
+        and its work is skipped.  `owner`: weak reference to the embeddings that
+        the operand is the forward node's copy of."""
         operands = (
             z,
             embeddings,
@@ -262,6 +343,7 @@ class SparseDenseGridQueryBackward(torch.autograd.Function):
         ctx.save_for_backward(*operands)
         ctx.grid_dim = grid_dim
         ctx.interpolation = interpolation
+        ctx.owner = owner
         if need_grad_embeddings and need_grad_offsets:
             return backend.query_backward_forward(*operands, grid_dim, interpolation)
         return backend.query_backward_forward(
@@ -283,11 +365,13 @@ class SparseDenseGridQueryBackward(torch.autograd.Function):
         ash/src/grid.cu:417-426) the incoming `grad_grad_embeddings` is not used
         and no gradient flows to `offsets` at second order.
         """
-        need_z, need_embeddings = _grad_requested(ctx, 0), _grad_requested(ctx, 1)
-        n_rest = _N_TABLE_ARGS + 3  # offsets, tables, grid_dim, interpolation, 2 flags
+        owned = ctx.owner is not None
+        need_z, need_embeddings = _grad_requested(ctx, 0), _grad_requested(ctx, 1, through=owned)
+        n_rest = _N_TABLE_ARGS + 4  # offsets, tables, grid_dim, interpolation, 2 flags, owner
         if grad_grad_offsets is None or not (need_z or need_embeddings):
             return (None, None) + (None,) * n_rest
-        target = _dense_target(ctx.saved_tensors[1]) if need_embeddings else None
+        embeddings = ctx.owner() if owned else ctx.saved_tensors[1]
+        target = _dense_target(embeddings) if need_embeddings and embeddings is not None else None
         _record_path("contract" if target is not None else "own" if need_embeddings else "skipped")
         if target is not None:
             grad_z, _, _ = backend.query_backward_backward(

@@ -4,12 +4,15 @@ The reference binds its native code with pybind11 (`import __ash`,
 ash/common.py:4-15 and ash/src/pybind.cpp:8-38).  Here the native side is a
 plain C-ABI shared library (include/ash_hip.h) loaded with ctypes; this module
 rebuilds the exact surface the rest of the package expects from the extension
-module: a `HashMap` class and the three `query_*` functions.
+module: a `HashMap` class and the three `query_*` functions.  The calls that
+programs make often go through `_ash_host` (csrc/ash_host.cpp), which checks
+operands, allocates outputs and calls the same C ABI from C++.
 
 There is no CPU or PyTorch fallback: if the library is missing, or a tensor is
 not on a HIP device, the calls raise.
 """
 import ctypes
+import importlib.util
 import itertools
 import os
 import threading
@@ -19,6 +22,7 @@ from typing import Dict, Optional, Tuple
 import torch
 
 _LIB_NAME = "libash_hip.so"
+_HOST_NAME = "_ash_host.so"
 _LIB_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib")
 
 _I64 = ctypes.c_int64
@@ -259,8 +263,6 @@ _SIGNATURES = {
 
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 
-_INTERPOLATION = {"linear": 0, "smooth_step": 1}
-
 # Stamps of the tables' contents: a table takes a new one whenever its keys may
 # have changed, and no two tables ever share one (a table made by `resize` may
 # sit at the address of the one it replaces), so that what callers derive from
@@ -279,8 +281,6 @@ COLLECT_MAX_BLOCKS = 1 << 20
 # Size of a second region that is attached before any key has asked for it
 # (2^16 slots of 20 bytes).
 GENERAL_JUST_IN_CASE_BYTES = 20 << 16
-# Longest row a look-up with rows gathers (the limit of ash_map_find_rows).
-MAX_ROW_BYTES = 32764
 # Which inserts (and erases) take the streaming path of the library (batch split
 # by bucket range, ranges handled in LDS) instead of the per-key kernel:
 # "auto" = when the library says the batch is large enough relative to the
@@ -306,6 +306,21 @@ def load_library(path: Optional[str] = None) -> ctypes.CDLL:
     return lib
 
 
+def load_host(lib: ctypes.CDLL):
+    """The native host module, calling into `lib`."""
+    path = os.path.join(_LIB_DIR, _HOST_NAME)
+    if not os.path.exists(path):
+        raise OSError(f"{path} does not exist")
+    spec = importlib.util.spec_from_file_location("_ash_host", path)
+    host = importlib.util.module_from_spec(spec)
+    try:
+        spec.loader.exec_module(host)
+    except ImportError as exc:
+        raise OSError(f"{_HOST_NAME}: {exc}") from exc
+    host.bind(lib._handle)
+    return host
+
+
 def _stream_of(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
@@ -320,6 +335,7 @@ class _Backend:
 
     def __init__(self, lib: ctypes.CDLL):
         self.lib = lib
+        self.host = load_host(lib)
         backend = self
 
         class HashMap(_HashMap):
@@ -675,139 +691,42 @@ class _Backend:
         the kernel does not take (rows that are not a multiple of 4 bytes,
         non-contiguous storage) are indexed by torch."""
         out: Dict[str, torch.Tensor] = {}
-        batch = []
-        if indices is not None:
-            indices = indices.reshape(-1)
-        n = indices.shape[0] if indices is not None else int(first)
+        names, batch = [], []
+        n = indices.numel() if indices is not None else int(first)
         for name, table in tables.items():
-            row_bytes = (table.numel() // max(table.shape[0], 1)) * table.element_size()
-            fits = (table.is_cuda and table.is_contiguous() and table.shape[0] > 0
-                    and row_bytes % 4 == 0 and row_bytes > 0 and not table.requires_grad
+            fits = (table.is_cuda and table.is_contiguous() and table.numel() > 0
+                    and table.numel() // table.shape[0] * table.element_size() % 4 == 0
+                    and not table.requires_grad
                     and (indices is None
                          or (indices.device == table.device and indices.dtype == torch.int64)))
-            if not fits:
-                out[name] = table[indices] if indices is not None else table[:n].clone()
-                continue
-            out[name] = torch.empty((n,) + tuple(table.shape[1:]), dtype=table.dtype,
-                                    device=table.device)
-            batch.append((table, out[name], row_bytes))
-        if indices is not None:
-            indices = indices.contiguous()
-        for start in range(0, len(batch), 4):
-            part = batch[start:start + 4]
-            if n == 0:
-                break
-            k = len(part)
-            c_src = (_PTR * k)(*[t.data_ptr() for t, _, _ in part])
-            c_dst = (_PTR * k)(*[d.data_ptr() for _, d, _ in part])
-            c_rows = (_I64 * k)(*[rb for _, _, rb in part])
-            c_count = (_I64 * k)(*[t.shape[0] for t, _, _ in part])
-            dev = part[0][0].device
-            with torch.cuda.device(dev):
-                self.check(self.lib.ash_gather_rows(
-                    k, c_src, c_dst, c_rows, c_count,
-                    indices.data_ptr() if indices is not None else None, n, _stream_of(dev)))
+            if fits:
+                names.append(name)
+                batch.append(table)
+            else:
+                out[name] = table[indices.reshape(-1)] if indices is not None else table[:n].clone()
+        if batch:
+            out.update(zip(names, self.host.gather_rows(batch, indices, n)))
         return {name: out[name] for name in tables}
 
     # -- look-up with rows (ash/hashmap.py:82-95, ash/embedding.py:30-38) -----
-    @staticmethod
-    def finds_rows_of(tables, device) -> bool:
+    def finds_rows_of(self, tables, device) -> bool:
         """Whether `find_rows` takes these tables (a list of tensors)."""
-        return 0 < len(tables) <= 4 and all(
-            t.device == device and t.is_contiguous() and t.numel() > 0 and t.shape[0] < 2**31
-            and _row_bytes(t) <= MAX_ROW_BYTES and _row_bytes(t) % 4 == 0
-            for t in tables
-        )
+        return self.host.finds_rows_of(tables, device.index)
 
     def find_rows(self, hashmap, keys, tables, zero_misses: bool = False,
                   need_indices: bool = True):
         """(indices or None, masks, [table[indices] for each table]) in one
         launch; rows of keys that are not stored are row 0 of the table, or
         zeros with `zero_misses`."""
-        keys = hashmap._keys(keys)
-        n, dev = keys.shape[0], hashmap.device()
-        indices = torch.empty(n, dtype=torch.int64, device=dev) if need_indices else None
-        masks = torch.empty(n, dtype=torch.bool, device=dev)
-        rows = [torch.empty((n,) + tuple(t.shape[1:]), dtype=t.dtype, device=dev) for t in tables]
-        k = len(tables)
-        with torch.cuda.device(dev):
-            self.check(self.lib.ash_map_find_rows(
-                hashmap._handle, keys.data_ptr(), n, k,
-                (_PTR * k)(*[t.data_ptr() for t in tables]),
-                (_PTR * k)(*[r.data_ptr() for r in rows]),
-                (_I64 * k)(*[_row_bytes(t) for t in tables]),
-                (_I64 * k)(*[t.shape[0] for t in tables]), int(zero_misses),
-                indices.data_ptr() if need_indices else None, masks.data_ptr(), _stream_of(dev)))
-        return indices, masks, rows
+        return self.host.find_rows(hashmap._address, hashmap.key_dim, hashmap._index, keys, tables,
+                                   zero_misses, need_indices)
 
-    def add_rows(self, rows, indices, masks, out_rows: int) -> torch.Tensor:
-        """(out_rows, width) tensor of zeros with rows[i] added at indices[i]
-        where masks[i]."""
-        _require_hip(rows, "rows")
-        n, width = rows.shape
-        out = torch.empty((out_rows, width), dtype=rows.dtype, device=rows.device)
-        if rows.dtype not in _DTYPE or indices.shape[0] != n or masks.shape[0] != n:
-            raise RuntimeError("add_rows: rows must be float32/float64, one index and mask per row")
-        with torch.cuda.device(rows.device):
-            self.check(self.lib.ash_add_rows(
-                rows.data_ptr(), indices.data_ptr(), masks.data_ptr(), n, width,
-                _DTYPE[rows.dtype], out.data_ptr(), out_rows, _stream_of(rows.device)))
-        return out
+    def embedding_rows(self, hashmap, keys, embedding) -> torch.Tensor:
+        """Rows of `embedding` under `keys`, zeros for keys that are not stored;
+        differentiable, to any order, with respect to the embedding."""
+        return self.host.embedding_rows(embedding, hashmap._address, hashmap.key_dim, hashmap._index, keys)
 
     # -- trilinear queries (ash/src/pybind.cpp:25-29) ---------------------
-    def _query_args(
-        self,
-        embeddings,
-        offsets,
-        grid_indices,
-        cell_indices,
-        masks,
-        lut_grid_nb2grid_idx,
-        lut_cell_nb2cell_idx,
-        lut_cell_nb2grid_nb,
-        interpolation,
-    ):
-        if interpolation not in _INTERPOLATION:
-            raise RuntimeError(f"Unknown interpolation functor: {interpolation}")
-        if embeddings.dtype not in _DTYPE:
-            raise RuntimeError(f"embeddings must be float32 or float64, got {embeddings.dtype}")
-        if embeddings.dim() != 3:
-            raise RuntimeError("embeddings must be (num_embeddings, cells_per_grid, dim)")
-        _require_hip(embeddings, "embeddings")
-        dev = embeddings.device
-        n = grid_indices.shape[0]
-
-        def prep(t, dtype, shape, name):
-            if t.device != dev:
-                raise RuntimeError(f"{name} is on {t.device}, embeddings on {dev}")
-            if t.dtype != dtype:
-                raise RuntimeError(f"{name} must be {dtype}, got {t.dtype}")
-            if tuple(t.shape) != shape and t.numel() != _numel(shape):
-                raise RuntimeError(f"{name} has shape {tuple(t.shape)}, expected {shape}")
-            return t.contiguous()
-
-        b, m, e = embeddings.shape
-        held = [
-            prep(embeddings, embeddings.dtype, (b, m, e), "embeddings"),
-            prep(offsets, torch.float32, (n, 3), "offsets"),
-            prep(grid_indices, torch.int64, (n,), "grid_indices"),
-            prep(cell_indices, torch.int64, (n,), "cell_indices"),
-            prep(masks, torch.bool, (n,), "masks"),
-            prep(lut_grid_nb2grid_idx, torch.int64, (b, 8), "lut_grid_nb2grid_idx"),
-            prep(lut_cell_nb2cell_idx, torch.int64, (m, 8), "lut_cell_nb2cell_idx"),
-            prep(lut_cell_nb2grid_nb, torch.int64, (m, 8), "lut_cell_nb2grid_nb"),
-        ]
-        args = _QueryArgs(
-            *[t.data_ptr() for t in held],
-            n,
-            b,
-            m,
-            e,
-            _INTERPOLATION[interpolation],
-            _DTYPE[embeddings.dtype],
-        )
-        return args, held, dev
-
     def query_forward(
         self,
         embeddings,
@@ -821,25 +740,9 @@ class _Backend:
         grid_dim,
         interpolation,
     ) -> torch.Tensor:
-        args, held, dev = self._query_args(
-            embeddings,
-            offsets,
-            grid_indices,
-            cell_indices,
-            masks,
-            lut_grid_nb2grid_idx,
-            lut_cell_nb2cell_idx,
-            lut_cell_nb2grid_nb,
-            interpolation,
-        )
-        out = torch.empty(
-            (args.num_queries, args.embedding_dim), dtype=embeddings.dtype, device=dev
-        )
-        with torch.cuda.device(dev):
-            self.check(
-                self.lib.ash_query_forward(ctypes.byref(args), out.data_ptr(), _stream_of(dev))
-            )
-        return out
+        return self.host.query_forward(
+            [embeddings, offsets, grid_indices, cell_indices, masks, lut_grid_nb2grid_idx,
+             lut_cell_nb2cell_idx, lut_cell_nb2grid_nb], interpolation)
 
     def grid_forward(
         self,
@@ -861,57 +764,10 @@ class _Backend:
         grid_indices, cell_indices, offsets).  The last three are what a
         backward pass needs; with need_operands False they are not produced
         (None)."""
-        if interpolation not in _INTERPOLATION:
-            raise RuntimeError(f"Unknown interpolation functor: {interpolation}")
-        if embeddings.dtype not in _DTYPE:
-            raise RuntimeError(f"embeddings must be float32 or float64, got {embeddings.dtype}")
-        if embeddings.dim() != 3 or not embeddings.is_contiguous():
-            raise RuntimeError("embeddings must be contiguous (num_embeddings, cells_per_grid, dim)")
-        _require_hip(embeddings, "embeddings")
-        dev = embeddings.device
-        if hashmap.device() != dev:
-            raise RuntimeError(f"the map is on {hashmap.device()}, embeddings on {dev}")
-        if x.dim() != 2 or x.shape[1] != 3 or x.dtype != torch.float32 or x.device != dev:
-            raise RuntimeError("positions must be float32 (N, 3) on the device of the embeddings")
-        x = x.contiguous()
-        if origin is not None:
-            if origin.device != dev or origin.dtype != torch.float32 or origin.numel() != 3:
-                raise RuntimeError("origin must be three float32 on the device of the embeddings")
-            origin = origin.contiguous()
-        b, m, e = embeddings.shape
-        n = x.shape[0]
-
-        def table(t, shape, name):
-            if t.device != dev or t.dtype != torch.int64 or tuple(t.shape) != shape:
-                raise RuntimeError(f"{name} must be int64 {shape} on {dev}")
-            return t.contiguous()
-
-        held = [table(lut_grid_nb2grid_idx, (b, 8), "lut_grid_nb2grid_idx"),
-                table(lut_cell_nb2cell_idx, (m, 8), "lut_cell_nb2cell_idx"),
-                table(lut_cell_nb2grid_nb, (m, 8), "lut_cell_nb2grid_nb")]
-        args = _QueryArgs(embeddings.data_ptr(), None, None, None, None,
-                          *[t.data_ptr() for t in held], n, b, m, e,
-                          _INTERPOLATION[interpolation], _DTYPE[embeddings.dtype])
-        out = torch.empty((n, e), dtype=embeddings.dtype, device=dev)
-        masks = torch.empty(n, dtype=torch.bool, device=dev)
-        grid_indices = cell_indices = offsets = None
-        if need_operands:
-            grid_indices = torch.empty(n, dtype=torch.int64, device=dev)
-            cell_indices = torch.empty(n, dtype=torch.int64, device=dev)
-            offsets = torch.empty((n, 3), dtype=torch.float32, device=dev)
-        with torch.cuda.device(dev):
-            self.check(
-                self.lib.ash_grid_forward(
-                    hashmap._handle, x.data_ptr(),
-                    origin.data_ptr() if origin is not None else None, float(cell_size),
-                    int(grid_dim), ctypes.byref(args),
-                    out.data_ptr(), masks.data_ptr(),
-                    grid_indices.data_ptr() if need_operands else None,
-                    cell_indices.data_ptr() if need_operands else None,
-                    offsets.data_ptr() if need_operands else None, _stream_of(dev),
-                )
-            )
-        return out, masks, grid_indices, cell_indices, offsets
+        return self.host.grid_forward(
+            hashmap._address, hashmap._index, x, embeddings, lut_grid_nb2grid_idx,
+            lut_cell_nb2cell_idx, lut_cell_nb2grid_nb, grid_dim, interpolation, need_operands,
+            origin, cell_size)
 
     def query_backward_forward(
         self,
@@ -935,41 +791,10 @@ class _Backend:
         skipped.  With `accumulate_into` (a gradient of the embeddings' shape
         that already holds other contributions) the embedding gradient is added
         to that tensor, which is also what is returned."""
-        args, held, dev = self._query_args(
-            embeddings,
-            offsets,
-            grid_indices,
-            cell_indices,
-            masks,
-            lut_grid_nb2grid_idx,
-            lut_cell_nb2cell_idx,
-            lut_cell_nb2grid_nb,
-            interpolation,
-        )
-        z = _as_like(z, embeddings, (args.num_queries, args.embedding_dim), "z")
-        entry = self.lib.ash_query_backward_forward
-        if accumulate_into is not None:
-            need_embeddings = True
-            grad_embeddings = _accumulator(accumulate_into, held[0])
-            entry = self.lib.ash_query_backward_forward_accumulate
-        else:
-            grad_embeddings = torch.empty_like(held[0]) if need_embeddings else None
-        grad_offsets = (
-            torch.empty((args.num_queries, 3), dtype=embeddings.dtype, device=dev)
-            if need_offsets
-            else None
-        )
-        with torch.cuda.device(dev):
-            self.check(
-                entry(
-                    ctypes.byref(args),
-                    z.data_ptr(),
-                    grad_embeddings.data_ptr() if need_embeddings else None,
-                    grad_offsets.data_ptr() if need_offsets else None,
-                    _stream_of(dev),
-                )
-            )
-        return grad_embeddings, grad_offsets
+        return self.host.query_backward_forward(
+            z, [embeddings, offsets, grid_indices, cell_indices, masks, lut_grid_nb2grid_idx,
+                lut_cell_nb2cell_idx, lut_cell_nb2grid_nb], interpolation, need_embeddings,
+            need_offsets, accumulate_into)
 
     def query_backward_forward_onto(self, grad_embeddings, z, *operands, need_offsets: bool = True):
         """query_backward_forward whose embedding gradient is added to
@@ -1000,44 +825,20 @@ class _Backend:
         """(grad_z, grad_embeddings, zero grad_offsets); outputs that are not
         needed are None and their work is skipped.  `accumulate_into` as for
         query_backward_forward."""
-        args, held, dev = self._query_args(
-            embeddings,
-            offsets,
-            grid_indices,
-            cell_indices,
-            masks,
-            lut_grid_nb2grid_idx,
-            lut_cell_nb2cell_idx,
-            lut_cell_nb2grid_nb,
-            interpolation,
-        )
-        n, e = args.num_queries, args.embedding_dim
-        z = _as_like(z, embeddings, (n, e), "z")
-        gg_off = _as_like(grad_grad_offsets, embeddings, (n, 3), "grad_grad_offsets")
-        grad_z = torch.empty((n, e), dtype=embeddings.dtype, device=dev) if need_z else None
-        entry = self.lib.ash_query_backward_backward
-        if accumulate_into is not None:
-            need_embeddings = True
-            grad_embeddings = _accumulator(accumulate_into, held[0])
-            entry = self.lib.ash_query_backward_backward_accumulate
-        else:
-            grad_embeddings = torch.empty_like(held[0]) if need_embeddings else None
-        with torch.cuda.device(dev):
-            self.check(
-                entry(
-                    ctypes.byref(args),
-                    gg_off.data_ptr(),
-                    z.data_ptr(),
-                    grad_z.data_ptr() if need_z else None,
-                    grad_embeddings.data_ptr() if need_embeddings else None,
-                    _stream_of(dev),
-                )
-            )
-        # the offsets second-order term is not produced (ash/src/grid.cu:417-418)
-        grad_offsets = torch.zeros((n, 3), dtype=embeddings.dtype, device=dev)
-        return grad_z, grad_embeddings, grad_offsets
+        grad_z, grad_embeddings = self.host.query_backward_backward(
+            grad_grad_offsets, z,
+            [embeddings, offsets, grid_indices, cell_indices, masks, lut_grid_nb2grid_idx,
+             lut_cell_nb2cell_idx, lut_cell_nb2grid_nb], interpolation, need_z, need_embeddings,
+            accumulate_into)
+        # the offsets second-order term is not produced (ash/src/grid.cu:417-418):
+        # zeros, all of them one element
+        zero = _ZEROS.get((embeddings.device, embeddings.dtype))
+        if zero is None:
+            zero = _ZEROS[embeddings.device, embeddings.dtype] = embeddings.new_zeros(())
+        return grad_z, grad_embeddings, zero.expand(grid_indices.shape[0], 3)
 
 
+_ZEROS: Dict[Tuple[torch.device, torch.dtype], torch.Tensor] = {}
 _STAGING: Dict[int, torch.Tensor] = {}
 
 
@@ -1053,37 +854,8 @@ def _status_staging() -> torch.Tensor:
     return staging
 
 
-def _accumulator(t: torch.Tensor, embeddings: torch.Tensor) -> torch.Tensor:
-    """Checks that `t` can take a gradient of `embeddings` in place."""
-    if (
-        t.shape != embeddings.shape
-        or t.dtype != embeddings.dtype
-        or t.device != embeddings.device
-        or not t.is_contiguous()
-    ):
-        raise RuntimeError("accumulate_into must be a contiguous tensor like the embeddings")
-    return t
-
-
-def _row_bytes(t: torch.Tensor) -> int:
-    return t.numel() // t.shape[0] * t.element_size()
-
-
-def _numel(shape) -> int:
-    n = 1
-    for s in shape:
-        n *= s
-    return n
-
-
-def _as_like(t: torch.Tensor, ref: torch.Tensor, shape, name: str) -> torch.Tensor:
-    if t.device != ref.device:
-        raise RuntimeError(f"{name} is on {t.device}, embeddings on {ref.device}")
-    if t.dtype != ref.dtype:
-        raise RuntimeError(f"{name} must be {ref.dtype}, got {t.dtype}")
-    if t.numel() != _numel(shape):
-        raise RuntimeError(f"{name} has shape {tuple(t.shape)}, expected {shape}")
-    return t.contiguous()
+def _staging_address() -> int:
+    return _status_staging().data_ptr()
 
 
 class _HashMap:
@@ -1143,6 +915,7 @@ class _HashMap:
                 )
             )
         self._handle = handle
+        self._address, self._index = handle.value, self._device.index
 
     def __del__(self):
         handle, self._handle = getattr(self, "_handle", None), None
@@ -1162,9 +935,7 @@ class _HashMap:
             raise RuntimeError(f"keys must be (N, {self.key_dim}), got {tuple(keys.shape)}")
         if keys.device != self._device:
             raise RuntimeError(f"keys are on {keys.device}, the map on {self._device}")
-        if keys.dtype != torch.int32:
-            keys = keys.to(torch.int32)
-        return keys.contiguous()
+        return keys.to(torch.int32).contiguous()
 
     def _scratch(self, nbytes: int) -> Optional[torch.Tensor]:
         return torch.empty(nbytes, dtype=torch.uint8, device=self._device) if nbytes else None
@@ -1204,11 +975,10 @@ class _HashMap:
     def counters(self) -> Dict[str, int]:
         """The table's counters as the handle knows them; copied from the
         device only when no earlier call has left them on the host."""
-        out = (_I64 * 7)()
-        with torch.cuda.device(self._device):
-            self._check(self._lib.ash_map_counters(
-                self._handle, _status_staging().data_ptr(), out, self._stream()))
-        return dict(zip(self._COUNTERS, out))
+        return dict(zip(self._COUNTERS, self._read_counters()))
+
+    def _read_counters(self):
+        return self._backend.host.counters(self._address, self._index, _staging_address())
 
     def status(self) -> Dict[str, int]:
         """The counters by a copy from the device, whatever the handle knows."""
@@ -1240,45 +1010,17 @@ class _HashMap:
         return n.value if rc == 1 else None
 
     def size(self) -> int:
-        return self.counters()["size"]
+        return self._read_counters()[0]
 
     def find(self, keys: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
-        keys = self._keys(keys)
-        n = keys.shape[0]
-        indices = torch.empty(n, dtype=torch.int64, device=self._device)
-        masks = torch.empty(n, dtype=torch.bool, device=self._device)
-        with torch.cuda.device(self._device):
-            self._check(
-                self._lib.ash_map_find(
-                    self._handle, keys.data_ptr(), n, indices.data_ptr(), masks.data_ptr(),
-                    self._stream(),
-                )
-            )
-        return indices, masks
+        return self._backend.host.find(self._address, self.key_dim, self._index, keys)
 
     def query_cells(
         self, x: torch.Tensor, grid_dim: int
     ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
         """Fused front end of `SparseDenseGrid.query`: positions in cell units ->
         (grid_indices, cell_indices, offsets, masks) in one kernel."""
-        if x.dim() != 2 or x.shape[1] != 3 or x.dtype != torch.float32:
-            raise RuntimeError("positions must be float32 (N, 3)")
-        if x.device != self._device:
-            raise RuntimeError(f"positions are on {x.device}, the map on {self._device}")
-        x = x.contiguous()
-        n = x.shape[0]
-        grid_indices = torch.empty(n, dtype=torch.int64, device=self._device)
-        cell_indices = torch.empty(n, dtype=torch.int64, device=self._device)
-        offsets = torch.empty((n, 3), dtype=torch.float32, device=self._device)
-        masks = torch.empty(n, dtype=torch.bool, device=self._device)
-        with torch.cuda.device(self._device):
-            self._check(
-                self._lib.ash_grid_query(
-                    self._handle, x.data_ptr(), n, int(grid_dim), grid_indices.data_ptr(),
-                    cell_indices.data_ptr(), offsets.data_ptr(), masks.data_ptr(), self._stream(),
-                )
-            )
-        return grid_indices, cell_indices, offsets, masks
+        return self._backend.host.query_cells(self._address, self._index, x, grid_dim)
 
     def _activation_buffers(self, cells: torch.Tensor) -> torch.Tensor:
         if self.key_dim != 3:
@@ -1435,7 +1177,7 @@ class _HashMap:
         self.version = next(_VERSIONS)
 
     def insert_keys(self, keys: torch.Tensor) -> None:
-        self._insert(self._keys(keys), 0, None, None, None)
+        self._insert(keys, [], [], [])
 
     def insert(
         self,
@@ -1443,75 +1185,31 @@ class _HashMap:
         values: Dict[str, torch.Tensor],
         external_values: Dict[str, torch.Tensor],
     ) -> None:
-        keys = self._keys(keys)
-        n = keys.shape[0]
-        names = list(values.keys())
-        if not names:
-            return self.insert_keys(keys)
-        src, dst, row_bytes = [], [], []
-        for name in names:
-            v, ext = values[name], external_values[name]
-            if v.shape[0] != n:
-                raise RuntimeError(f"value '{name}' has {v.shape[0]} rows for {n} keys")
-            if v.dtype != ext.dtype or v.shape[1:] != ext.shape[1:]:
-                raise RuntimeError(f"value '{name}' does not match its destination buffer")
-            if v.device != self._device or ext.device != self._device:
-                raise RuntimeError(f"value '{name}' is not on {self._device}")
-            if not ext.is_contiguous():
-                raise RuntimeError(f"destination buffer '{name}' must be contiguous")
-            if ext.shape[0] != self.capacity:
-                raise RuntimeError(f"destination buffer '{name}' must have `capacity` rows")
-            v = v.contiguous()
-            src.append(v)
-            dst.append(ext)
-            row_bytes.append((v.numel() // max(n, 1)) * v.element_size() if n else 0)
-        k = len(names)
-        self._insert(keys, k, (_PTR * k)(*[t.data_ptr() for t in src]),
-                     (_PTR * k)(*[t.data_ptr() for t in dst]), (_I64 * k)(*row_bytes), held=src)
+        self._insert(keys, list(values), list(values.values()), [external_values[name] for name in values])
 
-    def _insert(self, keys, k, c_src, c_dst, c_rows, held=None) -> None:
+    def _insert(self, keys, names, values, stores) -> None:
         """One ash_map_insert_auto (a second one after the second region has
         been attached, the first time a key does not fit the packed code)."""
-        n = keys.shape[0]
-        if n == 0:
-            return
         policy = _POLICY[BULK_INSERT]
-        if self._landing is None and n >= (1 << 12):
+        if self._landing is None and keys.shape[0] >= (1 << 12):
             # a batch that may take the streaming path: the map gets a landing
             # place of its own for the read-back queued behind such an insert
             self._landing = torch.zeros(16, dtype=torch.int32, pin_memory=True)
             self._check(self._lib.ash_map_set_staging(self._handle, self._landing.data_ptr()))
         for _ in range(2):
-            nbytes = _I64(0)
-            self._check(self._lib.ash_map_insert_scratch_bytes(
-                self._handle, n, k, c_rows, policy, ctypes.byref(nbytes)))
-            scratch = self._scratch(nbytes.value)
-            with torch.cuda.device(self._device):
-                rc = self._lib.ash_map_insert_auto(
-                    self._handle, keys.data_ptr(), n, k, c_src, c_dst, c_rows,
-                    scratch.data_ptr() if scratch is not None else None, nbytes.value, policy,
-                    _status_staging().data_ptr(), self._stream())
+            waiting = self._backend.host.insert(self._address, self.key_dim, self._index, self.capacity,
+                                                keys, names, values, stores, policy, _staging_address())
             self.version = next(_VERSIONS)
-            if rc != NEEDS_GENERAL:
-                return self._check(rc)
+            if not waiting:
+                return
             self._attach_general()
         raise RuntimeError("internal error: unpackable keys pending with region attached")
 
     def erase(self, keys: torch.Tensor) -> None:
-        keys = self._keys(keys)
-        n = keys.shape[0]
-        policy = _POLICY[BULK_ERASE]
-        nbytes = _I64(0)
-        self._check(self._lib.ash_map_erase_scratch_bytes(
-            self._handle, n, policy, ctypes.byref(nbytes)))
-        scratch = self._scratch(nbytes.value)
-        self.last_erase_path = "per-key" if scratch is None else "streaming"
+        streaming = self._backend.host.erase(self._address, self.key_dim, self._index, keys,
+                                             _POLICY[BULK_ERASE])
+        self.last_erase_path = "streaming" if streaming else "per-key"
         self.version = next(_VERSIONS)
-        with torch.cuda.device(self._device):
-            self._check(self._lib.ash_map_erase_auto(
-                self._handle, keys.data_ptr(), n,
-                scratch.data_ptr() if scratch is not None else None, nbytes.value, policy,
-                self._stream()))
 
     def clear(self) -> None:
         with torch.cuda.device(self._device):
@@ -1520,21 +1218,12 @@ class _HashMap:
 
     def items(self) -> Tuple[torch.Tensor, torch.Tensor]:
         n = self.size()
-        keys = torch.empty((n, self.key_dim), dtype=torch.int32, device=self._device)
-        indices = torch.empty(n, dtype=torch.int64, device=self._device)
         # whether entry i is listed under index i: the value rows of the listing
         # are then the first n rows of every value tensor (HashMap.items)
         dense = ctypes.c_int(0)
         self._check(self._lib.ash_map_items_in_index_order(self._handle, ctypes.byref(dense)))
         self.last_items_in_index_order = bool(dense.value)
-        if n > 0:
-            with torch.cuda.device(self._device):
-                self._check(
-                    self._lib.ash_map_items(
-                        self._handle, keys.data_ptr(), indices.data_ptr(), n, self._stream()
-                    )
-                )
-        return keys, indices
+        return self._backend.host.items(self._address, self.key_dim, self._index, n)
 
     def load_states(self, states: Dict[str, torch.Tensor]) -> None:
         keys = self._keys(states["active_keys"])

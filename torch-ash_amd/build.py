@@ -3,7 +3,8 @@
     python torch-ash_amd/build.py            # rebuild when sources are newer
     python torch-ash_amd/build.py --force    # always rebuild
 
-The library lands in torch-ash_amd/ash/lib/ so that it travels with the source
+and beside it _ash_host.so, the host side of its calls on torch tensors (plain
+C++ against the installed torch).  The libraries land in torch-ash_amd/ash/lib/ so that they travel with the source
 tree; nothing is installed into site-packages.
 """
 import argparse
@@ -16,6 +17,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT_DIR = os.path.join(HERE, "ash", "lib")
 OUT = os.path.join(OUT_DIR, "libash_hip.so")
+HOST_SOURCE = os.path.join(CSRC, "ash_host.cpp")
+HOST_OUT = os.path.join(OUT_DIR, "_ash_host.so")
 SOURCES = ["ash_map.hip", "ash_bulk.hip", "ash_query.hip", "ash_fusion.hip", "ash_mesh.hip"]
 HEADERS = [
     os.path.join(CSRC, "ash_probe.h"),
@@ -65,15 +68,67 @@ def source_fingerprint() -> str:
     return h.hexdigest()
 
 
-def is_stale() -> bool:
-    if not os.path.exists(OUT):
+def _older(out, deps) -> bool:
+    if not os.path.exists(out):
         return True
-    built = os.path.getmtime(OUT)
-    deps = [os.path.join(CSRC, s) for s in SOURCES] + HEADERS + [os.path.abspath(__file__)]
-    return any(os.path.getmtime(d) > built for d in deps)
+    built = os.path.getmtime(out)
+    return any(os.path.getmtime(d) > built for d in [*deps, os.path.abspath(__file__)])
+
+
+def is_stale() -> bool:
+    return _older(OUT, [os.path.join(CSRC, s) for s in SOURCES] + HEADERS)
+
+
+def host_is_stale() -> bool:
+    return _older(HOST_OUT, [HOST_SOURCE, HEADERS[-1]])
+
+
+def host_command(out: str):
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    libs = os.path.join(os.path.dirname(torch.__file__), "lib")
+    includes = [*cpp_extension.include_paths(), os.environ.get("ROCM_PATH", "/opt/rocm") + "/include",
+                sysconfig.get_paths()["include"]]
+    return [
+        os.environ.get("CXX") or shutil.which("g++") or "c++",
+        "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+        "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_API_INCLUDE_EXTENSION_H",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+        *[arg for path in dict.fromkeys(includes) for arg in ("-isystem", path)],
+        HOST_SOURCE, "-o", out, f"-L{libs}", "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10",
+        "-lc10_hip", f"-Wl,-rpath,{libs}",
+    ]
+
+
+def build_host(verbose: bool = True):
+    """Starts the compiler; returns what finishes the job."""
+    os.makedirs(OUT_DIR, exist_ok=True)
+    tmp = HOST_OUT + ".tmp"
+    cmd = host_command(tmp)
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    process = subprocess.Popen(cmd)
+
+    def finish():
+        if process.wait() != 0:
+            raise RuntimeError("compile failed: " + " ".join(cmd))
+        os.replace(tmp, HOST_OUT)
+
+    return finish
 
 
 def build(force: bool = False, verbose: bool = True) -> str:
+    finish_host = build_host(verbose) if force or host_is_stale() else lambda: None
+    try:
+        return build_kernels(force, verbose)
+    finally:
+        finish_host()
+
+
+def build_kernels(force: bool, verbose: bool) -> str:
     if not force and not is_stale():
         return OUT
     os.makedirs(OUT_DIR, exist_ok=True)

@@ -1,0 +1,594 @@
+// Host side of the calls in native code: argument checks, outputs from torch's
+// caching allocator, the current stream, one call of the C ABI.  Host code only
+// (no kernels, no GPU run-time calls of its own besides torch's); the kernels and
+// every decision about them stay behind include/ash_hip.h, whose functions are
+// looked up in the library that the Python loader has opened (`bind`).
+//
+// A call costs the host 4-6 us this way; the same in Python through ctypes took
+// 15-25 us, more than the kernels of a small batch (a find of a thousand keys
+// with their rows: 23 us of Python around 7 us of kernel).
+#include <torch/extension.h>
+
+#include <c10/hip/HIPStream.h>
+
+#include <dlfcn.h>
+
+#include <optional>
+#include <stdexcept>
+#include <string>
+#include <tuple>
+#include <vector>
+
+#include "../../include/ash_hip.h"
+
+namespace {
+
+using torch::Tensor;
+namespace py = pybind11;
+
+// --------------------------------------------------------------- the library
+#define ASH_FUNCTIONS(X)                                                              \
+    X(ash_last_error)                                                                 \
+    X(ash_map_find)                                                                   \
+    X(ash_map_find_rows)                                                              \
+    X(ash_add_rows)                                                                   \
+    X(ash_gather_rows)                                                                \
+    X(ash_map_insert_scratch_bytes)                                                   \
+    X(ash_map_insert_auto)                                                            \
+    X(ash_map_erase_scratch_bytes)                                                    \
+    X(ash_map_erase_auto)                                                             \
+    X(ash_map_items)                                                                  \
+    X(ash_map_counters)                                                               \
+    X(ash_grid_query)                                                                 \
+    X(ash_grid_forward)                                                               \
+    X(ash_query_forward)                                                              \
+    X(ash_query_backward_forward)                                                     \
+    X(ash_query_backward_forward_accumulate)                                          \
+    X(ash_query_backward_backward)                                                    \
+    X(ash_query_backward_backward_accumulate)
+
+struct Library {
+#define X(name) decltype(&::name) name = nullptr;
+    ASH_FUNCTIONS(X)
+#undef X
+} lib;
+
+[[noreturn]] void fail(const std::string& message) { throw std::runtime_error(message); }
+
+void need(bool ok, const char* message) {
+    if (!ok) fail(message);
+}
+
+void check(int status) {
+    if (status != 0) {
+        const char* m = lib.ash_last_error();
+        fail(m != nullptr && *m ? m : "libash_hip call failed");
+    }
+}
+
+// `handle`: what dlopen gave the Python loader
+void bind(uintptr_t handle) {
+    void* h = reinterpret_cast<void*>(handle);
+#define X(name)                                                                       \
+    lib.name = reinterpret_cast<decltype(&::name)>(dlsym(h, #name));                  \
+    if (lib.name == nullptr) fail("libash_hip.so does not export " #name);
+    ASH_FUNCTIONS(X)
+#undef X
+}
+
+// ------------------------------------------------------------------- helpers
+ash_map_t* map_of(uintptr_t handle) { return reinterpret_cast<ash_map_t*>(handle); }
+
+void* stream_of(int64_t device) {
+    return c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(device)).stream();
+}
+
+Tensor empty(at::IntArrayRef sizes, at::ScalarType type, int64_t device) {
+    return at::empty(sizes, at::TensorOptions().dtype(type).device(
+                                    at::kCUDA, static_cast<c10::DeviceIndex>(device)));
+}
+
+template <typename T>
+T* ptr(const Tensor& t) {
+    return t.defined() ? static_cast<T*>(t.data_ptr()) : nullptr;
+}
+
+std::string shape_of(const Tensor& t) {
+    std::string s = "(";
+    for (int64_t d = 0; d < t.dim(); ++d) {
+        s += std::to_string(t.size(d));
+        s += d + 1 < t.dim() ? ", " : t.dim() == 1 ? "," : "";
+    }
+    return s + ")";
+}
+
+Tensor keys_of(const Tensor& keys, int64_t dim, int64_t device) {
+    if (keys.dim() != 2 || keys.size(1) != dim) {
+        fail("keys must be (N, " + std::to_string(dim) + "), got " + shape_of(keys));
+    }
+    if (!keys.is_cuda() || keys.get_device() != device) {
+        fail("keys are on " + keys.device().str() + ", the map on cuda:" + std::to_string(device));
+    }
+    return keys.to(at::kInt).contiguous();
+}
+
+int64_t row_bytes_of(const Tensor& t) {
+    return t.numel() / t.size(0) * static_cast<int64_t>(t.element_size());
+}
+
+int32_t dtype_of(const Tensor& t, const char* what) {
+    if (t.scalar_type() == at::kFloat) return ASH_F32;
+    if (t.scalar_type() == at::kDouble) return ASH_F64;
+    fail(std::string(what) + " must be float32 or float64, got torch." +
+         (t.scalar_type() == at::kHalf ? "float16" : c10::toString(t.scalar_type())));
+}
+
+int32_t interpolation_of(const std::string& name) {
+    if (name == "linear") return ASH_INTERP_LINEAR;
+    if (name == "smooth_step") return ASH_INTERP_SMOOTH_STEP;
+    fail("Unknown interpolation functor: " + name);
+}
+
+// ------------------------------------------------------------------- look-up
+std::tuple<Tensor, Tensor> find(uintptr_t handle, int64_t dim, int64_t device, const Tensor& keys_in) {
+    const Tensor keys = keys_of(keys_in, dim, device);
+    const int64_t n = keys.size(0);
+    Tensor indices = empty({n}, at::kLong, device), masks = empty({n}, at::kBool, device);
+    check(lib.ash_map_find(map_of(handle), ptr<int32_t>(keys), n, ptr<int64_t>(indices),
+                           ptr<uint8_t>(masks), stream_of(device)));
+    return {indices, masks};
+}
+
+constexpr int64_t kMaxRowBytes = 32764;   // ash_map_find_rows
+constexpr size_t kMaxTables = 4;
+
+bool finds_rows_of(const std::vector<Tensor>& tables, int64_t device) {
+    if (tables.empty() || tables.size() > kMaxTables) return false;
+    for (const Tensor& t : tables) {
+        if (!t.is_cuda() || t.get_device() != device || !t.is_contiguous() || t.dim() < 1 ||
+            t.numel() == 0 || t.size(0) > 0x7FFFFFFFll) {
+            return false;
+        }
+        const int64_t bytes = row_bytes_of(t);
+        if (bytes > kMaxRowBytes || bytes % 4 != 0) return false;
+    }
+    return true;
+}
+
+std::tuple<Tensor, Tensor, std::vector<Tensor>> find_rows(uintptr_t handle, int64_t dim, int64_t device,
+                                                          const Tensor& keys_in,
+                                                          const std::vector<Tensor>& tables,
+                                                          bool zero_misses, bool need_indices) {
+    const Tensor keys = keys_of(keys_in, dim, device);
+    need(tables.size() <= kMaxTables, "find_rows takes up to 4 tensors per call");
+    const int64_t n = keys.size(0);
+    Tensor indices = need_indices ? empty({n}, at::kLong, device) : Tensor();
+    Tensor masks = empty({n}, at::kBool, device);
+    std::vector<Tensor> rows;
+    const void* src[kMaxTables];
+    void* dst[kMaxTables];
+    int64_t bytes[kMaxTables], count[kMaxTables];
+    for (const Tensor& t : tables) {
+        const size_t v = rows.size();
+        std::vector<int64_t> shape = t.sizes().vec();
+        shape[0] = n;
+        rows.push_back(empty(shape, t.scalar_type(), device));
+        src[v] = t.data_ptr();
+        dst[v] = rows[v].data_ptr();
+        bytes[v] = row_bytes_of(t);
+        count[v] = t.size(0);
+    }
+    check(lib.ash_map_find_rows(map_of(handle), ptr<int32_t>(keys), n, static_cast<int>(tables.size()),
+                                src, dst, bytes, count, zero_misses, ptr<int64_t>(indices),
+                                ptr<uint8_t>(masks), stream_of(device)));
+    return {indices, masks, rows};
+}
+
+Tensor add_rows(const Tensor& rows_in, const Tensor& indices, const Tensor& masks, int64_t out_rows) {
+    need(rows_in.is_cuda() && rows_in.dim() == 2, "rows must be (N, E) on a HIP device");
+    const int64_t n = rows_in.size(0), width = rows_in.size(1), device = rows_in.get_device();
+    need(indices.numel() == n && masks.numel() == n && indices.scalar_type() == at::kLong &&
+                 masks.scalar_type() == at::kBool && indices.is_cuda() && masks.is_cuda() &&
+                 indices.get_device() == device && masks.get_device() == device,
+         "add_rows: one int64 index and one mask per row are needed");
+    const Tensor rows = rows_in.contiguous();
+    Tensor out = empty({out_rows, width}, rows.scalar_type(), device);
+    check(lib.ash_add_rows(rows.data_ptr(), ptr<int64_t>(indices.contiguous()),
+                           ptr<uint8_t>(masks.contiguous()), n, width, dtype_of(rows, "rows"),
+                           out.data_ptr(), out_rows, stream_of(device)));
+    return out;
+}
+
+// Rows of `embedding` under `keys`, zeros for keys that are not stored.  Linear
+// in the embedding: its backward (AddRows) and the backward of that need
+// nothing but the indices found here.
+struct AddRows : torch::autograd::Function<AddRows> {
+    static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& z, const Tensor& indices,
+                          const Tensor& masks, int64_t num_rows) {
+        ctx->save_for_backward({indices, masks});
+        return add_rows(z, indices, masks, num_rows);
+    }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                   torch::autograd::variable_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        return {saved[1].unsqueeze(-1) * grads[0].index({saved[0]}), Tensor(), Tensor(), Tensor()};
+    }
+};
+
+struct Rows : torch::autograd::Function<Rows> {
+    static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& embedding,
+                          uintptr_t handle, int64_t dim, int64_t device, const Tensor& keys) {
+        auto [indices, masks, rows] = find_rows(handle, dim, device, keys, {embedding}, true, true);
+        ctx->save_for_backward({indices, masks});
+        ctx->saved_data["num_rows"] = embedding.size(0);
+        return rows[0];
+    }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                   torch::autograd::variable_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        const int64_t num_rows = ctx->saved_data["num_rows"].toInt();
+        Tensor grad = at::GradMode::is_enabled()
+                              ? AddRows::apply(grads[0], saved[0], saved[1], num_rows)
+                              : add_rows(grads[0], saved[0], saved[1], num_rows);
+        return {grad, Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+
+Tensor embedding_rows(const Tensor& embedding, uintptr_t handle, int64_t dim, int64_t device,
+                      const Tensor& keys) {
+    if (!(at::GradMode::is_enabled() && embedding.requires_grad())) {
+        return std::get<2>(find_rows(handle, dim, device, keys, {embedding}, true, false))[0];
+    }
+    return Rows::apply(embedding, handle, dim, device, keys);
+}
+
+// Up to four tables per launch; the first `first` rows where there are no indices.
+std::vector<Tensor> gather_rows(const std::vector<Tensor>& tables, const std::optional<Tensor>& indices,
+                                int64_t first) {
+    std::vector<Tensor> out;
+    Tensor index;
+    if (indices.has_value()) index = indices->reshape({-1}).contiguous();
+    const int64_t n = index.defined() ? index.size(0) : first;
+    for (const Tensor& t : tables) {
+        std::vector<int64_t> shape = t.sizes().vec();
+        shape[0] = n;
+        out.push_back(empty(shape, t.scalar_type(), t.get_device()));
+    }
+    for (size_t start = 0; start < tables.size() && n > 0; start += kMaxTables) {
+        const size_t k = std::min(kMaxTables, tables.size() - start);
+        const void* src[kMaxTables];
+        void* dst[kMaxTables];
+        int64_t bytes[kMaxTables], count[kMaxTables];
+        for (size_t v = 0; v < k; ++v) {
+            const Tensor& t = tables[start + v];
+            src[v] = t.data_ptr();
+            dst[v] = out[start + v].data_ptr();
+            bytes[v] = row_bytes_of(t);
+            count[v] = t.size(0);
+        }
+        check(lib.ash_gather_rows(static_cast<int>(k), src, dst, bytes, count, ptr<int64_t>(index), n,
+                                  stream_of(tables[start].get_device())));
+    }
+    return out;
+}
+
+// ----------------------------------------------------------------- mutations
+// One ash_map_insert_auto; true: the second region has to be attached and the
+// call issued again.
+bool insert(uintptr_t handle, int64_t dim, int64_t device, int64_t capacity, const Tensor& keys_in,
+            const std::vector<std::string>& names, const std::vector<Tensor>& values,
+            const std::vector<Tensor>& stores, int policy, uintptr_t staging) {
+    const Tensor keys = keys_of(keys_in, dim, device);
+    const int64_t n = keys.size(0);
+    const size_t k = names.size();
+    std::vector<Tensor> held;
+    std::vector<const void*> src;
+    std::vector<void*> dst;
+    std::vector<int64_t> bytes;
+    for (size_t i = 0; i < k; ++i) {
+        const Tensor &v = values[i], &ext = stores[i];
+        const std::string what = "value '" + names[i] + "'", where = "destination buffer '" + names[i] + "'";
+        if (v.dim() < 1 || v.size(0) != n) {
+            fail(what + " has " + std::to_string(v.dim() < 1 ? 0 : v.size(0)) + " rows for " +
+                 std::to_string(n) + " keys");
+        }
+        if (v.scalar_type() != ext.scalar_type() || v.sizes().slice(1) != ext.sizes().slice(1)) {
+            fail(what + " does not match its destination buffer");
+        }
+        if (!v.is_cuda() || !ext.is_cuda() || v.get_device() != device || ext.get_device() != device) {
+            fail(what + " is not on cuda:" + std::to_string(device));
+        }
+        if (!ext.is_contiguous()) fail(where + " must be contiguous");
+        if (ext.size(0) != capacity) fail(where + " must have `capacity` rows");
+        held.push_back(v.contiguous());
+        src.push_back(held.back().data_ptr());
+        dst.push_back(ext.data_ptr());
+        bytes.push_back(n > 0 ? row_bytes_of(v) : 0);
+    }
+    if (n == 0) return false;
+    int64_t scratch_bytes = 0;
+    check(lib.ash_map_insert_scratch_bytes(map_of(handle), n, static_cast<int>(k), bytes.data(), policy,
+                                           &scratch_bytes));
+    const Tensor scratch = scratch_bytes > 0 ? empty({scratch_bytes}, at::kByte, device) : Tensor();
+    void* stream = stream_of(device);
+    int status;
+    {
+        py::gil_scoped_release waits_for_the_device;
+        status = lib.ash_map_insert_auto(map_of(handle), ptr<int32_t>(keys), n, static_cast<int>(k),
+                                         src.data(), dst.data(), bytes.data(), ptr<void>(scratch),
+                                         scratch_bytes, policy, reinterpret_cast<int32_t*>(staging),
+                                         stream);
+    }
+    if (status == ASH_NEEDS_GENERAL) return true;
+    check(status);
+    return false;
+}
+
+// Whether the streaming path was taken.
+bool erase(uintptr_t handle, int64_t dim, int64_t device, const Tensor& keys_in, int policy) {
+    const Tensor keys = keys_of(keys_in, dim, device);
+    const int64_t n = keys.size(0);
+    int64_t scratch_bytes = 0;
+    check(lib.ash_map_erase_scratch_bytes(map_of(handle), n, policy, &scratch_bytes));
+    const Tensor scratch = scratch_bytes > 0 ? empty({scratch_bytes}, at::kByte, device) : Tensor();
+    check(lib.ash_map_erase_auto(map_of(handle), ptr<int32_t>(keys), n, ptr<void>(scratch), scratch_bytes,
+                                 policy, stream_of(device)));
+    return scratch_bytes > 0;
+}
+
+std::vector<int64_t> counters(uintptr_t handle, int64_t device, uintptr_t staging) {
+    std::vector<int64_t> out(7);
+    void* stream = stream_of(device);
+    int status;
+    {
+        py::gil_scoped_release waits_for_the_device;
+        status = lib.ash_map_counters(map_of(handle), reinterpret_cast<int32_t*>(staging), out.data(), stream);
+    }
+    check(status);
+    return out;
+}
+
+std::tuple<Tensor, Tensor> items(uintptr_t handle, int64_t dim, int64_t device, int64_t n) {
+    Tensor keys = empty({n, dim}, at::kInt, device), indices = empty({n}, at::kLong, device);
+    if (n > 0) {
+        check(lib.ash_map_items(map_of(handle), ptr<int32_t>(keys), ptr<int64_t>(indices), n,
+                                stream_of(device)));
+    }
+    return {keys, indices};
+}
+
+// ---------------------------------------------------------------------- grid
+Tensor positions_of(const Tensor& x) {
+    need(x.dim() == 2 && x.size(1) == 3 && x.scalar_type() == at::kFloat, "positions must be float32 (N, 3)");
+    return x.contiguous();
+}
+
+std::tuple<Tensor, Tensor, Tensor, Tensor> query_cells(uintptr_t handle, int64_t device, const Tensor& x_in,
+                                                       int grid_dim) {
+    const Tensor x = positions_of(x_in);
+    if (!x.is_cuda() || x.get_device() != device) {
+        fail("positions are on " + x.device().str() + ", the map on cuda:" + std::to_string(device));
+    }
+    const int64_t n = x.size(0);
+    Tensor grids = empty({n}, at::kLong, device), cells = empty({n}, at::kLong, device);
+    Tensor offsets = empty({n, 3}, at::kFloat, device), masks = empty({n}, at::kBool, device);
+    check(lib.ash_grid_query(map_of(handle), ptr<float>(x), n, grid_dim, ptr<int64_t>(grids),
+                             ptr<int64_t>(cells), ptr<float>(offsets), ptr<uint8_t>(masks),
+                             stream_of(device)));
+    return {grids, cells, offsets, masks};
+}
+
+Tensor table_of(const Tensor& t, int64_t rows, int64_t device, const char* name) {
+    if (!t.is_cuda() || t.get_device() != device || t.scalar_type() != at::kLong || t.dim() != 2 ||
+        t.size(0) != rows || t.size(1) != 8) {
+        fail(std::string(name) + " must be int64 (" + std::to_string(rows) + ", 8) on cuda:" +
+             std::to_string(device));
+    }
+    return t.contiguous();
+}
+
+using Optional = std::optional<Tensor>;
+
+// (features, masks, grid_indices, cell_indices, offsets); the last three None
+// unless `need_operands`.
+std::tuple<Tensor, Tensor, Optional, Optional, Optional> grid_forward(
+        uintptr_t handle, int64_t device, const Tensor& x_in, const Tensor& emb, const Tensor& lut_g,
+        const Tensor& lut_c2c, const Tensor& lut_c2g, int grid_dim, const std::string& interpolation,
+        bool need_operands, const Optional& origin_in, double cell_size) {
+    ash_query_args args = {};
+    args.interpolation = interpolation_of(interpolation);
+    args.dtype = dtype_of(emb, "embeddings");
+    need(emb.dim() == 3 && emb.is_contiguous(),
+         "embeddings must be contiguous (num_embeddings, cells_per_grid, dim)");
+    if (!emb.is_cuda()) fail("embeddings must live on a HIP device, got " + emb.device().str());
+    if (emb.get_device() != device) {
+        fail("the map is on cuda:" + std::to_string(device) + ", embeddings on " + emb.device().str());
+    }
+    need(x_in.dim() == 2 && x_in.size(1) == 3 && x_in.scalar_type() == at::kFloat && x_in.is_cuda() &&
+                 x_in.get_device() == device,
+         "positions must be float32 (N, 3) on the device of the embeddings");
+    const Tensor x = x_in.contiguous();
+    Tensor origin;
+    if (origin_in.has_value()) {
+        need(origin_in->is_cuda() && origin_in->get_device() == device &&
+                     origin_in->scalar_type() == at::kFloat && origin_in->numel() == 3,
+             "origin must be three float32 on the device of the embeddings");
+        origin = origin_in->contiguous();
+    }
+    const int64_t b = emb.size(0), m = emb.size(1), e = emb.size(2), n = x.size(0);
+    const Tensor g = table_of(lut_g, b, device, "lut_grid_nb2grid_idx");
+    const Tensor c2c = table_of(lut_c2c, m, device, "lut_cell_nb2cell_idx");
+    const Tensor c2g = table_of(lut_c2g, m, device, "lut_cell_nb2grid_nb");
+    args.embeddings = emb.data_ptr();
+    args.lut_grid_nb2grid_idx = ptr<int64_t>(g);
+    args.lut_cell_nb2cell_idx = ptr<int64_t>(c2c);
+    args.lut_cell_nb2grid_nb = ptr<int64_t>(c2g);
+    args.num_queries = n;
+    args.num_embeddings = b;
+    args.cells_per_grid = m;
+    args.embedding_dim = e;
+    Tensor out = empty({n, e}, emb.scalar_type(), device), masks = empty({n}, at::kBool, device);
+    Tensor grids, cells, offsets;
+    if (need_operands) {
+        grids = empty({n}, at::kLong, device);
+        cells = empty({n}, at::kLong, device);
+        offsets = empty({n, 3}, at::kFloat, device);
+    }
+    check(lib.ash_grid_forward(map_of(handle), ptr<float>(x), ptr<float>(origin),
+                               static_cast<float>(cell_size), grid_dim, &args, out.data_ptr(),
+                               ptr<uint8_t>(masks), ptr<int64_t>(grids), ptr<int64_t>(cells),
+                               ptr<float>(offsets), stream_of(device)));
+    if (!need_operands) return {out, masks, Optional(), Optional(), Optional()};
+    return {out, masks, grids, cells, offsets};
+}
+
+// The operands of the three query functions: checked, contiguous, held while
+// the launch is issued.
+struct Operands {
+    ash_query_args args = {};
+    Tensor emb, held[7];
+    int64_t device, n, e;
+
+    Operands(const std::vector<Tensor>& in, const std::string& interpolation) {
+        static const char* const names[] = {"offsets", "grid_indices", "cell_indices", "masks",
+                                            "lut_grid_nb2grid_idx", "lut_cell_nb2cell_idx",
+                                            "lut_cell_nb2grid_nb"};
+        need(in.size() == 8, "a query takes the embeddings and seven operands");
+        args.interpolation = interpolation_of(interpolation);
+        args.dtype = dtype_of(in[0], "embeddings");
+        need(in[0].dim() == 3, "embeddings must be (num_embeddings, cells_per_grid, dim)");
+        if (!in[0].is_cuda()) fail("embeddings must live on a HIP device, got " + in[0].device().str());
+        emb = in[0].contiguous();
+        device = emb.get_device();
+        n = in[2].dim() > 0 ? in[2].size(0) : 0;
+        const int64_t b = emb.size(0), m = emb.size(1);
+        e = emb.size(2);
+        const int64_t numel[7] = {n * 3, n, n, n, b * 8, m * 8, m * 8};
+        const at::ScalarType type[7] = {at::kFloat, at::kLong, at::kLong, at::kBool,
+                                        at::kLong, at::kLong, at::kLong};
+        for (int t = 0; t < 7; ++t) {
+            const Tensor& x = in[t + 1];
+            if (x.device() != emb.device()) {
+                fail(std::string(names[t]) + " is on " + x.device().str() + ", embeddings on " +
+                     emb.device().str());
+            }
+            if (x.scalar_type() != type[t]) {
+                fail(std::string(names[t]) + " must be " + c10::toString(type[t]) + ", got " +
+                     c10::toString(x.scalar_type()));
+            }
+            if (x.numel() != numel[t]) {
+                fail(std::string(names[t]) + " has shape " + shape_of(x) + ", expected " +
+                     std::to_string(numel[t]) + " elements");
+            }
+            held[t] = x.contiguous();
+        }
+        args.embeddings = emb.data_ptr();
+        args.offsets = ptr<float>(held[0]);
+        args.grid_indices = ptr<int64_t>(held[1]);
+        args.cell_indices = ptr<int64_t>(held[2]);
+        args.masks = ptr<uint8_t>(held[3]);
+        args.lut_grid_nb2grid_idx = ptr<int64_t>(held[4]);
+        args.lut_cell_nb2cell_idx = ptr<int64_t>(held[5]);
+        args.lut_cell_nb2grid_nb = ptr<int64_t>(held[6]);
+        args.num_queries = n;
+        args.num_embeddings = b;
+        args.cells_per_grid = m;
+        args.embedding_dim = e;
+    }
+
+    // `t` as a contiguous tensor like the embeddings with n x width elements
+    Tensor like(const Tensor& t, int64_t width, const char* name) const {
+        if (t.device() != emb.device()) {
+            fail(std::string(name) + " is on " + t.device().str() + ", embeddings on " + emb.device().str());
+        }
+        if (t.scalar_type() != emb.scalar_type()) {
+            fail(std::string(name) + " must be " + c10::toString(emb.scalar_type()) + ", got " +
+                 c10::toString(t.scalar_type()));
+        }
+        if (t.numel() != n * width) {
+            fail(std::string(name) + " has shape " + shape_of(t) + ", expected (" + std::to_string(n) +
+                 ", " + std::to_string(width) + ")");
+        }
+        return t.contiguous();
+    }
+
+    Tensor output(int64_t width) const { return empty({n, width}, emb.scalar_type(), device); }
+
+    // where the embedding gradient goes: a new tensor, or `into` added to
+    Tensor gradient(const Optional& into, bool wanted) const {
+        if (!into.has_value()) return wanted ? at::empty_like(emb) : Tensor();
+        need(into->sizes() == emb.sizes() && into->scalar_type() == emb.scalar_type() &&
+                     into->device() == emb.device() && into->is_contiguous(),
+             "accumulate_into must be a contiguous tensor like the embeddings");
+        return *into;
+    }
+};
+
+Optional maybe(const Tensor& t) { return t.defined() ? Optional(t) : Optional(); }
+
+Tensor query_forward(const std::vector<Tensor>& operands, const std::string& interpolation) {
+    Operands q(operands, interpolation);
+    Tensor out = q.output(q.e);
+    check(lib.ash_query_forward(&q.args, out.data_ptr(), stream_of(q.device)));
+    return out;
+}
+
+std::tuple<Optional, Optional> query_backward_forward(const Tensor& z_in, const std::vector<Tensor>& operands,
+                                                      const std::string& interpolation,
+                                                      bool need_embeddings, bool need_offsets,
+                                                      const Optional& accumulate_into) {
+    Operands q(operands, interpolation);
+    const Tensor z = q.like(z_in, q.e, "z");
+    const Tensor grad = q.gradient(accumulate_into, need_embeddings);
+    const Tensor offsets = need_offsets ? q.output(3) : Tensor();
+    auto entry = accumulate_into.has_value() ? lib.ash_query_backward_forward_accumulate
+                                             : lib.ash_query_backward_forward;
+    check(entry(&q.args, z.data_ptr(), ptr<void>(grad), ptr<void>(offsets), stream_of(q.device)));
+    return {maybe(grad), maybe(offsets)};
+}
+
+std::tuple<Optional, Optional> query_backward_backward(const Tensor& gg_in, const Tensor& z_in,
+                                                       const std::vector<Tensor>& operands,
+                                                       const std::string& interpolation, bool need_z,
+                                                       bool need_embeddings,
+                                                       const Optional& accumulate_into) {
+    Operands q(operands, interpolation);
+    const Tensor z = q.like(z_in, q.e, "z"), gg = q.like(gg_in, 3, "grad_grad_offsets");
+    const Tensor grad_z = need_z ? q.output(q.e) : Tensor();
+    const Tensor grad = q.gradient(accumulate_into, need_embeddings);
+    auto entry = accumulate_into.has_value() ? lib.ash_query_backward_backward_accumulate
+                                             : lib.ash_query_backward_backward;
+    check(entry(&q.args, gg.data_ptr(), z.data_ptr(), ptr<void>(grad_z), ptr<void>(grad),
+                stream_of(q.device)));
+    return {maybe(grad_z), maybe(grad)};
+}
+
+std::tuple<Optional, Tensor, std::vector<Tensor>> find_rows_py(uintptr_t handle, int64_t dim, int64_t device,
+                                                               const Tensor& keys,
+                                                               const std::vector<Tensor>& tables,
+                                                               bool zero_misses, bool need_indices) {
+    auto [indices, masks, rows] = find_rows(handle, dim, device, keys, tables, zero_misses, need_indices);
+    return {maybe(indices), masks, rows};
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_ash_host, m) {
+    m.doc() = "host side of libash_hip.so's calls on torch tensors";
+    m.def("bind", &bind);
+    m.def("find", &find);
+    m.def("finds_rows_of", &finds_rows_of);
+    m.def("find_rows", &find_rows_py);
+    m.def("add_rows", &add_rows);
+    m.def("embedding_rows", &embedding_rows);
+    m.def("gather_rows", &gather_rows);
+    m.def("insert", &insert);
+    m.def("erase", &erase);
+    m.def("counters", &counters);
+    m.def("items", &items);
+    m.def("query_cells", &query_cells);
+    m.def("grid_forward", &grid_forward);
+    m.def("query_forward", &query_forward);
+    m.def("query_backward_forward", &query_backward_forward);
+    m.def("query_backward_backward", &query_backward_backward);
+}

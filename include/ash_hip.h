@@ -349,9 +349,8 @@ int ash_map_erase_bulk(ash_map_t* map, const int32_t* keys, int64_t n, void* wor
  *   2. it takes the streaming path (ash_map_insert_bulk) when the batch is large
  *      enough relative to the table, else the per-key kernel, with `scratch` as
  *      the workspace of either (`policy` overrides the choice);
- *   3. it reads the counters, or -- streaming path, a landing place set with
- *      ash_map_set_staging, no key of the batch handed to the per-key kernel --
- *      queues their read-back behind the insert and returns without waiting
+ *   3. it reads the counters, or -- streaming path, no key of the
+ *      batch handed to the per-key kernel -- queues their read-back behind the insert and returns without waiting
  *      for it (ash_map_counters picks it up).
  * Returns ASH_NEEDS_GENERAL (and inserts everything else) when keys of the
  * batch do not fit the packed code and no second region is attached: attach
@@ -398,8 +397,8 @@ int ash_map_upkeep(ash_map_t* map, int64_t incoming, void* scratch, int64_t scra
  * graph would empty the table at every replay). */
 int ash_map_clear(ash_map_t* map, void* stream);
 
-/* Host read-back of the device counters; always a copy from the device, which
- * synchronises `stream`.
+/* Host read-back of the device counters; always asks the device, which waits
+ * for `stream`.
  *   out[0] size (= heap counter, ash/src/hashmap_gpu.cuh:157)
  *   out[1] keys dropped because the map was full (since the last clear)
  *   out[2] tombstoned slots
@@ -413,10 +412,10 @@ int ash_map_status(ash_map_t* map, int64_t out[5], void* stream);
  * latest ash_grid_collect_touched and out[6] = entries that live in the second
  * region.  The handle follows every call that changes them: after a clear they
  * are known to be zero, after ash_map_insert_auto they have been read (or are
- * on their way, see there) -- only when neither holds are they copied from the
- * device, which synchronises `stream`.  `staging`: eight int32 of page-locked
- * host memory of the calling thread's for that copy, or NULL (pageable memory:
- * about twice the latency).  No counterpart in the reference, whose `size()`
+ * on their way, see there) -- only when neither holds is the device asked,
+ * which waits for `stream`: a kernel writes them into page-locked words that
+ * the library keeps for the map, and the host polls those.  `staging` is not
+ * used any more (NULL).  No counterpart in the reference, whose `size()`
  * synchronises every time (ash/src/hashmap_gpu.cuh:157). */
 int ash_map_counters(ash_map_t* map, int32_t* staging, int64_t out[7], void* stream);
 /* 1 while the read-back that a streaming ash_map_insert_auto queued has not
@@ -425,10 +424,8 @@ int ash_map_counters_pending(ash_map_t* map);
 /* 1 and *size when the size is known without a copy from the device (waits for
  * a queued read-back if there is one), 0 when it is not, -1 on failure. */
 int ash_map_known_size(ash_map_t* map, int64_t* size);
-/* Gives the map sixteen int32 of page-locked host memory of its own (NULL takes
- * them away again): the landing place of the read-back that a streaming
- * ash_map_insert_auto queues behind itself.  Must outlive the map or be taken
- * away first. */
+/* Without effect, kept for bindings that call it: the page-locked words in
+ * which the device leaves counters belong to the library now. */
 int ash_map_set_staging(ash_map_t* map, int32_t* staging);
 
 /* Replaces `HashMap::size` (ash/src/hashmap_gpu.cuh:157); synchronises. */

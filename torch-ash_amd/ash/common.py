@@ -15,7 +15,6 @@ import ctypes
 import importlib.util
 import itertools
 import os
-import threading
 import warnings
 from typing import Dict, Optional, Tuple
 
@@ -839,24 +838,6 @@ class _Backend:
 
 
 _ZEROS: Dict[Tuple[torch.device, torch.dtype], torch.Tensor] = {}
-_STAGING: Dict[int, torch.Tensor] = {}
-
-
-def _status_staging() -> torch.Tensor:
-    """Page-locked landing place for a copy of a map's counters that the caller
-    waits for: one per host thread for all maps (such a copy is complete when
-    the call returns, and short-lived scratch sets would otherwise each allocate
-    their own)."""
-    key = threading.get_ident()
-    staging = _STAGING.get(key)
-    if staging is None:
-        staging = _STAGING[key] = torch.zeros(8, dtype=torch.int32, pin_memory=True)
-    return staging
-
-
-def _staging_address() -> int:
-    return _status_staging().data_ptr()
-
 
 class _HashMap:
     """Same surface as the pybind class `HashMap` (ash/src/pybind.cpp:9-23).
@@ -896,7 +877,6 @@ class _HashMap:
         self._general_bytes = general_bytes.value
         self._table = torch.empty(table_bytes.value, dtype=torch.uint8, device=self._device)
         self._general = None
-        self._landing = None   # page-locked int32[16] of this map's own, made on first use
         # counts the calls that may have changed the stored keys; lets callers
         # keep results derived from the key set (orderings, tables) while it stands
         self.version = next(_VERSIONS)
@@ -920,7 +900,7 @@ class _HashMap:
     def __del__(self):
         handle, self._handle = getattr(self, "_handle", None), None
         if handle:
-            # (waits for a copy that is still on its way into `_landing`)
+            # (waits for counters that the device is still to leave on the host)
             self._lib.ash_map_destroy(handle)
 
     # -- helpers ---------------------------------------------------------
@@ -966,7 +946,7 @@ class _HashMap:
         with torch.cuda.device(self._device):
             self._check(self._lib.ash_map_upkeep(
                 self._handle, incoming, scratch.data_ptr() if scratch is not None else None,
-                nbytes.value, _status_staging().data_ptr(), self._stream()))
+                nbytes.value, None, self._stream()))
 
     # -- pybind surface --------------------------------------------------
     def device(self) -> torch.device:
@@ -978,7 +958,7 @@ class _HashMap:
         return dict(zip(self._COUNTERS, self._read_counters()))
 
     def _read_counters(self):
-        return self._backend.host.counters(self._address, self._index, _staging_address())
+        return self._backend.host.counters(self._address, self._index)
 
     def status(self) -> Dict[str, int]:
         """The counters by a copy from the device, whatever the handle knows."""
@@ -1191,14 +1171,9 @@ class _HashMap:
         """One ash_map_insert_auto (a second one after the second region has
         been attached, the first time a key does not fit the packed code)."""
         policy = _POLICY[BULK_INSERT]
-        if self._landing is None and keys.shape[0] >= (1 << 12):
-            # a batch that may take the streaming path: the map gets a landing
-            # place of its own for the read-back queued behind such an insert
-            self._landing = torch.zeros(16, dtype=torch.int32, pin_memory=True)
-            self._check(self._lib.ash_map_set_staging(self._handle, self._landing.data_ptr()))
         for _ in range(2):
             waiting = self._backend.host.insert(self._address, self.key_dim, self._index, self.capacity,
-                                                keys, names, values, stores, policy, _staging_address())
+                                                keys, names, values, stores, policy)
             self.version = next(_VERSIONS)
             if not waiting:
                 return

@@ -304,7 +304,7 @@ __device__ __forceinline__ void give_up_row(const BulkPlan& pl, int32_t row, int
 template <int DIM, bool PROV>
 __global__ __launch_bounds__(kSplitThreads) void split_keys_kernel(
         MapDev m, BulkPlan pl, const int32_t* __restrict__ keys, int identity,
-        int32_t* __restrict__ early) {
+        int32_t* early, int32_t stamp) {
     __shared__ SplitShared sh;
     const int tid = threadIdx.x;
     if (tid < kMaxBins) sh.cnt[tid] = 0;
@@ -393,7 +393,8 @@ __global__ __launch_bounds__(kSplitThreads) void split_keys_kernel(
             atomicAdd(pl.hdr + kHdrTicket, 1) == static_cast<int32_t>(gridDim.x) - 1) {
             __hip_atomic_store(early, atomicAdd(pl.hdr + kHdrSpillKeys, 0), __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_SYSTEM);
-            __threadfence_system();
+            __hip_atomic_store(early + kLandingStamp, stamp, __ATOMIC_RELEASE,
+                               __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }
 }
@@ -1264,20 +1265,20 @@ int check_values(int n_values, const void* const* src, void* const* dst,
 
 template <bool PROV>
 int launch_split_keys(ash_map* map, const BulkPlan& pl, const int32_t* keys, int identity,
-                      int32_t* early, hipStream_t s) {
+                      int32_t* early, int32_t stamp, hipStream_t s) {
     const unsigned g = static_cast<unsigned>((pl.n + kSplitChunk - 1) / kSplitChunk);
     switch (map->key_dim) {
         case 1:
-            split_keys_kernel<1, PROV><<<g, kSplitThreads, 0, s>>>(map->d, pl, keys, identity, early);
+            split_keys_kernel<1, PROV><<<g, kSplitThreads, 0, s>>>(map->d, pl, keys, identity, early, stamp);
             break;
         case 2:
-            split_keys_kernel<2, PROV><<<g, kSplitThreads, 0, s>>>(map->d, pl, keys, identity, early);
+            split_keys_kernel<2, PROV><<<g, kSplitThreads, 0, s>>>(map->d, pl, keys, identity, early, stamp);
             break;
         case 3:
-            split_keys_kernel<3, PROV><<<g, kSplitThreads, 0, s>>>(map->d, pl, keys, identity, early);
+            split_keys_kernel<3, PROV><<<g, kSplitThreads, 0, s>>>(map->d, pl, keys, identity, early, stamp);
             break;
         default:
-            split_keys_kernel<4, PROV><<<g, kSplitThreads, 0, s>>>(map->d, pl, keys, identity, early);
+            split_keys_kernel<4, PROV><<<g, kSplitThreads, 0, s>>>(map->d, pl, keys, identity, early, stamp);
             break;
     }
     ASH_LAUNCH_CHECK();
@@ -1353,12 +1354,10 @@ int ash_map_bulk_workspace_bytes(ash_map_t* map, int64_t n, int n_values,
 
 }  // extern "C"
 
-// `early`: where to leave, right after the first split pass, the number of keys
-// that pass handed to the per-key kernel; `early_event` is recorded behind it.
 int ash::insert_bulk(ash_map* map, const int32_t* keys, int64_t n,
                      int n_values, const void* const* src, void* const* dst,
                      const int64_t* row_bytes, void* workspace,
-                     int64_t workspace_bytes, int32_t* early, hipEvent_t early_event,
+                     int64_t workspace_bytes, int32_t* early, int32_t stamp,
                      void* stream) {
     if (check_batch(map, keys, n)) return 1;
     if (check_values(n_values, src, dst, row_bytes)) return 1;
@@ -1399,14 +1398,8 @@ int ash::insert_bulk(ash_map* map, const int32_t* keys, int64_t n,
     const int ninit = ncursors > kHdrWords ? ncursors : kHdrWords;
     bulk_init_kernel<<<(ninit + 255) / 256, 256, 0, s>>>(map->d, pl, ncursors);
     ASH_LAUNCH_CHECK();
-    // (pass 1 leaves the early word itself; the event tells the host when)
-    auto publish = [&]() -> int {
-        if (early != nullptr && early_event != nullptr) ASH_HIP(hipEventRecord(early_event, s));
-        return 0;
-    };
     if (n_values == 0) {
-        if (launch_split_keys<false>(map, pl, keys, identity, early, s)) return 1;
-        if (publish()) return 1;
+        if (launch_split_keys<false>(map, pl, keys, identity, early, stamp, s)) return 1;
         split_records_kernel<false><<<(pl.bins << pl.lane_shift) * pl.chunks, kSplitThreads, 0, s>>>(map->d, pl);
         ASH_LAUNCH_CHECK();
         build_kernel<false><<<pl.parts, kBuildThreads, 0, s>>>(map->d, pl, stale, identity);
@@ -1417,8 +1410,7 @@ int ash::insert_bulk(ash_map* map, const int32_t* keys, int64_t n,
         }
         return insert_selected(map, true, pl.codes_a, pl.spill_a, pl.hdr + kHdrSpillA, none, s);
     }
-    if (launch_split_keys<true>(map, pl, keys, identity, early, s)) return 1;
-    if (publish()) return 1;
+    if (launch_split_keys<true>(map, pl, keys, identity, early, stamp, s)) return 1;
     split_records_kernel<true><<<(pl.bins << pl.lane_shift) * pl.chunks, kSplitThreads, 0, s>>>(map->d, pl);
     ASH_LAUNCH_CHECK();
     build_kernel<true><<<pl.parts, kBuildThreads, 0, s>>>(map->d, pl, stale, identity);
@@ -1441,7 +1433,7 @@ int ash_map_insert_bulk(ash_map_t* map, const int32_t* keys, int64_t n,
                         const int64_t* row_bytes, void* workspace,
                         int64_t workspace_bytes, void* stream) {
     return insert_bulk(map, keys, n, n_values, src, dst, row_bytes, workspace, workspace_bytes,
-                       nullptr, nullptr, stream);
+                       nullptr, 0, stream);
 }
 
 int ash_map_erase_bulk_query(ash_map_t* map, int64_t n, int64_t* bytes, int* worthwhile) {
@@ -1482,7 +1474,7 @@ int ash_map_erase_bulk(ash_map_t* map, const int32_t* keys, int64_t n, void* wor
     const int ninit = ncursors > kHdrWords ? ncursors : kHdrWords;
     bulk_init_kernel<<<(ninit + 255) / 256, 256, 0, s>>>(map->d, pl, ncursors);
     ASH_LAUNCH_CHECK();
-    if (launch_split_keys<false>(map, pl, keys, 0, nullptr, s)) return 1;
+    if (launch_split_keys<false>(map, pl, keys, 0, nullptr, 0, s)) return 1;
     split_records_kernel<false><<<(pl.bins << pl.lane_shift) * pl.chunks, kSplitThreads, 0, s>>>(map->d, pl);
     ASH_LAUNCH_CHECK();
     erase_range_kernel<<<pl.parts, kBuildThreads, 0, s>>>(map->d, pl);

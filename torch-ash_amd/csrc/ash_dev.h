@@ -73,6 +73,7 @@ enum Counter {
     kNumCounters = 64
 };
 constexpr int kHostCounters = 8;
+constexpr int kLandingStamp = 8;   // the word behind the counters in a landing place
 constexpr int64_t kHeaderBytes = 256;
 
 // General region: open addressing over 32-bit state words + 16-byte keys.
@@ -147,12 +148,10 @@ struct ash_map {
     int64_t table_bytes;
     bool general_attached;
     // --- bookkeeping of the counters on the host ------------------------
-    // page-locked int32[16] of the caller's (ash_map_set_staging) or null:
-    // [0, 8) landing place of a read-back, [8] the count a streaming insert
-    // publishes after its first pass
-    int32_t* staging;
-    hipEvent_t early_event, late_event;   // made on first use
-    bool late_in_flight;    // a copy into staging[0, 8) may still be under way
+    int32_t* line;          // page-locked words of the map's own (take_line), made on first use
+    int32_t stamp;          // of the latest words asked for
+    int32_t late_stamp;
+    bool late_in_flight;    // the device may still owe the words at kLineLate
     bool late_pending;      // ... and it is the latest state of the counters: nobody has looked at it yet
     bool counters_known;    // `counters` is what the device holds
     ash_counters counters;

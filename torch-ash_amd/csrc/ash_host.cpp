@@ -277,7 +277,7 @@ std::vector<Tensor> gather_rows(const std::vector<Tensor>& tables, const std::op
 // call issued again.
 bool insert(uintptr_t handle, int64_t dim, int64_t device, int64_t capacity, const Tensor& keys_in,
             const std::vector<std::string>& names, const std::vector<Tensor>& values,
-            const std::vector<Tensor>& stores, int policy, uintptr_t staging) {
+            const std::vector<Tensor>& stores, int policy) {
     const Tensor keys = keys_of(keys_in, dim, device);
     const int64_t n = keys.size(0);
     const size_t k = names.size();
@@ -316,8 +316,7 @@ bool insert(uintptr_t handle, int64_t dim, int64_t device, int64_t capacity, con
         py::gil_scoped_release waits_for_the_device;
         status = lib.ash_map_insert_auto(map_of(handle), ptr<int32_t>(keys), n, static_cast<int>(k),
                                          src.data(), dst.data(), bytes.data(), ptr<void>(scratch),
-                                         scratch_bytes, policy, reinterpret_cast<int32_t*>(staging),
-                                         stream);
+                                         scratch_bytes, policy, nullptr, stream);
     }
     if (status == ASH_NEEDS_GENERAL) return true;
     check(status);
@@ -336,13 +335,13 @@ bool erase(uintptr_t handle, int64_t dim, int64_t device, const Tensor& keys_in,
     return scratch_bytes > 0;
 }
 
-std::vector<int64_t> counters(uintptr_t handle, int64_t device, uintptr_t staging) {
+std::vector<int64_t> counters(uintptr_t handle, int64_t device) {
     std::vector<int64_t> out(7);
     void* stream = stream_of(device);
     int status;
     {
         py::gil_scoped_release waits_for_the_device;
-        status = lib.ash_map_counters(map_of(handle), reinterpret_cast<int32_t*>(staging), out.data(), stream);
+        status = lib.ash_map_counters(map_of(handle), nullptr, out.data(), stream);
     }
     check(status);
     return out;

@@ -26,7 +26,12 @@
 
 #include <hip/amd_detail/amd_hip_unsafe_atomics.h>
 
+#include <sched.h>
+
+#include <algorithm>
+#include <cstring>
 #include <mutex>
+#include <vector>
 
 // Scratch of ash_grid_activate_static, the entry point that allocates nothing:
 // the list of run heads that ash_grid_activate keeps in a caller-provided
@@ -1371,6 +1376,21 @@ __global__ void fold_waiting_keys_kernel(int32_t* ctr) {
     }
 }
 
+// The counters, left where the host reads them: `landing` is page-locked host
+// memory, its word kLandingStamp tells the host that the words before it are
+// those of this launch.
+__global__ void publish_counters_kernel(const int32_t* __restrict__ ctr, int32_t* landing,
+                                        int32_t stamp) {
+    if (threadIdx.x < kHostCounters) {
+        __hip_atomic_store(landing + threadIdx.x, ctr[threadIdx.x], __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    // (one wavefront: the release waits for the stores of all its lanes)
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(landing + kLandingStamp, stamp, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 __global__ void set_counter_kernel(int32_t* ctr, int which, int32_t value) {
     if (threadIdx.x == 0 && blockIdx.x == 0) ctr[which] = value;
 }
@@ -1798,6 +1818,83 @@ int check_map(const ash_map* map) {
     return 0;
 }
 
+// ------------------------------------------- words that the device leaves here
+// What the host wants to know of a running call (the counters, how many keys the
+// first pass of a streaming insert could not place) is written by kernels into
+// page-locked host memory, stamped with a number of the call's own, and the host
+// polls the stamp: no copy on the stream, no event, and the answer is seen about
+// a microsecond after it was written, where a copy and a stream synchronisation
+// took 12-15 us of an idle device's time.
+//
+// Every map that asks gets a line of kLineWords of its own from a pool for all
+// maps (its slabs serve the maps of the process, as many lines as maps that ever
+// lived at the same time) and gives it back when it is destroyed.
+constexpr int kLineWords = 64;
+constexpr int kLineNow = 0;      // counters, fetched and waited for
+constexpr int kLineLate = 16;    // counters, fetched behind a streaming insert
+constexpr int kLineEarly = 32;   // count left by the first pass of a streaming insert
+constexpr int kLinesPerSlab = 64;
+
+std::mutex g_lines_mutex;
+std::vector<int32_t*>& free_lines() {
+    static auto* lines = new std::vector<int32_t*>;   // (outlives maps destroyed at exit)
+    return *lines;
+}
+
+int take_line(ash_map* map) {
+    if (map->line != nullptr) return 0;
+    std::lock_guard<std::mutex> lock(g_lines_mutex);
+    std::vector<int32_t*>& lines = free_lines();
+    if (lines.empty()) {
+        void* slab = nullptr;
+        ASH_HIP(hipHostMalloc(&slab, kLinesPerSlab * kLineWords * sizeof(int32_t),
+                              hipHostMallocPortable | hipHostMallocCoherent));
+        memset(slab, 0, kLinesPerSlab * kLineWords * sizeof(int32_t));
+        for (int i = 0; i < kLinesPerSlab; ++i) {
+            lines.push_back(static_cast<int32_t*>(slab) + i * kLineWords);
+        }
+    }
+    map->line = lines.back();
+    lines.pop_back();
+    // stamps of this map start where the line's last owner stopped
+    for (int at : {kLineNow, kLineLate, kLineEarly}) {
+        map->stamp = std::max(map->stamp, map->line[at + kLandingStamp]);
+    }
+    return 0;
+}
+
+void give_back_line(ash_map* map) {
+    if (map->line == nullptr) return;
+    std::lock_guard<std::mutex> lock(g_lines_mutex);
+    free_lines().push_back(map->line);
+    map->line = nullptr;
+}
+
+// Waits until the device has written `stamp`.  The wait ends with the device's
+// work at the latest: every few milliseconds without an answer the device is
+// synchronised (errors show there), after which the word has to be there.
+int wait_for_stamp(const int32_t* word, int32_t stamp) {
+    const auto arrived = [&] { return __atomic_load_n(word, __ATOMIC_ACQUIRE) == stamp; };
+    for (int64_t spin = 0; spin < 4'000'000; ++spin) {
+        if (arrived()) return 0;
+        __builtin_ia32_pause();
+        if (spin > 20'000) sched_yield();
+    }
+    ASH_HIP(hipDeviceSynchronize());
+    if (!arrived()) ASH_FAIL("internal error: the device has not left its counters");
+    return 0;
+}
+
+// A read-back queued behind an insert that may still be under way has to arrive
+// before its words are read or written again.
+int settle_landing_place(ash_map* map) {
+    if (map->late_in_flight) {
+        if (wait_for_stamp(map->line + kLineLate + kLandingStamp, map->late_stamp)) return 1;
+        map->late_in_flight = false;
+    }
+    return 0;
+}
+
 // Whether a listing has entry i under index i: nothing has written to the heap
 // since it was last 0, 1, 2, ... (no erase, no load) and no entry lives in the
 // second region -- there is none, or the counters as the host knows them say
@@ -2057,8 +2154,8 @@ int ash_map_create(int key_dim, int64_t capacity, int32_t* heap, void* table_ws,
     map->table_stale = false;
     map->heap_dirty = true;   // the caller's buffer holds anything
     map->log_stale = false;
-    map->staging = nullptr;
-    map->early_event = map->late_event = nullptr;
+    map->line = nullptr;
+    map->stamp = map->late_stamp = 0;
     map->late_in_flight = map->late_pending = false;
     map->counters_known = true;   // a new map is empty and every counter is zero
     map->counters = {};
@@ -2121,9 +2218,12 @@ int ash_map_destroy(ash_map_t* map) {
     if (map == nullptr) return 0;
     // the device may still owe a write into the caller's page-locked landing
     // place; it must have arrived before the caller gives that memory back
-    if (map->late_in_flight && map->late_event != nullptr) (void)hipEventSynchronize(map->late_event);
-    if (map->early_event != nullptr) (void)hipEventDestroy(map->early_event);
-    if (map->late_event != nullptr) (void)hipEventDestroy(map->late_event);
+    if (map->late_in_flight) {
+        DeviceGuard guard;
+        (void)guard.enter(map->device);
+        (void)settle_landing_place(map);
+    }
+    give_back_line(map);
     delete map;
     return 0;
 }
@@ -2721,33 +2821,10 @@ void decode_counters(const int32_t* host, ash_counters& c) {
     c.general_tombstones = host[kCtrGenTombs];
 }
 
-int ensure_events(ash_map* map) {
-    if (map->early_event == nullptr) {
-        ASH_HIP(hipEventCreateWithFlags(&map->early_event, hipEventDisableTiming));
-    }
-    if (map->late_event == nullptr) {
-        ASH_HIP(hipEventCreateWithFlags(&map->late_event, hipEventDisableTiming));
-    }
-    return 0;
-}
-
-// A copy into the map's own landing place that may still be under way has to
-// arrive before that memory is written or read for something else.
-int settle_landing_place(ash_map* map) {
-    if (map->late_in_flight) {
-        ASH_HIP(hipEventSynchronize(map->late_event));
-        map->late_in_flight = false;
-    }
-    return 0;
-}
-
 // Brings map->counters up to date (the map's device is current): they are
 // known already, or a read-back queued behind the latest insert brings them,
-// or they are copied now, which waits for `s`.  `staging`: eight int32 of
-// page-locked host memory of the calling thread's, or null -- a copy into
-// pageable memory goes through the runtime's own staging and takes about twice
-// as long (25 against 13 us on an idle device).
-int refresh_counters(ash_map* map, int32_t* staging, hipStream_t s) {
+// or they are fetched now, which waits for `s`.
+int refresh_counters(ash_map* map, hipStream_t s) {
     if (map->replayed) {
         if (settle_landing_place(map)) return 1;
         map->counters_known = map->late_pending = false;
@@ -2756,16 +2833,17 @@ int refresh_counters(ash_map* map, int32_t* staging, hipStream_t s) {
     if (map->late_pending) {
         if (settle_landing_place(map)) return 1;
         map->late_pending = false;
-        decode_counters(map->staging, map->counters);
+        decode_counters(map->line + kLineLate, map->counters);
     } else {
         if (is_capturing(s)) {
             ASH_FAIL("the table's counters cannot be read while the stream is being captured");
         }
-        int32_t pageable[kHostCounters] = {0};
-        int32_t* host = staging != nullptr ? staging : pageable;
-        ASH_HIP(hipMemcpyAsync(host, map->d.ctr, sizeof(pageable), hipMemcpyDeviceToHost, s));
-        ASH_HIP(hipStreamSynchronize(s));
-        decode_counters(host, map->counters);
+        if (take_line(map)) return 1;
+        const int32_t stamp = ++map->stamp;
+        publish_counters_kernel<<<1, 64, 0, s>>>(map->d.ctr, map->line + kLineNow, stamp);
+        ASH_LAUNCH_CHECK();
+        if (wait_for_stamp(map->line + kLineNow + kLandingStamp, stamp)) return 1;
+        decode_counters(map->line + kLineNow, map->counters);
     }
     map->counters_known = true;
     map->unread_inserts = 0;
@@ -2802,11 +2880,11 @@ bool should_rebuild(const ash_map* map, int64_t size, int64_t tombstones, int64_
 // tombstones, looks at the counters and re-places the live entries into an
 // emptied table when too few empty slots would remain.
 int upkeep(ash_map* map, int64_t incoming, void* scratch, int64_t scratch_bytes,
-           int32_t* staging, hipStream_t s) {
-    if (map->late_pending && refresh_counters(map, staging, s)) return 1;
+           hipStream_t s) {
+    if (map->late_pending && refresh_counters(map, s)) return 1;
     if (map->unread_inserts >= kUpkeepEvery || map->replayed) map->maybe_tombstones = true;
     if (!map->maybe_tombstones) return 0;
-    if (refresh_counters(map, staging, s)) return 1;
+    if (refresh_counters(map, s)) return 1;
     const ash_counters& c = map->counters;
     map->maybe_tombstones = c.tombstones > 0;
     if (!should_rebuild(map, c.size, c.tombstones, incoming,
@@ -2837,24 +2915,17 @@ int upkeep(ash_map* map, int64_t incoming, void* scratch, int64_t scratch_bytes,
 }  // namespace
 
 int ash_map_set_staging(ash_map_t* map, int32_t* staging) {
-    if (check_map(map)) return 1;
-    if (settle_landing_place(map)) return 1;
-    if (map->late_pending) {
-        // what the old landing place holds is the latest state of the counters
-        decode_counters(map->staging, map->counters);
-        map->counters_known = true;
-        map->late_pending = false;
-    }
-    map->staging = staging;
-    return 0;
+    (void)staging;
+    return check_map(map);
 }
 
 int ash_map_counters(ash_map_t* map, int32_t* staging, int64_t out[7], void* stream) {
+    (void)staging;
     if (check_map(map)) return 1;
     if (out == nullptr) ASH_FAIL("null status output");
     DeviceGuard guard;
     ASH_HIP(guard.enter(map->device));
-    if (refresh_counters(map, staging, static_cast<hipStream_t>(stream))) return 1;
+    if (refresh_counters(map, static_cast<hipStream_t>(stream))) return 1;
     const ash_counters& c = map->counters;
     out[0] = c.size;
     out[1] = c.dropped;
@@ -2880,7 +2951,7 @@ int ash_map_known_size(ash_map_t* map, int64_t* size) {
     if (!map->counters_known) {
         if (!map->late_pending) return 0;
         DeviceGuard guard;
-        if (guard.enter(map->device) != hipSuccess || refresh_counters(map, nullptr, nullptr)) {
+        if (guard.enter(map->device) != hipSuccess || refresh_counters(map, nullptr)) {
             return -1;
         }
     }
@@ -2896,7 +2967,7 @@ int ash_map_status(ash_map_t* map, int64_t out[5], void* stream) {
     // always a copy from the device
     map->counters_known = false;
     map->late_pending = false;
-    if (refresh_counters(map, nullptr, static_cast<hipStream_t>(stream))) return 1;
+    if (refresh_counters(map, static_cast<hipStream_t>(stream))) return 1;
     const ash_counters& c = map->counters;
     out[0] = c.size;
     out[1] = c.dropped;
@@ -2908,12 +2979,13 @@ int ash_map_status(ash_map_t* map, int64_t out[5], void* stream) {
 
 int ash_map_upkeep(ash_map_t* map, int64_t incoming, void* scratch, int64_t scratch_bytes,
                    int32_t* staging, void* stream) {
+    (void)staging;
     if (check_map(map)) return 1;
     DeviceGuard guard;
     ASH_HIP(guard.enter(map->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (is_capturing(s)) return 0;
-    return upkeep(map, incoming, scratch, scratch_bytes, staging, s);
+    return upkeep(map, incoming, scratch, scratch_bytes, s);
 }
 
 namespace {
@@ -2964,6 +3036,7 @@ int ash_map_insert_auto(ash_map_t* map, const int32_t* keys, int64_t n, int n_va
                         const void* const* src, void* const* dst, const int64_t* row_bytes,
                         void* scratch, int64_t scratch_bytes, int policy, int32_t* staging,
                         void* stream) {
+    (void)staging;
     if (check_batch(map, keys, n)) return 1;
     if (n == 0) return 0;
     int path = 0;
@@ -2981,15 +3054,16 @@ int ash_map_insert_auto(ash_map_t* map, const int32_t* keys, int64_t n, int n_va
     const bool capturing = is_capturing(s);
     // (a capture replays launches only: no look at the counters, no upkeep;
     // refused keys stay in the counters for a later call to find)
-    if (!capturing && upkeep(map, n, scratch, scratch_bytes, staging, s)) return 1;
+    if (!capturing && upkeep(map, n, scratch, scratch_bytes, s)) return 1;
     if (path == kPathStreaming) {
         int32_t* early = nullptr;
-        if (!capturing && map->staging != nullptr) {
-            if (ensure_events(map) || settle_landing_place(map)) return 1;
-            early = map->staging + kHostCounters;
+        if (!capturing) {
+            if (take_line(map) || settle_landing_place(map)) return 1;
+            early = map->line + kLineEarly;
         }
+        const int32_t stamp = ++map->stamp;
         if (insert_bulk(map, keys, n, n_values, src, dst, row_bytes, scratch, scratch_bytes,
-                        early, early != nullptr ? map->early_event : nullptr, stream)) {
+                        early, stamp, stream)) {
             return 1;
         }
         if (capturing) return 0;
@@ -2998,11 +3072,11 @@ int ash_map_insert_auto(ash_map_t* map, const int32_t* keys, int64_t n, int n_va
             // waiting for the second region; their number arrives a quarter
             // into the call's work.  None: the counters are fetched behind the
             // insert without waiting for them.
-            ASH_HIP(hipEventSynchronize(map->early_event));
+            if (wait_for_stamp(early + kLandingStamp, stamp)) return 1;
             if (*early == 0) {
-                ASH_HIP(hipMemcpyAsync(map->staging, map->d.ctr, kHostCounters * sizeof(int32_t),
-                                       hipMemcpyDeviceToHost, s));
-                ASH_HIP(hipEventRecord(map->late_event, s));
+                map->late_stamp = stamp;
+                publish_counters_kernel<<<1, 64, 0, s>>>(map->d.ctr, map->line + kLineLate, stamp);
+                ASH_LAUNCH_CHECK();
                 map->late_in_flight = true;
                 map->late_pending = true;
                 map->unread_inserts = 0;
@@ -3017,7 +3091,7 @@ int ash_map_insert_auto(ash_map_t* map, const int32_t* keys, int64_t n, int n_va
         }
         if (capturing) return 0;
     }
-    if (refresh_counters(map, staging, s)) return 1;
+    if (refresh_counters(map, s)) return 1;
     if (map->counters.exotic_pending > 0 && map->general_attached) {
         fold_waiting_keys_kernel<<<1, 64, 0, s>>>(map->d.ctr);
         ASH_LAUNCH_CHECK();

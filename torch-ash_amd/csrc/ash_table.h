@@ -162,12 +162,13 @@ inline bool heap_in_order(const ash_map* map) { return !map->heap_dirty && !map-
 // false for one that took entries away.
 // `s`: the stream the call runs on (captured: see ash_map::replayed).
 void counters_changed(ash_map* map, bool inserted, hipStream_t s);
-// The streaming insert (ash_bulk.hip); `early`, `early_event` as for
-// ash_map_insert_bulk_early (both may be null).
+// The streaming insert (ash_bulk.hip); `early`: page-locked words (or null) where
+// its first pass leaves the number of keys that it hands to the per-key kernel,
+// and behind it, at kLandingStamp, `stamp`.
 int insert_bulk(ash_map* map, const int32_t* keys, int64_t n, int n_values,
                 const void* const* src, void* const* dst, const int64_t* row_bytes,
                 void* workspace, int64_t workspace_bytes, int32_t* early,
-                hipEvent_t early_event, void* stream);
+                int32_t stamp, void* stream);
 // Fills the bucket array if a clear() left that to the next user of the table.
 int settle_table(ash_map* map, hipStream_t s);
 // Before the first call that writes to the heap (an erase; a load brings a

@@ -237,6 +237,25 @@ int ash_grid_integrate_depth_flagged(ash_map_t* map, float* embeddings,
                                      const float* color, int height, int width,
                                      float trunc, float depth_max, void* stream);
 
+/* A frame of a fusion loop (demo/rgbd_fusion.py:200-254) in one call:
+ * ash_grid_activate_positions and ash_grid_integrate_depth_flagged, two
+ * launches.  Cell to world is cell * cell_to_world [+ world_origin], with
+ * world_origin float32[3] on the device or NULL.  group_counts (int32
+ * [ASH_FLAGGED_GROUPS] on the device, or NULL): a third, small launch adds up
+ * the touched blocks and leaves the counters for the host behind the two others;
+ * the next ash_map_counters waits for it and finds them in out[5].  Refused
+ * with group_counts on a stream that is being captured. */
+enum { ASH_FLAGGED_GROUPS = 8192 };
+int ash_grid_fuse_frame(ash_map_t* map, const float* positions, int64_t n,
+                        const float* origin, float cell_size, int dilation,
+                        int bidirectional, int bound_lo, int bound_hi, uint8_t* touched,
+                        int32_t* coords, float* embeddings, int64_t num_embeddings,
+                        int grid_dim, int embedding_dim, float cell_to_world,
+                        const float* world_origin, const float* intrinsic,
+                        const float* extrinsic, const float* depth, const float* color,
+                        int height, int width, float trunc, float depth_max,
+                        int32_t* group_counts, void* stream);
+
 /* Replaces `ray_find_near_far` (ash/src/sampler.cu:7-121, pybind.cpp:35): per
  * ray, march from t_min in steps of half a block while inside the box
  * [bbox_min, bbox_max] and report the range [near, far] that contains active

@@ -101,6 +101,12 @@ _SIGNATURES = {
          ctypes.POINTER(ctypes.c_float), _PTR, _PTR, _PTR, _PTR, ctypes.c_int, ctypes.c_int,
          ctypes.c_float, ctypes.c_float, _PTR],
     ),
+    "ash_grid_fuse_frame": (
+        ctypes.c_int,
+        [_PTR, _PTR, _I64, _PTR, ctypes.c_float, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+         ctypes.c_int, _PTR, _PTR, _PTR, _I64, ctypes.c_int, ctypes.c_int, ctypes.c_float]
+        + [_PTR] * 5 + [ctypes.c_int, ctypes.c_int, ctypes.c_float, ctypes.c_float, _PTR, _PTR],
+    ),
     "ash_grid_integrate_depth": (
         ctypes.c_int,
         [_PTR, _I64, ctypes.c_int, ctypes.c_int, _PTR, _PTR, _I64, ctypes.c_float,
@@ -277,6 +283,8 @@ RAY_STAGE_EXTRA = 2
 # Largest table whose touched rows ash_grid_collect_touched lists (the header's
 # ASH_COLLECT_MAX_BLOCKS).
 COLLECT_MAX_BLOCKS = 1 << 20
+# Workgroups of the integration that goes by flags (the header's ASH_FLAGGED_GROUPS).
+FLAGGED_GROUPS = 8192
 # Size of a second region that is attached before any key has asked for it
 # (2^16 slots of 20 bytes).
 GENERAL_JUST_IN_CASE_BYTES = 20 << 16
@@ -1154,6 +1162,50 @@ class _HashMap:
                 int(grid_dim), int(dilation), int(bool(bidirectional)), int(bound_lo),
                 int(bound_hi), self._touched.data_ptr(), self._block_coords.data_ptr(),
                 self._stream()))
+        self.version = next(_VERSIONS)
+
+    def fuse_frame(
+        self,
+        positions: torch.Tensor,
+        origin: Optional[torch.Tensor],
+        cell_size: float,
+        dilation: int,
+        bidirectional: bool,
+        bounds: Tuple[int, int],
+        embeddings: torch.Tensor,
+        grid_dim: int,
+        cell_to_world: Tuple[float, Optional[torch.Tensor]],
+        intrinsic: torch.Tensor,
+        extrinsic: torch.Tensor,
+        depth: torch.Tensor,
+        color: Optional[torch.Tensor],
+        trunc: float,
+        depth_max: float,
+        count: bool,
+    ) -> None:
+        """The activation of `activate_blocks` from world positions (cell units
+        = (positions - origin) / cell_size) and the depth integration over the
+        rows it touches, two launches; with `count` a third leaves the counters,
+        the number of touched blocks among them, where `counters` finds them.
+        Nothing waits for the device and nothing is allocated once the map's
+        arrays exist, so the launches can (without `count`) be captured into a
+        graph; keys refused for lack of capacity show in the counters at the
+        next call that reads them."""
+        self._activation_buffers(positions)
+        counts = None
+        if count:
+            counts = getattr(self, "_group_counts", None)
+            if counts is None:
+                counts = self._group_counts = torch.empty(FLAGGED_GROUPS, dtype=torch.int32,
+                                                          device=self._device)
+        if self._general is None:
+            # a key beyond the packed range would otherwise wait for a read-back
+            # that this path does not make
+            self._attach_general(just_in_case=True)
+        self._backend.host.fuse_frame(
+            self._address, self._index, positions, origin, cell_size, dilation, bool(bidirectional),
+            *bounds, self._touched, self._block_coords, embeddings, grid_dim, *cell_to_world,
+            intrinsic, extrinsic, depth, color, trunc, depth_max, counts)
         self.version = next(_VERSIONS)
 
     def insert_keys(self, keys: torch.Tensor) -> None:

@@ -80,19 +80,23 @@ def fuse_frame(
     its tensors, demo/rgbd_fusion.py:216-254; the kernels here read it where it
     is), the host only queues launches, and the reference's capacity warning
     comes with the next call that reads the table's counters."""
-    if not count_blocks and points.shape[0] > 0 and points.dtype == torch.float32:
+    if points.shape[0] > 0 and points.dtype == torch.float32:
         affine = grid._world_to_cell_affine(points)
         if affine is not None:
-            # three launches: the transform is applied inside the activation
-            # kernels, which flag the touched rows; the integration goes by the
-            # flags and takes them down
-            lo, hi = grid._block_bounds()
-            table = grid.engine.backend
-            table.activate_positions(points, affine[0], affine[1], grid.grid_dim, dilation, True,
-                                     lo, hi)
-            integrate_depth(grid, None, None, depth, intrinsic, extrinsic, trunc, depth_max,
-                            color, flagged_by=table)
-            return None
+            # the transform is applied inside the activation kernel, which flags
+            # the touched rows; the integration goes by the flags and takes them
+            # down, and counts them when asked to
+            engine = grid.engine
+            table = engine.backend
+            dropped_before = engine._dropped()
+            table.fuse_frame(points, *affine, dilation, True, grid._block_bounds(),
+                             grid.embeddings.data, grid.grid_dim, grid._cell_to_world_affine(),
+                             intrinsic, extrinsic, depth, color, trunc, depth_max, count_blocks)
+            if not count_blocks:
+                return None
+            touched = table.counters()["touched"]
+            engine._warn_if_overfull(points.shape[0], dropped_before)
+            return int(touched)
     if not count_blocks and points.shape[0] > 0 and grid.engine.capacity <= COLLECT_MAX_BLOCKS:
         cells = grid.transform_world_to_cell(points)
         if cells.dtype == torch.float32:

@@ -21,7 +21,7 @@ namespace ash {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kFlaggedGroups = 8192;    // workgroups of the integration that goes by flags
+constexpr int kFlaggedGroups = ASH_FLAGGED_GROUPS;   // of the integration that goes by flags
 
 struct IntegrateArgs {
     float* emb;                // [B, M, E]
@@ -37,6 +37,7 @@ struct IntegrateArgs {
     float cell_size;
     float origin[3];
     int has_origin;
+    const float* origin_dev;   // the origin on the device instead, or nullptr
     float trunc, depth_max;
 };
 
@@ -61,7 +62,9 @@ __device__ __forceinline__ CellObservation observe_cell(const IntegrateArgs& a, 
     for (int d = 0; d < 3; ++d) {
         const int ic = b[d] * g + c[d];
         p[d] = __fmul_rn(static_cast<float>(ic), a.cell_size);
-        if (a.has_origin) p[d] = __fadd_rn(p[d], a.origin[d]);
+        if (a.has_origin) {
+            p[d] = __fadd_rn(p[d], a.origin_dev != nullptr ? a.origin_dev[d] : a.origin[d]);
+        }
     }
     const float* T = a.extrinsic;
     const float* K = a.intrinsic;
@@ -208,14 +211,18 @@ __global__ __launch_bounds__(kBlock) void integrate_depth_counted_kernel(
 // are the low ones as a rule, so every workgroup gets its share of them),
 // kBlock flags per round, lists the flagged ones in LDS, takes the flags down
 // and updates the cells of the listed blocks, whose coordinates stand in
-// coords[row].  a.grid_idx is not used; a.n is the number of rows.
+// coords[row].  a.grid_idx is not used; a.n is the number of rows.  `counts`
+// (one word per workgroup, or null): how many flagged rows the workgroup met --
+// a plain store each; additions to one counter would serialise (7 ns each) and
+// outlast the integration.
 template <int G, int E>
 __global__ __launch_bounds__(kBlock) void integrate_depth_flagged_kernel(
-        IntegrateArgs a, uint8_t* __restrict__ touched) {
+        IntegrateArgs a, uint8_t* __restrict__ touched, int32_t* __restrict__ counts) {
     __shared__ int32_t s_rows[kBlock * 4];   // row and block coordinates of the flagged ones
     __shared__ int s_n;
     const int m = G > 0 ? G * G * G : a.m;
     const int64_t stride = gridDim.x;
+    int met = 0;
     for (int64_t first = blockIdx.x; first < a.n; first += stride * kBlock) {
         if (threadIdx.x == 0) s_n = 0;
         __syncthreads();
@@ -237,6 +244,7 @@ __global__ __launch_bounds__(kBlock) void integrate_depth_flagged_kernel(
         }
         __syncthreads();
         const int listed = s_n;
+        met += listed;
         for (int j = 0; j < listed; ++j) {
             const int32_t r = s_rows[j * 4 + 0];
             const int bx = s_rows[j * 4 + 1];
@@ -277,6 +285,7 @@ __global__ __launch_bounds__(kBlock) void integrate_depth_flagged_kernel(
         }
         __syncthreads();   // s_rows and s_n are rewritten by the next round
     }
+    if (counts != nullptr && threadIdx.x == 0) counts[blockIdx.x] = met;
 }
 
 }  // namespace
@@ -319,10 +328,33 @@ int fill_integrate_args(IntegrateArgs& a, float* embeddings, int64_t num_embeddi
     a.w = width;
     a.cell_size = cell_size;
     a.has_origin = origin != nullptr;
+    a.origin_dev = nullptr;
     for (int d = 0; d < 3; ++d) a.origin[d] = origin ? origin[d] : 0.f;
     a.trunc = trunc;
     a.depth_max = depth_max;
     if (n_blocks * a.m > (int64_t{1} << 40)) ASH_FAIL("too many cells in one call");
+    return 0;
+}
+
+// Rows are dealt out round robin: enough workgroups to fill the device, few
+// enough that each looks at its flags in one round as a rule.
+unsigned flagged_groups(const ash_map* map) {
+    const int64_t groups = map->capacity < kFlaggedGroups ? map->capacity : kFlaggedGroups;
+    return groups < 1 ? 1u : static_cast<unsigned>(groups);
+}
+
+int launch_flagged(const ash_map* map, IntegrateArgs a, uint8_t* touched, int32_t* counts,
+                   hipStream_t s) {
+    const unsigned groups = flagged_groups(map);
+    a.grid_idx = nullptr;
+    if (a.g == 8 && a.e == 2) {
+        integrate_depth_flagged_kernel<8, 2><<<groups, kBlock, 0, s>>>(a, touched, counts);
+    } else if (a.g == 8 && a.e == 5) {
+        integrate_depth_flagged_kernel<8, 5><<<groups, kBlock, 0, s>>>(a, touched, counts);
+    } else {
+        integrate_depth_flagged_kernel<0, 0><<<groups, kBlock, 0, s>>>(a, touched, counts);
+    }
+    ASH_LAUNCH_CHECK();
     return 0;
 }
 
@@ -380,25 +412,42 @@ extern "C" int ash_grid_integrate_depth_flagged(
                             trunc, depth_max)) {
         return 1;
     }
-    a.grid_idx = nullptr;
     DeviceGuard guard;
     ASH_HIP(guard.enter(map->device));
-    // rows are dealt out round robin: enough workgroups to fill the device,
-    // few enough that each looks at its flags in one round as a rule
-    int64_t groups = map->capacity < kFlaggedGroups ? map->capacity : kFlaggedGroups;
-    if (groups < 1) groups = 1;
-    if (a.g == 8 && a.e == 2) {
-        integrate_depth_flagged_kernel<8, 2><<<static_cast<unsigned>(groups), kBlock, 0,
-                                               static_cast<hipStream_t>(stream)>>>(a, touched);
-    } else if (a.g == 8 && a.e == 5) {
-        integrate_depth_flagged_kernel<8, 5><<<static_cast<unsigned>(groups), kBlock, 0,
-                                               static_cast<hipStream_t>(stream)>>>(a, touched);
-    } else {
-        integrate_depth_flagged_kernel<0, 0><<<static_cast<unsigned>(groups), kBlock, 0,
-                                               static_cast<hipStream_t>(stream)>>>(a, touched);
+    return launch_flagged(map, a, touched, nullptr, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int ash_grid_fuse_frame(
+        ash_map_t* map, const float* positions, int64_t n, const float* origin, float cell_size,
+        int dilation, int bidirectional, int bound_lo, int bound_hi, uint8_t* touched,
+        int32_t* coords, float* embeddings, int64_t num_embeddings, int grid_dim,
+        int embedding_dim, float cell_to_world, const float* world_origin,
+        const float* intrinsic, const float* extrinsic, const float* depth, const float* color,
+        int height, int width, float trunc, float depth_max, int32_t* group_counts,
+        void* stream) {
+    if (map == nullptr) ASH_FAIL("null map handle");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    IntegrateArgs a;
+    if (fill_integrate_args(a, embeddings, num_embeddings, grid_dim, embedding_dim,
+                            reinterpret_cast<const int64_t*>(touched), coords, map->capacity,
+                            cell_to_world, world_origin != nullptr ? a.origin : nullptr, intrinsic,
+                            extrinsic, depth, color, height, width, trunc, depth_max)) {
+        return 1;
     }
-    ASH_LAUNCH_CHECK();
-    return 0;
+    a.origin_dev = world_origin;
+    if (group_counts != nullptr && is_capturing(s)) {
+        ASH_FAIL("the table's counters cannot be read while the stream is being captured");
+    }
+    if (ash_grid_activate_positions(map, positions, n, origin, cell_size, grid_dim, dilation,
+                                    bidirectional, bound_lo, bound_hi, touched, coords, stream)) {
+        return 1;
+    }
+    DeviceGuard guard;
+    ASH_HIP(guard.enter(map->device));
+    if (launch_flagged(map, a, touched, group_counts, s)) return 1;
+    return group_counts == nullptr
+                   ? 0
+                   : queue_touched_count(map, group_counts, static_cast<int>(flagged_groups(map)), s);
 }
 
 extern "C" int ash_grid_integrate_depth(

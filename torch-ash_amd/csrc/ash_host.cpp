@@ -39,6 +39,8 @@ namespace py = pybind11;
     X(ash_map_erase_auto)                                                             \
     X(ash_map_items)                                                                  \
     X(ash_map_counters)                                                               \
+    X(ash_map_upkeep)                                                                 \
+    X(ash_grid_fuse_frame)                                                            \
     X(ash_grid_query)                                                                 \
     X(ash_grid_forward)                                                               \
     X(ash_query_forward)                                                              \
@@ -388,6 +390,62 @@ Tensor table_of(const Tensor& t, int64_t rows, int64_t device, const char* name)
 
 using Optional = std::optional<Tensor>;
 
+// `t` on the device as contiguous float32
+Tensor floats_on(const Tensor& t, int64_t device) {
+    return t.to(at::Device(at::kCUDA, static_cast<c10::DeviceIndex>(device)), at::kFloat).contiguous();
+}
+
+void fuse_frame(uintptr_t handle, int64_t device, const Tensor& positions_in, const Optional& origin,
+                double cell_size, int dilation, bool bidirectional, int bound_lo, int bound_hi,
+                const Tensor& touched, const Tensor& coords, const Tensor& emb, int grid_dim,
+                double cell_to_world, const Optional& world_origin, const Tensor& intrinsic_in,
+                const Tensor& extrinsic_in, const Tensor& depth_in, const Optional& color_in,
+                double trunc, double depth_max, const Optional& counts) {
+    const Tensor x = positions_of(positions_in);
+    need(x.is_cuda() && x.get_device() == device, "positions must be on the map's device");
+    need(emb.is_cuda() && emb.get_device() == device && emb.scalar_type() == at::kFloat &&
+                 emb.is_contiguous(),
+         "embeddings must be contiguous float32 on the map's device");
+    need(emb.dim() == 3 && emb.size(1) == static_cast<int64_t>(grid_dim) * grid_dim * grid_dim,
+         "embeddings must be (num_embeddings, grid_dim^3, embedding_dim)");
+    need(emb.size(0) >= touched.size(0), "one embedding row per index of the map is needed");
+    const Tensor intrinsic = floats_on(intrinsic_in, device), extrinsic = floats_on(extrinsic_in, device);
+    need(intrinsic.dim() == 2 && intrinsic.size(0) == 3 && intrinsic.size(1) == 3 &&
+                 extrinsic.dim() == 2 && extrinsic.size(0) == 4 && extrinsic.size(1) == 4,
+         "intrinsic must be 3x3 and extrinsic 4x4");
+    const Tensor depth = floats_on(depth_in, device);
+    need(depth.dim() == 2, "depth must be (H, W)");
+    Tensor color, from, to;
+    if (color_in.has_value()) {
+        color = floats_on(*color_in, device);
+        need(color.dim() == 3 && color.size(0) == depth.size(0) && color.size(1) == depth.size(1) &&
+                     color.size(2) == 3,
+             "color must be (H, W, 3)");
+    }
+    if (origin.has_value()) from = floats_on(*origin, device);
+    if (world_origin.has_value()) to = floats_on(*world_origin, device);
+    ash_map_t* map = map_of(handle);
+    void* stream = stream_of(device);
+    int64_t scratch_bytes = 0;
+    check(lib.ash_map_insert_scratch_bytes(map, 0, 0, nullptr, ASH_STREAMING_NEVER, &scratch_bytes));
+    const Tensor scratch = scratch_bytes > 0 ? empty({scratch_bytes}, at::kByte, device) : Tensor();
+    int status;
+    {
+        py::gil_scoped_release may_wait;
+        status = lib.ash_map_upkeep(map, x.size(0), ptr<void>(scratch), scratch_bytes, nullptr, stream);
+    }
+    check(status);
+    check(lib.ash_grid_fuse_frame(
+            map, ptr<float>(x), x.size(0), ptr<float>(from), static_cast<float>(cell_size), dilation,
+            bidirectional, bound_lo, bound_hi, ptr<uint8_t>(touched), ptr<int32_t>(coords),
+            ptr<float>(emb), emb.size(0), grid_dim, static_cast<int>(emb.size(2)),
+            static_cast<float>(cell_to_world), ptr<float>(to), ptr<float>(intrinsic),
+            ptr<float>(extrinsic), ptr<float>(depth), ptr<float>(color),
+            static_cast<int>(depth.size(0)), static_cast<int>(depth.size(1)),
+            static_cast<float>(trunc), static_cast<float>(depth_max),
+            counts.has_value() ? ptr<int32_t>(*counts) : nullptr, stream));
+}
+
 // (features, masks, grid_indices, cell_indices, offsets); the last three None
 // unless `need_operands`.
 std::tuple<Tensor, Tensor, Optional, Optional, Optional> grid_forward(
@@ -587,6 +645,7 @@ PYBIND11_MODULE(_ash_host, m) {
     m.def("items", &items);
     m.def("query_cells", &query_cells);
     m.def("grid_forward", &grid_forward);
+    m.def("fuse_frame", &fuse_frame);
     m.def("query_forward", &query_forward);
     m.def("query_backward_forward", &query_backward_forward);
     m.def("query_backward_backward", &query_backward_backward);

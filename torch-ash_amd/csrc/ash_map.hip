@@ -1391,6 +1391,39 @@ __global__ void publish_counters_kernel(const int32_t* __restrict__ ctr, int32_t
     }
 }
 
+// The same with the touched blocks added up first (one workgroup).
+__global__ __launch_bounds__(kBlock) void publish_touched_kernel(int32_t* __restrict__ ctr,
+                                                                 const int32_t* __restrict__ counts,
+                                                                 int n, int32_t* landing,
+                                                                 int32_t stamp) {
+    __shared__ int s_wave[kBlock / 64];
+    int sum = 0;
+    if (n == kBlock * 4 * (n / (kBlock * 4))) {
+        for (int i = threadIdx.x * 4; i < n; i += kBlock * 4) {
+            const int4 c = *reinterpret_cast<const int4*>(counts + i);
+            sum += c.x + c.y + c.z + c.w;
+        }
+    } else {
+        for (int i = threadIdx.x; i < n; i += kBlock) sum += counts[i];
+    }
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) sum += __shfl_xor(sum, d);
+    if ((threadIdx.x & 63) == 0) s_wave[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    int total = 0;
+#pragma unroll
+    for (int w = 0; w < kBlock / 64; ++w) total += s_wave[w];
+    if (threadIdx.x < kHostCounters) {
+        const int32_t v = threadIdx.x == kCtrTouched ? total : ctr[threadIdx.x];
+        if (threadIdx.x == kCtrTouched) ctr[kCtrTouched] = total;
+        __hip_atomic_store(landing + threadIdx.x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(landing + kLandingStamp, stamp, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 __global__ void set_counter_kernel(int32_t* ctr, int which, int32_t value) {
     if (threadIdx.x == 0 && blockIdx.x == 0) ctr[which] = value;
 }
@@ -2913,6 +2946,21 @@ int upkeep(ash_map* map, int64_t incoming, void* scratch, int64_t scratch_bytes,
 }
 
 }  // namespace
+
+}  // extern "C"
+
+int ash::queue_touched_count(ash_map* map, const int32_t* counts, int n, hipStream_t s) {
+    if (take_line(map) || settle_landing_place(map)) return 1;
+    map->late_stamp = ++map->stamp;
+    publish_touched_kernel<<<1, kBlock, 0, s>>>(map->d.ctr, counts, n, map->line + kLineLate,
+                                                map->late_stamp);
+    ASH_LAUNCH_CHECK();
+    map->counters_known = false;
+    map->late_in_flight = map->late_pending = true;
+    return 0;
+}
+
+extern "C" {
 
 int ash_map_set_staging(ash_map_t* map, int32_t* staging) {
     (void)staging;

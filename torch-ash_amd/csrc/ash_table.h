@@ -162,6 +162,9 @@ inline bool heap_in_order(const ash_map* map) { return !map->heap_dirty && !map-
 // false for one that took entries away.
 // `s`: the stream the call runs on (captured: see ash_map::replayed).
 void counters_changed(ash_map* map, bool inserted, hipStream_t s);
+// Adds up `n` words of `counts` into the counter of touched blocks and queues the
+// read-back of the counters behind the stream's work (ash_map.hip).
+int queue_touched_count(ash_map* map, const int32_t* counts, int n, hipStream_t s);
 // The streaming insert (ash_bulk.hip); `early`: page-locked words (or null) where
 // its first pass leaves the number of keys that it hands to the per-key kernel,
 // and behind it, at kLandingStamp, `stamp`.

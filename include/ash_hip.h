@@ -296,6 +296,39 @@ int ash_ray_sample_compact(const int64_t* counts, const int64_t* prefix, const f
                            int64_t stride, int64_t n, int64_t* ray_indices, float* t_nears,
                            float* t_fars, void* stream);
 
+/* The two functions on rays in world units, as SparseDenseGrid calls them
+ * (ash/grid.py:322-403): cell units are (x - origin) / cell_size with origin
+ * float32[3] on the device or NULL, results come back in world units, and the
+ * transforms of origins, box, ranges and results happen inside the kernels, in
+ * the order and rounding of the elementwise expressions they replace.  t_min and
+ * t_max in cell units.
+ * ray_sample: the march keeps its samples in `stage` (n * stride pairs, as
+ * ash_ray_sample_staged) and returns, having waited for it, the number of
+ * samples in out[0] and the largest count of a ray in out[1].  If that is at most
+ * `stride`, ash_ray_sample_place writes ray_indices (int64), t_nears and t_fars
+ * (out[0] entries each) and prefix (int64[n], running sums of the counts);
+ * otherwise the march has to be run again by ash_ray_sample.  ray_nears /
+ * ray_fars: n values in world units, or NULL for near_for_all / far_for_all
+ * (cell units) on every ray.  counts: int64[n]; groups: 2 *
+ * ash_ray_sample_groups(n) int64 on the device. */
+int ash_ray_find_near_far_world(ash_map_t* map, const float* ray_origins,
+                                const float* ray_directions, const float* origin,
+                                float cell_size, const float* bbox_min,
+                                const float* bbox_max, int64_t n, float t_min,
+                                float t_max, float grid2cell_multiplier,
+                                float* ray_nears, float* ray_fars, void* stream);
+int64_t ash_ray_sample_groups(int64_t n);
+int ash_ray_sample_march(ash_map_t* map, const float* ray_origins,
+                         const float* ray_directions, const float* origin,
+                         float cell_size, const float* ray_nears, const float* ray_fars,
+                         float near_for_all, float far_for_all, int64_t n,
+                         int64_t max_samples_per_ray, float grid2cell_multiplier,
+                         int64_t* counts, int64_t* groups, float* stage, int64_t stride,
+                         int64_t out[2], void* stream);
+int ash_ray_sample_place(const int64_t* counts, const int64_t* groups, const float* stage,
+                         int64_t stride, int64_t n, float cell_size, int64_t* ray_indices,
+                         float* t_nears, float* t_fars, int64_t* prefix, void* stream);
+
 /* Replaces `HashMap::insert_keys` (ash/src/hashmap_gpu.cuh:211-247).  New keys
  * pop one index each from the heap; duplicates (in the table or within the
  * batch) are ignored.  Keys beyond `capacity` are dropped and counted

@@ -134,6 +134,19 @@ _SIGNATURES = {
         [_PTR] * 5 + [_I64, _I64, ctypes.c_float, _PTR, _PTR, _I64, _PTR],
     ),
     "ash_ray_sample_compact": (ctypes.c_int, [_PTR] * 3 + [_I64, _I64] + [_PTR] * 4),
+    "ash_ray_find_near_far_world": (
+        ctypes.c_int,
+        [_PTR] * 4 + [ctypes.c_float, _PTR, _PTR, _I64] + [ctypes.c_float] * 3 + [_PTR] * 3,
+    ),
+    "ash_ray_sample_groups": (_I64, [_I64]),
+    "ash_ray_sample_march": (
+        ctypes.c_int,
+        [_PTR] * 4 + [ctypes.c_float, _PTR, _PTR, ctypes.c_float, ctypes.c_float, _I64, _I64,
+                      ctypes.c_float, _PTR, _PTR, _PTR, _I64, ctypes.POINTER(_I64), _PTR],
+    ),
+    "ash_ray_sample_place": (
+        ctypes.c_int, [_PTR] * 3 + [_I64, _I64, ctypes.c_float] + [_PTR] * 5,
+    ),
     "ash_map_insert_keys": (ctypes.c_int, [_PTR, _PTR, _I64, _PTR]),
     "ash_map_insert_needs_scratch": (ctypes.c_int, [ctypes.c_int, ctypes.POINTER(_I64)]),
     "ash_map_insert": (
@@ -540,6 +553,30 @@ class _Backend:
                 )
             )
         return nears, fars
+
+    def ray_find_near_far_world(
+        self, hashmap, ray_origins, ray_directions, origin, cell_size, bbox_min, bbox_max, t_min,
+        t_max, grid2cell_multiplier,
+    ) -> Tuple[torch.Tensor, torch.Tensor]:
+        """ray_find_near_far of world rays with cell units = (x - origin) /
+        cell_size: the transforms of rays, box and results in the same launch
+        (t_min and t_max in cell units)."""
+        return self.host.ray_near_far(hashmap._address, hashmap._index, ray_origins, ray_directions,
+                                      origin, cell_size, bbox_min, bbox_max, t_min, t_max,
+                                      grid2cell_multiplier)
+
+    def ray_sample_world(
+        self, hashmap, ray_origins, ray_directions, origin, cell_size, ray_nears, ray_fars,
+        max_samples_per_ray, grid2cell_multiplier,
+    ):
+        """ray_sample of world rays, everything in world units; None where the
+        samples do not fit a staging area (`ray_sample` takes such rays)."""
+        stride = max(1, int(max_samples_per_ray) + RAY_STAGE_EXTRA)
+        if ray_origins.shape[0] * stride > RAY_STAGE_LIMIT:
+            return None
+        return self.host.ray_sample(hashmap._address, hashmap._index, ray_origins, ray_directions,
+                                    origin, cell_size, ray_nears, ray_fars, int(max_samples_per_ray),
+                                    grid2cell_multiplier, stride)
 
     def ray_sample(
         self, hashmap, ray_origins, ray_directions, ray_nears, ray_fars, bbox_min, bbox_max,

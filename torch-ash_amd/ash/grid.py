@@ -482,6 +482,16 @@ class SparseDenseGrid(ASHModule):
         the inclusive prefix sum of the per-ray sample counts (N,).  Sample
         positions are rays_o[ray_indices] + (t_near + t_far) / 2 *
         rays_d[ray_indices]."""
+        affine = self._world_to_cell_affine(rays_o)
+        if affine is not None and hasattr(backend, "ray_sample_world") and all(
+            not torch.is_tensor(r) or r.dtype == torch.float32 for r in (rays_o, rays_d, rays_near, rays_far)
+        ):
+            # transforms, march, running sums and results in three launches
+            samples = backend.ray_sample_world(
+                self.engine.backend, rays_o, rays_d, *affine, rays_near, rays_far,
+                max_samples_per_ray, float(self.grid_dim))
+            if samples is not None:
+                return samples
         bbox_min, bbox_max = self.get_bbox()
         ray_indices, t_nears, t_fars, ray_prefix_sum = backend.ray_sample(
             self.engine.backend,
@@ -503,6 +513,13 @@ class SparseDenseGrid(ASHModule):
         """Per-ray range that contains active blocks (ash/grid.py:379-403), in
         world units; near is negative where a ray meets no active block."""
         bbox_min, bbox_max = self.get_bbox()
+        affine = self._world_to_cell_affine(rays_o)
+        if affine is not None and hasattr(backend, "ray_find_near_far_world") and all(
+            r.dtype == torch.float32 for r in (rays_o, rays_d, bbox_min, bbox_max)
+        ):
+            return backend.ray_find_near_far_world(
+                self.engine.backend, rays_o, rays_d, *affine, bbox_min, bbox_max,
+                t_min / self.cell_size, t_max / self.cell_size, float(self.grid_dim))
         ray_nears, ray_fars = backend.ray_find_near_far(
             self.engine.backend,
             self.transform_world_to_cell(rays_o),

@@ -19,7 +19,8 @@ OUT_DIR = os.path.join(HERE, "ash", "lib")
 OUT = os.path.join(OUT_DIR, "libash_hip.so")
 HOST_SOURCE = os.path.join(CSRC, "ash_host.cpp")
 HOST_OUT = os.path.join(OUT_DIR, "_ash_host.so")
-SOURCES = ["ash_map.hip", "ash_bulk.hip", "ash_query.hip", "ash_fusion.hip", "ash_mesh.hip"]
+SOURCES = ["ash_map.hip", "ash_bulk.hip", "ash_query.hip", "ash_fusion.hip", "ash_mesh.hip",
+           "ash_rays.hip"]
 HEADERS = [
     os.path.join(CSRC, "ash_probe.h"),
     os.path.join(CSRC, "ash_dev.h"),

@@ -73,7 +73,14 @@ enum Counter {
     kNumCounters = 64
 };
 constexpr int kHostCounters = 8;
-constexpr int kLandingStamp = 8;   // the word behind the counters in a landing place
+// Page-locked words of a map (take_line) in which kernels leave answers for the
+// host; each place carries its stamp kLandingStamp words behind its start.
+constexpr int kLandingStamp = 8;
+constexpr int kLineWords = 64;
+constexpr int kLineNow = 0;      // counters, fetched and waited for
+constexpr int kLineLate = 16;    // counters, fetched behind a streaming insert or a fusion frame
+constexpr int kLineEarly = 32;   // count left by the first pass of a streaming insert
+constexpr int kLineRays = 48;    // number of samples and largest count of a ray (64 bits each)
 constexpr int64_t kHeaderBytes = 256;
 
 // General region: open addressing over 32-bit state words + 16-byte keys.

@@ -41,6 +41,10 @@ namespace py = pybind11;
     X(ash_map_counters)                                                               \
     X(ash_map_upkeep)                                                                 \
     X(ash_grid_fuse_frame)                                                            \
+    X(ash_ray_find_near_far_world)                                                    \
+    X(ash_ray_sample_groups)                                                          \
+    X(ash_ray_sample_march)                                                           \
+    X(ash_ray_sample_place)                                                           \
     X(ash_grid_query)                                                                 \
     X(ash_grid_forward)                                                               \
     X(ash_query_forward)                                                              \
@@ -379,6 +383,89 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> query_cells(uintptr_t handle, int64_t
     return {grids, cells, offsets, masks};
 }
 
+using Optional = std::optional<Tensor>;
+
+// `t` on the device as contiguous float32
+Tensor floats_on(const Tensor& t, int64_t device) {
+    return t.to(at::Device(at::kCUDA, static_cast<c10::DeviceIndex>(device)), at::kFloat).contiguous();
+}
+
+// ---------------------------------------------------------------------- rays
+struct RayOperands {
+    Tensor o, d, origin;
+    RayOperands(const Tensor& origins, const Tensor& directions, const Optional& from, int64_t device) {
+        o = floats_on(origins, device);
+        d = floats_on(directions, device);
+        need(o.dim() == 2 && o.size(1) == 3 && d.sizes() == o.sizes(),
+             "ray origins and directions must both be (N, 3)");
+        if (from.has_value()) origin = floats_on(*from, device);
+    }
+};
+
+std::tuple<Tensor, Tensor> ray_near_far(uintptr_t handle, int64_t device, const Tensor& origins,
+                                        const Tensor& directions, const Optional& origin,
+                                        double cell_size, const Tensor& bbox_min, const Tensor& bbox_max,
+                                        double t_min, double t_max, double grid2cell) {
+    const RayOperands r(origins, directions, origin, device);
+    const Tensor lo = floats_on(bbox_min, device), hi = floats_on(bbox_max, device);
+    need(lo.numel() == 3 && hi.numel() == 3, "the box has three coordinates per corner");
+    const int64_t n = r.o.size(0);
+    Tensor nears = empty({n}, at::kFloat, device), fars = empty({n}, at::kFloat, device);
+    check(lib.ash_ray_find_near_far_world(
+            map_of(handle), ptr<float>(r.o), ptr<float>(r.d), ptr<float>(r.origin),
+            static_cast<float>(cell_size), ptr<float>(lo), ptr<float>(hi), n, static_cast<float>(t_min),
+            static_cast<float>(t_max), static_cast<float>(grid2cell), ptr<float>(nears),
+            ptr<float>(fars), stream_of(device)));
+    return {nears, fars};
+}
+
+// A range per ray (world units, brought to cell units by the kernel), or one
+// number for all of them, in world units as well.
+struct RayRange {
+    Tensor each;
+    float for_all = 0.f;
+    RayRange(const py::object& range, double cell_size, int64_t n, int64_t device) {
+        if (THPVariable_Check(range.ptr())) {
+            each = floats_on(py::cast<Tensor>(range), device).expand({n}).contiguous();
+        } else {
+            for_all = static_cast<float>(py::cast<double>(range) / cell_size);
+        }
+    }
+};
+
+// (ray_indices, t_nears, t_fars, prefix), or None where a ray has more samples
+// than `stride`.
+std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> ray_sample(
+        uintptr_t handle, int64_t device, const Tensor& origins, const Tensor& directions,
+        const Optional& origin, double cell_size, const py::object& nears, const py::object& fars,
+        int64_t max_samples, double grid2cell, int64_t stride) {
+    const RayOperands r(origins, directions, origin, device);
+    const int64_t n = r.o.size(0);
+    const RayRange near(nears, cell_size, n, device), far(fars, cell_size, n, device);
+    const Tensor counts = empty({n}, at::kLong, device), prefix = empty({n}, at::kLong, device);
+    const Tensor groups = empty({lib.ash_ray_sample_groups(n), 2}, at::kLong, device);
+    const Tensor stage = empty({n, stride, 2}, at::kFloat, device);
+    void* stream = stream_of(device);
+    int64_t out[2] = {0, 0};
+    int status;
+    {
+        py::gil_scoped_release waits_for_the_device;
+        status = lib.ash_ray_sample_march(
+                map_of(handle), ptr<float>(r.o), ptr<float>(r.d), ptr<float>(r.origin),
+                static_cast<float>(cell_size), ptr<float>(near.each), ptr<float>(far.each),
+                near.for_all, far.for_all, n, max_samples, static_cast<float>(grid2cell),
+                ptr<int64_t>(counts), ptr<int64_t>(groups), ptr<float>(stage), stride, out, stream);
+    }
+    check(status);
+    if (out[1] > stride) return std::nullopt;
+    Tensor indices = empty({out[0]}, at::kLong, device);
+    Tensor t_nears = empty({out[0]}, at::kFloat, device), t_fars = empty({out[0]}, at::kFloat, device);
+    check(lib.ash_ray_sample_place(ptr<int64_t>(counts), ptr<int64_t>(groups), ptr<float>(stage), stride,
+                                   n, static_cast<float>(cell_size), ptr<int64_t>(indices),
+                                   ptr<float>(t_nears), ptr<float>(t_fars), ptr<int64_t>(prefix), stream));
+    return std::make_tuple(indices, t_nears, t_fars, prefix);
+}
+
 Tensor table_of(const Tensor& t, int64_t rows, int64_t device, const char* name) {
     if (!t.is_cuda() || t.get_device() != device || t.scalar_type() != at::kLong || t.dim() != 2 ||
         t.size(0) != rows || t.size(1) != 8) {
@@ -386,13 +473,6 @@ Tensor table_of(const Tensor& t, int64_t rows, int64_t device, const char* name)
              std::to_string(device));
     }
     return t.contiguous();
-}
-
-using Optional = std::optional<Tensor>;
-
-// `t` on the device as contiguous float32
-Tensor floats_on(const Tensor& t, int64_t device) {
-    return t.to(at::Device(at::kCUDA, static_cast<c10::DeviceIndex>(device)), at::kFloat).contiguous();
 }
 
 void fuse_frame(uintptr_t handle, int64_t device, const Tensor& positions_in, const Optional& origin,
@@ -646,6 +726,8 @@ PYBIND11_MODULE(_ash_host, m) {
     m.def("query_cells", &query_cells);
     m.def("grid_forward", &grid_forward);
     m.def("fuse_frame", &fuse_frame);
+    m.def("ray_near_far", &ray_near_far);
+    m.def("ray_sample", &ray_sample);
     m.def("query_forward", &query_forward);
     m.def("query_backward_forward", &query_backward_forward);
     m.def("query_backward_backward", &query_backward_backward);

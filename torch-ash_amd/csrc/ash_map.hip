@@ -231,66 +231,6 @@ __device__ __forceinline__ bool find_key(const MapDev& m, const int32_t (&k)[DIM
     return found;
 }
 
-// The same look-up when the eight lanes of a group all hold the same key (and
-// the same `active`): the group reads the key's bucket once, 16 bytes per lane,
-// instead of taking turns with eight different keys.
-template <int DIM>
-__device__ __forceinline__ bool find_key_shared(const MapDev& m, const int32_t (&k)[DIM],
-                                                bool active, int32_t& res) {
-    const int lane = threadIdx.x & 63;
-    const int j = lane & (kGroup - 1);
-    const int gbase = lane & ~(kGroup - 1);
-    const bool v0 = (2 * j) < kSlots;
-    const bool v1 = (2 * j + 1) < kSlots;
-    uint64_t code;
-    const bool fits = pack_key<DIM>(k, code);
-    bool pend = active && fits;
-    uint32_t b = bucket_of(code, m.nb);
-    uint32_t steps = 0;
-    res = 0;
-    bool found = false;
-    while (__ballot(pend)) {
-        uint4 line = make_uint4(0u, 0u, 0u, 0u);
-        if (pend) {
-            line = *(reinterpret_cast<const uint4*>(m.buckets +
-                                                    static_cast<size_t>(b) * kBucketQwords) + j);
-        }
-        const uint64_t qa = static_cast<uint64_t>(line.x) | (static_cast<uint64_t>(line.y) << 32);
-        const uint64_t qb = static_cast<uint64_t>(line.z) | (static_cast<uint64_t>(line.w) << 32);
-        const uint32_t gm0 = static_cast<uint32_t>(__ballot(pend && v0 && qa == code) >> gbase) & 0xFFu;
-        const uint32_t gm1 = static_cast<uint32_t>(__ballot(pend && v1 && qb == code) >> gbase) & 0xFFu;
-        const uint32_t ge0 = static_cast<uint32_t>(__ballot(pend && v0 && qa == kEmpty) >> gbase) & 0xFFu;
-        const uint32_t ge1 = static_cast<uint32_t>(__ballot(pend && v1 && qb == kEmpty) >> gbase) & 0xFFu;
-        int slot = -1;
-        if (gm0) {
-            slot = 2 * __builtin_ctz(gm0);
-        } else if (gm1) {
-            slot = 2 * __builtin_ctz(gm1) + 1;
-        }
-        const int t = kValDword0 + (slot < 0 ? 0 : slot);
-        const int comp = t & 3;
-        const uint32_t sel = comp == 0 ? line.x : comp == 1 ? line.y : comp == 2 ? line.z : line.w;
-        const int32_t val = __shfl(static_cast<int>(sel), gbase + (t >> 2));
-        if (pend) {
-            if (slot >= 0) {
-                found = true;
-                res = val;
-                pend = false;
-            } else if (ge0 | ge1) {
-                pend = false;
-            } else {
-                b = next_bucket(b, m.nb);
-                if (++steps >= kPartBuckets) pend = false;
-            }
-        }
-    }
-    if (active && !fits) {
-        uint32_t pos;
-        found = gen_find<DIM>(m, k, res, pos);
-    }
-    return found;
-}
-
 template <int DIM>
 __global__ __launch_bounds__(kBlock) void find_kernel(
         MapDev m, const int32_t* __restrict__ keys, int64_t n,
@@ -853,204 +793,6 @@ __global__ __launch_bounds__(kHeapBlock) void activate_runs_kernel(
             __syncthreads();   // insert_key's own words are rewritten by the next round
         }
     }
-}
-
-// --------------------------------------------------------------------- rays
-// ash/src/sampler.cu:7-67 and :122-214.  Positions are
-// origin + t * direction as a fused multiply-add (what nvcc makes of the
-// reference's expression); everything is in cell units and a block is
-// `grid2cell` cells wide.
-__device__ __forceinline__ void ray_block(const float (&o)[3], const float (&d)[3],
-                                          float t, float cell2grid,
-                                          int32_t (&block)[3], float (&x)[3]) {
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        x[a] = fmaf(t, d[a], o[a]);
-        block[a] = static_cast<int32_t>(floorf(__fmul_rn(x[a], cell2grid)));
-    }
-}
-
-// One wavefront per ray: the march of ray_find_near_far visits the parameters
-// t_0 = t_min, t_{k+1} = t_k + step regardless of what it finds, so lane l of
-// round r takes step 64 r + l (its t by the same chain of additions), the 64
-// lookups go out together, and the near / far recurrence is then replayed over
-// the hits in step order.  The march ends at the first step that is at or
-// beyond t_max or outside the box, exactly where the sequential loop stops.
-__global__ __launch_bounds__(kBlock) void ray_near_far_kernel(
-        MapDev m, const float* __restrict__ origins,
-        const float* __restrict__ directions, const float* __restrict__ bbox_min,
-        const float* __restrict__ bbox_max, int64_t n, float t_min, float t_max,
-        float grid2cell, float* __restrict__ nears, float* __restrict__ fars) {
-    const int lane = threadIdx.x & 63;
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * (kBlock / 64) + (threadIdx.x >> 6);
-    if (i >= n) return;  // whole wavefronts leave together
-    const float cell2grid = static_cast<float>(1.0 / grid2cell);
-    const float t_grid_step = static_cast<float>(grid2cell * 0.5);
-    float o[3], d[3], lo[3], hi[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        o[a] = origins[i * 3 + a];
-        d[a] = directions[i * 3 + a];
-        lo[a] = bbox_min[a];
-        hi[a] = bbox_max[a];
-    }
-    float t = t_min;
-    for (int j = 0; j < 63; ++j) {
-        if (j < lane) t += t_grid_step;
-    }
-    float near = -1.f, far = t_max;
-    for (;;) {
-        int32_t block[3];
-        float x[3];
-        ray_block(o, d, t, cell2grid, block, x);
-        bool go = t < t_max;
-#pragma unroll
-        for (int a = 0; a < 3; ++a) go = go && x[a] >= lo[a] && x[a] <= hi[a];
-        const uint64_t stop = __ballot(!go);
-        const int first_stop = stop ? __builtin_ctzll(stop) : 64;
-        const bool active = lane < first_stop;
-        // steps are half a block apart, so neighbouring lanes often stand in
-        // the same block: only the first lane of such a run goes to the table,
-        // the others take its answer
-        bool head = true;
-        {
-            int same = lane > 0;
-#pragma unroll
-            for (int a = 0; a < 3; ++a) same &= __shfl_up(block[a], 1) == block[a];
-            head = !same;
-        }
-        int32_t idx;
-        const bool asked = find_key_alone<3>(m, block, active && head, idx);
-        const uint64_t heads = __ballot(head);
-        const int my_head = 63 - __builtin_clzll(heads & (~0ull >> (63 - lane)));
-        const bool found = __shfl(static_cast<int>(asked), my_head) != 0;
-        uint64_t hits = __ballot(found && active);
-        while (hits) {
-            const int l = __builtin_ctzll(hits);
-            const float t_hit = __shfl(t, l);
-            near = near < 0.f ? t_hit : fmaxf(near - t_grid_step, t_min);
-            far = fminf(t_hit + t_grid_step, t_max);
-            hits &= hits - 1;
-        }
-        if (first_stop < 64) break;
-        for (int j = 0; j < 64; ++j) t += t_grid_step;
-    }
-    if (lane == 0) {
-        nears[i] = near;
-        fars[i] = far;
-    }
-}
-
-// counts != nullptr: allocation pass; otherwise the assignment pass, which
-// writes the samples of ray i at prefix[i - 1] .. prefix[i].  An allocation
-// pass with `stage` also keeps the first `stride` samples of ray i as pairs
-// (t_near, t_far) at stage[2 * (i * stride + k)], so that the assignment pass
-// can be a copy instead of a second march.
-// LPR lanes per ray: 1 (every lane looks its block up by itself,
-// find_key_alone), or 8 lanes that march the same ray in step and share every
-// look-up (find_key_shared) -- eight times the wavefronts for the same rays,
-// which is what hides the latency of a march that is one dependent look-up
-// after the other when the rays are few.
-template <int LPR>
-__global__ __launch_bounds__(kBlock) void ray_sample_kernel(
-        MapDev m, const float* __restrict__ origins,
-        const float* __restrict__ directions, const float* __restrict__ ray_nears,
-        const float* __restrict__ ray_fars, int64_t n, float max_samples,
-        float grid2cell, int64_t* __restrict__ counts,
-        const int64_t* __restrict__ prefix, int64_t* __restrict__ ray_indices,
-        float* __restrict__ t_nears, float* __restrict__ t_fars,
-        float2* __restrict__ stage, int64_t stride) {
-    const int64_t gid = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-    const int64_t i = gid / LPR;
-    const bool writer = gid % LPR == 0;   // the lane of a ray that stores its results
-    const bool active = i < n;
-    const float cell2grid = static_cast<float>(1.0 / grid2cell);
-    float o[3], d[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        o[a] = active ? origins[i * 3 + a] : 0.f;
-        d[a] = active ? directions[i * 3 + a] : 0.f;
-    }
-    const float ray_near = active ? ray_nears[i] : 0.f;
-    const float ray_far = active ? ray_fars[i] : 0.f;
-    const float t_step = fmaxf(0.7f, __fdiv_rn(ray_far - ray_near, max_samples));
-    const float t_grid_step = __fmul_rn(t_step, grid2cell);
-    const int64_t start = (counts == nullptr && active && i > 0) ? prefix[i - 1] : 0;
-    float t = ray_near, t_near = ray_near;
-    int64_t local = 0;
-    bool live = active && t < ray_far;
-    // One step of the march, given whether the block under t is stored.
-    auto step = [&](bool found) {
-        const float before = t;
-        if (!found) {
-            t += t_grid_step;
-        } else {
-            t += t_step;
-            if (!writer) {
-            } else if (counts == nullptr) {
-                ray_indices[start + local] = i;
-                t_nears[start + local] = t_near;
-                t_fars[start + local] = t;
-            } else if (stage != nullptr && local < stride) {
-                stage[i * stride + local] = make_float2(t_near, t);
-            }
-            t_near = t;
-            ++local;
-        }
-        // a step that no longer advances t (range far beyond fp32
-        // resolution) would never end; the reference has no such guard
-        live = t < ray_far && t > before;
-    };
-    // The reference looks the block under t up at every step.  Samples are a
-    // fraction of a block apart, so consecutive steps mostly ask for the same
-    // block: a lane answers those from its last look-up and the wavefront goes
-    // to the table only when some lane has entered another block -- a dozen
-    // round trips to memory per ray instead of one per step, same answers.
-    int32_t known[3] = {0, 0, 0};
-    bool have = false;
-    bool known_found = false;
-    while (__ballot(live)) {
-        int32_t block[3] = {0, 0, 0};
-        float x[3];
-        bool ask = false;
-        while (live) {
-            ray_block(o, d, t, cell2grid, block, x);
-            if (!have || block[0] != known[0] || block[1] != known[1] || block[2] != known[2]) {
-                ask = true;
-                break;
-            }
-            step(known_found);
-        }
-        int32_t idx;
-        const bool found = LPR == 8 ? find_key_shared<3>(m, block, live && ask, idx)
-                                    : find_key_alone<3>(m, block, live && ask, idx);
-        if (live && ask) {
-#pragma unroll
-            for (int a = 0; a < 3; ++a) known[a] = block[a];
-            known_found = found;
-            have = true;
-            step(found);
-        }
-    }
-    if (active && writer && counts != nullptr) counts[i] = local;
-}
-
-// Assignment pass from the staged samples: one thread per staged slot.
-__global__ __launch_bounds__(kBlock) void ray_compact_kernel(
-        const int64_t* __restrict__ counts, const int64_t* __restrict__ prefix,
-        const float2* __restrict__ stage, int64_t stride, int64_t n,
-        int64_t* __restrict__ ray_indices, float* __restrict__ t_nears,
-        float* __restrict__ t_fars) {
-    const int64_t slot = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-    if (slot >= n * stride) return;
-    const int64_t i = slot / stride;
-    const int64_t k = slot - i * stride;
-    if (k >= counts[i]) return;
-    const int64_t out = (i > 0 ? prefix[i - 1] : 0) + k;
-    const float2 s = stage[slot];
-    ray_indices[out] = i;
-    t_nears[out] = s.x;
-    t_fars[out] = s.y;
 }
 
 // Workgroup size of erase: the heap counter and the tombstone counter are each
@@ -1823,108 +1565,8 @@ inline unsigned looping_grid(int64_t n) {
     return static_cast<unsigned>(g);
 }
 
-// Few rays cannot fill the device with one lane each; below this many they
-// march with eight lanes per ray (32 768 rays: 110 against 120 us; from 65 536
-// rays on one lane per ray is the faster one, 1.6x at half a million).
-constexpr int64_t kRaysPerLaneMin = int64_t{1} << 16;
-
-int launch_ray_sample(ash_map_t* map, const float* origins, const float* directions,
-                      const float* nears, const float* fars, int64_t n, float max_samples,
-                      float grid2cell, int64_t* counts, const int64_t* prefix,
-                      int64_t* ray_indices, float* t_nears, float* t_fars, float2* stage,
-                      int64_t stride, hipStream_t s) {
-    if (n < kRaysPerLaneMin) {
-        ray_sample_kernel<8><<<grid_for(n * 8), kBlock, 0, s>>>(
-                map->d, origins, directions, nears, fars, n, max_samples, grid2cell, counts,
-                prefix, ray_indices, t_nears, t_fars, stage, stride);
-    } else {
-        ray_sample_kernel<1><<<grid_for(n), kBlock, 0, s>>>(
-                map->d, origins, directions, nears, fars, n, max_samples, grid2cell, counts,
-                prefix, ray_indices, t_nears, t_fars, stage, stride);
-    }
-    return 0;
-}
-
-
 int check_map(const ash_map* map) {
     if (map == nullptr) ASH_FAIL("null map handle");
-    return 0;
-}
-
-// ------------------------------------------- words that the device leaves here
-// What the host wants to know of a running call (the counters, how many keys the
-// first pass of a streaming insert could not place) is written by kernels into
-// page-locked host memory, stamped with a number of the call's own, and the host
-// polls the stamp: no copy on the stream, no event, and the answer is seen about
-// a microsecond after it was written, where a copy and a stream synchronisation
-// took 12-15 us of an idle device's time.
-//
-// Every map that asks gets a line of kLineWords of its own from a pool for all
-// maps (its slabs serve the maps of the process, as many lines as maps that ever
-// lived at the same time) and gives it back when it is destroyed.
-constexpr int kLineWords = 64;
-constexpr int kLineNow = 0;      // counters, fetched and waited for
-constexpr int kLineLate = 16;    // counters, fetched behind a streaming insert
-constexpr int kLineEarly = 32;   // count left by the first pass of a streaming insert
-constexpr int kLinesPerSlab = 64;
-
-std::mutex g_lines_mutex;
-std::vector<int32_t*>& free_lines() {
-    static auto* lines = new std::vector<int32_t*>;   // (outlives maps destroyed at exit)
-    return *lines;
-}
-
-int take_line(ash_map* map) {
-    if (map->line != nullptr) return 0;
-    std::lock_guard<std::mutex> lock(g_lines_mutex);
-    std::vector<int32_t*>& lines = free_lines();
-    if (lines.empty()) {
-        void* slab = nullptr;
-        ASH_HIP(hipHostMalloc(&slab, kLinesPerSlab * kLineWords * sizeof(int32_t),
-                              hipHostMallocPortable | hipHostMallocCoherent));
-        memset(slab, 0, kLinesPerSlab * kLineWords * sizeof(int32_t));
-        for (int i = 0; i < kLinesPerSlab; ++i) {
-            lines.push_back(static_cast<int32_t*>(slab) + i * kLineWords);
-        }
-    }
-    map->line = lines.back();
-    lines.pop_back();
-    // stamps of this map start where the line's last owner stopped
-    for (int at : {kLineNow, kLineLate, kLineEarly}) {
-        map->stamp = std::max(map->stamp, map->line[at + kLandingStamp]);
-    }
-    return 0;
-}
-
-void give_back_line(ash_map* map) {
-    if (map->line == nullptr) return;
-    std::lock_guard<std::mutex> lock(g_lines_mutex);
-    free_lines().push_back(map->line);
-    map->line = nullptr;
-}
-
-// Waits until the device has written `stamp`.  The wait ends with the device's
-// work at the latest: every few milliseconds without an answer the device is
-// synchronised (errors show there), after which the word has to be there.
-int wait_for_stamp(const int32_t* word, int32_t stamp) {
-    const auto arrived = [&] { return __atomic_load_n(word, __ATOMIC_ACQUIRE) == stamp; };
-    for (int64_t spin = 0; spin < 4'000'000; ++spin) {
-        if (arrived()) return 0;
-        __builtin_ia32_pause();
-        if (spin > 20'000) sched_yield();
-    }
-    ASH_HIP(hipDeviceSynchronize());
-    if (!arrived()) ASH_FAIL("internal error: the device has not left its counters");
-    return 0;
-}
-
-// A read-back queued behind an insert that may still be under way has to arrive
-// before its words are read or written again.
-int settle_landing_place(ash_map* map) {
-    if (map->late_in_flight) {
-        if (wait_for_stamp(map->line + kLineLate + kLandingStamp, map->late_stamp)) return 1;
-        map->late_in_flight = false;
-    }
     return 0;
 }
 
@@ -1992,6 +1634,87 @@ int clear_table(ash_map* map, hipStream_t s, bool write_heap, int32_t size, bool
 }
 
 }  // namespace
+
+// ------------------------------------------- words that the device leaves here
+// What the host wants to know of a running call (the counters, how many keys the
+// first pass of a streaming insert could not place) is written by kernels into
+// page-locked host memory, stamped with a number of the call's own, and the host
+// polls the stamp: no copy on the stream, no event, and the answer is seen about
+// a microsecond after it was written, where a copy and a stream synchronisation
+// took 12-15 us of an idle device's time.
+//
+// Every map that asks gets a line of kLineWords of its own from a pool for all
+// maps (its slabs serve the maps of the process, as many lines as maps that ever
+// lived at the same time) and gives it back when it is destroyed.
+namespace {
+
+constexpr int kLinesPerSlab = 64;
+
+std::mutex g_lines_mutex;
+std::vector<int32_t*>& free_lines() {
+    static auto* lines = new std::vector<int32_t*>;   // (outlives maps destroyed at exit)
+    return *lines;
+}
+
+}  // namespace
+
+int take_line(ash_map* map) {
+    if (map->line != nullptr) return 0;
+    std::lock_guard<std::mutex> lock(g_lines_mutex);
+    std::vector<int32_t*>& lines = free_lines();
+    if (lines.empty()) {
+        void* slab = nullptr;
+        ASH_HIP(hipHostMalloc(&slab, kLinesPerSlab * kLineWords * sizeof(int32_t),
+                              hipHostMallocPortable | hipHostMallocCoherent));
+        memset(slab, 0, kLinesPerSlab * kLineWords * sizeof(int32_t));
+        for (int i = 0; i < kLinesPerSlab; ++i) {
+            lines.push_back(static_cast<int32_t*>(slab) + i * kLineWords);
+        }
+    }
+    map->line = lines.back();
+    lines.pop_back();
+    // stamps of this map start where the line's last owner stopped
+    for (int at : {kLineNow, kLineLate, kLineEarly, kLineRays}) {
+        map->stamp = std::max(map->stamp, map->line[at + kLandingStamp]);
+    }
+    return 0;
+}
+
+namespace {
+
+void give_back_line(ash_map* map) {
+    if (map->line == nullptr) return;
+    std::lock_guard<std::mutex> lock(g_lines_mutex);
+    free_lines().push_back(map->line);
+    map->line = nullptr;
+}
+
+}  // namespace
+
+// Waits until the device has written `stamp`.  The wait ends with the device's
+// work at the latest: after some seconds without an answer the device is
+// synchronised (errors show there), after which the word has to be there.
+int wait_for_stamp(const int32_t* word, int32_t stamp) {
+    const auto arrived = [&] { return __atomic_load_n(word, __ATOMIC_ACQUIRE) == stamp; };
+    for (int64_t spin = 0; spin < 4'000'000; ++spin) {
+        if (arrived()) return 0;
+        __builtin_ia32_pause();
+        if (spin > 20'000) sched_yield();
+    }
+    ASH_HIP(hipDeviceSynchronize());
+    if (!arrived()) ASH_FAIL("internal error: the device has not left its counters");
+    return 0;
+}
+
+// A read-back queued behind an insert that may still be under way has to arrive
+// before its words are read or written again.
+int settle_landing_place(ash_map* map) {
+    if (map->late_in_flight) {
+        if (wait_for_stamp(map->line + kLineLate + kLandingStamp, map->late_stamp)) return 1;
+        map->late_in_flight = false;
+    }
+    return 0;
+}
 
 int give_up_heap_order(ash_map* map, hipStream_t s) {
     if (map->heap_dirty) return 0;
@@ -2528,120 +2251,6 @@ int ash_grid_activate_positions(ash_map_t* map, const float* positions, int64_t 
     if (groups > 0x7FFFFFFFll) ASH_FAIL("too many positions in one call");
     activate_runs_kernel<<<static_cast<unsigned>(groups), kHeapBlock, 0, s>>>(
             map->d, a, touched, coords);
-    ASH_LAUNCH_CHECK();
-    return 0;
-}
-
-int ash_ray_find_near_far(ash_map_t* map, const float* ray_origins,
-                          const float* ray_directions, const float* bbox_min,
-                          const float* bbox_max, int64_t n, float t_min,
-                          float t_max, float t_step, float grid2cell_multiplier,
-                          float* ray_nears, float* ray_fars, void* stream) {
-    (void)t_step;  // unused by the reference as well (ash/src/sampler.cu:21)
-    if (check_batch(map, ray_origins, n)) return 1;
-    if (map->key_dim != 3) {
-        ASH_FAIL("hashmap is not a GPU hashmap of type <int, 3>, ray sample not supported");
-    }
-    if (!(grid2cell_multiplier > 0.f)) ASH_FAIL("grid2cell_multiplier must be positive");
-    if (n == 0) return 0;
-    if (ray_directions == nullptr || bbox_min == nullptr || bbox_max == nullptr ||
-        ray_nears == nullptr || ray_fars == nullptr) {
-        ASH_FAIL("null pointer in ray_find_near_far");
-    }
-    DeviceGuard guard;
-    ASH_HIP(guard.enter(map->device));
-    if (settle_table(map, static_cast<hipStream_t>(stream))) return 1;
-    // every step must advance t (else the march never ends), and their number
-    // must stay finite
-    const float half_block = static_cast<float>(grid2cell_multiplier * 0.5);
-    if (t_min < t_max) {
-        if (!(t_max + half_block > t_max) ||
-            !((static_cast<double>(t_max) - t_min) / half_block < 1e8)) {
-            ASH_FAIL("ray_find_near_far: the step is too small for this range");
-        }
-    }
-    ray_near_far_kernel<<<grid_for(n, kBlock / 64), kBlock, 0, static_cast<hipStream_t>(stream)>>>(
-            map->d, ray_origins, ray_directions, bbox_min, bbox_max, n, t_min,
-            t_max, grid2cell_multiplier, ray_nears, ray_fars);
-    ASH_LAUNCH_CHECK();
-    return 0;
-}
-
-int ash_ray_sample(ash_map_t* map, const float* ray_origins,
-                   const float* ray_directions, const float* ray_nears,
-                   const float* ray_fars, int64_t n, int64_t max_samples_per_ray,
-                   float grid2cell_multiplier, int64_t* counts,
-                   const int64_t* prefix, int64_t* ray_indices, float* t_nears,
-                   float* t_fars, void* stream) {
-    if (check_batch(map, ray_origins, n)) return 1;
-    if (map->key_dim != 3) {
-        ASH_FAIL("hashmap is not a GPU hashmap of type <int, 3>, ray sample not supported");
-    }
-    if (!(grid2cell_multiplier > 0.f)) ASH_FAIL("grid2cell_multiplier must be positive");
-    if (max_samples_per_ray < 1) ASH_FAIL("max_samples_per_ray must be positive");
-    if (n == 0) return 0;
-    if (ray_directions == nullptr || ray_nears == nullptr || ray_fars == nullptr) {
-        ASH_FAIL("null pointer in ray_sample");
-    }
-    const bool assign = prefix != nullptr && ray_indices != nullptr &&
-                        t_nears != nullptr && t_fars != nullptr;
-    if ((counts != nullptr) == assign) {
-        ASH_FAIL("ray_sample: pass either counts (allocation pass) or prefix and "
-                 "the three outputs (assignment pass)");
-    }
-    DeviceGuard guard;
-    ASH_HIP(guard.enter(map->device));
-    if (settle_table(map, static_cast<hipStream_t>(stream))) return 1;
-    launch_ray_sample(map, ray_origins, ray_directions, ray_nears, ray_fars, n,
-                      static_cast<float>(max_samples_per_ray), grid2cell_multiplier, counts,
-                      prefix, ray_indices, t_nears, t_fars, nullptr, 0,
-                      static_cast<hipStream_t>(stream));
-    ASH_LAUNCH_CHECK();
-    return 0;
-}
-
-int ash_ray_sample_staged(ash_map_t* map, const float* ray_origins,
-                          const float* ray_directions, const float* ray_nears,
-                          const float* ray_fars, int64_t n, int64_t max_samples_per_ray,
-                          float grid2cell_multiplier, int64_t* counts, float* stage,
-                          int64_t stride, void* stream) {
-    if (check_batch(map, ray_origins, n)) return 1;
-    if (map->key_dim != 3) {
-        ASH_FAIL("hashmap is not a GPU hashmap of type <int, 3>, ray sample not supported");
-    }
-    if (!(grid2cell_multiplier > 0.f)) ASH_FAIL("grid2cell_multiplier must be positive");
-    if (max_samples_per_ray < 1) ASH_FAIL("max_samples_per_ray must be positive");
-    if (stride < 1) ASH_FAIL("ray_sample_staged: stride must be positive");
-    if (n == 0) return 0;
-    if (ray_directions == nullptr || ray_nears == nullptr || ray_fars == nullptr ||
-        counts == nullptr || stage == nullptr) {
-        ASH_FAIL("null pointer in ray_sample_staged");
-    }
-    if (reinterpret_cast<uintptr_t>(stage) % 8 != 0) ASH_FAIL("ray_sample_staged: stage must be 8-byte aligned");
-    DeviceGuard guard;
-    ASH_HIP(guard.enter(map->device));
-    if (settle_table(map, static_cast<hipStream_t>(stream))) return 1;
-    launch_ray_sample(map, ray_origins, ray_directions, ray_nears, ray_fars, n,
-                      static_cast<float>(max_samples_per_ray), grid2cell_multiplier, counts,
-                      nullptr, nullptr, nullptr, nullptr, reinterpret_cast<float2*>(stage),
-                      stride, static_cast<hipStream_t>(stream));
-    ASH_LAUNCH_CHECK();
-    return 0;
-}
-
-int ash_ray_sample_compact(const int64_t* counts, const int64_t* prefix, const float* stage,
-                           int64_t stride, int64_t n, int64_t* ray_indices, float* t_nears,
-                           float* t_fars, void* stream) {
-    if (n < 0 || stride < 1) ASH_FAIL("ray_sample_compact: bad sizes");
-    if (n == 0) return 0;
-    if (counts == nullptr || prefix == nullptr || stage == nullptr || ray_indices == nullptr ||
-        t_nears == nullptr || t_fars == nullptr) {
-        ASH_FAIL("null pointer in ray_sample_compact");
-    }
-    if (n > ((int64_t{1} << 32) - kBlock) / stride) ASH_FAIL("ray_sample_compact: too many slots");
-    ray_compact_kernel<<<grid_for(n * stride), kBlock, 0, static_cast<hipStream_t>(stream)>>>(
-            counts, prefix, reinterpret_cast<const float2*>(stage), stride, n, ray_indices,
-            t_nears, t_fars);
     ASH_LAUNCH_CHECK();
     return 0;
 }

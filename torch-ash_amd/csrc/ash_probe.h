@@ -34,6 +34,12 @@ __device__ __forceinline__ uint32_t quad_or(uint32_t v) {
     return v;
 }
 
+// The value of the lane before this one (lane 0: its own), by a shift of the
+// whole wavefront.  Every lane takes part.
+__device__ __forceinline__ int32_t lane_before(int32_t v) {
+    return __builtin_amdgcn_update_dpp(v, v, 0x138, 0xF, 0xF, false);
+}
+
 template <int R>
 struct Round {
     static constexpr int value = R;
@@ -171,7 +177,7 @@ __device__ __forceinline__ bool find_block_by_runs(const MapDev& m, const int32_
     const int lane = threadIdx.x & 63;
     int same = lane > 0;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) same &= __shfl_up(k[d], 1) == k[d];
+    for (int d = 0; d < 3; ++d) same &= lane_before(k[d]) == k[d];
     const bool head = !same;
     const bool asked = find_key_alone<3>(m, k, active && head, res);
     const uint64_t heads = __ballot(head);

@@ -1,0 +1,638 @@
+// Rays through the active blocks of a grid (ash/src/sampler.cu:7-67 and
+// :122-214): the near / far range of a ray and the samples inside blocks.
+//
+// Positions are origin + t * direction as a fused multiply-add (what nvcc makes
+// of the reference's expression); the march is in cell units and a block is
+// `grid2cell` cells wide.  Rays may come in world units: the kernels then bring
+// them to cell units and their results back, operation by operation as torch
+// evaluates `(x - origin) / cell_size` and `t * cell_size` on the device.
+#include "ash_probe.h"
+
+#include "../../include/ash_hip.h"
+
+#include <cmath>
+
+namespace ash {
+namespace {
+
+constexpr int kBlock = 256;
+
+// World units: cell units = (x - origin) * inv_cell, world = t * cell.  Neutral:
+// origin null, inv_cell = cell = 1.
+struct RayUnits {
+    const float* origin;
+    float inv_cell, cell;
+};
+
+__device__ __forceinline__ float to_cells(const RayUnits& u, float x, int axis) {
+    const float o = u.origin != nullptr ? u.origin[axis] : 0.f;
+    return __fmul_rn(__fsub_rn(x, o), u.inv_cell);
+}
+
+// Lane `l`'s value, and a condition that is the same in every lane.
+__device__ __forceinline__ float lane_value(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ bool uniform(bool c) {
+    return __builtin_amdgcn_readfirstlane(static_cast<int>(c)) != 0;
+}
+
+__device__ __forceinline__ void ray_block(const float (&o)[3], const float (&d)[3],
+                                          float t, float cell2grid,
+                                          int32_t (&block)[3], float (&x)[3]) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        x[a] = fmaf(t, d[a], o[a]);
+        block[a] = static_cast<int32_t>(floorf(__fmul_rn(x[a], cell2grid)));
+    }
+}
+
+// One wavefront per ray: the march of ray_find_near_far visits the parameters
+// t_0 = t_min, t_{k+1} = t_k + step regardless of what it finds, so lane l of
+// round r takes step 64 r + l, the 64 look-ups go out together, and the near /
+// far recurrence is then replayed over the hits in step order.  The march ends
+// at the first step that is at or beyond t_max or outside the box, exactly where
+// the sequential loop stops.
+//
+// The kernel is bound by vector instructions.  The parameters are the same for
+// every ray, so the host works the chain of additions out (the same IEEE
+// additions) for the first kChain steps and hands it over with the launch, 64
+// additions per round less; and the recurrence takes `far` from the last hit and
+// `near`, once it is set, only from the number of hits (two instructions each
+// instead of a walk over their parameters).
+constexpr int kChain = 512;
+
+struct StepChain {
+    float t[kChain];
+};
+
+__global__ __launch_bounds__(kBlock) void ray_near_far_kernel(
+        MapDev m, const float* __restrict__ origins,
+        const float* __restrict__ directions, RayUnits u, const float* __restrict__ bbox_min,
+        const float* __restrict__ bbox_max, int64_t n, float t_min, float t_max,
+        float grid2cell, float* __restrict__ nears, float* __restrict__ fars, StepChain chain) {
+    const int lane = threadIdx.x & 63;
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * (kBlock / 64) + (threadIdx.x >> 6);
+    if (i >= n) return;  // whole wavefronts leave together
+    const float cell2grid = static_cast<float>(1.0 / grid2cell);
+    const float t_grid_step = static_cast<float>(grid2cell * 0.5);
+    float o[3], d[3], lo[3], hi[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        o[a] = to_cells(u, origins[i * 3 + a], a);
+        d[a] = directions[i * 3 + a];
+        lo[a] = to_cells(u, bbox_min[a], a);
+        hi[a] = to_cells(u, bbox_max[a], a);
+    }
+    float near = -1.f, far = t_max;
+    float t = 0.f;
+    for (int first = 0;; first += 64) {
+        if (first < kChain) {
+            t = chain.t[first + lane];
+        } else {
+            for (int j = 0; j < 64; ++j) t += t_grid_step;
+        }
+        int32_t block[3];
+        float x[3];
+        ray_block(o, d, t, cell2grid, block, x);
+        bool go = t < t_max;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) go = go && x[a] >= lo[a] && x[a] <= hi[a];
+        const uint64_t stop = __ballot(!go);
+        const int first_stop = stop ? __builtin_ctzll(stop) : 64;
+        // (steps are half a block apart: neighbouring lanes often stand in the
+        // same block and share a look-up)
+        int32_t idx;
+        const bool active = lane < first_stop;
+        const bool found = find_block_by_runs(m, block, active, idx);
+        uint64_t hits = __ballot(found && active);
+        if (hits) {
+            far = fminf(lane_value(t, 63 - __builtin_clzll(hits)) + t_grid_step, t_max);
+            if (t_min >= 0.f) {   // near never turns negative again
+                int steps = __popcll(hits);
+                if (uniform(near < 0.f)) {
+                    near = lane_value(t, __builtin_ctzll(hits));
+                    --steps;
+                }
+                for (; steps > 0; --steps) near = fmaxf(near - t_grid_step, t_min);
+            } else {
+                while (hits) {
+                    const float t_hit = lane_value(t, __builtin_ctzll(hits));
+                    near = near < 0.f ? t_hit : fmaxf(near - t_grid_step, t_min);
+                    hits &= hits - 1;
+                }
+            }
+        }
+        if (first_stop < 64) break;
+    }
+    if (lane == 0) {
+        nears[i] = __fmul_rn(near, u.cell);
+        fars[i] = __fmul_rn(far, u.cell);
+    }
+}
+
+// What the sampling march knows of a ray: a lane's block and whether it is
+// stored.
+struct KnownBlock {
+    int32_t at[3];
+    bool have, stored;
+};
+
+// The march of ray_sample.  counts != nullptr: allocation pass; otherwise the
+// assignment pass, which writes the samples of ray i at prefix[i - 1] ..
+// prefix[i].  An allocation pass with `stage` also keeps the first `stride`
+// samples of ray i as pairs (t_near, t_far) at stage[i * stride + k], so that
+// the assignment pass can be a copy instead of a second march; with `groups` it
+// leaves the sum and the largest of its workgroup's counts there.
+//
+// The reference looks the block under t up at every step, one dependent look-up
+// after the other; where the march may stand next is known beforehand, though.
+// LPR = 8: the eight lanes of a ray look up the block under t, the blocks where
+// four steps on through stored blocks lead, and those where three steps over
+// empty ones lead, all at once, and the march goes on without memory until it
+// stands in a block that none of the lanes holds, which starts the next round.  LPR = 1: every lane marches a ray of its own and
+// answers from its latest look-up while it stays in the same block, which takes
+// fewer instructions where there are rays enough to hide the look-ups.
+struct GroupSamples {
+    int64_t sum, most;
+};
+
+template <int LPR>
+__global__ __launch_bounds__(kBlock) void ray_sample_kernel(
+        MapDev m, const float* __restrict__ origins,
+        const float* __restrict__ directions, RayUnits u, const float* __restrict__ ray_nears,
+        const float* __restrict__ ray_fars, float near_for_all, float far_for_all, int64_t n,
+        float max_samples, float grid2cell, int64_t* __restrict__ counts,
+        const int64_t* __restrict__ prefix, int64_t* __restrict__ ray_indices,
+        float* __restrict__ t_nears, float* __restrict__ t_fars,
+        float2* __restrict__ stage, int64_t stride, GroupSamples* __restrict__ groups) {
+    const int lane = threadIdx.x & 63;
+    const int64_t gid = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    const int64_t i = gid / LPR;
+    const int j = LPR == 1 ? 0 : static_cast<int>(gid % LPR);
+    const bool writer = j == 0;   // the lane of a ray that stores its results
+    const bool active = i < n;
+    const float cell2grid = static_cast<float>(1.0 / grid2cell);
+    float o[3], d[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        o[a] = active ? to_cells(u, origins[i * 3 + a], a) : 0.f;
+        d[a] = active ? directions[i * 3 + a] : 0.f;
+    }
+    float ray_near = near_for_all, ray_far = far_for_all;
+    if (active && ray_nears != nullptr) ray_near = __fmul_rn(ray_nears[i], u.inv_cell);
+    if (active && ray_fars != nullptr) ray_far = __fmul_rn(ray_fars[i], u.inv_cell);
+    const float t_step = fmaxf(0.7f, __fdiv_rn(ray_far - ray_near, max_samples));
+    const float t_grid_step = __fmul_rn(t_step, grid2cell);
+    const int64_t start = (counts == nullptr && active && i > 0) ? prefix[i - 1] : 0;
+    float t = ray_near, t_near = ray_near;
+    int64_t local = 0;
+    bool live = active && t < ray_far;
+    // One step of the march, given whether the block under t is stored.
+    auto step = [&](bool stored) {
+        const float before = t;
+        if (!stored) {
+            t += t_grid_step;
+        } else {
+            t += t_step;
+            if (!writer) {
+            } else if (counts == nullptr) {
+                ray_indices[start + local] = i;
+                t_nears[start + local] = t_near;
+                t_fars[start + local] = t;
+            } else if (stage != nullptr && local < stride) {
+                stage[i * stride + local] = make_float2(t_near, t);
+            }
+            t_near = t;
+            ++local;
+        }
+        // a step that no longer advances t (range far beyond fp32
+        // resolution) would never end; the reference has no such guard
+        live = t < ray_far && t > before;
+    };
+    KnownBlock known = {{0, 0, 0}, false, false};
+    // how far ahead of t this lane looks: half a block or a step, whichever is
+    // more, at a time for lanes 1..4, empty steps for lanes 5..7
+    const float ahead = j < 5 ? static_cast<float>(j) * fmaxf(t_step, 0.5f * grid2cell)
+                              : static_cast<float>(j - 4) * t_grid_step;
+    while (__ballot(live)) {
+        int32_t block[3] = {0, 0, 0};
+        float x[3];
+        bool ask = false;
+        while (live) {
+            ray_block(o, d, t, cell2grid, block, x);
+            const bool here = known.have && block[0] == known.at[0] && block[1] == known.at[1] &&
+                              block[2] == known.at[2];
+            if constexpr (LPR == 1) {
+                if (!here) {
+                    ask = true;
+                    break;
+                }
+                step(known.stored);
+            } else {
+                // (the lanes of a ray are in this loop together or not at all)
+                const uint32_t shift = lane & ~(LPR - 1);
+                const uint32_t any = static_cast<uint32_t>(__ballot(here) >> shift) & ((1u << LPR) - 1u);
+                if (any == 0u) {
+                    ask = true;
+                    break;
+                }
+                const uint32_t stored = static_cast<uint32_t>(__ballot(here && known.stored) >> shift) &
+                                        ((1u << LPR) - 1u);
+                step(stored != 0u);
+            }
+        }
+        bool mine = live && ask;
+        if constexpr (LPR > 1) {
+            // the lane's own block ahead; the lane before it may hold the same
+            if (mine && j > 0) {
+                ray_block(o, d, t + ahead, cell2grid, block, x);
+                mine = t + ahead < ray_far;
+            }
+            int same = 1;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) same &= lane_before(block[a]) == block[a];
+            if (j > 0 && same) mine = false;
+        }
+        int32_t idx;
+        const bool stored = find_key_alone<3>(m, block, mine, idx);
+        if (live && ask) {
+#pragma unroll
+            for (int a = 0; a < 3; ++a) known.at[a] = block[a];
+            known.have = mine;
+            known.stored = stored && mine;
+            if constexpr (LPR == 1) step(stored);
+        }
+    }
+    if (active && writer && counts != nullptr) counts[i] = local;
+    if (groups != nullptr) {
+        int64_t sum = active && writer ? local : 0, most = sum;
+#pragma unroll
+        for (int b = 32; b > 0; b >>= 1) {
+            sum += __shfl_xor(sum, b);
+            const int64_t other = __shfl_xor(most, b);
+            most = other > most ? other : most;
+        }
+        __shared__ GroupSamples s_wave[kBlock / 64];
+        if (lane == 0) s_wave[threadIdx.x >> 6] = {sum, most};
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            GroupSamples g = s_wave[0];
+#pragma unroll
+            for (int w = 1; w < kBlock / 64; ++w) {
+                g.sum += s_wave[w].sum;
+                g.most = s_wave[w].most > g.most ? s_wave[w].most : g.most;
+            }
+            groups[blockIdx.x] = g;
+        }
+    }
+}
+
+// One workgroup turns the sums of the march's workgroups into running sums (what
+// lies before each, in place) and leaves the number of samples and the largest
+// count of a ray for the host.
+constexpr int kScanThreads = 1024;
+
+__global__ __launch_bounds__(kScanThreads) void ray_scan_kernel(GroupSamples* __restrict__ groups,
+                                                                int n, int32_t* landing,
+                                                                int32_t stamp) {
+    __shared__ int64_t s_sum[kScanThreads / 64];
+    __shared__ int64_t s_most[kScanThreads / 64];
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const int per = (n + kScanThreads - 1) / kScanThreads;
+    const int first = threadIdx.x * per;
+    const int last = first + per < n ? first + per : n;
+    int64_t sum = 0, most = 0;
+    for (int g = first; g < last; ++g) {
+        sum += groups[g].sum;
+        most = groups[g].most > most ? groups[g].most : most;
+    }
+    int64_t incl = sum;
+#pragma unroll
+    for (int b = 1; b < 64; b <<= 1) {
+        const int64_t up = __shfl_up(incl, b);
+        if (lane >= b) incl += up;
+        const int64_t other = __shfl_xor(most, b);
+        most = other > most ? other : most;
+    }
+    if (lane == 63) s_sum[wave] = incl;
+    if (lane == 0) s_most[wave] = most;
+    __syncthreads();
+    int64_t before = incl - sum, total = 0;
+    for (int w = 0; w < kScanThreads / 64; ++w) {
+        if (w < wave) before += s_sum[w];
+        total += s_sum[w];
+        most = s_most[w] > most ? s_most[w] : most;
+    }
+    for (int g = first; g < last; ++g) {
+        const int64_t own = groups[g].sum;
+        groups[g].sum = before;
+        before += own;
+    }
+    if (threadIdx.x == 0) {
+        const int32_t words[4] = {static_cast<int32_t>(total), static_cast<int32_t>(total >> 32),
+                                  static_cast<int32_t>(most), static_cast<int32_t>(most >> 32)};
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            __hip_atomic_store(landing + w, words[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        __hip_atomic_store(landing + kLandingStamp, stamp, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+// The staged samples of `rays` rays, the share of one workgroup of the march,
+// copied to their place: eight lanes per ray, both sides in runs.  Also the
+// running sums of the counts.
+__global__ __launch_bounds__(kBlock) void ray_place_kernel(
+        const int64_t* __restrict__ counts, const GroupSamples* __restrict__ groups,
+        const float2* __restrict__ stage, int64_t stride, int64_t n, int rays, float cell,
+        int64_t* __restrict__ ray_indices, float* __restrict__ t_nears,
+        float* __restrict__ t_fars, int64_t* __restrict__ prefix) {
+    __shared__ int64_t s_incl[kBlock];
+    __shared__ int64_t s_wave[kBlock / 64];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int64_t first = static_cast<int64_t>(blockIdx.x) * rays;
+    const int64_t own = tid < rays && first + tid < n ? counts[first + tid] : 0;
+    int64_t incl = own;
+#pragma unroll
+    for (int b = 1; b < 64; b <<= 1) {
+        const int64_t up = __shfl_up(incl, b);
+        if (lane >= b) incl += up;
+    }
+    if (lane == 63) s_wave[tid >> 6] = incl;
+    __syncthreads();
+    incl += groups[blockIdx.x].sum;
+    for (int w = 0; w < (tid >> 6); ++w) incl += s_wave[w];
+    s_incl[tid] = incl;
+    if (tid < rays && first + tid < n) prefix[first + tid] = incl;
+    __syncthreads();
+    for (int r = tid >> 3; r < rays && first + r < n; r += kBlock / 8) {
+        const int64_t to = r > 0 ? s_incl[r - 1] : groups[blockIdx.x].sum;
+        const int64_t count = s_incl[r] - to;
+        const float2* from = stage + (first + r) * stride;
+        for (int64_t k = tid & 7; k < count; k += 8) {
+            const float2 s = from[k];
+            ray_indices[to + k] = first + r;
+            t_nears[to + k] = __fmul_rn(s.x, cell);
+            t_fars[to + k] = __fmul_rn(s.y, cell);
+        }
+    }
+}
+
+// Assignment pass from the staged samples and running sums of the caller's: one
+// thread per staged slot.
+__global__ __launch_bounds__(kBlock) void ray_compact_kernel(
+        const int64_t* __restrict__ counts, const int64_t* __restrict__ prefix,
+        const float2* __restrict__ stage, int64_t stride, int64_t n,
+        int64_t* __restrict__ ray_indices, float* __restrict__ t_nears,
+        float* __restrict__ t_fars) {
+    const int64_t slot = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    if (slot >= n * stride) return;
+    const int64_t i = slot / stride;
+    const int64_t k = slot - i * stride;
+    if (k >= counts[i]) return;
+    const int64_t out = (i > 0 ? prefix[i - 1] : 0) + k;
+    const float2 s = stage[slot];
+    ray_indices[out] = i;
+    t_nears[out] = s.x;
+    t_fars[out] = s.y;
+}
+
+// Lanes per ray of the sampling march: below this many rays there are not
+// enough wavefronts to hide a look-up per block, see ray_sample_kernel.
+constexpr int64_t kRaysPerLaneMin = int64_t{1} << 16;
+
+int lanes_per_ray(int64_t n) { return n < kRaysPerLaneMin ? 8 : 1; }
+
+unsigned march_groups(int64_t n) {
+    return static_cast<unsigned>((n * lanes_per_ray(n) + kBlock - 1) / kBlock);
+}
+
+struct March {
+    const float *origins, *directions;
+    RayUnits units;
+    const float *nears, *fars;
+    float near_for_all, far_for_all;
+    int64_t n;
+    float max_samples, grid2cell;
+};
+
+int launch_march(ash_map_t* map, const March& r, int64_t* counts, const int64_t* prefix,
+                 int64_t* ray_indices, float* t_nears, float* t_fars, float* stage, int64_t stride,
+                 GroupSamples* groups, hipStream_t s) {
+    auto kernel = lanes_per_ray(r.n) == 8 ? ray_sample_kernel<8> : ray_sample_kernel<1>;
+    kernel<<<march_groups(r.n), kBlock, 0, s>>>(
+            map->d, r.origins, r.directions, r.units, r.nears, r.fars, r.near_for_all, r.far_for_all,
+            r.n, r.max_samples, r.grid2cell, counts, prefix, ray_indices, t_nears, t_fars,
+            reinterpret_cast<float2*>(stage), stride, groups);
+    ASH_LAUNCH_CHECK();
+    return 0;
+}
+
+constexpr RayUnits kCellUnits = {nullptr, 1.f, 1.f};
+
+int check_rays(const ash_map_t* map, const float* origins, const float* directions, int64_t n,
+               float grid2cell, float cell_size) {
+    if (check_batch(map, origins, n)) return 1;
+    if (map->key_dim != 3) {
+        ASH_FAIL("hashmap is not a GPU hashmap of type <int, 3>, ray sample not supported");
+    }
+    if (!(grid2cell > 0.f)) ASH_FAIL("grid2cell_multiplier must be positive");
+    if (!(cell_size > 0.f) || !(cell_size < INFINITY)) ASH_FAIL("cell_size must be positive and finite");
+    if (n > 0 && directions == nullptr) ASH_FAIL("null ray directions");
+    return 0;
+}
+
+int near_far(ash_map_t* map, const float* origins, const float* directions, const RayUnits& units,
+             const float* bbox_min, const float* bbox_max, int64_t n, float t_min, float t_max,
+             float grid2cell, float* nears, float* fars, hipStream_t s) {
+    if (check_rays(map, origins, directions, n, grid2cell, units.cell)) return 1;
+    if (n == 0) return 0;
+    if (bbox_min == nullptr || bbox_max == nullptr || nears == nullptr || fars == nullptr) {
+        ASH_FAIL("null pointer in ray_find_near_far");
+    }
+    DeviceGuard guard;
+    ASH_HIP(guard.enter(map->device));
+    if (settle_table(map, s)) return 1;
+    // every step must advance t (else the march never ends), and their number
+    // must stay finite
+    const float half_block = static_cast<float>(grid2cell * 0.5);
+    if (t_min < t_max) {
+        if (!(t_max + half_block > t_max) ||
+            !((static_cast<double>(t_max) - t_min) / half_block < 1e8)) {
+            ASH_FAIL("ray_find_near_far: the step is too small for this range");
+        }
+    }
+    StepChain chain;
+    float t = t_min;
+    for (int k = 0; k < kChain; ++k) {
+        chain.t[k] = t;
+        t += half_block;
+    }
+    ray_near_far_kernel<<<static_cast<unsigned>((n + kBlock / 64 - 1) / (kBlock / 64)), kBlock, 0, s>>>(
+            map->d, origins, directions, units, bbox_min, bbox_max, n, t_min, t_max, grid2cell,
+            nears, fars, chain);
+    ASH_LAUNCH_CHECK();
+    return 0;
+}
+
+}  // namespace
+}  // namespace ash
+
+using namespace ash;
+
+extern "C" {
+
+int ash_ray_find_near_far(ash_map_t* map, const float* ray_origins,
+                          const float* ray_directions, const float* bbox_min,
+                          const float* bbox_max, int64_t n, float t_min,
+                          float t_max, float t_step, float grid2cell_multiplier,
+                          float* ray_nears, float* ray_fars, void* stream) {
+    (void)t_step;  // unused by the reference as well (ash/src/sampler.cu:21)
+    return near_far(map, ray_origins, ray_directions, kCellUnits, bbox_min, bbox_max, n, t_min,
+                    t_max, grid2cell_multiplier, ray_nears, ray_fars,
+                    static_cast<hipStream_t>(stream));
+}
+
+int ash_ray_find_near_far_world(ash_map_t* map, const float* ray_origins,
+                                const float* ray_directions, const float* origin, float cell_size,
+                                const float* bbox_min, const float* bbox_max, int64_t n, float t_min,
+                                float t_max, float grid2cell_multiplier, float* ray_nears,
+                                float* ray_fars, void* stream) {
+    return near_far(map, ray_origins, ray_directions, {origin, 1.0f / cell_size, cell_size}, bbox_min,
+                    bbox_max, n, t_min, t_max, grid2cell_multiplier, ray_nears, ray_fars,
+                    static_cast<hipStream_t>(stream));
+}
+
+int ash_ray_sample(ash_map_t* map, const float* ray_origins,
+                   const float* ray_directions, const float* ray_nears,
+                   const float* ray_fars, int64_t n, int64_t max_samples_per_ray,
+                   float grid2cell_multiplier, int64_t* counts,
+                   const int64_t* prefix, int64_t* ray_indices, float* t_nears,
+                   float* t_fars, void* stream) {
+    if (check_rays(map, ray_origins, ray_directions, n, grid2cell_multiplier, 1.f)) return 1;
+    if (max_samples_per_ray < 1) ASH_FAIL("max_samples_per_ray must be positive");
+    if (n == 0) return 0;
+    if (ray_nears == nullptr || ray_fars == nullptr) ASH_FAIL("null pointer in ray_sample");
+    const bool assign = prefix != nullptr && ray_indices != nullptr &&
+                        t_nears != nullptr && t_fars != nullptr;
+    if ((counts != nullptr) == assign) {
+        ASH_FAIL("ray_sample: pass either counts (allocation pass) or prefix and "
+                 "the three outputs (assignment pass)");
+    }
+    DeviceGuard guard;
+    ASH_HIP(guard.enter(map->device));
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (settle_table(map, s)) return 1;
+    return launch_march(map, {ray_origins, ray_directions, kCellUnits, ray_nears, ray_fars, 0.f, 0.f, n,
+                              static_cast<float>(max_samples_per_ray), grid2cell_multiplier},
+                        counts, prefix, ray_indices, t_nears, t_fars, nullptr, 0, nullptr, s);
+}
+
+int ash_ray_sample_staged(ash_map_t* map, const float* ray_origins,
+                          const float* ray_directions, const float* ray_nears,
+                          const float* ray_fars, int64_t n, int64_t max_samples_per_ray,
+                          float grid2cell_multiplier, int64_t* counts, float* stage,
+                          int64_t stride, void* stream) {
+    if (check_rays(map, ray_origins, ray_directions, n, grid2cell_multiplier, 1.f)) return 1;
+    if (max_samples_per_ray < 1) ASH_FAIL("max_samples_per_ray must be positive");
+    if (stride < 1) ASH_FAIL("ray_sample_staged: stride must be positive");
+    if (n == 0) return 0;
+    if (ray_nears == nullptr || ray_fars == nullptr || counts == nullptr || stage == nullptr) {
+        ASH_FAIL("null pointer in ray_sample_staged");
+    }
+    if (reinterpret_cast<uintptr_t>(stage) % 8 != 0) ASH_FAIL("ray_sample_staged: stage must be 8-byte aligned");
+    DeviceGuard guard;
+    ASH_HIP(guard.enter(map->device));
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (settle_table(map, s)) return 1;
+    return launch_march(map, {ray_origins, ray_directions, kCellUnits, ray_nears, ray_fars, 0.f, 0.f, n,
+                              static_cast<float>(max_samples_per_ray), grid2cell_multiplier},
+                        counts, nullptr, nullptr, nullptr, nullptr, stage, stride, nullptr, s);
+}
+
+int ash_ray_sample_compact(const int64_t* counts, const int64_t* prefix, const float* stage,
+                           int64_t stride, int64_t n, int64_t* ray_indices, float* t_nears,
+                           float* t_fars, void* stream) {
+    if (n < 0 || stride < 1) ASH_FAIL("ray_sample_compact: bad sizes");
+    if (n == 0) return 0;
+    if (counts == nullptr || prefix == nullptr || stage == nullptr || ray_indices == nullptr ||
+        t_nears == nullptr || t_fars == nullptr) {
+        ASH_FAIL("null pointer in ray_sample_compact");
+    }
+    if (n > ((int64_t{1} << 32) - kBlock) / stride) ASH_FAIL("ray_sample_compact: too many slots");
+    ray_compact_kernel<<<static_cast<unsigned>((n * stride + kBlock - 1) / kBlock), kBlock, 0,
+                         static_cast<hipStream_t>(stream)>>>(
+            counts, prefix, reinterpret_cast<const float2*>(stage), stride, n, ray_indices,
+            t_nears, t_fars);
+    ASH_LAUNCH_CHECK();
+    return 0;
+}
+
+int64_t ash_ray_sample_groups(int64_t n) { return n > 0 ? static_cast<int64_t>(march_groups(n)) : 0; }
+
+int ash_ray_sample_march(ash_map_t* map, const float* ray_origins, const float* ray_directions,
+                         const float* origin, float cell_size, const float* ray_nears,
+                         const float* ray_fars, float near_for_all, float far_for_all, int64_t n,
+                         int64_t max_samples_per_ray, float grid2cell_multiplier, int64_t* counts,
+                         int64_t* groups, float* stage, int64_t stride, int64_t out[2],
+                         void* stream) {
+    if (check_rays(map, ray_origins, ray_directions, n, grid2cell_multiplier, cell_size)) return 1;
+    if (max_samples_per_ray < 1) ASH_FAIL("max_samples_per_ray must be positive");
+    if (stride < 1) ASH_FAIL("ray_sample_march: stride must be positive");
+    if (out == nullptr) ASH_FAIL("null output pointer");
+    out[0] = out[1] = 0;
+    if (n == 0) return 0;
+    if (counts == nullptr || groups == nullptr || stage == nullptr) {
+        ASH_FAIL("null pointer in ray_sample_march");
+    }
+    if (reinterpret_cast<uintptr_t>(stage) % 8 != 0) ASH_FAIL("ray_sample_march: stage must be 8-byte aligned");
+    if (n > (int64_t{1} << 32)) ASH_FAIL("ray_sample_march: too many rays");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (is_capturing(s)) {
+        ASH_FAIL("the number of samples cannot be read while the stream is being captured");
+    }
+    DeviceGuard guard;
+    ASH_HIP(guard.enter(map->device));
+    if (settle_table(map, s)) return 1;
+    if (take_line(map)) return 1;
+    auto* g = reinterpret_cast<GroupSamples*>(groups);
+    if (launch_march(map, {ray_origins, ray_directions, {origin, 1.0f / cell_size, cell_size}, ray_nears,
+                           ray_fars, near_for_all, far_for_all, n,
+                           static_cast<float>(max_samples_per_ray), grid2cell_multiplier},
+                     counts, nullptr, nullptr, nullptr, nullptr, stage, stride, g, s)) {
+        return 1;
+    }
+    int32_t* landing = map->line + kLineRays;
+    const int32_t stamp = ++map->stamp;
+    ray_scan_kernel<<<1, kScanThreads, 0, s>>>(g, static_cast<int>(march_groups(n)), landing, stamp);
+    ASH_LAUNCH_CHECK();
+    if (wait_for_stamp(landing + kLandingStamp, stamp)) return 1;
+    for (int w = 0; w < 2; ++w) {
+        out[w] = static_cast<int64_t>(static_cast<uint32_t>(landing[2 * w])) |
+                 (static_cast<int64_t>(landing[2 * w + 1]) << 32);
+    }
+    return 0;
+}
+
+int ash_ray_sample_place(const int64_t* counts, const int64_t* groups, const float* stage,
+                         int64_t stride, int64_t n, float cell_size, int64_t* ray_indices,
+                         float* t_nears, float* t_fars, int64_t* prefix, void* stream) {
+    if (n < 0 || stride < 1) ASH_FAIL("ray_sample_place: bad sizes");
+    if (n == 0) return 0;
+    if (counts == nullptr || groups == nullptr || stage == nullptr || prefix == nullptr) {
+        ASH_FAIL("null pointer in ray_sample_place");
+    }
+    PointerGuard guard;
+    ASH_HIP(guard.enter_for(counts));
+    ray_place_kernel<<<march_groups(n), kBlock, 0, static_cast<hipStream_t>(stream)>>>(
+            counts, reinterpret_cast<const GroupSamples*>(groups),
+            reinterpret_cast<const float2*>(stage), stride, n, kBlock / lanes_per_ray(n), cell_size,
+            ray_indices, t_nears, t_fars, prefix);
+    ASH_LAUNCH_CHECK();
+    return 0;
+}
+
+}  // extern "C"

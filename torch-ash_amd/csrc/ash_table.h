@@ -162,6 +162,10 @@ inline bool heap_in_order(const ash_map* map) { return !map->heap_dirty && !map-
 // false for one that took entries away.
 // `s`: the stream the call runs on (captured: see ash_map::replayed).
 void counters_changed(ash_map* map, bool inserted, hipStream_t s);
+// The map's page-locked words (made on first use), and the wait for one of them.
+int take_line(ash_map* map);
+int wait_for_stamp(const int32_t* word, int32_t stamp);
+int settle_landing_place(ash_map* map);
 // Adds up `n` words of `counts` into the counter of touched blocks and queues the
 // read-back of the counters behind the stream's work (ash_map.hip).
 int queue_touched_count(ash_map* map, const int32_t* counts, int n, hipStream_t s);

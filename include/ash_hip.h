@@ -695,6 +695,22 @@ int ash_convolution_forward_listed(const void* inputs, const void* weights,
                                    int64_t num_cell_nbs, int64_t num_grid_nbs,
                                    int32_t dtype, uint8_t* listed, void* stream);
 
+/* The same convolution for the tables that SparseDenseGrid builds, which are
+ * then not needed: cell c = x + G y + G^2 z, tap k = (dx + r) + W (dy + r) +
+ * W^2 (dz + r) with W = `window` = 2 r + 1, neighbour block (bx + 1) + 3 (by + 1)
+ * + 9 (bz + 1) of lut_grid_nb2grid_idx int64[B, 27]; every cell of a listed
+ * block takes part.  inputs, outputs: [B, G^3, E], 16-byte aligned; weights
+ * [W^3, E]; listed: one scratch byte per block.  For the sizes that
+ * ash_convolution_cube_supported says (non-zero): float32, G = 8, windows of 3,
+ * 5 and 7, up to 8 channels and 4 GiB. */
+int ash_convolution_cube_supported(int64_t num_embeddings, int grid_dim, int window,
+                                   int64_t embedding_dim, int32_t dtype);
+int ash_convolution_cube(const void* inputs, const void* weights,
+                         const int64_t* grid_indices, const int64_t* lut_grid_nb2grid_idx,
+                         void* outputs, int64_t num_grids, int64_t num_embeddings,
+                         int grid_dim, int window, int64_t embedding_dim, int32_t dtype,
+                         uint8_t* listed, void* stream);
+
 /* Replace the two launches of `isosurface_extraction` (ash/src/grid.cu:453-602,
  * pybind.cpp:30; the reference counts, allocates and runs the same kernel again
  * to fill).  sdfs / weights scalar[num_embeddings, cells_per_grid];

@@ -1,0 +1,50 @@
+"""ash_convolution_cube against the kernels that go by the per-cell tables
+(ash_convolution_forward): the same taps in the same order, so bit for bit."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+def _grid(gpu_ash, channels, blocks, seed):
+    grid = gpu_ash.SparseDenseGrid(3, blocks + 9, channels, 8, device=DEV)
+    g = torch.Generator().manual_seed(seed)
+    # a clump (inner blocks have all neighbours) and loners
+    keys = torch.unique(torch.randint(0, 5, (3 * blocks, 3), generator=g), dim=0)[: max(1, blocks - 5)]
+    keys = torch.cat([keys, torch.tensor([[50, 0, 0], [0, 50, 0], [0, 51, 1], [-7, 0, 3]])])[:blocks]
+    grid.engine.insert_keys(keys.int().to(DEV))
+    with torch.no_grad():
+        grid.embeddings.copy_(torch.randn(grid.embeddings.shape, generator=g))
+    return grid, g
+
+
+@pytest.mark.parametrize("window", [3, 5, 7])
+@pytest.mark.parametrize("channels", [1, 2, 3, 4, 5, 6, 7, 8])
+def test_cube_equals_tables(gpu_ash, channels, window):
+    backend = gpu_ash.grid.backend
+    grid, g = _grid(gpu_ash, channels, 90, seed=channels * 10 + window)
+    weights = torch.randn(window, window, window, channels, generator=g).to(DEV)
+    c2g, c2c, lut = grid._window_tables(window // 2)
+    _, listed = grid.engine.items()
+    for rows in (listed, listed[::3].contiguous(), listed[:1], listed[:0]):
+        got = backend.convolution_cube(grid.embeddings.data, weights, rows, lut, 8)
+        want = backend.convolution_forward(
+            grid.embeddings.data, weights.view(-1, channels),
+            torch.ones(len(rows), 512, dtype=torch.bool, device=DEV), rows, grid.cell_indices, lut, c2c,
+            c2g, 8)
+        assert torch.equal(got, want)
+    assert float(want.abs().sum()) == 0     # nothing listed: all rows cleared
+    assert torch.equal(grid.convolution(grid.embeddings.data, weights),
+                       backend.convolution_cube(grid.embeddings.data, weights, listed, lut, 8))
+
+
+def test_sizes_left_to_the_other_kernels(gpu_ash):
+    backend = gpu_ash.grid.backend
+    supported = backend.lib.ash_convolution_cube_supported
+    assert supported(262_143, 8, 3, 8, 0) and not supported(262_144, 8, 3, 8, 0)   # 4 GiB
+    assert not supported(10, 4, 3, 4, 0) and not supported(10, 8, 9, 4, 0)
+    assert not supported(10, 8, 3, 9, 0) and not supported(10, 8, 3, 4, 1)
+    grid, g = _grid(gpu_ash, 9, 70, seed=1)
+    out = grid.convolution(grid.embeddings.data, torch.randn(3, 3, 3, 9, generator=g).to(DEV))
+    assert out.shape == grid.embeddings.shape and float(out.detach().abs().sum()) > 0

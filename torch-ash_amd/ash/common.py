@@ -249,6 +249,13 @@ _SIGNATURES = {
         ctypes.c_int,
         [_PTR] * 9 + [_I64] * 6 + [ctypes.c_int32, _PTR, _PTR],
     ),
+    "ash_convolution_cube_supported": (
+        ctypes.c_int, [_I64, ctypes.c_int, ctypes.c_int, _I64, ctypes.c_int32]
+    ),
+    "ash_convolution_cube": (
+        ctypes.c_int,
+        [_PTR] * 5 + [_I64, _I64, ctypes.c_int, ctypes.c_int, _I64, ctypes.c_int32, _PTR, _PTR],
+    ),
     "ash_marching_cubes_workspace_ints": (ctypes.c_int64, [_I64, _I64]),
     "ash_marching_cubes_classify": (
         ctypes.c_int,
@@ -520,6 +527,39 @@ class _Backend:
                     _DTYPE[inputs.dtype], listed.data_ptr(), _stream_of(dev),
                 )
             )
+        return outputs
+
+    def convolution_cube(self, inputs, weights, grid_indices, lut_grid_nb2grid_idx, grid_dim):
+        """convolution_forward of every cell of the listed blocks for a cube
+        window and the tables that SparseDenseGrid builds (of which only the
+        per-block one is needed), or None for sizes that
+        `convolution_forward` takes."""
+        b, m, e = inputs.shape
+        window = weights.shape[0]
+        if inputs.dtype not in _DTYPE or not self.lib.ash_convolution_cube_supported(
+            b, grid_dim, window, e, _DTYPE[inputs.dtype]
+        ) or inputs.data_ptr() % 16:
+            return None
+        _require_hip(inputs, "inputs")
+        dev = inputs.device
+        if not inputs.is_contiguous() or m != grid_dim**3:
+            raise RuntimeError("inputs must be contiguous (B, grid_dim^3, E)")
+        weights = weights.to(dev, inputs.dtype).contiguous()
+        if weights.shape != (window, window, window, e):
+            raise RuntimeError(f"weights must be ({window}, {window}, {window}, {e})")
+        lut_g = lut_grid_nb2grid_idx.to(dev, torch.int64).contiguous()
+        if lut_g.shape != (b, 27):
+            raise RuntimeError("neighbour table does not match the inputs")
+        gi = grid_indices.reshape(-1).to(dev, torch.int64).contiguous()
+        outputs = torch.empty_like(inputs)
+        listed = torch.empty(b, dtype=torch.uint8, device=dev)
+        self.check(
+            self.lib.ash_convolution_cube(
+                inputs.data_ptr(), weights.data_ptr(), gi.data_ptr(), lut_g.data_ptr(),
+                outputs.data_ptr(), gi.numel(), b, grid_dim, window, e, _DTYPE[inputs.dtype],
+                listed.data_ptr(), _stream_of(dev),
+            )
+        )
         return outputs
 
     # -- rays (ash/src/pybind.cpp:35-37) ----------------------------------

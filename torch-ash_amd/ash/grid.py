@@ -569,8 +569,13 @@ class SparseDenseGrid(ASHModule):
         assert weights.shape[3] == inputs.shape[-1]
         assert weights.device == inputs.device
 
-        lut_cell_nb2grid_nb, lut_cell_nb2cell_idx, lut_grid_nb2grid_idx = self._window_tables(radius)
         _, grid_indices = self._blocks_in_spatial_order()
+        if hasattr(backend, "convolution_cube") and 1 <= radius <= self.grid_dim:
+            outputs = backend.convolution_cube(inputs, weights, grid_indices,
+                                               self._window_block_table(radius), self.grid_dim)
+            if outputs is not None:
+                return outputs
+        lut_cell_nb2grid_nb, lut_cell_nb2cell_idx, lut_grid_nb2grid_idx = self._window_tables(radius)
         cell_indices = self.cell_indices
         num_cell_nbs = lut_cell_nb2grid_nb.shape[1]
         return backend.convolution_forward(
@@ -586,26 +591,24 @@ class SparseDenseGrid(ASHModule):
         )
 
     def _window_tables(self, radius: int):
-        """The three tables of a (2 radius + 1)^3 window: the per-cell pair
-        depends on the block size alone and is built once per radius, the
-        per-block one is kept while the table holds the same keys (as the
-        Z-order listing)."""
-        cell_tables = getattr(self, "_window_cell_tables", None)
-        if cell_tables is None:
-            cell_tables = self._window_cell_tables = {}
-        if radius not in cell_tables:
-            cell_tables[radius] = self.construct_cell_neighbor_lut(radius, bidirectional=True)
-        lut_cell_nb2grid_nb, lut_cell_nb2cell_idx = cell_tables[radius]
+        """The three tables of a (2 radius + 1)^3 window; the per-cell pair
+        depends on the block size alone and is built once per radius."""
+        kept = self.__dict__.setdefault("_kept_cell_tables", {})
+        if radius not in kept:
+            kept[radius] = self.construct_cell_neighbor_lut(radius, bidirectional=True)
+        return (*kept[radius], self._window_block_table(radius))
+
+    def _window_block_table(self, radius: int):
+        """The per-block table of such a window, kept while the table holds the
+        same keys (as the Z-order listing)."""
         grid_radius = (radius + self.grid_dim - 1) // self.grid_dim
         table = self.engine.backend
         stamp = (id(table), getattr(table, "version", None), grid_radius)
-        cached = getattr(self, "_window_block_table", None)
-        if stamp[1] is not None and cached is not None and cached[0] == stamp:
-            lut_grid_nb2grid_idx = cached[1]
-        else:
-            _, lut_grid_nb2grid_idx = self.construct_grid_neighbor_lut(grid_radius, bidirectional=True)
-            self._window_block_table = (stamp, lut_grid_nb2grid_idx)
-        return lut_cell_nb2grid_nb, lut_cell_nb2cell_idx, lut_grid_nb2grid_idx
+        kept = getattr(self, "_kept_block_table", None)
+        if stamp[1] is None or kept is None or kept[0] != stamp:
+            _, lut = self.construct_grid_neighbor_lut(grid_radius, bidirectional=True)
+            kept = self._kept_block_table = (stamp, lut)
+        return kept[1]
 
     @torch.no_grad()
     def isosurface_points(

@@ -20,11 +20,12 @@ OUT = os.path.join(OUT_DIR, "libash_hip.so")
 HOST_SOURCE = os.path.join(CSRC, "ash_host.cpp")
 HOST_OUT = os.path.join(OUT_DIR, "_ash_host.so")
 SOURCES = ["ash_map.hip", "ash_bulk.hip", "ash_query.hip", "ash_fusion.hip", "ash_mesh.hip",
-           "ash_rays.hip"]
+           "ash_rays.hip", "ash_conv.hip"]
 HEADERS = [
     os.path.join(CSRC, "ash_probe.h"),
     os.path.join(CSRC, "ash_dev.h"),
     os.path.join(CSRC, "ash_table.h"),
+    os.path.join(CSRC, "ash_walk.h"),
     os.path.join(CSRC, "ash_mc_table.h"),
     os.path.join(HERE, os.pardir, "include", "ash_hip.h"),
 ]

@@ -1,0 +1,397 @@
+// Sparse convolution over blocks of 8^3 cells with a cube window, for rows of up
+// to eight float32 channels: the case of SparseDenseGrid.convolution and
+// gaussian_filter_ on the grids of the demos (ash/src/grid.cu:948-1043;
+// ash_query.hip holds the kernels for every other shape).
+//
+// The layout is the one the Python layer builds (cell c = x + 8 y + 64 z; tap k =
+// (dx + r) + W (dy + r) + W^2 (dz + r); neighbour block (bx + 1) + 3 (by + 1) + 9
+// (bz + 1)), so no per-cell table is read, checked or needed.
+//
+// Two wavefronts per channel, lane = (x, z), four cells along y per lane: the
+// channels of a block are an even load whatever their number (five channels in
+// instances for eight left three quarters of the second turn idle), a row of
+// the tile is read once for all cells that need it, and a tap's weight is one
+// scalar for the wavefront.  (Eight cells per lane read the tile less often but
+// hold twice the elements in flight: the same time for windows of 3, 1.4 times
+// for windows of 7.)  Every cell still sees its taps in table order, one fused
+// multiply-add per tap, as in the other kernels.
+//
+// 60 000 blocks, tables and instances for powers of two before: five channels
+// 3^3 1275 -> 490 us, 7^3 4.3 -> 3.8 ms; two channels 501 -> 179 us, 2.2 -> 1.0
+// ms; 1000 blocks, 7^3: 990 -> 95 us (every workgroup used to check the tables).
+// 3^3 windows of five channels move 1.55 GB beyond the L2s (the halo along x
+// takes most lines of two neighbours), 3.2 TB/s; 7^3 are bound by vector
+// instructions.
+//
+// The block's own rows are contiguous in memory whatever their width: they come
+// in as two 16-byte pieces per thread, and leave the same way, through LDS.
+// The halo comes element by element (consecutive lanes, consecutive words of a
+// row).  Where an element goes in the tile never changes from block to block
+// and is kept in registers.  Software pipeline: while a block is computed the
+// next block's elements are on their way into registers and the row numbers of
+// the one after are fetched.  Rows of missing blocks are staged as zeros (with
+// finite weights adding 0 * w leaves a sum as it is).
+#include "ash_table.h"
+#include "ash_walk.h"
+
+#include "../../include/ash_hip.h"
+
+namespace ash {
+namespace {
+
+constexpr int kG = 8;
+constexpr int kM = kG * kG * kG;
+constexpr int kMaxChannels = 8;
+constexpr int kY = 4;   // cells along y per lane
+constexpr int kFillBlock = 256;
+
+template <int E, int W>
+struct Shape {
+    static constexpr int kParts = kG / kY;                         // wavefronts per channel
+    static constexpr int kThreads = 64 * E * kParts;
+    static constexpr int kOwnEach = kM * E / 4 / kThreads;        // 16-byte pieces per thread
+    static constexpr int kR = W / 2;
+    static constexpr int kT = kG + 2 * kR;
+    // words between the z layers of a channel's plane: 8 or 24 modulo 32, so
+    // that the four groups of lanes (eight words along x, one z each) that are
+    // served together meet different banks
+    static constexpr int layer() {
+        int p = kT * kT;
+        while (p % 32 != 8 && p % 32 != 24) ++p;
+        return p;
+    }
+    static constexpr int kLayer = layer();
+    static constexpr int kPlane = kLayer * kT;
+    static constexpr int kHalo = kT * kT * kT - kM;               // rows
+    static constexpr int kHaloEach = (kHalo * E + kThreads - 1) / kThreads;   // elements per thread
+    static constexpr int kTaps = W * W;                           // of one dz
+    // results on their way out: a z layer's rows, four words apart from the next
+    // layer's (banks)
+    static constexpr int kOutLayer = 64 * E + 4;
+    static constexpr int kTileWords = E * kPlane;
+    static constexpr int kOutWords = kG * kOutLayer;
+    static constexpr int kWeightWords = E * W * 64;
+    // wavefronts per SIMD that the tile leaves room for
+    static constexpr int kMostWaves = W == 3 ? 6 : 5;
+    static constexpr int waves() {
+        const int lds = 4 * (kTileWords + kOutWords + kWeightWords) + 1024;
+        const int fit = (160 * 1024 / lds * E * kParts + 3) / 4;
+        return fit < 1 ? 1 : (fit > kMostWaves ? kMostWaves : fit);
+    }
+};
+
+struct ConvArgs {
+    const float* in;
+    const float* w;
+    const int64_t* grid_indices;
+    const int64_t* lut_g;   // [B, 27]
+    float* out;
+    int64_t n_grids, B;
+};
+
+template <int E, int W>
+__global__ __launch_bounds__((Shape<E, W>::kThreads), (Shape<E, W>::waves())) void
+convolution_block8_kernel(ConvArgs a) {
+    using S = Shape<E, W>;
+    typedef float v4 __attribute__((ext_vector_type(4)));
+    __shared__ __align__(16) float s_tile[S::kTileWords];
+    __shared__ __align__(16) float s_out[S::kOutWords];
+    __shared__ float s_w[S::kWeightWords];
+    __shared__ int32_t s_nb[2][28];   // rows of the 27 neighbour blocks, and the block's own
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q = wave / S::kParts;             // the wavefront's channel
+    const int y0 = wave % S::kParts * kY;        // and the first of its cells along y
+    constexpr int R = S::kR, T = S::kT;
+
+    // weights by channel and dz, one tap per lane
+    for (int t = tid; t < S::kWeightWords; t += S::kThreads) {
+        const int tap = t & 63;
+        const int dz = (t >> 6) % W;
+        const int ch = (t >> 6) / W;
+        s_w[t] = tap < S::kTaps ? a.w[(dz * S::kTaps + tap) * E + ch] : 0.f;
+    }
+    // Where this thread's elements of the block's own rows go in the tile
+    uint32_t own_dst[S::kOwnEach][2];   // two 16-bit places per word
+#pragma unroll
+    for (int i = 0; i < S::kOwnEach; ++i) {
+        uint32_t place[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int e = 4 * (tid + i * S::kThreads) + c;
+            const int cell = e / E;
+            place[c] = static_cast<uint32_t>((e - cell * E) * S::kPlane + (cell & 7) + R +
+                                             T * (((cell >> 3) & 7) + R) +
+                                             S::kLayer * ((cell >> 6) + R));
+        }
+        own_dst[i][0] = place[0] | (place[1] << 16);
+        own_dst[i][1] = place[2] | (place[3] << 16);
+    }
+    // and its elements of the halo: place in the tile << 17 | neighbour << 12 |
+    // word within that block's rows
+    constexpr uint32_t kNone = 0xFFFFFFFFu;
+    uint32_t halo[S::kHaloEach];
+#pragma unroll
+    for (int i = 0; i < S::kHaloEach; ++i) {
+        const int h = tid + i * S::kThreads;
+        halo[i] = kNone;
+        if (h < S::kHalo * E) {
+            int p = h / E;
+            const int ch = h - p * E;
+            int at[3];   // tile coordinates of the p-th row of the halo
+            constexpr int kSlab = T * T, kRing = T * T - kG * kG;
+            if (p < 2 * R * kSlab) {
+                at[2] = p / kSlab;
+                if (at[2] >= R) at[2] += kG;
+                p %= kSlab;
+                at[1] = p / T;
+                at[0] = p % T;
+            } else {
+                p -= 2 * R * kSlab;
+                at[2] = R + p / kRing;
+                p %= kRing;
+                if (p < 2 * R * T) {
+                    at[1] = p / T;
+                    if (at[1] >= R) at[1] += kG;
+                    at[0] = p % T;
+                } else {
+                    p -= 2 * R * T;
+                    at[1] = R + p / (2 * R);
+                    at[0] = p % (2 * R);
+                    if (at[0] >= R) at[0] += kG;
+                }
+            }
+            int nb = 0, cell = 0, step3 = 1, step8 = 1;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                const int b = at[d] < R ? -1 : (at[d] >= R + kG ? 1 : 0);
+                nb += (b + 1) * step3;
+                cell += (at[d] - R - b * kG) * step8;
+                step3 *= 3;
+                step8 *= kG;
+            }
+            halo[i] = (static_cast<uint32_t>(ch * S::kPlane + at[0] + T * at[1] + S::kLayer * at[2]) << 17) |
+                      static_cast<uint32_t>(nb << 12) | static_cast<uint32_t>(cell * E + ch);
+        }
+    }
+
+    const TileWalk walk(a.n_grids);
+    auto fetch_rows = [&](int64_t b) -> int32_t {   // lanes 0..26 neighbours, 27 the block
+        if (tid > 27 || b >= walk.end) return -1;
+        const int64_t g = a.grid_indices[b];
+        if (g < 0 || g >= a.B) return -1;
+        if (tid == 27) return static_cast<int32_t>(g);
+        const int64_t row = a.lut_g[g * 27 + tid];
+        return (row >= 0 && row < a.B) ? static_cast<int32_t>(row) : -1;
+    };
+    // (byte offsets fit 32 bits: the tensors are below 4 GiB, which the host
+    // checks; one register per address and no 64-bit arithmetic.  Words of
+    // missing blocks are read from the start of the tensor and dropped.)
+    v4 own[S::kOwnEach];
+    float ring[S::kHaloEach];
+    uint64_t have = 0;   // bit i: ring[i] holds a word of a stored block
+    const char* const in = reinterpret_cast<const char*>(a.in);
+    constexpr uint32_t kBlockBytes = kM * E * 4;
+    auto load_block = [&](const int32_t* nb) {
+        const uint32_t g = nb[27] < 0 ? 0u : static_cast<uint32_t>(nb[27]);
+#pragma unroll
+        for (int i = 0; i < S::kOwnEach; ++i) {
+            own[i] = *reinterpret_cast<const v4*>(in + (g * kBlockBytes +
+                                                        16u * static_cast<uint32_t>(tid + i * S::kThreads)));
+        }
+        have = 0;
+#pragma unroll
+        for (int i = 0; i < S::kHaloEach; ++i) {
+            const int32_t row = halo[i] == kNone ? -1 : nb[(halo[i] >> 12) & 31u];
+            const uint32_t at = row < 0 ? 0u : static_cast<uint32_t>(row) * kBlockBytes + (halo[i] & 0xFFFu) * 4u;
+            if (row >= 0) have |= uint64_t{1} << i;
+            ring[i] = *reinterpret_cast<const float*>(in + at);
+        }
+    };
+
+    int64_t blk = walk.next;
+    int buf = 0;
+    int32_t rows_reg = fetch_rows(blk);
+    if (tid <= 27) s_nb[0][tid] = rows_reg;
+    rows_reg = fetch_rows(blk + walk.step);
+    __syncthreads();
+    if (blk < walk.end) load_block(s_nb[0]);
+    const int x = lane & 7, z = lane >> 3;
+    const float* const window = s_tile + q * S::kPlane + x + T * y0 + S::kLayer * z;
+    float* const result = s_out + (x + kG * y0) * E + z * S::kOutLayer + q;
+
+    for (; blk < walk.end; blk += walk.step, buf ^= 1) {
+        const int32_t g = s_nb[buf][27];
+#pragma unroll
+        for (int i = 0; i < S::kOwnEach; ++i) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) s_tile[(own_dst[i][c >> 1] >> (16 * (c & 1))) & 0xFFFFu] = own[i][c];
+        }
+#pragma unroll
+        for (int i = 0; i < S::kHaloEach; ++i) {
+            if (halo[i] != kNone) s_tile[halo[i] >> 17] = ((have >> i) & 1u) ? ring[i] : 0.f;
+        }
+        if (tid <= 27) s_nb[buf ^ 1][tid] = rows_reg;
+        __syncthreads();   // the tile is complete
+        rows_reg = fetch_rows(blk + 2 * walk.step);
+        if (blk + walk.step < walk.end) load_block(s_nb[buf ^ 1]);
+
+        float acc[kY];
+#pragma unroll
+        for (int j = 0; j < kY; ++j) acc[j] = 0.f;
+#pragma unroll 1
+        for (int dz = 0; dz < W; ++dz) {
+            const float* layer = window + S::kLayer * dz;
+            const float taps = s_w[(q * W + dz) * 64 + lane];
+#pragma unroll
+            for (int y = 0; y < kY + 2 * R; ++y) {
+                float row[W];
+#pragma unroll
+                for (int dx = 0; dx < W; ++dx) row[dx] = layer[T * y + dx];
+#pragma unroll
+                for (int j = 0; j < kY; ++j) {
+                    const int dy = y - j;
+                    if (dy < 0 || dy >= W) continue;
+#pragma unroll
+                    for (int dx = 0; dx < W; ++dx) {
+                        const float tap = __int_as_float(
+                                __builtin_amdgcn_readlane(__float_as_int(taps), dy * W + dx));
+                        acc[j] = fmaf(row[dx], tap, acc[j]);
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < kY; ++j) result[j * kG * E] = acc[j];
+        __syncthreads();   // the results are complete, and the tile has been read
+        if (g >= 0) {
+            v4* rows = reinterpret_cast<v4*>(a.out) +
+                       static_cast<uint64_t>(static_cast<uint32_t>(g)) * (kM * E / 4);
+#pragma unroll
+            for (int i = 0; i < S::kOwnEach; ++i) {
+                const int f = tid + i * S::kThreads;
+                const int out_z = f / (16 * E);
+                rows[f] = *reinterpret_cast<const v4*>(s_out + 4 * f + 4 * out_z);
+            }
+        }
+    }
+}
+
+// listed[b] = 1 for every block of the listing.
+__global__ __launch_bounds__(kFillBlock) void mark_kernel(const int64_t* __restrict__ grid_indices,
+                                                          int64_t n, int64_t B,
+                                                          uint8_t* __restrict__ listed) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kFillBlock + threadIdx.x;
+    if (i >= n) return;
+    const int64_t g = grid_indices[i];
+    if (g >= 0 && g < B) listed[g] = 1;
+}
+
+__global__ __launch_bounds__(kFillBlock) void clear_marks_kernel(uint8_t* __restrict__ listed, int64_t B) {
+    const int64_t i = (static_cast<int64_t>(blockIdx.x) * kFillBlock + threadIdx.x) * 4;
+    for (int64_t b = i; b < i + 4 && b < B; ++b) listed[b] = 0;
+}
+
+// Zeroes the rows of the blocks that are not listed, one workgroup per block at
+// a time.
+__global__ __launch_bounds__(kFillBlock) void zero_others_kernel(uint4* __restrict__ out,
+                                                                 const uint8_t* __restrict__ listed,
+                                                                 int64_t B, int64_t units) {
+    for (int64_t b = blockIdx.x; b < B; b += gridDim.x) {
+        if (listed[b]) continue;   // the same for the whole workgroup
+        uint4* rows = out + b * units;
+        for (int64_t u = threadIdx.x; u < units; u += kFillBlock) rows[u] = make_uint4(0u, 0u, 0u, 0u);
+    }
+}
+
+template <int E, int W>
+int launch(const ConvArgs& a, hipStream_t s) {
+    // as many workgroups as the device holds at once: they walk the listing
+    static const int per_cu = [] {
+        int n = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                    &n, convolution_block8_kernel<E, W>, Shape<E, W>::kThreads, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            n = 1;
+        }
+        return n < 1 ? 1 : n;
+    }();
+    int64_t groups = static_cast<int64_t>(per_cu) * 256;
+    if (groups > a.n_grids) groups = a.n_grids;
+    convolution_block8_kernel<E, W><<<static_cast<unsigned>(groups), Shape<E, W>::kThreads, 0, s>>>(a);
+    ASH_LAUNCH_CHECK();
+    return 0;
+}
+
+template <int E>
+int launch_window(const ConvArgs& a, int window, hipStream_t s) {
+    switch (window) {
+        case 3: return launch<E, 3>(a, s);
+        case 5: return launch<E, 5>(a, s);
+        default: return launch<E, 7>(a, s);
+    }
+}
+
+}  // namespace
+}  // namespace ash
+
+using namespace ash;
+
+extern "C" {
+
+int ash_convolution_cube_supported(int64_t num_embeddings, int grid_dim, int window,
+                                   int64_t embedding_dim, int32_t dtype) {
+    return dtype == ASH_F32 && grid_dim == kG && (window == 3 || window == 5 || window == 7) &&
+           embedding_dim >= 1 && embedding_dim <= kMaxChannels && num_embeddings >= 1 &&
+           num_embeddings * embedding_dim * kM * 4 <= 0xFFFFFFFFll;
+}
+
+int ash_convolution_cube(const void* inputs, const void* weights, const int64_t* grid_indices,
+                         const int64_t* lut_grid_nb2grid_idx, void* outputs, int64_t num_grids,
+                         int64_t num_embeddings, int grid_dim, int window, int64_t embedding_dim,
+                         int32_t dtype, uint8_t* listed, void* stream) {
+    if (num_grids < 0 || num_embeddings < 1) ASH_FAIL("convolution_cube: bad sizes");
+    if (!ash_convolution_cube_supported(num_embeddings, grid_dim, window, embedding_dim, dtype)) {
+        ASH_FAIL("convolution_cube takes float32 blocks of 8^3 cells, windows of 3, 5 or 7, up to 8 "
+                 "channels and up to 4 GiB");
+    }
+    if (inputs == nullptr || weights == nullptr || lut_grid_nb2grid_idx == nullptr ||
+        outputs == nullptr || listed == nullptr || (num_grids > 0 && grid_indices == nullptr)) {
+        ASH_FAIL("null pointer in convolution_cube");
+    }
+    if ((reinterpret_cast<uintptr_t>(inputs) | reinterpret_cast<uintptr_t>(outputs)) % 16 != 0) {
+        ASH_FAIL("convolution_cube: inputs and outputs must be 16-byte aligned");
+    }
+    PointerGuard guard;
+    ASH_HIP(guard.enter_for(inputs));
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const int64_t B = num_embeddings;
+    clear_marks_kernel<<<static_cast<unsigned>((B + 4 * kFillBlock - 1) / (4 * kFillBlock)), kFillBlock, 0, s>>>(
+            listed, B);
+    ASH_LAUNCH_CHECK();
+    if (num_grids > 0) {
+        mark_kernel<<<static_cast<unsigned>((num_grids + kFillBlock - 1) / kFillBlock), kFillBlock, 0, s>>>(
+                grid_indices, num_grids, B, listed);
+        ASH_LAUNCH_CHECK();
+    }
+    zero_others_kernel<<<static_cast<unsigned>(B < 8192 ? B : 8192), kFillBlock, 0, s>>>(
+            static_cast<uint4*>(outputs), listed, B, kM * embedding_dim / 4);
+    ASH_LAUNCH_CHECK();
+    if (num_grids == 0) return 0;
+    const ConvArgs a = {static_cast<const float*>(inputs), static_cast<const float*>(weights),
+                        grid_indices, lut_grid_nb2grid_idx, static_cast<float*>(outputs),
+                        num_grids, num_embeddings};
+    switch (embedding_dim) {
+        case 1: return launch_window<1>(a, window, s);
+        case 2: return launch_window<2>(a, window, s);
+        case 3: return launch_window<3>(a, window, s);
+        case 4: return launch_window<4>(a, window, s);
+        case 5: return launch_window<5>(a, window, s);
+        case 6: return launch_window<6>(a, window, s);
+        case 7: return launch_window<7>(a, window, s);
+        default: return launch_window<8>(a, window, s);
+    }
+}
+
+}  // extern "C"

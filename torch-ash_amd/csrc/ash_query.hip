@@ -25,6 +25,7 @@
 // a wavefront that hit the same row are summed in registers first and issue
 // one atomic per run (ray-ordered samples produce long runs).
 #include "ash_probe.h"
+#include "ash_walk.h"
 
 #include <type_traits>
 
@@ -39,7 +40,6 @@ namespace ash {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kXcds = 8;
 constexpr int64_t kMaxLdsCells = 2048;  // 2048 * 8 * 3 B = 48 KiB
 constexpr uint32_t kNoRow = 0xFFFFFFFFu;
 constexpr int kLdsPerCu = 160 * 1024;
@@ -178,24 +178,6 @@ __host__ __device__ inline size_t table_offset(const QDev& a, int lpq, bool lds_
     if (lds_lut) bytes += static_cast<size_t>(a.M) * 8 * 3;
     return (bytes + 15) & ~static_cast<size_t>(15);
 }
-
-// Tile walk: workgroup w serves XCD (w mod 8); each XCD owns a contiguous
-// eighth of the tiles and its workgroups stride through it.
-struct TileWalk {
-    int64_t next;
-    int64_t end;
-    int64_t step;
-    __device__ __forceinline__ TileWalk(int64_t ntiles) {
-        const int64_t per_xcd = (ntiles + kXcds - 1) / kXcds;
-        const int xcd = blockIdx.x % kXcds;
-        const int slot = blockIdx.x / kXcds;
-        step = (gridDim.x + kXcds - 1 - xcd) / kXcds;  // workgroups on this XCD
-        next = xcd * per_xcd + slot;
-        end = (xcd + 1) * per_xcd;
-        if (end > ntiles) end = ntiles;
-        if (step < 1) step = 1;
-    }
-};
 
 // What a query brings.  The mask, the indices and the offsets are asked for
 // together (one trip to memory, not two); what a masked query has there is read

@@ -501,6 +501,16 @@ int ash_map_items(ash_map_t* map, int32_t* keys_out, int64_t* indices_out,
  * state only, no synchronisation.  No counterpart in the reference. */
 int ash_map_items_in_index_order(ash_map_t* map, int* dense);
 
+/* The per-block neighbour table of a map with three-dimensional keys
+ * (ash/grid.py:566-617, there a listing, a find and two scatters): row i < num_rows
+ * belongs to index i; coords int32[num_rows, 3] its key, lut int64[num_rows, W^3]
+ * the indices of the keys at its offsets, -1 for rows without a key and for keys
+ * that are not stored.  W = radius + 1, or 2 radius + 1 when bidirectional
+ * (radius 0..15); offset k = (k % W, k / W % W, k / W^2), less `radius` each when
+ * bidirectional.  No synchronisation. */
+int ash_map_neighbors(ash_map_t* map, int64_t num_rows, int radius, int bidirectional,
+                      int32_t* coords, int64_t* lut, void* stream);
+
 /* Replaces `HashMap::load_states` (ash/src/hashmap_gpu.cuh:407-450): the map
  * is emptied, then (keys[i] -> indices[i]) are stored, size := n and the heap
  * := heap_src (skipped when heap_src is NULL or already the map's heap). */

@@ -194,6 +194,8 @@ _SIGNATURES = {
     "ash_map_counters": (ctypes.c_int, [_PTR, _PTR, ctypes.POINTER(_I64), _PTR]),
     "ash_map_counters_pending": (ctypes.c_int, [_PTR]),
     "ash_map_known_size": (ctypes.c_int, [_PTR, ctypes.POINTER(_I64)]),
+    "ash_map_neighbors": (
+        ctypes.c_int, [_PTR, _I64, ctypes.c_int, ctypes.c_int, _PTR, _PTR, _PTR]),
     "ash_map_set_staging": (ctypes.c_int, [_PTR, _PTR]),
     "ash_map_insert_scratch_bytes": (
         ctypes.c_int,
@@ -1368,6 +1370,17 @@ class _HashMap:
                 f"load_states: {refused} pairs were refused (duplicate keys, or indices / heap "
                 "entries outside the capacity); nothing was loaded"
             )
+    def neighbor_rows(
+        self, num_rows: int, radius: int, bidirectional: bool
+    ) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
+        """(coords int32 (num_rows, 3), lut int64 (num_rows, K)): key of every
+        index and the indices of the keys at its offsets, -1 where there are
+        none; None for windows that one launch does not take."""
+        if self.key_dim != 3 or not 0 <= radius <= 15:
+            return None
+        return self._backend.host.neighbors(self._address, self._index, num_rows, radius,
+                                            bool(bidirectional))
+
 
 
 class _MissingBackend:

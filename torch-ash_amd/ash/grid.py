@@ -766,6 +766,12 @@ class SparseDenseGrid(ASHModule):
 
         grid_coords[active_indices] = active_coords
         lut[active_indices] = nb_indices.view(-1, num_nbs)
+        table = self.engine.backend
+        tables = (table.neighbor_rows(self.num_embeddings, radius, bidirectional)
+                  if hasattr(table, "neighbor_rows") else None)
+        if tables is not None:
+            return tables
+
         return grid_coords, lut
 
     @torch.no_grad()

@@ -40,6 +40,7 @@ namespace py = pybind11;
     X(ash_map_items)                                                                  \
     X(ash_map_counters)                                                               \
     X(ash_map_upkeep)                                                                 \
+    X(ash_map_neighbors)                                                              \
     X(ash_grid_fuse_frame)                                                            \
     X(ash_ray_find_near_far_world)                                                    \
     X(ash_ray_sample_groups)                                                          \
@@ -365,6 +366,17 @@ std::tuple<Tensor, Tensor> items(uintptr_t handle, int64_t dim, int64_t device, 
 // ---------------------------------------------------------------------- grid
 Tensor positions_of(const Tensor& x) {
     need(x.dim() == 2 && x.size(1) == 3 && x.scalar_type() == at::kFloat, "positions must be float32 (N, 3)");
+// (coords (rows, 3), lut (rows, K)) of the keys at offsets within `radius`
+std::pair<Tensor, Tensor> neighbors(uintptr_t handle, int64_t device, int64_t rows, int radius,
+                                    bool bidirectional) {
+    const int64_t width = bidirectional ? 2 * radius + 1 : radius + 1;
+    const Tensor coords = empty({rows, 3}, at::kInt, device);
+    const Tensor lut = empty({rows, width * width * width}, at::kLong, device);
+    check(lib.ash_map_neighbors(map_of(handle), rows, radius, bidirectional, ptr<int32_t>(coords),
+                                ptr<int64_t>(lut), stream_of(device)));
+    return {coords, lut};
+}
+
     return x.contiguous();
 }
 
@@ -732,3 +744,4 @@ PYBIND11_MODULE(_ash_host, m) {
     m.def("query_backward_forward", &query_backward_forward);
     m.def("query_backward_backward", &query_backward_backward);
 }
+    m.def("neighbors", &neighbors);

@@ -721,6 +721,35 @@ int ash_convolution_cube(const void* inputs, const void* weights,
                          int grid_dim, int window, int64_t embedding_dim, int32_t dtype,
                          uint8_t* listed, void* stream);
 
+/* The triangle mesh of ash_marching_cubes_* for blocks of 8^3 cells and the
+ * tables that SparseDenseGrid builds (cell c = x + 8 y + 64 z, neighbour row
+ * dx + 2 dy + 4 dz of lut_grid_nb2grid_idx int64[B, 8]), with the same numbering.
+ * The value of cell c of row g lies at sdfs[(g * 512 + c) * sdf_stride], its
+ * weight likewise (strides in elements, 1..64): channels of wider rows need no
+ * copy.  Blocks that the listing does not name count as missing.
+ *
+ *   workspace: ash_surface_block8_workspace_bytes bytes, 16-byte aligned, handed
+ *   from the first call to the second; out[2] = number of vertices, of triangles.
+ *
+ * The first call waits for the device (`map` lends the place where the numbers
+ * arrive).  The second writes positions float32[n_vertices, 3] -- cell units, or
+ * with to_world cell * cell_to_world (+ origin float32[3], may be NULL), rounded
+ * after either step -- and triangles int32[n_triangles, 3]. */
+int64_t ash_surface_block8_workspace_bytes(int64_t num_grids, int64_t num_embeddings);
+int ash_surface_block8_classify(ash_map_t* map, const void* sdfs, int64_t sdf_stride,
+                                const void* weights, int64_t weight_stride,
+                                const int64_t* grid_indices, const int64_t* lut_grid_nb2grid_idx,
+                                int64_t num_grids, int64_t num_embeddings, float iso_value,
+                                float weight_thr, int32_t dtype, void* workspace, int64_t out[2],
+                                void* stream);
+int ash_surface_block8_extract(const void* sdfs, int64_t sdf_stride, const int64_t* grid_indices,
+                               const int32_t* grid_coords_table,
+                               const int64_t* lut_grid_nb2grid_idx, int64_t num_grids,
+                               int64_t num_embeddings, float iso_value, int32_t dtype,
+                               void* workspace, int64_t n_vertices, int64_t n_triangles,
+                               int to_world, float cell_to_world, const float* origin,
+                               float* positions, int32_t* triangles, void* stream);
+
 /* Replace the two launches of `isosurface_extraction` (ash/src/grid.cu:453-602,
  * pybind.cpp:30; the reference counts, allocates and runs the same kernel again
  * to fill).  sdfs / weights scalar[num_embeddings, cells_per_grid];

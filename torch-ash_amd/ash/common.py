@@ -138,6 +138,17 @@ _SIGNATURES = {
         ctypes.c_int,
         [_PTR] * 4 + [ctypes.c_float, _PTR, _PTR, _I64] + [ctypes.c_float] * 3 + [_PTR] * 3,
     ),
+    "ash_surface_block8_workspace_bytes": (_I64, [_I64, _I64]),
+    "ash_surface_block8_classify": (
+        ctypes.c_int,
+        [_PTR, _PTR, _I64, _PTR, _I64, _PTR, _PTR, _I64, _I64, ctypes.c_float, ctypes.c_float,
+         ctypes.c_int32, _PTR, _PTR, _PTR],
+    ),
+    "ash_surface_block8_extract": (
+        ctypes.c_int,
+        [_PTR, _I64] + [_PTR] * 3 + [_I64, _I64, ctypes.c_float, ctypes.c_int32, _PTR, _I64, _I64,
+                                     ctypes.c_int, ctypes.c_float, _PTR, _PTR, _PTR, _PTR],
+    ),
     "ash_ray_sample_groups": (_I64, [_I64]),
     "ash_ray_sample_march": (
         ctypes.c_int,
@@ -183,6 +194,8 @@ _SIGNATURES = {
             _PTR,
         ],
     ),
+    "ash_map_neighbors": (
+        ctypes.c_int, [_PTR, _I64, ctypes.c_int, ctypes.c_int, _PTR, _PTR, _PTR]),
     "ash_map_items_in_index_order": (ctypes.c_int, [_PTR, ctypes.POINTER(ctypes.c_int)]),
     "ash_map_erase": (ctypes.c_int, [_PTR, _PTR, _I64, _PTR]),
     "ash_map_erase_bulk_query": (
@@ -194,8 +207,6 @@ _SIGNATURES = {
     "ash_map_counters": (ctypes.c_int, [_PTR, _PTR, ctypes.POINTER(_I64), _PTR]),
     "ash_map_counters_pending": (ctypes.c_int, [_PTR]),
     "ash_map_known_size": (ctypes.c_int, [_PTR, ctypes.POINTER(_I64)]),
-    "ash_map_neighbors": (
-        ctypes.c_int, [_PTR, _I64, ctypes.c_int, ctypes.c_int, _PTR, _PTR, _PTR]),
     "ash_map_set_staging": (ctypes.c_int, [_PTR, _PTR]),
     "ash_map_insert_scratch_bytes": (
         ctypes.c_int,
@@ -486,6 +497,34 @@ class _Backend:
                     )
                 )
         return triangles, vertices
+
+    def surface_mesh_block8(
+        self, hashmap, sdfs, weights, grid_indices, grid_coords_table, lut_grid_nb2grid_idx,
+        grid_dim, iso_value, weight_thr, to_world,
+    ):
+        """marching_cubes for blocks of 8^3 cells and the tables that
+        SparseDenseGrid builds (the per-cell ones are then not needed), or None
+        for other block sizes.  `sdfs` and `weights` may be channels of wider
+        rows; `to_world`: (scale, origin or None) to apply to the vertices, or
+        None."""
+        if int(grid_dim) != 8 or sdfs.dtype not in _DTYPE:
+            return None
+        _require_hip(sdfs, "sdfs")
+        dev = sdfs.device
+        b = sdfs.shape[0]
+
+        def channel(t):
+            t = t.reshape(b, 512)
+            step = t.stride(1)
+            return t if t.stride(0) == 512 * step and 1 <= step <= 64 else t.contiguous()
+
+        scale, origin = (1.0, None) if to_world is None else to_world
+        return self.host.surface_mesh(
+            hashmap._address, hashmap._index, channel(sdfs), channel(weights.to(dev, sdfs.dtype)),
+            grid_indices.reshape(-1).to(dev, torch.int64).contiguous(),
+            grid_coords_table.to(dev, torch.int32).contiguous(),
+            lut_grid_nb2grid_idx.to(dev, torch.int64).contiguous(), float(iso_value),
+            float(weight_thr), to_world is not None, scale, origin)
 
     # -- sparse convolution (ash/src/pybind.cpp:33) -------------------------
     def convolution_forward(
@@ -1331,6 +1370,17 @@ class _HashMap:
         self.last_items_in_index_order = bool(dense.value)
         return self._backend.host.items(self._address, self.key_dim, self._index, n)
 
+    def neighbor_rows(
+        self, num_rows: int, radius: int, bidirectional: bool
+    ) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
+        """(coords int32 (num_rows, 3), lut int64 (num_rows, K)): key of every
+        index and the indices of the keys at its offsets, -1 where there are
+        none; None for windows that one launch does not take."""
+        if self.key_dim != 3 or not 0 <= radius <= 15:
+            return None
+        return self._backend.host.neighbors(self._address, self._index, num_rows, radius,
+                                            bool(bidirectional))
+
     def load_states(self, states: Dict[str, torch.Tensor]) -> None:
         keys = self._keys(states["active_keys"])
         indices = states["active_indices"].to(self._device, torch.int64).contiguous()
@@ -1370,17 +1420,6 @@ class _HashMap:
                 f"load_states: {refused} pairs were refused (duplicate keys, or indices / heap "
                 "entries outside the capacity); nothing was loaded"
             )
-    def neighbor_rows(
-        self, num_rows: int, radius: int, bidirectional: bool
-    ) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
-        """(coords int32 (num_rows, 3), lut int64 (num_rows, K)): key of every
-        index and the indices of the keys at its offsets, -1 where there are
-        none; None for windows that one launch does not take."""
-        if self.key_dim != 3 or not 0 <= radius <= 15:
-            return None
-        return self._backend.host.neighbors(self._address, self._index, num_rows, radius,
-                                            bool(bidirectional))
-
 
 
 class _MissingBackend:

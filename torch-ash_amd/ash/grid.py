@@ -127,6 +127,7 @@ class SparseDenseGrid(ASHModule):
         self.transform_world_to_cell = lambda x: x
         self.transform_cell_to_world = lambda x: x
         self._remember_world_to_cell(lambda: (None, 1.0))
+        self._remember_cell_to_world(lambda: (1.0, None))
 
         self.in_dim = in_dim
         self.num_embeddings = num_embeddings
@@ -427,10 +428,24 @@ class SparseDenseGrid(ASHModule):
             return None
         return origin, float(cell_size)
 
-    def _cell_to_world_affine(self) -> Tuple[float, Optional[torch.Tensor]]:
-        """`transform_cell_to_world` as (scale, origin): world = cell * scale
-        [+ origin]."""
-        return 1.0, None
+    def _remember_cell_to_world(self, affine) -> None:
+        """The same for `transform_cell_to_world`: cell -> cell * scale
+        [+ origin] with (scale, origin) = affine()."""
+        self._cell_to_world_affine = affine
+        self._cell_to_world_known = self.transform_cell_to_world
+
+    def _known_cell_to_world(self, like: torch.Tensor):
+        """(scale, origin or None) if a kernel can apply `transform_cell_to_world`
+        to float32 positions on the device of `like` itself, else None."""
+        if self.transform_cell_to_world is not self._cell_to_world_known:
+            return None
+        scale, origin = self._cell_to_world_affine()
+        if torch.is_tensor(scale) or (origin is not None and (
+            not torch.is_tensor(origin) or origin.dtype != torch.float32
+            or origin.device != like.device or origin.shape != (3,)
+        )):
+            return None
+        return float(scale), origin
 
     @torch.no_grad()
     def _linearize_cell_coords(self, cell_coords: torch.Tensor) -> torch.Tensor:
@@ -650,6 +665,14 @@ class SparseDenseGrid(ASHModule):
         if self.grid_coords is None or self.lut_grid_nb2grid_idx is None:
             self.construct_grid_neighbor_lut_(radius=1, bidirectional=False)
         _, grid_indices = self._blocks_in_spatial_order()
+        if hasattr(backend, "surface_mesh_block8"):
+            to_world = self._known_cell_to_world(tsdfs)
+            mesh = backend.surface_mesh_block8(
+                self.engine.backend, tsdfs, weights, grid_indices, self.grid_coords,
+                self.lut_grid_nb2grid_idx, self.grid_dim, iso_value, weight_thr, to_world)
+            if mesh is not None:
+                triangles, vertices = mesh
+                return triangles, vertices if to_world else self.transform_cell_to_world(vertices)
         triangles, vertices = backend.marching_cubes(
             tsdfs,
             weights,
@@ -743,6 +766,12 @@ class SparseDenseGrid(ASHModule):
         """Per-block tables over all `num_embeddings` rows (ash/grid.py:566-617):
         grid_coords int32 (B, 3) and lut_grid_nb2grid_idx int64 (B, K), both -1
         in rows of inactive blocks and for missing neighbours."""
+        table = self.engine.backend
+        tables = (table.neighbor_rows(self.num_embeddings, radius, bidirectional)
+                  if hasattr(table, "neighbor_rows") else None)
+        if tables is not None:
+            return tables
+
         active_coords, active_indices = self.engine.items()
         nb_offsets, _ = enumerate_neighbor_coord_offsets(
             self.in_dim, radius, bidirectional, self.device
@@ -766,12 +795,6 @@ class SparseDenseGrid(ASHModule):
 
         grid_coords[active_indices] = active_coords
         lut[active_indices] = nb_indices.view(-1, num_nbs)
-        table = self.engine.backend
-        tables = (table.neighbor_rows(self.num_embeddings, radius, bidirectional)
-                  if hasattr(table, "neighbor_rows") else None)
-        if tables is not None:
-            return tables
-
         return grid_coords, lut
 
     @torch.no_grad()
@@ -802,7 +825,7 @@ class UnBoundedSparseDenseGrid(SparseDenseGrid):
         self.transform_world_to_cell = lambda x: x / self.cell_size
         self.transform_cell_to_world = lambda x: x * self.cell_size
         self._remember_world_to_cell(lambda: (None, self.cell_size))
-        self._cell_to_world_affine = lambda: (self.cell_size, None)
+        self._remember_cell_to_world(lambda: (self.cell_size, None))
         self.bbox_min = None
         self.bbox_max = None
 
@@ -857,7 +880,7 @@ class BoundedSparseDenseGrid(SparseDenseGrid):
         self.transform_world_to_cell = lambda x: (x - self.bbox_min) / self.cell_size
         self.transform_cell_to_world = lambda x: x * self.cell_size + self.bbox_min
         self._remember_world_to_cell(lambda: (self.bbox_min, self.cell_size))
-        self._cell_to_world_affine = lambda: (self.cell_size, self.bbox_min)
+        self._remember_cell_to_world(lambda: (self.cell_size, self.bbox_min))
 
     def grids_in_bound(self, grid_coords: torch.Tensor) -> torch.Tensor:
         inside = ((grid_coords >= 0) & (grid_coords < self.sparse_grid_dim)).all(dim=-1)

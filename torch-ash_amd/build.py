@@ -20,7 +20,7 @@ OUT = os.path.join(OUT_DIR, "libash_hip.so")
 HOST_SOURCE = os.path.join(CSRC, "ash_host.cpp")
 HOST_OUT = os.path.join(OUT_DIR, "_ash_host.so")
 SOURCES = ["ash_map.hip", "ash_bulk.hip", "ash_query.hip", "ash_fusion.hip", "ash_mesh.hip",
-           "ash_rays.hip", "ash_conv.hip"]
+           "ash_rays.hip", "ash_conv.hip", "ash_surface.hip"]
 HEADERS = [
     os.path.join(CSRC, "ash_probe.h"),
     os.path.join(CSRC, "ash_dev.h"),

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+#include <mutex>
 #include <string>
 
 namespace ash {
@@ -80,7 +82,7 @@ constexpr int kLineWords = 64;
 constexpr int kLineNow = 0;      // counters, fetched and waited for
 constexpr int kLineLate = 16;    // counters, fetched behind a streaming insert or a fusion frame
 constexpr int kLineEarly = 32;   // count left by the first pass of a streaming insert
-constexpr int kLineRays = 48;    // number of samples and largest count of a ray (64 bits each)
+constexpr int kLinePair = 48;    // two 64-bit numbers of a call that waits for them (pair_lock)
 constexpr int64_t kHeaderBytes = 256;
 
 // General region: open addressing over 32-bit state words + 16-byte keys.
@@ -156,7 +158,8 @@ struct ash_map {
     bool general_attached;
     // --- bookkeeping of the counters on the host ------------------------
     int32_t* line;          // page-locked words of the map's own (take_line), made on first use
-    int32_t stamp;          // of the latest words asked for
+    std::atomic<int32_t> stamp;   // of the latest words asked for
+    std::mutex pair_lock;   // held by the call that waits for the words at kLinePair
     int32_t late_stamp;
     bool late_in_flight;    // the device may still owe the words at kLineLate
     bool late_pending;      // ... and it is the latest state of the counters: nobody has looked at it yet

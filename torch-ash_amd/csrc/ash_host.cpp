@@ -46,6 +46,9 @@ namespace py = pybind11;
     X(ash_ray_sample_groups)                                                          \
     X(ash_ray_sample_march)                                                           \
     X(ash_ray_sample_place)                                                           \
+    X(ash_surface_block8_workspace_bytes)                                             \
+    X(ash_surface_block8_classify)                                                    \
+    X(ash_surface_block8_extract)                                                     \
     X(ash_grid_query)                                                                 \
     X(ash_grid_forward)                                                               \
     X(ash_query_forward)                                                              \
@@ -363,9 +366,6 @@ std::tuple<Tensor, Tensor> items(uintptr_t handle, int64_t dim, int64_t device, 
     return {keys, indices};
 }
 
-// ---------------------------------------------------------------------- grid
-Tensor positions_of(const Tensor& x) {
-    need(x.dim() == 2 && x.size(1) == 3 && x.scalar_type() == at::kFloat, "positions must be float32 (N, 3)");
 // (coords (rows, 3), lut (rows, K)) of the keys at offsets within `radius`
 std::pair<Tensor, Tensor> neighbors(uintptr_t handle, int64_t device, int64_t rows, int radius,
                                     bool bidirectional) {
@@ -377,6 +377,9 @@ std::pair<Tensor, Tensor> neighbors(uintptr_t handle, int64_t device, int64_t ro
     return {coords, lut};
 }
 
+// ---------------------------------------------------------------------- grid
+Tensor positions_of(const Tensor& x) {
+    need(x.dim() == 2 && x.size(1) == 3 && x.scalar_type() == at::kFloat, "positions must be float32 (N, 3)");
     return x.contiguous();
 }
 
@@ -476,6 +479,55 @@ std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> ray_sample(
                                    n, static_cast<float>(cell_size), ptr<int64_t>(indices),
                                    ptr<float>(t_nears), ptr<float>(t_fars), ptr<int64_t>(prefix), stream));
     return std::make_tuple(indices, t_nears, t_fars, prefix);
+}
+
+// (triangles, vertices).  `sdfs`, `weights`: a value per cell at the stride of
+// their last dimension; `lut`, `grid_coords`, `grid_indices`: contiguous.
+std::pair<Tensor, Tensor> surface_mesh(uintptr_t handle, int64_t device, const Tensor& sdfs,
+                                       const Tensor& weights, const Tensor& grid_indices,
+                                       const Tensor& grid_coords, const Tensor& lut, double iso,
+                                       double weight_thr, bool to_world, double cell_to_world,
+                                       const Optional& origin) {
+    const int64_t b = sdfs.size(0), n = grid_indices.size(0);
+    for (const Tensor* t : {&sdfs, &weights, &grid_indices, &grid_coords, &lut}) {
+        need(t->is_cuda() && t->get_device() == device, "all tensors must be on the map's device");
+    }
+    for (const Tensor* t : {&sdfs, &weights}) {
+        need(t->dim() == 2 && t->size(0) == b && t->size(1) == 512 && t->scalar_type() == sdfs.scalar_type() &&
+                     (b == 1 || t->stride(0) == 512 * t->stride(1)),
+             "field and weights must be (num_embeddings, 512), evenly strided, of one type");
+    }
+    need(sdfs.scalar_type() == at::kFloat || sdfs.scalar_type() == at::kDouble,
+         "sdfs must be float32 or float64");
+    need(grid_indices.scalar_type() == at::kLong && grid_indices.dim() == 1 &&
+                 lut.scalar_type() == at::kLong && lut.dim() == 2 && lut.size(0) == b && lut.size(1) == 8 &&
+                 grid_coords.scalar_type() == at::kInt && grid_coords.dim() == 2 &&
+                 grid_coords.size(0) == b && grid_coords.size(1) == 3 && grid_indices.is_contiguous() &&
+                 lut.is_contiguous() && grid_coords.is_contiguous(),
+         "coordinate / neighbour tables do not match the grid");
+    Tensor from;
+    if (origin.has_value()) from = floats_on(*origin, device);
+    const int32_t dtype = sdfs.scalar_type() == at::kFloat ? ASH_F32 : ASH_F64;
+    const Tensor workspace = empty({lib.ash_surface_block8_workspace_bytes(n, b)}, at::kByte, device);
+    void* stream = stream_of(device);
+    int64_t out[2] = {0, 0};
+    int status;
+    {
+        py::gil_scoped_release waits_for_the_device;
+        status = lib.ash_surface_block8_classify(
+                map_of(handle), ptr<void>(sdfs), sdfs.stride(1), ptr<void>(weights), weights.stride(1),
+                ptr<int64_t>(grid_indices), ptr<int64_t>(lut), n, b, static_cast<float>(iso),
+                static_cast<float>(weight_thr), dtype, ptr<void>(workspace), out, stream);
+    }
+    check(status);
+    const Tensor vertices = empty({out[0], 3}, at::kFloat, device);
+    const Tensor triangles = empty({out[1], 3}, at::kInt, device);
+    check(lib.ash_surface_block8_extract(
+            ptr<void>(sdfs), sdfs.stride(1), ptr<int64_t>(grid_indices), ptr<int32_t>(grid_coords),
+            ptr<int64_t>(lut), n, b, static_cast<float>(iso), dtype, ptr<void>(workspace), out[0], out[1],
+            to_world, static_cast<float>(cell_to_world), ptr<float>(from), ptr<float>(vertices),
+            ptr<int32_t>(triangles), stream));
+    return {triangles, vertices};
 }
 
 Tensor table_of(const Tensor& t, int64_t rows, int64_t device, const char* name) {
@@ -735,13 +787,14 @@ PYBIND11_MODULE(_ash_host, m) {
     m.def("erase", &erase);
     m.def("counters", &counters);
     m.def("items", &items);
+    m.def("neighbors", &neighbors);
     m.def("query_cells", &query_cells);
     m.def("grid_forward", &grid_forward);
     m.def("fuse_frame", &fuse_frame);
     m.def("ray_near_far", &ray_near_far);
     m.def("ray_sample", &ray_sample);
+    m.def("surface_mesh", &surface_mesh);
     m.def("query_forward", &query_forward);
     m.def("query_backward_forward", &query_backward_forward);
     m.def("query_backward_backward", &query_backward_backward);
 }
-    m.def("neighbors", &neighbors);

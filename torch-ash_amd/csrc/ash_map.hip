@@ -1751,8 +1751,8 @@ int take_line(ash_map* map) {
     map->line = lines.back();
     lines.pop_back();
     // stamps of this map start where the line's last owner stopped
-    for (int at : {kLineNow, kLineLate, kLineEarly, kLineRays}) {
-        map->stamp = std::max(map->stamp, map->line[at + kLandingStamp]);
+    for (int at : {kLineNow, kLineLate, kLineEarly, kLinePair}) {
+        map->stamp = std::max(map->stamp.load(), map->line[at + kLandingStamp]);
     }
     return 0;
 }

@@ -597,6 +597,7 @@ int ash_ray_sample_march(ash_map_t* map, const float* ray_origins, const float* 
     DeviceGuard guard;
     ASH_HIP(guard.enter(map->device));
     if (settle_table(map, s)) return 1;
+    std::lock_guard<std::mutex> one_answer(map->pair_lock);
     if (take_line(map)) return 1;
     auto* g = reinterpret_cast<GroupSamples*>(groups);
     if (launch_march(map, {ray_origins, ray_directions, {origin, 1.0f / cell_size, cell_size}, ray_nears,
@@ -605,7 +606,7 @@ int ash_ray_sample_march(ash_map_t* map, const float* ray_origins, const float* 
                      counts, nullptr, nullptr, nullptr, nullptr, stage, stride, g, s)) {
         return 1;
     }
-    int32_t* landing = map->line + kLineRays;
+    int32_t* landing = map->line + kLinePair;
     const int32_t stamp = ++map->stamp;
     ray_scan_kernel<<<1, kScanThreads, 0, s>>>(g, static_cast<int>(march_groups(n)), landing, stamp);
     ASH_LAUNCH_CHECK();

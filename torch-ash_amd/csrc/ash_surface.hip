@@ -1,0 +1,753 @@
+// Marching cubes over blocks of 8^3 cells in the layout the Python layer builds
+// (cell c = x + 8 y + 64 z, neighbour b of the 2^3 window at bit pattern z y x):
+// SparseDenseGrid.surface_mesh (ash/src/grid.cu:606-946 of the reference;
+// ash_mesh.hip holds the kernels for other block sizes and for callers' tables).
+//
+// What the surface needs of a cell is two bits -- it weighs enough, it lies
+// below the iso value -- so one pass over the field turns a block into 128
+// bytes, and everything up to the vertex positions works on those:
+//
+//   bits     field and weights, read once and in order, wherever their values
+//            lie in the rows (a channel of a wider tensor is not copied out
+//            first): per block 8 + 8 words of 64 cells, a z layer each
+//   classify a lane per row of eight cells along x: the cells the surface
+//            crosses, their edges' owners and the number of their triangles,
+//            eight cells at a time.  A row's three flag bytes (+x, +y, +z edge)
+//            go to the block's own 64 words; what a block owes its neighbours
+//            is at most nine 64-bit words, OR-ed into their face words
+//   count    faces joined to the rows; where the points of a row start within
+//            its block (8 bits from its layer, 16 from the block), where the
+//            block's start within a group of 64
+//   scan     running sums over the groups, totals to the host
+//   points, triangles
+//            a wavefront per block lists the block's points / triangles in LDS
+//            and consecutive lanes handle consecutive ones.  A vertex id is the
+//            start of the row plus the flags below the edge's
+//
+// 60 000 blocks, field and weights in rows of five channels, us: bits 121,
+// classify 29, count and scan 23, points 47, triangles 66, together 292; with
+// case bytes, a slot word per cell and the two channels copied out first: copies
+// 274, clear, classify, count, points and triangles 415.
+//
+// Vertices are numbered along the listing, cells in order within a block, the
+// axes in order within a cell, and triangles likewise: as in ash_mesh.hip.
+#include "ash_table.h"
+#include "ash_mc_table.h"
+#include "ash_walk.h"
+
+#include "../../include/ash_hip.h"
+
+#include <type_traits>
+
+namespace ash {
+namespace {
+
+constexpr int kG = 8;
+constexpr int kM = kG * kG * kG;
+constexpr int kBlock = 256;
+constexpr int kGroupBlocks = 64;      // blocks of the listing per running sum
+constexpr int kCountThreads = 1024;
+constexpr int kScanThreads = 1024;
+constexpr int64_t kMaxStride = 64;
+// One-wavefront workgroups of a walk over the blocks: several times what the
+// device holds, because blocks differ in work (60 000 blocks, triangles / points /
+// classify: 4096 workgroups 100 / 74 / 37 us, 8192 83 / 52 / 28, 16384 77 / 47 /
+// 28, 65536 91 / 44 / 38, where setting up shows)
+constexpr int kWalkGroups = 16384;
+constexpr int kRoundTriangles = 1024;   // of a block, listed at a time (blocks at a surface have some 250)
+constexpr uint32_t kRowBits = 0x00FFFFFFu;
+enum Face { kXy, kXz, kYx, kYz, kZx, kZy };   // face of the block, axis of the edges
+
+struct Sums {
+    int64_t points, triangles;
+};
+
+// The workspace: per row of the field tensor unless stated otherwise.
+struct Work {
+    uint64_t* bits;     // [B, 16]  bit x + 8 y of word z: weighs enough; of word 8 + z: below iso
+    uint64_t* faces;    // [B, 8]   edges of the low-face cells that neighbours flag
+    uint32_t* rows;     // [B, 64]  three flag bytes | points before in the layer << 24
+    uint16_t* layer;    // [B, 8]   points before the layer in the block
+    uint32_t* first;    // [B]      first point of the block
+    uint2* local;       // [n]      points and triangles before the listed block in its group
+    Sums* groups;       // [ceil(n / kGroupBlocks)]
+};
+
+struct SurfaceArgs {
+    const void* sdfs;
+    const void* weights;
+    const int64_t* grid_indices;
+    const int32_t* grid_coords;   // [B, 3]
+    const int64_t* lut_g;         // [B, 8]
+    Work w;
+    int64_t n, B;
+    int64_t sdf_stride, weight_stride;   // elements between cells
+    float iso, weight_thr;
+    // world = cell * scale (+ origin), applied if `to_world`
+    const float* origin;
+    float scale;
+    bool to_world;
+    int64_t n_points, n_triangles;
+    float* positions;
+    int32_t* triangles;
+};
+
+int64_t groups_of(int64_t n) { return (n + kGroupBlocks - 1) / kGroupBlocks; }
+
+int64_t align16(int64_t bytes) { return (bytes + 15) & ~int64_t{15}; }
+
+int64_t lay_out(Work& w, char* base, int64_t n, int64_t B) {
+    int64_t at = 0;
+    auto take = [&](auto*& p, int64_t count) {
+        p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(base + at);
+        at += align16(count * static_cast<int64_t>(sizeof(*p)));
+    };
+    take(w.bits, 16 * B);
+    take(w.faces, 8 * B);
+    take(w.rows, 64 * B);
+    take(w.layer, 8 * B);
+    take(w.first, B);
+    take(w.local, n);
+    take(w.groups, groups_of(n));
+    return at;
+}
+
+// Blocks that are not listed count as missing: their bits stay clear.
+__global__ __launch_bounds__(kBlock) void clear_bits_kernel(uint4* bits, int64_t units) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    if (i < units) bits[i] = make_uint4(0u, 0u, 0u, 0u);
+}
+
+// One wavefront per listed block, a lane per cell of a layer: sixteen loads in
+// flight, the two values of a cell usually in one line.  Bound by memory (each
+// line of the field once, in order).
+template <typename T>
+__global__ __launch_bounds__(kBlock) void bits_kernel(SurfaceArgs a) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t b = static_cast<int64_t>(blockIdx.x) * (kBlock / 64) + wave;
+    if (b >= a.n) return;
+    const int64_t g = a.grid_indices[b];
+    if (g < 0 || g >= a.B) return;
+    const T* sdfs = static_cast<const T*>(a.sdfs) + g * kM * a.sdf_stride;
+    const T* weights = static_cast<const T*>(a.weights) + g * kM * a.weight_stride;
+    const int s = static_cast<int>(a.sdf_stride), t = static_cast<int>(a.weight_stride);
+    T v[kG], w[kG];
+#pragma unroll
+    for (int z = 0; z < kG; ++z) {
+        v[z] = sdfs[(z * 64 + lane) * s];
+        w[z] = weights[(z * 64 + lane) * t];
+    }
+    uint64_t mine = 0;
+#pragma unroll
+    for (int z = 0; z < kG; ++z) {
+        const uint64_t ok = __ballot(w[z] >= static_cast<T>(a.weight_thr));
+        const uint64_t below = __ballot(v[z] - static_cast<T>(a.iso) < T(0));
+        if (lane == z) mine = ok;
+        if (lane == 8 + z) mine = below;
+    }
+    if (lane < 16) a.w.bits[g * 16 + lane] = mine;
+    if (lane >= 16 && lane < 24) a.w.faces[g * 8 + (lane - 16)] = 0;
+}
+
+// ------------------------------------------------------ a block and its corners
+// The listing positions a one-wavefront workgroup walks, with what it needs of
+// a block fetched one block (rows) and two blocks (index) ahead: lane l works
+// for source s = l / 8, the block itself for s = 0, else neighbour s.
+struct Blocks {
+    const SurfaceArgs& a;
+    TileWalk walk;
+    int64_t at;         // listing position
+    int64_t own, row;   // the block's row; the row of the lane's source, -1 if missing
+    int64_t next_own, next_row, third_own;
+
+    __device__ __forceinline__ int64_t index(int64_t b) const {
+        if (b >= walk.end) return -1;
+        const int64_t g = a.grid_indices[b];
+        return (g >= 0 && g < a.B) ? g : -1;
+    }
+    __device__ __forceinline__ int64_t source(int64_t g) const {
+        const int s = (threadIdx.x & 63) >> 3;
+        if (g < 0) return -1;
+        if (s == 0) return g;
+        const int64_t r = a.lut_g[g * 8 + s];
+        return (r >= 0 && r < a.B) ? r : -1;
+    }
+    __device__ __forceinline__ Blocks(const SurfaceArgs& args)
+        : a(args), walk(args.n), at(walk.next) {
+        own = index(at);
+        next_own = index(at + walk.step);
+        row = source(own);
+        third_own = index(at + 2 * walk.step);
+        next_row = source(next_own);
+    }
+    __device__ __forceinline__ bool more() const { return at < walk.end; }
+    // (the loads of `third_own` are waited for one block later)
+    __device__ __forceinline__ void advance() {
+        at += walk.step;
+        own = next_own;
+        row = next_row;
+        next_own = third_own;
+        third_own = index(at + 2 * walk.step);
+        next_row = source(next_own);
+    }
+    // 16 of the 128 bytes of the lane's source
+    __device__ __forceinline__ uint4 piece() const {
+        if (row < 0) return make_uint4(0u, 0u, 0u, 0u);
+        return reinterpret_cast<const uint4*>(a.w.bits + row * 16)[threadIdx.x & 7];
+    }
+};
+
+// What lane (y, z) = (lane & 7, lane >> 3) knows of its row of cells: the bits
+// "below" of the rows (y + dy, z + dz), nine cells long, in rows[dy + 2 dz], and
+// the cells of the row (y, z) that the surface crosses.
+struct RowCells {
+    uint32_t below[4];
+    uint32_t crossed;
+};
+
+// `bits`: the 128 bytes of the eight sources.
+__device__ __forceinline__ RowCells row_cells(const uint8_t* bits) {
+    const int lane = threadIdx.x & 63;
+    RowCells r;
+    uint32_t ok = 0xFFu, any = 0u, all = 0xFFu;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int y = (lane & 7) + (q & 1), z = (lane >> 3) + (q >> 1);
+        const uint8_t* from = bits + (((y >> 3) << 1) | ((z >> 3) << 2)) * 128 + (y & 7) + 8 * (z & 7);
+        const uint32_t o = from[0] | ((from[128] & 1u) << 8);
+        const uint32_t b = from[64] | ((from[128 + 64] & 1u) << 8);
+        ok &= o & (o >> 1);
+        any |= b | (b >> 1);
+        all &= b & (b >> 1);
+        r.below[q] = b;
+    }
+    r.crossed = ok & any & ~all & 0xFFu;
+    return r;
+}
+
+__device__ __forceinline__ uint32_t case_of(const RowCells& r, int x) {
+    return ((r.below[0] >> x) & 3u) | (((r.below[1] >> x) & 3u) << 2) |
+           (((r.below[2] >> x) & 3u) << 4) | (((r.below[3] >> x) & 3u) << 6);
+}
+
+__device__ __forceinline__ uint32_t lane_up(uint32_t v, int d) {
+    return static_cast<uint32_t>(__shfl(static_cast<int>(v), ((threadIdx.x & 63) - d) & 63));
+}
+
+__global__ __launch_bounds__(64) void classify_kernel(SurfaceArgs a) {
+    __shared__ __align__(16) uint8_t s_bits[8 * 128];
+    __shared__ uint8_t s_count[256];
+    __shared__ __align__(8) uint8_t s_face[4 * 8];
+    const int lane = threadIdx.x;
+    const int y = lane & 7, z = lane >> 3;
+    for (int i = lane; i < 256; i += 64) s_count[i] = static_cast<uint8_t>(kMcTriangleCount[i]);
+    Blocks blk(a);
+    uint4 piece = blk.piece();
+    for (; blk.more(); blk.advance(), piece = blk.piece()) {
+        __syncthreads();   // the previous block's bits and faces have been read
+        reinterpret_cast<uint4*>(s_bits)[lane] = piece;
+        __syncthreads();
+        const int64_t g = blk.own;
+        if (g < 0) {   // the same for the whole wavefront
+            if (lane == 0) a.w.local[blk.at] = make_uint2(0u, 0u);
+            continue;
+        }
+        const RowCells r = row_cells(s_bits);
+        if (__ballot(r.crossed != 0u) == 0) {
+            a.w.rows[g * 64 + lane] = 0u;
+            if (lane == 0) a.w.local[blk.at] = make_uint2(0u, 0u);
+            continue;
+        }
+        // Crossed edges of the crossed cells, by the row of their owner: +x
+        // edges of all four rows (eight bits), +y edges of the two rows at y,
+        // +z edges of the two at z (nine bits: cell 8 belongs to the next block)
+        const uint32_t c = r.crossed, c9 = c | (c << 1);
+        uint32_t ex[4], ey[2], ez[2];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) ex[q] = c & (r.below[q] ^ (r.below[q] >> 1));
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+            ey[d] = c9 & (r.below[2 * d] ^ r.below[2 * d + 1]);
+            ez[d] = c9 & (r.below[d] ^ r.below[d + 2]);
+        }
+        const uint32_t here = ex[0] | ((ey[0] & 0xFFu) << 8) | ((ez[0] & 0xFFu) << 16);
+        const uint32_t corner = ex[3];
+        uint32_t to_y = ex[1] | ((ez[1] & 0xFFu) << 16);
+        uint32_t to_z = ex[2] | ((ey[1] & 0xFFu) << 8);
+        const uint32_t from_z = lane_up(to_z, 8);
+        if (const uint32_t up = lane_up(corner, 8); z > 0) to_y |= up;
+        if (const uint32_t up = lane_up(corner, 1); y > 0) to_z |= up;
+        uint32_t own = here;
+        if (const uint32_t up = lane_up(to_y, 1); y > 0) own |= up;
+        if (z > 0) own |= from_z;
+        a.w.rows[g * 64 + lane] = own;
+
+        if (y == 7) {
+            s_face[z] = static_cast<uint8_t>(to_y);
+            s_face[8 + z] = static_cast<uint8_t>(to_y >> 16);
+        }
+        if (z == 7) {
+            s_face[16 + y] = static_cast<uint8_t>(to_z);
+            s_face[24 + y] = static_cast<uint8_t>(to_z >> 8);
+        }
+        __syncthreads();
+        const uint64_t y0 = __ballot(ey[0] >> 8), y1 = __ballot(ey[1] >> 8);   // by row
+        const uint64_t z0 = __ballot(ez[0] >> 8), z1 = __ballot(ez[1] >> 8);
+        constexpr uint64_t kLowY = 0x0101010101010101ull;
+        uint64_t owed = 0;
+        int to = 0, face = 0;
+        auto owe = [&](int l, int s, int f, uint64_t word) {
+            if (lane == l) {
+                owed = word;
+                to = s;
+                face = f;
+            }
+        };
+        const uint64_t* faces = reinterpret_cast<const uint64_t*>(s_face);
+        owe(0, 1, kXy, y0 | (y1 << 8));
+        owe(1, 1, kXz, z0 | ((z1 & ~(kLowY << 7)) << 1));
+        owe(2, 2, kYx, faces[0]);
+        owe(3, 2, kYz, faces[1]);
+        owe(4, 4, kZx, faces[2]);
+        owe(5, 4, kZy, faces[3]);
+        owe(6, 5, kXy, y1 >> 56);
+        owe(7, 3, kXz, (z1 >> 7) & kLowY);
+        owe(8, 6, kYx, static_cast<uint32_t>(__builtin_amdgcn_readlane(corner, 63)));
+        const int64_t dest = __shfl(blk.row, to * 8);
+        if (owed != 0 && dest >= 0) {
+            atomicOr(reinterpret_cast<unsigned long long*>(a.w.faces + dest * 8 + face),
+                     static_cast<unsigned long long>(owed));
+        }
+
+        int triangles = 0;
+        for (uint32_t left = c; left != 0u; left &= left - 1u) {
+            triangles += s_count[case_of(r, __builtin_ctz(left))];
+        }
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) triangles += __shfl_xor(triangles, d);
+        if (lane == 0) a.w.local[blk.at] = make_uint2(0u, static_cast<uint32_t>(triangles));
+    }
+}
+
+// Sixteen wavefronts, four blocks each: the 64 blocks of a group.
+__global__ __launch_bounds__(kCountThreads) void count_kernel(SurfaceArgs a) {
+    constexpr int kEach = kGroupBlocks / (kCountThreads / 64);
+    __shared__ int s_points[kGroupBlocks];
+    const int lane = threadIdx.x & 63;
+    // (the same for the whole wavefront: the faces come through the scalar cache)
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int y = lane & 7, z = lane >> 3;
+    const int64_t b0 = static_cast<int64_t>(blockIdx.x) * kGroupBlocks;
+    int64_t g[kEach];
+    uint32_t w[kEach];
+    uint64_t face[kEach][6];
+#pragma unroll
+    for (int k = 0; k < kEach; ++k) {
+        const int64_t b = b0 + wave * kEach + k;
+        g[k] = b < a.n ? a.grid_indices[b] : -1;
+        if (g[k] >= a.B) g[k] = -1;
+    }
+#pragma unroll
+    for (int k = 0; k < kEach; ++k) {
+        w[k] = g[k] < 0 ? 0u : a.w.rows[g[k] * 64 + lane];
+#pragma unroll
+        for (int f = 0; f < 6; ++f) face[k][f] = g[k] < 0 ? 0u : a.w.faces[g[k] * 8 + f];
+    }
+#pragma unroll
+    for (int k = 0; k < kEach; ++k) {
+        const auto byte = [&](int f, int i) { return static_cast<uint32_t>(face[k][f] >> (8 * i)) & 0xFFu; };
+        w[k] |= (static_cast<uint32_t>(face[k][kXy] >> lane) & 1u) << 8;
+        w[k] |= (static_cast<uint32_t>(face[k][kXz] >> lane) & 1u) << 16;
+        if (y == 0) w[k] |= byte(kYx, z) | (byte(kYz, z) << 16);
+        if (z == 0) w[k] |= byte(kZx, y) | (byte(kZy, y) << 8);
+        const int own = __popc(w[k]);
+        int incl = own;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int up = __shfl_up(incl, d);
+            if (lane >= d) incl += up;
+        }
+        const int before = incl - own;
+        const int layer = __shfl(before, lane & ~7);
+        if (g[k] >= 0) {
+            a.w.rows[g[k] * 64 + lane] = w[k] | (static_cast<uint32_t>(before - layer) << 24);
+            if (y == 0) a.w.layer[g[k] * 8 + z] = static_cast<uint16_t>(layer);
+        }
+        if (lane == 63) s_points[wave * kEach + k] = incl;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        const int64_t b = b0 + lane;
+        const int points = s_points[lane];
+        const int triangles = b < a.n ? static_cast<int>(a.w.local[b].y) : 0;
+        int p = points, t = triangles;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int up = __shfl_up(p, d), ut = __shfl_up(t, d);
+            if (lane >= d) {
+                p += up;
+                t += ut;
+            }
+        }
+        if (b < a.n) a.w.local[b] = make_uint2(p - points, t - triangles);
+        if (lane == 63) a.w.groups[blockIdx.x] = {p, t};
+    }
+}
+
+// Sums of the groups -> what lies before each; totals for the host.
+__global__ __launch_bounds__(kScanThreads) void scan_groups_kernel(Sums* __restrict__ groups, int64_t n,
+                                                                   int32_t* landing, int32_t stamp) {
+    __shared__ Sums s_part[kScanThreads / 64];
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const int64_t per = (n + kScanThreads - 1) / kScanThreads;
+    const int64_t first = threadIdx.x * per < n ? threadIdx.x * per : n;
+    const int64_t last = first + per < n ? first + per : n;
+    Sums mine = {0, 0};
+    for (int64_t i = first; i < last; ++i) {
+        mine.points += groups[i].points;
+        mine.triangles += groups[i].triangles;
+    }
+    Sums incl = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int64_t up = __shfl_up(incl.points, d), ut = __shfl_up(incl.triangles, d);
+        if (lane >= d) {
+            incl.points += up;
+            incl.triangles += ut;
+        }
+    }
+    if (lane == 63) s_part[wave] = incl;
+    __syncthreads();
+    Sums before = {incl.points - mine.points, incl.triangles - mine.triangles}, total = {0, 0};
+    for (int w = 0; w < kScanThreads / 64; ++w) {
+        if (w < wave) {
+            before.points += s_part[w].points;
+            before.triangles += s_part[w].triangles;
+        }
+        total.points += s_part[w].points;
+        total.triangles += s_part[w].triangles;
+    }
+    for (int64_t i = first; i < last; ++i) {
+        const Sums own = groups[i];
+        groups[i] = before;
+        before.points += own.points;
+        before.triangles += own.triangles;
+    }
+    if (threadIdx.x == 0) {
+        const int32_t words[4] = {
+                static_cast<int32_t>(total.points), static_cast<int32_t>(total.points >> 32),
+                static_cast<int32_t>(total.triangles), static_cast<int32_t>(total.triangles >> 32)};
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            __hip_atomic_store(landing + w, words[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        __hip_atomic_store(landing + kLandingStamp, stamp, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+// Rounded twice, as the module's multiplication and addition are.
+__device__ __forceinline__ float to_world(float p, float scale, const float* origin, int k) {
+#pragma clang fp contract(off)
+    const float scaled = p * scale;
+    return origin == nullptr ? scaled : scaled + origin[k];
+}
+
+// The zero crossing of every flagged edge, linear between its two ends
+// (ash/src/grid.cu:748-771).  Bound by the lines of the field that its cells and
+// their partners lie in.
+template <typename T>
+__global__ __launch_bounds__(64) void points_kernel(SurfaceArgs a) {
+    __shared__ uint16_t s_point[3 * kM];   // cell | axis << 9
+    const T* sdfs = static_cast<const T*>(a.sdfs);
+    const int lane = threadIdx.x;
+    const int row0 = (lane & 7) * kG + (lane >> 3) * 64;   // first cell of the lane's row
+    Blocks blk(a);
+    for (; blk.more(); blk.advance()) {
+        const int64_t g = blk.own;
+        if (g < 0) continue;   // the same for the whole wavefront
+        const uint32_t word = a.w.rows[g * 64 + lane];
+        const uint32_t flags = word & kRowBits;
+        if (__ballot(flags != 0u) == 0) continue;
+        int at = a.w.layer[g * 8 + (lane >> 3)] + static_cast<int>(word >> 24);
+        const int64_t first = a.w.groups[blk.at / kGroupBlocks].points + a.w.local[blk.at].x;
+        if (lane == 0) a.w.first[g] = static_cast<uint32_t>(first);
+        const int total = __shfl(at + __popc(flags), 63);
+        __syncthreads();   // the previous block's list has been read
+        for (uint32_t left = (flags | (flags >> 8) | (flags >> 16)) & 0xFFu; left != 0u; left &= left - 1u) {
+            const int x = __builtin_ctz(left);
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                if ((flags >> (8 * d + x)) & 1u) s_point[at++] = static_cast<uint16_t>((row0 + x) | (d << 9));
+            }
+        }
+        __syncthreads();
+        const int32_t corner[3] = {a.grid_coords[g * 3] * kG, a.grid_coords[g * 3 + 1] * kG,
+                                   a.grid_coords[g * 3 + 2] * kG};
+        for (int q0 = 0; q0 < total; q0 += 64) {
+            const int q = q0 + lane;
+            const int entry = q < total ? s_point[q] : 0;
+            const int cell = entry & (kM - 1);
+            const int d = entry >> 9;
+            const int shift = 3 * d;
+            const int past = ((cell >> shift) & 7) == 7;
+            // (all lanes take part: the row is that of another lane)
+            const int64_t next = __shfl(blk.row, past ? 8 << d : 0);
+            if (q >= total || first + q >= a.n_points) continue;   // (the latter never with the totals of the scan)
+            const int partner = past ? cell & ~(7 << shift) : cell + (1 << shift);
+            const T self = sdfs[(g * kM + cell) * a.sdf_stride] - static_cast<T>(a.iso);
+            float ratio = 0.f;
+            if (next >= 0) {
+                const T other = sdfs[(next * kM + partner) * a.sdf_stride] - static_cast<T>(a.iso);
+                ratio = static_cast<float>(self / (self - other));
+            }
+            float* out = a.positions + (first + q) * 3;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const float p = static_cast<float>(corner[k] + ((cell >> (3 * k)) & 7)) +
+                                (d == k ? ratio : 0.f);
+                out[k] = a.to_world ? to_world(p, a.scale, a.origin, k) : p;
+            }
+        }
+    }
+}
+
+// Triangles of every crossed cell as ids of the points on its edges
+// (ash/src/grid.cu:796-842); the table's rows have the orientation the reference
+// writes.
+__global__ __launch_bounds__(64) void triangles_kernel(SurfaceArgs a) {
+    constexpr int kRows = (kG + 1) * (kG + 1);
+    __shared__ __align__(16) uint8_t s_bits[8 * 128];
+    __shared__ uint64_t s_table[256];
+    __shared__ uint8_t s_count[256];
+    __shared__ uint8_t s_case[kM];
+    __shared__ uint16_t s_triangle[kRoundTriangles];   // cell | number in the cell << 9
+    __shared__ uint32_t s_flags[2 * kRows];               // rows (y, z) of the block and of its +x neighbours
+    __shared__ uint32_t s_first[2 * kRows];
+    const int lane = threadIdx.x;
+    const int row0 = (lane & 7) * kG + (lane >> 3) * 64;
+    for (int i = lane; i < 256; i += 64) {
+        s_table[i] = kMcPackedRows[i];
+        s_count[i] = static_cast<uint8_t>(kMcTriangleCount[i]);
+    }
+    Blocks blk(a);
+    uint4 piece = blk.piece();
+    for (; blk.more(); blk.advance(), piece = blk.piece()) {
+        __syncthreads();   // the previous block's lists have been read
+        reinterpret_cast<uint4*>(s_bits)[lane] = piece;
+        __syncthreads();
+        if (blk.own < 0) continue;   // the same for the whole wavefront
+        const RowCells r = row_cells(s_bits);
+        if (__ballot(r.crossed != 0u) == 0) continue;
+        const int64_t first = a.w.groups[blk.at / kGroupBlocks].triangles + a.w.local[blk.at].y;
+#pragma unroll
+        for (int k = 0; k < (2 * kRows + 63) / 64; ++k) {
+            const int i = k * 64 + lane;
+            const int side = i >= kRows, p = i - side * kRows;
+            const int y = p % (kG + 1), z = p / (kG + 1);
+            const int s = side | ((y >> 3) << 1) | ((z >> 3) << 2);
+            const int64_t g = __shfl(blk.row, (s & 7) * 8);
+            if (i >= 2 * kRows) continue;
+            uint32_t word = 0, id = 0;
+            if (g >= 0) {
+                word = a.w.rows[g * 64 + (y & 7) + 8 * (z & 7)];
+                id = a.w.first[g] + a.w.layer[g * 8 + (z & 7)] + (word >> 24);
+            }
+            s_flags[i] = word & kRowBits;
+            s_first[i] = id;
+        }
+        int mine = 0;
+        for (uint32_t left = r.crossed; left != 0u; left &= left - 1u) {
+            const int x = __builtin_ctz(left);
+            const uint32_t code = case_of(r, x);
+            s_case[row0 + x] = static_cast<uint8_t>(code);
+            mine += s_count[code];
+        }
+        int at = mine;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int up = __shfl_up(at, d);
+            if (lane >= d) at += up;
+        }
+        const int total = __shfl(at, 63);
+        at -= mine;
+        for (int q0 = 0; q0 < total; q0 += kRoundTriangles) {
+            if (q0 > 0) __syncthreads();   // the previous round's list has been read
+            int to = at - q0;
+            for (uint32_t left = r.crossed; left != 0u; left &= left - 1u) {
+                const int x = __builtin_ctz(left);
+                const int n = s_count[case_of(r, x)];
+                for (int t = 0; t < n; ++t, ++to) {
+                    if (static_cast<unsigned>(to) < kRoundTriangles) {
+                        s_triangle[to] = static_cast<uint16_t>((row0 + x) | (t << 9));
+                    }
+                }
+            }
+            __syncthreads();
+            const int listed = total - q0 < kRoundTriangles ? total - q0 : kRoundTriangles;
+            for (int q = lane; q < listed; q += 64) {
+                if (first + q0 + q >= a.n_triangles) continue;   // never with the totals of the scan
+                const int cell = s_triangle[q] & (kM - 1);
+                const int t = s_triangle[q] >> 9;
+                const uint32_t edges = static_cast<uint32_t>(s_table[s_case[cell]] >> (12 * t));
+                const int x = cell & 7, y = (cell >> 3) & 7, z = cell >> 6;
+                int32_t* out = a.triangles + (first + q0 + q) * 3;
+#pragma unroll
+                for (int v = 0; v < 3; ++v) {
+                    // edge e = 4 axis + j starts at the corner made by a zero bit
+                    // put into j at position `axis`
+                    const int e = static_cast<int>(edges >> (4 * v)) & 15;
+                    const int axis = e >> 2, j = e & 3;
+                    const int low = (j & ((1 << axis) - 1)) | ((j >> axis) << (axis + 1));
+                    const int px = x + (low & 1);
+                    const int i = (px >> 3) * kRows + y + ((low >> 1) & 1) + (kG + 1) * (z + (low >> 2));
+                    const uint32_t flags = s_flags[i];
+                    const uint32_t before = ((1u << (px & 7)) - 1u) * 0x010101u;
+                    const uint32_t lower = ((1u << (8 * axis)) - 1u) & (0x010101u << (px & 7));
+                    out[v] = static_cast<int32_t>(s_first[i] + __popc(flags & (before | lower)));
+                }
+            }
+        }
+    }
+}
+
+unsigned walk_grid(int64_t n) { return static_cast<unsigned>(n < kWalkGroups ? n : kWalkGroups); }
+
+int fill(SurfaceArgs& a, const void* sdfs, int64_t sdf_stride, const int64_t* grid_indices,
+         const int64_t* lut, int64_t n, int64_t B, float iso, int32_t dtype, void* workspace) {
+    if (dtype != ASH_F32 && dtype != ASH_F64) ASH_FAIL("unknown dtype");
+    if (n < 0 || B < 1 || n > (int64_t{1} << 31) || B > (int64_t{1} << 31)) {
+        ASH_FAIL("surface extraction: bad sizes");
+    }
+    if (sdf_stride < 1 || sdf_stride > kMaxStride) ASH_FAIL("surface extraction: bad stride");
+    if (n > 0 && (sdfs == nullptr || grid_indices == nullptr || lut == nullptr || workspace == nullptr)) {
+        ASH_FAIL("null pointer in surface extraction");
+    }
+    if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0) {
+        ASH_FAIL("surface extraction: the workspace must be 16-byte aligned");
+    }
+    a.sdfs = sdfs;
+    a.sdf_stride = sdf_stride;
+    a.grid_indices = grid_indices;
+    a.lut_g = lut;
+    a.n = n;
+    a.B = B;
+    a.iso = iso;
+    lay_out(a.w, static_cast<char*>(workspace), n, B);
+    return 0;
+}
+
+}  // namespace
+}  // namespace ash
+
+using namespace ash;
+
+extern "C" {
+
+int64_t ash_surface_block8_workspace_bytes(int64_t num_grids, int64_t num_embeddings) {
+    if (num_grids < 0 || num_embeddings < 1) return 0;
+    Work w;
+    return lay_out(w, nullptr, num_grids, num_embeddings);
+}
+
+int ash_surface_block8_classify(ash_map_t* map, const void* sdfs, int64_t sdf_stride,
+                                const void* weights, int64_t weight_stride,
+                                const int64_t* grid_indices, const int64_t* lut_grid_nb2grid_idx,
+                                int64_t num_grids, int64_t num_embeddings, float iso_value,
+                                float weight_thr, int32_t dtype, void* workspace, int64_t out[2],
+                                void* stream) {
+    if (map == nullptr) ASH_FAIL("null map handle");
+    if (out == nullptr) ASH_FAIL("null output pointer");
+    SurfaceArgs a = {};
+    if (fill(a, sdfs, sdf_stride, grid_indices, lut_grid_nb2grid_idx, num_grids, num_embeddings,
+             iso_value, dtype, workspace)) {
+        return 1;
+    }
+    if (weight_stride < 1 || weight_stride > kMaxStride) ASH_FAIL("surface extraction: bad stride");
+    out[0] = out[1] = 0;
+    if (num_grids == 0) return 0;
+    if (weights == nullptr) ASH_FAIL("null pointer in surface extraction");
+    a.weights = weights;
+    a.weight_stride = weight_stride;
+    a.weight_thr = weight_thr;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (is_capturing(s)) {
+        ASH_FAIL("the number of triangles cannot be read while the stream is being captured");
+    }
+    DeviceGuard guard;
+    ASH_HIP(guard.enter(map->device));
+    std::lock_guard<std::mutex> one_answer(map->pair_lock);
+    if (take_line(map)) return 1;
+    const int64_t units = num_embeddings * 8;
+    clear_bits_kernel<<<static_cast<unsigned>((units + kBlock - 1) / kBlock), kBlock, 0, s>>>(
+            reinterpret_cast<uint4*>(a.w.bits), units);
+    ASH_LAUNCH_CHECK();
+    const unsigned by_four = static_cast<unsigned>((num_grids + kBlock / 64 - 1) / (kBlock / 64));
+    if (dtype == ASH_F32) {
+        bits_kernel<float><<<by_four, kBlock, 0, s>>>(a);
+    } else {
+        bits_kernel<double><<<by_four, kBlock, 0, s>>>(a);
+    }
+    ASH_LAUNCH_CHECK();
+    classify_kernel<<<walk_grid(num_grids), 64, 0, s>>>(a);
+    ASH_LAUNCH_CHECK();
+    const int64_t groups = groups_of(num_grids);
+    count_kernel<<<static_cast<unsigned>(groups), kCountThreads, 0, s>>>(a);
+    ASH_LAUNCH_CHECK();
+    int32_t* landing = map->line + kLinePair;
+    const int32_t stamp = ++map->stamp;
+    scan_groups_kernel<<<1, kScanThreads, 0, s>>>(a.w.groups, groups, landing, stamp);
+    ASH_LAUNCH_CHECK();
+    if (wait_for_stamp(landing + kLandingStamp, stamp)) return 1;
+    for (int w = 0; w < 2; ++w) {
+        out[w] = static_cast<int64_t>(static_cast<uint32_t>(landing[2 * w])) |
+                 (static_cast<int64_t>(landing[2 * w + 1]) << 32);
+    }
+    if (out[0] > 0x7FFFFFFFll) ASH_FAIL("marching_cubes: more than 2^31 vertices");
+    if (out[1] > 0x7FFFFFFFll / 3) ASH_FAIL("marching_cubes: too many triangles");
+    return 0;
+}
+
+int ash_surface_block8_extract(const void* sdfs, int64_t sdf_stride, const int64_t* grid_indices,
+                               const int32_t* grid_coords_table,
+                               const int64_t* lut_grid_nb2grid_idx, int64_t num_grids,
+                               int64_t num_embeddings, float iso_value, int32_t dtype,
+                               void* workspace, int64_t n_vertices, int64_t n_triangles,
+                               int to_world, float cell_to_world, const float* origin,
+                               float* positions, int32_t* triangles, void* stream) {
+    SurfaceArgs a = {};
+    if (fill(a, sdfs, sdf_stride, grid_indices, lut_grid_nb2grid_idx, num_grids, num_embeddings,
+             iso_value, dtype, workspace)) {
+        return 1;
+    }
+    if (n_vertices < 0 || n_triangles < 0) ASH_FAIL("marching_cubes: negative counts");
+    if (num_grids == 0 || n_vertices == 0) return 0;
+    if (grid_coords_table == nullptr || positions == nullptr || (n_triangles > 0 && triangles == nullptr)) {
+        ASH_FAIL("null pointer in marching_cubes");
+    }
+    a.grid_coords = grid_coords_table;
+    a.to_world = to_world != 0;
+    a.scale = cell_to_world;
+    a.origin = origin;
+    a.n_points = n_vertices;
+    a.n_triangles = n_triangles;
+    a.positions = positions;
+    a.triangles = triangles;
+    PointerGuard guard;
+    ASH_HIP(guard.enter_for(sdfs));
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (dtype == ASH_F32) {
+        points_kernel<float><<<walk_grid(num_grids), 64, 0, s>>>(a);
+    } else {
+        points_kernel<double><<<walk_grid(num_grids), 64, 0, s>>>(a);
+    }
+    ASH_LAUNCH_CHECK();
+    if (n_triangles > 0) {
+        triangles_kernel<<<walk_grid(num_grids), 64, 0, s>>>(a);
+        ASH_LAUNCH_CHECK();
+    }
+    return 0;
+}
+
+}  // extern "C"

@@ -272,7 +272,8 @@ convolution_block8_kernel(ConvArgs a) {
             for (int i = 0; i < S::kOwnEach; ++i) {
                 const int f = tid + i * S::kThreads;
                 const int out_z = f / (16 * E);
-                rows[f] = *reinterpret_cast<const v4*>(s_out + 4 * f + 4 * out_z);
+                __builtin_nontemporal_store(*reinterpret_cast<const v4*>(s_out + 4 * f + 4 * out_z),
+                                            rows + f);
             }
         }
     }

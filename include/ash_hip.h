@@ -310,15 +310,23 @@ int ash_ray_sample_compact(const int64_t* counts, const int64_t* prefix, const f
  * otherwise the march has to be run again by ash_ray_sample.  ray_nears /
  * ray_fars: n values in world units, or NULL for near_for_all / far_for_all
  * (cell units) on every ray.  counts: int64[n]; groups: 2 *
- * ash_ray_sample_groups(n) int64 on the device. */
-int ash_ray_find_near_far_world(ash_map_t* map, const float* ray_origins,
+ * ash_ray_sample_groups(n) int64 on the device.
+ * volume: scratch of ash_ray_volume_bytes(volume_lo, volume_hi, n, sampling) bytes
+ * (sampling: 0 for near_far, 1 for the march), 16-byte aligned, for a map of the
+ * blocks volume_lo .. volume_hi (on every axis) that the call makes and then asks
+ * instead of the table, or NULL; where that function returns 0 there is none.
+ * Blocks outside are looked up as ever. */
+int64_t ash_ray_volume_bytes(int lo, int hi, int64_t n, int sampling);
+int ash_ray_find_near_far_world(ash_map_t* map, uint8_t* volume, int volume_lo,
+                                int volume_hi, const float* ray_origins,
                                 const float* ray_directions, const float* origin,
                                 float cell_size, const float* bbox_min,
                                 const float* bbox_max, int64_t n, float t_min,
                                 float t_max, float grid2cell_multiplier,
                                 float* ray_nears, float* ray_fars, void* stream);
 int64_t ash_ray_sample_groups(int64_t n);
-int ash_ray_sample_march(ash_map_t* map, const float* ray_origins,
+int ash_ray_sample_march(ash_map_t* map, uint8_t* volume, int volume_lo, int volume_hi,
+                         const float* ray_origins,
                          const float* ray_directions, const float* origin,
                          float cell_size, const float* ray_nears, const float* ray_fars,
                          float near_for_all, float far_for_all, int64_t n,

@@ -134,9 +134,11 @@ _SIGNATURES = {
         [_PTR] * 5 + [_I64, _I64, ctypes.c_float, _PTR, _PTR, _I64, _PTR],
     ),
     "ash_ray_sample_compact": (ctypes.c_int, [_PTR] * 3 + [_I64, _I64] + [_PTR] * 4),
+    "ash_ray_volume_bytes": (_I64, [ctypes.c_int, ctypes.c_int, _I64, ctypes.c_int]),
     "ash_ray_find_near_far_world": (
         ctypes.c_int,
-        [_PTR] * 4 + [ctypes.c_float, _PTR, _PTR, _I64] + [ctypes.c_float] * 3 + [_PTR] * 3,
+        [_PTR, _PTR, ctypes.c_int, ctypes.c_int] + [_PTR] * 3
+        + [ctypes.c_float, _PTR, _PTR, _I64] + [ctypes.c_float] * 3 + [_PTR] * 3,
     ),
     "ash_surface_block8_workspace_bytes": (_I64, [_I64, _I64]),
     "ash_surface_block8_classify": (
@@ -152,8 +154,9 @@ _SIGNATURES = {
     "ash_ray_sample_groups": (_I64, [_I64]),
     "ash_ray_sample_march": (
         ctypes.c_int,
-        [_PTR] * 4 + [ctypes.c_float, _PTR, _PTR, ctypes.c_float, ctypes.c_float, _I64, _I64,
-                      ctypes.c_float, _PTR, _PTR, _PTR, _I64, ctypes.POINTER(_I64), _PTR],
+        [_PTR, _PTR, ctypes.c_int, ctypes.c_int] + [_PTR] * 3
+        + [ctypes.c_float, _PTR, _PTR, ctypes.c_float, ctypes.c_float, _I64, _I64,
+           ctypes.c_float, _PTR, _PTR, _PTR, _I64, ctypes.POINTER(_I64), _PTR],
     ),
     "ash_ray_sample_place": (
         ctypes.c_int, [_PTR] * 3 + [_I64, _I64, ctypes.c_float] + [_PTR] * 5,
@@ -637,18 +640,19 @@ class _Backend:
 
     def ray_find_near_far_world(
         self, hashmap, ray_origins, ray_directions, origin, cell_size, bbox_min, bbox_max, t_min,
-        t_max, grid2cell_multiplier,
+        t_max, grid2cell_multiplier, block_bounds=(0, -1),
     ) -> Tuple[torch.Tensor, torch.Tensor]:
         """ray_find_near_far of world rays with cell units = (x - origin) /
         cell_size: the transforms of rays, box and results in the same launch
-        (t_min and t_max in cell units)."""
+        (t_min and t_max in cell units).  block_bounds: where the blocks of the
+        grid lie (lo, hi; a range that is small enough speeds the look-ups up)."""
         return self.host.ray_near_far(hashmap._address, hashmap._index, ray_origins, ray_directions,
                                       origin, cell_size, bbox_min, bbox_max, t_min, t_max,
-                                      grid2cell_multiplier)
+                                      grid2cell_multiplier, *block_bounds)
 
     def ray_sample_world(
         self, hashmap, ray_origins, ray_directions, origin, cell_size, ray_nears, ray_fars,
-        max_samples_per_ray, grid2cell_multiplier,
+        max_samples_per_ray, grid2cell_multiplier, block_bounds=(0, -1),
     ):
         """ray_sample of world rays, everything in world units; None where the
         samples do not fit a staging area (`ray_sample` takes such rays)."""
@@ -657,7 +661,7 @@ class _Backend:
             return None
         return self.host.ray_sample(hashmap._address, hashmap._index, ray_origins, ray_directions,
                                     origin, cell_size, ray_nears, ray_fars, int(max_samples_per_ray),
-                                    grid2cell_multiplier, stride)
+                                    grid2cell_multiplier, stride, *block_bounds)
 
     def ray_sample(
         self, hashmap, ray_origins, ray_directions, ray_nears, ray_fars, bbox_min, bbox_max,

@@ -504,7 +504,7 @@ class SparseDenseGrid(ASHModule):
             # transforms, march, running sums and results in three launches
             samples = backend.ray_sample_world(
                 self.engine.backend, rays_o, rays_d, *affine, rays_near, rays_far,
-                max_samples_per_ray, float(self.grid_dim))
+                max_samples_per_ray, float(self.grid_dim), self._block_bounds())
             if samples is not None:
                 return samples
         bbox_min, bbox_max = self.get_bbox()
@@ -534,7 +534,8 @@ class SparseDenseGrid(ASHModule):
         ):
             return backend.ray_find_near_far_world(
                 self.engine.backend, rays_o, rays_d, *affine, bbox_min, bbox_max,
-                t_min / self.cell_size, t_max / self.cell_size, float(self.grid_dim))
+                t_min / self.cell_size, t_max / self.cell_size, float(self.grid_dim),
+                self._block_bounds())
         ray_nears, ray_fars = backend.ray_find_near_far(
             self.engine.backend,
             self.transform_world_to_cell(rays_o),

@@ -42,6 +42,7 @@ namespace py = pybind11;
     X(ash_map_upkeep)                                                                 \
     X(ash_map_neighbors)                                                              \
     X(ash_grid_fuse_frame)                                                            \
+    X(ash_ray_volume_bytes)                                                           \
     X(ash_ray_find_near_far_world)                                                    \
     X(ash_ray_sample_groups)                                                          \
     X(ash_ray_sample_march)                                                           \
@@ -417,17 +418,25 @@ struct RayOperands {
     }
 };
 
+// Scratch for the map of the blocks in bounds, undefined where there is none
+Tensor ray_volume(int lo, int hi, int64_t n, bool sampling, int64_t device) {
+    const int64_t bytes = lib.ash_ray_volume_bytes(lo, hi, n, sampling);
+    return bytes > 0 ? empty({bytes}, at::kByte, device) : Tensor();
+}
+
 std::tuple<Tensor, Tensor> ray_near_far(uintptr_t handle, int64_t device, const Tensor& origins,
                                         const Tensor& directions, const Optional& origin,
                                         double cell_size, const Tensor& bbox_min, const Tensor& bbox_max,
-                                        double t_min, double t_max, double grid2cell) {
+                                        double t_min, double t_max, double grid2cell, int block_lo,
+                                        int block_hi) {
     const RayOperands r(origins, directions, origin, device);
     const Tensor lo = floats_on(bbox_min, device), hi = floats_on(bbox_max, device);
     need(lo.numel() == 3 && hi.numel() == 3, "the box has three coordinates per corner");
     const int64_t n = r.o.size(0);
     Tensor nears = empty({n}, at::kFloat, device), fars = empty({n}, at::kFloat, device);
+    const Tensor volume = ray_volume(block_lo, block_hi, n, false, device);
     check(lib.ash_ray_find_near_far_world(
-            map_of(handle), ptr<float>(r.o), ptr<float>(r.d), ptr<float>(r.origin),
+            map_of(handle), ptr<uint8_t>(volume), block_lo, block_hi, ptr<float>(r.o), ptr<float>(r.d), ptr<float>(r.origin),
             static_cast<float>(cell_size), ptr<float>(lo), ptr<float>(hi), n, static_cast<float>(t_min),
             static_cast<float>(t_max), static_cast<float>(grid2cell), ptr<float>(nears),
             ptr<float>(fars), stream_of(device)));
@@ -453,21 +462,22 @@ struct RayRange {
 std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> ray_sample(
         uintptr_t handle, int64_t device, const Tensor& origins, const Tensor& directions,
         const Optional& origin, double cell_size, const py::object& nears, const py::object& fars,
-        int64_t max_samples, double grid2cell, int64_t stride) {
+        int64_t max_samples, double grid2cell, int64_t stride, int block_lo, int block_hi) {
     const RayOperands r(origins, directions, origin, device);
     const int64_t n = r.o.size(0);
     const RayRange near(nears, cell_size, n, device), far(fars, cell_size, n, device);
     const Tensor counts = empty({n}, at::kLong, device), prefix = empty({n}, at::kLong, device);
     const Tensor groups = empty({lib.ash_ray_sample_groups(n), 2}, at::kLong, device);
     const Tensor stage = empty({n, stride, 2}, at::kFloat, device);
+    const Tensor volume = ray_volume(block_lo, block_hi, n, true, device);
     void* stream = stream_of(device);
     int64_t out[2] = {0, 0};
     int status;
     {
         py::gil_scoped_release waits_for_the_device;
         status = lib.ash_ray_sample_march(
-                map_of(handle), ptr<float>(r.o), ptr<float>(r.d), ptr<float>(r.origin),
-                static_cast<float>(cell_size), ptr<float>(near.each), ptr<float>(far.each),
+                map_of(handle), ptr<uint8_t>(volume), block_lo, block_hi, ptr<float>(r.o),
+                ptr<float>(r.d), ptr<float>(r.origin), static_cast<float>(cell_size), ptr<float>(near.each), ptr<float>(far.each),
                 near.for_all, far.for_all, n, max_samples, static_cast<float>(grid2cell),
                 ptr<int64_t>(counts), ptr<int64_t>(groups), ptr<float>(stage), stride, out, stream);
     }

@@ -37,6 +37,77 @@ __device__ __forceinline__ bool uniform(bool c) {
     return __builtin_amdgcn_readfirstlane(static_cast<int>(c)) != 0;
 }
 
+// A byte per block of the cube lo .. lo + edge - 1 (each axis), 1 where the block
+// is stored, in bricks of 4 x 4 x 8 blocks: a ray stays within a line of 128 for
+// some eight steps.  With it a look-up is one load and fifteen instructions
+// instead of the six loads and eighty of a bucket.
+struct Volume {
+    const uint8_t* at;   // null: none
+    int32_t lo;
+    uint32_t edge;
+};
+
+// More than this does not stay in an XCD's L2.
+constexpr int64_t kMaxVolume = int64_t{4} << 20;
+// Making it takes two launches of 4 us each, which so many rays gain back: near
+// and far of 2000 rays 16 -> 16 us, 8000 30 -> 20, 32 768 83 -> 35; samples of
+// 8000 rays 32 - 57 -> 36 - 48 (few blocks and short rays - many and long),
+// 32 768 37 - 77 -> 38 - 55.
+constexpr int64_t kVolumeRaysNearFar = 4096, kVolumeRaysSampling = 8192;
+
+__host__ __device__ __forceinline__ int64_t volume_bytes(int64_t edge) {
+    const int64_t flat = (edge + 3) / 4, tall = (edge + 7) / 8;
+    return flat * flat * tall * 128;
+}
+
+__device__ __forceinline__ bool in_volume(const Volume& v, const int32_t (&block)[3], uint32_t& at) {
+    uint32_t p[3];
+    bool inside = true;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        p[a] = static_cast<uint32_t>(block[a]) - static_cast<uint32_t>(v.lo);
+        inside = inside && p[a] < v.edge;
+    }
+    const uint32_t flat = (v.edge + 3) >> 2;
+    at = (((p[2] >> 3) * flat + (p[1] >> 2)) * flat + (p[0] >> 2)) * 128u + (p[0] & 3u) +
+         4u * (p[1] & 3u) + 16u * (p[2] & 7u);
+    return inside;
+}
+
+__global__ __launch_bounds__(kBlock) void clear_volume_kernel(uint4* __restrict__ to, int64_t units) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    if (i < units) to[i] = make_uint4(0u, 0u, 0u, 0u);
+}
+
+// Marks the stored blocks, from the log (keys of the general region lie outside
+// every cube that fits).
+__global__ __launch_bounds__(kBlock) void mark_volume_kernel(MapDev m, int identity, Volume v,
+                                                             uint8_t* __restrict__ to) {
+    const int64_t limit = identity ? static_cast<int64_t>(m.ctr[kCtrSize])
+                                   : static_cast<int64_t>(m.capacity);
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    const uint64_t code = i < limit ? m.klog[i] : kEmpty;
+    if (code >= kTomb) return;
+    int32_t block[3];
+    unpack_key<3>(code, block);
+    uint32_t at;
+    if (in_volume(v, block, at)) to[at] = 1;
+}
+
+// Whether the block is stored, every lane for itself.
+__device__ __forceinline__ bool is_stored(const MapDev& m, const Volume& v, const int32_t (&block)[3],
+                                          bool active) {
+    uint32_t at;
+    const bool inside = in_volume(v, block, at);
+    bool stored = false;
+    if (active && inside) stored = v.at[at] != 0;
+    if (active && !inside) {
+        int32_t idx;
+        stored = find_key_alone<3>(m, block, true, idx);
+    }
+    return stored;
+}
+
 __device__ __forceinline__ void ray_block(const float (&o)[3], const float (&d)[3],
                                           float t, float cell2grid,
                                           int32_t (&block)[3], float (&x)[3]) {
@@ -45,6 +116,18 @@ __device__ __forceinline__ void ray_block(const float (&o)[3], const float (&d)[
         x[a] = fmaf(t, d[a], o[a]);
         block[a] = static_cast<int32_t>(floorf(__fmul_rn(x[a], cell2grid)));
     }
+}
+
+// The same from the table; the first lane of a run of equal blocks asks.
+__device__ __forceinline__ bool is_stored_by_runs(const MapDev& m, const int32_t (&block)[3], bool active) {
+    const int lane = threadIdx.x & 63;
+    int same = lane > 0 && active && lane_before(static_cast<int32_t>(active)) != 0;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) same &= lane_before(block[a]) == block[a];
+    int32_t idx;
+    const bool asked = find_key_alone<3>(m, block, active && !same, idx);
+    const uint64_t heads = __ballot(!same);
+    return __shfl(static_cast<int>(asked), 63 - __builtin_clzll(heads & (~0ull >> (63 - lane)))) != 0;
 }
 
 // One wavefront per ray: the march of ray_find_near_far visits the parameters
@@ -66,8 +149,9 @@ struct StepChain {
     float t[kChain];
 };
 
+template <bool VOLUME>
 __global__ __launch_bounds__(kBlock) void ray_near_far_kernel(
-        MapDev m, const float* __restrict__ origins,
+        MapDev m, Volume volume, const float* __restrict__ origins,
         const float* __restrict__ directions, RayUnits u, const float* __restrict__ bbox_min,
         const float* __restrict__ bbox_max, int64_t n, float t_min, float t_max,
         float grid2cell, float* __restrict__ nears, float* __restrict__ fars, StepChain chain) {
@@ -100,11 +184,16 @@ __global__ __launch_bounds__(kBlock) void ray_near_far_kernel(
         for (int a = 0; a < 3; ++a) go = go && x[a] >= lo[a] && x[a] <= hi[a];
         const uint64_t stop = __ballot(!go);
         const int first_stop = stop ? __builtin_ctzll(stop) : 64;
-        // (steps are half a block apart: neighbouring lanes often stand in the
-        // same block and share a look-up)
-        int32_t idx;
         const bool active = lane < first_stop;
-        const bool found = find_block_by_runs(m, block, active, idx);
+        bool found;
+        if constexpr (VOLUME) {
+            found = is_stored(m, volume, block, active);
+        } else {
+            // (steps are half a block apart: neighbouring lanes often stand in the
+            // same block and share a look-up)
+            int32_t idx;
+            found = find_block_by_runs(m, block, active, idx);
+        }
         uint64_t hits = __ballot(found && active);
         if (hits) {
             far = fminf(lane_value(t, 63 - __builtin_clzll(hits)) + t_grid_step, t_max);
@@ -131,13 +220,6 @@ __global__ __launch_bounds__(kBlock) void ray_near_far_kernel(
     }
 }
 
-// What the sampling march knows of a ray: a lane's block and whether it is
-// stored.
-struct KnownBlock {
-    int32_t at[3];
-    bool have, stored;
-};
-
 // The march of ray_sample.  counts != nullptr: allocation pass; otherwise the
 // assignment pass, which writes the samples of ray i at prefix[i - 1] ..
 // prefix[i].  An allocation pass with `stage` also keeps the first `stride`
@@ -146,20 +228,20 @@ struct KnownBlock {
 // leaves the sum and the largest of its workgroup's counts there.
 //
 // The reference looks the block under t up at every step, one dependent look-up
-// after the other; where the march may stand next is known beforehand, though.
-// LPR = 8: the eight lanes of a ray look up the block under t, the blocks where
-// four steps on through stored blocks lead, and those where three steps over
-// empty ones lead, all at once, and the march goes on without memory until it
-// stands in a block that none of the lanes holds, which starts the next round.  LPR = 1: every lane marches a ray of its own and
-// answers from its latest look-up while it stays in the same block, which takes
-// fewer instructions where there are rays enough to hide the look-ups.
+// after the other.  What it does next depends on one bit only, though, so the
+// LPR lanes of a ray stand on the next LPR positions of the march as it goes on
+// if all of them are stored (or all are not: whichever the latest one was), look
+// them up at once, and the march takes as many of these steps as turn out that
+// way, and the first one that does not.  (32 768 rays of 31 samples in 200 000
+// blocks: 113 us when the eight lanes looked blocks up ahead and a step went by
+// whether one of them held the block under t, 55 now.)
 struct GroupSamples {
     int64_t sum, most;
 };
 
-template <int LPR>
+template <int LPR, bool VOLUME>
 __global__ __launch_bounds__(kBlock) void ray_sample_kernel(
-        MapDev m, const float* __restrict__ origins,
+        MapDev m, Volume volume, const float* __restrict__ origins,
         const float* __restrict__ directions, RayUnits u, const float* __restrict__ ray_nears,
         const float* __restrict__ ray_fars, float near_for_all, float far_for_all, int64_t n,
         float max_samples, float grid2cell, int64_t* __restrict__ counts,
@@ -169,7 +251,7 @@ __global__ __launch_bounds__(kBlock) void ray_sample_kernel(
     const int lane = threadIdx.x & 63;
     const int64_t gid = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
     const int64_t i = gid / LPR;
-    const int j = LPR == 1 ? 0 : static_cast<int>(gid % LPR);
+    const int j = static_cast<int>(gid % LPR);
     const bool writer = j == 0;   // the lane of a ray that stores its results
     const bool active = i < n;
     const float cell2grid = static_cast<float>(1.0 / grid2cell);
@@ -188,80 +270,64 @@ __global__ __launch_bounds__(kBlock) void ray_sample_kernel(
     float t = ray_near, t_near = ray_near;
     int64_t local = 0;
     bool live = active && t < ray_far;
-    // One step of the march, given whether the block under t is stored.
-    auto step = [&](bool stored) {
-        const float before = t;
-        if (!stored) {
-            t += t_grid_step;
-        } else {
-            t += t_step;
-            if (!writer) {
-            } else if (counts == nullptr) {
-                ray_indices[start + local] = i;
-                t_nears[start + local] = t_near;
-                t_fars[start + local] = t;
-            } else if (stage != nullptr && local < stride) {
-                stage[i * stride + local] = make_float2(t_near, t);
-            }
-            t_near = t;
-            ++local;
+    auto keep = [&](int64_t k, float from, float to) {
+        if (counts == nullptr) {
+            ray_indices[start + k] = i;
+            t_nears[start + k] = from;
+            t_fars[start + k] = to;
+        } else if (stage != nullptr && k < stride) {
+            stage[i * stride + k] = make_float2(from, to);
         }
-        // a step that no longer advances t (range far beyond fp32
-        // resolution) would never end; the reference has no such guard
-        live = t < ray_far && t > before;
     };
-    KnownBlock known = {{0, 0, 0}, false, false};
-    // how far ahead of t this lane looks: half a block or a step, whichever is
-    // more, at a time for lanes 1..4, empty steps for lanes 5..7
-    const float ahead = j < 5 ? static_cast<float>(j) * fmaxf(t_step, 0.5f * grid2cell)
-                              : static_cast<float>(j - 4) * t_grid_step;
+    const int shift = lane & ~(LPR - 1);
+    const uint64_t all = LPR == 64 ? ~0ull : (1ull << LPR) - 1ull;
+    bool run_stored = true;   // what the positions ahead are taken for
     while (__ballot(live)) {
-        int32_t block[3] = {0, 0, 0};
+        const float by = run_stored ? t_step : t_grid_step;
+        float at = t, before = -INFINITY;
+#pragma unroll
+        for (int k = 1; k < LPR; ++k) {
+            before = j >= k ? at : before;
+            at = j >= k ? at + by : at;
+        }
+        const float next = at + by;
+        // (a step that no longer advances t -- range far beyond fp32 resolution --
+        // would never end; the reference has no such guard)
+        const bool stands = live && at < ray_far && at > before;
+        int32_t block[3];
         float x[3];
-        bool ask = false;
-        while (live) {
-            ray_block(o, d, t, cell2grid, block, x);
-            const bool here = known.have && block[0] == known.at[0] && block[1] == known.at[1] &&
-                              block[2] == known.at[2];
-            if constexpr (LPR == 1) {
-                if (!here) {
-                    ask = true;
-                    break;
-                }
-                step(known.stored);
-            } else {
-                // (the lanes of a ray are in this loop together or not at all)
-                const uint32_t shift = lane & ~(LPR - 1);
-                const uint32_t any = static_cast<uint32_t>(__ballot(here) >> shift) & ((1u << LPR) - 1u);
-                if (any == 0u) {
-                    ask = true;
-                    break;
-                }
-                const uint32_t stored = static_cast<uint32_t>(__ballot(here && known.stored) >> shift) &
-                                        ((1u << LPR) - 1u);
-                step(stored != 0u);
-            }
+        ray_block(o, d, at, cell2grid, block, x);
+        bool stored;
+        if constexpr (VOLUME) {
+            stored = is_stored(m, volume, block, stands);
+        } else {
+            stored = is_stored_by_runs(m, block, stands);
         }
-        bool mine = live && ask;
-        if constexpr (LPR > 1) {
-            // the lane's own block ahead; the lane before it may hold the same
-            if (mine && j > 0) {
-                ray_block(o, d, t + ahead, cell2grid, block, x);
-                mine = t + ahead < ray_far;
-            }
-            int same = 1;
-#pragma unroll
-            for (int a = 0; a < 3; ++a) same &= lane_before(block[a]) == block[a];
-            if (j > 0 && same) mine = false;
+        const uint64_t others = (__ballot(!stands || stored != run_stored) >> shift) & all;
+        const uint64_t ends = (__ballot(!stands) >> shift) & all;
+        // steps taken, and whether the march then stands on the other kind
+        const int run = others == 0 ? LPR : __builtin_ctzll(others);
+        const bool turn = others != 0 && ((ends >> run) & 1ull) == 0;
+        const float reached = run > 0 ? __shfl(next, shift + run - 1) : t;
+        const float last = run > 0 ? __shfl(at, shift + run - 1) : -INFINITY;
+        if (!live) continue;
+        if (run_stored) {
+            if (j < run) keep(local + j, j > 0 ? at : t_near, next);
+            local += run;
+            if (run > 0) t_near = reached;
         }
-        int32_t idx;
-        const bool stored = find_key_alone<3>(m, block, mine, idx);
-        if (live && ask) {
-#pragma unroll
-            for (int a = 0; a < 3; ++a) known.at[a] = block[a];
-            known.have = mine;
-            known.stored = stored && mine;
-            if constexpr (LPR == 1) step(stored);
+        t = reached;
+        live = t < ray_far && t > last;
+        if (turn) {
+            const float from = t;
+            run_stored = !run_stored;
+            t += run_stored ? t_step : t_grid_step;
+            if (run_stored) {
+                if (writer) keep(local, t_near, t);
+                ++local;
+                t_near = t;
+            }
+            live = t < ray_far && t > from;
         }
     }
     if (active && writer && counts != nullptr) counts[i] = local;
@@ -400,11 +466,13 @@ __global__ __launch_bounds__(kBlock) void ray_compact_kernel(
     t_fars[out] = s.y;
 }
 
-// Lanes per ray of the sampling march: below this many rays there are not
-// enough wavefronts to hide a look-up per block, see ray_sample_kernel.
-constexpr int64_t kRaysPerLaneMin = int64_t{1} << 16;
+// Lanes per ray of the sampling march: eight, and four where there are rays
+// enough that the positions looked up in vain weigh more than the rounds (100 000
+// rays of up to 32 / 128 samples: 57 / 96 us and 46 / 90; 8000 rays: 39 / 48 and
+// 39 / 55).
+constexpr int64_t kFewLanesFrom = int64_t{1} << 16;
 
-int lanes_per_ray(int64_t n) { return n < kRaysPerLaneMin ? 8 : 1; }
+int lanes_per_ray(int64_t n) { return n < kFewLanesFrom ? 8 : 4; }
 
 unsigned march_groups(int64_t n) {
     return static_cast<unsigned>((n * lanes_per_ray(n) + kBlock - 1) / kBlock);
@@ -419,14 +487,35 @@ struct March {
     float max_samples, grid2cell;
 };
 
-int launch_march(ash_map_t* map, const March& r, int64_t* counts, const int64_t* prefix,
+int launch_march(ash_map_t* map, const Volume& volume, const March& r, int64_t* counts, const int64_t* prefix,
                  int64_t* ray_indices, float* t_nears, float* t_fars, float* stage, int64_t stride,
                  GroupSamples* groups, hipStream_t s) {
-    auto kernel = lanes_per_ray(r.n) == 8 ? ray_sample_kernel<8> : ray_sample_kernel<1>;
+    const bool eight = lanes_per_ray(r.n) == 8;
+    auto kernel = volume.at != nullptr
+                          ? (eight ? ray_sample_kernel<8, true> : ray_sample_kernel<4, true>)
+                          : (eight ? ray_sample_kernel<8, false> : ray_sample_kernel<4, false>);
     kernel<<<march_groups(r.n), kBlock, 0, s>>>(
-            map->d, r.origins, r.directions, r.units, r.nears, r.fars, r.near_for_all, r.far_for_all,
+            map->d, volume, r.origins, r.directions, r.units, r.nears, r.fars, r.near_for_all, r.far_for_all,
             r.n, r.max_samples, r.grid2cell, counts, prefix, ray_indices, t_nears, t_fars,
             reinterpret_cast<float2*>(stage), stride, groups);
+    ASH_LAUNCH_CHECK();
+    return 0;
+}
+
+// The volume of the map's blocks in lo .. hi, if there is room for one.
+int make_volume(ash_map_t* map, uint8_t* bytes, int lo, int hi, Volume& v, hipStream_t s) {
+    v = {};
+    if (bytes == nullptr) return 0;
+    const int64_t edge = static_cast<int64_t>(hi) - lo + 1;
+    if (edge < 1 || volume_bytes(edge) > kMaxVolume) ASH_FAIL("rays: too many blocks for a volume");
+    if (reinterpret_cast<uintptr_t>(bytes) % 16 != 0) ASH_FAIL("rays: the volume must be 16-byte aligned");
+    v = {bytes, lo, static_cast<uint32_t>(edge)};
+    const int64_t units = volume_bytes(edge) / 16;
+    clear_volume_kernel<<<static_cast<unsigned>((units + kBlock - 1) / kBlock), kBlock, 0, s>>>(
+            reinterpret_cast<uint4*>(bytes), units);
+    ASH_LAUNCH_CHECK();
+    mark_volume_kernel<<<static_cast<unsigned>((map->capacity + kBlock - 1) / kBlock), kBlock, 0, s>>>(
+            map->d, heap_in_order(map) ? 1 : 0, v, bytes);
     ASH_LAUNCH_CHECK();
     return 0;
 }
@@ -445,7 +534,7 @@ int check_rays(const ash_map_t* map, const float* origins, const float* directio
     return 0;
 }
 
-int near_far(ash_map_t* map, const float* origins, const float* directions, const RayUnits& units,
+int near_far(ash_map_t* map, uint8_t* bytes, int lo, int hi, const float* origins, const float* directions, const RayUnits& units,
              const float* bbox_min, const float* bbox_max, int64_t n, float t_min, float t_max,
              float grid2cell, float* nears, float* fars, hipStream_t s) {
     if (check_rays(map, origins, directions, n, grid2cell, units.cell)) return 1;
@@ -465,14 +554,17 @@ int near_far(ash_map_t* map, const float* origins, const float* directions, cons
             ASH_FAIL("ray_find_near_far: the step is too small for this range");
         }
     }
+    Volume volume;
+    if (make_volume(map, bytes, lo, hi, volume, s)) return 1;
     StepChain chain;
     float t = t_min;
     for (int k = 0; k < kChain; ++k) {
         chain.t[k] = t;
         t += half_block;
     }
-    ray_near_far_kernel<<<static_cast<unsigned>((n + kBlock / 64 - 1) / (kBlock / 64)), kBlock, 0, s>>>(
-            map->d, origins, directions, units, bbox_min, bbox_max, n, t_min, t_max, grid2cell,
+    auto kernel = volume.at != nullptr ? ray_near_far_kernel<true> : ray_near_far_kernel<false>;
+    kernel<<<static_cast<unsigned>((n + kBlock / 64 - 1) / (kBlock / 64)), kBlock, 0, s>>>(
+            map->d, volume, origins, directions, units, bbox_min, bbox_max, n, t_min, t_max, grid2cell,
             nears, fars, chain);
     ASH_LAUNCH_CHECK();
     return 0;
@@ -491,17 +583,26 @@ int ash_ray_find_near_far(ash_map_t* map, const float* ray_origins,
                           float t_max, float t_step, float grid2cell_multiplier,
                           float* ray_nears, float* ray_fars, void* stream) {
     (void)t_step;  // unused by the reference as well (ash/src/sampler.cu:21)
-    return near_far(map, ray_origins, ray_directions, kCellUnits, bbox_min, bbox_max, n, t_min,
+    return near_far(map, nullptr, 0, 0, ray_origins, ray_directions, kCellUnits, bbox_min, bbox_max, n, t_min,
                     t_max, grid2cell_multiplier, ray_nears, ray_fars,
                     static_cast<hipStream_t>(stream));
 }
 
-int ash_ray_find_near_far_world(ash_map_t* map, const float* ray_origins,
+int64_t ash_ray_volume_bytes(int lo, int hi, int64_t n, int sampling) {
+    if (n < (sampling ? kVolumeRaysSampling : kVolumeRaysNearFar)) return 0;
+    const int64_t edge = static_cast<int64_t>(hi) - lo + 1;
+    if (edge < 1 || edge > kMaxVolume) return 0;
+    const int64_t bytes = volume_bytes(edge);
+    return bytes <= kMaxVolume ? bytes : 0;
+}
+
+int ash_ray_find_near_far_world(ash_map_t* map, uint8_t* volume, int volume_lo, int volume_hi,
+                                const float* ray_origins,
                                 const float* ray_directions, const float* origin, float cell_size,
                                 const float* bbox_min, const float* bbox_max, int64_t n, float t_min,
                                 float t_max, float grid2cell_multiplier, float* ray_nears,
                                 float* ray_fars, void* stream) {
-    return near_far(map, ray_origins, ray_directions, {origin, 1.0f / cell_size, cell_size}, bbox_min,
+    return near_far(map, volume, volume_lo, volume_hi, ray_origins, ray_directions, {origin, 1.0f / cell_size, cell_size}, bbox_min,
                     bbox_max, n, t_min, t_max, grid2cell_multiplier, ray_nears, ray_fars,
                     static_cast<hipStream_t>(stream));
 }
@@ -526,7 +627,7 @@ int ash_ray_sample(ash_map_t* map, const float* ray_origins,
     ASH_HIP(guard.enter(map->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (settle_table(map, s)) return 1;
-    return launch_march(map, {ray_origins, ray_directions, kCellUnits, ray_nears, ray_fars, 0.f, 0.f, n,
+    return launch_march(map, {}, {ray_origins, ray_directions, kCellUnits, ray_nears, ray_fars, 0.f, 0.f, n,
                               static_cast<float>(max_samples_per_ray), grid2cell_multiplier},
                         counts, prefix, ray_indices, t_nears, t_fars, nullptr, 0, nullptr, s);
 }
@@ -548,7 +649,7 @@ int ash_ray_sample_staged(ash_map_t* map, const float* ray_origins,
     ASH_HIP(guard.enter(map->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (settle_table(map, s)) return 1;
-    return launch_march(map, {ray_origins, ray_directions, kCellUnits, ray_nears, ray_fars, 0.f, 0.f, n,
+    return launch_march(map, {}, {ray_origins, ray_directions, kCellUnits, ray_nears, ray_fars, 0.f, 0.f, n,
                               static_cast<float>(max_samples_per_ray), grid2cell_multiplier},
                         counts, nullptr, nullptr, nullptr, nullptr, stage, stride, nullptr, s);
 }
@@ -573,7 +674,8 @@ int ash_ray_sample_compact(const int64_t* counts, const int64_t* prefix, const f
 
 int64_t ash_ray_sample_groups(int64_t n) { return n > 0 ? static_cast<int64_t>(march_groups(n)) : 0; }
 
-int ash_ray_sample_march(ash_map_t* map, const float* ray_origins, const float* ray_directions,
+int ash_ray_sample_march(ash_map_t* map, uint8_t* scratch, int volume_lo, int volume_hi,
+                         const float* ray_origins, const float* ray_directions,
                          const float* origin, float cell_size, const float* ray_nears,
                          const float* ray_fars, float near_for_all, float far_for_all, int64_t n,
                          int64_t max_samples_per_ray, float grid2cell_multiplier, int64_t* counts,
@@ -599,8 +701,10 @@ int ash_ray_sample_march(ash_map_t* map, const float* ray_origins, const float* 
     if (settle_table(map, s)) return 1;
     std::lock_guard<std::mutex> one_answer(map->pair_lock);
     if (take_line(map)) return 1;
+    Volume volume;
+    if (make_volume(map, scratch, volume_lo, volume_hi, volume, s)) return 1;
     auto* g = reinterpret_cast<GroupSamples*>(groups);
-    if (launch_march(map, {ray_origins, ray_directions, {origin, 1.0f / cell_size, cell_size}, ray_nears,
+    if (launch_march(map, volume, {ray_origins, ray_directions, {origin, 1.0f / cell_size, cell_size}, ray_nears,
                            ray_fars, near_for_all, far_for_all, n,
                            static_cast<float>(max_samples_per_ray), grid2cell_multiplier},
                      counts, nullptr, nullptr, nullptr, nullptr, stage, stride, g, s)) {

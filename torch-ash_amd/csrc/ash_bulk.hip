@@ -67,6 +67,7 @@ enum { kHdrSpillKeys = 0, kHdrSpillA = 1, kHdrWasEmpty = 3,
        kHdrHoles = 6,     // listed holes
        kHdrTaken = 7,     // holes handed to high winners
        kHdrTicket = 8,    // workgroups of pass 1 that are done
+       kHdrTicketLast = 9,   // ... of the last launch
        kHdrWords = 64 };
 
 struct BulkPlan {
@@ -1357,8 +1358,8 @@ int ash_map_bulk_workspace_bytes(ash_map_t* map, int64_t n, int n_values,
 int ash::insert_bulk(ash_map* map, const int32_t* keys, int64_t n,
                      int n_values, const void* const* src, void* const* dst,
                      const int64_t* row_bytes, void* workspace,
-                     int64_t workspace_bytes, int32_t* early, int32_t stamp,
-                     void* stream) {
+                     int64_t workspace_bytes, int32_t* early, int32_t* late, int32_t stamp,
+                     bool* published, void* stream) {
     if (check_batch(map, keys, n)) return 1;
     if (check_values(n_values, src, dst, row_bytes)) return 1;
     if (workspace == nullptr) ASH_FAIL("null bulk workspace");
@@ -1394,6 +1395,18 @@ int ash::insert_bulk(ash_map* map, const int32_t* keys, int64_t n,
     // holds then: a captured call takes the variant that reads the heap)
     const int identity = heap_in_order(map) ? 1 : 0;
 
+    // What the last launch leaves for the host, once the first pass is known to
+    // have handed nothing to the per-key kernel.
+    Publish publish = {};
+    auto none_spilled = [&](Publish& p) -> int {
+        if (early == nullptr) return 0;
+        if (wait_for_stamp(early + kLandingStamp, stamp)) return 1;
+        if (*early == 0) {
+            p = {late, stamp, pl.hdr + kHdrTicketLast};
+            *published = true;
+        }
+        return 0;
+    };
     const int ncursors = static_cast<int>(pl.bins << pl.fine_shift);   // (>= bins << lane_shift)
     const int ninit = ncursors > kHdrWords ? ncursors : kHdrWords;
     bulk_init_kernel<<<(ninit + 255) / 256, 256, 0, s>>>(map->d, pl, ncursors);
@@ -1405,10 +1418,13 @@ int ash::insert_bulk(ash_map* map, const int32_t* keys, int64_t n,
         build_kernel<false><<<pl.parts, kBuildThreads, 0, s>>>(map->d, pl, stale, identity);
         ASH_LAUNCH_CHECK();
         map->table_stale = false;
-        if (insert_selected(map, false, keys, pl.spill_keys, pl.hdr + kHdrSpillKeys, none, s)) {
+        if (none_spilled(publish)) return 1;
+        // (the first pass alone writes that list)
+        if (publish.landing == nullptr &&
+            insert_selected(map, false, keys, pl.spill_keys, pl.hdr + kHdrSpillKeys, none, s)) {
             return 1;
         }
-        return insert_selected(map, true, pl.codes_a, pl.spill_a, pl.hdr + kHdrSpillA, none, s);
+        return insert_selected(map, true, pl.codes_a, pl.spill_a, pl.hdr + kHdrSpillA, none, s, publish);
     }
     if (launch_split_keys<true>(map, pl, keys, identity, early, stamp, s)) return 1;
     split_records_kernel<true><<<(pl.bins << pl.lane_shift) * pl.chunks, kSplitThreads, 0, s>>>(map->d, pl);
@@ -1423,7 +1439,8 @@ int ash::insert_bulk(ash_map* map, const int32_t* keys, int64_t n,
     copy_rows_kernel<<<static_cast<unsigned>(blocks), kCopyThreads, 0, s>>>(map->d, pl, user, identity);
     ASH_LAUNCH_CHECK();
     if (launch_settle_rows(map, pl, keys, user, identity, s)) return 1;
-    return insert_selected(map, false, keys, pl.spill_keys, pl.hdr + kHdrSpillKeys, user, s);
+    if (none_spilled(publish)) return 1;
+    return insert_selected(map, false, keys, pl.spill_keys, pl.hdr + kHdrSpillKeys, user, s, publish);
 }
 
 extern "C" {
@@ -1433,7 +1450,7 @@ int ash_map_insert_bulk(ash_map_t* map, const int32_t* keys, int64_t n,
                         const int64_t* row_bytes, void* workspace,
                         int64_t workspace_bytes, void* stream) {
     return insert_bulk(map, keys, n, n_values, src, dst, row_bytes, workspace, workspace_bytes,
-                       nullptr, 0, stream);
+                       nullptr, nullptr, 0, nullptr, stream);
 }
 
 int ash_map_erase_bulk_query(ash_map_t* map, int64_t n, int64_t* bytes, int* worthwhile) {

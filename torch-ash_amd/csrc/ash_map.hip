@@ -517,6 +517,20 @@ __global__ __launch_bounds__(kHeapBlock) void insert_kernel(
     insert_one<DIM, MODE, false>(m, keys, i, i < n, va, assigned, given);
 }
 
+// The counters, left where the host reads them: `landing` is page-locked host
+// memory, its word kLandingStamp tells the host that the words before it are
+// those of this launch.  For one workgroup.
+__device__ __forceinline__ void leave_counters(const int32_t* ctr, int32_t* landing, int32_t stamp) {
+    if (threadIdx.x < kHostCounters) {
+        const int32_t v = __hip_atomic_load(ctr + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(landing + threadIdx.x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    // (one wavefront: the release waits for the stores of all its lanes)
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(landing + kLandingStamp, stamp, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 // The same insert over a selection made on the device: thread t of the
 // selection handles row sel[t], t < *nsel.  The grid is fixed; workgroups
 // stride over the selection, which is empty in the common case.
@@ -524,7 +538,7 @@ template <int DIM, int MODE, bool CODES>
 __global__ __launch_bounds__(kHeapBlock) void insert_selected_kernel(
         MapDev m, const int32_t* __restrict__ keys,
         const int32_t* __restrict__ sel, const int32_t* __restrict__ nsel,
-        ValueArgs va) {
+        ValueArgs va, Publish publish) {
     const int64_t total = *nsel;
     for (int64_t base = static_cast<int64_t>(blockIdx.x) * kHeapBlock;
          base < total; base += static_cast<int64_t>(gridDim.x) * kHeapBlock) {
@@ -534,6 +548,18 @@ __global__ __launch_bounds__(kHeapBlock) void insert_selected_kernel(
         insert_one<DIM, MODE, CODES>(m, keys, i, active, va, nullptr, nullptr);
         __syncthreads();
     }
+    if (publish.landing == nullptr) return;
+    if (total == 0) {   // nothing has changed the counters
+        if (blockIdx.x != 0) return;
+    } else {            // the workgroup that ends last
+        __shared__ bool s_last;
+        __threadfence();
+        __syncthreads();
+        if (threadIdx.x == 0) s_last = atomicAdd(publish.ticket, 1) == static_cast<int32_t>(gridDim.x) - 1;
+        __syncthreads();
+        if (!s_last) return;
+    }
+    leave_counters(m.ctr, publish.landing, publish.stamp);
 }
 
 // Block activation around a batch of positions (ash/grid.py:121-159): the
@@ -1195,19 +1221,9 @@ __global__ void fold_waiting_keys_kernel(int32_t* ctr) {
     }
 }
 
-// The counters, left where the host reads them: `landing` is page-locked host
-// memory, its word kLandingStamp tells the host that the words before it are
-// those of this launch.
 __global__ void publish_counters_kernel(const int32_t* __restrict__ ctr, int32_t* landing,
                                         int32_t stamp) {
-    if (threadIdx.x < kHostCounters) {
-        __hip_atomic_store(landing + threadIdx.x, ctr[threadIdx.x], __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-    // (one wavefront: the release waits for the stores of all its lanes)
-    if (threadIdx.x == 0) {
-        __hip_atomic_store(landing + kLandingStamp, stamp, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+    leave_counters(ctr, landing, stamp);
 }
 
 // The same with the touched blocks added up first (one workgroup).
@@ -1836,30 +1852,30 @@ int launch_insert(ash_map* map, const int32_t* keys, int64_t n,
 template <int MODE>
 int launch_selected(ash_map* map, bool codes, const int32_t* keys,
                     const int32_t* sel, const int32_t* nsel,
-                    const ValueArgs& va, hipStream_t s) {
+                    const ValueArgs& va, hipStream_t s, const Publish& publish) {
     // the selection is empty or short as a rule: a grid that costs little to
     // launch, whose workgroups stride over a long one
     constexpr unsigned g = 128;
     if (codes) {
         insert_selected_kernel<1, MODE, true>
-                <<<g, kHeapBlock, 0, s>>>(map->d, keys, sel, nsel, va);
+                <<<g, kHeapBlock, 0, s>>>(map->d, keys, sel, nsel, va, publish);
     } else {
         switch (map->key_dim) {
             case 1:
                 insert_selected_kernel<1, MODE, false>
-                        <<<g, kHeapBlock, 0, s>>>(map->d, keys, sel, nsel, va);
+                        <<<g, kHeapBlock, 0, s>>>(map->d, keys, sel, nsel, va, publish);
                 break;
             case 2:
                 insert_selected_kernel<2, MODE, false>
-                        <<<g, kHeapBlock, 0, s>>>(map->d, keys, sel, nsel, va);
+                        <<<g, kHeapBlock, 0, s>>>(map->d, keys, sel, nsel, va, publish);
                 break;
             case 3:
                 insert_selected_kernel<3, MODE, false>
-                        <<<g, kHeapBlock, 0, s>>>(map->d, keys, sel, nsel, va);
+                        <<<g, kHeapBlock, 0, s>>>(map->d, keys, sel, nsel, va, publish);
                 break;
             default:
                 insert_selected_kernel<4, MODE, false>
-                        <<<g, kHeapBlock, 0, s>>>(map->d, keys, sel, nsel, va);
+                        <<<g, kHeapBlock, 0, s>>>(map->d, keys, sel, nsel, va, publish);
                 break;
         }
     }
@@ -1928,12 +1944,12 @@ int erase_selected(ash_map* map, bool codes, const void* keys, const int32_t* se
 
 int insert_selected(ash_map* map, bool codes, const void* keys,
                     const int32_t* sel, const int32_t* nsel,
-                    const ValueArgs& va, hipStream_t s) {
+                    const ValueArgs& va, hipStream_t s, const Publish& publish) {
     const int32_t* k = static_cast<const int32_t*>(keys);
     if (va.n > 0) {
-        return launch_selected<kInsertFused>(map, codes, k, sel, nsel, va, s);
+        return launch_selected<kInsertFused>(map, codes, k, sel, nsel, va, s, publish);
     }
-    return launch_selected<kInsertKeys>(map, codes, k, sel, nsel, va, s);
+    return launch_selected<kInsertKeys>(map, codes, k, sel, nsel, va, s, publish);
 }
 
 }  // namespace ash
@@ -2796,26 +2812,23 @@ int ash_map_insert_auto(ash_map_t* map, const int32_t* keys, int64_t n, int n_va
             early = map->line + kLineEarly;
         }
         const int32_t stamp = ++map->stamp;
+        // Only keys that the first pass hands to the per-key kernel can be
+        // waiting for the second region; their number arrives a quarter into
+        // the call's work.  None: the counters come with the insert's last
+        // launch, and nobody waits for them here.
+        bool published = false;
         if (insert_bulk(map, keys, n, n_values, src, dst, row_bytes, scratch, scratch_bytes,
-                        early, stamp, stream)) {
+                        early, early != nullptr ? map->line + kLineLate : nullptr, stamp, &published,
+                        stream)) {
             return 1;
         }
         if (capturing) return 0;
-        if (early != nullptr) {
-            // Only keys that the first pass hands to the per-key kernel can be
-            // waiting for the second region; their number arrives a quarter
-            // into the call's work.  None: the counters are fetched behind the
-            // insert without waiting for them.
-            if (wait_for_stamp(early + kLandingStamp, stamp)) return 1;
-            if (*early == 0) {
-                map->late_stamp = stamp;
-                publish_counters_kernel<<<1, 64, 0, s>>>(map->d.ctr, map->line + kLineLate, stamp);
-                ASH_LAUNCH_CHECK();
-                map->late_in_flight = true;
-                map->late_pending = true;
-                map->unread_inserts = 0;
-                return 0;
-            }
+        if (published) {
+            map->late_stamp = stamp;
+            map->late_in_flight = true;
+            map->late_pending = true;
+            map->unread_inserts = 0;
+            return 0;
         }
     } else {
         if (ash_map_insert(map, keys, n, n_values, src, dst, row_bytes,

@@ -139,9 +139,17 @@ struct PointerGuard : DeviceGuard {
 // sel holds row numbers; true: `keys` are packed 64-bit codes.  The value rows
 // of va.src are addressed by the same selected row number.  Defined in
 // ash_map.hip.
+// `publish`: what the last launch of a call leaves for the host, see
+// publish_counters_kernel; `ticket` (zero) counts its workgroups.
+struct Publish {
+    int32_t* landing;   // null: nothing
+    int32_t stamp;
+    int32_t* ticket;
+};
 int insert_selected(ash_map* map, bool codes, const void* keys,
                     const int32_t* sel, const int32_t* nsel,
-                    const ValueArgs& va, hipStream_t s);
+                    const ValueArgs& va, hipStream_t s,
+                    const Publish& publish = {});
 
 // Erases the selected keys with the per-key kernel; arguments as for
 // insert_selected.
@@ -171,11 +179,13 @@ int settle_landing_place(ash_map* map);
 int queue_touched_count(ash_map* map, const int32_t* counts, int n, hipStream_t s);
 // The streaming insert (ash_bulk.hip); `early`: page-locked words (or null) where
 // its first pass leaves the number of keys that it hands to the per-key kernel,
-// and behind it, at kLandingStamp, `stamp`.
+// and behind it, at kLandingStamp, `stamp`.  With `early` the call waits for that
+// number; is it zero, the last launch leaves the counters at `late` (with `stamp`)
+// and *published is set.
 int insert_bulk(ash_map* map, const int32_t* keys, int64_t n, int n_values,
                 const void* const* src, void* const* dst, const int64_t* row_bytes,
-                void* workspace, int64_t workspace_bytes, int32_t* early,
-                int32_t stamp, void* stream);
+                void* workspace, int64_t workspace_bytes, int32_t* early, int32_t* late,
+                int32_t stamp, bool* published, void* stream);
 // Fills the bucket array if a clear() left that to the next user of the table.
 int settle_table(ash_map* map, hipStream_t s);
 // Before the first call that writes to the heap (an erase; a load brings a

@@ -83,3 +83,22 @@ def test_second_order_gradient_is_carried_through_the_forward_node(gpu_ash, embe
     (value + eikonal + 0.5 * (grid.embeddings**2).sum()).backward()
     want = want + grid.embeddings.detach()
     check("decay")
+
+
+def test_zero_offset_gradients_are_the_callers_own(gpu_ash):
+    """The second-order offset gradient is zeros that a caller may write to:
+    a tensor per call, no element of which another call sees."""
+    backend = gpu_ash.grid_query.backend
+    emb = torch.randn(1, 8, 2, device="cuda")
+    n = 5
+    ops = [emb, torch.rand(n, 3, device="cuda"), torch.zeros(n, dtype=torch.int64, device="cuda"),
+           torch.zeros(n, dtype=torch.int64, device="cuda"), torch.ones(n, dtype=torch.bool, device="cuda"),
+           torch.zeros(1, 8, dtype=torch.int64, device="cuda"),
+           torch.zeros(8, 8, dtype=torch.int64, device="cuda"),
+           torch.zeros(8, 8, dtype=torch.int64, device="cuda")]
+    u, z = torch.randn(n, 3, device="cuda"), torch.randn(n, 2, device="cuda")
+    first = backend.query_backward_backward(None, u, z, *ops, 2, "linear")[2]
+    first[0, 0] = 7.0
+    first += 1.0
+    second = backend.query_backward_backward(None, u, z, *ops, 2, "linear")[2]
+    assert second.shape == (n, 3) and not second.any()

@@ -950,7 +950,8 @@ class _Backend:
         need_z: bool = True,
         need_embeddings: bool = True,
         accumulate_into: Optional[torch.Tensor] = None,
-    ) -> Tuple[Optional[torch.Tensor], Optional[torch.Tensor], torch.Tensor]:
+        need_offsets: bool = True,
+    ) -> Tuple[Optional[torch.Tensor], Optional[torch.Tensor], Optional[torch.Tensor]]:
         """(grad_z, grad_embeddings, zero grad_offsets); outputs that are not
         needed are None and their work is skipped.  `accumulate_into` as for
         query_backward_forward."""
@@ -959,15 +960,13 @@ class _Backend:
             [embeddings, offsets, grid_indices, cell_indices, masks, lut_grid_nb2grid_idx,
              lut_cell_nb2cell_idx, lut_cell_nb2grid_nb], interpolation, need_z, need_embeddings,
             accumulate_into)
-        # the offsets second-order term is not produced (ash/src/grid.cu:417-418):
-        # zeros, all of them one element
-        zero = _ZEROS.get((embeddings.device, embeddings.dtype))
-        if zero is None:
-            zero = _ZEROS[embeddings.device, embeddings.dtype] = embeddings.new_zeros(())
-        return grad_z, grad_embeddings, zero.expand(grid_indices.shape[0], 3)
+        # the offsets second-order term is not produced (ash/src/grid.cu:417-418)
+        zeros = embeddings.new_zeros(grid_indices.shape[0], 3) if need_offsets else None
+        return grad_z, grad_embeddings, zeros
 
+    # for callers that drop the zero grad_offsets above
+    WITHOUT_OFFSETS = {"need_offsets": False}
 
-_ZEROS: Dict[Tuple[torch.device, torch.dtype], torch.Tensor] = {}
 
 class _HashMap:
     """Same surface as the pybind class `HashMap` (ash/src/pybind.cpp:9-23).

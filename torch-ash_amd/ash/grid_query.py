@@ -372,6 +372,7 @@ class SparseDenseGridQueryBackward(torch.autograd.Function):
             return (None, None) + (None,) * n_rest
         embeddings = ctx.owner() if owned else ctx.saved_tensors[1]
         target = _dense_target(embeddings) if need_embeddings and embeddings is not None else None
+        unused = getattr(backend, "WITHOUT_OFFSETS", {})
         _record_path("contract" if target is not None else "own" if need_embeddings else "skipped")
         if target is not None:
             grad_z, _, _ = backend.query_backward_backward(
@@ -383,6 +384,7 @@ class SparseDenseGridQueryBackward(torch.autograd.Function):
                 need_z=need_z,
                 need_embeddings=True,
                 accumulate_into=target,
+                **unused,
             )
             return (grad_z, None) + (None,) * n_rest
         if need_z and need_embeddings:
@@ -392,6 +394,7 @@ class SparseDenseGridQueryBackward(torch.autograd.Function):
                 *ctx.saved_tensors,
                 ctx.grid_dim,
                 ctx.interpolation,
+                **unused,
             )
         else:
             grad_z, grad_embeddings, _ = backend.query_backward_backward(
@@ -402,5 +405,6 @@ class SparseDenseGridQueryBackward(torch.autograd.Function):
                 ctx.interpolation,
                 need_z=need_z,
                 need_embeddings=need_embeddings,
+                **unused,
             )
         return (grad_z, grad_embeddings) + (None,) * n_rest

@@ -72,3 +72,25 @@ def test_gradient_of_embedding_rows(gpu_ash, dtype, width, n):
     u = torch.randn(701, width, device=DEV, dtype=dtype)
     (back,) = torch.autograd.grad(got, z, u)
     assert torch.equal(back, u[indices] * masks.unsqueeze(1))
+
+
+def test_embedding_under_transforms_and_forward_mode(gpu_ash):
+    """A batch of parameters (vmap) and a forward-mode tangent go through
+    torch's own operations, as they always did."""
+    emb = gpu_ash.HashEmbedding(3, 200, 4, DEV)
+    g = torch.Generator().manual_seed(3)
+    keys = torch.unique(torch.randint(-30, 30, (150, 3), generator=g, dtype=torch.int32), dim=0)
+    emb.spatial_init_(keys.to(DEV))
+    q = _queries(keys, 333, seed=4)
+    indices, masks = emb.engine.find(q)
+
+    def rows(table):
+        return torch.func.functional_call(emb, {"embedding": table}, (q,))
+
+    stack = torch.randn(3, 200, 4, device=DEV)
+    want = stack[:, indices] * masks.view(1, -1, 1)
+    assert torch.equal(torch.func.vmap(rows)(stack), want)
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(stack[0], stack[1])
+        value, tangent = torch.autograd.forward_ad.unpack_dual(rows(dual))
+    assert torch.equal(value, want[0]) and torch.equal(tangent, want[1])

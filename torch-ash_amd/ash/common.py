@@ -19,6 +19,7 @@ import warnings
 from typing import Dict, Optional, Tuple
 
 import torch
+from torch.autograd import forward_ad
 
 _LIB_NAME = "libash_hip.so"
 _HOST_NAME = "_ash_host.so"
@@ -371,6 +372,19 @@ def _stream_of(device: torch.device) -> int:
 def _require_hip(t: torch.Tensor, what: str) -> None:
     if not t.is_cuda:
         raise RuntimeError(f"{what} must live on a HIP device, got {t.device}")
+
+
+def stands_alone(t: torch.Tensor) -> bool:
+    """Whether a kernel may take `t` by its address and a graph node of the
+    package's own may stand for torch's operations on it.  Not for a subclass,
+    inside a function transform (vmap and the like), with a forward-mode tangent
+    or while a trace is recorded: there torch's operations have to be seen."""
+    return (
+        type(t) in (torch.Tensor, torch.nn.Parameter)
+        and torch._C._functorch.peek_interpreter_stack() is None
+        and not torch._C._is_tracing()
+        and (forward_ad._current_level < 0 or forward_ad.unpack_dual(t).tangent is None)
+    )
 
 
 class _Backend:

@@ -1752,8 +1752,8 @@ std::vector<int32_t*>& free_lines() {
 }  // namespace
 
 int take_line(ash_map* map) {
-    if (map->line != nullptr) return 0;
     std::lock_guard<std::mutex> lock(g_lines_mutex);
+    if (map->line != nullptr) return 0;   // (read under the lock: two threads may ask first)
     std::vector<int32_t*>& lines = free_lines();
     if (lines.empty()) {
         void* slab = nullptr;

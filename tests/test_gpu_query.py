@@ -871,3 +871,40 @@ def test_module_forward_replays_in_a_hip_graph(gpu_ash):
             torch.cuda.synchronize()
             assert torch.equal(captured[0], features) and torch.equal(captured[1], masks)
             assert 1000 < int(masks.sum()) < x.shape[0] and float(features.abs().sum()) > 100.0
+
+
+@pytest.mark.parametrize("cells", [1, 27, 2047, 2048, 2049])
+@pytest.mark.parametrize("embedding_dim", [1, 4, 16])
+def test_any_tables_at_the_edge_of_the_cell_codes(gpu_ash, oracle, cells, embedding_dim):
+    """Up to 2048 cells per block a corner is a 16-bit code in LDS (11 bits of
+    cell, 3 of neighbour block), above that it is read from the tables; here with
+    tables that no grid would make: any corner in any block, missing ones among
+    them."""
+    g = torch.Generator().manual_seed(cells)
+    blocks, n = 6, 3001
+
+    def ints(hi, *shape):
+        return torch.randint(0, hi, shape, generator=g)
+
+    lut_g = ints(blocks, blocks, 8)
+    lut_g[1, 5] = lut_g[4, 0] = -1
+    c2c, c2g = ints(cells, cells, 8), ints(8, cells, 8)
+    c2c[-1, :2] = cells - 1
+    masks = torch.rand(n, generator=g) < 0.9
+    emb = torch.rand(blocks, cells, embedding_dim, generator=g) * 2 - 1
+    ops = (emb, torch.rand(n, 3, generator=g), ints(blocks, n), ints(cells, n), masks, lut_g, c2c, c2g)
+    dev = tuple(t.to(DEV) for t in ops)
+    backend = gpu_ash.grid_query.backend
+    z, u = torch.rand(n, embedding_dim, generator=g) - 0.5, torch.rand(n, 3, generator=g) - 0.5
+    sums = oracle.query_term_sums(u, z, *ops, 2, "smooth_step")
+    y, y_ref = backend.query_forward(*dev, 2, "smooth_step"), oracle.query_forward(*ops, 2, "smooth_step")
+    assert torch.allclose(y.cpu(), y_ref, rtol=RTOL32, atol=ATOL32)
+    got = backend.query_backward_forward(z.to(DEV), *dev, 2, "smooth_step")
+    ref = oracle.query_backward_forward(z, *ops, 2, "smooth_step")
+    dense = dict(eps=_eps(torch.float32), rtol=RTOL32, atol=ATOL32)
+    assert torch.allclose(got[1].cpu(), ref[1], rtol=RTOL32, atol=ATOL32)
+    assert_close_sums(got[0], ref[0], sums["bf_embeddings"], what="grad_embeddings", **dense)
+    got = backend.query_backward_backward(None, u.to(DEV), z.to(DEV), *dev, 2, "smooth_step")
+    ref = oracle.query_backward_backward(None, u, z, *ops, 2, "smooth_step")
+    assert torch.allclose(got[0].cpu(), ref[0], rtol=RTOL32, atol=ATOL32)
+    assert_close_sums(got[1], ref[1], sums["bb_embeddings"], what="grad_embeddings (2nd order)", **dense)

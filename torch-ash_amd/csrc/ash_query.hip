@@ -40,7 +40,7 @@ namespace ash {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int64_t kMaxLdsCells = 2048;  // 2048 * 8 * 3 B = 48 KiB
+constexpr int64_t kMaxLdsCells = 2048;  // 2048 * 8 * 2 B = 32 KiB
 constexpr uint32_t kNoRow = 0xFFFFFFFFu;
 constexpr int kLdsPerCu = 160 * 1024;
 // Wavefronts per SIMD the kernels are compiled for: the highest occupancy that
@@ -122,52 +122,60 @@ __device__ __forceinline__ void corner_weight_grad(const AxisTerms<T>& t, int c,
 
 // ------------------------------------------------------------ LDS layout
 // [ tile: row[8][256] uint32, off[3][256] float ]  (only when LPQ > 1)
-// [ per-cell tables: c2c[M*8] uint16, c2g[M*8] uint8 ]  (only when lds_lut)
+// [ per-cell table: uint16[M][8] ]  (only when lds_lut)
 // [ one LineTable per wavefront ]  (E = 4 backward kernels that produce grad_embeddings)
 struct Tile {
     uint32_t row[8][kBlock];
     float off[3][kBlock];
 };
 
+// A cell's eight corners, one 16-bit code each (cell of the corner, below
+// kMaxLdsCells, and number of its neighbour block above it): one 16-byte read
+// per query.
 struct CellLut {
-    const uint16_t* c2c;
-    const uint8_t* c2g;
+    const uint4* codes;
 };
 
+constexpr int kCodeCellBits = 11;
+static_assert(kMaxLdsCells == int64_t{1} << kCodeCellBits, "cells of a code");
+
 template <bool LDS>
-__device__ __forceinline__ void cell_neighbor(const QDev& a, const CellLut& lut,
-                                              int64_t cell, int c, int& nb_cell,
-                                              int& nb_grid) {
+__device__ __forceinline__ void cell_neighbors(const QDev& a, const CellLut& lut, int64_t cell,
+                                               uint32_t (&nb_cell)[8], uint32_t (&nb_grid)[8]) {
     if constexpr (LDS) {
-        nb_cell = lut.c2c[cell * 8 + c];
-        nb_grid = lut.c2g[cell * 8 + c];
+        const uint4 v = lut.codes[cell];
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const uint32_t code = (w[c >> 1] >> (16 * (c & 1))) & 0xFFFFu;
+            nb_cell[c] = code & (kMaxLdsCells - 1);
+            nb_grid[c] = code >> kCodeCellBits;
+        }
     } else {
-        int64_t v = a.lut_c2c[cell * 8 + c];
-        v = v < 0 ? 0 : (v >= a.M ? a.M - 1 : v);
-        nb_cell = static_cast<int>(v);
-        nb_grid = static_cast<int>(a.lut_c2g[cell * 8 + c]) & 7;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            int64_t v = a.lut_c2c[cell * 8 + c];
+            v = v < 0 ? 0 : (v >= a.M ? a.M - 1 : v);
+            nb_cell[c] = static_cast<uint32_t>(v);
+            nb_grid[c] = static_cast<uint32_t>(a.lut_c2g[cell * 8 + c]) & 7u;
+        }
     }
 }
 
 template <bool LDS>
 __device__ __forceinline__ CellLut stage_cell_lut(const QDev& a,
                                                   unsigned char* smem) {
-    CellLut lut;
-    lut.c2c = nullptr;
-    lut.c2g = nullptr;
+    CellLut lut = {nullptr};
     if constexpr (LDS) {
-        uint16_t* s_c2c = reinterpret_cast<uint16_t*>(smem);
-        uint8_t* s_c2g = smem + a.M * 8 * 2;
+        uint16_t* codes = reinterpret_cast<uint16_t*>(smem);
         const int64_t n = a.M * 8;
         for (int64_t t = threadIdx.x; t < n; t += kBlock) {
             int64_t v = a.lut_c2c[t];
             v = v < 0 ? 0 : (v >= a.M ? a.M - 1 : v);
-            s_c2c[t] = static_cast<uint16_t>(v);
-            s_c2g[t] = static_cast<uint8_t>(a.lut_c2g[t] & 7);
+            codes[t] = static_cast<uint16_t>(v | ((a.lut_c2g[t] & 7) << kCodeCellBits));
         }
         __syncthreads();
-        lut.c2c = s_c2c;
-        lut.c2g = s_c2g;
+        lut.codes = reinterpret_cast<const uint4*>(smem);
     }
     return lut;
 }
@@ -175,7 +183,7 @@ __device__ __forceinline__ CellLut stage_cell_lut(const QDev& a,
 // Where the line tables of the float4 backward kernels start in dynamic LDS.
 __host__ __device__ inline size_t table_offset(const QDev& a, int lpq, bool lds_lut) {
     size_t bytes = lpq > 1 ? sizeof(Tile) : 0;
-    if (lds_lut) bytes += static_cast<size_t>(a.M) * 8 * 3;
+    if (lds_lut) bytes += static_cast<size_t>(a.M) * 8 * 2;
     return (bytes + 15) & ~static_cast<size_t>(15);
 }
 
@@ -222,26 +230,24 @@ __device__ __forceinline__ void resolve_rows(const QDev& a, const CellLut& lut,
     // Block indices are below 2^31 and a missing block is -1, so the low
     // dword of each int64 table entry carries everything.
     const int32_t* lut_g32 = reinterpret_cast<const int32_t*>(a.lut_g) + gi * 16;
-    int32_t g0 = -1;
-    if (valid) g0 = lut_g32[0];
-    const uint32_t nblocks = static_cast<uint32_t>(a.B);
-    const uint32_t cells = static_cast<uint32_t>(a.M);
+    uint32_t nb_cell[8], nb_grid[8];
+    int32_t own = -1, other[8];
+    if (valid) own = lut_g32[0];
+    cell_neighbors<LDS>(a, lut, ci, nb_cell, nb_grid);
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-        row[c] = 0;
-        if (valid) {
-            int nb_cell, nb_grid;
-            cell_neighbor<LDS>(a, lut, ci, c, nb_cell, nb_grid);
-            int32_t g = g0;
-            if (nb_grid != 0) g = lut_g32[nb_grid * 2];
-            if (static_cast<uint32_t>(g) >= nblocks) {
-                valid = false;
-            } else {
-                row[c] = static_cast<uint32_t>(g) * cells +
-                         static_cast<uint32_t>(nb_cell);
-            }
-        }
+        other[c] = -1;
+        if (valid && nb_grid[c] != 0) other[c] = lut_g32[nb_grid[c] * 2];
     }
+    const uint32_t cells = static_cast<uint32_t>(a.M);
+    uint32_t most = 0;   // a missing block is the largest number
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        const uint32_t g = static_cast<uint32_t>(nb_grid[c] != 0 ? other[c] : own);
+        most = g > most ? g : most;
+        row[c] = g * cells + nb_cell[c];
+    }
+    valid = valid && most < static_cast<uint32_t>(a.B);
     if (!valid) row[0] = kNoRow;
 }
 

@@ -878,8 +878,9 @@ def test_module_forward_replays_in_a_hip_graph(gpu_ash):
 def test_any_tables_at_the_edge_of_the_cell_codes(gpu_ash, oracle, cells, embedding_dim):
     """Up to 2048 cells per block a corner is a 16-bit code in LDS (11 bits of
     cell, 3 of neighbour block), above that it is read from the tables; here with
-    tables that no grid would make: any corner in any block, missing ones among
-    them."""
+    tables that no grid would make: the first corner is the cell itself, as
+    everywhere (queries of one cell are told by it), the others lie in any block,
+    missing ones among them."""
     g = torch.Generator().manual_seed(cells)
     blocks, n = 6, 3001
 
@@ -887,9 +888,11 @@ def test_any_tables_at_the_edge_of_the_cell_codes(gpu_ash, oracle, cells, embedd
         return torch.randint(0, hi, shape, generator=g)
 
     lut_g = ints(blocks, blocks, 8)
+    lut_g[:, 0] = torch.arange(blocks)
     lut_g[1, 5] = lut_g[4, 0] = -1
     c2c, c2g = ints(cells, cells, 8), ints(8, cells, 8)
-    c2c[-1, :2] = cells - 1
+    c2c[:, 0], c2g[:, 0] = torch.arange(cells), 0
+    c2c[-1, 1:3] = cells - 1
     masks = torch.rand(n, generator=g) < 0.9
     emb = torch.rand(blocks, cells, embedding_dim, generator=g) * 2 - 1
     ops = (emb, torch.rand(n, 3, generator=g), ints(blocks, n), ints(cells, n), masks, lut_g, c2c, c2g)

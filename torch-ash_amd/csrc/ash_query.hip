@@ -43,11 +43,9 @@ constexpr int kBlock = 256;
 constexpr int64_t kMaxLdsCells = 2048;  // 2048 * 8 * 2 B = 32 KiB
 constexpr uint32_t kNoRow = 0xFFFFFFFFu;
 constexpr int kLdsPerCu = 160 * 1024;
-// Wavefronts per SIMD the kernels are compiled for: the highest occupancy that
-// needs no register spills (measured: spilling costs more than the extra
-// wavefronts bring).  The one-lane-per-query gather fits 4, the
-// channel-parallel kernels, which hold 8 rows plus the run-merge state per
-// lane, fit 3.
+// Wavefronts per SIMD the kernels must leave room for.  Most take 50 - 95
+// registers and run at five to eight; the bounds only keep the widest instances
+// from spilling.
 constexpr int kWavesGather = 4;
 constexpr int kWavesWide = 3;
 
@@ -218,6 +216,15 @@ __device__ __forceinline__ QueryInputs load_inputs(const QDev& a, int64_t q) {
 
 // Phase 1 for one query: the 8 corner rows (kNoRow in row[0] when the query is
 // masked out, out of range, or misses a neighbour block) and the offsets.
+// Latency bounds it, so the eight table entries are asked for together and
+// checked afterwards.  Leaving at the first missing corner made every entry wait
+// for the one before it, up to eight trips to the L2 in nearly every wavefront
+// (one of its lanes stands at a block's edge), and the branches kept 126 - 168
+// registers alive instead of 53 - 94, three or four wavefronts per SIMD instead
+// of five to eight.  2^22 ray samples, rows of four, 200 k blocks: forward with
+// its operands 166 -> 131 us, gradient of the positions 158 -> 87, backward 296
+// -> 219, second order 262 -> 212; 10^6 samples, rows of sixteen: 75 -> 56, 140
+// -> 121, 293 -> 220, 200 -> 167.
 template <bool LDS>
 __device__ __forceinline__ void resolve_rows(const QDev& a, const CellLut& lut,
                                              const QueryInputs& in, uint32_t (&row)[8],

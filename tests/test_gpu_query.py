@@ -911,3 +911,33 @@ def test_any_tables_at_the_edge_of_the_cell_codes(gpu_ash, oracle, cells, embedd
     ref = oracle.query_backward_backward(None, u, z, *ops, 2, "smooth_step")
     assert torch.allclose(got[0].cpu(), ref[0], rtol=RTOL32, atol=ATOL32)
     assert_close_sums(got[1], ref[1], sums["bb_embeddings"], what="grad_embeddings (2nd order)", **dense)
+
+
+@pytest.mark.parametrize("cells", [512, 576, 577])
+@pytest.mark.parametrize("n", [1, 63, 511, 513, 40_001])
+def test_gradient_rows_by_workgroups_of_either_width(gpu_ash, oracle, cells, n):
+    """Rows of four channels: eight wavefronts share the cells' codes up to 576
+    cells per block, four above; unordered queries, whose rows leave past the line
+    tables sixteen at a time, and ordered ones."""
+    g = torch.Generator().manual_seed(n)
+    blocks = 40
+    lut_g = torch.randint(0, blocks, (blocks, 8), generator=g)
+    lut_g[:, 0] = torch.arange(blocks)
+    c2c, c2g = torch.randint(0, cells, (cells, 8), generator=g), torch.randint(0, 8, (cells, 8), generator=g)
+    c2c[:, 0], c2g[:, 0] = torch.arange(cells), 0
+    gi, ci = torch.randint(0, blocks, (n,), generator=g), torch.randint(0, cells, (n,), generator=g)
+    if n > 1:   # the second half in order
+        gi[n // 2:], ci[n // 2:] = 3, torch.sort(ci[n // 2:])[0]
+    ops = (torch.rand(blocks, cells, 4, generator=g) - 0.5, torch.rand(n, 3, generator=g), gi, ci,
+           torch.rand(n, generator=g) < 0.95, lut_g, c2c, c2g)
+    dev = tuple(t.to(DEV) for t in ops)
+    backend = gpu_ash.grid_query.backend
+    z, u = torch.rand(n, 4, generator=g) - 0.5, torch.rand(n, 3, generator=g) - 0.5
+    sums = oracle.query_term_sums(u, z, *ops, 2, "linear")
+    dense = dict(eps=_eps(torch.float32), rtol=RTOL32, atol=ATOL32)
+    got, _ = backend.query_backward_forward(z.to(DEV), *dev, 2, "linear")
+    ref, _ = oracle.query_backward_forward(z, *ops, 2, "linear")
+    assert_close_sums(got, ref, sums["bf_embeddings"], what="grad_embeddings", **dense)
+    got = backend.query_backward_backward(None, u.to(DEV), z.to(DEV), *dev, 2, "linear")[1]
+    ref = oracle.query_backward_backward(None, u, z, *ops, 2, "linear")[1]
+    assert_close_sums(got, ref, sums["bb_embeddings"], what="grad_embeddings (2nd order)", **dense)

@@ -160,14 +160,14 @@ __device__ __forceinline__ void cell_neighbors(const QDev& a, const CellLut& lut
     }
 }
 
-template <bool LDS>
+template <bool LDS, int THREADS = kBlock>
 __device__ __forceinline__ CellLut stage_cell_lut(const QDev& a,
                                                   unsigned char* smem) {
     CellLut lut = {nullptr};
     if constexpr (LDS) {
         uint16_t* codes = reinterpret_cast<uint16_t*>(smem);
         const int64_t n = a.M * 8;
-        for (int64_t t = threadIdx.x; t < n; t += kBlock) {
+        for (int64_t t = threadIdx.x; t < n; t += THREADS) {
             int64_t v = a.lut_c2c[t];
             v = v < 0 ? 0 : (v >= a.M ? a.M - 1 : v);
             codes[t] = static_cast<uint16_t>(v | ((a.lut_c2g[t] & 7) << kCodeCellBits));
@@ -852,6 +852,7 @@ __device__ __forceinline__ void sum_runs(const Runs& r, float (&v)[4]) {
 constexpr int kLineSlots = 128;   // lines per wavefront's table
 constexpr int kLineProbes = 4;
 constexpr int kLineRest = 7;
+constexpr int kLineOut = 16;      // rows that leave past the table by one instruction
 constexpr uint32_t kLineFree = 0xFFFFFFFFu;
 // float k of slot h sits at k * kLinePitch + h: the sixteen floats of a line
 // and the same float of neighbouring slots fall into different banks
@@ -864,10 +865,10 @@ struct LineTable {
     // of used slots in the same place
     union {
         struct {
-            uint32_t row[64];
-            float v[64 * 4];
+            uint32_t row[kLineOut];
+            float v[kLineOut * 4];
         } out;
-        uint32_t used[kLineSlots];
+        uint8_t used[kLineSlots];
     };
 };
 
@@ -952,16 +953,17 @@ struct LineAcc {
         if (out == 0) return;
         const int n = __popcll(out);
         spilled += n;
-        wave_lds_fence();
-        if (want && !placed) {
-            const int at = __popcll(out & ((1ull << lane) - 1ull));
-            tab->out.row[at] = row;
-            *reinterpret_cast<float4*>(tab->out.v + at * 4) = make_float4(v[0], v[1], v[2], v[3]);
-        }
-        wave_lds_fence();
-        for (int i = 0; i < n; i += 16) {
-            const int e = i + (lane >> 2);
-            if (e < n) {
+        const int mine = __popcll(out & ((1ull << lane) - 1ull));
+        for (int i = 0; i < n; i += kLineOut) {
+            const int at = mine - i;
+            wave_lds_fence();
+            if (want && !placed && at >= 0 && at < kLineOut) {
+                tab->out.row[at] = row;
+                *reinterpret_cast<float4*>(tab->out.v + at * 4) = make_float4(v[0], v[1], v[2], v[3]);
+            }
+            wave_lds_fence();
+            const int e = lane >> 2;
+            if (i + e < n) {
                 unsafeAtomicAdd(grad + static_cast<uint64_t>(tab->out.row[e]) * 4 + (lane & 3),
                                 tab->out.v[e * 4 + (lane & 3)]);
             }
@@ -981,8 +983,8 @@ struct LineAcc {
             const uint64_t below = (1ull << lane) - 1ull;
             const int nlo = __popcll(mlo);
             const int n = nlo + __popcll(mhi);
-            if (lo) tab->used[__popcll(mlo & below)] = lane;
-            if (hi) tab->used[nlo + __popcll(mhi & below)] = lane + 64;
+            if (lo) tab->used[__popcll(mlo & below)] = static_cast<uint8_t>(lane);
+            if (hi) tab->used[nlo + __popcll(mhi & below)] = static_cast<uint8_t>(lane + 64);
             wave_lds_fence();
             // four lines per instruction, sixteen lines per turn: the reads of
             // a turn are issued together
@@ -1049,25 +1051,25 @@ __device__ __forceinline__ LineTable* line_table(unsigned char* smem, const QDev
 }
 
 // First-order backward, E = 4 (formulas as in query_backward_forward_kernel).
-template <bool LDS, int OUT>
-__global__ __launch_bounds__(kBlock, kWavesWide) void
+template <bool LDS, int OUT, int THREADS>
+__global__ __launch_bounds__(THREADS, kWavesWide) void
 query_backward_forward_vec_kernel(
         QDev a, const float* __restrict__ z, float* __restrict__ grad_emb,
         float* __restrict__ grad_off) {
     extern __shared__ __align__(16) unsigned char smem[];
-    const CellLut lut = stage_cell_lut<LDS>(a, smem);
+    const CellLut lut = stage_cell_lut<LDS, THREADS>(a, smem);
     const int lane = threadIdx.x & 63;
     const float* __restrict__ emb = static_cast<const float*>(a.emb);
     constexpr bool want_emb = (OUT & 1) != 0;
     constexpr bool want_off = (OUT & 2) != 0;
     LineAcc acc;
     acc.start(line_table(smem, a, LDS, want_emb), lane);
-    const int64_t ntiles = (a.N + kBlock - 1) / kBlock;
+    const int64_t ntiles = (a.N + THREADS - 1) / THREADS;
     TileWalk walk(ntiles);
     for (int64_t tile = walk.next; tile < walk.end; tile += walk.step) {
         uint32_t row[8];
         float o[3];
-        const int64_t q = tile * kBlock + threadIdx.x;
+        const int64_t q = tile * THREADS + threadIdx.x;
         const QueryInputs in = load_inputs(a, q);
         resolve_rows<LDS>(a, lut, in, row, o);
         const bool on = row[0] != kNoRow;
@@ -1125,25 +1127,25 @@ query_backward_forward_vec_kernel(
 
 // Backward of the backward, E = 4 (formulas as in
 // query_backward_backward_kernel).
-template <bool LDS, int OUT>
-__global__ __launch_bounds__(kBlock, kWavesWide) void
+template <bool LDS, int OUT, int THREADS>
+__global__ __launch_bounds__(THREADS, kWavesWide) void
 query_backward_backward_vec_kernel(
         QDev a, const float* __restrict__ gg_off, const float* __restrict__ z,
         float* __restrict__ grad_z, float* __restrict__ grad_emb) {
     extern __shared__ __align__(16) unsigned char smem[];
-    const CellLut lut = stage_cell_lut<LDS>(a, smem);
+    const CellLut lut = stage_cell_lut<LDS, THREADS>(a, smem);
     const int lane = threadIdx.x & 63;
     const float* __restrict__ emb = static_cast<const float*>(a.emb);
     constexpr bool want_emb = (OUT & 1) != 0;
     constexpr bool want_z = (OUT & 2) != 0;
     LineAcc acc;
     acc.start(line_table(smem, a, LDS, want_emb), lane);
-    const int64_t ntiles = (a.N + kBlock - 1) / kBlock;
+    const int64_t ntiles = (a.N + THREADS - 1) / THREADS;
     TileWalk walk(ntiles);
     for (int64_t tile = walk.next; tile < walk.end; tile += walk.step) {
         uint32_t row[8];
         float o[3];
-        const int64_t q = tile * kBlock + threadIdx.x;
+        const int64_t q = tile * THREADS + threadIdx.x;
         const QueryInputs in = load_inputs(a, q);
         resolve_rows<LDS>(a, lut, in, row, o);
         const bool on = row[0] != kNoRow;
@@ -2158,10 +2160,8 @@ int pow2_ceil(int v) {
 
 bool lut_in_lds(const QDev& d) { return d.M <= kMaxLdsCells; }
 
-size_t smem_bytes(const QDev& d, int lpq, bool line_tables = false) {
-    size_t bytes = table_offset(d, lpq, lut_in_lds(d));
-    if (line_tables) bytes += (kBlock / 64) * sizeof(LineTable);
-    return bytes;
+size_t smem_bytes(const QDev& d, int lpq, int line_tables = 0) {
+    return table_offset(d, lpq, lut_in_lds(d)) + line_tables * sizeof(LineTable);
 }
 
 // Enough persistent workgroups to fill every CU as far as LDS allows.
@@ -2276,23 +2276,38 @@ bool aligned16(const void* p) {
     return reinterpret_cast<uintptr_t>(p) % 16 == 0;
 }
 
+// Workgroups of the kernels with line tables (OUT bit 0) share one table of
+// cells between eight wavefronts where two of them fit a CU (blocks of up to 576
+// cells): 80 KB each and sixteen wavefronts on a CU, where three of 44 KB with
+// four are twelve.  2^22 ray samples on 200 k blocks of 8^3: backward 221 -> 190
+// us, second order 214 -> 187; 1.5 x 10^6 unordered queries 541 and 542 us as
+// before (their rows leave past the tables, bound by requests).
+int vec_threads(const QDev& d, int out) {
+    const bool wide = lut_in_lds(d) && (out & 1) != 0 && 2 * smem_bytes(d, 1, 2 * kBlock / 64) <= kLdsPerCu;
+    return wide ? 2 * kBlock : kBlock;
+}
+
 int launch_bwd_fwd_vec(const QDev& d, const void* z, void* ge, void* go,
                        hipStream_t s) {
-    const size_t smem = smem_bytes(d, 1, ge != nullptr);
-    const unsigned g = persistent_grid((d.N + kBlock - 1) / kBlock, smem);
     const int out = (ge != nullptr ? 1 : 0) | (go != nullptr ? 2 : 0);
-#define ASH_BF(L, O)                                                          \
-    query_backward_forward_vec_kernel<L, O><<<g, kBlock, smem, s>>>(     \
+    const int threads = vec_threads(d, out);
+    const size_t smem = smem_bytes(d, 1, ge != nullptr ? threads / 64 : 0);
+    const unsigned g = persistent_grid((d.N + threads - 1) / threads, smem);
+#define ASH_BF(L, O, T)                                                       \
+    query_backward_forward_vec_kernel<L, O, T><<<g, T, smem, s>>>(    \
             d, static_cast<const float*>(z), static_cast<float*>(ge),         \
             static_cast<float*>(go))
-    if (lut_in_lds(d)) {
-        if (out == 3) ASH_BF(true, 3);
-        else if (out == 1) ASH_BF(true, 1);
-        else ASH_BF(true, 2);
+    if (threads > kBlock) {
+        if (out == 3) ASH_BF(true, 3, 2 * kBlock);
+        else ASH_BF(true, 1, 2 * kBlock);
+    } else if (lut_in_lds(d)) {
+        if (out == 3) ASH_BF(true, 3, kBlock);
+        else if (out == 1) ASH_BF(true, 1, kBlock);
+        else ASH_BF(true, 2, kBlock);
     } else {
-        if (out == 3) ASH_BF(false, 3);
-        else if (out == 1) ASH_BF(false, 1);
-        else ASH_BF(false, 2);
+        if (out == 3) ASH_BF(false, 3, kBlock);
+        else if (out == 1) ASH_BF(false, 1, kBlock);
+        else ASH_BF(false, 2, kBlock);
     }
 #undef ASH_BF
     ASH_LAUNCH_CHECK();
@@ -2301,21 +2316,25 @@ int launch_bwd_fwd_vec(const QDev& d, const void* z, void* ge, void* go,
 
 int launch_bwd_bwd_vec(const QDev& d, const void* gg, const void* z, void* gz,
                        void* ge, hipStream_t s) {
-    const size_t smem = smem_bytes(d, 1, ge != nullptr);
-    const unsigned g = persistent_grid((d.N + kBlock - 1) / kBlock, smem);
     const int out = (ge != nullptr ? 1 : 0) | (gz != nullptr ? 2 : 0);
-#define ASH_BB(L, O)                                                          \
-    query_backward_backward_vec_kernel<L, O><<<g, kBlock, smem, s>>>(    \
+    const int threads = vec_threads(d, out);
+    const size_t smem = smem_bytes(d, 1, ge != nullptr ? threads / 64 : 0);
+    const unsigned g = persistent_grid((d.N + threads - 1) / threads, smem);
+#define ASH_BB(L, O, T)                                                       \
+    query_backward_backward_vec_kernel<L, O, T><<<g, T, smem, s>>>(   \
             d, static_cast<const float*>(gg), static_cast<const float*>(z),   \
             static_cast<float*>(gz), static_cast<float*>(ge))
-    if (lut_in_lds(d)) {
-        if (out == 3) ASH_BB(true, 3);
-        else if (out == 1) ASH_BB(true, 1);
-        else ASH_BB(true, 2);
+    if (threads > kBlock) {
+        if (out == 3) ASH_BB(true, 3, 2 * kBlock);
+        else ASH_BB(true, 1, 2 * kBlock);
+    } else if (lut_in_lds(d)) {
+        if (out == 3) ASH_BB(true, 3, kBlock);
+        else if (out == 1) ASH_BB(true, 1, kBlock);
+        else ASH_BB(true, 2, kBlock);
     } else {
-        if (out == 3) ASH_BB(false, 3);
-        else if (out == 1) ASH_BB(false, 1);
-        else ASH_BB(false, 2);
+        if (out == 3) ASH_BB(false, 3, kBlock);
+        else if (out == 1) ASH_BB(false, 1, kBlock);
+        else ASH_BB(false, 2, kBlock);
     }
 #undef ASH_BB
     ASH_LAUNCH_CHECK();

@@ -873,16 +873,23 @@ def test_module_forward_replays_in_a_hip_graph(gpu_ash):
             assert 1000 < int(masks.sum()) < x.shape[0] and float(features.abs().sum()) > 100.0
 
 
-@pytest.mark.parametrize("cells", [1, 27, 2047, 2048, 2049])
-@pytest.mark.parametrize("embedding_dim", [1, 4, 16])
-def test_any_tables_at_the_edge_of_the_cell_codes(gpu_ash, oracle, cells, embedding_dim):
-    """Up to 2048 cells per block a corner is a 16-bit code in LDS (11 bits of
-    cell, 3 of neighbour block), above that it is read from the tables; here with
+_MANY = (1 << 19) + 77   # more queries than the kernels serve without tables in LDS
+
+
+@pytest.mark.parametrize("cells,n,embedding_dim",
+                         [(c, 3001, e) for c in (1, 27, 2049) for e in (1, 4, 16)]
+                         + [(c, _MANY, e) for c, e in ((1, 4), (27, 2), (2047, 6), (2048, 1), (2048, 4), (2048, 8),
+                                                       (2049, 4))]
+                         + [(512, _MANY - 77, 4)])
+def test_any_tables_at_the_edge_of_the_cell_codes(gpu_ash, oracle, cells, n, embedding_dim):
+    """For more than 2^19 queries and up to 2048 cells per block a corner is a
+    16-bit code in LDS (11 bits of cell, 3 of neighbour block), otherwise it is
+    read from the tables; here with
     tables that no grid would make: the first corner is the cell itself, as
     everywhere (queries of one cell are told by it), the others lie in any block,
     missing ones among them."""
     g = torch.Generator().manual_seed(cells)
-    blocks, n = 6, 3001
+    blocks = 600 if n > 1 << 16 else 6
 
     def ints(hi, *shape):
         return torch.randint(0, hi, shape, generator=g)
@@ -913,14 +920,14 @@ def test_any_tables_at_the_edge_of_the_cell_codes(gpu_ash, oracle, cells, embedd
     assert_close_sums(got[1], ref[1], sums["bb_embeddings"], what="grad_embeddings (2nd order)", **dense)
 
 
-@pytest.mark.parametrize("cells", [512, 576, 577])
-@pytest.mark.parametrize("n", [1, 63, 511, 513, 40_001])
+@pytest.mark.parametrize("cells,n", [(512, n) for n in (1, 63, 511, 513, 40_001)]
+                         + [(c, _MANY) for c in (8, 576, 577)])
 def test_gradient_rows_by_workgroups_of_either_width(gpu_ash, oracle, cells, n):
     """Rows of four channels: eight wavefronts share the cells' codes up to 576
     cells per block, four above; unordered queries, whose rows leave past the line
     tables sixteen at a time, and ordered ones."""
     g = torch.Generator().manual_seed(n)
-    blocks = 40
+    blocks = 40 if n < 1 << 19 else 5000
     lut_g = torch.randint(0, blocks, (blocks, 8), generator=g)
     lut_g[:, 0] = torch.arange(blocks)
     c2c, c2g = torch.randint(0, cells, (cells, 8), generator=g), torch.randint(0, 8, (cells, 8), generator=g)

@@ -165,12 +165,19 @@ __device__ __forceinline__ CellLut stage_cell_lut(const QDev& a,
                                                   unsigned char* smem) {
     CellLut lut = {nullptr};
     if constexpr (LDS) {
-        uint16_t* codes = reinterpret_cast<uint16_t*>(smem);
-        const int64_t n = a.M * 8;
-        for (int64_t t = threadIdx.x; t < n; t += THREADS) {
-            int64_t v = a.lut_c2c[t];
-            v = v < 0 ? 0 : (v >= a.M ? a.M - 1 : v);
-            codes[t] = static_cast<uint16_t>(v | ((a.lut_c2g[t] & 7) << kCodeCellBits));
+        // a cell at a time: its sixteen table entries come by eight loads in flight
+        uint4* codes = reinterpret_cast<uint4*>(smem);
+        const int cells = static_cast<int>(a.M);
+#pragma unroll 2
+        for (int cell = threadIdx.x; cell < cells; cell += THREADS) {
+            uint32_t nb_cell[8], nb_grid[8], w[4];
+            cell_neighbors<false>(a, lut, cell, nb_cell, nb_grid);
+#pragma unroll
+            for (int c = 0; c < 8; c += 2) {
+                w[c >> 1] = nb_cell[c] | (nb_grid[c] << kCodeCellBits) | (nb_cell[c + 1] << 16) |
+                            (nb_grid[c + 1] << (16 + kCodeCellBits));
+            }
+            codes[cell] = make_uint4(w[0], w[1], w[2], w[3]);
         }
         __syncthreads();
         lut.codes = reinterpret_cast<const uint4*>(smem);
@@ -2158,7 +2165,17 @@ int pow2_ceil(int v) {
     return p;
 }
 
-bool lut_in_lds(const QDev& d) { return d.M <= kMaxLdsCells; }
+// Whether the per-cell tables go to LDS.  Up to 2^19 queries a workgroup of a
+// full device meets one tile, and filling its LDS (sixteen table entries a cell,
+// a trip to the L2 and a barrier) costs more than reading the tables where they
+// are.  Blocks of 8^3, ray-ordered queries: forward of 131 k rows of four 7.5 ->
+// 6.1 us, 524 k 23.5 -> 17.2; gradient of the positions 524 k 21.3 -> 14.3; rows
+// of sixteen 131 k 9.8 -> 8.3.  Unordered ones, rows of four: 100 k 15.5 -> 14.3,
+// 500 k 56.1 and 56.0.  Above, ordered and unordered queries part (1 M: 33.9
+// against 27.1, and 109 against 117), and at 4 M LDS is ahead for both (132
+// against 139, 701 against 745 for rows of sixteen).
+constexpr int64_t kMaxDirectQueries = int64_t{1} << 19;
+bool lut_in_lds(const QDev& d) { return d.M <= kMaxLdsCells && d.N > kMaxDirectQueries; }
 
 size_t smem_bytes(const QDev& d, int lpq, int line_tables = 0) {
     return table_offset(d, lpq, lut_in_lds(d)) + line_tables * sizeof(LineTable);

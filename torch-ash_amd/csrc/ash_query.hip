@@ -43,11 +43,25 @@ constexpr int kBlock = 256;
 constexpr int64_t kMaxLdsCells = 2048;  // 2048 * 8 * 2 B = 32 KiB
 constexpr uint32_t kNoRow = 0xFFFFFFFFu;
 constexpr int kLdsPerCu = 160 * 1024;
-// Wavefronts per SIMD the kernels must leave room for.  Most take 50 - 95
-// registers and run at five to eight; the bounds only keep the widest instances
-// from spilling.
-constexpr int kWavesGather = 4;
-constexpr int kWavesWide = 3;
+// Wavefronts per SIMD, which is workgroups per CU.  Forward kernels are held to
+// the 64 registers of eight, but for the widest rows (64 - 70 registers, seven),
+// which would spill; the backward ones are bound by their registers (both
+// gradients: 67 - 71, seven; in double precision 88 - 112, four, and five for
+// one) or by LDS.  A persistent grid is as many workgroups as are resident: the
+// eighth of a CU where seven fit started when the others were done.  Backward of
+// 1 - 1.5 M ray samples, rows of sixteen 215 -> 178 us, eight 138 -> 120, five
+// 220 -> 206; forward of 2^22, rows of four, 132 -> 126.
+constexpr int kWavesFull = 8;
+constexpr int kWavesWide = 7;
+constexpr int kWavesBackward = 3;
+constexpr int forward_waves(int vec, int lpq) {
+    return vec > 4 || (vec == 4 && lpq > 2) ? kWavesWide : kWavesFull;
+}
+template <typename T>
+constexpr int backward_waves(int out) {
+    if (sizeof(T) == 8) return out == 3 ? 4 : 5;
+    return out == 3 ? kWavesWide : kWavesFull;
+}
 
 struct QDev {
     const void* emb;
@@ -168,7 +182,7 @@ __device__ __forceinline__ CellLut stage_cell_lut(const QDev& a,
         // a cell at a time: its sixteen table entries come by eight loads in flight
         uint4* codes = reinterpret_cast<uint4*>(smem);
         const int cells = static_cast<int>(a.M);
-#pragma unroll 2
+#pragma unroll 1
         for (int cell = threadIdx.x; cell < cells; cell += THREADS) {
             uint32_t nb_cell[8], nb_grid[8], w[4];
             cell_neighbors<false>(a, lut, cell, nb_cell, nb_grid);
@@ -403,7 +417,7 @@ __device__ __forceinline__ void forward_rows(const QDev& a, const T* __restrict_
 }
 
 template <typename T, int VEC, int LPQ, bool LDS>
-__global__ __launch_bounds__(kBlock, (LPQ == 1 && VEC <= 4) ? kWavesGather : kWavesWide) void
+__global__ __launch_bounds__(kBlock, forward_waves(VEC, LPQ)) void
 query_forward_kernel(
         QDev a, T* __restrict__ out) {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -493,7 +507,7 @@ __device__ __forceinline__ QueryInputs front_inputs(const QDev& a, const FrontDe
 }
 
 template <typename T, int VEC, int LPQ, bool LDS, bool AUX>
-__global__ __launch_bounds__(kBlock, (LPQ == 1 && VEC <= 4) ? kWavesGather : kWavesWide) void
+__global__ __launch_bounds__(kBlock, forward_waves(VEC, LPQ)) void
 grid_forward_kernel(QDev a, FrontDev f, T* __restrict__ out) {
     extern __shared__ __align__(16) unsigned char smem[];
     Tile* tile_s = reinterpret_cast<Tile*>(smem);
@@ -597,7 +611,7 @@ __device__ __forceinline__ void accumulate_row(T* __restrict__ grad_emb,
 // (ash/src/grid.cu:177-255).  One lane per channel.
 // OUT: bit 0 = produce grad_embeddings, bit 1 = produce grad_offsets.
 template <typename T, int LPQ, bool LDS, int OUT>
-__global__ __launch_bounds__(kBlock, kWavesWide) void
+__global__ __launch_bounds__(kBlock, kWavesBackward) void
 query_backward_forward_kernel(
         QDev a, const T* __restrict__ z, T* __restrict__ grad_emb,
         T* __restrict__ grad_off) {
@@ -668,7 +682,7 @@ query_backward_forward_kernel(
 // grad_z[i,k] = sum_c d_c * emb[row_c,k]   (ash/src/grid.cu:309-387).
 // OUT: bit 0 = produce grad_embeddings, bit 1 = produce grad_z.
 template <typename T, int LPQ, bool LDS, int OUT>
-__global__ __launch_bounds__(kBlock, kWavesWide) void
+__global__ __launch_bounds__(kBlock, kWavesBackward) void
 query_backward_backward_kernel(
         QDev a, const T* __restrict__ gg_off, const T* __restrict__ z,
         T* __restrict__ grad_z, T* __restrict__ grad_emb) {
@@ -1059,7 +1073,7 @@ __device__ __forceinline__ LineTable* line_table(unsigned char* smem, const QDev
 
 // First-order backward, E = 4 (formulas as in query_backward_forward_kernel).
 template <bool LDS, int OUT, int THREADS>
-__global__ __launch_bounds__(THREADS, kWavesWide) void
+__global__ __launch_bounds__(THREADS, kWavesBackward) void
 query_backward_forward_vec_kernel(
         QDev a, const float* __restrict__ z, float* __restrict__ grad_emb,
         float* __restrict__ grad_off) {
@@ -1135,7 +1149,7 @@ query_backward_forward_vec_kernel(
 // Backward of the backward, E = 4 (formulas as in
 // query_backward_backward_kernel).
 template <bool LDS, int OUT, int THREADS>
-__global__ __launch_bounds__(THREADS, kWavesWide) void
+__global__ __launch_bounds__(THREADS, kWavesBackward) void
 query_backward_backward_vec_kernel(
         QDev a, const float* __restrict__ gg_off, const float* __restrict__ z,
         float* __restrict__ grad_z, float* __restrict__ grad_emb) {
@@ -2210,7 +2224,7 @@ unsigned persistent_grid(int64_t ntiles, size_t smem, int max_per_cu) {
 template <typename T, int VEC, int LPQ>
 int launch_forward(const QDev& d, void* out, hipStream_t s) {
     const size_t smem = smem_bytes(d, LPQ);
-    const unsigned g = persistent_grid((d.N + kBlock - 1) / kBlock, smem);
+    const unsigned g = persistent_grid((d.N + kBlock - 1) / kBlock, smem, forward_waves(VEC, LPQ));
     if (lut_in_lds(d)) {
         query_forward_kernel<T, VEC, LPQ, true>
                 <<<g, kBlock, smem, s>>>(d, static_cast<T*>(out));
@@ -2225,7 +2239,7 @@ int launch_forward(const QDev& d, void* out, hipStream_t s) {
 template <typename T, int VEC, int LPQ>
 int launch_grid_forward(const QDev& d, const FrontDev& f, void* out, hipStream_t s) {
     const size_t smem = smem_bytes(d, LPQ);
-    const unsigned g = persistent_grid((d.N + kBlock - 1) / kBlock, smem);
+    const unsigned g = persistent_grid((d.N + kBlock - 1) / kBlock, smem, forward_waves(VEC, LPQ));
     const bool aux = f.gidx_out != nullptr;
 #define ASH_GF(L, A)                                                          \
     grid_forward_kernel<T, VEC, LPQ, L, A><<<g, kBlock, smem, s>>>(d, f, static_cast<T*>(out))
@@ -2245,8 +2259,9 @@ template <typename T, int LPQ>
 int launch_bwd_fwd(const QDev& d, const void* z, void* ge, void* go,
                    hipStream_t s) {
     const size_t smem = smem_bytes(d, LPQ);
-    const unsigned g = persistent_grid((d.N + kBlock - 1) / kBlock, smem);
     const int out = (ge != nullptr ? 1 : 0) | (go != nullptr ? 2 : 0);
+    const unsigned g = persistent_grid((d.N + kBlock - 1) / kBlock, smem,
+                                       backward_waves<T>(out));
 #define ASH_BF(L, O)                                                          \
     query_backward_forward_kernel<T, LPQ, L, O><<<g, kBlock, smem, s>>>(      \
             d, static_cast<const T*>(z), static_cast<T*>(ge),                 \
@@ -2269,8 +2284,9 @@ template <typename T, int LPQ>
 int launch_bwd_bwd(const QDev& d, const void* gg, const void* z, void* gz,
                    void* ge, hipStream_t s) {
     const size_t smem = smem_bytes(d, LPQ);
-    const unsigned g = persistent_grid((d.N + kBlock - 1) / kBlock, smem);
     const int out = (ge != nullptr ? 1 : 0) | (gz != nullptr ? 2 : 0);
+    const unsigned g = persistent_grid((d.N + kBlock - 1) / kBlock, smem,
+                                       backward_waves<T>(out));
 #define ASH_BB(L, O)                                                          \
     query_backward_backward_kernel<T, LPQ, L, O><<<g, kBlock, smem, s>>>(     \
             d, static_cast<const T*>(gg), static_cast<const T*>(z),           \

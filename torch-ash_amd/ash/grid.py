@@ -70,7 +70,13 @@ class _FusedGridForward(torch.autograd.Function):
     that brought it.  One dense gradient leaves the node instead of two that
     autograd would add up over the whole parameter (configuration 4: a second
     zero fill of 0.23 ms and an addition of 0.98 ms).  Where something else
-    holds that tensor, a hook say, the two are added out of place."""
+    holds that tensor, a hook say, the two are added out of place.
+
+    A pass may come here for that gradient alone (a gradient-norm loss taken
+    backward by itself).  It needs nothing of what the node has saved, which may
+    be gone by then, and what a later pass of the features' own needs must
+    outlive it, although the engine frees a node's saved tensors after every pass
+    that goes through the node (`_outlive`)."""
 
     @staticmethod
     def forward(ctx, embeddings, x, table, lut_grid_nb2grid_idx, lut_cell_nb2cell_idx,
@@ -87,20 +93,43 @@ class _FusedGridForward(torch.autograd.Function):
         ctx.grid_dim = grid_dim
         ctx.interpolation = interpolation
         ctx.cell_size = cell_size
+        ctx.spent = False
+        ctx.outliving = None
         ctx.mark_non_differentiable(masks)
         ctx.set_materialize_grads(False)
         return features, masks, again
 
     @staticmethod
     def backward(ctx, z, _grad_masks, carried):
-        *operands, again = ctx.saved_tensors
+        last = not torch._C._autograd._get_current_graph_task_keep_graph()
         if z is None:   # only the gradient of the gradient was asked for
+            if last and not ctx.spent and ctx.outliving is None:
+                _FusedGridForward._outlive(ctx)
             return (carried,) + (None,) * 9
+        if ctx.outliving is None:
+            *operands, again = ctx.saved_tensors
+        else:
+            # (a gradient recorded from here leads straight to the embeddings)
+            operands, versions = ctx.outliving
+            again = None
+            if [t._version for t in operands] != versions:
+                raise RuntimeError("one of the variables needed for gradient computation has been "
+                                   "modified by an inplace operation since an earlier pass")
         grad_embeddings, grad_x = first_order_backward(ctx, z, operands, 0, 1, again, carried)
+        if last:
+            ctx.spent, ctx.outliving = True, None
         if grad_x is not None and ctx.cell_size != 1.0:
             # d cell / d x of x -> (x - origin) / cell_size, as autograd has it
             grad_x = grad_x / ctx.cell_size
         return (grad_embeddings, grad_x) + (None,) * 8
+
+    @staticmethod
+    def _outlive(ctx):
+        """Keeps the operands, with their versions, beyond the running pass.
+        None of them is an output of this node (its copy of the embeddings is
+        left out), so the node does not come to hold itself."""
+        operands = ctx.saved_tensors[:-1]
+        ctx.outliving = operands, [t._version for t in operands]
 
 
 class SparseDenseGrid(ASHModule):

@@ -4,7 +4,6 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <atomic>
 #include <mutex>
 #include <string>
 
@@ -75,14 +74,14 @@ enum Counter {
     kNumCounters = 64
 };
 constexpr int kHostCounters = 8;
-// Page-locked words of a map (take_line) in which kernels leave answers for the
-// host; each place carries its stamp kLandingStamp words behind its start.
+// Page-locked words in which kernels leave answers for the host: a line per call
+// that waits for its answer (Answer), and one of its own for a map (take_line)
+// with two places.  Each place carries its stamp kLandingStamp words behind its
+// start.
 constexpr int kLandingStamp = 8;
-constexpr int kLineWords = 64;
-constexpr int kLineNow = 0;      // counters, fetched and waited for
-constexpr int kLineLate = 16;    // counters, fetched behind a streaming insert or a fusion frame
-constexpr int kLineEarly = 32;   // count left by the first pass of a streaming insert
-constexpr int kLinePair = 48;    // two 64-bit numbers of a call that waits for them (pair_lock)
+constexpr int kLineWords = 32;
+constexpr int kLineLate = 0;     // counters, fetched behind a streaming insert or a fusion frame
+constexpr int kLineEarly = 16;   // count left by the first pass of a streaming insert
 constexpr int64_t kHeaderBytes = 256;
 
 // General region: open addressing over 32-bit state words + 16-byte keys.
@@ -157,9 +156,12 @@ struct ash_map {
     int64_t table_bytes;
     bool general_attached;
     // --- bookkeeping of the counters on the host ------------------------
+    // Several threads may read the counters of one map at a time: what follows,
+    // up to `counters`, is looked at and brought up to date under this lock (not
+    // held while a call waits for words of its own)
+    std::mutex counter_lock;
     int32_t* line;          // page-locked words of the map's own (take_line), made on first use
-    std::atomic<int32_t> stamp;   // of the latest words asked for
-    std::mutex pair_lock;   // held by the call that waits for the words at kLinePair
+    int32_t stamp;          // of the latest words asked for there
     int32_t late_stamp;
     bool late_in_flight;    // the device may still owe the words at kLineLate
     bool late_pending;      // ... and it is the latest state of the counters: nobody has looked at it yet

@@ -1736,9 +1736,10 @@ int clear_table(ash_map* map, hipStream_t s, bool write_heap, int32_t size, bool
 // a microsecond after it was written, where a copy and a stream synchronisation
 // took 12-15 us of an idle device's time.
 //
-// Every map that asks gets a line of kLineWords of its own from a pool for all
-// maps (its slabs serve the maps of the process, as many lines as maps that ever
-// lived at the same time) and gives it back when it is destroyed.
+// A call that waits takes a line of kLineWords for itself and returns it (two
+// threads that read one map's counters have one each), and a map keeps one from
+// its first streaming insert or counted frame until it is destroyed.  The pool
+// serves the process: as many lines as were ever in use at the same time.
 namespace {
 
 constexpr int kLinesPerSlab = 64;
@@ -1749,11 +1750,8 @@ std::vector<int32_t*>& free_lines() {
     return *lines;
 }
 
-}  // namespace
-
-int take_line(ash_map* map) {
+int take_free_line(int32_t** line) {
     std::lock_guard<std::mutex> lock(g_lines_mutex);
-    if (map->line != nullptr) return 0;   // (read under the lock: two threads may ask first)
     std::vector<int32_t*>& lines = free_lines();
     if (lines.empty()) {
         void* slab = nullptr;
@@ -1764,25 +1762,46 @@ int take_line(ash_map* map) {
             lines.push_back(static_cast<int32_t*>(slab) + i * kLineWords);
         }
     }
-    map->line = lines.back();
+    *line = lines.back();
     lines.pop_back();
-    // stamps of this map start where the line's last owner stopped
-    for (int at : {kLineNow, kLineLate, kLineEarly, kLinePair}) {
-        map->stamp = std::max(map->stamp.load(), map->line[at + kLandingStamp]);
-    }
     return 0;
 }
 
-namespace {
-
-void give_back_line(ash_map* map) {
-    if (map->line == nullptr) return;
+// (no launch may still owe words there)
+void give_back_line(int32_t* line) {
+    if (line == nullptr) return;
     std::lock_guard<std::mutex> lock(g_lines_mutex);
-    free_lines().push_back(map->line);
-    map->line = nullptr;
+    free_lines().push_back(line);
+}
+
+int32_t next_stamp(int32_t stamp) {   // (2^31 - 1 goes on at -2^31)
+    return static_cast<int32_t>(static_cast<uint32_t>(stamp) + 1u);
 }
 
 }  // namespace
+
+int Answer::take() {
+    if (take_free_line(&words)) return 1;
+    stamp = next_stamp(words[kLandingStamp]);   // where the line's last owner stopped
+    return 0;
+}
+
+int Answer::wait() {
+    lost_ = wait_for_stamp(words + kLandingStamp, stamp) != 0;
+    return lost_ ? 1 : 0;
+}
+
+Answer::~Answer() {
+    if (!lost_) give_back_line(words);
+}
+
+int take_line(ash_map* map) {
+    std::lock_guard<std::mutex> lock(map->counter_lock);
+    if (map->line != nullptr) return 0;
+    if (take_free_line(&map->line)) return 1;
+    map->stamp = std::max(map->line[kLineLate + kLandingStamp], map->line[kLineEarly + kLandingStamp]);
+    return 0;
+}
 
 // Waits until the device has written `stamp`.  The wait ends with the device's
 // work at the latest: after some seconds without an answer the device is
@@ -1799,14 +1818,31 @@ int wait_for_stamp(const int32_t* word, int32_t stamp) {
     return 0;
 }
 
+namespace {
+
 // A read-back queued behind an insert that may still be under way has to arrive
-// before its words are read or written again.
-int settle_landing_place(ash_map* map) {
+// before its words are read or written again.  The caller holds the map's
+// counter_lock.
+int settle_late_words(ash_map* map) {
     if (map->late_in_flight) {
         if (wait_for_stamp(map->line + kLineLate + kLandingStamp, map->late_stamp)) return 1;
         map->late_in_flight = false;
     }
     return 0;
+}
+
+// The launch before this call leaves the counters at kLineLate with `stamp`: they
+// are the latest state of the counters.  The caller holds the map's counter_lock.
+void late_words_queued(ash_map* map, int32_t stamp) {
+    map->late_stamp = stamp;
+    map->late_in_flight = map->late_pending = true;
+}
+
+}  // namespace
+
+int settle_landing_place(ash_map* map) {
+    std::lock_guard<std::mutex> lock(map->counter_lock);
+    return settle_late_words(map);
 }
 
 int give_up_heap_order(ash_map* map, hipStream_t s) {
@@ -2065,14 +2101,14 @@ int ash_map_attach_general(ash_map_t* map, void* general_ws,
 
 int ash_map_destroy(ash_map_t* map) {
     if (map == nullptr) return 0;
-    // the device may still owe a write into the caller's page-locked landing
-    // place; it must have arrived before the caller gives that memory back
+    // words that the device may still owe must have arrived before their line
+    // serves another map or call
     if (map->late_in_flight) {
         DeviceGuard guard;
         (void)guard.enter(map->device);
         (void)settle_landing_place(map);
     }
-    give_back_line(map);
+    if (!map->late_in_flight) give_back_line(map->line);
     delete map;
     return 0;
 }
@@ -2558,31 +2594,39 @@ void decode_counters(const int32_t* host, ash_counters& c) {
 
 // Brings map->counters up to date (the map's device is current): they are
 // known already, or a read-back queued behind the latest insert brings them,
-// or they are fetched now, which waits for `s`.
-int refresh_counters(ash_map* map, hipStream_t s) {
+// or they are fetched now, which waits for `s`.  `ask`: fetched in any case;
+// `copy`: a copy of them, for callers whose map other threads may read as well.
+int refresh_counters(ash_map* map, hipStream_t s, bool ask = false, ash_counters* copy = nullptr) {
+    std::unique_lock<std::mutex> lock(map->counter_lock);
+    if (ask) map->counters_known = map->late_pending = false;
     if (map->replayed) {
-        if (settle_landing_place(map)) return 1;
+        if (settle_late_words(map)) return 1;
         map->counters_known = map->late_pending = false;
     }
-    if (map->counters_known) return 0;
-    if (map->late_pending) {
-        if (settle_landing_place(map)) return 1;
-        map->late_pending = false;
-        decode_counters(map->line + kLineLate, map->counters);
-    } else {
-        if (is_capturing(s)) {
-            ASH_FAIL("the table's counters cannot be read while the stream is being captured");
+    if (!map->counters_known) {
+        if (map->late_pending) {
+            if (settle_late_words(map)) return 1;
+            map->late_pending = false;
+            decode_counters(map->line + kLineLate, map->counters);
+        } else {
+            if (is_capturing(s)) {
+                ASH_FAIL("the table's counters cannot be read while the stream is being captured");
+            }
+            // (each of several readers waits for its own stream, not for the others)
+            lock.unlock();
+            Answer answer;
+            if (answer.take()) return 1;
+            publish_counters_kernel<<<1, 64, 0, s>>>(map->d.ctr, answer.words, answer.stamp);
+            ASH_LAUNCH_CHECK();
+            if (answer.wait()) return 1;
+            lock.lock();
+            decode_counters(answer.words, map->counters);
         }
-        if (take_line(map)) return 1;
-        const int32_t stamp = ++map->stamp;
-        publish_counters_kernel<<<1, 64, 0, s>>>(map->d.ctr, map->line + kLineNow, stamp);
-        ASH_LAUNCH_CHECK();
-        if (wait_for_stamp(map->line + kLineNow + kLandingStamp, stamp)) return 1;
-        decode_counters(map->line + kLineNow, map->counters);
+        map->counters_known = true;
+        map->unread_inserts = 0;
+        if (map->counters.dropped > 0 || map->counters.tombstones > 0) map->maybe_tombstones = true;
     }
-    map->counters_known = true;
-    map->unread_inserts = 0;
-    if (map->counters.dropped > 0 || map->counters.tombstones > 0) map->maybe_tombstones = true;
+    if (copy != nullptr) *copy = map->counters;
     return 0;
 }
 
@@ -2652,13 +2696,14 @@ int upkeep(ash_map* map, int64_t incoming, void* scratch, int64_t scratch_bytes,
 }  // extern "C"
 
 int ash::queue_touched_count(ash_map* map, const int32_t* counts, int n, hipStream_t s) {
-    if (take_line(map) || settle_landing_place(map)) return 1;
-    map->late_stamp = ++map->stamp;
-    publish_touched_kernel<<<1, kBlock, 0, s>>>(map->d.ctr, counts, n, map->line + kLineLate,
-                                                map->late_stamp);
+    if (take_line(map)) return 1;
+    std::lock_guard<std::mutex> lock(map->counter_lock);
+    if (settle_late_words(map)) return 1;
+    const int32_t stamp = map->stamp = next_stamp(map->stamp);
+    publish_touched_kernel<<<1, kBlock, 0, s>>>(map->d.ctr, counts, n, map->line + kLineLate, stamp);
     ASH_LAUNCH_CHECK();
     map->counters_known = false;
-    map->late_in_flight = map->late_pending = true;
+    late_words_queued(map, stamp);
     return 0;
 }
 
@@ -2675,8 +2720,8 @@ int ash_map_counters(ash_map_t* map, int32_t* staging, int64_t out[7], void* str
     if (out == nullptr) ASH_FAIL("null status output");
     DeviceGuard guard;
     ASH_HIP(guard.enter(map->device));
-    if (refresh_counters(map, static_cast<hipStream_t>(stream))) return 1;
-    const ash_counters& c = map->counters;
+    ash_counters c;
+    if (refresh_counters(map, static_cast<hipStream_t>(stream), false, &c)) return 1;
     out[0] = c.size;
     out[1] = c.dropped;
     out[2] = c.tombstones;
@@ -2715,10 +2760,8 @@ int ash_map_status(ash_map_t* map, int64_t out[5], void* stream) {
     DeviceGuard guard;
     ASH_HIP(guard.enter(map->device));
     // always a copy from the device
-    map->counters_known = false;
-    map->late_pending = false;
-    if (refresh_counters(map, static_cast<hipStream_t>(stream))) return 1;
-    const ash_counters& c = map->counters;
+    ash_counters c;
+    if (refresh_counters(map, static_cast<hipStream_t>(stream), true, &c)) return 1;
     out[0] = c.size;
     out[1] = c.dropped;
     out[2] = c.tombstones;
@@ -2811,7 +2854,7 @@ int ash_map_insert_auto(ash_map_t* map, const int32_t* keys, int64_t n, int n_va
             if (take_line(map) || settle_landing_place(map)) return 1;
             early = map->line + kLineEarly;
         }
-        const int32_t stamp = ++map->stamp;
+        const int32_t stamp = map->stamp = next_stamp(map->stamp);
         // Only keys that the first pass hands to the per-key kernel can be
         // waiting for the second region; their number arrives a quarter into
         // the call's work.  None: the counters come with the insert's last
@@ -2824,10 +2867,9 @@ int ash_map_insert_auto(ash_map_t* map, const int32_t* keys, int64_t n, int n_va
         }
         if (capturing) return 0;
         if (published) {
-            map->late_stamp = stamp;
-            map->late_in_flight = true;
-            map->late_pending = true;
+            std::lock_guard<std::mutex> lock(map->counter_lock);
             map->unread_inserts = 0;
+            late_words_queued(map, stamp);
             return 0;
         }
     } else {

@@ -699,8 +699,8 @@ int ash_ray_sample_march(ash_map_t* map, uint8_t* scratch, int volume_lo, int vo
     DeviceGuard guard;
     ASH_HIP(guard.enter(map->device));
     if (settle_table(map, s)) return 1;
-    std::lock_guard<std::mutex> one_answer(map->pair_lock);
-    if (take_line(map)) return 1;
+    Answer answer;
+    if (answer.take()) return 1;
     Volume volume;
     if (make_volume(map, scratch, volume_lo, volume_hi, volume, s)) return 1;
     auto* g = reinterpret_cast<GroupSamples*>(groups);
@@ -710,14 +710,12 @@ int ash_ray_sample_march(ash_map_t* map, uint8_t* scratch, int volume_lo, int vo
                      counts, nullptr, nullptr, nullptr, nullptr, stage, stride, g, s)) {
         return 1;
     }
-    int32_t* landing = map->line + kLinePair;
-    const int32_t stamp = ++map->stamp;
-    ray_scan_kernel<<<1, kScanThreads, 0, s>>>(g, static_cast<int>(march_groups(n)), landing, stamp);
+    ray_scan_kernel<<<1, kScanThreads, 0, s>>>(g, static_cast<int>(march_groups(n)), answer.words, answer.stamp);
     ASH_LAUNCH_CHECK();
-    if (wait_for_stamp(landing + kLandingStamp, stamp)) return 1;
+    if (answer.wait()) return 1;
     for (int w = 0; w < 2; ++w) {
-        out[w] = static_cast<int64_t>(static_cast<uint32_t>(landing[2 * w])) |
-                 (static_cast<int64_t>(landing[2 * w + 1]) << 32);
+        out[w] = static_cast<int64_t>(static_cast<uint32_t>(answer.words[2 * w])) |
+                 (static_cast<int64_t>(answer.words[2 * w + 1]) << 32);
     }
     return 0;
 }

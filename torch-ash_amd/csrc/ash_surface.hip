@@ -677,8 +677,8 @@ int ash_surface_block8_classify(ash_map_t* map, const void* sdfs, int64_t sdf_st
     }
     DeviceGuard guard;
     ASH_HIP(guard.enter(map->device));
-    std::lock_guard<std::mutex> one_answer(map->pair_lock);
-    if (take_line(map)) return 1;
+    Answer answer;
+    if (answer.take()) return 1;
     const int64_t units = num_embeddings * 8;
     clear_bits_kernel<<<static_cast<unsigned>((units + kBlock - 1) / kBlock), kBlock, 0, s>>>(
             reinterpret_cast<uint4*>(a.w.bits), units);
@@ -695,14 +695,12 @@ int ash_surface_block8_classify(ash_map_t* map, const void* sdfs, int64_t sdf_st
     const int64_t groups = groups_of(num_grids);
     count_kernel<<<static_cast<unsigned>(groups), kCountThreads, 0, s>>>(a);
     ASH_LAUNCH_CHECK();
-    int32_t* landing = map->line + kLinePair;
-    const int32_t stamp = ++map->stamp;
-    scan_groups_kernel<<<1, kScanThreads, 0, s>>>(a.w.groups, groups, landing, stamp);
+    scan_groups_kernel<<<1, kScanThreads, 0, s>>>(a.w.groups, groups, answer.words, answer.stamp);
     ASH_LAUNCH_CHECK();
-    if (wait_for_stamp(landing + kLandingStamp, stamp)) return 1;
+    if (answer.wait()) return 1;
     for (int w = 0; w < 2; ++w) {
-        out[w] = static_cast<int64_t>(static_cast<uint32_t>(landing[2 * w])) |
-                 (static_cast<int64_t>(landing[2 * w + 1]) << 32);
+        out[w] = static_cast<int64_t>(static_cast<uint32_t>(answer.words[2 * w])) |
+                 (static_cast<int64_t>(answer.words[2 * w + 1]) << 32);
     }
     if (out[0] > 0x7FFFFFFFll) ASH_FAIL("marching_cubes: more than 2^31 vertices");
     if (out[1] > 0x7FFFFFFFll / 3) ASH_FAIL("marching_cubes: too many triangles");

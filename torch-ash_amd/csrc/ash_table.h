@@ -170,9 +170,26 @@ inline bool heap_in_order(const ash_map* map) { return !map->heap_dirty && !map-
 // false for one that took entries away.
 // `s`: the stream the call runs on (captured: see ash_map::replayed).
 void counters_changed(ash_map* map, bool inserted, hipStream_t s);
-// The map's page-locked words (made on first use), and the wait for one of them.
+// Page-locked words of one call's own, in which a kernel leaves what the call
+// waits for: up to kLandingStamp words, and behind them the call's stamp.
+class Answer {
+  public:
+    Answer() = default;
+    Answer(const Answer&) = delete;
+    Answer& operator=(const Answer&) = delete;
+    ~Answer();
+    int take();   // `words` and `stamp` are the call's from here on
+    int wait();   // until the device has left them
+    int32_t* words = nullptr;
+    int32_t stamp = 0;
+
+  private:
+    bool lost_ = false;   // the device may still owe the words
+};
+// The map's own page-locked words (made on first use), and the wait for one of them.
 int take_line(ash_map* map);
 int wait_for_stamp(const int32_t* word, int32_t stamp);
+// Waits for the counters that a launch may still owe at kLineLate.
 int settle_landing_place(ash_map* map);
 // Adds up `n` words of `counts` into the counter of touched blocks and queues the
 // read-back of the counters behind the stream's work (ash_map.hip).

@@ -1,6 +1,7 @@
 """Calls that wait for words the device leaves on the host, from several threads
 on one map: each has words of its own and waits for its own stream."""
 import threading
+import time
 
 import pytest
 import torch
@@ -60,6 +61,22 @@ def test_queued_counters_read_by_several_threads(gpu_ash, queued):
         table.insert(keys[:n])
         assert _together(4, lambda _: table.size()) == [n] * 4
         assert bool(table.find(keys[:n]).all())
+
+
+def test_a_streaming_insert_that_waits_leaves_the_core(gpu_ash):
+    """Behind some hundredths of a second of work the waiting thread sleeps."""
+    keys = torch.arange(900_000, dtype=torch.int32, device=DEV).view(-1, 3)
+    table = gpu_ash.HashSet(3, 600_000, DEV)
+    work = torch.randn(8192, 8192, device=DEV)
+    torch.tanh(work @ work)
+    torch.cuda.synchronize()
+    for _ in range(12):
+        work = torch.tanh(work @ work)
+    wall, cpu = time.perf_counter(), time.thread_time()
+    table.insert(keys)
+    assert table.size() == 300_000
+    wall, cpu = time.perf_counter() - wall, time.thread_time() - cpu
+    assert wall > 0.02 and cpu < 0.5 * wall, (wall, cpu)
 
 
 def test_rays_sampled_by_several_threads(gpu_ash):

@@ -26,11 +26,11 @@
 
 #include <hip/amd_detail/amd_hip_unsafe_atomics.h>
 
-#include <sched.h>
-
 #include <algorithm>
+#include <chrono>
 #include <cstring>
 #include <mutex>
+#include <thread>
 #include <vector>
 
 // Scratch of ash_grid_activate_static, the entry point that allocates nothing:
@@ -1778,6 +1778,15 @@ int32_t next_stamp(int32_t stamp) {   // (2^31 - 1 goes on at -2^31)
     return static_cast<int32_t>(static_cast<uint32_t>(stamp) + 1u);
 }
 
+// Looks for `stamp` for about as long as a short call takes; true: it has come.
+bool has_come(const int32_t* word, int32_t stamp) {
+    for (int spin = 0; spin < 20'000; ++spin) {
+        if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == stamp) return true;
+        __builtin_ia32_pause();
+    }
+    return __atomic_load_n(word, __ATOMIC_ACQUIRE) == stamp;
+}
+
 }  // namespace
 
 int Answer::take() {
@@ -1786,9 +1795,18 @@ int Answer::take() {
     return 0;
 }
 
-int Answer::wait() {
-    lost_ = wait_for_stamp(words + kLandingStamp, stamp) != 0;
-    return lost_ ? 1 : 0;
+// Where work that takes longer is queued ahead the stream, of which the launch
+// that leaves the words is the last, is waited for instead of polling on; errors
+// show there, and the words have to be there afterwards.
+int Answer::wait(hipStream_t s) {
+    const int32_t* word = words + kLandingStamp;
+    lost_ = true;
+    if (!has_come(word, stamp)) {
+        ASH_HIP(hipStreamSynchronize(s));
+        if (!has_come(word, stamp)) ASH_FAIL("internal error: the device has not left its answer");
+    }
+    lost_ = false;
+    return 0;
 }
 
 Answer::~Answer() {
@@ -1803,18 +1821,22 @@ int take_line(ash_map* map) {
     return 0;
 }
 
-// Waits until the device has written `stamp`.  The wait ends with the device's
-// work at the latest: after some seconds without an answer the device is
-// synchronised (errors show there), after which the word has to be there.
+// Waits until the device has written `stamp` with more work queued behind the
+// launch that does: an event there would cost 3 of the 75 us of a set of 1 M keys,
+// the stream's end comes too late for what is to be queued next, and the stream
+// may be gone.  Where more than a short call is queued ahead, the word is looked
+// for every tenth of a millisecond (no core is kept busy and no other stream
+// waited for); only when a minute has passed the device is synchronised, where
+// an error would show.
 int wait_for_stamp(const int32_t* word, int32_t stamp) {
-    const auto arrived = [&] { return __atomic_load_n(word, __ATOMIC_ACQUIRE) == stamp; };
-    for (int64_t spin = 0; spin < 4'000'000; ++spin) {
-        if (arrived()) return 0;
-        __builtin_ia32_pause();
-        if (spin > 20'000) sched_yield();
+    bool come = has_come(word, stamp);
+    for (int look = 0; !come && look < 600'000; ++look) {
+        std::this_thread::sleep_for(std::chrono::microseconds(100));
+        come = __atomic_load_n(word, __ATOMIC_ACQUIRE) == stamp;
     }
+    if (come) return 0;
     ASH_HIP(hipDeviceSynchronize());
-    if (!arrived()) ASH_FAIL("internal error: the device has not left its counters");
+    if (!has_come(word, stamp)) ASH_FAIL("internal error: the device has not left its counters");
     return 0;
 }
 
@@ -2618,7 +2640,7 @@ int refresh_counters(ash_map* map, hipStream_t s, bool ask = false, ash_counters
             if (answer.take()) return 1;
             publish_counters_kernel<<<1, 64, 0, s>>>(map->d.ctr, answer.words, answer.stamp);
             ASH_LAUNCH_CHECK();
-            if (answer.wait()) return 1;
+            if (answer.wait(s)) return 1;
             lock.lock();
             decode_counters(answer.words, map->counters);
         }

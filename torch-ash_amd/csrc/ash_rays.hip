@@ -712,7 +712,7 @@ int ash_ray_sample_march(ash_map_t* map, uint8_t* scratch, int volume_lo, int vo
     }
     ray_scan_kernel<<<1, kScanThreads, 0, s>>>(g, static_cast<int>(march_groups(n)), answer.words, answer.stamp);
     ASH_LAUNCH_CHECK();
-    if (answer.wait()) return 1;
+    if (answer.wait(s)) return 1;
     for (int w = 0; w < 2; ++w) {
         out[w] = static_cast<int64_t>(static_cast<uint32_t>(answer.words[2 * w])) |
                  (static_cast<int64_t>(answer.words[2 * w + 1]) << 32);

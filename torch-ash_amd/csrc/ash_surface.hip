@@ -697,7 +697,7 @@ int ash_surface_block8_classify(ash_map_t* map, const void* sdfs, int64_t sdf_st
     ASH_LAUNCH_CHECK();
     scan_groups_kernel<<<1, kScanThreads, 0, s>>>(a.w.groups, groups, answer.words, answer.stamp);
     ASH_LAUNCH_CHECK();
-    if (answer.wait()) return 1;
+    if (answer.wait(s)) return 1;
     for (int w = 0; w < 2; ++w) {
         out[w] = static_cast<int64_t>(static_cast<uint32_t>(answer.words[2 * w])) |
                  (static_cast<int64_t>(answer.words[2 * w + 1]) << 32);

@@ -178,8 +178,8 @@ class Answer {
     Answer(const Answer&) = delete;
     Answer& operator=(const Answer&) = delete;
     ~Answer();
-    int take();   // `words` and `stamp` are the call's from here on
-    int wait();   // until the device has left them
+    int take();                // `words` and `stamp` are the call's from here on
+    int wait(hipStream_t s);   // `s`: the stream whose latest launch leaves them
     int32_t* words = nullptr;
     int32_t stamp = 0;
 

@@ -74,6 +74,36 @@ def test_gradient_of_embedding_rows(gpu_ash, dtype, width, n):
     assert torch.equal(back, u[indices] * masks.unsqueeze(1))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_gradient_under_the_deterministic_flag(gpu_ash, dtype):
+    """Rows that many keys share: the sums torch's backward of indexing takes,
+    bit for bit, whichever pass the flag is first seen by."""
+    emb = gpu_ash.HashEmbedding(3, 60, 8, DEV)
+    emb.embedding = torch.nn.Parameter(torch.randn(60, 8, device=DEV, dtype=dtype))
+    g = torch.Generator().manual_seed(2)
+    keys = torch.unique(torch.randint(-30, 30, (50, 3), generator=g, dtype=torch.int32), dim=0)
+    emb.spatial_init_(keys.to(DEV))
+    q = _queries(keys, 50_001, seed=9)
+    indices, masks = emb.engine.find(q)
+    z = torch.randn(len(q), 8, generator=g, dtype=dtype).to(DEV)
+    table = emb.embedding.detach().clone().requires_grad_(True)
+    (masks.unsqueeze(-1) * table[indices]).backward(z)
+    y = emb(q)
+    try:
+        torch.use_deterministic_algorithms(True)
+        for out in (y, emb(q), emb(q)):
+            (got,) = torch.autograd.grad(out, emb.embedding, z)
+            assert torch.equal(got, table.grad)
+        # and on to the gradient of the gradient
+        zz = z.clone().requires_grad_(True)
+        (got,) = torch.autograd.grad(emb(q), emb.embedding, zz, create_graph=True)
+        u = torch.randn(60, 8, device=DEV, dtype=dtype)
+        (back,) = torch.autograd.grad(got, zz, u)
+    finally:
+        torch.use_deterministic_algorithms(False)
+    assert torch.equal(got, table.grad) and torch.equal(back, u[indices] * masks.unsqueeze(1))
+
+
 def test_embedding_under_transforms_and_forward_mode(gpu_ash):
     """A batch of parameters (vmap) and a forward-mode tangent go through
     torch's own operations, as they always did."""

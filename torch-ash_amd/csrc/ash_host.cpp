@@ -238,6 +238,14 @@ struct Rows : torch::autograd::Function<Rows> {
                                                    torch::autograd::variable_list grads) {
         const auto saved = ctx->get_saved_variables();
         const int64_t num_rows = ctx->saved_data["num_rows"].toInt();
+        if (at::globalContext().deterministicAlgorithms()) {
+            // add_rows adds by atomics, in any order: where torch is asked for the
+            // same numbers on every run, its own backward of indexing, which sorts
+            const Tensor rows = saved[1].unsqueeze(-1) * grads[0];
+            return {at::zeros({num_rows, rows.size(1)}, rows.options())
+                            .index_put({saved[0]}, rows, /*accumulate=*/true),
+                    Tensor(), Tensor(), Tensor(), Tensor()};
+        }
         Tensor grad = at::GradMode::is_enabled()
                               ? AddRows::apply(grads[0], saved[0], saved[1], num_rows)
                               : add_rows(grads[0], saved[0], saved[1], num_rows);

@@ -20,8 +20,10 @@
 // 3^3 1275 -> 490 us, 7^3 4.3 -> 3.8 ms; two channels 501 -> 179 us, 2.2 -> 1.0
 // ms; 1000 blocks, 7^3: 990 -> 95 us (every workgroup used to check the tables).
 // 3^3 windows of five channels move 1.55 GB beyond the L2s (the halo along x
-// takes most lines of two neighbours), 3.2 TB/s; 7^3 are bound by vector
-// instructions.
+// takes most lines of two neighbours), 3.2 TB/s.  7^3 windows of two channels are
+// bound by vector instructions (issued in 0.87 of the cycles; 1941 per wavefront
+// and block, 1372 of them multiply-adds and 343 tap reads), of five by the one
+// workgroup of ten wavefronts that a CU's registers hold (0.59).
 //
 // The block's own rows are contiguous in memory whatever their width: they come
 // in as two 16-byte pieces per thread, and leave the same way, through LDS.
@@ -71,8 +73,13 @@ struct Shape {
     static constexpr int kTileWords = E * kPlane;
     static constexpr int kOutWords = kG * kOutLayer;
     static constexpr int kWeightWords = E * W * 64;
-    // wavefronts per SIMD that the tile leaves room for
-    static constexpr int kMostWaves = W == 3 ? 6 : 5;
+    // wavefronts per SIMD that the tile leaves room for.  No more than the
+    // registers allow without spills: 64 for windows of 3 and 74 - 76 for 5 are
+    // below what the bound leaves them, 108 for 7 are four wavefronts.  (Five,
+    // 96 registers, spill 10 - 12 of them.  20 000 blocks, 7^3: one channel 222
+    // -> 192 us, two 344 -> 340, three 814 -> 651, five 1181 -> 1112; 2000
+    // blocks: 47 -> 50, 61 -> 62, 105 -> 94, 150 -> 140.)
+    static constexpr int kMostWaves = W == 3 ? 6 : (W == 5 ? 5 : 4);
     static constexpr int waves() {
         const int lds = 4 * (kTileWords + kOutWords + kWeightWords) + 1024;
         const int fit = (160 * 1024 / lds * E * kParts + 3) / 4;

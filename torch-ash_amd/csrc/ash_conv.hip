@@ -316,18 +316,10 @@ __global__ __launch_bounds__(kFillBlock) void zero_others_kernel(uint4* __restri
 template <int E, int W>
 int launch(const ConvArgs& a, hipStream_t s) {
     // as many workgroups as the device holds at once: they walk the listing
-    static const int per_cu = [] {
-        int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                    &n, convolution_block8_kernel<E, W>, Shape<E, W>::kThreads, 0) != hipSuccess) {
-            (void)hipGetLastError();
-            n = 1;
-        }
-        return n < 1 ? 1 : n;
-    }();
-    int64_t groups = static_cast<int64_t>(per_cu) * 256;
+    constexpr auto kernel = convolution_block8_kernel<E, W>;
+    int64_t groups = static_cast<int64_t>(compute_units()) * resident_per_cu<kernel>(Shape<E, W>::kThreads);
     if (groups > a.n_grids) groups = a.n_grids;
-    convolution_block8_kernel<E, W><<<static_cast<unsigned>(groups), Shape<E, W>::kThreads, 0, s>>>(a);
+    kernel<<<static_cast<unsigned>(groups), Shape<E, W>::kThreads, 0, s>>>(a);
     ASH_LAUNCH_CHECK();
     return 0;
 }

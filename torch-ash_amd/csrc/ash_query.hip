@@ -46,11 +46,14 @@ constexpr int kLdsPerCu = 160 * 1024;
 // Wavefronts per SIMD, which is workgroups per CU.  Forward kernels are held to
 // the 64 registers of eight, but for the widest rows (64 - 70 registers, seven),
 // which would spill; the backward ones are bound by their registers (both
-// gradients: 67 - 71, seven; in double precision 88 - 112, four, and five for
-// one) or by LDS.  A persistent grid is as many workgroups as are resident: the
-// eighth of a CU where seven fit started when the others were done.  Backward of
-// 1 - 1.5 M ray samples, rows of sixteen 215 -> 178 us, eight 138 -> 120, five
-// 220 -> 206; forward of 2^22, rows of four, 132 -> 126.
+// gradients: 51 - 71, seven; in double precision 88 - 112, four) or by LDS.  A
+// persistent grid is as many workgroups as are resident: the eighth of a CU where
+// seven fit started when the others were done.  Backward of 1 - 1.5 M ray samples,
+// rows of sixteen 215 -> 178 us, eight 138 -> 120, five 220 -> 206; forward of
+// 2^22, rows of four, 132 -> 126.  One gradient in double precision takes 50 - 87
+// registers, five to eight workgroups, and is launched with five: with as many as
+// each instance has room for (the occupancy query) 1 M and 3 M ray samples took
+// 0.93 - 1.08 of the time, 1.00 on average over rows of 1 to 16.
 constexpr int kWavesFull = 8;
 constexpr int kWavesWide = 7;
 constexpr int kWavesBackward = 3;
@@ -2197,24 +2200,12 @@ size_t smem_bytes(const QDev& d, int lpq, int line_tables = 0) {
 
 // Enough persistent workgroups to fill every CU as far as LDS allows.
 unsigned persistent_grid(int64_t ntiles, size_t smem, int max_per_cu) {
-    static int cus = 0;
-    if (cus == 0) {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount,
-                                  dev) == hipSuccess &&
-            n > 0) {
-            cus = n;
-        } else {
-            cus = 256;
-        }
-    }
     int per_cu = max_per_cu;
     if (smem > 0) {
         const int fit = static_cast<int>(kLdsPerCu / smem);
         if (fit < per_cu) per_cu = fit < 1 ? 1 : fit;
     }
-    int64_t g = static_cast<int64_t>(cus) * per_cu;
+    int64_t g = static_cast<int64_t>(compute_units()) * per_cu;
     if (g > ntiles) g = ntiles;
     g = (g + kXcds - 1) / kXcds * kXcds;  // whole rounds over the XCDs
     if (g < kXcds) g = kXcds;

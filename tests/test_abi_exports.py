@@ -51,6 +51,21 @@ def test_library_is_built_from_the_sources_beside_it(lib):
     assert lib.ash_source_fingerprint().decode() == build.source_fingerprint()
 
 
+def test_host_module_is_built_from_the_source_beside_it(lib):
+    """The same for the module that makes the calls on torch tensors."""
+    import importlib.util
+
+    import torch  # noqa: F401  (the module's libraries)
+
+    parts = []
+    for name, path in (("ash_build", ("build.py",)), ("_ash_host", ("ash", "lib", "_ash_host.so"))):
+        spec = importlib.util.spec_from_file_location(name, os.path.join(ROOT, "torch-ash_amd", *path))
+        parts.append(importlib.util.module_from_spec(spec))
+        spec.loader.exec_module(parts[-1])
+    build, host = parts
+    assert host.source_fingerprint == build.host_fingerprint()
+
+
 def _error(lib):
     return lib.ash_last_error().decode()
 

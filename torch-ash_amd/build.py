@@ -70,6 +70,19 @@ def source_fingerprint() -> str:
     return h.hexdigest()
 
 
+def host_fingerprint() -> str:
+    """The same for the host module (its source and the header of the C ABI),
+    compiled in as _ash_host.source_fingerprint."""
+    import hashlib
+
+    h = hashlib.sha256()
+    for path in (HOST_SOURCE, HEADERS[-1]):
+        h.update(os.path.basename(path).encode())
+        with open(path, "rb") as f:
+            h.update(f.read())
+    return h.hexdigest()
+
+
 def _older(out, deps) -> bool:
     if not os.path.exists(out):
         return True
@@ -98,6 +111,7 @@ def host_command(out: str):
         os.environ.get("CXX") or shutil.which("g++") or "c++",
         "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
         "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_API_INCLUDE_EXTENSION_H",
+        f'-DASH_HOST_FINGERPRINT="{host_fingerprint()}"',
         f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
         *[arg for path in dict.fromkeys(includes) for arg in ("-isystem", path)],
         HOST_SOURCE, "-o", out, f"-L{libs}", "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10",

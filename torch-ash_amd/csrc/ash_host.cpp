@@ -21,6 +21,10 @@
 
 #include "../../include/ash_hip.h"
 
+#ifndef ASH_HOST_FINGERPRINT
+#define ASH_HOST_FINGERPRINT "unknown"
+#endif
+
 namespace {
 
 using torch::Tensor;
@@ -794,11 +798,12 @@ std::tuple<Optional, Tensor, std::vector<Tensor>> find_rows_py(uintptr_t handle,
 
 PYBIND11_MODULE(_ash_host, m) {
     m.doc() = "host side of libash_hip.so's calls on torch tensors";
+    // (build.py: host_fingerprint)
+    m.attr("source_fingerprint") = ASH_HOST_FINGERPRINT;
     m.def("bind", &bind);
     m.def("find", &find);
     m.def("finds_rows_of", &finds_rows_of);
     m.def("find_rows", &find_rows_py);
-    m.def("add_rows", &add_rows);
     m.def("embedding_rows", &embedding_rows);
     m.def("gather_rows", &gather_rows);
     m.def("insert", &insert);

@@ -280,7 +280,7 @@ __global__ __launch_bounds__(kBlock) void ray_sample_kernel(
         }
     };
     const int shift = lane & ~(LPR - 1);
-    const uint64_t all = LPR == 64 ? ~0ull : (1ull << LPR) - 1ull;
+    constexpr uint64_t all = (1ull << LPR) - 1ull;   // (4 or 8 lanes)
     bool run_stored = true;   // what the positions ahead are taken for
     while (__ballot(live)) {
         const float by = run_stored ? t_step : t_grid_step;

@@ -473,8 +473,9 @@ int ash_map_status(ash_map_t* map, int64_t out[5], void* stream);
  * region.  The handle follows every call that changes them: after a clear they
  * are known to be zero, after ash_map_insert_auto they have been read (or are
  * on their way, see there) -- only when neither holds is the device asked,
- * which waits for `stream`: a kernel writes them into page-locked words that
- * the library keeps for the map, and the host polls those.  `staging` is not
+ * which waits for `stream`: a kernel writes them into page-locked words of the
+ * call's own, and the host looks for them there.  Several threads may read the
+ * counters of one map at a time, each on its own stream.  `staging` is not
  * used any more (NULL).  No counterpart in the reference, whose `size()`
  * synchronises every time (ash/src/hashmap_gpu.cuh:157). */
 int ash_map_counters(ash_map_t* map, int32_t* staging, int64_t out[7], void* stream);

@@ -17,10 +17,11 @@
 // multiply-add per tap, as in the other kernels.
 //
 // 60 000 blocks, tables and instances for powers of two before: five channels
-// 3^3 1275 -> 490 us, 7^3 4.3 -> 3.8 ms; two channels 501 -> 179 us, 2.2 -> 1.0
-// ms; 1000 blocks, 7^3: 990 -> 95 us (every workgroup used to check the tables).
-// 3^3 windows of five channels move 1.55 GB beyond the L2s (the halo along x
-// takes most lines of two neighbours), 3.2 TB/s.  7^3 windows of two channels are
+// 3^3 1275 -> 477 us, 7^3 4.3 -> 3.5 ms; two channels 501 -> 159 us, 2.2 -> 1.0
+// ms; 1000 blocks, 7^3: 990 -> 94 us (every workgroup used to check the tables).
+// 3^3 windows of five channels move 1.72 GB beyond the L2s, 3.9 TB/s: 0.61 GB of
+// results and 1.11 of rows, 1.8 times what there are (the halo along x takes most
+// lines of two neighbours).  7^3 windows of two channels are
 // bound by vector instructions (issued in 0.87 of the cycles; 1941 per wavefront
 // and block, 1372 of them multiply-adds and 343 tap reads), of five by the one
 // workgroup of ten wavefronts that a CU's registers hold (0.59).

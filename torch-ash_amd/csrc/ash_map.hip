@@ -1778,9 +1778,9 @@ int32_t next_stamp(int32_t stamp) {   // (2^31 - 1 goes on at -2^31)
     return static_cast<int32_t>(static_cast<uint32_t>(stamp) + 1u);
 }
 
-// Looks for `stamp` for about as long as a short call takes; true: it has come.
-bool has_come(const int32_t* word, int32_t stamp) {
-    for (int spin = 0; spin < 20'000; ++spin) {
+// Looks for `stamp` `looks` times, 20 - 50 ns apart; true: it has come.
+bool has_come(const int32_t* word, int32_t stamp, int looks) {
+    for (int look = 0; look < looks; ++look) {
         if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == stamp) return true;
         __builtin_ia32_pause();
     }
@@ -1795,15 +1795,16 @@ int Answer::take() {
     return 0;
 }
 
-// Where work that takes longer is queued ahead the stream, of which the launch
-// that leaves the words is the last, is waited for instead of polling on; errors
+// Looks for the words for some ten milliseconds.  Where work that takes longer is
+// queued ahead the stream, of which the launch that leaves them is the last, is
+// waited for (which keeps a core just as busy and comes back 5 us later); errors
 // show there, and the words have to be there afterwards.
 int Answer::wait(hipStream_t s) {
     const int32_t* word = words + kLandingStamp;
     lost_ = true;
-    if (!has_come(word, stamp)) {
+    if (!has_come(word, stamp, 400'000)) {
         ASH_HIP(hipStreamSynchronize(s));
-        if (!has_come(word, stamp)) ASH_FAIL("internal error: the device has not left its answer");
+        if (!has_come(word, stamp, 1)) ASH_FAIL("internal error: the device has not left its answer");
     }
     lost_ = false;
     return 0;
@@ -1829,14 +1830,14 @@ int take_line(ash_map* map) {
 // waited for); only when a minute has passed the device is synchronised, where
 // an error would show.
 int wait_for_stamp(const int32_t* word, int32_t stamp) {
-    bool come = has_come(word, stamp);
+    bool come = has_come(word, stamp, 20'000);
     for (int look = 0; !come && look < 600'000; ++look) {
         std::this_thread::sleep_for(std::chrono::microseconds(100));
         come = __atomic_load_n(word, __ATOMIC_ACQUIRE) == stamp;
     }
     if (come) return 0;
     ASH_HIP(hipDeviceSynchronize());
-    if (!has_come(word, stamp)) ASH_FAIL("internal error: the device has not left its counters");
+    if (!has_come(word, stamp, 1)) ASH_FAIL("internal error: the device has not left its counters");
     return 0;
 }
 

@@ -43,13 +43,19 @@ def _losses(grid, x):
     return xq, (y**2).mean(), (gx.norm(dim=-1) - 1).abs().mean(), y
 
 
-def _check(grid, x):
+def _check(ash, grid, x):
+    def added(*losses):
+        with ash.dense_grad(grid):
+            for loss in losses:
+                loss.backward()
+
     ways = {
         "together": lambda a, b: (a + b).backward(),
         "value first": lambda a, b: (a.backward(), b.backward()),
         "gradient first": lambda a, b: (b.backward(), a.backward()),
         "value retained": lambda a, b: (a.backward(retain_graph=True), b.backward()),
         "gradient retained": lambda a, b: (b.backward(retain_graph=True), a.backward()),
+        "added to .grad": lambda a, b: added(b, a),
     }
     want = None
     for name, way in ways.items():
@@ -92,9 +98,9 @@ def _check(grid, x):
 
 
 def test_passes_one_after_the_other(fused_ash):
-    _check(*_grid(fused_ash, torch.device("cpu")))
+    _check(fused_ash, *_grid(fused_ash, torch.device("cpu")))
 
 
 @pytest.mark.gpu
 def test_passes_one_after_the_other_on_the_device(gpu_ash):
-    _check(*_grid(gpu_ash, torch.device("cuda:0")))
+    _check(gpu_ash, *_grid(gpu_ash, torch.device("cuda:0")))

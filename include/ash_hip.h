@@ -573,6 +573,18 @@ int ash_map_find_rows(ash_map_t* map, const int32_t* keys, int64_t n, int n_valu
                       const int64_t* src_rows, int zero_misses, int64_t* indices,
                       uint8_t* masks, void* stream);
 
+/* The same with scratch memory: batches of a million keys and more that read two
+ * tables or more look the keys up first and read the rows in the tables' order
+ * then.  ash_map_find_rows_scratch_bytes says how much memory that takes for
+ * such a call, 0 where it is no gain; a call with none, less, or memory that is
+ * not 16-byte aligned reads the rows key by key.  The results are the same. */
+int64_t ash_map_find_rows_scratch_bytes(const ash_map_t* map, int64_t n, int n_values,
+                                        const int64_t* row_bytes, const int64_t* src_rows);
+int ash_map_find_rows_scratch(ash_map_t* map, const int32_t* keys, int64_t n, int n_values,
+                              const void* const* src, void* const* dst, const int64_t* row_bytes,
+                              const int64_t* src_rows, int zero_misses, int64_t* indices,
+                              uint8_t* masks, void* scratch, int64_t scratch_bytes, void* stream);
+
 /* The gradient of that look-up with respect to a table (autograd of
  * ash/embedding.py:38): out (out_rows x width, 16-byte aligned) is cleared and
  * rows[i] (width elements of `dtype`) is added to out[indices[i]] where

@@ -1,6 +1,8 @@
 """The look-up with rows (ash_map_find_rows) and its transpose (ash_add_rows)
 against torch's indexing on the indices that `find` returns: exact for the rows,
 to the rounding of a reordered sum for the gradient."""
+import ctypes
+
 import pytest
 import torch
 
@@ -124,3 +126,40 @@ def test_embedding_under_transforms_and_forward_mode(gpu_ash):
         dual = torch.autograd.forward_ad.make_dual(stack[0], stack[1])
         value, tangent = torch.autograd.forward_ad.unpack_dual(rows(dual))
     assert torch.equal(value, want[0]) and torch.equal(tangent, want[1])
+
+
+@pytest.mark.parametrize("dim,n,widths,alike", [
+    (3, 1 << 21, (3, 1), False), (3, (1 << 21) + 1, (1, 4, 3), False), (1, (1 << 21) + 4095, (5, 1, 1, 1), False),
+    (4, 2_500_001, (1, 4), False), (2, 1 << 21, (3, 3), True)])
+def test_rows_of_large_batches_in_index_order(gpu_ash, dim, n, widths, alike):
+    """Two million queries and more on two tables and more: rows are read in index
+    order, and equal those that batches below the limit get key by key."""
+    g = torch.Generator(device=DEV).manual_seed(dim)
+    stored = 1_200_000
+    keys = torch.randint(-(1 << 28 if dim == 1 else 9000), 1 << 28 if dim == 1 else 9000, (stored, dim), generator=g,
+                         device=DEV, dtype=torch.int32)
+    engine = gpu_ash.ASHEngine(dim, stored + 100_000, DEV)
+    engine.insert_keys(keys)
+    q = keys[torch.randint(stored, (n,), generator=g, device=DEV)]
+    q[torch.rand(n, generator=g, device=DEV) < 0.3, 0] += 1 << 20 if dim < 4 else 20_000
+    if alike:
+        q[:] = keys[7]
+    q[1, 0] = 1 << 29
+    rows = engine.capacity
+    # the last table ends before the stored indices do: zeros from there on
+    tables = [torch.randint(1 << 30, (rows - (300_000 if v == len(widths) - 1 else 0), w), generator=g, device=DEV,
+                            dtype=torch.int32) for v, w in enumerate(widths)]
+    row_bytes, src_rows = ((ctypes.c_int64 * len(widths))(*each) for each in
+                           ((4 * w for w in widths), (len(t) for t in tables)))
+    assert gpu_ash.common.load_library().ash_map_find_rows_scratch_bytes(
+        engine.backend._address, n, len(widths), row_bytes, src_rows) > 0
+    for zero_misses in (False, True):
+        got_i, got_m, got = gpu_ash.core.backend.find_rows(engine.backend, q, tables, zero_misses=zero_misses)
+        parts = [gpu_ash.core.backend.find_rows(engine.backend, p, tables, zero_misses=zero_misses)
+                 for p in q.split(500_000)]
+        assert torch.equal(got_i, torch.cat([p[0] for p in parts]))
+        assert torch.equal(got_m, torch.cat([p[1] for p in parts]))
+        for v, r in enumerate(got):
+            assert torch.equal(r, torch.cat([p[2][v] for p in parts]))
+    none, got_m, again = gpu_ash.core.backend.find_rows(engine.backend, q, tables, zero_misses=True, need_indices=False)
+    assert none is None and all(torch.equal(a, b) for a, b in zip(again, got))

@@ -243,6 +243,14 @@ _SIGNATURES = {
         [_PTR, _PTR, _I64, ctypes.c_int, ctypes.POINTER(_PTR), ctypes.POINTER(_PTR),
          ctypes.POINTER(_I64), ctypes.POINTER(_I64), ctypes.c_int, _PTR, _PTR, _PTR],
     ),
+    "ash_map_find_rows_scratch_bytes": (
+        _I64, [_PTR, _I64, ctypes.c_int, ctypes.POINTER(_I64), ctypes.POINTER(_I64)]
+    ),
+    "ash_map_find_rows_scratch": (
+        ctypes.c_int,
+        [_PTR, _PTR, _I64, ctypes.c_int, ctypes.POINTER(_PTR), ctypes.POINTER(_PTR),
+         ctypes.POINTER(_I64), ctypes.POINTER(_I64), ctypes.c_int, _PTR, _PTR, _PTR, _I64, _PTR],
+    ),
     "ash_add_rows": (
         ctypes.c_int,
         [_PTR, _PTR, _PTR, _I64, _I64, ctypes.c_int, _PTR, _I64, _PTR],

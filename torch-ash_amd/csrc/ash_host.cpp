@@ -34,7 +34,8 @@ namespace py = pybind11;
 #define ASH_FUNCTIONS(X)                                                              \
     X(ash_last_error)                                                                 \
     X(ash_map_find)                                                                   \
-    X(ash_map_find_rows)                                                              \
+    X(ash_map_find_rows_scratch_bytes)                                                \
+    X(ash_map_find_rows_scratch)                                                      \
     X(ash_add_rows)                                                                   \
     X(ash_gather_rows)                                                                \
     X(ash_map_insert_scratch_bytes)                                                   \
@@ -101,6 +102,16 @@ void* stream_of(int64_t device) {
 Tensor empty(at::IntArrayRef sizes, at::ScalarType type, int64_t device) {
     return at::empty(sizes, at::TensorOptions().dtype(type).device(
                                     at::kCUDA, static_cast<c10::DeviceIndex>(device)));
+}
+
+// Memory that a call can do without: none where the device has none left.
+Tensor scratch_if_there(int64_t bytes, int64_t device) {
+    if (bytes <= 0) return Tensor();
+    try {
+        return empty({bytes}, at::kByte, device);
+    } catch (const c10::OutOfMemoryError&) {
+        return Tensor();
+    }
 }
 
 template <typename T>
@@ -193,9 +204,13 @@ std::tuple<Tensor, Tensor, std::vector<Tensor>> find_rows(uintptr_t handle, int6
         bytes[v] = row_bytes_of(t);
         count[v] = t.size(0);
     }
-    check(lib.ash_map_find_rows(map_of(handle), ptr<int32_t>(keys), n, static_cast<int>(tables.size()),
-                                src, dst, bytes, count, zero_misses, ptr<int64_t>(indices),
-                                ptr<uint8_t>(masks), stream_of(device)));
+    const int n_tables = static_cast<int>(tables.size());
+    const Tensor scratch = scratch_if_there(
+            lib.ash_map_find_rows_scratch_bytes(map_of(handle), n, n_tables, bytes, count), device);
+    check(lib.ash_map_find_rows_scratch(map_of(handle), ptr<int32_t>(keys), n, n_tables, src, dst, bytes,
+                                        count, zero_misses, ptr<int64_t>(indices), ptr<uint8_t>(masks),
+                                        ptr<void>(scratch), scratch.defined() ? scratch.numel() : 0,
+                                        stream_of(device)));
     return {indices, masks, rows};
 }
 

@@ -1444,6 +1444,277 @@ __global__ __launch_bounds__(kBlock) void find_rows_kernel(
     }
 }
 
+// ------------------------------------- look-up with rows, rows in index order
+// find_rows_kernel asks for three random lines per key when two tables are read
+// (bucket, row, row), and the device delivers 50 - 58 G random lines a second
+// whatever part of a line is wanted and wherever behind the L2s it comes from (250
+// G where an L2 has them): 16 M keys with rows of 12 and 4 bytes take 942 us, of
+// which 600 are lines of rows.  Here the rows are read a part of the tables at a
+// time, which then sits in an L2:
+//   1. look-up; a chunk of kSortChunk queries is sorted by the part its indices
+//      lie in (in LDS) and leaves its indices in that order, the bounds of its
+//      parts and, for every query, its place in that order;
+//   2. per part: the indices that all chunks have left for it, their rows copied
+//      side by side to the indices' places (the workgroups of an XCD stand in
+//      one or two parts at a time, see gather_parts_kernel);
+//   3. per chunk: the rows, read through, dealt to the queries from LDS.
+// The look-up keeps its one random line per key; everything else streams: 2 + 4
+// bytes per key out, 4 + row in, row out, 2 + row in.  Chunks own their regions, so
+// there is nothing to count beforehand and nothing that can overflow, whatever the
+// indices are.  The same 16 M keys: 359 (of them 300 for the buckets' lines) + 275
+// + 99 us.  The second pass is bound by requests to the L2s, two per key; parts of
+// 1/128 and 1/512 of the tables: 278 and 299 us, of 1/64, more than an L2 holds, 324.
+constexpr int kSortThreads = 512;
+constexpr int kSortKeys = 8;                            // per thread
+constexpr int kSortChunk = kSortThreads * kSortKeys;
+constexpr int kSortParts = 256;
+static_assert(kSortParts % 8 == 0, "parts are dealt to eight XCDs");
+constexpr int kSortBounds = kSortParts + 2;
+// Records of a chunk and part that pass 2 takes; pass 3 reads the rows of further
+// ones itself, so that a wavefront's work is bounded when queries crowd in few
+// parts (8 M queries of one key: 719 us without the bound, 210 with it, 117 key by key)
+constexpr uint32_t kSortLongest = 256;
+constexpr int kSortMaxWords = 8;                        // of a query's rows, all tables together
+constexpr int kSortRuns = 8;                            // chunks per wavefront of pass 2
+constexpr int kSortAhead = 4;                           // groups of 64 records in flight there
+constexpr uint32_t kNoPlace = 0xFFFFu;
+
+struct RowSort {
+    int64_t n;
+    uint32_t chunks;
+    uint32_t scale;       // part of index i: umulhi(i, scale)
+    uint32_t words;       // of a query's rows
+    int32_t* index;       // chunks * kSortChunk, a chunk's in part order
+    uint16_t* place;      // n
+    uint16_t* bounds;     // chunks * kSortBounds: where a chunk's parts start, its end, and
+                          // whether a part of it is longer than kSortLongest
+    uint32_t* rows;       // chunks * kSortChunk * words
+};
+
+template <int DIM>
+__global__ __launch_bounds__(kSortThreads) void find_sort_kernel(
+        MapDev m, const int32_t* __restrict__ keys, RowSort sort, int64_t* __restrict__ idx_out,
+        uint8_t* __restrict__ mask_out) {
+    static_assert(kSortChunk <= 0xFFFF, "places and bounds are 16-bit words");
+    __shared__ int32_t s_index[kSortChunk];
+    __shared__ uint32_t s_where[kSortChunk];   // part << 16 | rank within the part
+    __shared__ int32_t s_count[kSortParts];
+    __shared__ int32_t s_first[kSortParts];
+    __shared__ int32_t s_wave[kSortThreads / 64];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int64_t base = static_cast<int64_t>(blockIdx.x) * kSortChunk;
+    static_assert(kSortParts <= kSortThreads, "a thread per part");
+    if (tid < kSortParts) s_count[tid] = 0;
+    __syncthreads();
+#pragma unroll 1
+    for (int j = 0; j < kSortKeys; ++j) {
+        const int64_t i = base + j * kSortThreads + tid;
+        const bool active = i < sort.n;
+        int32_t k[DIM];
+        load_key<DIM>(keys, i, active, k);
+        int32_t res = 0;
+        const bool found = find_key<DIM>(m, k, active, res);
+        if (active) {
+            if (idx_out != nullptr) idx_out[i] = found ? static_cast<int64_t>(res) : 0;
+            if (mask_out != nullptr) mask_out[i] = found ? 1 : 0;
+        }
+        uint32_t where = ~0u;
+        if (found) {
+            // (an index beyond every table reads zeros in pass 2, in whichever part)
+            uint32_t part = __umulhi(static_cast<uint32_t>(res), sort.scale);
+            if (part >= kSortParts) part = kSortParts - 1;
+            where = (part << 16) | static_cast<uint32_t>(atomicAdd(&s_count[part], 1));
+        }
+        s_index[j * kSortThreads + tid] = res;
+        s_where[j * kSortThreads + tid] = where;
+    }
+    __syncthreads();
+    const int count = tid < kSortParts ? s_count[tid] : 0;
+    int incl = count;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int up = __shfl_up(incl, d);
+        if (lane >= d) incl += up;
+    }
+    if (lane == 63) s_wave[tid >> 6] = incl;
+    int32_t res[kSortKeys];
+#pragma unroll
+    for (int j = 0; j < kSortKeys; ++j) res[j] = s_index[j * kSortThreads + tid];
+    __syncthreads();
+    int first = incl - count, total = 0;
+#pragma unroll
+    for (int w = 0; w < kSortThreads / 64; ++w) {
+        if (w < (tid >> 6)) first += s_wave[w];
+        total += s_wave[w];
+    }
+    uint16_t* bounds = sort.bounds + static_cast<int64_t>(blockIdx.x) * kSortBounds;
+    if (tid < kSortParts) {
+        s_first[tid] = first;
+        bounds[tid] = static_cast<uint16_t>(first);
+    }
+    const int longer = __syncthreads_or(count > static_cast<int>(kSortLongest));
+    if (tid == 0) {
+        bounds[kSortParts] = static_cast<uint16_t>(total);
+        bounds[kSortParts + 1] = longer ? 1 : 0;
+    }
+#pragma unroll
+    for (int j = 0; j < kSortKeys; ++j) {
+        const int64_t i = base + j * kSortThreads + tid;
+        const uint32_t where = s_where[j * kSortThreads + tid];
+        uint32_t place = kNoPlace;
+        if (where != ~0u) {
+            place = static_cast<uint32_t>(s_first[where >> 16]) + (where & 0xFFFFu);
+            s_index[place] = (where & 0xFFFFu) < kSortLongest ? res[j] : ~res[j];
+        }
+        if (i < sort.n) sort.place[i] = static_cast<uint16_t>(place);
+    }
+    __syncthreads();
+    for (int t = tid; t < total; t += kSortThreads) sort.index[base + t] = s_index[t];
+}
+
+// Pass 2: a wavefront copies the rows of one part for kSortRuns chunks (the first
+// kSortLongest of a chunk's).  Workgroups are dealt to the XCDs in turn, so
+// workgroup w serves the parts w mod 8 + 8 i, one after the other: what an XCD's
+// workgroups stand in at a time is one or two parts, 1 / 256 of the tables each.  A
+// lane copies one word of a row, always the same one, so that the words of a row are
+// asked for together and the rows leave as whole lines.
+template <int WORDS>
+__global__ __launch_bounds__(kBlock) void gather_parts_kernel(RowTables tabs, RowSort sort,
+                                                              uint32_t groups) {
+    constexpr uint32_t kWaves = kBlock / 64;
+    constexpr uint32_t kXcdCount = 8;
+    constexpr int kRecords = 64 / WORDS;                              // per step
+    constexpr int kSteps = (64 + kRecords - 1) / kRecords;            // for the records of 64 lanes
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t turn = blockIdx.x / kXcdCount;
+    const uint32_t part = turn / groups * kXcdCount + blockIdx.x % kXcdCount;
+    const uint32_t c0 = (turn % groups * kWaves + threadIdx.x / 64) * kSortRuns;
+    if (c0 >= sort.chunks) return;   // whole wavefronts
+    // lane r < kSortRuns: the run of chunk c0 + r
+    uint32_t from = 0, count = 0;
+    if (lane < kSortRuns && c0 + lane < sort.chunks) {
+        const uint16_t* b = sort.bounds + static_cast<int64_t>(c0 + lane) * kSortBounds + part;
+        from = b[0];
+        count = b[1] - from;
+        if (count > kSortLongest) count = kSortLongest;
+    }
+    uint32_t ends = count;
+#pragma unroll
+    for (int d = 1; d < kSortRuns; d <<= 1) {
+        const uint32_t up = __shfl_up(ends, d);
+        if (lane >= static_cast<uint32_t>(d)) ends += up;
+    }
+    // place of record t of run r: t + shift of r (modulo 2^32)
+    const uint32_t shift = (c0 + lane) * kSortChunk + from - (ends - count);
+    const uint32_t total = __shfl(ends, kSortRuns - 1);
+    if (total == 0) return;
+    // the lane's word: of which table, and where in its rows
+    const uint32_t record = lane / WORDS, word = lane % WORDS;
+    const uint32_t* column = nullptr;
+    uint32_t units = 0, rows = 0, before = 0;
+    for (int v = 0; v < tabs.n; ++v) {
+        if (word >= before) {
+            column = static_cast<const uint32_t*>(tabs.src[v]) + (word - before);
+            units = tabs.units[v];
+            rows = tabs.src_rows[v];
+        }
+        before += tabs.units[v];
+    }
+    for (uint32_t t0 = 0; t0 < total; t0 += 64 * kSortAhead) {
+        uint32_t at[kSortAhead], index[kSortAhead];
+#pragma unroll
+        for (int a = 0; a < kSortAhead; ++a) {
+            const uint32_t t = t0 + a * 64 + lane;
+            uint32_t run = 0;
+#pragma unroll
+            for (int r = 0; r < kSortRuns - 1; ++r) {
+                run += t >= static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(ends), r)) ? 1u : 0u;
+            }
+            at[a] = t + static_cast<uint32_t>(__shfl(static_cast<int>(shift), static_cast<int>(run)));
+            index[a] = t < total ? static_cast<uint32_t>(sort.index[at[a]]) : 0u;
+        }
+        uint32_t w[kSortAhead][kSteps];
+#pragma unroll
+        for (int a = 0; a < kSortAhead; ++a) {
+#pragma unroll
+            for (int st = 0; st < kSteps; ++st) {
+                const uint32_t rec = st * kRecords + record;
+                const uint32_t i = __shfl(index[a], static_cast<int>(rec & 63u));
+                w[a][st] = 0u;
+                if (record < kRecords && rec < 64 && t0 + a * 64 + rec < total && i < rows) {
+                    w[a][st] = column[static_cast<size_t>(i) * units];
+                }
+            }
+        }
+#pragma unroll
+        for (int a = 0; a < kSortAhead; ++a) {
+#pragma unroll
+            for (int st = 0; st < kSteps; ++st) {
+                const uint32_t rec = st * kRecords + record;
+                const uint32_t to = __shfl(at[a], static_cast<int>(rec & 63u));
+                if (record < kRecords && rec < 64 && t0 + a * 64 + rec < total) {
+                    sort.rows[static_cast<size_t>(to) * WORDS + word] = w[a][st];
+                }
+            }
+        }
+    }
+}
+
+// Pass 3: a chunk's rows to its queries.
+constexpr int kDealThreads = 1024;
+
+__global__ __launch_bounds__(kDealThreads) void deal_rows_kernel(RowTables tabs, RowSort sort, int miss_row) {
+    extern __shared__ __align__(16) uint32_t s_rows[];   // kSortChunk * words, and the places
+    uint16_t* s_place = reinterpret_cast<uint16_t*>(s_rows + kSortChunk * sort.words);
+    const int64_t base = static_cast<int64_t>(blockIdx.x) * kSortChunk;
+    const uint32_t queries = sort.n - base < kSortChunk ? static_cast<uint32_t>(sort.n - base) : kSortChunk;
+    const uint16_t* bounds = sort.bounds + static_cast<int64_t>(blockIdx.x) * kSortBounds;
+    const uint32_t found = bounds[kSortParts], total = found * sort.words;
+    const uint32_t* rows = sort.rows + static_cast<size_t>(base) * sort.words;
+    // (whole pieces: a chunk's region is kSortChunk rows long)
+    for (uint32_t t = threadIdx.x; t < (total + 3) / 4; t += kDealThreads) {
+        reinterpret_cast<uint4*>(s_rows)[t] = reinterpret_cast<const uint4*>(rows)[t];
+    }
+    for (uint32_t t = threadIdx.x; t < queries; t += kDealThreads) s_place[t] = sort.place[base + t];
+    __syncthreads();
+    if (bounds[kSortParts + 1] != 0) {
+        // rows that pass 2 has left: queries that crowd in few parts, and so in the caches
+        for (uint32_t t = threadIdx.x; t < found; t += kDealThreads) {
+            const int32_t kept = sort.index[base + t];
+            if (kept >= 0) continue;
+            const uint32_t index = static_cast<uint32_t>(~kept);
+            uint32_t* row = s_rows + t * sort.words;
+            for (int v = 0; v < tabs.n; ++v) {
+                const uint32_t units = tabs.units[v];
+                const uint32_t* src = static_cast<const uint32_t*>(tabs.src[v]) + static_cast<size_t>(index) * units;
+                for (uint32_t u = 0; u < units; ++u) row[u] = index < tabs.src_rows[v] ? src[u] : 0u;
+                row += units;
+            }
+        }
+        __syncthreads();
+    }
+    uint32_t column = 0;
+    for (int v = 0; v < tabs.n; ++v) {
+        const uint32_t units = tabs.units[v], magic = tabs.magic[v];
+        uint32_t* out = static_cast<uint32_t*>(tabs.dst[v]) + static_cast<size_t>(base) * units;
+        const bool miss_reads = miss_row >= 0 && static_cast<uint32_t>(miss_row) < tabs.src_rows[v];
+        for (uint32_t t = threadIdx.x; t < queries * units; t += kDealThreads) {
+            const uint32_t q = units == 1 ? t : __umulhi(t, magic);
+            const uint32_t word = t - q * units;
+            const uint32_t place = s_place[q];
+            uint32_t w = 0u;
+            if (place != kNoPlace) {
+                w = s_rows[place * sort.words + column + word];
+            } else if (miss_reads) {
+                w = static_cast<const uint32_t*>(tabs.src[v])[static_cast<size_t>(miss_row) * units + word];
+            }
+            __builtin_nontemporal_store(w, out + t);
+        }
+        column += units;
+    }
+}
+
 // 16 bytes per thread, the words of a shorter tail one by one.
 __global__ __launch_bounds__(kBlock) void clear_rows_kernel(uint32_t* __restrict__ p, int64_t words) {
     const int64_t t = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) * 4;
@@ -2011,6 +2282,92 @@ int insert_selected(ash_map* map, bool codes, const void* keys,
     return launch_selected<kInsertKeys>(map, codes, k, sel, nsel, va, s, publish);
 }
 
+namespace {
+
+// When the rows are read in index order, and what that takes.  Measured (keys
+// found, key by key -> in index order, us):
+//   two tables or more; of one (rows of 12 bytes) the passes cost what its lines do
+//   2 M queries and more: rows of 12 + 4 bytes, 1.5 M rows: 1 M queries 46 -> 58,
+//     2 M 90 -> 81, 4 M 183 -> 151, 8 M 374 -> 280
+//   a quarter of the tables' rows and more, fewer share no lines in a part: 12 M
+//     rows: 2 M queries 118 -> 117, 4 M 234 -> 217, 8 M 467 -> 366; 24 M rows: 4 M
+//     236 -> 238, 8 M 471 -> 399, 16 M 942 -> 734
+//   16 MB of tables: 6 MB (of which an XCD's L2 holds most) and 4 M queries 111 ->
+//     123, 12 MB 200 -> 173
+//   rows of up to kSortMaxWords words together: a chunk's have to fit the LDS.
+constexpr int64_t kSortMinQueries = int64_t{1} << 21;
+constexpr int64_t kSortMinBytes = int64_t{16} << 20;
+
+int64_t plan_row_sort(int64_t n, int n_values, const int64_t* row_bytes, const int64_t* src_rows,
+                      void* scratch, RowSort* sort) {
+    if (n < kSortMinQueries || n > 0x7FFF0000ll || n_values < 2 || n_values > kMaxFusedValues) return 0;
+    int64_t words = 0, rows = 0, table_bytes = 0;
+    for (int v = 0; v < n_values; ++v) {
+        if (row_bytes[v] <= 0 || row_bytes[v] % 4 != 0 || src_rows[v] < 0 || src_rows[v] > 0x7FFFFFFFll) return 0;
+        if (row_bytes[v] > 4 * kSortMaxWords) return 0;
+        words += row_bytes[v] / 4;
+        rows = std::max(rows, src_rows[v]);
+        table_bytes += row_bytes[v] * src_rows[v];
+    }
+    if (words > kSortMaxWords || rows <= kSortParts || n < rows / 4 || table_bytes < kSortMinBytes) return 0;
+    const int64_t chunks = (n + kSortChunk - 1) / kSortChunk;
+    int64_t off = 0;
+    auto take = [&](int64_t bytes) {
+        char* p = scratch != nullptr ? static_cast<char*>(scratch) + off : nullptr;
+        off += (bytes + 255) & ~int64_t{255};
+        return p;
+    };
+    void* index = take(chunks * kSortChunk * 4);
+    void* place = take(n * 2);
+    void* bounds = take(chunks * kSortBounds * 2);
+    void* out = take(chunks * kSortChunk * words * 4);
+    if (sort != nullptr) {
+        *sort = {n, static_cast<uint32_t>(chunks),
+                 static_cast<uint32_t>((static_cast<uint64_t>(kSortParts) << 32) / static_cast<uint64_t>(rows)),
+                 static_cast<uint32_t>(words), static_cast<int32_t*>(index), static_cast<uint16_t*>(place),
+                 static_cast<uint16_t*>(bounds), static_cast<uint32_t*>(out)};
+    }
+    return off;
+}
+
+int find_rows_sorted(ash_map* map, const int32_t* keys, RowTables tabs, const RowSort& sort, int miss,
+                     int64_t* indices, uint8_t* masks, hipStream_t s) {
+    // the passes address rows by words
+    for (int v = 0; v < tabs.n; ++v) {
+        if ((tabs.wide >> v) & 1u) tabs.units[v] *= 4;
+        tabs.magic[v] = static_cast<uint32_t>((0x100000000ull + tabs.units[v] - 1) / tabs.units[v]);
+    }
+    tabs.wide = 0;
+    switch (map->key_dim) {
+        case 1: find_sort_kernel<1><<<sort.chunks, kSortThreads, 0, s>>>(map->d, keys, sort, indices, masks); break;
+        case 2: find_sort_kernel<2><<<sort.chunks, kSortThreads, 0, s>>>(map->d, keys, sort, indices, masks); break;
+        case 3: find_sort_kernel<3><<<sort.chunks, kSortThreads, 0, s>>>(map->d, keys, sort, indices, masks); break;
+        default: find_sort_kernel<4><<<sort.chunks, kSortThreads, 0, s>>>(map->d, keys, sort, indices, masks); break;
+    }
+    ASH_LAUNCH_CHECK();
+    constexpr uint32_t kRunsPerGroup = kSortRuns * (kBlock / 64);
+    const uint32_t groups = (sort.chunks + kRunsPerGroup - 1) / kRunsPerGroup;
+    const unsigned g = groups * kSortParts;
+    switch (sort.words) {
+        case 2: gather_parts_kernel<2><<<g, kBlock, 0, s>>>(tabs, sort, groups); break;
+        case 3: gather_parts_kernel<3><<<g, kBlock, 0, s>>>(tabs, sort, groups); break;
+        case 4: gather_parts_kernel<4><<<g, kBlock, 0, s>>>(tabs, sort, groups); break;
+        case 5: gather_parts_kernel<5><<<g, kBlock, 0, s>>>(tabs, sort, groups); break;
+        case 6: gather_parts_kernel<6><<<g, kBlock, 0, s>>>(tabs, sort, groups); break;
+        case 7: gather_parts_kernel<7><<<g, kBlock, 0, s>>>(tabs, sort, groups); break;
+        default: gather_parts_kernel<8><<<g, kBlock, 0, s>>>(tabs, sort, groups); break;
+    }
+    ASH_LAUNCH_CHECK();
+    const size_t lds = static_cast<size_t>(kSortChunk) * (sort.words * 4 + 2);
+    ASH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(deal_rows_kernel),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+    deal_rows_kernel<<<sort.chunks, kDealThreads, lds, s>>>(tabs, sort, miss);
+    ASH_LAUNCH_CHECK();
+    return 0;
+}
+
+}  // namespace
+
 }  // namespace ash
 
 using namespace ash;
@@ -2168,6 +2525,20 @@ int ash_map_find_rows(ash_map_t* map, const int32_t* keys, int64_t n, int n_valu
                       const void* const* src, void* const* dst, const int64_t* row_bytes,
                       const int64_t* src_rows, int zero_misses, int64_t* indices,
                       uint8_t* masks, void* stream) {
+    return ash_map_find_rows_scratch(map, keys, n, n_values, src, dst, row_bytes, src_rows, zero_misses,
+                                     indices, masks, nullptr, 0, stream);
+}
+
+int64_t ash_map_find_rows_scratch_bytes(const ash_map_t* map, int64_t n, int n_values,
+                                        const int64_t* row_bytes, const int64_t* src_rows) {
+    if (map == nullptr || row_bytes == nullptr || src_rows == nullptr) return 0;
+    return plan_row_sort(n, n_values, row_bytes, src_rows, nullptr, nullptr);
+}
+
+int ash_map_find_rows_scratch(ash_map_t* map, const int32_t* keys, int64_t n, int n_values,
+                              const void* const* src, void* const* dst, const int64_t* row_bytes,
+                              const int64_t* src_rows, int zero_misses, int64_t* indices,
+                              uint8_t* masks, void* scratch, int64_t scratch_bytes, void* stream) {
     if (check_batch(map, keys, n)) return 1;
     if (n_values < 0 || n_values > kMaxFusedValues) {
         ASH_FAIL("find_rows takes up to " + std::to_string(kMaxFusedValues) + " tensors per call");
@@ -2199,8 +2570,15 @@ int ash_map_find_rows(ash_map_t* map, const int32_t* keys, int64_t n, int n_valu
     ASH_HIP(guard.enter(map->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (settle_table(map, s)) return 1;
-    const unsigned g = grid_for(n);
     const int miss = zero_misses ? -1 : 0;
+    if (scratch != nullptr && reinterpret_cast<uintptr_t>(scratch) % 16 == 0) {
+        RowSort sort;
+        const int64_t need = plan_row_sort(n, n_values, row_bytes, src_rows, scratch, &sort);
+        if (need > 0 && scratch_bytes >= need) {
+            return find_rows_sorted(map, keys, tabs, sort, miss, indices, masks, s);
+        }
+    }
+    const unsigned g = grid_for(n);
     switch (map->key_dim) {
         case 1:
             find_rows_kernel<1><<<g, kBlock, 0, s>>>(map->d, keys, n, tabs, miss, indices, masks);

@@ -686,6 +686,16 @@ int ash_query_backward_backward_accumulate(const ash_query_args* a,
                                            void* grad_z, void* grad_embeddings,
                                            void* stream);
 
+/* ash_query_backward_forward(a, z, grad_embeddings, grad_offsets) and, in the same
+ * pass over the queries, the grad_embeddings of ash_query_backward_backward(a,
+ * grad_grad_offsets, z_second): one gradient that holds the sum of the two (a
+ * training step with a value loss and a gradient-norm loss).  grad_embeddings
+ * must not be NULL and is zero-filled here unless `accumulate`; grad_offsets may
+ * be NULL. */
+int ash_query_backward_both(const ash_query_args* a, const void* z, const void* grad_grad_offsets,
+                            const void* z_second, void* grad_embeddings, void* grad_offsets,
+                            int32_t accumulate, void* stream);
+
 /* Replaces `convolution_forward` (ash/src/grid.cu:948-1043, pybind.cpp:33).
  * inputs / outputs scalar[num_embeddings, cells_per_grid, embedding_dim];
  * weights scalar[num_cell_nbs, embedding_dim] (one weight per window tap and

@@ -1,0 +1,185 @@
+"""The embedding gradients of the first- and the second-order backward in one
+pass over the queries: the kernels against the oracle, and the passes of the
+engine in which the second-order node may and may not leave its share to the
+forward node."""
+import threading
+
+import pytest
+import torch
+
+import workloads
+from helpers import assert_close_sums
+from test_gpu_query import _eps, _make_grid, _operands, _queries, _to_cpu, _tol
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+# 600 001 queries: tables of cells in LDS; blocks of 4^3 also the wide workgroups
+@pytest.mark.parametrize("dtype,grid_dim,width,n", [
+    (dtype, 4, width, n) for dtype in (torch.float32, torch.float64) for width in (1, 2, 3, 4, 5, 8, 16)
+    for n in (1, 257)] + [(torch.float32, 4, 4, 600_001), (torch.float32, 8, 4, 600_001),
+                          (torch.float32, 11, 4, 600_001), (torch.float32, 4, 5, 600_001),
+                          (torch.float64, 4, 3, 600_001)])
+@pytest.mark.parametrize("need_offsets", [True, False])
+def test_both_orders_against_the_oracle(gpu_ash, oracle, dtype, grid_dim, width, n, need_offsets):
+    grid = _make_grid(gpu_ash, grid_dim, width, 1, dtype=dtype, seed=width, holes=2)
+    ops = _operands(grid, _queries(grid_dim, 1, n, seed=n, margin=1.0))
+    g = torch.Generator().manual_seed(n)
+    z, u, z2 = ((torch.rand(n, w, generator=g, dtype=dtype) - 0.5).to(DEV) for w in (width, 3, width))
+    start = (torch.rand(ops[0].shape, generator=g, dtype=dtype) - 0.5).to(DEV)
+    host = gpu_ash.grid_query.backend.host
+    cpu = _to_cpu(ops)
+    want, want_off = oracle.query_backward_forward(z.cpu(), *cpu, grid_dim, "smooth_step")
+    want = want + oracle.query_backward_backward(None, u.cpu(), z2.cpu(), *cpu, grid_dim, "smooth_step")[1]
+    sums = (oracle.query_term_sums(u, z, *cpu, grid_dim, "smooth_step")["bf_embeddings"]
+            + oracle.query_term_sums(u, z2, *cpu, grid_dim, "smooth_step")["bb_embeddings"])
+    bound = dict(eps=_eps(dtype), **_tol(dtype))
+    got, got_off = host.query_backward_both(z, u, z2, list(ops), "smooth_step", need_offsets, None)
+    assert_close_sums(got, want, sums, what="zeroed", **bound)
+    acc, _ = host.query_backward_both(z, u, z2, list(ops), "smooth_step", need_offsets, start)
+    assert acc.data_ptr() == start.data_ptr()
+    began = acc.cpu().double() - got.cpu().double()   # what was there, up to the same rounding
+    g = torch.Generator().manual_seed(n)
+    for w in (width, 3, width):
+        torch.rand(n, w, generator=g, dtype=dtype)
+    first = torch.rand(ops[0].shape, generator=g, dtype=dtype) - 0.5
+    assert_close_sums(began, first, 2 * sums + 2 * first.double().abs(), what="added", **bound)
+    if need_offsets:
+        assert torch.allclose(got_off.cpu(), want_off, **_tol(dtype))
+    else:
+        assert got_off is None
+
+
+def test_rows_of_four_off_their_alignment(gpu_ash):
+    """z of the second order at an address that is no multiple of 16."""
+    grid = _make_grid(gpu_ash, 4, 4, 1, seed=3)
+    ops = _operands(grid, _queries(4, 1, 1000, seed=4))
+    z, u = torch.rand(1000, 4, device=DEV), torch.rand(1000, 3, device=DEV)
+    z2 = torch.rand(4001, device=DEV)[1:].view(1000, 4)
+    host = gpu_ash.grid_query.backend.host
+    got, _ = host.query_backward_both(z, u, z2, list(ops), "linear", False, None)
+    want, _ = host.query_backward_both(z, u, z2.clone(), list(ops), "linear", False, None)
+    assert torch.allclose(got, want, rtol=1e-5, atol=1e-5)
+
+
+class _Fails(torch.autograd.Function):
+    armed = False
+
+    @staticmethod
+    def forward(ctx, y):
+        return y.clone()
+
+    @staticmethod
+    def backward(ctx, z):
+        if _Fails.armed:
+            raise ValueError("on purpose")
+        return z
+
+
+@pytest.fixture()
+def scene(gpu_ash, monkeypatch):
+    grid, radii, centres = workloads.build_grid(gpu_ash, 300, 4, sparse_grid_dim=32, device=DEV)
+    x = workloads.ray_queries(grid, radii, centres, num_rays=64, samples_per_ray=30)
+    backend = gpu_ash.grid_query.backend
+    put_off, real = [], backend.query_backward_backward
+    monkeypatch.setattr(backend, "query_backward_backward",
+                        lambda *a, **k: (put_off.append(k.get("later", False)), real(*a, **k))[1], raising=False)
+    return gpu_ash, grid, x, put_off
+
+
+def _grad(grid, loss, **how):
+    grid.embeddings.grad = None
+    loss.backward(**how)
+    return grid.embeddings.grad.clone()
+
+
+def _close(got, want):
+    return torch.allclose(got, want, rtol=1e-4, atol=1e-6 * float(want.abs().max()))
+
+
+def _norm_loss(y, xq, channel):
+    (gx,) = torch.autograd.grad(y[:, channel].sum(), xq, create_graph=True)
+    return (gx.norm(dim=-1) - 1).abs().mean()
+
+
+def _separately(grid, x, channels):
+    total = 0
+    for what in ("value", *channels):
+        xq = x.clone().requires_grad_(True)
+        y, _ = grid(xq, "smooth_step")
+        total = total + _grad(grid, (y**2).mean() if what == "value" else _norm_loss(y, xq, what))
+    return total
+
+
+def test_several_second_order_nodes_of_one_forward(scene):
+    ash, grid, x, put_off = scene
+    want = _separately(grid, x, (0, 2, 3))
+    for inside in (False, True):
+        del put_off[:]
+        xq = x.clone().requires_grad_(True)
+        y, _ = grid(xq, "smooth_step")
+        loss = (y**2).mean() + sum(_norm_loss(y, xq, c) for c in (0, 2, 3))
+        grid.embeddings.grad = None
+        if inside:
+            with ash.dense_grad(grid):
+                loss.backward()
+        else:
+            loss.backward()
+        assert put_off == [True] * 3 and _close(grid.embeddings.grad, want)
+
+
+def test_a_pass_that_fails_in_between_leaves_nothing_behind(scene):
+    ash, grid, x, put_off = scene
+    want = _separately(grid, x, (0,))
+    xq = x.clone().requires_grad_(True)
+    y, _ = grid(xq, "smooth_step")
+    # nodes are run latest first, as each thread counts them: recorded in a thread
+    # of its own, this one is run after the second-order node
+    value = []
+    thread = threading.Thread(target=lambda: value.append((_Fails.apply(y)**2).mean()))
+    thread.start()
+    thread.join()
+    loss = value[0] + _norm_loss(y, xq, 0)
+    _Fails.armed = True
+    del put_off[:]
+    try:
+        with pytest.raises(ValueError, match="on purpose"):
+            loss.backward(retain_graph=True)
+    finally:
+        _Fails.armed = False
+    assert put_off == [True]
+    assert _close(_grad(grid, loss, retain_graph=True), want) and _close(_grad(grid, loss), want)
+
+
+def test_gradients_that_somebody_sees_are_whole(scene):
+    ash, grid, x, put_off = scene
+    xq = x.clone().requires_grad_(True)
+    y, _ = grid(xq, "smooth_step")
+    second = _grad(grid, _norm_loss(y, xq, 0))
+    xq = x.clone().requires_grad_(True)
+    y, _ = grid(xq, "smooth_step")
+    seen = []
+    y.grad_fn.register_prehook(lambda grads: seen.extend(g.clone() for g in grads
+                                                         if g is not None and g.shape == second.shape))
+    loss = (y**2).mean() + _norm_loss(y, xq, 0)
+    del put_off[:]
+    total = _grad(grid, loss)
+    assert put_off == [False] and len(seen) == 1 and _close(seen[0], second)
+    assert _close(total, _separately(grid, x, (0,)))
+
+
+def test_a_gradient_recorded_under_another_stream(scene):
+    ash, grid, x, put_off = scene
+    want = _separately(grid, x, (0,))
+    xq = x.clone().requires_grad_(True)
+    y, _ = grid(xq, "smooth_step")
+    value = (y**2).mean()
+    other = torch.cuda.Stream()
+    other.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(other):
+        norm = _norm_loss(y, xq, 0)
+    torch.cuda.current_stream().wait_stream(other)
+    del put_off[:]
+    # (recorded on the forward's stream all the same)
+    assert _close(_grad(grid, value + norm), want) and put_off == [True]

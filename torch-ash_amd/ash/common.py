@@ -305,6 +305,10 @@ _SIGNATURES = {
         ctypes.c_int,
         [ctypes.POINTER(_QueryArgs), _PTR, _PTR, _PTR, _PTR],
     ),
+    "ash_query_backward_both": (
+        ctypes.c_int,
+        [ctypes.POINTER(_QueryArgs)] + [_PTR] * 5 + [ctypes.c_int32, _PTR],
+    ),
     "ash_query_backward_backward_accumulate": (
         ctypes.c_int,
         [ctypes.POINTER(_QueryArgs), _PTR, _PTR, _PTR, _PTR, _PTR],
@@ -936,23 +940,39 @@ class _Backend:
         need_embeddings: bool = True,
         need_offsets: bool = True,
         accumulate_into: Optional[torch.Tensor] = None,
+        along=(),
     ) -> Tuple[Optional[torch.Tensor], Optional[torch.Tensor]]:
         """(grad_embeddings, grad_offsets); an output that is not needed is
         None and its work (for grad_embeddings: dense zero fill + atomics) is
         skipped.  With `accumulate_into` (a gradient of the embeddings' shape
         that already holds other contributions) the embedding gradient is added
-        to that tensor, which is also what is returned."""
-        return self.host.query_backward_forward(
-            z, [embeddings, offsets, grid_indices, cell_indices, masks, lut_grid_nb2grid_idx,
-                lut_cell_nb2cell_idx, lut_cell_nb2grid_nb], interpolation, need_embeddings,
-            need_offsets, accumulate_into)
+        to that tensor, which is also what is returned.  `along`: what
+        query_backward_backward has put off for the same queries, pairs
+        (grad_grad_offsets, z), taken along in grad_embeddings -- the first pair
+        in the same pass over the queries."""
+        operands = [embeddings, offsets, grid_indices, cell_indices, masks, lut_grid_nb2grid_idx,
+                    lut_cell_nb2cell_idx, lut_cell_nb2grid_nb]
+        if not along:
+            return self.host.query_backward_forward(
+                z, operands, interpolation, need_embeddings, need_offsets, accumulate_into)
+        grad_embeddings, grad_offsets = self.host.query_backward_both(
+            z, *along[0], operands, interpolation, need_offsets, accumulate_into)
+        for pair in along[1:]:
+            self.host.query_backward_backward(*pair, operands, interpolation, False, True, grad_embeddings)
+        return grad_embeddings, grad_offsets
 
-    def query_backward_forward_onto(self, grad_embeddings, z, *operands, need_offsets: bool = True):
+    def query_backward_forward_onto(self, grad_embeddings, z, *operands, need_offsets: bool = True, **along):
         """query_backward_forward whose embedding gradient is added to
         `grad_embeddings`, a tensor that no one else holds; returns
         grad_offsets."""
         return _Backend.query_backward_forward(self, z, *operands, need_offsets=need_offsets,
-                                               accumulate_into=grad_embeddings)[1]
+                                               accumulate_into=grad_embeddings, **along)[1]
+
+    def query_backward_backward_onto(self, grad_embeddings, grad_grad_offsets, z, *operands) -> None:
+        """query_backward_backward with no other result than an embedding
+        gradient added to `grad_embeddings`."""
+        _Backend.query_backward_backward(self, None, grad_grad_offsets, z, *operands, need_z=False,
+                                         accumulate_into=grad_embeddings, need_offsets=False)
 
     def query_backward_backward(
         self,
@@ -973,15 +993,22 @@ class _Backend:
         need_embeddings: bool = True,
         accumulate_into: Optional[torch.Tensor] = None,
         need_offsets: bool = True,
+        later: bool = False,
     ) -> Tuple[Optional[torch.Tensor], Optional[torch.Tensor], Optional[torch.Tensor]]:
         """(grad_z, grad_embeddings, zero grad_offsets); outputs that are not
         needed are None and their work is skipped.  `accumulate_into` as for
-        query_backward_forward."""
-        grad_z, grad_embeddings = self.host.query_backward_backward(
-            grad_grad_offsets, z,
-            [embeddings, offsets, grid_indices, cell_indices, masks, lut_grid_nb2grid_idx,
-             lut_cell_nb2cell_idx, lut_cell_nb2grid_nb], interpolation, need_z, need_embeddings,
-            accumulate_into)
+        query_backward_forward.  `later`: grad_embeddings comes without the
+        contributions of this call (zeros, or `accumulate_into` as it is); the
+        caller has query_backward_forward or query_backward_backward_onto add
+        them.  There is no grad_z then."""
+        operands = [embeddings, offsets, grid_indices, cell_indices, masks, lut_grid_nb2grid_idx,
+                    lut_cell_nb2cell_idx, lut_cell_nb2grid_nb]
+        if later:
+            grad_z, grad_embeddings = None, self.host.query_gradient_later(
+                grad_grad_offsets, z, operands, interpolation, accumulate_into)
+        else:
+            grad_z, grad_embeddings = self.host.query_backward_backward(
+                grad_grad_offsets, z, operands, interpolation, need_z, need_embeddings, accumulate_into)
         # the offsets second-order term is not produced (ash/src/grid.cu:417-418)
         zeros = embeddings.new_zeros(grid_indices.shape[0], 3) if need_offsets else None
         return grad_z, grad_embeddings, zeros

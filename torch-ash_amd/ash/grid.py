@@ -95,6 +95,7 @@ class _FusedGridForward(torch.autograd.Function):
         ctx.cell_size = cell_size
         ctx.spent = False
         ctx.outliving = None
+        ctx.later = grid_query._Later() if hasattr(backend, "query_backward_backward_onto") else None
         ctx.mark_non_differentiable(masks)
         ctx.set_materialize_grads(False)
         return features, masks, again
@@ -103,6 +104,9 @@ class _FusedGridForward(torch.autograd.Function):
     def backward(ctx, z, _grad_masks, carried):
         last = not torch._C._autograd._get_current_graph_task_keep_graph()
         if z is None:   # only the gradient of the gradient was asked for
+            parts = ctx.later.take() if ctx.later is not None else ()
+            if parts:
+                carried = grid_query.add_put_off(parts, carried, ctx.grid_dim, ctx.interpolation)
             if last and not ctx.spent and ctx.outliving is None:
                 _FusedGridForward._outlive(ctx)
             return (carried,) + (None,) * 9
@@ -115,7 +119,8 @@ class _FusedGridForward(torch.autograd.Function):
             if [t._version for t in operands] != versions:
                 raise RuntimeError("one of the variables needed for gradient computation has been "
                                    "modified by an inplace operation since an earlier pass")
-        grad_embeddings, grad_x = first_order_backward(ctx, z, operands, 0, 1, again, carried)
+        grad_embeddings, grad_x = first_order_backward(ctx, z, operands, 0, 1, again, carried,
+                                                        ctx.later)
         if last:
             ctx.spent, ctx.outliving = True, None
         if grad_x is not None and ctx.cell_size != 1.0:

@@ -10,6 +10,7 @@
 #include <torch/extension.h>
 
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_function.h>
 
 #include <dlfcn.h>
 
@@ -60,6 +61,7 @@ namespace py = pybind11;
     X(ash_query_forward)                                                              \
     X(ash_query_backward_forward)                                                     \
     X(ash_query_backward_forward_accumulate)                                          \
+    X(ash_query_backward_both)                                                        \
     X(ash_query_backward_backward)                                                    \
     X(ash_query_backward_backward_accumulate)
 
@@ -785,6 +787,22 @@ std::tuple<Optional, Optional> query_backward_forward(const Tensor& z_in, const 
     return {maybe(grad), maybe(offsets)};
 }
 
+std::tuple<Tensor, Optional> query_backward_both(const Tensor& z_in, const Tensor& gg_in,
+                                                 const Tensor& z_second_in,
+                                                 const std::vector<Tensor>& operands,
+                                                 const std::string& interpolation, bool need_offsets,
+                                                 const Optional& accumulate_into) {
+    Operands q(operands, interpolation);
+    const Tensor z = q.like(z_in, q.e, "z"), gg = q.like(gg_in, 3, "grad_grad_offsets");
+    const Tensor z_second = q.like(z_second_in, q.e, "z of the second order");
+    const Tensor grad = q.gradient(accumulate_into, true);
+    const Tensor offsets = need_offsets ? q.output(3) : Tensor();
+    check(lib.ash_query_backward_both(&q.args, z.data_ptr(), gg.data_ptr(), z_second.data_ptr(),
+                                      grad.data_ptr(), ptr<void>(offsets), accumulate_into.has_value(),
+                                      stream_of(q.device)));
+    return {grad, maybe(offsets)};
+}
+
 std::tuple<Optional, Optional> query_backward_backward(const Tensor& gg_in, const Tensor& z_in,
                                                        const std::vector<Tensor>& operands,
                                                        const std::string& interpolation, bool need_z,
@@ -799,6 +817,33 @@ std::tuple<Optional, Optional> query_backward_backward(const Tensor& gg_in, cons
     check(entry(&q.args, gg.data_ptr(), z.data_ptr(), ptr<void>(grad_z), ptr<void>(grad),
                 stream_of(q.device)));
     return {maybe(grad_z), maybe(grad)};
+}
+
+// The embedding gradient of a query_backward_backward whose contributions are
+// still to come (query_backward_both): `accumulate_into`, or zeros.  Everything is
+// checked here, where the call is made.
+Tensor query_gradient_later(const Tensor& gg_in, const Tensor& z_in, const std::vector<Tensor>& operands,
+                            const std::string& interpolation, const Optional& accumulate_into) {
+    Operands q(operands, interpolation);
+    q.like(z_in, q.e, "z");
+    q.like(gg_in, 3, "grad_grad_offsets");
+    const Tensor grad = q.gradient(accumulate_into, true);
+    if (!accumulate_into.has_value()) {
+        q.args.num_queries = 0;   // nothing but the zeros
+        check(lib.ash_query_backward_forward(&q.args, nullptr, grad.data_ptr(), nullptr, stream_of(q.device)));
+    }
+    return grad;
+}
+
+// Whether nobody looks at the gradient that the node of `ctx` hands to the node
+// behind its input `input`: no hook behind the one or before the other.
+bool hands_over_unseen(const py::object& ctx, size_t input) {
+    if (!THPFunction_Check(ctx.ptr())) return false;
+    const auto node = reinterpret_cast<THPFunction*>(ctx.ptr())->cdata.lock();
+    if (!node || input >= node->num_outputs() || !node->post_hooks().empty()) return false;
+    const auto& next = node->next_edge(input).function;
+    return next && next->pre_hooks().empty() && next->tensor_pre_hooks().empty() &&
+           next->retains_grad_hooks().empty();
 }
 
 std::tuple<Optional, Tensor, std::vector<Tensor>> find_rows_py(uintptr_t handle, int64_t dim, int64_t device,
@@ -834,5 +879,8 @@ PYBIND11_MODULE(_ash_host, m) {
     m.def("surface_mesh", &surface_mesh);
     m.def("query_forward", &query_forward);
     m.def("query_backward_forward", &query_backward_forward);
+    m.def("query_backward_both", &query_backward_both);
+    m.def("query_gradient_later", &query_gradient_later);
+    m.def("hands_over_unseen", &hands_over_unseen);
     m.def("query_backward_backward", &query_backward_backward);
 }

@@ -56,14 +56,15 @@ constexpr int kLdsPerCu = 160 * 1024;
 // 0.93 - 1.08 of the time, 1.00 on average over rows of 1 to 16.
 constexpr int kWavesFull = 8;
 constexpr int kWavesWide = 7;
+constexpr int kWavesBoth = 6;   // positions' gradient and both orders' of the rows: 60 - 78 registers
 constexpr int kWavesBackward = 3;
 constexpr int forward_waves(int vec, int lpq) {
     return vec > 4 || (vec == 4 && lpq > 2) ? kWavesWide : kWavesFull;
 }
 template <typename T>
 constexpr int backward_waves(int out) {
-    if (sizeof(T) == 8) return out == 3 ? 4 : 5;
-    return out == 3 ? kWavesWide : kWavesFull;
+    if (sizeof(T) == 8) return (out & 3) == 3 ? 4 : 5;
+    return out == 7 ? kWavesBoth : out == 3 ? kWavesWide : kWavesFull;
 }
 
 struct QDev {
@@ -133,6 +134,31 @@ __device__ __forceinline__ void corner_weight_grad(const AxisTerms<T>& t, int c,
     g[0] = t.dw[0][b0] * t.w[1][b1] * t.w[2][b2];
     g[1] = t.w[0][b0] * t.dw[1][b1] * t.w[2][b2];
     g[2] = t.w[0][b0] * t.w[1][b1] * t.dw[2][b2];
+}
+
+// grad w_c . u for the eight corners, with the products of the first two axes
+// taken once for both sides of the third: half the operations of the sum of
+// corner_weight_grad's three terms, and one rounding less on each.
+template <typename T>
+struct SlopeTerms {
+    T w01[4], d01[4], d2[2];
+};
+
+template <typename T>
+__device__ __forceinline__ void slope_terms(const AxisTerms<T>& t, const T (&u)[3], SlopeTerms<T>& s) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int b0 = i & 1, b1 = i >> 1;
+        s.w01[i] = t.w[0][b0] * t.w[1][b1];
+        s.d01[i] = (t.dw[0][b0] * u[0]) * t.w[1][b1] + t.w[0][b0] * (t.dw[1][b1] * u[1]);
+    }
+    s.d2[0] = t.dw[2][0] * u[2];
+    s.d2[1] = t.dw[2][1] * u[2];
+}
+
+template <typename T>
+__device__ __forceinline__ T corner_slope(const AxisTerms<T>& t, const SlopeTerms<T>& s, int c) {
+    return s.d01[c & 3] * t.w[2][c >> 2] + s.w01[c & 3] * s.d2[c >> 2];
 }
 
 // ------------------------------------------------------------ LDS layout
@@ -612,12 +638,17 @@ __device__ __forceinline__ void accumulate_row(T* __restrict__ grad_emb,
 // grad_embeddings[row_c, k] += w_c * z[i,k];
 // grad_offsets[i,:] = sum_c (emb[row_c,:] . z[i,:]) * grad w_c
 // (ash/src/grid.cu:177-255).  One lane per channel.
-// OUT: bit 0 = produce grad_embeddings, bit 1 = produce grad_offsets.
+// OUT: bit 0 = produce grad_embeddings, bit 1 = produce grad_offsets; bit 2 (with
+// bit 0) = and add to grad_embeddings what the backward of the backward does for
+// gg_off and z2 (below): the two contributions of a query go to the same eight
+// rows, and the requests for these are what either kernel is bound by (131 k ray
+// samples, rows of five: 28 + 23 -> 29 us; 2^22, rows of four, in the kernel for
+// these: 187 + 184 -> 254).
 template <typename T, int LPQ, bool LDS, int OUT>
 __global__ __launch_bounds__(kBlock, kWavesBackward) void
 query_backward_forward_kernel(
         QDev a, const T* __restrict__ z, T* __restrict__ grad_emb,
-        T* __restrict__ grad_off) {
+        T* __restrict__ grad_off, const T* __restrict__ gg_off, const T* __restrict__ z2) {
     extern __shared__ __align__(16) unsigned char smem[];
     Tile* tile_s = reinterpret_cast<Tile*>(smem);
     const CellLut lut =
@@ -629,6 +660,7 @@ query_backward_forward_kernel(
     const T* __restrict__ emb = static_cast<const T*>(a.emb);
     constexpr bool want_emb = (OUT & 1) != 0;
     constexpr bool want_off = (OUT & 2) != 0;
+    constexpr bool second = (OUT & 4) != 0;
     const int64_t ntiles = (a.N + kBlock - 1) / kBlock;
     TileWalk walk(ntiles);
     for (int64_t tile = walk.next; tile < walk.end; tile += walk.step) {
@@ -641,6 +673,15 @@ query_backward_forward_kernel(
             const bool valid = row[0] != kNoRow;
             const bool on = valid && chv;
             const T zk = on ? z[q * a.E + ch] : T(0);
+            T zk2 = T(0), gg[3] = {T(0), T(0), T(0)};
+            if constexpr (second) {
+                if (on) zk2 = z2[q * a.E + ch];
+                if (valid) {
+                    gg[0] = gg_off[q * 3 + 0];
+                    gg[1] = gg_off[q * 3 + 1];
+                    gg[2] = gg_off[q * 3 + 2];
+                }
+            }
             GroupRuns<LPQ> runs;
             runs.any = false;
             if (want_emb && a.merge) runs = find_group_runs<LPQ>(row[0], on, lane);
@@ -653,12 +694,16 @@ query_backward_forward_kernel(
             }
             AxisTerms<T> t;
             axis_terms<T, true>(o, a.smooth, t);
+            SlopeTerms<T> slope;
+            if constexpr (second) slope_terms<T>(t, gg, slope);
             T go[3] = {T(0), T(0), T(0)};
 #pragma unroll
             for (int c = 0; c < 8; ++c) {
                 if constexpr (want_emb) {
                     const T w = corner_weight<T>(t, c);
-                    accumulate_row<T, LPQ>(grad_emb, row[c], a.E, ch, on, w * zk, runs);
+                    T v = w * zk;
+                    if constexpr (second) v += corner_slope<T>(t, slope, c) * zk2;
+                    accumulate_row<T, LPQ>(grad_emb, row[c], a.E, ch, on, v, runs);
                 }
                 if constexpr (want_off) {
                     T gw[3];
@@ -1079,13 +1124,15 @@ template <bool LDS, int OUT, int THREADS>
 __global__ __launch_bounds__(THREADS, kWavesBackward) void
 query_backward_forward_vec_kernel(
         QDev a, const float* __restrict__ z, float* __restrict__ grad_emb,
-        float* __restrict__ grad_off) {
+        float* __restrict__ grad_off, const float* __restrict__ gg_off,
+        const float* __restrict__ z2) {
     extern __shared__ __align__(16) unsigned char smem[];
     const CellLut lut = stage_cell_lut<LDS, THREADS>(a, smem);
     const int lane = threadIdx.x & 63;
     const float* __restrict__ emb = static_cast<const float*>(a.emb);
     constexpr bool want_emb = (OUT & 1) != 0;
     constexpr bool want_off = (OUT & 2) != 0;
+    constexpr bool second = (OUT & 4) != 0;
     LineAcc acc;
     acc.start(line_table(smem, a, LDS, want_emb), lane);
     const int64_t ntiles = (a.N + THREADS - 1) / THREADS;
@@ -1097,11 +1144,19 @@ query_backward_forward_vec_kernel(
         const QueryInputs in = load_inputs(a, q);
         resolve_rows<LDS>(a, lut, in, row, o);
         const bool on = row[0] != kNoRow;
-        float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
+        float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f), y4 = z4;
+        float gg[3] = {0.f, 0.f, 0.f};
         if (on) {
             typedef float v4f __attribute__((ext_vector_type(4)));
             const v4f zl = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(z + q * 4));
             z4 = make_float4(zl.x, zl.y, zl.z, zl.w);
+            if constexpr (second) {
+                const v4f zs = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(z2 + q * 4));
+                y4 = make_float4(zs.x, zs.y, zs.z, zs.w);
+                gg[0] = __builtin_nontemporal_load(gg_off + q * 3 + 0);
+                gg[1] = __builtin_nontemporal_load(gg_off + q * 3 + 1);
+                gg[2] = __builtin_nontemporal_load(gg_off + q * 3 + 2);
+            }
         }
         AxisTerms<float> t;
         axis_terms<float, true>(o, a.smooth, t);
@@ -1138,10 +1193,19 @@ query_backward_forward_vec_kernel(
         }
         if constexpr (want_emb) {
             const Runs runs = tile_runs(row[0], on, lane);
+            SlopeTerms<float> slope;
+            if constexpr (second) slope_terms<float>(t, gg, slope);
 #pragma unroll
             for (int c = 0; c < 8; ++c) {
                 const float w = corner_weight<float>(t, c);
                 float v[4] = {w * z4.x, w * z4.y, w * z4.z, w * z4.w};
+                if constexpr (second) {
+                    const float d = corner_slope<float>(t, slope, c);
+                    v[0] += d * y4.x;
+                    v[1] += d * y4.y;
+                    v[2] += d * y4.z;
+                    v[3] += d * y4.w;
+                }
                 accumulate_row4(acc, grad_emb, row[c], on, runs, v, lane);
             }
             acc.flush(grad_emb, lane);
@@ -2246,23 +2310,39 @@ int launch_grid_forward(const QDev& d, const FrontDev& f, void* out, hipStream_t
     return 0;
 }
 
+// What a first-order backward takes along of the second order: nothing, or the
+// gradient with respect to the offsets' gradient and the z of that pass.
+struct Second {
+    const void* gg;
+    const void* z;
+};
+
+int gradients_wanted(const void* ge, const void* go, const Second& also) {
+    return (ge != nullptr ? 1 : 0) | (go != nullptr ? 2 : 0) | (also.gg != nullptr ? 4 : 0);
+}
+
 template <typename T, int LPQ>
-int launch_bwd_fwd(const QDev& d, const void* z, void* ge, void* go,
+int launch_bwd_fwd(const QDev& d, const void* z, void* ge, void* go, const Second& also,
                    hipStream_t s) {
     const size_t smem = smem_bytes(d, LPQ);
-    const int out = (ge != nullptr ? 1 : 0) | (go != nullptr ? 2 : 0);
+    const int out = gradients_wanted(ge, go, also);
     const unsigned g = persistent_grid((d.N + kBlock - 1) / kBlock, smem,
                                        backward_waves<T>(out));
 #define ASH_BF(L, O)                                                          \
     query_backward_forward_kernel<T, LPQ, L, O><<<g, kBlock, smem, s>>>(      \
             d, static_cast<const T*>(z), static_cast<T*>(ge),                 \
-            static_cast<T*>(go))
+            static_cast<T*>(go), static_cast<const T*>(also.gg),              \
+            static_cast<const T*>(also.z))
     if (lut_in_lds(d)) {
-        if (out == 3) ASH_BF(true, 3);
+        if (out == 7) ASH_BF(true, 7);
+        else if (out == 5) ASH_BF(true, 5);
+        else if (out == 3) ASH_BF(true, 3);
         else if (out == 1) ASH_BF(true, 1);
         else ASH_BF(true, 2);
     } else {
-        if (out == 3) ASH_BF(false, 3);
+        if (out == 7) ASH_BF(false, 7);
+        else if (out == 5) ASH_BF(false, 5);
+        else if (out == 3) ASH_BF(false, 3);
         else if (out == 1) ASH_BF(false, 1);
         else ASH_BF(false, 2);
     }
@@ -2311,25 +2391,32 @@ int vec_threads(const QDev& d, int out) {
     return wide ? 2 * kBlock : kBlock;
 }
 
-int launch_bwd_fwd_vec(const QDev& d, const void* z, void* ge, void* go,
+int launch_bwd_fwd_vec(const QDev& d, const void* z, void* ge, void* go, const Second& also,
                        hipStream_t s) {
-    const int out = (ge != nullptr ? 1 : 0) | (go != nullptr ? 2 : 0);
+    const int out = gradients_wanted(ge, go, also);
     const int threads = vec_threads(d, out);
     const size_t smem = smem_bytes(d, 1, ge != nullptr ? threads / 64 : 0);
     const unsigned g = persistent_grid((d.N + threads - 1) / threads, smem);
 #define ASH_BF(L, O, T)                                                       \
     query_backward_forward_vec_kernel<L, O, T><<<g, T, smem, s>>>(    \
             d, static_cast<const float*>(z), static_cast<float*>(ge),         \
-            static_cast<float*>(go))
+            static_cast<float*>(go), static_cast<const float*>(also.gg),      \
+            static_cast<const float*>(also.z))
     if (threads > kBlock) {
-        if (out == 3) ASH_BF(true, 3, 2 * kBlock);
+        if (out == 7) ASH_BF(true, 7, 2 * kBlock);
+        else if (out == 5) ASH_BF(true, 5, 2 * kBlock);
+        else if (out == 3) ASH_BF(true, 3, 2 * kBlock);
         else ASH_BF(true, 1, 2 * kBlock);
     } else if (lut_in_lds(d)) {
-        if (out == 3) ASH_BF(true, 3, kBlock);
+        if (out == 7) ASH_BF(true, 7, kBlock);
+        else if (out == 5) ASH_BF(true, 5, kBlock);
+        else if (out == 3) ASH_BF(true, 3, kBlock);
         else if (out == 1) ASH_BF(true, 1, kBlock);
         else ASH_BF(true, 2, kBlock);
     } else {
-        if (out == 3) ASH_BF(false, 3, kBlock);
+        if (out == 7) ASH_BF(false, 7, kBlock);
+        else if (out == 5) ASH_BF(false, 5, kBlock);
+        else if (out == 3) ASH_BF(false, 3, kBlock);
         else if (out == 1) ASH_BF(false, 1, kBlock);
         else ASH_BF(false, 2, kBlock);
     }
@@ -2464,22 +2551,22 @@ int dispatch_grid_forward(const QDev& d, const FrontDev& f, void* out, hipStream
 }
 
 template <typename T>
-int dispatch_bwd_fwd(const QDev& d, const void* z, void* ge, void* go,
+int dispatch_bwd_fwd(const QDev& d, const void* z, void* ge, void* go, const Second& also,
                      hipStream_t s) {
     if constexpr (sizeof(T) == 4) {
-        if (rows_as_float4(d, z, ge, nullptr)) return launch_bwd_fwd_vec(d, z, ge, go, s);
+        if (rows_as_float4(d, z, ge, also.z)) return launch_bwd_fwd_vec(d, z, ge, go, also, s);
     }
     switch (pow2_ceil(d.E)) {
         case 1:
-            return launch_bwd_fwd<T, 1>(d, z, ge, go, s);
+            return launch_bwd_fwd<T, 1>(d, z, ge, go, also, s);
         case 2:
-            return launch_bwd_fwd<T, 2>(d, z, ge, go, s);
+            return launch_bwd_fwd<T, 2>(d, z, ge, go, also, s);
         case 4:
-            return launch_bwd_fwd<T, 4>(d, z, ge, go, s);
+            return launch_bwd_fwd<T, 4>(d, z, ge, go, also, s);
         case 8:
-            return launch_bwd_fwd<T, 8>(d, z, ge, go, s);
+            return launch_bwd_fwd<T, 8>(d, z, ge, go, also, s);
         default:
-            return launch_bwd_fwd<T, 16>(d, z, ge, go, s);
+            return launch_bwd_fwd<T, 16>(d, z, ge, go, also, s);
     }
 }
 
@@ -2566,7 +2653,7 @@ int ash_grid_forward(ash_map_t* map, const float* x, const float* origin, float 
 namespace {
 
 int backward_forward(const ash_query_args* a, const void* z, void* grad_embeddings,
-                     void* grad_offsets, void* stream, bool clear) {
+                     void* grad_offsets, void* stream, bool clear, const Second& also = {}) {
     QDev d;
     if (check_args(a, d)) return 1;
     if (grad_embeddings == nullptr && grad_offsets == nullptr) {
@@ -2583,9 +2670,9 @@ int backward_forward(const ash_query_args* a, const void* z, void* grad_embeddin
     if (z == nullptr) ASH_FAIL("null pointer");
     return a->dtype == ASH_F64
                    ? dispatch_bwd_fwd<double>(d, z, grad_embeddings,
-                                              grad_offsets, s)
+                                              grad_offsets, also, s)
                    : dispatch_bwd_fwd<float>(d, z, grad_embeddings,
-                                             grad_offsets, s);
+                                             grad_offsets, also, s);
 }
 
 int backward_backward(const ash_query_args* a, const void* grad_grad_offsets,
@@ -2625,6 +2712,17 @@ int ash_query_backward_forward_accumulate(const ash_query_args* a, const void* z
                                           void* stream) {
     if (grad_embeddings == nullptr) ASH_FAIL("accumulate: null grad_embeddings");
     return backward_forward(a, z, grad_embeddings, grad_offsets, stream, false);
+}
+
+int ash_query_backward_both(const ash_query_args* a, const void* z, const void* grad_grad_offsets,
+                            const void* z_second, void* grad_embeddings, void* grad_offsets,
+                            int32_t accumulate, void* stream) {
+    if (grad_embeddings == nullptr) ASH_FAIL("backward_both: null grad_embeddings");
+    if (a != nullptr && a->num_queries > 0 && (grad_grad_offsets == nullptr || z_second == nullptr)) {
+        ASH_FAIL("null pointer");
+    }
+    return backward_forward(a, z, grad_embeddings, grad_offsets, stream, accumulate == 0,
+                            {grad_grad_offsets, z_second});
 }
 
 int ash_query_backward_backward(const ash_query_args* a,

@@ -48,3 +48,23 @@ def test_sizes_left_to_the_other_kernels(gpu_ash):
     grid, g = _grid(gpu_ash, 9, 70, seed=1)
     out = grid.convolution(grid.embeddings.data, torch.randn(3, 3, 3, 9, generator=g).to(DEV))
     assert out.shape == grid.embeddings.shape and float(out.detach().abs().sum()) > 0
+
+
+@pytest.mark.parametrize("channels,window", [(3, 3), (5, 3), (7, 3), (5, 5), (5, 7)])
+def test_workgroups_that_walk_several_blocks(gpu_ash, channels, window):
+    """More blocks than the device holds workgroups (at most seven a CU), an odd
+    number of channels: wavefronts that only load and store go round as well."""
+    blocks = 2003
+    grid = gpu_ash.SparseDenseGrid(3, blocks + 9, channels, 8, device=DEV)
+    g = torch.Generator().manual_seed(channels)
+    keys = torch.unique(torch.randint(0, 16, (3 * blocks, 3), generator=g), dim=0)[:blocks]
+    grid.engine.insert_keys(keys.int().to(DEV))
+    weights = torch.randn(window, window, window, channels, generator=g).to(DEV)
+    with torch.no_grad():
+        grid.embeddings.copy_(torch.randn(grid.embeddings.shape, generator=g))
+    c2g, c2c, lut = grid._window_tables(window // 2)
+    _, listed = grid.engine.items()
+    want = gpu_ash.grid.backend.convolution_forward(
+        grid.embeddings.data, weights.view(-1, channels), torch.ones(blocks, 512, dtype=torch.bool, device=DEV),
+        listed, grid.cell_indices, lut, c2c, c2g, 8)
+    assert torch.equal(gpu_ash.grid.backend.convolution_cube(grid.embeddings.data, weights, listed, lut, 8), want)

@@ -7,27 +7,24 @@
 // (dx + r) + W (dy + r) + W^2 (dz + r); neighbour block (bx + 1) + 3 (by + 1) + 9
 // (bz + 1)), so no per-cell table is read, checked or needed.
 //
-// Two wavefronts per channel, lane = (x, z), four cells along y per lane: the
-// channels of a block are an even load whatever their number (five channels in
-// instances for eight left three quarters of the second turn idle), a row of
-// the tile is read once for all cells that need it, and a tap's weight is one
-// scalar for the wavefront.  (Eight cells per lane read the tile less often but
-// hold twice the elements in flight: the same time for windows of 3, 1.4 times
-// for windows of 7.)  Every cell still sees its taps in table order, one fused
-// multiply-add per tap, as in the other kernels.
+// One or two wavefronts per channel (Shape::kOneEach), lane = (x, z), eight or
+// four cells along y per lane: a row of the tile is read once for all cells that
+// need it, and a tap's weight is one scalar for the wavefront.  Every cell still
+// sees its taps in table order, one fused multiply-add per tap, as in the other
+// kernels.
 //
-// 60 000 blocks, tables and instances for powers of two before: five channels
-// 3^3 1275 -> 477 us, 7^3 4.3 -> 3.5 ms; two channels 501 -> 159 us, 2.2 -> 1.0
-// ms; 1000 blocks, 7^3: 990 -> 94 us (every workgroup used to check the tables).
-// 3^3 windows of five channels move 1.72 GB beyond the L2s, 3.9 TB/s: 0.61 GB of
-// results and 1.11 of rows, 1.8 times what there are (the halo along x takes most
-// lines of two neighbours).  7^3 windows of two channels are
-// bound by vector instructions (issued in 0.87 of the cycles; 1941 per wavefront
-// and block, 1372 of them multiply-adds and 343 tap reads), of five by the one
-// workgroup of ten wavefronts that a CU's registers hold (0.59).
+// 60 000 blocks: five channels 3^3 346 us (440 before one wavefront each, 1275
+// with tables and instances for powers of two), two channels 143 (501); 1000
+// blocks, 7^3: 94 (990: every workgroup used to check the tables).  3^3 windows of
+// five channels move 1.56 GB beyond the L2s, 4.5 TB/s: 0.61 GB of results and 0.95
+// of rows, 1.5 times what there are (the halo along x takes most lines of two
+// neighbours); vector instructions are issued in 0.59 of the cycles, the LDS is
+// busy in 0.54.  7^3 windows of two channels are bound by vector instructions
+// (0.87 of the cycles; 1941 per wavefront and block, 1372 of them multiply-adds
+// and 343 tap reads).
 //
 // The block's own rows are contiguous in memory whatever their width: they come
-// in as two 16-byte pieces per thread, and leave the same way, through LDS.
+// in as 16-byte pieces and leave the same way, through LDS.
 // The halo comes element by element (consecutive lanes, consecutive words of a
 // row).  Where an element goes in the tile never changes from block to block
 // and is kept in registers.  Software pipeline: while a block is computed the
@@ -45,14 +42,10 @@ namespace {
 constexpr int kG = 8;
 constexpr int kM = kG * kG * kG;
 constexpr int kMaxChannels = 8;
-constexpr int kY = 4;   // cells along y per lane
 constexpr int kFillBlock = 256;
 
 template <int E, int W>
 struct Shape {
-    static constexpr int kParts = kG / kY;                         // wavefronts per channel
-    static constexpr int kThreads = 64 * E * kParts;
-    static constexpr int kOwnEach = kM * E / 4 / kThreads;        // 16-byte pieces per thread
     static constexpr int kR = W / 2;
     static constexpr int kT = kG + 2 * kR;
     // words between the z layers of a channel's plane: 8 or 24 modulo 32, so
@@ -65,26 +58,44 @@ struct Shape {
     }
     static constexpr int kLayer = layer();
     static constexpr int kPlane = kLayer * kT;
-    static constexpr int kHalo = kT * kT * kT - kM;               // rows
-    static constexpr int kHaloEach = (kHalo * E + kThreads - 1) / kThreads;   // elements per thread
-    static constexpr int kTaps = W * W;                           // of one dz
     // results on their way out: a z layer's rows, four words apart from the next
     // layer's (banks)
     static constexpr int kOutLayer = 64 * E + 4;
     static constexpr int kTileWords = E * kPlane;
     static constexpr int kOutWords = kG * kOutLayer;
     static constexpr int kWeightWords = E * W * 64;
+    static constexpr int kFit = 160 * 1024 / (4 * (kTileWords + kOutWords + kWeightWords) + 1024);
+    // Cells along y per lane, and with them wavefronts per channel.  Two per
+    // channel, but for odd numbers of channels, where that is no multiple of the
+    // four SIMDs: a CU then takes fewer workgroups than its registers hold (five
+    // channels, ten wavefronts of 64 registers: two, not three, and the third of
+    // the grid ran behind, 16 wavefronts per CU on average).  There one wavefront
+    // per channel, and helpers up to a multiple of four that only load and
+    // store; where the LDS holds a single workgroup, two per channel are better.
+    // 40 000 blocks, 3^3: three channels 157 -> 129 us, five 293 -> 236, seven
+    // 400 -> 321; 12 000 blocks, 5^3: 155 -> 139, 244 -> 234, 390 -> 298; 4000,
+    // 7^3: 160 -> 146, 261 -> 223, seven (one workgroup) 311 against 324.  Even
+    // numbers that way: 0 - 20 % slower; one channel with helpers 56 -> 71.
+    static constexpr bool kOneEach = E % 2 == 1 && E > 1 && kFit > 1;
+    static constexpr int kY = kOneEach ? 8 : 4;
+    static constexpr int kParts = kG / kY;
+    static constexpr int kWorkers = E * kParts;                    // wavefronts that compute
+    static constexpr int kThreads = 64 * (kOneEach ? (kWorkers + 3) / 4 * 4 : kWorkers);
+    static constexpr int kPieces = kM * E / 4;                     // of 16 bytes, a block's own rows
+    static constexpr int kOwnEach = (kPieces + kThreads - 1) / kThreads;   // per thread
+    static constexpr int kHalo = kT * kT * kT - kM;               // rows
+    static constexpr int kHaloEach = (kHalo * E + kThreads - 1) / kThreads;   // elements per thread
+    static constexpr int kTaps = W * W;                           // of one dz
     // wavefronts per SIMD that the tile leaves room for.  No more than the
-    // registers allow without spills: 64 for windows of 3 and 74 - 76 for 5 are
-    // below what the bound leaves them, 108 for 7 are four wavefronts.  (Five,
-    // 96 registers, spill 10 - 12 of them.  20 000 blocks, 7^3: one channel 222
-    // -> 192 us, two 344 -> 340, three 814 -> 651, five 1181 -> 1112; 2000
-    // blocks: 47 -> 50, 61 -> 62, 105 -> 94, 150 -> 140.)
-    static constexpr int kMostWaves = W == 3 ? 6 : (W == 5 ? 5 : 4);
+    // registers allow: 64 for windows of 3 and 74 - 80 for 5 are eight and six
+    // (five channels, 5^3, spill 14 of them and gain all the same: 245 -> 234), 108
+    // - 128 for 7 are four.  (Five, 96 registers, for 7: 20 000 blocks, one channel
+    // 192 -> 222 us, two 340 -> 344; three, five channels 223 -> 286.)
+    static constexpr int kMostWaves = W == 3 ? 8 : (W == 5 ? 6 : 4);
     static constexpr int waves() {
-        const int lds = 4 * (kTileWords + kOutWords + kWeightWords) + 1024;
-        const int fit = (160 * 1024 / lds * E * kParts + 3) / 4;
-        return fit < 1 ? 1 : (fit > kMostWaves ? kMostWaves : fit);
+        const int each = (kThreads / 64 + 3) / 4;   // of one workgroup
+        const int fit = kFit < kMostWaves / each ? kFit : kMostWaves / each;
+        return fit < 1 ? each : fit * each;
     }
 };
 
@@ -110,8 +121,8 @@ convolution_block8_kernel(ConvArgs a) {
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int q = wave / S::kParts;             // the wavefront's channel
-    const int y0 = wave % S::kParts * kY;        // and the first of its cells along y
-    constexpr int R = S::kR, T = S::kT;
+    const int y0 = wave % S::kParts * S::kY;     // and the first of its cells along y
+    constexpr int R = S::kR, T = S::kT, kY = S::kY;
 
     // weights by channel and dz, one tap per lane
     for (int t = tid; t < S::kWeightWords; t += S::kThreads) {
@@ -205,8 +216,10 @@ convolution_block8_kernel(ConvArgs a) {
         const uint32_t g = nb[27] < 0 ? 0u : static_cast<uint32_t>(nb[27]);
 #pragma unroll
         for (int i = 0; i < S::kOwnEach; ++i) {
-            own[i] = *reinterpret_cast<const v4*>(in + (g * kBlockBytes +
-                                                        16u * static_cast<uint32_t>(tid + i * S::kThreads)));
+            const int piece = tid + i * S::kThreads;
+            if (S::kPieces % S::kThreads == 0 || piece < S::kPieces) {
+                own[i] = *reinterpret_cast<const v4*>(in + (g * kBlockBytes + 16u * static_cast<uint32_t>(piece)));
+            }
         }
         have = 0;
 #pragma unroll
@@ -233,6 +246,7 @@ convolution_block8_kernel(ConvArgs a) {
         const int32_t g = s_nb[buf][27];
 #pragma unroll
         for (int i = 0; i < S::kOwnEach; ++i) {
+            if (S::kPieces % S::kThreads != 0 && tid + i * S::kThreads >= S::kPieces) continue;
 #pragma unroll
             for (int c = 0; c < 4; ++c) s_tile[(own_dst[i][c >> 1] >> (16 * (c & 1))) & 0xFFFFu] = own[i][c];
         }
@@ -245,33 +259,35 @@ convolution_block8_kernel(ConvArgs a) {
         rows_reg = fetch_rows(blk + 2 * walk.step);
         if (blk + walk.step < walk.end) load_block(s_nb[buf ^ 1]);
 
-        float acc[kY];
+        if (wave < S::kWorkers) {
+            float acc[kY];
 #pragma unroll
-        for (int j = 0; j < kY; ++j) acc[j] = 0.f;
+            for (int j = 0; j < kY; ++j) acc[j] = 0.f;
 #pragma unroll 1
-        for (int dz = 0; dz < W; ++dz) {
-            const float* layer = window + S::kLayer * dz;
-            const float taps = s_w[(q * W + dz) * 64 + lane];
+            for (int dz = 0; dz < W; ++dz) {
+                const float* layer = window + S::kLayer * dz;
+                const float taps = s_w[(q * W + dz) * 64 + lane];
 #pragma unroll
-            for (int y = 0; y < kY + 2 * R; ++y) {
-                float row[W];
+                for (int y = 0; y < kY + 2 * R; ++y) {
+                    float row[W];
 #pragma unroll
-                for (int dx = 0; dx < W; ++dx) row[dx] = layer[T * y + dx];
+                    for (int dx = 0; dx < W; ++dx) row[dx] = layer[T * y + dx];
 #pragma unroll
-                for (int j = 0; j < kY; ++j) {
-                    const int dy = y - j;
-                    if (dy < 0 || dy >= W) continue;
+                    for (int j = 0; j < kY; ++j) {
+                        const int dy = y - j;
+                        if (dy < 0 || dy >= W) continue;
 #pragma unroll
-                    for (int dx = 0; dx < W; ++dx) {
-                        const float tap = __int_as_float(
-                                __builtin_amdgcn_readlane(__float_as_int(taps), dy * W + dx));
-                        acc[j] = fmaf(row[dx], tap, acc[j]);
+                        for (int dx = 0; dx < W; ++dx) {
+                            const float tap = __int_as_float(
+                                    __builtin_amdgcn_readlane(__float_as_int(taps), dy * W + dx));
+                            acc[j] = fmaf(row[dx], tap, acc[j]);
+                        }
                     }
                 }
             }
-        }
 #pragma unroll
-        for (int j = 0; j < kY; ++j) result[j * kG * E] = acc[j];
+            for (int j = 0; j < kY; ++j) result[j * kG * E] = acc[j];
+        }
         __syncthreads();   // the results are complete, and the tile has been read
         if (g >= 0) {
             v4* rows = reinterpret_cast<v4*>(a.out) +
@@ -279,6 +295,7 @@ convolution_block8_kernel(ConvArgs a) {
 #pragma unroll
             for (int i = 0; i < S::kOwnEach; ++i) {
                 const int f = tid + i * S::kThreads;
+                if (S::kPieces % S::kThreads != 0 && f >= S::kPieces) continue;
                 const int out_z = f / (16 * E);
                 __builtin_nontemporal_store(*reinterpret_cast<const v4*>(s_out + 4 * f + 4 * out_z),
                                             rows + f);

@@ -487,14 +487,21 @@ __device__ __forceinline__ int staged(int lb, int q) {
 enum { kPlaced = 0, kKnown = 1, kFull = 2 };
 
 // Inserts `code` into the LDS copy of the partition, starting at local bucket
-// lb and going round inside the partition (next_bucket's rule).  kPlaced: the
-// calling thread owns slot `where` (local bucket * 16 + slot) now; kKnown: the
-// code was there already (or another thread of this round placed it); kFull:
-// every bucket of the partition has been visited.
+// lb and going round inside the partition (next_bucket's rule): into the first
+// slot that is empty or a tombstone, by the per-key kernel's steps (insert_key,
+// ash_map.hip).  kPlaced: the calling thread owns slot `where` (local bucket * 16
+// + slot) now; kKnown: the code was there already (or another thread of this round
+// placed it); kFull: every bucket of the partition has been visited.  `reused`
+// counts tombstones that hold a key now; a range that started empty has none
+// (TOMBS false).
+template <bool TOMBS>
 __device__ __forceinline__ int place_code(uint4* tab, uint64_t code, int lb, int nbk,
-                                          int& where) {
+                                          int& where, int* reused) {
     unsigned long long* tab64 = reinterpret_cast<unsigned long long*>(tab);
-    for (int visited = 0; visited < nbk; ++visited) {
+    bool claiming = false;
+    int tomb_lb = -1, tomb_visited = 0;   // the first bucket with a tombstone
+    int visited = 0;
+    while (visited < nbk) {
         uint64_t c[kSlots];
 #pragma unroll
         for (int q = 0; q < kSlots / 2; ++q) {
@@ -503,24 +510,42 @@ __device__ __forceinline__ int place_code(uint4* tab, uint64_t code, int lb, int
             c[2 * q + 1] = static_cast<uint64_t>(w.z) | (static_cast<uint64_t>(w.w) << 32);
         }
         bool known = false;
-        uint32_t em = 0;
+        uint32_t em = 0, tm = 0;
 #pragma unroll
         for (int s = 0; s < kSlots; ++s) {
             known |= c[s] == code;
             em |= (c[s] == kEmpty ? 1u : 0u) << s;
+            if constexpr (TOMBS) tm |= (c[s] == kTomb ? 1u : 0u) << s;
         }
         if (known) return kKnown;
-        while (em) {
-            const int s = __builtin_ctz(em);
-            const unsigned long long old =
-                    atomicCAS(tab64 + staged(lb, s >> 1) * 2 + (s & 1), kEmpty, code);
-            if (old == kEmpty) {
-                where = lb * kBucketQwords + s;
-                return kPlaced;
+        if (TOMBS && !claiming && em == 0 && visited + 1 < nbk) {
+            if (tm != 0 && tomb_lb < 0) {
+                tomb_lb = lb;
+                tomb_visited = visited;
             }
-            if (old == code) return kKnown;
-            em &= em - 1;
+        } else if (TOMBS && !claiming && tomb_lb >= 0) {
+            claiming = true;
+            lb = tomb_lb;
+            visited = tomb_visited;
+            continue;
+        } else {
+            claiming = true;
+            em |= tm;
+            while (em) {
+                const int s = __builtin_ctz(em);
+                const unsigned long long free = (tm >> s) & 1u ? kTomb : kEmpty;
+                const unsigned long long old =
+                        atomicCAS(tab64 + staged(lb, s >> 1) * 2 + (s & 1), free, code);
+                if (old == free) {
+                    where = lb * kBucketQwords + s;
+                    if (free == kTomb) atomicAdd(reused, 1);
+                    return kPlaced;
+                }
+                if (old == code) return kKnown;
+                em &= em - 1;
+            }
         }
+        ++visited;
         if (++lb == nbk) lb = 0;
     }
     return kFull;
@@ -596,8 +621,9 @@ __device__ __forceinline__ void drop_repeats(uint4* tab, int lb, int n, Dropped 
 enum { kRecIdle = 0, kRecPlaced = 1, kRecLost = 2 };
 constexpr int kWaitList = 128;
 
+// (four wavefronts per SIMD: the two workgroups that the LDS holds)
 template <bool PROV>
-__global__ __launch_bounds__(kBuildThreads) void build_kernel(
+__global__ __launch_bounds__(kBuildThreads, 4) void build_kernel(
         MapDev m, BulkPlan pl, int stale, int identity) {
     // Records per thread and round.  With rows the partitions of a batch of the
     // order of the table take one round of five (16 M keys into 24 M: 2048 +- 45
@@ -614,6 +640,7 @@ __global__ __launch_bounds__(kBuildThreads) void build_kernel(
     __shared__ int s_wcnt[kRecSlots * (kBuildThreads / 64)];
     __shared__ int s_base;
     __shared__ int s_losers;
+    __shared__ int s_reused;                // tombstones that hold a key now
     __shared__ int s_drawn[kPartBuckets];   // numbers drawn per bucket (range that starts empty)
     __shared__ int s_seen[kPartBuckets];    // of which drop_repeats has compared this many
     // records that wait for the probing path: the first kWaitList of them here,
@@ -648,6 +675,7 @@ __global__ __launch_bounds__(kBuildThreads) void build_kernel(
     const int64_t bbase = static_cast<int64_t>(p) * pl.cap_part;
     if (tid == 0) {
         s_losers = 0;
+        s_reused = 0;
         s_nwait = 0;
     }
     // (slot kRecs: a record taken from the waiting list, last round only)
@@ -766,7 +794,8 @@ __global__ __launch_bounds__(kBuildThreads) void build_kernel(
             wslot[k] = -1;
             if (!((which >> k) & 1u)) continue;
             const int lb = static_cast<int>(bucket_of(codes[k], m.nb) - b0);
-            const int how = place_code(tab, codes[k], lb, nbk, wslot[k]);
+            const int how = counted ? place_code<false>(tab, codes[k], lb, nbk, wslot[k], nullptr)
+                                    : place_code<true>(tab, codes[k], lb, nbk, wslot[k], &s_reused);
             if (how == kFull) atomicAdd(m.ctr + kCtrDropped, 1);   // refused
             state[k] = how == kPlaced ? kRecPlaced : kRecLost;
         }
@@ -853,7 +882,7 @@ __global__ __launch_bounds__(kBuildThreads) void build_kernel(
                     codes[x] = s_wait_code[tid];
                     rows[x] = s_wait_row[tid];
                     const int lb = static_cast<int>(bucket_of(codes[x], m.nb) - b0);
-                    const int how = place_code(tab, codes[x], lb, nbk, wslot[x]);
+                    const int how = place_code<false>(tab, codes[x], lb, nbk, wslot[x], nullptr);
                     if (how == kFull) atomicAdd(m.ctr + kCtrDropped, 1);   // refused
                     state[x] = how == kPlaced ? kRecPlaced : kRecLost;
                 }
@@ -885,6 +914,8 @@ __global__ __launch_bounds__(kBuildThreads) void build_kernel(
             __builtin_nontemporal_store(y, reinterpret_cast<v4u*>(gl) + t);
         }
     }
+    // (final, like s_losers: every round ends with a barrier)
+    if (tid == 0 && s_reused) atomicSub(m.ctr + kCtrTombs, s_reused);
     if constexpr (PROV) {
         if (tid == 0 && s_losers) atomicAdd(pl.hdr + kHdrLosers, s_losers);
     }

@@ -65,6 +65,7 @@ struct ProbeResult {
     int slot;        // matching slot (status == kProbeFound)
     int32_t val;     // index stored with the matching slot
     uint32_t emask;  // bit s set <=> slot s was empty in this snapshot
+    uint32_t tmask;  // ... held a tombstone (asked for with TOMBS)
 };
 
 // Every lane of the wavefront calls this together.  Lane L owns key L; in
@@ -75,6 +76,7 @@ struct ProbeResult {
 // A quad, because what its lanes tell each other -- whose key, which slot,
 // which index -- are quad permutations, modifiers of a vector instruction, where
 // groups of eight have to go through ballots and the LDS pipeline.
+template <bool TOMBS = false>
 __device__ __forceinline__ void probe_pass(const MapDev& m, uint64_t code,
                                            uint32_t b, bool pend, int lane,
                                            ProbeResult& out) {
@@ -102,7 +104,7 @@ __device__ __forceinline__ void probe_pass(const MapDev& m, uint64_t code,
         // (codes 8 and 9, in the quad's first lane; indices in the others)
         const uint64_t q8 = j == 0 ? hi[r].x | (static_cast<uint64_t>(hi[r].y) << 32) : 0ull;
         const uint64_t q9 = j == 0 ? hi[r].z | (static_cast<uint64_t>(hi[r].w) << 32) : 0ull;
-        uint32_t v = 0;   // bits 0..3: slot + 1 of the match, bits 4..13: empty slots
+        uint32_t v = 0;   // bits 0..3: slot + 1 of the match, 4..13: empty slots, 14..23: tombstones
         if (j == 0 && q8 == want) v = 9;
         if (j == 0 && q9 == want) v = 10;
         if (q0 == want) v = 2 * j + 1;
@@ -111,13 +113,20 @@ __device__ __forceinline__ void probe_pass(const MapDev& m, uint64_t code,
         if (q1 == kEmpty) v |= 32u << (2 * j);
         if (q8 == kEmpty) v |= 16u << 8;
         if (q9 == kEmpty) v |= 16u << 9;
+        if constexpr (TOMBS) {
+            if (q0 == kTomb) v |= 16384u << (2 * j);
+            if (q1 == kTomb) v |= 32768u << (2 * j);
+            if (q8 == kTomb) v |= 16384u << 8;
+            if (q9 == kTomb) v |= 16384u << 9;
+        }
         v = quad_or(v);
         const int slot = static_cast<int>(v & 15u) - 1;
         const int comp = slot & 3;   // index of slot s: dword 20 + s of the bucket
         const uint32_t word = comp == 0 ? hi[r].x : comp == 1 ? hi[r].y : comp == 2 ? hi[r].z : hi[r].w;
         const uint32_t val = quad_or(j == ((4 + slot) >> 2) ? word : 0u);
         if (j == r) {
-            out.emask = v >> 4;
+            out.emask = (v >> 4) & ((1u << kSlots) - 1u);
+            if constexpr (TOMBS) out.tmask = v >> (4 + kSlots);
             out.status = slot >= 0 ? kProbeFound : (out.emask ? kProbeHasEmpty : kProbeFull);
             out.slot = slot;
             out.val = static_cast<int32_t>(val);
@@ -309,7 +318,11 @@ __device__ __forceinline__ void insert_key(
     uint32_t wb = 0, gp = 0;
     int ws = 0;
 
-    // Phase A: claim a slot per new key.
+    // Phase A: claim a slot per new key.  First its sequence is followed to the end
+    // (a bucket with an empty slot, or the whole range): a key that is met there is
+    // stored already.
+    bool claiming = false;
+    uint32_t free_slots = 0;   // of the bucket the sequence ended in
     while (__ballot(pend)) {
         ProbeResult p;
         probe_pass(m, code, b, pend, lane, p);
@@ -320,36 +333,78 @@ __device__ __forceinline__ void insert_key(
                     atomicAdd(m.ctr + kCtrLoadDup, 1);
                 }
                 if constexpr (MODE == kInsertReport) seen = p.val;
+            } else if (p.status == kProbeHasEmpty || ++steps >= kPartBuckets) {
+                pend = false;
+                claiming = true;
+                free_slots = p.emask;
             } else {
-                uint32_t em = p.emask;
-                while (em) {
-                    const int s = __builtin_ctz(em);
-                    const unsigned long long old =
-                            atomicCAS(slot_ptr(m, b, s), kEmpty, code);
-                    if (old == kEmpty) {
-                        won = true;
-                        wb = b;
-                        ws = s;
-                        pend = false;
-                        break;
-                    }
-                    if (old == code) {
-                        pend = false;
-                        if constexpr (MODE == kInsertLoad) {
-                            atomicAdd(m.ctr + kCtrLoadDup, 1);
-                        }
-                        break;
-                    }
-                    em &= em - 1;
+                b = next_bucket(b, m.nb);
+            }
+        }
+    }
+    // Then the key takes the first slot of its sequence that is free, empty or a
+    // tombstone (nearly always one of the bucket looked at just now, the
+    // sequence's first).  Slots are tried in the order of the sequence, and
+    // nothing frees a slot while keys are inserted, so threads that store the same
+    // key meet in the same slot, whatever others have taken in between.
+    // (Tombstones that are left alone pile up: keys that come and go behind a run of
+    // full buckets lengthen it by what they leave each time, until the range is full
+    // and refuses keys.  A million stored keys, 65 537 that come, are read and go:
+    // 125 us a pass, but 1000 - 2700 after sixty passes on one map in twelve.)
+    bool looked = steps == 0;   // free_slots are those of bucket b
+    bool reused = false;
+    if (claiming && !looked) {
+        b = bucket_of(code, m.nb);
+        steps = 0;
+    }
+    while (__ballot(claiming)) {
+        ProbeResult p;
+        p.status = kProbeHasEmpty;
+        p.emask = free_slots;
+        p.tmask = 0;
+        if (__ballot(claiming && !looked)) {
+            ProbeResult again;
+            probe_pass<true>(m, code, b, claiming && !looked, lane, again);
+            if (!looked) p = again;
+        }
+        if (claiming) {
+            if (p.status == kProbeFound) {
+                claiming = false;
+                if constexpr (MODE == kInsertLoad) {
+                    atomicAdd(m.ctr + kCtrLoadDup, 1);
                 }
-                if (pend) {
-                    b = next_bucket(b, m.nb);
-                    if (++steps >= kPartBuckets) {
-                        pend = false;
-                        refused = true;
+                if constexpr (MODE == kInsertReport) seen = p.val;
+            }
+            uint32_t em = claiming ? p.emask | p.tmask : 0u;
+            while (em) {
+                const int s = __builtin_ctz(em);
+                const unsigned long long free = (p.tmask >> s) & 1u ? kTomb : kEmpty;
+                const unsigned long long old = atomicCAS(slot_ptr(m, b, s), free, code);
+                if (old == free) {
+                    won = true;
+                    reused = free == kTomb;
+                    wb = b;
+                    ws = s;
+                    claiming = false;
+                    break;
+                }
+                if (old == code) {
+                    claiming = false;
+                    if constexpr (MODE == kInsertLoad) {
+                        atomicAdd(m.ctr + kCtrLoadDup, 1);
                     }
+                    break;
+                }
+                em &= em - 1;
+            }
+            if (claiming && !looked) {
+                b = next_bucket(b, m.nb);
+                if (++steps >= kPartBuckets) {
+                    claiming = false;
+                    refused = true;
                 }
             }
+            looked = false;   // (the first bucket once more: it may hold tombstones)
         }
     }
     if (active && !fits) {
@@ -371,7 +426,9 @@ __device__ __forceinline__ void insert_key(
     // Phase B: one heap-counter update per block, indices for the winners.
     const bool w = won || gwon;
     int32_t idx = -1;
+    const int nreused = __popcll(__ballot(reused));
     if constexpr (MODE == kInsertLoad) {
+        if (lane == 0 && nreused > 0) atomicSub(m.ctr + kCtrTombs, nreused);
         if (w) {
             // the index comes with the key (`given` null: the key's own number,
             // when the keys are the entries of the key log)
@@ -394,16 +451,24 @@ __device__ __forceinline__ void insert_key(
         }
     } else {
         __shared__ int s_cnt[kHeapBlock / 64];
+        __shared__ int s_reused[kHeapBlock / 64];
         __shared__ int s_base;
         const uint64_t wm = __ballot(w);
         const int nw = __popcll(wm);
         const int rank = __popcll(wm & ((1ull << lane) - 1ull));
-        if (lane == 0) s_cnt[wave] = nw;
+        if (lane == 0) {
+            s_cnt[wave] = nw;
+            s_reused[wave] = nreused;
+        }
         __syncthreads();
         if (threadIdx.x == 0) {
-            int tot = 0;
+            int tot = 0, again = 0;
 #pragma unroll
-            for (int q = 0; q < kHeapBlock / 64; ++q) tot += s_cnt[q];
+            for (int q = 0; q < kHeapBlock / 64; ++q) {
+                tot += s_cnt[q];
+                again += s_reused[q];
+            }
+            if (again > 0) atomicSub(m.ctr + kCtrTombs, again);
             int base = 0;
             if (tot > 0) {
                 base = atomicAdd(m.ctr + kCtrSize, tot);

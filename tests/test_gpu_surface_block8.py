@@ -51,3 +51,18 @@ def test_same_mesh_as_the_tables(gpu_ash, blocks, stride, dtype, bounded):
                            sdf, weights, listed, grid.grid_coords, grid.lut_grid_nb2grid_idx,
                            grid.cell_coords, grid.lut_cell_nb2cell_idx, grid.lut_cell_nb2grid_nb, 8,
                            0.1, 1.0)[1] + 1.0)
+
+
+@pytest.mark.parametrize("stride,sdf,weight", [(2, 1, 0), (3, 0, 2), (4, 0, 1), (4, 3, 0), (5, 4, 0), (5, 1, 3),
+                                               (6, 0, 5), (7, 0, 3), (8, 0, 7), (8, 4, 7), (9, 0, 8)])
+def test_channels_anywhere_in_their_rows(gpu_ash, stride, sdf, weight):
+    """Field and weights as channels of rows of two to eight (and nine) floats,
+    the first of them 16-byte aligned or not, rows that nobody lists among them."""
+    grid, g = _grid(gpu_ash, 150, False, seed=stride)
+    rows = torch.randn(grid.num_embeddings, 512, stride, generator=g).to(DEV)
+    rows[..., weight] = (torch.rand(rows.shape[:2], generator=g) * 10).to(DEV)
+    f, w = rows[..., sdf], rows[..., weight]
+    triangles, vertices = grid.surface_mesh(f, w, 0.1, 1.0)
+    apart = grid.surface_mesh(f.contiguous(), w.contiguous(), 0.1, 1.0)
+    assert len(triangles) > 1000
+    assert torch.equal(triangles, apart[0]) and torch.equal(vertices, apart[1])

@@ -68,3 +68,25 @@ def test_workgroups_that_walk_several_blocks(gpu_ash, channels, window):
         grid.embeddings.data, weights.view(-1, channels), torch.ones(blocks, 512, dtype=torch.bool, device=DEV),
         listed, grid.cell_indices, lut, c2c, c2g, 8)
     assert torch.equal(gpu_ash.grid.backend.convolution_cube(grid.embeddings.data, weights, listed, lut, 8), want)
+
+
+@pytest.mark.parametrize("blocks,channels,window", [(1, 8, 7), (3000, 5, 3), (700_000, 1, 3)])
+def test_rows_of_unlisted_blocks_are_cleared(gpu_ash, blocks, channels, window):
+    """Fewer blocks than a workgroup looks at, more than there are workgroups, and
+    more flags than the workgroups look at in one round (at most 16 a CU of 128
+    threads); the first, the last and some in between are listed."""
+    backend = gpu_ash.grid.backend
+    g = torch.Generator().manual_seed(blocks)
+    inputs = torch.randn(blocks, 512, channels, device=DEV)
+    weights = torch.randn(window, window, window, channels, generator=g).to(DEV)
+    lut = torch.full((blocks, 27), -1, dtype=torch.int64, device=DEV)
+    lut[:, 13] = torch.arange(blocks, device=DEV)
+    some = torch.unique(torch.cat([torch.tensor([0, blocks - 1]), torch.randint(blocks, (blocks // 3,), generator=g)]))
+    listed = some[torch.randperm(len(some), generator=g)].to(DEV)
+    everywhere = backend.convolution_cube(inputs, weights, torch.arange(blocks, device=DEV), lut, 8)
+    for rows in (listed, listed[:0]):
+        torch.full_like(inputs, 7.0)     # the result's memory does not start as zeros
+        got = backend.convolution_cube(inputs, weights, rows, lut, 8)
+        want = torch.zeros_like(inputs)
+        want[rows] = everywhere[rows]
+        assert torch.equal(got, want)

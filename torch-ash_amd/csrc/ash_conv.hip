@@ -13,8 +13,8 @@
 // sees its taps in table order, one fused multiply-add per tap, as in the other
 // kernels.
 //
-// 60 000 blocks: five channels 3^3 346 us (440 before one wavefront each, 1275
-// with tables and instances for powers of two), two channels 143 (501); 1000
+// 60 000 blocks: five channels 3^3 347 us a call (440 before one wavefront each, 1275
+// with tables and instances for powers of two), two channels 126 (501); 1000
 // blocks, 7^3: 94 (990: every workgroup used to check the tables).  3^3 windows of
 // five channels move 1.56 GB beyond the L2s, 4.5 TB/s: 0.61 GB of results and 0.95
 // of rows, 1.5 times what there are (the halo along x takes most lines of two
@@ -105,6 +105,7 @@ struct ConvArgs {
     const int64_t* grid_indices;
     const int64_t* lut_g;   // [B, 27]
     float* out;
+    const uint8_t* listed;  // [B]: rows of the others become zeros
     int64_t n_grids, B;
 };
 
@@ -234,6 +235,30 @@ convolution_block8_kernel(ConvArgs a) {
     int64_t blk = walk.next;
     int buf = 0;
     int32_t rows_reg = fetch_rows(blk);
+    // Zeros for the blocks that are not listed: each workgroup looks at a share of
+    // the flags, one per thread, while its first rows are on their way (a launch
+    // of their own, one flag after the other per workgroup: 60 000 blocks, all
+    // listed, 9.8 us).
+    int32_t* const s_bare = reinterpret_cast<int32_t*>(s_out);
+    static_assert(S::kOutWords > S::kThreads, "a row number per thread, and their number");
+    for (int64_t first = blockIdx.x; first < a.B; first += static_cast<int64_t>(gridDim.x) * S::kThreads) {
+        if (tid == 0) s_bare[S::kThreads] = 0;
+        __syncthreads();
+        const int64_t b = first + static_cast<int64_t>(gridDim.x) * tid;
+        if (b < a.B && a.listed[b] == 0) {
+            s_bare[atomicAdd(&s_bare[S::kThreads], 1)] = static_cast<int32_t>(b);
+        }
+        __syncthreads();
+        const int bare = s_bare[S::kThreads];
+        for (int j = 0; j < bare; ++j) {
+            v4* rows = reinterpret_cast<v4*>(a.out) +
+                       static_cast<uint64_t>(static_cast<uint32_t>(s_bare[j])) * (kM * E / 4);
+            for (int f = tid; f < S::kPieces; f += S::kThreads) {
+                __builtin_nontemporal_store(v4{0.f, 0.f, 0.f, 0.f}, rows + f);
+            }
+        }
+        __syncthreads();   // the list is written again by the next round
+    }
     if (tid <= 27) s_nb[0][tid] = rows_reg;
     rows_reg = fetch_rows(blk + walk.step);
     __syncthreads();
@@ -319,24 +344,14 @@ __global__ __launch_bounds__(kFillBlock) void clear_marks_kernel(uint8_t* __rest
     for (int64_t b = i; b < i + 4 && b < B; ++b) listed[b] = 0;
 }
 
-// Zeroes the rows of the blocks that are not listed, one workgroup per block at
-// a time.
-__global__ __launch_bounds__(kFillBlock) void zero_others_kernel(uint4* __restrict__ out,
-                                                                 const uint8_t* __restrict__ listed,
-                                                                 int64_t B, int64_t units) {
-    for (int64_t b = blockIdx.x; b < B; b += gridDim.x) {
-        if (listed[b]) continue;   // the same for the whole workgroup
-        uint4* rows = out + b * units;
-        for (int64_t u = threadIdx.x; u < units; u += kFillBlock) rows[u] = make_uint4(0u, 0u, 0u, 0u);
-    }
-}
-
 template <int E, int W>
 int launch(const ConvArgs& a, hipStream_t s) {
-    // as many workgroups as the device holds at once: they walk the listing
+    // as many workgroups as the device holds at once: they walk the listing, and
+    // the flags of all blocks
     constexpr auto kernel = convolution_block8_kernel<E, W>;
     int64_t groups = static_cast<int64_t>(compute_units()) * resident_per_cu<kernel>(Shape<E, W>::kThreads);
-    if (groups > a.n_grids) groups = a.n_grids;
+    const int64_t most = a.n_grids > a.B ? a.n_grids : a.B;
+    if (groups > most) groups = most;
     kernel<<<static_cast<unsigned>(groups), Shape<E, W>::kThreads, 0, s>>>(a);
     ASH_LAUNCH_CHECK();
     return 0;
@@ -393,13 +408,9 @@ int ash_convolution_cube(const void* inputs, const void* weights, const int64_t*
                 grid_indices, num_grids, B, listed);
         ASH_LAUNCH_CHECK();
     }
-    zero_others_kernel<<<static_cast<unsigned>(B < 8192 ? B : 8192), kFillBlock, 0, s>>>(
-            static_cast<uint4*>(outputs), listed, B, kM * embedding_dim / 4);
-    ASH_LAUNCH_CHECK();
-    if (num_grids == 0) return 0;
     const ConvArgs a = {static_cast<const float*>(inputs), static_cast<const float*>(weights),
                         grid_indices, lut_grid_nb2grid_idx, static_cast<float*>(outputs),
-                        num_grids, num_embeddings};
+                        listed, num_grids, num_embeddings};
     switch (embedding_dim) {
         case 1: return launch_window<1>(a, window, s);
         case 2: return launch_window<2>(a, window, s);

@@ -171,3 +171,31 @@ def test_ranges_beyond_fp32_resolution_end(gpu_ash, oracle):
     with pytest.raises(RuntimeError, match="step is too small"):
         backend.ray_find_near_far(engine.backend, o.to(DEV), d.to(DEV), lo.to(DEV), hi.to(DEV),
                                   0.0, 1.0e12, 1.0, 8.0)
+
+
+@pytest.mark.parametrize("grid2cell", [8.0, 3.0, 0.7])   # the last: no exact steps, nor recurrence
+@pytest.mark.parametrize("t_min,t_max", [
+    (0.0, 700.0), (0.5, 700.0), (1 / 3, 700.0),          # parameters exact, exact, from the chain
+    (0.0, 2047.0), (0.3, 2044.5), (0.3, 4000.0),         # at the chain's end and beyond it
+    (0.0, 9000.0), (-20.0, 300.0), (5.0, 5.0), (7.0, 1.0), (3.0, 3.1), (90.0, 2.0 ** 22)])
+def test_near_far_in_a_volume_matches_oracle(gpu_ash, oracle, t_min, t_max, grid2cell):
+    """Every way the range goes: two rays per wavefront where its arithmetic is
+    exact, one else.  An odd number of rays, steps of all rounds, rays whose
+    march the box ends and rays whose march t_max ends."""
+    engine, omap, blocks, g = _scene(gpu_ash, oracle, seed=709)
+    n, extent = 4097, 64 * grid2cell
+    o, d = _rays(g, n, extent, blocks * grid2cell / 8)
+    o[::5] *= 6       # many steps until the box ends the march, or outside it at once
+    d[:7] = torch.tensor([[0, 0, 0], [1e-3, 0, 0], [0, -0.0, 1], [float("nan"), 0, 1], [0, float("inf"), 1],
+                          [1e30, 0, 1], [1e-4, 1e-4, -1e-4]])
+    lo, hi = torch.full((3,), -2.0 * extent), torch.full((3,), 7 * extent)
+    if t_max > 1e6:
+        hi = torch.full((3,), extent)
+        d[:7] = d[7:14]
+    want = oracle.ray_find_near_far(omap, o, d, lo, hi, t_min, t_max, 1.0, grid2cell)
+    got = gpu_ash.grid.backend.ray_find_near_far_world(
+        engine.backend, o.to(DEV), d.to(DEV), None, 1.0, lo.to(DEV), hi.to(DEV), t_min, t_max, grid2cell,
+        (0, 64))
+    for a, b in zip(got, want):
+        assert torch.equal(a.cpu(), b)
+    assert t_max - t_min < 10 or t_max > 1e6 or int((want[0] >= 0).sum()) > n // 8

@@ -50,9 +50,9 @@ struct Volume {
 // More than this does not stay in an XCD's L2.
 constexpr int64_t kMaxVolume = int64_t{4} << 20;
 // Making it takes two launches of 4 us each, which so many rays gain back: near
-// and far of 2000 rays 16 -> 16 us, 8000 30 -> 20, 32 768 83 -> 35; samples of
-// 8000 rays 32 - 57 -> 36 - 48 (few blocks and short rays - many and long),
-// 32 768 37 - 77 -> 38 - 55.
+// and far of 3000 rays 15 -> 15 us, 4096 17 -> 14, 8192 29 -> 15, 32 768 79 -> 27;
+// samples of 8000 rays 32 - 57 -> 36 - 48 (few blocks and short rays - many and
+// long), 32 768 37 - 77 -> 38 - 55.
 constexpr int64_t kVolumeRaysNearFar = 4096, kVolumeRaysSampling = 8192;
 
 __host__ __device__ __forceinline__ int64_t volume_bytes(int64_t edge) {
@@ -69,8 +69,9 @@ __device__ __forceinline__ bool in_volume(const Volume& v, const int32_t (&block
         inside = inside && p[a] < v.edge;
     }
     const uint32_t flat = (v.edge + 3) >> 2;
-    at = (((p[2] >> 3) * flat + (p[1] >> 2)) * flat + (p[0] >> 2)) * 128u + (p[0] & 3u) +
-         4u * (p[1] & 3u) + 16u * (p[2] & 7u);
+    // (of a block inside, no factor has more than 24 bits)
+    const uint32_t brick = __umul24(__umul24(p[2] >> 3, flat) + (p[1] >> 2), flat) + (p[0] >> 2);
+    at = (brick << 7) | ((p[2] & 7u) << 4) | ((p[1] & 3u) << 2) | (p[0] & 3u);
     return inside;
 }
 
@@ -94,18 +95,30 @@ __global__ __launch_bounds__(kBlock) void mark_volume_kernel(MapDev m, int ident
     if (in_volume(v, block, at)) to[at] = 1;
 }
 
-// Whether the block is stored, every lane for itself.
-__device__ __forceinline__ bool is_stored(const MapDev& m, const Volume& v, const int32_t (&block)[3],
-                                          bool active) {
-    uint32_t at;
-    const bool inside = in_volume(v, block, at);
-    bool stored = false;
-    if (active && inside) stored = v.at[at] != 0;
-    if (active && !inside) {
-        int32_t idx;
-        stored = find_key_alone<3>(m, block, true, idx);
+// Whether the blocks are stored, every lane for itself: K look-ups per lane, none
+// in a branch, so that all are on their way together; the table is asked only if a
+// block lies outside the volume.
+template <int K>
+__device__ __forceinline__ void are_stored(const MapDev& m, const Volume& v, const int32_t (&block)[K][3],
+                                           const bool (&active)[K], bool (&stored)[K]) {
+    bool inside[K], others = false;
+    uint8_t word[K];
+#pragma unroll
+    for (int h = 0; h < K; ++h) {
+        uint32_t at;
+        inside[h] = in_volume(v, block[h], at) & active[h];
+        word[h] = v.at[inside[h] ? at : 0u];
+        others = others | (active[h] & !inside[h]);
     }
-    return stored;
+#pragma unroll
+    for (int h = 0; h < K; ++h) stored[h] = inside[h] & (word[h] != 0);
+    if (__ballot(others) != 0) {
+#pragma unroll
+        for (int h = 0; h < K; ++h) {
+            int32_t idx;
+            stored[h] = stored[h] | find_key_alone<3>(m, block[h], active[h] & !inside[h], idx);
+        }
+    }
 }
 
 __device__ __forceinline__ void ray_block(const float (&o)[3], const float (&d)[3],
@@ -137,16 +150,25 @@ __device__ __forceinline__ bool is_stored_by_runs(const MapDev& m, const int32_t
 // at the first step that is at or beyond t_max or outside the box, exactly where
 // the sequential loop stops.
 //
-// The kernel is bound by vector instructions.  The parameters are the same for
-// every ray, so the host works the chain of additions out (the same IEEE
-// additions) for the first kChain steps and hands it over with the launch, 64
-// additions per round less; and the recurrence takes `far` from the last hit and
-// `near`, once it is set, only from the number of hits (two instructions each
-// instead of a walk over their parameters).
+// The parameters are the same for every ray, so the host works the chain of
+// additions out (the same IEEE additions) for the first kChain steps and hands it
+// over with the launch, 64 additions per round less; and the recurrence takes
+// `far` from the last hit and `near`, once it is set, only from the number of hits:
+// all its subtractions at once where they are exact (Exact::near_below), else one
+// after the other (two instructions each).
 constexpr int kChain = 512;
 
 struct StepChain {
     float t[kChain];
+};
+
+// What floats hold without rounding, as the host finds it: `near`, as long as it is
+// not negative, minus any number of steps if `near` is at most near_below (both are
+// then whole multiples of the last place of `near`), and, with `steps`, the
+// parameter of every step up to the first at or beyond t_max, t_min + k * step.
+struct Exact {
+    float near_below;
+    bool steps;
 };
 
 template <bool VOLUME>
@@ -154,7 +176,7 @@ __global__ __launch_bounds__(kBlock) void ray_near_far_kernel(
         MapDev m, Volume volume, const float* __restrict__ origins,
         const float* __restrict__ directions, RayUnits u, const float* __restrict__ bbox_min,
         const float* __restrict__ bbox_max, int64_t n, float t_min, float t_max,
-        float grid2cell, float* __restrict__ nears, float* __restrict__ fars, StepChain chain) {
+        float grid2cell, float* __restrict__ nears, float* __restrict__ fars, Exact exact, StepChain chain) {
     const int lane = threadIdx.x & 63;
     const int64_t i = static_cast<int64_t>(blockIdx.x) * (kBlock / 64) + (threadIdx.x >> 6);
     if (i >= n) return;  // whole wavefronts leave together
@@ -176,25 +198,25 @@ __global__ __launch_bounds__(kBlock) void ray_near_far_kernel(
         } else {
             for (int j = 0; j < 64; ++j) t += t_grid_step;
         }
-        int32_t block[3];
+        int32_t block[1][3];
         float x[3];
-        ray_block(o, d, t, cell2grid, block, x);
+        ray_block(o, d, t, cell2grid, block[0], x);
         bool go = t < t_max;
 #pragma unroll
         for (int a = 0; a < 3; ++a) go = go && x[a] >= lo[a] && x[a] <= hi[a];
         const uint64_t stop = __ballot(!go);
         const int first_stop = stop ? __builtin_ctzll(stop) : 64;
-        const bool active = lane < first_stop;
-        bool found;
+        const bool active[1] = {lane < first_stop};
+        bool found[1];
         if constexpr (VOLUME) {
-            found = is_stored(m, volume, block, active);
+            are_stored(m, volume, block, active, found);
         } else {
             // (steps are half a block apart: neighbouring lanes often stand in the
             // same block and share a look-up)
             int32_t idx;
-            found = find_block_by_runs(m, block, active, idx);
+            found[0] = find_block_by_runs(m, block[0], active[0], idx);
         }
-        uint64_t hits = __ballot(found && active);
+        uint64_t hits = __ballot(found[0] && active[0]);
         if (hits) {
             far = fminf(lane_value(t, 63 - __builtin_clzll(hits)) + t_grid_step, t_max);
             if (t_min >= 0.f) {   // near never turns negative again
@@ -203,7 +225,11 @@ __global__ __launch_bounds__(kBlock) void ray_near_far_kernel(
                     near = lane_value(t, __builtin_ctzll(hits));
                     --steps;
                 }
-                for (; steps > 0; --steps) near = fmaxf(near - t_grid_step, t_min);
+                if (uniform(near <= exact.near_below)) {
+                    near = fmaxf(fmaf(static_cast<float>(-steps), t_grid_step, near), t_min);
+                } else {
+                    for (; steps > 0; --steps) near = fmaxf(near - t_grid_step, t_min);
+                }
             } else {
                 while (hits) {
                     const float t_hit = lane_value(t, __builtin_ctzll(hits));
@@ -215,6 +241,86 @@ __global__ __launch_bounds__(kBlock) void ray_near_far_kernel(
         if (first_stop < 64) break;
     }
     if (lane == 0) {
+        nears[i] = __fmul_rn(near, u.cell);
+        fars[i] = __fmul_rn(far, u.cell);
+    }
+}
+
+// The same march for two rays per wavefront, lane j of a ray on steps 64 r + j and
+// 64 r + 32 + j of round r: where the recurrence is exact and a volume stands,
+// t_min is not negative and the parameters are at hand (exact, or all in the
+// chain).  A ray then needs no more than its first and its last hit and their
+// number, and half as many wavefronts wait for their rays' words.  Bound by vector
+// instructions (issued in 0.9 of the cycles): 32 768 rays across 200 000 blocks 22
+// us; 35 a wavefront per ray with the recurrence a hit at a time, 27 with it at once.
+__global__ __launch_bounds__(kBlock) void ray_near_far_pairs_kernel(
+        MapDev m, Volume volume, const float* __restrict__ origins,
+        const float* __restrict__ directions, RayUnits u, const float* __restrict__ bbox_min,
+        const float* __restrict__ bbox_max, int64_t n, float t_min, float t_max,
+        float grid2cell, float* __restrict__ nears, float* __restrict__ fars, Exact exact, StepChain chain) {
+    const int lane = threadIdx.x & 63;
+    const int j = lane & 31, shift = lane & 32;
+    const int64_t pair = static_cast<int64_t>(blockIdx.x) * (kBlock / 64) + (threadIdx.x >> 6);
+    if (2 * pair >= n) return;  // whole wavefronts leave together
+    const int64_t i = 2 * pair + (shift >> 5);
+    const int64_t from = i < n ? i : n - 1;
+    const float cell2grid = static_cast<float>(1.0 / grid2cell);
+    const float t_grid_step = static_cast<float>(grid2cell * 0.5);
+    float o[3], d[3], lo[3], hi[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        o[a] = to_cells(u, origins[from * 3 + a], a);
+        d[a] = directions[from * 3 + a];
+        lo[a] = to_cells(u, bbox_min[a], a);
+        hi[a] = to_cells(u, bbox_max[a], a);
+    }
+    auto parameter = [&](int k) {
+        return exact.steps ? fmaf(static_cast<float>(k), t_grid_step, t_min) : chain.t[k];
+    };
+    bool live = i < n;
+    int hits = 0, first_hit = 0, last_hit = 0;
+    // (without exact steps the chain ends at or beyond t_max)
+    for (int first = 0; exact.steps || first < kChain; first += 64) {
+        uint32_t stop[2], hit[2];
+        bool go[2], found[2];
+        int32_t block[2][3];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const float t = parameter(first + 32 * h + j);
+            float x[3];
+            ray_block(o, d, t, cell2grid, block[h], x);
+            go[h] = live & (t < t_max);
+#pragma unroll
+            for (int a = 0; a < 3; ++a) go[h] = go[h] & (x[a] >= lo[a]) & (x[a] <= hi[a]);
+        }
+        are_stored(m, volume, block, go, found);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint64_t stops = __ballot(!go[h]), stands = __ballot(found[h]);
+            stop[h] = shift != 0 ? static_cast<uint32_t>(stops >> 32) : static_cast<uint32_t>(stops);
+            hit[h] = shift != 0 ? static_cast<uint32_t>(stands >> 32) : static_cast<uint32_t>(stands);
+        }
+        // nothing from the first stop on counts
+        if (stop[0] != 0u) {
+            hit[0] &= (stop[0] & (0u - stop[0])) - 1u;
+            hit[1] = 0u;
+        } else if (stop[1] != 0u) {
+            hit[1] &= (stop[1] & (0u - stop[1])) - 1u;
+        }
+        if ((hit[0] | hit[1]) != 0u) {
+            if (hits == 0) first_hit = first + (hit[0] != 0u ? __ffs(hit[0]) - 1 : 31 + __ffs(hit[1]));
+            last_hit = first + (hit[1] != 0u ? 63 - __clz(hit[1]) : 31 - __clz(hit[0]));
+            hits += __popc(hit[0]) + __popc(hit[1]);
+        }
+        live = live && (stop[0] | stop[1]) == 0u;
+        if (__ballot(live) == 0) break;
+    }
+    if (j == 0 && i < n) {
+        float near = -1.f, far = t_max;
+        if (hits > 0) {
+            near = fmaxf(fmaf(static_cast<float>(1 - hits), t_grid_step, parameter(first_hit)), t_min);
+            far = fminf(parameter(last_hit) + t_grid_step, t_max);
+        }
         nears[i] = __fmul_rn(near, u.cell);
         fars[i] = __fmul_rn(far, u.cell);
     }
@@ -293,18 +399,18 @@ __global__ __launch_bounds__(kBlock) void ray_sample_kernel(
         const float next = at + by;
         // (a step that no longer advances t -- range far beyond fp32 resolution --
         // would never end; the reference has no such guard)
-        const bool stands = live && at < ray_far && at > before;
-        int32_t block[3];
+        const bool stands[1] = {live && at < ray_far && at > before};
+        int32_t block[1][3];
         float x[3];
-        ray_block(o, d, at, cell2grid, block, x);
-        bool stored;
+        ray_block(o, d, at, cell2grid, block[0], x);
+        bool stored[1];
         if constexpr (VOLUME) {
-            stored = is_stored(m, volume, block, stands);
+            are_stored(m, volume, block, stands, stored);
         } else {
-            stored = is_stored_by_runs(m, block, stands);
+            stored[0] = is_stored_by_runs(m, block[0], stands[0]);
         }
-        const uint64_t others = (__ballot(!stands || stored != run_stored) >> shift) & all;
-        const uint64_t ends = (__ballot(!stands) >> shift) & all;
+        const uint64_t others = (__ballot(!stands[0] || stored[0] != run_stored) >> shift) & all;
+        const uint64_t ends = (__ballot(!stands[0]) >> shift) & all;
         // steps taken, and whether the march then stands on the other kind
         const int run = others == 0 ? LPR : __builtin_ctzll(others);
         const bool turn = others != 0 && ((ends >> run) & 1ull) == 0;
@@ -534,6 +640,14 @@ int check_rays(const ash_map_t* map, const float* origins, const float* directio
     return 0;
 }
 
+// The value of the lowest bit set in |x| (zero for zero, infinity and NaN).
+float last_place(float x) {
+    int e = 0;
+    if (!std::isfinite(x) || x == 0.f) return 0.f;
+    const auto digits = static_cast<uint32_t>(std::ldexp(std::frexp(std::fabs(x), &e), 24));
+    return std::ldexp(static_cast<float>(digits & (0u - digits)), e - 24);
+}
+
 int near_far(ash_map_t* map, uint8_t* bytes, int lo, int hi, const float* origins, const float* directions, const RayUnits& units,
              const float* bbox_min, const float* bbox_max, int64_t n, float t_min, float t_max,
              float grid2cell, float* nears, float* fars, hipStream_t s) {
@@ -562,10 +676,18 @@ int near_far(ash_map_t* map, uint8_t* bytes, int lo, int hi, const float* origin
         chain.t[k] = t;
         t += half_block;
     }
-    auto kernel = volume.at != nullptr ? ray_near_far_kernel<true> : ray_near_far_kernel<false>;
-    kernel<<<static_cast<unsigned>((n + kBlock / 64 - 1) / (kBlock / 64)), kBlock, 0, s>>>(
+    const float per_place = 16777216.f;   // 2^24
+    const float unit = last_place(half_block), start = t_min == 0.f ? unit : last_place(t_min);
+    const Exact exact = {unit * per_place,
+                         t_min >= 0.f && t_max + half_block <= (start < unit ? start : unit) * per_place};
+    const bool pairs = volume.at != nullptr && t_min >= 0.f && t_max <= exact.near_below &&
+                       (exact.steps || t >= t_max);
+    const int64_t rays = (kBlock / 64) * (pairs ? 2 : 1);   // per workgroup
+    auto kernel = pairs ? ray_near_far_pairs_kernel
+                        : (volume.at != nullptr ? ray_near_far_kernel<true> : ray_near_far_kernel<false>);
+    kernel<<<static_cast<unsigned>((n + rays - 1) / rays), kBlock, 0, s>>>(
             map->d, volume, origins, directions, units, bbox_min, bbox_max, n, t_min, t_max, grid2cell,
-            nears, fars, chain);
+            nears, fars, exact, chain);
     ASH_LAUNCH_CHECK();
     return 0;
 }

@@ -66,3 +66,25 @@ def test_channels_anywhere_in_their_rows(gpu_ash, stride, sdf, weight):
     apart = grid.surface_mesh(f.contiguous(), w.contiguous(), 0.1, 1.0)
     assert len(triangles) > 1000
     assert torch.equal(triangles, apart[0]) and torch.equal(vertices, apart[1])
+
+
+@pytest.mark.parametrize("light", [0.0, 0.03, 0.12, 0.2, 0.4])   # of the cells weigh too little
+@pytest.mark.parametrize("field", ["checkerboard", "noise"])
+def test_any_number_of_crossed_cells_in_a_block(gpu_ash, field, light):
+    """Triangles are listed 192 crossed cells at a time, 64 a turn: from every
+    cell of a block (light = 0 inside the clump) down to a few."""
+    grid, g = _grid(gpu_ash, 300, False, seed=11)
+    if field == "checkerboard":   # four triangles a cell, the most its code asks for
+        c = torch.arange(8)
+        sign = 1.0 - 2.0 * ((c.view(8, 1, 1) + c.view(1, 8, 1) + c.view(1, 1, 8)) % 2)
+        sdf = sign.reshape(1, 512).repeat(grid.num_embeddings, 1).to(DEV)
+    else:
+        sdf = torch.randn(grid.num_embeddings, 512, generator=g).to(DEV)
+    weights = (torch.rand(sdf.shape, generator=g) >= light).float().to(DEV)
+    triangles, vertices = grid.surface_mesh(sdf, weights, 0.0, 0.5)
+    _, listed = grid._blocks_in_spatial_order()
+    want, points = gpu_ash.grid.backend.marching_cubes(
+        sdf, weights, listed, grid.grid_coords, grid.lut_grid_nb2grid_idx, grid.cell_coords,
+        grid.lut_cell_nb2cell_idx, grid.lut_cell_nb2grid_nb, 8, 0.0, 0.5)
+    assert torch.equal(triangles, want) and torch.equal(vertices, grid.transform_cell_to_world(points))
+    assert len(want) > 300

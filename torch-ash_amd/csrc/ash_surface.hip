@@ -53,9 +53,10 @@ constexpr int64_t kMaxStride = 64;
 // One-wavefront workgroups of a walk over the blocks: several times what the
 // device holds, because blocks differ in work (60 000 blocks, triangles / points /
 // classify: 4096 workgroups 100 / 74 / 37 us, 8192 83 / 52 / 28, 16384 77 / 47 /
-// 28, 65536 91 / 44 / 38, where setting up shows)
+// 28, 65536 91 / 44 / 38, where setting up shows; with a lane per crossed cell and
+// blocks fetched ahead 16384 55 / 48 / 25, 32768 55 / 46 / 28)
 constexpr int kWalkGroups = 16384;
-constexpr int kRoundTriangles = 1024;   // of a block, listed at a time (blocks at a surface have some 250)
+constexpr int kRoundCells = 192;      // crossed cells of a block whose triangles (up to five) are listed at a time
 constexpr uint32_t kRowBits = 0x00FFFFFFu;
 enum Face { kXy, kXz, kYx, kYz, kZx, kZy };   // face of the block, axis of the edges
 
@@ -302,6 +303,46 @@ __device__ __forceinline__ uint32_t lane_up(uint32_t v, int d) {
     return static_cast<uint32_t>(__shfl(static_cast<int>(v), ((threadIdx.x & 63) - d) & 63));
 }
 
+// The sum of the values of the lanes up to this one: every lane takes part, and no
+// step goes through LDS (60 000 blocks, counts 18.3 -> 15.5 us, classify 26 -> 25).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int moved(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
+}
+__device__ __forceinline__ int sum_up_to(int v) {
+    v += moved<0x111, 0xF>(v);   // lanes 1, 2, 4 and 8 before, of the row of 16
+    v += moved<0x112, 0xF>(v);
+    v += moved<0x114, 0xF>(v);
+    v += moved<0x118, 0xF>(v);
+    v += moved<0x142, 0xA>(v);   // the last lane of the row before
+    v += moved<0x143, 0xC>(v);   // and of the lower half
+    return v;
+}
+__device__ __forceinline__ int last_lane(int v) { return __builtin_amdgcn_readlane(v, 63); }
+
+// Lists the crossed cells of a block in order, and the lanes' rows of "below" for
+// case_at; returns their number.  What there is to do for a cell is then done by a
+// lane per cell, some two rounds for a block; by a lane per row, each for its own
+// cells, a round takes as many turns as the longest row has cells (five to eight;
+// 60 000 blocks, 3.9 M triangles: 66 us, 54 this way).
+__device__ __forceinline__ int list_crossed(const RowCells& r, uint2* rows, uint16_t* cells) {
+    const int lane = threadIdx.x & 63;
+    rows[lane] = make_uint2(r.below[0] | (r.below[1] << 16), r.below[2] | (r.below[3] << 16));
+    const int own = __popc(r.crossed);
+    const int upto = sum_up_to(own);
+    const int row0 = (lane & 7) * kG + (lane >> 3) * 64;
+    int at = upto - own;
+    for (uint32_t left = r.crossed; left != 0u; left &= left - 1u) {
+        cells[at++] = static_cast<uint16_t>(row0 + __builtin_ctz(left));
+    }
+    return last_lane(upto);
+}
+__device__ __forceinline__ uint32_t case_at(const uint2* rows, int cell) {
+    const uint2 r = rows[cell >> 3];
+    const uint32_t y0 = r.x >> (cell & 7), y1 = r.y >> (cell & 7);
+    return (y0 & 3u) | ((y0 >> 14) & 12u) | ((y1 & 3u) << 4) | ((y1 >> 10) & 0xC0u);
+}
+
 __global__ __launch_bounds__(64) void classify_kernel(SurfaceArgs a) {
     __shared__ __align__(16) uint8_t s_bits[8 * 128];
     __shared__ uint8_t s_count[256];
@@ -392,8 +433,7 @@ __global__ __launch_bounds__(64) void classify_kernel(SurfaceArgs a) {
         for (uint32_t left = c; left != 0u; left &= left - 1u) {
             triangles += s_count[case_of(r, __builtin_ctz(left))];
         }
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) triangles += __shfl_xor(triangles, d);
+        triangles = last_lane(sum_up_to(triangles));
         if (lane == 0) a.w.local[blk.at] = make_uint2(0u, static_cast<uint32_t>(triangles));
     }
 }
@@ -430,12 +470,7 @@ __global__ __launch_bounds__(kCountThreads) void count_kernel(SurfaceArgs a) {
         if (y == 0) w[k] |= byte(kYx, z) | (byte(kYz, z) << 16);
         if (z == 0) w[k] |= byte(kZx, y) | (byte(kZy, y) << 8);
         const int own = __popc(w[k]);
-        int incl = own;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int up = __shfl_up(incl, d);
-            if (lane >= d) incl += up;
-        }
+        const int incl = sum_up_to(own);
         const int before = incl - own;
         const int layer = __shfl(before, lane & ~7);
         if (g[k] >= 0) {
@@ -449,15 +484,7 @@ __global__ __launch_bounds__(kCountThreads) void count_kernel(SurfaceArgs a) {
         const int64_t b = b0 + lane;
         const int points = s_points[lane];
         const int triangles = b < a.n ? static_cast<int>(a.w.local[b].y) : 0;
-        int p = points, t = triangles;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int up = __shfl_up(p, d), ut = __shfl_up(t, d);
-            if (lane >= d) {
-                p += up;
-                t += ut;
-            }
-        }
+        const int p = sum_up_to(points), t = sum_up_to(triangles);
         if (b < a.n) a.w.local[b] = make_uint2(p - points, t - triangles);
         if (lane == 63) a.w.groups[blockIdx.x] = {p, t};
     }
@@ -602,11 +629,13 @@ __global__ __launch_bounds__(64) void triangles_kernel(SurfaceArgs a) {
     __shared__ uint64_t s_table[256];
     __shared__ uint8_t s_count[256];
     __shared__ uint8_t s_case[kM];
-    __shared__ uint16_t s_triangle[kRoundTriangles];   // cell | number in the cell << 9
+    __shared__ uint2 s_rows[64];
+    __shared__ uint16_t s_triangle[5 * kRoundCells];   // cell | number in the cell << 9
+    uint16_t* const s_cell = reinterpret_cast<uint16_t*>(s_bits);   // (the bits are read by then)
+    static_assert(sizeof(s_bits) >= kM * sizeof(uint16_t), "all cells of a block");
     __shared__ uint32_t s_flags[2 * kRows];               // rows (y, z) of the block and of its +x neighbours
     __shared__ uint32_t s_first[2 * kRows];
     const int lane = threadIdx.x;
-    const int row0 = (lane & 7) * kG + (lane >> 3) * 64;
     for (int i = lane; i < 256; i += 64) {
         s_table[i] = kMcPackedRows[i];
         s_count[i] = static_cast<uint8_t>(kMcTriangleCount[i]);
@@ -621,7 +650,7 @@ __global__ __launch_bounds__(64) void triangles_kernel(SurfaceArgs a) {
         if (blk.own < 0) continue;   // the same for the whole wavefront
         const RowCells r = row_cells(s_bits);
         if (__ballot(r.crossed != 0u) == 0) continue;
-        const int64_t first = a.w.groups[blk.at / kGroupBlocks].triangles + a.w.local[blk.at].y;
+        int64_t first = a.w.groups[blk.at / kGroupBlocks].triangles + a.w.local[blk.at].y;
 #pragma unroll
         for (int k = 0; k < (2 * kRows + 63) / 64; ++k) {
             const int i = k * 64 + lane;
@@ -638,42 +667,34 @@ __global__ __launch_bounds__(64) void triangles_kernel(SurfaceArgs a) {
             s_flags[i] = word & kRowBits;
             s_first[i] = id;
         }
-        int mine = 0;
-        for (uint32_t left = r.crossed; left != 0u; left &= left - 1u) {
-            const int x = __builtin_ctz(left);
-            const uint32_t code = case_of(r, x);
-            s_case[row0 + x] = static_cast<uint8_t>(code);
-            mine += s_count[code];
-        }
-        int at = mine;
+        __syncthreads();   // the block's bits have been read
+        const int crossed = list_crossed(r, s_rows, s_cell);
+        __syncthreads();
+        for (int c0 = 0; c0 < crossed; c0 += kRoundCells) {
+            if (c0 > 0) __syncthreads();   // the previous round's list has been read
+            int listed = 0;
+            for (int c = c0; c < crossed && c < c0 + kRoundCells; c += 64) {
+                const bool any = c + lane < crossed;
+                const int cell = any ? s_cell[c + lane] : 0;
+                const uint32_t code = case_at(s_rows, cell);
+                const int n = any ? s_count[code] : 0;
+                if (any) s_case[cell] = static_cast<uint8_t>(code);
+                const int upto = sum_up_to(n);
+                const int to = listed + upto - n;
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int up = __shfl_up(at, d);
-            if (lane >= d) at += up;
-        }
-        const int total = __shfl(at, 63);
-        at -= mine;
-        for (int q0 = 0; q0 < total; q0 += kRoundTriangles) {
-            if (q0 > 0) __syncthreads();   // the previous round's list has been read
-            int to = at - q0;
-            for (uint32_t left = r.crossed; left != 0u; left &= left - 1u) {
-                const int x = __builtin_ctz(left);
-                const int n = s_count[case_of(r, x)];
-                for (int t = 0; t < n; ++t, ++to) {
-                    if (static_cast<unsigned>(to) < kRoundTriangles) {
-                        s_triangle[to] = static_cast<uint16_t>((row0 + x) | (t << 9));
-                    }
+                for (int t = 0; t < 5; ++t) {
+                    if (t < n) s_triangle[to + t] = static_cast<uint16_t>(cell | (t << 9));
                 }
+                listed += last_lane(upto);
             }
             __syncthreads();
-            const int listed = total - q0 < kRoundTriangles ? total - q0 : kRoundTriangles;
             for (int q = lane; q < listed; q += 64) {
-                if (first + q0 + q >= a.n_triangles) continue;   // never with the totals of the scan
+                if (first + q >= a.n_triangles) continue;   // never with the totals of the scan
                 const int cell = s_triangle[q] & (kM - 1);
                 const int t = s_triangle[q] >> 9;
                 const uint32_t edges = static_cast<uint32_t>(s_table[s_case[cell]] >> (12 * t));
                 const int x = cell & 7, y = (cell >> 3) & 7, z = cell >> 6;
-                int32_t* out = a.triangles + (first + q0 + q) * 3;
+                int32_t* out = a.triangles + (first + q) * 3;
 #pragma unroll
                 for (int v = 0; v < 3; ++v) {
                     // edge e = 4 axis + j starts at the corner made by a zero bit
@@ -689,6 +710,7 @@ __global__ __launch_bounds__(64) void triangles_kernel(SurfaceArgs a) {
                     out[v] = static_cast<int32_t>(s_first[i] + __popc(flags & (before | lower)));
                 }
             }
+            first += listed;
         }
     }
 }

@@ -84,3 +84,48 @@ def test_copies_of_a_key_meet_in_one_freed_slot(gpu_ash, monkeypatch, policy):
         assert len(torch.unique(keys, dim=0)) == len(torch.unique(indices)) == len(near)
         indices, masks = engine.find(near)
         assert bool(masks.all()) and len(torch.unique(indices)) == len(near)
+
+
+def test_refused_keys_leave_slots_that_later_inserts_take(gpu_ash, monkeypatch):
+    """Inserts that do not look for tombstones (none known), into a full map whose
+    refused keys have left some, with copies; then those that do, captured ones
+    and replays among them."""
+    monkeypatch.setattr(common, "BULK_INSERT", "never")
+    near = _keys_near(100, 40, 380, 1)
+    engine = gpu_ash.ASHEngine(3, 330, DEV)
+
+    def stored():
+        keys, indices = engine.items()
+        assert len(torch.unique(keys, dim=0)) == len(torch.unique(indices)) == engine.size()
+        found, masks = engine.find(near)
+        assert int(masks.sum()) == engine.size() == len(torch.unique(found[masks]))
+        return engine.size()
+
+    for _ in range(3):                       # 50 keys are refused each time
+        engine.insert_keys(near.repeat(4, 1))
+        assert stored() == 330
+    for turn in range(4):
+        engine.erase(near[turn * 20:turn * 20 + 200])
+        engine.insert_keys(near[turn * 20 + 30:turn * 20 + 130].repeat(3, 1))
+        assert stored() <= 330
+    engine.erase(near)
+    assert stored() == 0
+    engine.insert_keys(near[:300])
+    assert stored() == 300
+    few = near[250:300].repeat(2, 1)
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    engine.erase(few)
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        engine.backend.insert_keys(few)       # (everything is loaded before the capture)
+        engine.erase(few)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            engine.backend.insert_keys(few)
+    torch.cuda.synchronize()
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert stored() == 300
+        engine.erase(few)
+        assert stored() == 250

@@ -622,7 +622,7 @@ enum { kRecIdle = 0, kRecPlaced = 1, kRecLost = 2 };
 constexpr int kWaitList = 128;
 
 // (four wavefronts per SIMD: the two workgroups that the LDS holds)
-template <bool PROV>
+template <bool PROV, bool TOMBS>
 __global__ __launch_bounds__(kBuildThreads, 4) void build_kernel(
         MapDev m, BulkPlan pl, int stale, int identity) {
     // Records per thread and round.  With rows the partitions of a batch of the
@@ -795,7 +795,7 @@ __global__ __launch_bounds__(kBuildThreads, 4) void build_kernel(
             if (!((which >> k) & 1u)) continue;
             const int lb = static_cast<int>(bucket_of(codes[k], m.nb) - b0);
             const int how = counted ? place_code<false>(tab, codes[k], lb, nbk, wslot[k], nullptr)
-                                    : place_code<true>(tab, codes[k], lb, nbk, wslot[k], &s_reused);
+                                    : place_code<TOMBS>(tab, codes[k], lb, nbk, wslot[k], &s_reused);
             if (how == kFull) atomicAdd(m.ctr + kCtrDropped, 1);   // refused
             state[k] = how == kPlaced ? kRecPlaced : kRecLost;
         }
@@ -1459,7 +1459,8 @@ int ash::insert_bulk(ash_map* map, const int32_t* keys, int64_t n,
         if (launch_split_keys<false>(map, pl, keys, identity, early, stamp, s)) return 1;
         split_records_kernel<false><<<(pl.bins << pl.lane_shift) * pl.chunks, kSplitThreads, 0, s>>>(map->d, pl);
         ASH_LAUNCH_CHECK();
-        build_kernel<false><<<pl.parts, kBuildThreads, 0, s>>>(map->d, pl, stale, identity);
+        auto build = tombs_in(map) ? build_kernel<false, true> : build_kernel<false, false>;
+        build<<<pl.parts, kBuildThreads, 0, s>>>(map->d, pl, stale, identity);
         ASH_LAUNCH_CHECK();
         map->table_stale = false;
         if (none_spilled(publish)) return 1;
@@ -1473,7 +1474,8 @@ int ash::insert_bulk(ash_map* map, const int32_t* keys, int64_t n,
     if (launch_split_keys<true>(map, pl, keys, identity, early, stamp, s)) return 1;
     split_records_kernel<true><<<(pl.bins << pl.lane_shift) * pl.chunks, kSplitThreads, 0, s>>>(map->d, pl);
     ASH_LAUNCH_CHECK();
-    build_kernel<true><<<pl.parts, kBuildThreads, 0, s>>>(map->d, pl, stale, identity);
+    auto build = tombs_in(map) ? build_kernel<true, true> : build_kernel<true, false>;
+    build<<<pl.parts, kBuildThreads, 0, s>>>(map->d, pl, stale, identity);
     ASH_LAUNCH_CHECK();
     map->table_stale = false;
     int64_t words = 0;

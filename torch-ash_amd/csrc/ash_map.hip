@@ -298,7 +298,8 @@ enum InsertMode {
 
 // The insert proper for a key held in registers (`code` is its packed form if
 // `fits`); `i` is the row of the key's value rows / `assigned` / `given` entry.
-template <int DIM, int MODE>
+// TOMBS: the table may hold tombstones (the same for the whole launch).
+template <int DIM, int MODE, bool TOMBS>
 __device__ __forceinline__ void insert_key(
         const MapDev& m, const int32_t (&k)[DIM], uint64_t code, bool fits,
         int64_t i, bool active, const ValueArgs& va,
@@ -318,14 +319,27 @@ __device__ __forceinline__ void insert_key(
     uint32_t wb = 0, gp = 0;
     int ws = 0;
 
-    // Phase A: claim a slot per new key.  First its sequence is followed to the end
-    // (a bucket with an empty slot, or the whole range): a key that is met there is
-    // stored already.
-    bool claiming = false;
-    uint32_t free_slots = 0;   // of the bucket the sequence ended in
+    // Phase A: claim a slot per new key.  Its sequence is followed to the end (a bucket
+    // with an empty slot, or the whole range): a key that is met there is stored
+    // already.  Else it takes the first slot of the sequence that is free, empty or a
+    // tombstone.  Slots are tried in the order of the sequence, and nothing frees a
+    // slot while keys are inserted, so threads that store the same key meet in the
+    // same slot, whatever others have taken in between.
+    // (Tombstones that are left alone pile up: keys that come and go behind a run of
+    // full buckets lengthen it by what they leave each time, until the range is full
+    // and refuses keys.  A million stored keys, 65 537 that come, are read and go:
+    // 125 us a pass, but 1000 - 2700 after sixty passes on one map in twelve.)
+    // One loop with one look at a bucket in it: with a second loop that starts over,
+    // the kernel's instructions take their time to arrive (172 keys 6.9 -> 9.4 us,
+    // 41 000 14.2 -> 16.2); hence the first tombstones met are kept until the end of
+    // the sequence is (172 keys 7.5).  Without TOMBS (the host knows of none) nobody
+    // looks for them, and the buckets on the way have nothing to take.
+    bool claiming = false;   // the sequence has been followed to its end
+    bool reused = false;
+    uint32_t first_tombs = 0, first_b = 0, first_steps = 0;   // in a bucket on the way
     while (__ballot(pend)) {
         ProbeResult p;
-        probe_pass(m, code, b, pend, lane, p);
+        probe_pass<TOMBS>(m, code, b, pend, lane, p);
         if (pend) {
             if (p.status == kProbeFound) {
                 pend = false;
@@ -333,78 +347,54 @@ __device__ __forceinline__ void insert_key(
                     atomicAdd(m.ctr + kCtrLoadDup, 1);
                 }
                 if constexpr (MODE == kInsertReport) seen = p.val;
-            } else if (p.status == kProbeHasEmpty || ++steps >= kPartBuckets) {
-                pend = false;
-                claiming = true;
-                free_slots = p.emask;
             } else {
-                b = next_bucket(b, m.nb);
-            }
-        }
-    }
-    // Then the key takes the first slot of its sequence that is free, empty or a
-    // tombstone (nearly always one of the bucket looked at just now, the
-    // sequence's first).  Slots are tried in the order of the sequence, and
-    // nothing frees a slot while keys are inserted, so threads that store the same
-    // key meet in the same slot, whatever others have taken in between.
-    // (Tombstones that are left alone pile up: keys that come and go behind a run of
-    // full buckets lengthen it by what they leave each time, until the range is full
-    // and refuses keys.  A million stored keys, 65 537 that come, are read and go:
-    // 125 us a pass, but 1000 - 2700 after sixty passes on one map in twelve.)
-    bool looked = steps == 0;   // free_slots are those of bucket b
-    bool reused = false;
-    if (claiming && !looked) {
-        b = bucket_of(code, m.nb);
-        steps = 0;
-    }
-    while (__ballot(claiming)) {
-        ProbeResult p;
-        p.status = kProbeHasEmpty;
-        p.emask = free_slots;
-        p.tmask = 0;
-        if (__ballot(claiming && !looked)) {
-            ProbeResult again;
-            probe_pass<true>(m, code, b, claiming && !looked, lane, again);
-            if (!looked) p = again;
-        }
-        if (claiming) {
-            if (p.status == kProbeFound) {
-                claiming = false;
-                if constexpr (MODE == kInsertLoad) {
-                    atomicAdd(m.ctr + kCtrLoadDup, 1);
-                }
-                if constexpr (MODE == kInsertReport) seen = p.val;
-            }
-            uint32_t em = claiming ? p.emask | p.tmask : 0u;
-            while (em) {
-                const int s = __builtin_ctz(em);
-                const unsigned long long free = (p.tmask >> s) & 1u ? kTomb : kEmpty;
-                const unsigned long long old = atomicCAS(slot_ptr(m, b, s), free, code);
-                if (old == free) {
-                    won = true;
-                    reused = free == kTomb;
-                    wb = b;
-                    ws = s;
-                    claiming = false;
-                    break;
-                }
-                if (old == code) {
-                    claiming = false;
-                    if constexpr (MODE == kInsertLoad) {
-                        atomicAdd(m.ctr + kCtrLoadDup, 1);
+                uint32_t em = p.emask;   // (without TOMBS: of the sequence's last bucket)
+                if constexpr (TOMBS) {
+                    if (!claiming) {
+                        if (first_tombs == 0) {
+                            first_tombs = p.tmask;
+                            first_b = b;
+                            first_steps = steps;
+                        }
+                        claiming = p.status == kProbeHasEmpty || steps + 1 >= kPartBuckets;
+                        if (claiming && first_tombs != 0 && first_steps != steps) {
+                            p.emask = 0;
+                            p.tmask = first_tombs;
+                            b = first_b;
+                            steps = first_steps;
+                        }
                     }
-                    break;
+                    em = claiming ? p.emask | p.tmask : 0u;
                 }
-                em &= em - 1;
-            }
-            if (claiming && !looked) {
-                b = next_bucket(b, m.nb);
-                if (++steps >= kPartBuckets) {
-                    claiming = false;
-                    refused = true;
+                while (em) {
+                    const int s = __builtin_ctz(em);
+                    const unsigned long long free = TOMBS && ((p.tmask >> s) & 1u) ? kTomb : kEmpty;
+                    const unsigned long long old = atomicCAS(slot_ptr(m, b, s), free, code);
+                    if (old == free) {
+                        won = true;
+                        reused = free == kTomb;
+                        wb = b;
+                        ws = s;
+                        pend = false;
+                        break;
+                    }
+                    if (old == code) {
+                        pend = false;
+                        if constexpr (MODE == kInsertLoad) {
+                            atomicAdd(m.ctr + kCtrLoadDup, 1);
+                        }
+                        break;
+                    }
+                    em &= em - 1;
+                }
+                if (pend) {
+                    b = next_bucket(b, m.nb);
+                    if (++steps >= kPartBuckets) {
+                        pend = false;
+                        refused = true;
+                    }
                 }
             }
-            looked = false;   // (the first bucket once more: it may hold tombstones)
         }
     }
     if (active && !fits) {
@@ -426,9 +416,9 @@ __device__ __forceinline__ void insert_key(
     // Phase B: one heap-counter update per block, indices for the winners.
     const bool w = won || gwon;
     int32_t idx = -1;
-    const int nreused = __popcll(__ballot(reused));
+    const int nreused = TOMBS ? __popcll(__ballot(reused)) : 0;
     if constexpr (MODE == kInsertLoad) {
-        if (lane == 0 && nreused > 0) atomicSub(m.ctr + kCtrTombs, nreused);
+        if (TOMBS && lane == 0 && nreused > 0) atomicSub(m.ctr + kCtrTombs, nreused);
         if (w) {
             // the index comes with the key (`given` null: the key's own number,
             // when the keys are the entries of the key log)
@@ -458,7 +448,7 @@ __device__ __forceinline__ void insert_key(
         const int rank = __popcll(wm & ((1ull << lane) - 1ull));
         if (lane == 0) {
             s_cnt[wave] = nw;
-            s_reused[wave] = nreused;
+            if constexpr (TOMBS) s_reused[wave] = nreused;
         }
         __syncthreads();
         if (threadIdx.x == 0) {
@@ -466,7 +456,7 @@ __device__ __forceinline__ void insert_key(
 #pragma unroll
             for (int q = 0; q < kHeapBlock / 64; ++q) {
                 tot += s_cnt[q];
-                again += s_reused[q];
+                if constexpr (TOMBS) again += s_reused[q];
             }
             if (again > 0) atomicSub(m.ctr + kCtrTombs, again);
             int base = 0;
@@ -556,7 +546,7 @@ __device__ __forceinline__ void insert_key(
 
 // One key per thread, every thread of the workgroup calls this together.
 // CODES: `keys` holds packed 64-bit codes instead of int32[DIM] rows.
-template <int DIM, int MODE, bool CODES>
+template <int DIM, int MODE, bool TOMBS, bool CODES>
 __device__ __forceinline__ void insert_one(
         const MapDev& m, const int32_t* __restrict__ keys, int64_t i,
         bool active, const ValueArgs& va, int32_t* __restrict__ assigned,
@@ -571,15 +561,15 @@ __device__ __forceinline__ void insert_one(
         load_key<DIM>(keys, i, active, k);
         fits = pack_key<DIM>(k, code);
     }
-    insert_key<DIM, MODE>(m, k, code, fits, i, active, va, assigned, given);
+    insert_key<DIM, MODE, TOMBS>(m, k, code, fits, i, active, va, assigned, given);
 }
 
-template <int DIM, int MODE>
+template <int DIM, int MODE, bool TOMBS>
 __global__ __launch_bounds__(kHeapBlock) void insert_kernel(
         MapDev m, const int32_t* __restrict__ keys, int64_t n, ValueArgs va,
         int32_t* __restrict__ assigned, const int64_t* __restrict__ given) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * kHeapBlock + threadIdx.x;
-    insert_one<DIM, MODE, false>(m, keys, i, i < n, va, assigned, given);
+    insert_one<DIM, MODE, TOMBS, false>(m, keys, i, i < n, va, assigned, given);
 }
 
 // The counters, left where the host reads them: `landing` is page-locked host
@@ -599,7 +589,7 @@ __device__ __forceinline__ void leave_counters(const int32_t* ctr, int32_t* land
 // The same insert over a selection made on the device: thread t of the
 // selection handles row sel[t], t < *nsel.  The grid is fixed; workgroups
 // stride over the selection, which is empty in the common case.
-template <int DIM, int MODE, bool CODES>
+template <int DIM, int MODE, bool TOMBS, bool CODES>
 __global__ __launch_bounds__(kHeapBlock) void insert_selected_kernel(
         MapDev m, const int32_t* __restrict__ keys,
         const int32_t* __restrict__ sel, const int32_t* __restrict__ nsel,
@@ -610,7 +600,7 @@ __global__ __launch_bounds__(kHeapBlock) void insert_selected_kernel(
         const int64_t t = base + threadIdx.x;
         const bool active = t < total;
         const int64_t i = active ? sel[t] : 0;
-        insert_one<DIM, MODE, CODES>(m, keys, i, active, va, nullptr, nullptr);
+        insert_one<DIM, MODE, TOMBS, CODES>(m, keys, i, active, va, nullptr, nullptr);
         __syncthreads();
     }
     if (publish.landing == nullptr) return;
@@ -697,7 +687,7 @@ __global__ __launch_bounds__(kHeadsBlock) void activate_heads_kernel(
     }
 }
 
-template <bool MARK>
+template <bool MARK, bool TOMBS>
 __global__ __launch_bounds__(kHeapBlock) void activate_kernel(
         MapDev m, const int32_t* __restrict__ heads, int off_lo, int width,
         int bound_lo, int bound_hi, uint8_t* __restrict__ touched,
@@ -725,7 +715,7 @@ __global__ __launch_bounds__(kHeapBlock) void activate_kernel(
         if constexpr (!MARK) {
             uint64_t code;
             const bool fits = pack_key<3>(k, code);
-            insert_key<3, kInsertKeys>(m, k, code, fits, 0, ok, none, nullptr, nullptr);
+            insert_key<3, kInsertKeys, TOMBS>(m, k, code, fits, 0, ok, none, nullptr, nullptr);
             __syncthreads();
         } else {
             int32_t idx = 0;
@@ -786,6 +776,7 @@ constexpr int kDistinctSlots = 2048;     // two LDS slots per candidate of a chu
 // and the row is flagged at once; a key that another thread is storing at
 // that moment is flagged by that thread, which is handed the index.  No second
 // launch has to wait for the indices to settle.
+template <bool TOMBS>
 __global__ __launch_bounds__(kHeapBlock) void activate_runs_kernel(
         MapDev m, RunsArgs a, uint8_t* __restrict__ touched, int32_t* __restrict__ coords) {
     __shared__ unsigned long long s_set[kDistinctSlots];
@@ -874,7 +865,7 @@ __global__ __launch_bounds__(kHeapBlock) void activate_runs_kernel(
             uint64_t code;
             const bool fits = pack_key<3>(k, code);
             int32_t row = -1;
-            insert_key<3, kInsertReport>(m, k, code, fits, 0, ok, none, nullptr, nullptr, &row);
+            insert_key<3, kInsertReport, TOMBS>(m, k, code, fits, 0, ok, none, nullptr, nullptr, &row);
             if (ok && row >= 0) {
                 touched[row] = 1;
                 coords[static_cast<int64_t>(row) * 3 + 0] = k[0];
@@ -1949,7 +1940,7 @@ __global__ __launch_bounds__(kHeapBlock) void replace_from_log_kernel(MapDev m, 
         const int64_t i = first + threadIdx.x;
         const uint64_t code = i < limit ? m.klog[i] : kEmpty;
         const int32_t k[1] = {0};
-        insert_key<1, kInsertLoad>(m, k, code, true, i, code < kTomb, none, nullptr, nullptr);
+        insert_key<1, kInsertLoad, false>(m, k, code, true, i, code < kTomb, none, nullptr, nullptr);
     }
 }
 
@@ -2217,29 +2208,41 @@ int give_up_heap_order(ash_map* map, hipStream_t s) {
 
 namespace {
 
+template <int MODE, bool TOMBS>
+int launch_insert_to(ash_map* map, const int32_t* keys, int64_t n,
+                     const ValueArgs& va, int32_t* assigned, const int64_t* given,
+                     hipStream_t s) {
+    const unsigned g = grid_for(n, kHeapBlock);
+    auto kernel = map->key_dim == 1   ? insert_kernel<1, MODE, TOMBS>
+                  : map->key_dim == 2 ? insert_kernel<2, MODE, TOMBS>
+                  : map->key_dim == 3 ? insert_kernel<3, MODE, TOMBS>
+                                      : insert_kernel<4, MODE, TOMBS>;
+    kernel<<<g, kHeapBlock, 0, s>>>(map->d, keys, n, va, assigned, given);
+    ASH_LAUNCH_CHECK();
+    return 0;
+}
+
 template <int MODE>
 int launch_insert(ash_map* map, const int32_t* keys, int64_t n,
                   const ValueArgs& va, int32_t* assigned, const int64_t* given,
                   hipStream_t s) {
-    const unsigned g = grid_for(n, kHeapBlock);
-    switch (map->key_dim) {
-        case 1:
-            insert_kernel<1, MODE><<<g, kHeapBlock, 0, s>>>(map->d, keys, n, va,
-                                                        assigned, given);
-            break;
-        case 2:
-            insert_kernel<2, MODE><<<g, kHeapBlock, 0, s>>>(map->d, keys, n, va,
-                                                        assigned, given);
-            break;
-        case 3:
-            insert_kernel<3, MODE><<<g, kHeapBlock, 0, s>>>(map->d, keys, n, va,
-                                                        assigned, given);
-            break;
-        default:
-            insert_kernel<4, MODE><<<g, kHeapBlock, 0, s>>>(map->d, keys, n, va,
-                                                        assigned, given);
-            break;
-    }
+    return tombs_in(map) ? launch_insert_to<MODE, true>(map, keys, n, va, assigned, given, s)
+                         : launch_insert_to<MODE, false>(map, keys, n, va, assigned, given, s);
+}
+
+template <int MODE, bool TOMBS>
+int launch_selected_to(ash_map* map, bool codes, const int32_t* keys,
+                       const int32_t* sel, const int32_t* nsel,
+                       const ValueArgs& va, hipStream_t s, const Publish& publish) {
+    // the selection is empty or short as a rule: a grid that costs little to
+    // launch, whose workgroups stride over a long one
+    constexpr unsigned g = 128;
+    auto kernel = codes               ? insert_selected_kernel<1, MODE, TOMBS, true>
+                  : map->key_dim == 1 ? insert_selected_kernel<1, MODE, TOMBS, false>
+                  : map->key_dim == 2 ? insert_selected_kernel<2, MODE, TOMBS, false>
+                  : map->key_dim == 3 ? insert_selected_kernel<3, MODE, TOMBS, false>
+                                      : insert_selected_kernel<4, MODE, TOMBS, false>;
+    kernel<<<g, kHeapBlock, 0, s>>>(map->d, keys, sel, nsel, va, publish);
     ASH_LAUNCH_CHECK();
     return 0;
 }
@@ -2248,34 +2251,8 @@ template <int MODE>
 int launch_selected(ash_map* map, bool codes, const int32_t* keys,
                     const int32_t* sel, const int32_t* nsel,
                     const ValueArgs& va, hipStream_t s, const Publish& publish) {
-    // the selection is empty or short as a rule: a grid that costs little to
-    // launch, whose workgroups stride over a long one
-    constexpr unsigned g = 128;
-    if (codes) {
-        insert_selected_kernel<1, MODE, true>
-                <<<g, kHeapBlock, 0, s>>>(map->d, keys, sel, nsel, va, publish);
-    } else {
-        switch (map->key_dim) {
-            case 1:
-                insert_selected_kernel<1, MODE, false>
-                        <<<g, kHeapBlock, 0, s>>>(map->d, keys, sel, nsel, va, publish);
-                break;
-            case 2:
-                insert_selected_kernel<2, MODE, false>
-                        <<<g, kHeapBlock, 0, s>>>(map->d, keys, sel, nsel, va, publish);
-                break;
-            case 3:
-                insert_selected_kernel<3, MODE, false>
-                        <<<g, kHeapBlock, 0, s>>>(map->d, keys, sel, nsel, va, publish);
-                break;
-            default:
-                insert_selected_kernel<4, MODE, false>
-                        <<<g, kHeapBlock, 0, s>>>(map->d, keys, sel, nsel, va, publish);
-                break;
-        }
-    }
-    ASH_LAUNCH_CHECK();
-    return 0;
+    return tombs_in(map) ? launch_selected_to<MODE, true>(map, codes, keys, sel, nsel, va, s, publish)
+                         : launch_selected_to<MODE, false>(map, codes, keys, sel, nsel, va, s, publish);
 }
 
 }  // namespace
@@ -2750,10 +2727,11 @@ int launch_activate(ash_map_t* map, const float* cells, int64_t n, int grid_dim,
     int64_t blocks = (n * width * width * width + kHeapBlock - 1) / kHeapBlock;
     if (blocks > 2048) blocks = 2048;
     const unsigned gb = static_cast<unsigned>(blocks);
-    activate_kernel<false><<<gb, kHeapBlock, 0, s>>>(
+    auto insert = tombs_in(map) ? activate_kernel<false, true> : activate_kernel<false, false>;
+    insert<<<gb, kHeapBlock, 0, s>>>(
             map->d, heads, lo, width, bound_lo, bound_hi, touched, coords);
     ASH_LAUNCH_CHECK();
-    activate_kernel<true><<<gb, kHeapBlock, 0, s>>>(
+    activate_kernel<true, false><<<gb, kHeapBlock, 0, s>>>(
             map->d, heads, lo, width, bound_lo, bound_hi, touched, coords);
     ASH_LAUNCH_CHECK();
     return 0;
@@ -2844,8 +2822,8 @@ int ash_grid_activate_positions(ash_map_t* map, const float* positions, int64_t 
     a.bound_hi = bound_hi;
     const int64_t groups = (n + kRunPositions - 1) / kRunPositions;
     if (groups > 0x7FFFFFFFll) ASH_FAIL("too many positions in one call");
-    activate_runs_kernel<<<static_cast<unsigned>(groups), kHeapBlock, 0, s>>>(
-            map->d, a, touched, coords);
+    auto kernel = tombs_in(map) ? activate_runs_kernel<true> : activate_runs_kernel<false>;
+    kernel<<<static_cast<unsigned>(groups), kHeapBlock, 0, s>>>(map->d, a, touched, coords);
     ASH_LAUNCH_CHECK();
     return 0;
 }

@@ -189,6 +189,10 @@ class Answer {
 // The map's own page-locked words (made on first use), and the wait for one of them.
 int take_line(ash_map* map);
 int wait_for_stamp(const int32_t* word, int32_t stamp);
+// May the table hold tombstones, for an insert?  (Replays of a captured launch meet
+// any table; refused keys whose counters nobody has read yet may have left some,
+// which then wait for a later insert.)
+inline bool tombs_in(const ash_map* map) { return map->maybe_tombstones || map->replayed; }
 // Waits for the counters that a launch may still owe at kLineLate.
 int settle_landing_place(ash_map* map);
 // Adds up `n` words of `counts` into the counter of touched blocks and queues the

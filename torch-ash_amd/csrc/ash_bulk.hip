@@ -492,8 +492,8 @@ enum { kPlaced = 0, kKnown = 1, kFull = 2 };
 // ash_map.hip).  kPlaced: the calling thread owns slot `where` (local bucket * 16
 // + slot) now; kKnown: the code was there already (or another thread of this round
 // placed it); kFull: every bucket of the partition has been visited.  `reused`
-// counts tombstones that hold a key now; a range that started empty has none
-// (TOMBS false).
+// counts tombstones that hold a key now (TOMBS false: a range that started empty,
+// or a table that is known to have none).
 template <bool TOMBS>
 __device__ __forceinline__ int place_code(uint4* tab, uint64_t code, int lb, int nbk,
                                           int& where, int* reused) {

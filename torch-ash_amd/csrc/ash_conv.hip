@@ -16,8 +16,8 @@
 // 60 000 blocks: five channels 3^3 347 us a call (440 before one wavefront each, 1275
 // with tables and instances for powers of two), two channels 126 (501); 1000
 // blocks, 7^3: 94 (990: every workgroup used to check the tables).  3^3 windows of
-// five channels move 1.56 GB beyond the L2s, 4.5 TB/s: 0.61 GB of results and 0.95
-// of rows, 1.5 times what there are (the halo along x takes most lines of two
+// five channels move 1.47 GB beyond the L2s, 4.3 TB/s: 0.61 GB of results and 0.86
+// of rows, 1.4 times what there are (the halo along x takes most lines of two
 // neighbours); vector instructions are issued in 0.59 of the cycles, the LDS is
 // busy in 0.54.  7^3 windows of two channels are bound by vector instructions
 // (0.87 of the cycles; 1941 per wavefront and block, 1372 of them multiply-adds

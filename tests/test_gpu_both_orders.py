@@ -83,6 +83,7 @@ def scene(gpu_ash, monkeypatch):
     x = workloads.ray_queries(grid, radii, centres, num_rays=64, samples_per_ray=30)
     backend = gpu_ash.grid_query.backend
     put_off, real = [], backend.query_backward_backward
+    monkeypatch.setattr(gpu_ash.grid_query, "PUT_OFF_FROM", 0)
     monkeypatch.setattr(backend, "query_backward_backward",
                         lambda *a, **k: (put_off.append(k.get("later", False)), real(*a, **k))[1], raising=False)
     return gpu_ash, grid, x, put_off
@@ -183,3 +184,15 @@ def test_a_gradient_recorded_under_another_stream(scene):
     del put_off[:]
     # (recorded on the forward's stream all the same)
     assert _close(_grad(grid, value + norm), want) and put_off == [True]
+
+
+@pytest.mark.parametrize("more", [0, -1])
+def test_few_queries_are_not_put_off(scene, monkeypatch, more):
+    ash, grid, x, put_off = scene
+    monkeypatch.setattr(ash.grid_query, "PUT_OFF_FROM", len(x) - more)
+    want = _separately(grid, x, (0, 2))
+    del put_off[:]
+    xq = x.clone().requires_grad_(True)
+    y, _ = grid(xq, "smooth_step")
+    got = _grad(grid, (y**2).mean() + _norm_loss(y, xq, 0) + _norm_loss(y, xq, 2))
+    assert put_off == [more == 0] * 2 and _close(got, want)

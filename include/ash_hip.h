@@ -573,11 +573,15 @@ int ash_map_find_rows(ash_map_t* map, const int32_t* keys, int64_t n, int n_valu
                       const int64_t* src_rows, int zero_misses, int64_t* indices,
                       uint8_t* masks, void* stream);
 
-/* The same with scratch memory: batches of a million keys and more that read two
+/* The same with scratch memory: batches of 2^21 keys and more that read two
  * tables or more look the keys up first and read the rows in the tables' order
- * then.  ash_map_find_rows_scratch_bytes says how much memory that takes for
- * such a call, 0 where it is no gain; a call with none, less, or memory that is
- * not 16-byte aligned reads the rows key by key.  The results are the same. */
+ * then, 4096 keys at a time where enough of them are stored.
+ * ash_map_find_rows_scratch_bytes says how much memory that takes for such a call
+ * (some 6 bytes per key and its row once more), 0 where it is no gain: tables of
+ * less than 16 MB, rows of more than 32 bytes together, few keys for the tables'
+ * rows (a quarter of them for rows of up to 16 bytes, as many for wider ones, less
+ * again from 900 MB of tables on).  A call with none, less, or memory that is not
+ * 16-byte aligned reads the rows key by key.  The results are the same. */
 int64_t ash_map_find_rows_scratch_bytes(const ash_map_t* map, int64_t n, int n_values,
                                         const int64_t* row_bytes, const int64_t* src_rows);
 int ash_map_find_rows_scratch(ash_map_t* map, const int32_t* keys, int64_t n, int n_values,

@@ -163,3 +163,53 @@ def test_rows_of_large_batches_in_index_order(gpu_ash, dim, n, widths, alike):
             assert torch.equal(r, torch.cat([p[2][v] for p in parts]))
     none, got_m, again = gpu_ash.core.backend.find_rows(engine.backend, q, tables, zero_misses=True, need_indices=False)
     assert none is None and all(torch.equal(a, b) for a, b in zip(again, got))
+
+
+@pytest.mark.parametrize("n", [2_400_257, 2_400_257 + 511])   # a last chunk of 1 and of 512 queries
+@pytest.mark.parametrize("widths", [(1, 1), (3, 1), (4, 3), (4, 4)])
+def test_chunks_of_few_stored_keys_are_served_key_by_key(gpu_ash, widths, n):
+    """Rows in index order, from one chunk of 4096 queries to the next: none, all and
+    a share next to every bound (three, four, six and seven eighths) of the keys are
+    stored."""
+    g = torch.Generator(device=DEV).manual_seed(n)
+    rows = 2_300_000
+    at = torch.arange(rows, device=DEV)
+    keys = torch.stack([at & 1023, (at >> 10) & 1023, at >> 20], 1).int()
+    engine = gpu_ash.ASHEngine(3, rows, DEV)
+    engine.insert_keys(keys)
+    q = keys[torch.randint(rows, (n,), generator=g, device=DEV)]
+    stored = torch.tensor([0, 1535, 1536, 2047, 2048, 3071, 3072, 3583, 3584, 4095, 4096], device=DEV)
+    of = torch.arange(n, device=DEV)
+    chunk, place = of // 4096, of % 4096
+    q[(place * 1237 % 4096) >= stored[chunk % len(stored)], 0] += 4096
+    tables = [torch.randint(1 << 30, (rows, w), generator=g, device=DEV, dtype=torch.int32) for w in widths]
+    row_bytes, src_rows = ((ctypes.c_int64 * len(widths))(*each) for each in
+                           ((4 * w for w in widths), (len(t) for t in tables)))
+    assert gpu_ash.common.load_library().ash_map_find_rows_scratch_bytes(
+        engine.backend._address, n, len(widths), row_bytes, src_rows) > 0
+    for zero_misses in (False, True):
+        got_i, got_m, got = gpu_ash.core.backend.find_rows(engine.backend, q, tables, zero_misses=zero_misses)
+        parts = [gpu_ash.core.backend.find_rows(engine.backend, p, tables, zero_misses=zero_misses)
+                 for p in q.split(500_000)]
+        assert torch.equal(got_i, torch.cat([p[0] for p in parts]))
+        assert torch.equal(got_m, torch.cat([p[1] for p in parts]))
+        for v, r in enumerate(got):
+            assert torch.equal(r, torch.cat([p[2][v] for p in parts]))
+
+
+@pytest.mark.parametrize("widths,rows,queries", [   # the least number of queries, None: never
+    ((1, 1), 12_000_000, 3_000_000), ((3, 1), 12_000_000, 3_000_000), ((3, 2), 12_000_000, 12_000_000),
+    ((4, 4), 12_000_000, 12_000_000), ((3, 3), 41_000_000, 10_250_000), ((4, 4), 31_000_000, 15_500_000),
+    ((3, 1), 4_000_000, 1 << 21), ((3, 1), 1_000_000, None), ((4, 5), 4_000_000, None), ((4,), 12_000_000, None)])
+def test_which_batches_read_rows_in_index_order(gpu_ash, widths, rows, queries):
+    engine = gpu_ash.ASHEngine(3, 100, DEV)
+    row_bytes, src_rows = ((ctypes.c_int64 * len(widths))(*each) for each in
+                           ((4 * w for w in widths), (rows for w in widths)))
+
+    def scratch(n):
+        return gpu_ash.common.load_library().ash_map_find_rows_scratch_bytes(
+            engine.backend._address, n, len(widths), row_bytes, src_rows)
+
+    assert scratch((queries or 100_000_000) - 1) == 0
+    # an index and a place per query, its rows, and little beside them
+    assert queries is None or 0 < scratch(queries) < queries * (7 + 4 * sum(widths))

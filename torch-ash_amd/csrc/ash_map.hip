@@ -1463,29 +1463,11 @@ __device__ __forceinline__ void copy_found_rows(const Unit* __restrict__ src, Un
     }
 }
 
-// find and the gather of the rows in one launch: the indices never travel
-// through memory unless the caller wants them, and the line of a key's bucket
-// and the lines of its rows are asked for by the same wavefront.  16 M keys
-// with rows of 12 and 4 bytes: see the table of the design notes.
-template <int DIM>
-__global__ __launch_bounds__(kBlock) void find_rows_kernel(
-        MapDev m, const int32_t* __restrict__ keys, int64_t n, RowTables tabs, int miss_row,
-        int64_t* __restrict__ idx_out, uint8_t* __restrict__ mask_out) {
+// ... and of all tables, for the wavefront's keys first .. first + 63 of n.
+__device__ __forceinline__ void copy_rows_of_wave(const RowTables& tabs, int32_t from, int64_t first, int64_t n) {
     typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-    const bool active = i < n;
-    int32_t k[DIM];
-    load_key<DIM>(keys, i, active, k);
-    int32_t res = 0;
-    const bool found = find_key<DIM>(m, k, active, res);
-    if (active) {
-        if (idx_out != nullptr) idx_out[i] = found ? static_cast<int64_t>(res) : 0;
-        if (mask_out != nullptr) mask_out[i] = found ? 1 : 0;
-    }
-    const int64_t first = i - (threadIdx.x & 63);
     if (first >= n) return;   // whole wavefronts leave together
     const int rows = n - first < 64 ? static_cast<int>(n - first) : 64;
-    const int32_t from = found ? res : miss_row;
     for (int v = 0; v < tabs.n; ++v) {
         const uint32_t units = tabs.units[v];
         const size_t at = static_cast<size_t>(first) * units;
@@ -1498,6 +1480,27 @@ __global__ __launch_bounds__(kBlock) void find_rows_kernel(
                                       tabs.magic[v], tabs.src_rows[v], from, rows);
         }
     }
+}
+
+// find and the gather of the rows in one launch: the indices never travel
+// through memory unless the caller wants them, and the line of a key's bucket
+// and the lines of its rows are asked for by the same wavefront.  16 M keys
+// with rows of 12 and 4 bytes: see the table of the design notes.
+template <int DIM>
+__global__ __launch_bounds__(kBlock) void find_rows_kernel(
+        MapDev m, const int32_t* __restrict__ keys, int64_t n, RowTables tabs, int miss_row,
+        int64_t* __restrict__ idx_out, uint8_t* __restrict__ mask_out) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    const bool active = i < n;
+    int32_t k[DIM];
+    load_key<DIM>(keys, i, active, k);
+    int32_t res = 0;
+    const bool found = find_key<DIM>(m, k, active, res);
+    if (active) {
+        if (idx_out != nullptr) idx_out[i] = found ? static_cast<int64_t>(res) : 0;
+        if (mask_out != nullptr) mask_out[i] = found ? 1 : 0;
+    }
+    copy_rows_of_wave(tabs, found ? res : miss_row, i - (threadIdx.x & 63), n);
 }
 
 // ------------------------------------- look-up with rows, rows in index order
@@ -1514,6 +1517,7 @@ __global__ __launch_bounds__(kBlock) void find_rows_kernel(
 //      side by side to the indices' places (the workgroups of an XCD stand in
 //      one or two parts at a time, see gather_parts_kernel);
 //   3. per chunk: the rows, read through, dealt to the queries from LDS.
+// A chunk with few stored keys gets its rows key by key in pass 1 (plan_row_sort).
 // The look-up keeps its one random line per key; everything else streams: 2 + 4
 // bytes per key out, 4 + row in, row out, 2 + row in.  Chunks own their regions, so
 // there is nothing to count beforehand and nothing that can overflow, whatever the
@@ -1534,23 +1538,26 @@ constexpr int kSortMaxWords = 8;                        // of a query's rows, al
 constexpr int kSortRuns = 8;                            // chunks per wavefront of pass 2
 constexpr int kSortAhead = 4;                           // groups of 64 records in flight there
 constexpr uint32_t kNoPlace = 0xFFFFu;
+// the last word of a chunk's bounds: a part of it is longer than kSortLongest; pass 1
+// has written its rows
+enum : uint16_t { kBoundsLong = 1, kBoundsServed = 2 };
 
 struct RowSort {
     int64_t n;
     uint32_t chunks;
     uint32_t scale;       // part of index i: umulhi(i, scale)
     uint32_t words;       // of a query's rows
+    int eighths;          // a chunk with fewer eighths of its keys stored is served key by key
     int32_t* index;       // chunks * kSortChunk, a chunk's in part order
     uint16_t* place;      // n
-    uint16_t* bounds;     // chunks * kSortBounds: where a chunk's parts start, its end, and
-                          // whether a part of it is longer than kSortLongest
+    uint16_t* bounds;     // chunks * kSortBounds: where a chunk's parts start, its end, kBounds*
     uint32_t* rows;       // chunks * kSortChunk * words
 };
 
 template <int DIM>
 __global__ __launch_bounds__(kSortThreads) void find_sort_kernel(
-        MapDev m, const int32_t* __restrict__ keys, RowSort sort, int64_t* __restrict__ idx_out,
-        uint8_t* __restrict__ mask_out) {
+        MapDev m, const int32_t* __restrict__ keys, RowSort sort, RowTables tabs, int miss_row,
+        int64_t* __restrict__ idx_out, uint8_t* __restrict__ mask_out) {
     static_assert(kSortChunk <= 0xFFFF, "places and bounds are 16-bit words");
     __shared__ int32_t s_index[kSortChunk];
     __shared__ uint32_t s_where[kSortChunk];   // part << 16 | rank within the part
@@ -1563,6 +1570,7 @@ __global__ __launch_bounds__(kSortThreads) void find_sort_kernel(
     static_assert(kSortParts <= kSortThreads, "a thread per part");
     if (tid < kSortParts) s_count[tid] = 0;
     __syncthreads();
+    uint16_t* bounds = sort.bounds + static_cast<int64_t>(blockIdx.x) * kSortBounds;
 #pragma unroll 1
     for (int j = 0; j < kSortKeys; ++j) {
         const int64_t i = base + j * kSortThreads + tid;
@@ -1604,7 +1612,17 @@ __global__ __launch_bounds__(kSortThreads) void find_sort_kernel(
         if (w < (tid >> 6)) first += s_wave[w];
         total += s_wave[w];
     }
-    uint16_t* bounds = sort.bounds + static_cast<int64_t>(blockIdx.x) * kSortBounds;
+    const int queries = sort.n - base < kSortChunk ? static_cast<int>(sort.n - base) : kSortChunk;
+    if (total * 8 < sort.eighths * queries) {
+        // the chunk's rows key by key; the other passes find nothing of it
+        if (tid < kSortBounds) bounds[tid] = tid == kSortParts + 1 ? kBoundsServed : 0;
+#pragma unroll 1
+        for (int j = 0; j < kSortKeys; ++j) {
+            const int q = j * kSortThreads + tid;
+            copy_rows_of_wave(tabs, s_where[q] != ~0u ? s_index[q] : miss_row, base + (q & ~63), sort.n);
+        }
+        return;
+    }
     if (tid < kSortParts) {
         s_first[tid] = first;
         bounds[tid] = static_cast<uint16_t>(first);
@@ -1612,7 +1630,7 @@ __global__ __launch_bounds__(kSortThreads) void find_sort_kernel(
     const int longer = __syncthreads_or(count > static_cast<int>(kSortLongest));
     if (tid == 0) {
         bounds[kSortParts] = static_cast<uint16_t>(total);
-        bounds[kSortParts + 1] = longer ? 1 : 0;
+        bounds[kSortParts + 1] = longer ? kBoundsLong : 0;
     }
 #pragma unroll
     for (int j = 0; j < kSortKeys; ++j) {
@@ -1726,6 +1744,7 @@ __global__ __launch_bounds__(kDealThreads) void deal_rows_kernel(RowTables tabs,
     const int64_t base = static_cast<int64_t>(blockIdx.x) * kSortChunk;
     const uint32_t queries = sort.n - base < kSortChunk ? static_cast<uint32_t>(sort.n - base) : kSortChunk;
     const uint16_t* bounds = sort.bounds + static_cast<int64_t>(blockIdx.x) * kSortBounds;
+    if (bounds[kSortParts + 1] == kBoundsServed) return;
     const uint32_t found = bounds[kSortParts], total = found * sort.words;
     const uint32_t* rows = sort.rows + static_cast<size_t>(base) * sort.words;
     // (whole pieces: a chunk's region is kSortChunk rows long)
@@ -1734,7 +1753,7 @@ __global__ __launch_bounds__(kDealThreads) void deal_rows_kernel(RowTables tabs,
     }
     for (uint32_t t = threadIdx.x; t < queries; t += kDealThreads) s_place[t] = sort.place[base + t];
     __syncthreads();
-    if (bounds[kSortParts + 1] != 0) {
+    if (bounds[kSortParts + 1] == kBoundsLong) {
         // rows that pass 2 has left: queries that crowd in few parts, and so in the caches
         for (uint32_t t = threadIdx.x; t < found; t += kDealThreads) {
             const int32_t kept = sort.index[base + t];
@@ -2326,19 +2345,35 @@ int insert_selected(ash_map* map, bool codes, const void* keys,
 
 namespace {
 
-// When the rows are read in index order, and what that takes.  Measured (keys
-// found, key by key -> in index order, us):
+// When the rows are read in index order, and what that takes.  Measured (key by
+// key -> in index order, us; keys stored unless said otherwise):
 //   two tables or more; of one (rows of 12 bytes) the passes cost what its lines do
 //   2 M queries and more: rows of 12 + 4 bytes, 1.5 M rows: 1 M queries 46 -> 58,
 //     2 M 90 -> 81, 4 M 183 -> 151, 8 M 374 -> 280
-//   a quarter of the tables' rows and more, fewer share no lines in a part: 12 M
-//     rows: 2 M queries 118 -> 117, 4 M 234 -> 217, 8 M 467 -> 366; 24 M rows: 4 M
-//     236 -> 238, 8 M 471 -> 399, 16 M 942 -> 734
 //   16 MB of tables: 6 MB (of which an XCD's L2 holds most) and 4 M queries 111 ->
 //     123, 12 MB 200 -> 173
+//   queries per row of the tables, of which fewer share no lines in a part: for rows
+//     of up to 16 bytes together a quarter (400 MB of tables: 8 bytes 743 -> 610, 16
+//     bytes 391 -> 359), for wider ones one (400 MB: a half 20 bytes 617 -> 583, 24
+//     bytes 510 -> 513, 32 bytes 403 -> 427; one 1185 -> 1052, 1014 -> 948, 768 ->
+//     774).  From 900 MB of tables on, where a random line costs a translation as
+//     well, a quarter does for rows of up to 24 bytes (1 GB: 781 -> 706) and a half
+//     for 32 (a quarter 572 -> 587, a half 1132 -> 1042).  Parts that an L2 does not
+//     hold are no loss there: 3 GB, rows of 16 bytes 3747 -> 3079.
 //   rows of up to kSortMaxWords words together: a chunk's have to fit the LDS.
+// A key that is not stored costs key by key only the line of its bucket.  Pass 1 hence
+// counts a chunk's stored keys, and below a share of them serves the chunk itself: of
+// 8 bytes three eighths (400 MB, 25 M queries: four tenths stored 1036 -> 962, three
+// 946 -> 1027), of 16 a half (seven tenths 623 -> 591, a half 536 -> 551), of wider
+// ones seven eighths, six from 900 MB on.  What is left of the passes costs such a
+// chunk 2 - 12 % over key by key while three tenths of its keys are stored (22 % where
+// the call takes 0.1 - 0.2 ms) and up to 30 % (a tenth of a millisecond at 25 M) where
+// next to none is; through all three passes that was 45 %.
+// (Looking at a chunk's first 512 keys and then going key by key at once: the
+// registers of both ways together cost 10 - 40 %.)
 constexpr int64_t kSortMinQueries = int64_t{1} << 21;
 constexpr int64_t kSortMinBytes = int64_t{16} << 20;
+constexpr int64_t kSortFarBytes = int64_t{900} << 20;
 
 int64_t plan_row_sort(int64_t n, int n_values, const int64_t* row_bytes, const int64_t* src_rows,
                       void* scratch, RowSort* sort) {
@@ -2351,7 +2386,9 @@ int64_t plan_row_sort(int64_t n, int n_values, const int64_t* row_bytes, const i
         rows = std::max(rows, src_rows[v]);
         table_bytes += row_bytes[v] * src_rows[v];
     }
-    if (words > kSortMaxWords || rows <= kSortParts || n < rows / 4 || table_bytes < kSortMinBytes) return 0;
+    if (words > kSortMaxWords || rows <= kSortParts || table_bytes < kSortMinBytes) return 0;
+    const bool far = table_bytes >= kSortFarBytes;
+    if (n < (words <= 4 || (far && words <= 6) ? rows / 4 : far ? rows / 2 : rows)) return 0;
     const int64_t chunks = (n + kSortChunk - 1) / kSortChunk;
     int64_t off = 0;
     auto take = [&](int64_t bytes) {
@@ -2366,7 +2403,8 @@ int64_t plan_row_sort(int64_t n, int n_values, const int64_t* row_bytes, const i
     if (sort != nullptr) {
         *sort = {n, static_cast<uint32_t>(chunks),
                  static_cast<uint32_t>((static_cast<uint64_t>(kSortParts) << 32) / static_cast<uint64_t>(rows)),
-                 static_cast<uint32_t>(words), static_cast<int32_t*>(index), static_cast<uint16_t*>(place),
+                 static_cast<uint32_t>(words), words <= 2 ? 3 : words <= 4 ? 4 : far ? 6 : 7,
+                 static_cast<int32_t*>(index), static_cast<uint16_t*>(place),
                  static_cast<uint16_t*>(bounds), static_cast<uint32_t*>(out)};
     }
     return off;
@@ -2374,19 +2412,19 @@ int64_t plan_row_sort(int64_t n, int n_values, const int64_t* row_bytes, const i
 
 int find_rows_sorted(ash_map* map, const int32_t* keys, RowTables tabs, const RowSort& sort, int miss,
                      int64_t* indices, uint8_t* masks, hipStream_t s) {
-    // the passes address rows by words
+    switch (map->key_dim) {
+        case 1: find_sort_kernel<1><<<sort.chunks, kSortThreads, 0, s>>>(map->d, keys, sort, tabs, miss, indices, masks); break;
+        case 2: find_sort_kernel<2><<<sort.chunks, kSortThreads, 0, s>>>(map->d, keys, sort, tabs, miss, indices, masks); break;
+        case 3: find_sort_kernel<3><<<sort.chunks, kSortThreads, 0, s>>>(map->d, keys, sort, tabs, miss, indices, masks); break;
+        default: find_sort_kernel<4><<<sort.chunks, kSortThreads, 0, s>>>(map->d, keys, sort, tabs, miss, indices, masks); break;
+    }
+    ASH_LAUNCH_CHECK();
+    // these two address rows by words
     for (int v = 0; v < tabs.n; ++v) {
         if ((tabs.wide >> v) & 1u) tabs.units[v] *= 4;
         tabs.magic[v] = static_cast<uint32_t>((0x100000000ull + tabs.units[v] - 1) / tabs.units[v]);
     }
     tabs.wide = 0;
-    switch (map->key_dim) {
-        case 1: find_sort_kernel<1><<<sort.chunks, kSortThreads, 0, s>>>(map->d, keys, sort, indices, masks); break;
-        case 2: find_sort_kernel<2><<<sort.chunks, kSortThreads, 0, s>>>(map->d, keys, sort, indices, masks); break;
-        case 3: find_sort_kernel<3><<<sort.chunks, kSortThreads, 0, s>>>(map->d, keys, sort, indices, masks); break;
-        default: find_sort_kernel<4><<<sort.chunks, kSortThreads, 0, s>>>(map->d, keys, sort, indices, masks); break;
-    }
-    ASH_LAUNCH_CHECK();
     constexpr uint32_t kRunsPerGroup = kSortRuns * (kBlock / 64);
     const uint32_t groups = (sort.chunks + kRunsPerGroup - 1) / kRunsPerGroup;
     const unsigned g = groups * kSortParts;

@@ -522,7 +522,12 @@ int ash_map_neighbors(ash_map_t* map, int64_t num_rows, int radius, int bidirect
 
 /* Replaces `HashMap::load_states` (ash/src/hashmap_gpu.cuh:407-450): the map
  * is emptied, then (keys[i] -> indices[i]) are stored, size := n and the heap
- * := heap_src (skipped when heap_src is NULL or already the map's heap). */
+ * := heap_src (skipped when heap_src is NULL or already the map's heap).  Pairs
+ * that are refused are counted in ash_map_status's out[4], which a caller looks at:
+ * where it is not zero, the state is to be dropped (ash_map_clear) or another one
+ * loaded.  From a heap with entries outside 0 .. capacity-1 nothing is taken: until
+ * then the size is the capacity and inserts are refused as by a full map, but for
+ * as many as have been erased. */
 int ash_map_load(ash_map_t* map, const int32_t* keys, const int64_t* indices,
                  int64_t n, const int32_t* heap_src, void* stream);
 

@@ -312,6 +312,41 @@ def test_states_that_address_no_row_are_refused(gpu_ash):
     assert other.size() == len(keys) and bool(other.find(keys)[1].all())
 
 
+@pytest.mark.parametrize("policy", [NEVER, ALWAYS])
+@pytest.mark.parametrize("stored", [0, 3000])
+def test_nothing_is_taken_from_a_heap_that_addresses_no_row(gpu_ash, policy, stored):
+    """A caller of the C ABI that goes on after such a load: inserts are refused as
+    by a full map -- no index outside the table is drawn, and no key is stored twice
+    because another one has given its slot back -- but for as many as were erased."""
+    raw = RawMap(gpu_ash, 3, 20_000)
+    rng = np.random.default_rng(7)
+    pool = torch.unique(_keys(rng, 40_000, 40), dim=0)
+    pool = pool[torch.from_numpy(rng.permutation(len(pool)))].to(DEV)
+    old, new = pool[:stored].contiguous(), pool[3000:8000]
+    heap = torch.arange(20_000, dtype=torch.int32, device=DEV)
+    heap[stored + 1::2] = torch.tensor([20_000, -7], dtype=torch.int32, device=DEV).repeat(10_000)[:len(heap[stored + 1::2])]
+    indices = torch.arange(stored, device=DEV)
+    raw.check(raw.lib.ash_map_load(raw.handle, old.data_ptr(), indices.data_ptr(), stored, heap.data_ptr(), raw.stream))
+    c = raw.counters()
+    assert c["refused"] == int(((heap < 0) | (heap >= 20_000)).sum()) > 0 and c["size"] == 20_000
+    batch = new.repeat(8, 1)[torch.from_numpy(rng.permutation(8 * len(new))).to(DEV)]
+    for _ in range(3):                      # the later ones among the tombstones of the first
+        raw.insert(batch, policy)
+        assert not bool(raw.find(new)[1].any()) and bool(raw.find(old)[1].all())
+        assert raw.counters()["size"] == 20_000
+    gone = min(stored, 500)
+    if gone:
+        raw.erase(old[:gone], policy)
+        raw.insert(batch, policy)
+        found, mask = raw.find(pool)
+        assert int(mask.sum()) == stored == len(torch.unique(found[mask])) and not bool(mask[:gone].any())
+        assert raw.counters()["size"] == 20_000
+    raw.check(raw.lib.ash_map_clear(raw.handle, raw.stream))
+    raw.insert(batch, policy)
+    found, mask = raw.find(new)
+    assert bool(mask.all()) and sorted(found.tolist()) == list(range(len(new)))
+
+
 def test_rows_of_indices_outside_the_table_read_as_zero(gpu_ash):
     """ash_gather_rows gives a zero row for an index outside the source table
     where torch's `values[name][indices]` (ash/hashmap.py:87-95) raises or wraps

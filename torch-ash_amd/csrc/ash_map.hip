@@ -305,6 +305,7 @@ __device__ __forceinline__ void insert_key(
         int64_t i, bool active, const ValueArgs& va,
         int32_t* __restrict__ assigned, const int64_t* __restrict__ given,
         int32_t* report = nullptr) {
+    static_assert(!(TOMBS && MODE == kInsertLoad), "loads start from an emptied table");
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     int32_t seen = -1;     // kInsertReport: the index read beside a key that was there
@@ -322,9 +323,14 @@ __device__ __forceinline__ void insert_key(
     // Phase A: claim a slot per new key.  Its sequence is followed to the end (a bucket
     // with an empty slot, or the whole range): a key that is met there is stored
     // already.  Else it takes the first slot of the sequence that is free, empty or a
-    // tombstone.  Slots are tried in the order of the sequence, and nothing frees a
-    // slot while keys are inserted, so threads that store the same key meet in the
-    // same slot, whatever others have taken in between.
+    // tombstone.  Slots are tried in the order of the sequence, so threads that store
+    // the same key meet in the same slot, whatever others have taken in between --
+    // unless a slot before it comes free meanwhile, which it does where a key finds
+    // the heap exhausted and gives its slot back (phase B).  Whoever takes that one
+    // has seen it free, and so draws from the heap after that key did: the counter
+    // has reached the capacity, does not fall below it again in the same launch, and
+    // the newcomer is refused as well.  Of two threads that store one key in two slots
+    // at most one gets an index.
     // (Tombstones that are left alone pile up: keys that come and go behind a run of
     // full buckets lengthen it by what they leave each time, until the range is full
     // and refuses keys.  A million stored keys, 65 537 that come, are read and go:
@@ -418,7 +424,6 @@ __device__ __forceinline__ void insert_key(
     int32_t idx = -1;
     const int nreused = TOMBS ? __popcll(__ballot(reused)) : 0;
     if constexpr (MODE == kInsertLoad) {
-        if (TOMBS && lane == 0 && nreused > 0) atomicSub(m.ctr + kCtrTombs, nreused);
         if (w) {
             // the index comes with the key (`given` null: the key's own number,
             // when the keys are the entries of the key log)
@@ -476,12 +481,8 @@ __device__ __forceinline__ void insert_key(
         for (int q = 0; q < wave; ++q) top += s_cnt[q];
         if (w) {
             if (top < m.capacity) {
-                idx = m.heap[top];
-                // (a heap that a state dict brought may hold anything: an entry
-                // that addresses no row is treated like an exhausted heap)
-                if (static_cast<uint32_t>(idx) >= static_cast<uint32_t>(m.capacity)) idx = -1;
-            }
-            if (idx < 0) {
+                idx = m.heap[top];   // (addresses a row: check_heap_kernel)
+            } else {
                 // Heap exhausted: give the slot up again.
                 if (won) {
                     atomicExch(slot_ptr(m, wb, ws), kTomb);
@@ -1964,6 +1965,8 @@ __global__ __launch_bounds__(kHeapBlock) void replace_from_log_kernel(MapDev m, 
 }
 
 // Entries of a heap that address no row, counted with the pairs a load refuses.
+// Inserts write to the rows and log entries that they draw from the heap; from one
+// with such entries nothing is drawn: it counts as exhausted until a clear or a load.
 __global__ __launch_bounds__(kBlock) void check_heap_kernel(const int32_t* __restrict__ heap,
                                                            int64_t capacity,
                                                            int32_t* __restrict__ ctr) {
@@ -1973,7 +1976,10 @@ __global__ __launch_bounds__(kBlock) void check_heap_kernel(const int32_t* __res
          i += stride) {
         bad += static_cast<uint32_t>(heap[i]) >= static_cast<uint32_t>(capacity) ? 1 : 0;
     }
-    if (bad) atomicAdd(ctr + kCtrLoadDup, bad);
+    if (bad) {
+        atomicAdd(ctr + kCtrLoadDup, bad);
+        atomicMax(ctr + kCtrSize, static_cast<int32_t>(capacity));
+    }
 }
 
 // ---------------------------------------------------------------- host
@@ -3567,8 +3573,8 @@ int ash_map_rebuild(ash_map_t* map, int32_t* keys_scratch,
         return 0;
     }
     ValueArgs va = {};
-    return launch_insert<kInsertLoad>(map, keys_scratch, n, va, nullptr,
-                                      indices_scratch, s);
+    return launch_insert_to<kInsertLoad, false>(map, keys_scratch, n, va, nullptr,
+                                                indices_scratch, s);
 }
 
 int ash_map_neighbors(ash_map_t* map, int64_t num_rows, int radius, int bidirectional,
@@ -3622,14 +3628,13 @@ int ash_map_load(ash_map_t* map, const int32_t* keys, const int64_t* indices,
                                static_cast<size_t>(map->capacity) * 4,
                                hipMemcpyDeviceToDevice, s));
     }
-    // later inserts take their indices from this heap unchecked: entries that
-    // address no row are counted with the pairs the load refuses
+    // later inserts take their indices from this heap unchecked
     check_heap_kernel<<<looping_grid(map->capacity), kBlock, 0, s>>>(map->d.heap, map->capacity,
                                                                    map->d.ctr);
     ASH_LAUNCH_CHECK();
     if (n == 0) return 0;
     ValueArgs va = {};
-    return launch_insert<kInsertLoad>(map, keys, n, va, nullptr, indices, s);
+    return launch_insert_to<kInsertLoad, false>(map, keys, n, va, nullptr, indices, s);
 }
 
 }  // extern "C"

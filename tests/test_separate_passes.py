@@ -97,6 +97,24 @@ def _check(ash, grid, x):
             value.backward()
 
 
+@pytest.mark.parametrize("arrived", [False, True])
+def test_put_off_parts_are_added_to_one_tensor(cpu_ash, monkeypatch, arrived):
+    """Several contributions that a second-order node has put off: one tensor takes
+    them all, copied or made once, and what somebody else holds stays as it is."""
+    gq = cpu_ash.grid_query
+    targets = []
+    monkeypatch.setattr(gq.backend, "query_backward_backward_onto",
+                        lambda target, *rest: (targets.append(target), target.add_(1.0)), raising=False)
+    embeddings, own = torch.randn(5, 8, 2), torch.zeros(5, 8, 2)
+    carried = torch.randn(5, 8, 2) if arrived else None
+    kept = carried.clone() if arrived else torch.zeros(5, 8, 2)
+    parts = [((None, None), (embeddings,), target) for target in (None, own, None, None)]
+    got = gq.add_put_off(parts, carried, 2, "linear")
+    assert torch.equal(got, kept + 3) and torch.equal(own, torch.ones(5, 8, 2))
+    assert not arrived or torch.equal(carried, kept)
+    assert {t.data_ptr() for t in targets} == {got.data_ptr(), own.data_ptr()}
+
+
 def test_passes_one_after_the_other(fused_ash):
     _check(fused_ash, *_grid(fused_ash, torch.device("cpu")))
 

@@ -247,14 +247,14 @@ class _Later:
 
 def add_put_off(parts, carried, grid_dim, interpolation):
     """The gradient `carried` with `parts` of a `_Later`, by themselves."""
+    if any(target is None for _, _, target in parts):
+        if carried is None:
+            carried = torch.zeros_like(parts[0][1][0], memory_format=torch.contiguous_format)
+        elif not (_HOLDERS_ALONE and _holders(carried) == _HOLDERS_ALONE and carried.is_contiguous()):
+            carried = carried.clone(memory_format=torch.contiguous_format)
     for (u, z), operands, target in parts:
-        if target is None:
-            if carried is None or not (_HOLDERS_ALONE and _holders(carried) == _HOLDERS_ALONE
-                                       and carried.is_contiguous()):
-                carried = torch.zeros_like(operands[0]) if carried is None else carried.clone(
-                    memory_format=torch.contiguous_format)
-            target = carried
-        backend.query_backward_backward_onto(target, u, z, *operands, grid_dim, interpolation)
+        backend.query_backward_backward_onto(carried if target is None else target, u, z, *operands,
+                                             grid_dim, interpolation)
     return carried
 
 

@@ -106,7 +106,7 @@ def test_put_off_parts_are_added_to_one_tensor(cpu_ash, monkeypatch, arrived):
     monkeypatch.setattr(gq.backend, "query_backward_backward_onto",
                         lambda target, *rest: (targets.append(target), target.add_(1.0)), raising=False)
     embeddings, own = torch.randn(5, 8, 2), torch.zeros(5, 8, 2)
-    carried = torch.randn(5, 8, 2) if arrived else None
+    carried = torch.randint(9, (5, 8, 2)).float() if arrived else None
     kept = carried.clone() if arrived else torch.zeros(5, 8, 2)
     somebody = [carried]   # (more than a node and what it calls hold of a gradient)
     parts = [((None, None), (embeddings,), target) for target in (None, own, None, None)]

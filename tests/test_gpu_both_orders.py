@@ -153,6 +153,24 @@ def test_a_pass_that_fails_in_between_leaves_nothing_behind(scene):
     assert _close(_grad(grid, loss, retain_graph=True), want) and _close(_grad(grid, loss), want)
 
 
+def test_putting_off_copies_nothing(gpu_ash):
+    """Operands that are not contiguous are copied where they are used, not where
+    they are put off."""
+    grid = _make_grid(gpu_ash, 4, 4, 1, seed=3)
+    ops = _operands(grid, _queries(4, 1, 100_000, seed=4))
+    z, u = torch.ones(1, 4, device=DEV).expand(100_000, 4), torch.ones(1, 3, device=DEV).expand(100_000, 3)
+    host = gpu_ash.grid_query.backend.host
+    start = torch.zeros_like(ops[0])
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    got = host.query_gradient_later(u, z, list(ops), "linear", start)
+    assert got.data_ptr() == start.data_ptr() and torch.cuda.max_memory_allocated() == before
+    for wrong in ((u, z[:, :3]), (u[:-1], z), (u, z.double()), (u.cpu(), z)):
+        with pytest.raises(RuntimeError):
+            host.query_gradient_later(*wrong, list(ops), "linear", start)
+
+
 def test_gradients_that_somebody_sees_are_whole(scene):
     ash, grid, x, put_off = scene
     xq = x.clone().requires_grad_(True)

@@ -736,8 +736,8 @@ struct Operands {
         args.embedding_dim = e;
     }
 
-    // `t` as a contiguous tensor like the embeddings with n x width elements
-    Tensor like(const Tensor& t, int64_t width, const char* name) const {
+    // `t` has to be a tensor like the embeddings with n x width elements
+    void must_be_like(const Tensor& t, int64_t width, const char* name) const {
         if (t.device() != emb.device()) {
             fail(std::string(name) + " is on " + t.device().str() + ", embeddings on " + emb.device().str());
         }
@@ -749,6 +749,10 @@ struct Operands {
             fail(std::string(name) + " has shape " + shape_of(t) + ", expected (" + std::to_string(n) +
                  ", " + std::to_string(width) + ")");
         }
+    }
+
+    Tensor like(const Tensor& t, int64_t width, const char* name) const {
+        must_be_like(t, width, name);
         return t.contiguous();
     }
 
@@ -821,12 +825,12 @@ std::tuple<Optional, Optional> query_backward_backward(const Tensor& gg_in, cons
 
 // The embedding gradient of a query_backward_backward whose contributions are
 // still to come (query_backward_both): `accumulate_into`, or zeros.  Everything is
-// checked here, where the call is made.
+// checked here, where the call is made, and made contiguous where it is read.
 Tensor query_gradient_later(const Tensor& gg_in, const Tensor& z_in, const std::vector<Tensor>& operands,
                             const std::string& interpolation, const Optional& accumulate_into) {
     Operands q(operands, interpolation);
-    q.like(z_in, q.e, "z");
-    q.like(gg_in, 3, "grad_grad_offsets");
+    q.must_be_like(z_in, q.e, "z");
+    q.must_be_like(gg_in, 3, "grad_grad_offsets");
     const Tensor grad = q.gradient(accumulate_into, true);
     if (!accumulate_into.has_value()) {
         q.args.num_queries = 0;   // nothing but the zeros

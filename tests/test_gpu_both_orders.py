@@ -2,6 +2,7 @@
 pass over the queries: the kernels against the oracle, and the passes of the
 engine in which the second-order node may and may not leave its share to the
 forward node."""
+import gc
 import threading
 
 import pytest
@@ -151,6 +152,36 @@ def test_a_pass_that_fails_in_between_leaves_nothing_behind(scene):
         _Fails.armed = False
     assert put_off == [True]
     assert _close(_grad(grid, loss, retain_graph=True), want) and _close(_grad(grid, loss), want)
+
+
+def test_a_pass_that_fails_keeps_no_operands(scene):
+    """... nor the memory of what it had put off, while the graph lives."""
+    ash, grid, x, put_off = scene
+    xq = x.clone().requires_grad_(True)
+    y, _ = grid(xq, "smooth_step")
+    value = []
+    thread = threading.Thread(target=lambda: value.append((_Fails.apply(y)**2).mean()))
+    thread.start()
+    thread.join()
+    loss = value[0] + _norm_loss(y, xq, 0)
+    grid.embeddings.grad = None
+    loss.backward(retain_graph=True)         # what a first pass leaves for good
+    grid.embeddings.grad = None
+    xq.grad = None
+    gc.collect()
+    before = torch.cuda.memory_allocated()
+    _Fails.armed = True
+    del put_off[:]
+    try:
+        for _ in range(3):
+            try:
+                loss.backward(retain_graph=True)
+            except ValueError:
+                pass
+    finally:
+        _Fails.armed = False
+    gc.collect()
+    assert put_off == [True] * 3 and torch.cuda.memory_allocated() == before
 
 
 def test_putting_off_copies_nothing(gpu_ash):

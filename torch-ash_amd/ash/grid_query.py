@@ -207,6 +207,19 @@ def _learn_holders() -> None:
 PUT_OFF_FROM = 1 << 16
 
 
+class _Pass:
+    """What is put off in one pass of the engine, which holds this object, as one of
+    the pass's final callbacks, until the pass ends, in whichever way."""
+
+    __slots__ = ("parts", "__weakref__")
+
+    def __init__(self):
+        self.parts = []   # ((grad_grad_offsets, z), operands, parameter's .grad or None)
+
+    def __call__(self):
+        self.parts = []
+
+
 class _Later:
     """What second-order nodes leave for the backward of the forward node they
     were recorded from: their contributions to the embedding gradient go to the
@@ -220,12 +233,12 @@ class _Later:
     one or before the other.  (They share a stream: the second-order node is
     recorded by the forward node's own backward, which the engine runs on the
     stream of the forward.)  Kept by the pass, so that what one leaves behind that
-    fails in between is not taken up by another."""
+    fails in between is not taken up by another, and goes with it."""
 
-    __slots__ = ("parts",)
+    __slots__ = ("passes",)
 
     def __init__(self):
-        self.parts = {}   # pass -> [((grad_grad_offsets, z), operands, parameter's .grad or None)]
+        self.passes = {}   # id of a pass -> weak reference to its _Pass
 
     def room(self, ctx, edges):
         """The list of the running pass if `ctx`, a second-order node whose second
@@ -237,12 +250,32 @@ class _Later:
                     or not torch._C._will_engine_execute_node(edges[1][0])
                     or not backend.host.hands_over_unseen(ctx, 1)):
                 return None
+            here = self._of(task)
+            if here is None:
+                here = _Pass()
+                torch.autograd.Variable._execution_engine.queue_callback(here)
+                for known, each in list(self.passes.items()):
+                    if each() is None:
+                        self.passes.pop(known, None)
+                self.passes[task] = weakref.ref(here)
+            return here.parts
         except Exception:  # outside an engine pass, or another torch
             return None
-        return self.parts.setdefault(task, [])
+
+    def _of(self, task):
+        each = self.passes.get(task)
+        return None if each is None else each()
 
     def take(self):
-        return self.parts.pop(torch._C._current_graph_task_id(), ()) if self.parts else ()
+        if not self.passes:
+            return ()
+        task = torch._C._current_graph_task_id()
+        here = self._of(task)
+        if here is None:
+            return ()
+        del self.passes[task]
+        parts, here.parts = here.parts, []
+        return parts
 
 
 def add_put_off(parts, carried, grid_dim, interpolation):

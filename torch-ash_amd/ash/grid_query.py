@@ -200,11 +200,16 @@ def _learn_holders() -> None:
         pass
 
 
-# Queries from which second-order nodes leave their share to the forward node: the
-# pass that is saved takes 22 us for 131 000 of five channels, some 10 for 48 000 and
-# next to nothing for few; the bookkeeping takes 2 - 7 us of the host, which such
-# steps wait for (48 000 queries 497 -> 504 us).
-PUT_OFF_FROM = 1 << 16
+# Queries from which second-order nodes leave their share to the forward node, by the
+# wall time of a training step of 20 000 blocks (own share -> put off, us).  Fewer wait
+# for the host, 350 - 490 us by its clock, and the kernel time saved (22 us for 131 000
+# of five channels) reaches nobody: 131 000 of 1, 4, 5, 16 channels 331 -> 335, 469 ->
+# 470, 504 -> 497, 472 -> 476; 262 000 352 -> 355, 485 -> 488, 488 -> 493, 474 -> 478.
+# From here on the kernels bound the steps with wide rows: 393 000 495 -> 491, 497 ->
+# 494, 429 -> 415, 477 -> 468; 524 000 of 5 and 16 channels 370 -> 354 and 568 -> 485;
+# 1 M of 5, 594 -> 450.  Narrow rows gain later, of one and four channels from 2 M on
+# (507 -> 493 and 555 -> 497), and lose nothing in between.
+PUT_OFF_FROM = 3 << 17
 
 
 class _Pass:

@@ -871,8 +871,9 @@ class _Backend:
     def find_rows(self, hashmap, keys, tables, zero_misses: bool = False,
                   need_indices: bool = True):
         """(indices or None, masks, [table[indices] for each table]) in one
-        launch; rows of keys that are not stored are row 0 of the table, or
-        zeros with `zero_misses`."""
+        launch, large batches on several tables in three with scratch memory;
+        rows of keys that are not stored are row 0 of the table, or zeros with
+        `zero_misses`."""
         return self.host.find_rows(hashmap._address, hashmap.key_dim, hashmap._index, keys, tables,
                                    zero_misses, need_indices)
 

@@ -87,10 +87,13 @@ struct Shape {
     static constexpr int kHaloEach = (kHalo * E + kThreads - 1) / kThreads;   // elements per thread
     static constexpr int kTaps = W * W;                           // of one dz
     // wavefronts per SIMD that the tile leaves room for.  No more than the
-    // registers allow: 64 for windows of 3 and 74 - 80 for 5 are eight and six
-    // (five channels, 5^3, spill 14 of them and gain all the same: 245 -> 234), 108
+    // registers allow: 64 for windows of 3 and 72 - 80 for 5 are eight and six, 108
     // - 128 for 7 are four.  (Five, 96 registers, for 7: 20 000 blocks, one channel
-    // 192 -> 222 us, two 340 -> 344; three, five channels 223 -> 286.)
+    // 192 -> 222 us, two 340 -> 344; three, five channels 223 -> 286.)  Five channels,
+    // 5^3, spill 14 registers with six and gain all the same, five against six: 300
+    // blocks 33.8 -> 30.7 us, 1000 40 -> 40, 3000 81 -> 82, 6000 129 -> 125, 12 000
+    // 241 -> 222, 25 000 495 -> 457; four and six channels 165 -> 151 and 281 -> 244
+    // at 12 000 without spilling, the others alike.
     static constexpr int kMostWaves = W == 3 ? 8 : (W == 5 ? 6 : 4);
     static constexpr int waves() {
         const int each = (kThreads / 64 + 3) / 4;   // of one workgroup

@@ -25,7 +25,7 @@
 //            start of the row plus the flags below the edge's
 //
 // 60 000 blocks, field and weights in rows of five channels, us: listing 9, bits
-// 98, classify 27, count and scan 23, points 47, triangles 65, together 270; with
+// 99, classify 26, count and scan 20, points 48, triangles 56, together 258; with
 // case bytes, a slot word per cell and the two channels copied out first: copies
 // 274, clear, classify, count, points and triangles 415.
 //

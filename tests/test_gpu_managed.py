@@ -313,12 +313,15 @@ def test_states_that_address_no_row_are_refused(gpu_ash):
 
 
 @pytest.mark.parametrize("policy", [NEVER, ALWAYS])
-@pytest.mark.parametrize("stored", [0, 3000])
-def test_nothing_is_taken_from_a_heap_that_addresses_no_row(gpu_ash, policy, stored):
+@pytest.mark.parametrize("stored,second_region", [(0, False), (3000, False), (3000, True)])
+def test_nothing_is_taken_from_a_heap_that_addresses_no_row(gpu_ash, policy, stored, second_region):
     """A caller of the C ABI that goes on after such a load: inserts are refused as
     by a full map -- no index outside the table is drawn, and no key is stored twice
     because another one has given its slot back -- but for as many as were erased."""
     raw = RawMap(gpu_ash, 3, 20_000)
+    if second_region:     # entries are then put back from a listing when tombstones pile up
+        raw.general = torch.empty(64 * 20, dtype=torch.uint8, device=DEV)
+        raw.check(raw.lib.ash_map_attach_general(raw.handle, raw.general.data_ptr(), 64 * 20, raw.stream))
     rng = np.random.default_rng(7)
     pool = torch.unique(_keys(rng, 40_000, 40), dim=0)
     pool = pool[torch.from_numpy(rng.permutation(len(pool)))].to(DEV)

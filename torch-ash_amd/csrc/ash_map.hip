@@ -3160,6 +3160,9 @@ int upkeep(ash_map* map, int64_t incoming, void* scratch, int64_t scratch_bytes,
     }
     int32_t* keys = nullptr;
     int64_t* indices = nullptr;
+    // (after a load that has refused pairs the size is not the number of entries,
+    // and what a listing leaves unwritten would be put back as well)
+    if (map->general_attached && c.load_refused > 0) return 0;
     if (map->general_attached && c.size > 0) {
         // entries of the second region do not stand in the key log: the pairs
         // are listed into the caller's scratch and put back from there

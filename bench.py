@@ -88,8 +88,8 @@ VALUE_ROW_BYTES = 2 * (12 + 4)               # color + depth, read and written
 #   atomic_requests: TCC_ATOMIC (all of them are forwarded to the memory side:
 #     TCC_EA0_ATOMIC reads the same).
 MEASURED_COUNTERS = {
-    "insert_values": (2_566_000_000 + 1_949_000_000, 0.382, 16_331_000),
-    "insert_keys": (2_306_000_000 + 1_687_000_000, 0.282, 16_396_000),
+    "insert_values": (2_566_000_000 + 1_949_000_000, 0.381, 16_332_000),
+    "insert_keys": (2_305_000_000 + 1_687_000_000, 0.282, 16_397_000),
     "find": (2_230_000_000 + 145_000_000, 0.064, 0),
     "erase": (2_236_000_000 + 1_217_000_000, 0.467, 16_031_000),
     # the two keys-only split passes and the range pass
@@ -105,7 +105,7 @@ MEASURED_COUNTERS = {
     # kernel only: the zero fill of the dense gradient adds 1.64 GB written
     "cfg4_backward": (438_000_000 + 149_000_000 + 1_638_400_000, 0.113, 2_344_000),
     "cfg4_double_backward": (486_000_000 + 166_000_000 + 1_638_400_000, 0.122, 2_344_000),
-    "cfg4_grid_query": (71_000_000 + 122_000_000, 0.399, 0),
+    "cfg4_grid_query": (71_000_000 + 122_000_000, 0.398, 0),
     "cfg4_module_forward": (325_000_000 + 72_000_000, 0.404, 0),
     "cfg4_module_forward_for_training": (326_000_000 + 189_000_000, 0.437, 0),
 }
@@ -119,7 +119,7 @@ MEASURED_COUNTERS = {
 COUNTERS_SOURCE = {
     "profiles": ["profiles/bench_hbm_traffic_pmc.md",
                  "profiles/bench_l2_hit_rate_and_atomics_pmc.md"],
-    "csrc_sha256": "621f728f1c104d2ab81694c2771a2ec28a422c6115b226859f5ca0acb0222773",
+    "csrc_sha256": "576cd81fe65654a3e10f373df0c45eeb1808ff868efdaac6c490bcebe8988f58",
 }
 
 

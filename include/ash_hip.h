@@ -472,7 +472,8 @@ int ash_map_status(ash_map_t* map, int64_t out[5], void* stream);
  * latest ash_grid_collect_touched and out[6] = entries that live in the second
  * region.  The handle follows every call that changes them: after a clear they
  * are known to be zero, after ash_map_insert_auto they have been read (or are
- * on their way, see there) -- only when neither holds is the device asked,
+ * on their way, see there), an ash_map_erase of up to 2^17 keys leaves them on
+ * their way as a rule -- only when neither holds is the device asked,
  * which waits for `stream`: a kernel writes them into page-locked words of the
  * call's own, and the host looks for them there.  Several threads may read the
  * counters of one map at a time, each on its own stream.  `staging` is not

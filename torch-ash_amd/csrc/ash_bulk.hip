@@ -305,7 +305,7 @@ __device__ __forceinline__ void give_up_row(const BulkPlan& pl, int32_t row, int
 template <int DIM, bool PROV>
 __global__ __launch_bounds__(kSplitThreads) void split_keys_kernel(
         MapDev m, BulkPlan pl, const int32_t* __restrict__ keys, int identity,
-        int32_t* early, int32_t stamp) {
+        uint64_t* early, int32_t stamp) {
     __shared__ SplitShared sh;
     const int tid = threadIdx.x;
     const int64_t base = static_cast<int64_t>(blockIdx.x) * kSplitChunk;
@@ -390,7 +390,7 @@ __global__ __launch_bounds__(kSplitThreads) void split_keys_kernel(
         if (tid == 0 && sh.losers) atomicAdd(pl.hdr + kHdrLosers, sh.losers);
     }
     if (early != nullptr) {
-        // `early`: page-locked host memory.  The workgroup that finishes last
+        // `early`: a word of the host's.  The workgroup that finishes last
         // leaves there how many rows this pass has handed to the per-key
         // kernel, for a host that waits for nothing else of the call.  (Every
         // update of that count has returned its value to the thread that made
@@ -399,10 +399,7 @@ __global__ __launch_bounds__(kSplitThreads) void split_keys_kernel(
         __syncthreads();
         if (tid == 0 &&
             atomicAdd(pl.hdr + kHdrTicket, 1) == static_cast<int32_t>(gridDim.x) - 1) {
-            __hip_atomic_store(early, atomicAdd(pl.hdr + kHdrSpillKeys, 0), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_SYSTEM);
-            __hip_atomic_store(early + kLandingStamp, stamp, __ATOMIC_RELEASE,
-                               __HIP_MEMORY_SCOPE_SYSTEM);
+            leave_word(early, atomicAdd(pl.hdr + kHdrSpillKeys, 0), stamp);
         }
     }
 }
@@ -1310,7 +1307,7 @@ int check_values(int n_values, const void* const* src, void* const* dst,
 
 template <bool PROV>
 int launch_split_keys(ash_map* map, const BulkPlan& pl, const int32_t* keys, int identity,
-                      int32_t* early, int32_t stamp, hipStream_t s) {
+                      uint64_t* early, int32_t stamp, hipStream_t s) {
     const unsigned g = static_cast<unsigned>((pl.n + kSplitChunk - 1) / kSplitChunk);
     switch (map->key_dim) {
         case 1:
@@ -1402,7 +1399,7 @@ int ash_map_bulk_workspace_bytes(ash_map_t* map, int64_t n, int n_values,
 int ash::insert_bulk(ash_map* map, const int32_t* keys, int64_t n,
                      int n_values, const void* const* src, void* const* dst,
                      const int64_t* row_bytes, void* workspace,
-                     int64_t workspace_bytes, int32_t* early, int32_t* late, int32_t stamp,
+                     int64_t workspace_bytes, uint64_t* early, uint64_t* late, int32_t stamp,
                      bool* published, void* stream) {
     if (check_batch(map, keys, n)) return 1;
     if (check_values(n_values, src, dst, row_bytes)) return 1;
@@ -1444,8 +1441,8 @@ int ash::insert_bulk(ash_map* map, const int32_t* keys, int64_t n,
     Publish publish = {};
     auto none_spilled = [&](Publish& p) -> int {
         if (early == nullptr) return 0;
-        if (wait_for_stamp(early + kLandingStamp, stamp)) return 1;
-        if (*early == 0) {
+        if (wait_for_words(early, 1, stamp)) return 1;
+        if (value_of(*early) == 0) {
             p = {late, stamp, pl.hdr + kHdrTicketLast};
             *published = true;
         }

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <mutex>
 #include <string>
 
@@ -71,17 +72,22 @@ enum Counter {
     kCtrLogHigh = 8,   // log entries at or beyond the size and below this index may hold keys of an earlier filling
     kCtrCursor = 9,    // output cursor of items()
     kCtrTicket = 10,   // workgroups of a running ash_grid_collect_touched that have read their input
+    // A word for each launch under way whose last workgroup does something for all
+    // of them (next_ticket): counts those that are done, zero before and after.
+    kCtrTickets = 16,
     kNumCounters = 64
 };
+constexpr int kTickets = 16;
 constexpr int kHostCounters = 8;
 // Page-locked words in which kernels leave answers for the host: a line per call
 // that waits for its answer (Answer), and one of its own for a map (take_line)
-// with two places.  Each place carries its stamp kLandingStamp words behind its
-// start.
-constexpr int kLandingStamp = 8;
-constexpr int kLineWords = 32;
-constexpr int kLineLate = 0;     // counters, fetched behind a streaming insert or a fusion frame
-constexpr int kLineEarly = 16;   // count left by the first pass of a streaming insert
+// with two places.  A word is 64 bits, the value below and the call's stamp above
+// it, written at once: the host knows each word by its stamp, and a kernel need not
+// wait until one word has arrived before it sends the next.  (A stamp behind the
+// words wants a release in between: a trip over the bus, and the L2 written back.)
+constexpr int kLineWords = 16;
+constexpr int kLineLate = 0;     // counters, left by a streaming insert, an erase or a fusion frame
+constexpr int kLineEarly = 8;    // count left by the first pass of a streaming insert
 constexpr int64_t kHeaderBytes = 256;
 
 // General region: open addressing over 32-bit state words + 16-byte keys.
@@ -160,17 +166,19 @@ struct ash_map {
     // up to `counters`, is looked at and brought up to date under this lock (not
     // held while a call waits for words of its own)
     std::mutex counter_lock;
-    int32_t* line;          // page-locked words of the map's own (take_line), made on first use
+    uint64_t* line;         // page-locked words of the map's own (take_line), made on first use
     int32_t stamp;          // of the latest words asked for there
     int32_t late_stamp;
     bool late_in_flight;    // the device may still owe the words at kLineLate
     bool late_pending;      // ... and it is the latest state of the counters: nobody has looked at it yet
+    bool late_of_erase;     // ... left by an erase
     bool counters_known;    // `counters` is what the device holds
     ash_counters counters;
     // an erase, refused keys or a run of inserts whose counters nobody read
     // may have left tombstones: the next managed insert looks at the counters
     bool maybe_tombstones;
     int unread_inserts;
+    std::atomic<uint32_t> tickets;   // taken so far (next_ticket)
     // A call that changes the map has been captured into a graph: replays
     // change the device's state behind the host's back, so from then on nothing
     // the host remembers of it is trusted -- the counters are copied from the

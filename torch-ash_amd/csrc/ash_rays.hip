@@ -466,7 +466,7 @@ __global__ __launch_bounds__(kBlock) void ray_sample_kernel(
 constexpr int kScanThreads = 1024;
 
 __global__ __launch_bounds__(kScanThreads) void ray_scan_kernel(GroupSamples* __restrict__ groups,
-                                                                int n, int32_t* landing,
+                                                                int n, uint64_t* landing,
                                                                 int32_t stamp) {
     __shared__ int64_t s_sum[kScanThreads / 64];
     __shared__ int64_t s_most[kScanThreads / 64];
@@ -506,10 +506,7 @@ __global__ __launch_bounds__(kScanThreads) void ray_scan_kernel(GroupSamples* __
         const int32_t words[4] = {static_cast<int32_t>(total), static_cast<int32_t>(total >> 32),
                                   static_cast<int32_t>(most), static_cast<int32_t>(most >> 32)};
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            __hip_atomic_store(landing + w, words[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        }
-        __hip_atomic_store(landing + kLandingStamp, stamp, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        for (int w = 0; w < 4; ++w) leave_word(landing + w, words[w], stamp);
     }
 }
 
@@ -834,11 +831,8 @@ int ash_ray_sample_march(ash_map_t* map, uint8_t* scratch, int volume_lo, int vo
     }
     ray_scan_kernel<<<1, kScanThreads, 0, s>>>(g, static_cast<int>(march_groups(n)), answer.words, answer.stamp);
     ASH_LAUNCH_CHECK();
-    if (answer.wait(s)) return 1;
-    for (int w = 0; w < 2; ++w) {
-        out[w] = static_cast<int64_t>(static_cast<uint32_t>(answer.words[2 * w])) |
-                 (static_cast<int64_t>(answer.words[2 * w + 1]) << 32);
-    }
+    if (answer.wait(s, 4)) return 1;
+    for (int w = 0; w < 2; ++w) out[w] = answer.pair(2 * w);
     return 0;
 }
 

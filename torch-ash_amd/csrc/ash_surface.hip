@@ -492,7 +492,7 @@ __global__ __launch_bounds__(kCountThreads) void count_kernel(SurfaceArgs a) {
 
 // Sums of the groups -> what lies before each; totals for the host.
 __global__ __launch_bounds__(kScanThreads) void scan_groups_kernel(Sums* __restrict__ groups, int64_t n,
-                                                                   int32_t* landing, int32_t stamp) {
+                                                                   uint64_t* landing, int32_t stamp) {
     __shared__ Sums s_part[kScanThreads / 64];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -535,10 +535,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_groups_kernel(Sums* __restr
                 static_cast<int32_t>(total.points), static_cast<int32_t>(total.points >> 32),
                 static_cast<int32_t>(total.triangles), static_cast<int32_t>(total.triangles >> 32)};
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            __hip_atomic_store(landing + w, words[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        }
-        __hip_atomic_store(landing + kLandingStamp, stamp, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        for (int w = 0; w < 4; ++w) leave_word(landing + w, words[w], stamp);
     }
 }
 
@@ -837,11 +834,8 @@ int ash_surface_block8_classify(ash_map_t* map, const void* sdfs, int64_t sdf_st
     ASH_LAUNCH_CHECK();
     scan_groups_kernel<<<1, kScanThreads, 0, s>>>(a.w.groups, groups, answer.words, answer.stamp);
     ASH_LAUNCH_CHECK();
-    if (answer.wait(s)) return 1;
-    for (int w = 0; w < 2; ++w) {
-        out[w] = static_cast<int64_t>(static_cast<uint32_t>(answer.words[2 * w])) |
-                 (static_cast<int64_t>(answer.words[2 * w + 1]) << 32);
-    }
+    if (answer.wait(s, 4)) return 1;
+    for (int w = 0; w < 2; ++w) out[w] = answer.pair(2 * w);
     if (out[0] > 0x7FFFFFFFll) ASH_FAIL("marching_cubes: more than 2^31 vertices");
     if (out[1] > 0x7FFFFFFFll / 3) ASH_FAIL("marching_cubes: too many triangles");
     return 0;

@@ -142,7 +142,7 @@ struct PointerGuard : DeviceGuard {
 // `publish`: what the last launch of a call leaves for the host, see
 // publish_counters_kernel; `ticket` (zero) counts its workgroups.
 struct Publish {
-    int32_t* landing;   // null: nothing
+    uint64_t* landing;   // null: nothing
     int32_t stamp;
     int32_t* ticket;
 };
@@ -170,8 +170,17 @@ inline bool heap_in_order(const ash_map* map) { return !map->heap_dirty && !map-
 // false for one that took entries away.
 // `s`: the stream the call runs on (captured: see ash_map::replayed).
 void counters_changed(ash_map* map, bool inserted, hipStream_t s);
+// Leaves `value` for the host in a word of its line (kLineWords).
+__device__ __forceinline__ void leave_word(uint64_t* word, int32_t value, int32_t stamp) {
+    __hip_atomic_store(word, static_cast<uint64_t>(static_cast<uint32_t>(value)) |
+                                     (static_cast<uint64_t>(static_cast<uint32_t>(stamp)) << 32),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+inline int32_t value_of(uint64_t word) { return static_cast<int32_t>(static_cast<uint32_t>(word)); }
+inline int32_t stamp_of(uint64_t word) { return static_cast<int32_t>(static_cast<uint32_t>(word >> 32)); }
+
 // Page-locked words of one call's own, in which a kernel leaves what the call
-// waits for: up to kLandingStamp words, and behind them the call's stamp.
+// waits for, each under the call's stamp.
 class Answer {
   public:
     Answer() = default;
@@ -179,16 +188,22 @@ class Answer {
     Answer& operator=(const Answer&) = delete;
     ~Answer();
     int take();                // `words` and `stamp` are the call's from here on
-    int wait(hipStream_t s);   // `s`: the stream whose latest launch leaves them
-    int32_t* words = nullptr;
+    // `s`: the stream whose latest launch leaves the first `count` words
+    int wait(hipStream_t s, int count);
+    int64_t pair(int w) const {   // words w (below) and w + 1
+        return static_cast<int64_t>(static_cast<uint32_t>(value_of(words[w]))) |
+               (static_cast<int64_t>(value_of(words[w + 1])) << 32);
+    }
+    void abandon() { lost_ = true; }   // nobody waits for words that may still come
+    uint64_t* words = nullptr;
     int32_t stamp = 0;
 
   private:
     bool lost_ = false;   // the device may still owe the words
 };
-// The map's own page-locked words (made on first use), and the wait for one of them.
+// The map's own page-locked words (made on first use), and the wait for some of them.
 int take_line(ash_map* map);
-int wait_for_stamp(const int32_t* word, int32_t stamp);
+int wait_for_words(const uint64_t* words, int count, int32_t stamp);
 // May the table hold tombstones, for an insert?  (Replays of a captured launch meet
 // any table; refused keys whose counters nobody has read yet may have left some,
 // which then wait for a later insert.)
@@ -198,14 +213,13 @@ int settle_landing_place(ash_map* map);
 // Adds up `n` words of `counts` into the counter of touched blocks and queues the
 // read-back of the counters behind the stream's work (ash_map.hip).
 int queue_touched_count(ash_map* map, const int32_t* counts, int n, hipStream_t s);
-// The streaming insert (ash_bulk.hip); `early`: page-locked words (or null) where
+// The streaming insert (ash_bulk.hip); `early`: page-locked word (or null) where
 // its first pass leaves the number of keys that it hands to the per-key kernel,
-// and behind it, at kLandingStamp, `stamp`.  With `early` the call waits for that
-// number; is it zero, the last launch leaves the counters at `late` (with `stamp`)
-// and *published is set.
+// under `stamp`.  With `early` the call waits for that number; is it zero, the last
+// launch leaves the counters at `late` (under `stamp`) and *published is set.
 int insert_bulk(ash_map* map, const int32_t* keys, int64_t n, int n_values,
                 const void* const* src, void* const* dst, const int64_t* row_bytes,
-                void* workspace, int64_t workspace_bytes, int32_t* early, int32_t* late,
+                void* workspace, int64_t workspace_bytes, uint64_t* early, uint64_t* late,
                 int32_t stamp, bool* published, void* stream);
 // Fills the bucket array if a clear() left that to the next user of the table.
 int settle_table(ash_map* map, hipStream_t s);

@@ -450,12 +450,17 @@ int ash_map_upkeep(ash_map_t* map, int64_t incoming, void* scratch, int64_t scra
  * that state: inserts only read it, and nothing but this library may write to
  * it while the map lives; while it is in that state listings read the log of
  * stored keys only below the size, so the log is left as it is and emptied
- * beyond the size by the first erase); the fill of the bucket array runs with the next
+ * beyond the size by the first erase); the fill of the bucket array of all but
+ * small tables runs with the next
  * call that reads or updates the table, on that call's stream, and not at all
  * when that call is an ash_map_insert_bulk, which rewrites every bucket.  A
  * call whose stream is being captured refuses to run that pending fill (the
  * graph would empty the table at every replay). */
 int ash_map_clear(ash_map_t* map, void* stream);
+/* The same with up to four value tables zeroed (ash/hashmap.py:100-103), as a rule
+ * in the same launch: rows[v] 16-byte aligned, row_bytes[v] bytes in all. */
+int ash_map_clear_rows(ash_map_t* map, int n_values, void* const* rows,
+                       const int64_t* row_bytes, void* stream);
 
 /* Host read-back of the device counters; always asks the device, which waits
  * for `stream`.

@@ -207,6 +207,10 @@ _SIGNATURES = {
     ),
     "ash_map_erase_bulk": (ctypes.c_int, [_PTR, _PTR, _I64, _PTR, _I64, _PTR]),
     "ash_map_clear": (ctypes.c_int, [_PTR, _PTR]),
+    "ash_map_clear_rows": (
+        ctypes.c_int,
+        [_PTR, ctypes.c_int, ctypes.POINTER(_PTR), ctypes.POINTER(_I64), _PTR],
+    ),
     "ash_map_status": (ctypes.c_int, [_PTR, ctypes.POINTER(_I64), _PTR]),
     "ash_map_counters": (ctypes.c_int, [_PTR, _PTR, ctypes.POINTER(_I64), _PTR]),
     "ash_map_counters_pending": (ctypes.c_int, [_PTR]),
@@ -1409,9 +1413,13 @@ class _HashMap:
         self.last_erase_path = "streaming" if streaming else "per-key"
         self.version = next(_VERSIONS)
 
-    def clear(self) -> None:
-        with torch.cuda.device(self._device):
-            self._check(self._lib.ash_map_clear(self._handle, self._stream()))
+    def zeroes(self, t: torch.Tensor) -> bool:
+        """Whether `clear` can zero `t` along with the table."""
+        return stands_alone(t) and self._backend.host.can_zero(t, self._index)
+
+    def clear(self, rows=()) -> None:
+        """`rows`: up to four tensors (`zeroes`) to be zeroed in the same launch."""
+        self._backend.host.clear(self._address, self._index, list(rows))
         self.version = next(_VERSIONS)
 
     def items(self) -> Tuple[torch.Tensor, torch.Tensor]:

@@ -194,6 +194,18 @@ class ASHEngine(nn.Module):
         self.backend.clear()
         self._dropped_seen = 0
 
+    def clear_with(self, stores) -> None:
+        """clear(), and the tensors `stores` zeroed (ash/hashmap.py:100-103)."""
+        zeroes = getattr(self.backend, "zeroes", None)
+        along = [] if zeroes is None else [rows for rows in stores if zeroes(rows)][:4]
+        for rows in stores:
+            if not any(rows is each for each in along):
+                rows.zero_()
+        if not along:
+            return self.clear()
+        self.backend.clear(along)
+        self._dropped_seen = 0
+
     def size(self) -> int:
         return self.backend.size()
 

@@ -1385,7 +1385,7 @@ int ash_map_bulk_workspace_bytes(ash_map_t* map, int64_t n, int n_values,
         // bucket (half with value rows): 1 M keys into a new table of capacity
         // 2 M take 77 us instead of 138.  Not for batches far beyond what the
         // table holds (piles of duplicates would queue on a few ranges).
-        if (map->table_stale && n >= (int64_t{1} << 18) && n <= 12 * nb &&
+        if (map->table_stale && streams_into_emptied(n, nb) &&
             (n_values > 0 ? 2 * n >= nb : 3 * n >= nb)) {
             big = true;
         }
@@ -1430,7 +1430,7 @@ int ash::insert_bulk(ash_map* map, const int32_t* keys, int64_t n,
         user.row_dwords[v] = static_cast<int32_t>(row_bytes[v] / 4);
     }
     const ValueArgs none = {};
-    const int stale = map->table_stale ? 1 : 0;
+    const int stale = map->table_stale && !map->table_filled ? 1 : 0;
     counters_changed(map, true, s);
     // (captured into a graph, the choice would be replayed whatever the heap
     // holds then: a captured call takes the variant that reads the heap)
@@ -1459,7 +1459,7 @@ int ash::insert_bulk(ash_map* map, const int32_t* keys, int64_t n,
         auto build = tombs_in(map) ? build_kernel<false, true> : build_kernel<false, false>;
         build<<<pl.parts, kBuildThreads, 0, s>>>(map->d, pl, stale, identity);
         ASH_LAUNCH_CHECK();
-        map->table_stale = false;
+        map->table_stale = map->table_filled = false;
         if (none_spilled(publish)) return 1;
         // (the first pass alone writes that list)
         if (publish.landing == nullptr &&
@@ -1474,7 +1474,7 @@ int ash::insert_bulk(ash_map* map, const int32_t* keys, int64_t n,
     auto build = tombs_in(map) ? build_kernel<true, true> : build_kernel<true, false>;
     build<<<pl.parts, kBuildThreads, 0, s>>>(map->d, pl, stale, identity);
     ASH_LAUNCH_CHECK();
-    map->table_stale = false;
+    map->table_stale = map->table_filled = false;
     int64_t words = 0;
     for (int v = 0; v < n_values; ++v) words = words > n * user.row_dwords[v] ? words : n * user.row_dwords[v];
     int64_t blocks = (words + kCopyThreads - 1) / kCopyThreads;

@@ -41,6 +41,7 @@ namespace py = pybind11;
     X(ash_gather_rows)                                                                \
     X(ash_map_insert_scratch_bytes)                                                   \
     X(ash_map_insert_auto)                                                            \
+    X(ash_map_clear_rows)                                                             \
     X(ash_map_erase_scratch_bytes)                                                    \
     X(ash_map_erase_auto)                                                             \
     X(ash_map_items)                                                                  \
@@ -373,6 +374,27 @@ bool erase(uintptr_t handle, int64_t dim, int64_t device, const Tensor& keys_in,
     check(lib.ash_map_erase_auto(map_of(handle), ptr<int32_t>(keys), n, ptr<void>(scratch), scratch_bytes,
                                  policy, stream_of(device)));
     return scratch_bytes > 0;
+}
+
+// What torch's zero_() does to a plain tensor by one fill of its memory.
+bool can_zero(const Tensor& t, int64_t device) {
+    return t.is_cuda() && t.get_device() == device && t.layout() == at::kStrided && t.is_contiguous() &&
+           !t.requires_grad() && !t.is_inference() &&
+           reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+}
+
+void clear(uintptr_t handle, int64_t device, const std::vector<Tensor>& zeroed) {
+    need(zeroed.size() <= kMaxTables, "clear takes up to 4 tensors per call");
+    void* rows[kMaxTables];
+    int64_t bytes[kMaxTables];
+    for (size_t v = 0; v < zeroed.size(); ++v) {
+        need(can_zero(zeroed[v], device), "clear takes contiguous tensors on the map's device");
+        rows[v] = zeroed[v].data_ptr();
+        bytes[v] = static_cast<int64_t>(zeroed[v].nbytes());
+    }
+    check(lib.ash_map_clear_rows(map_of(handle), static_cast<int>(zeroed.size()), rows, bytes,
+                                 stream_of(device)));
+    for (const Tensor& t : zeroed) t.unsafeGetTensorImpl()->bump_version();
 }
 
 std::vector<int64_t> counters(uintptr_t handle, int64_t device) {
@@ -872,6 +894,8 @@ PYBIND11_MODULE(_ash_host, m) {
     m.def("gather_rows", &gather_rows);
     m.def("insert", &insert);
     m.def("erase", &erase);
+    m.def("can_zero", &can_zero);
+    m.def("clear", &clear);
     m.def("counters", &counters);
     m.def("items", &items);
     m.def("neighbors", &neighbors);

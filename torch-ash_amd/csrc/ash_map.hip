@@ -1273,21 +1273,79 @@ __global__ __launch_bounds__(kBlock) void empty_log_tail_kernel(
     }
 }
 
-// `keep_log`: the key log is left as it is; the counter kCtrLogHigh then
-// remembers how far it may hold entries (the size so far, or what an earlier
-// call remembered).  `tickets`: of a table that has never been used.
+// The counters of an emptied table.  (Words of launches under way, kCtrTickets, are
+// zero at rest and left alone.)
 __global__ __launch_bounds__(kBlock) void reset_heap_kernel(
         int32_t* __restrict__ heap, int64_t capacity, int32_t* __restrict__ ctr,
-        int32_t size_value, bool write_heap, bool keep_log, bool tickets) {
+        int32_t size_value, bool write_heap) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
     if (write_heap && i < capacity) heap[i] = static_cast<int32_t>(i);
-    if (i < kNumCounters) {
+    if (i < kCtrTickets || (i >= kCtrTickets + kTickets && i < kNumCounters)) {
+        ctr[i] = i == kCtrSize ? size_value : 0;
+    }
+}
+
+// A clear in one launch: counters, and stretches of memory that are filled with one
+// word (value rows with zeros, the bucket array, the second region's states and the
+// key log with ones) or counted up (the heap).  A workgroup takes kClearUnits pieces
+// of 16 bytes of one stretch, so that workgroups handed out one after the other walk
+// through memory in order.  Bound by the stores of large stretches (tables of 288 and
+// 96 MB, with the counters: two fills of torch's and a launch for the counters 36.6 +
+// 13.9 + 4.7 -> 47 us, 8.2 TB/s), and by the launch itself for small ones, which is
+// why it is one (a launch in a busy stream costs 4 us however little it does; a set of
+// 5640 keys emptied, filled and asked 41.5 -> 34.2 us).
+constexpr int kClearUnits = 4 * kBlock;
+constexpr int kClearSpans = kMaxFusedValues + 4;
+
+struct ClearSpan {
+    uint4* p;
+    int64_t n16;       // whole pieces
+    uint32_t word;
+    uint8_t tail;      // bytes behind them
+    bool count;        // 0, 1, 2, ... instead of `word`
+    uint32_t first;    // the stretch's first workgroup
+};
+
+struct ClearArgs {
+    int n;
+    ClearSpan span[kClearSpans];
+};
+
+enum { kCountersAsTheyAre = 0, kCountersReset = 1, kCountersFresh = 2 };
+
+// `counters`: left alone, reset, or those of a table that has never been used.  The
+// key log beyond the size is left as it is where `keep_log`; kCtrLogHigh then
+// remembers how far it may hold entries (the size so far, or what an earlier call
+// remembered).
+__global__ __launch_bounds__(kBlock) void clear_kernel(ClearArgs a, int32_t* __restrict__ ctr,
+                                                       int counters, bool keep_log) {
+    if (blockIdx.x == 0 && counters != kCountersAsTheyAre && threadIdx.x < kNumCounters) {
         // (one wavefront: every lane has read before any lane writes)
+        const int i = threadIdx.x;
         const int32_t size = ctr[kCtrSize], high = ctr[kCtrLogHigh];
         int32_t v = 0;
-        if (i == kCtrSize) v = size_value;
-        if (i == kCtrLogHigh && keep_log) v = size > high ? size : high;
-        if (tickets || i < kCtrTickets || i >= kCtrTickets + kTickets) ctr[i] = v;
+        if (i == kCtrLogHigh && keep_log && counters == kCountersReset) v = size > high ? size : high;
+        if (counters == kCountersFresh || i < kCtrTickets || i >= kCtrTickets + kTickets) ctr[i] = v;
+    }
+    if (a.n == 0) return;
+    int k = 0;
+    while (k + 1 < a.n && blockIdx.x >= a.span[k + 1].first) ++k;
+    const ClearSpan& span = a.span[k];
+    const int64_t base = static_cast<int64_t>(blockIdx.x - span.first) * kClearUnits + threadIdx.x;
+#pragma unroll
+    for (int u = 0; u < kClearUnits / kBlock; ++u) {
+        const int64_t i = base + u * kBlock;
+        if (i < span.n16) {
+            const uint32_t w = static_cast<uint32_t>(4 * i);
+            span.p[i] = span.count ? make_uint4(w, w + 1, w + 2, w + 3)
+                                   : make_uint4(span.word, span.word, span.word, span.word);
+        } else if (i == span.n16) {
+            uint8_t* rest = reinterpret_cast<uint8_t*>(span.p + i);
+            for (int b = 0; b < span.tail; ++b) {
+                rest[b] = static_cast<uint8_t>((span.count ? static_cast<uint32_t>(4 * i) + b / 4 : span.word) >>
+                                               (8 * (b % 4)));
+            }
+        }
     }
 }
 
@@ -2050,20 +2108,13 @@ int fill_buckets(ash_map* map, hipStream_t s) {
     fill16_kernel<<<capped_grid(n16), kBlock, 0, s>>>(
             reinterpret_cast<uint4*>(map->d.buckets), n16, 0xFFFFFFFFu);
     ASH_LAUNCH_CHECK();
-    map->table_stale = false;
+    map->table_stale = map->table_filled = false;
     return 0;
 }
 
-// `lazy`: leave the bucket array to the next call that needs it (settle_table).
-// `lazy` also leaves the key log while the heap is in its initial order.
-// `fresh`: the workspace has not been used yet.
-int clear_table(ash_map* map, hipStream_t s, bool write_heap, int32_t size, bool lazy = false,
-                bool fresh = false) {
-    if (lazy) {
-        map->table_stale = true;
-    } else if (fill_buckets(map, s)) {
-        return 1;
-    }
+// Empties the table and sets the size to `size`.
+int clear_table(ash_map* map, hipStream_t s, bool write_heap, int32_t size) {
+    if (fill_buckets(map, s)) return 1;
     if (map->general_attached) {
         const int64_t g16 = static_cast<int64_t>(map->d.gslots) / 4;
         fill16_kernel<<<capped_grid(g16), kBlock, 0, s>>>(
@@ -2072,31 +2123,91 @@ int clear_table(ash_map* map, hipStream_t s, bool write_heap, int32_t size, bool
     }
     // The key log: every index is free again.  While nothing has written to the
     // heap since its last reset the indices in use are 0 .. size-1 and nothing
-    // reads the log beyond the size: a lazy clear leaves the log alone and only
-    // notes how far it holds entries (reset_heap_kernel); otherwise that part
-    // of the log (read on the device, before the counters are reset below) is
-    // emptied, or all of it once the heap has been written to.
-    const bool keep_log = lazy && !map->heap_dirty;
-    if (keep_log) {
-        map->log_stale = true;
-    } else {
-        const int64_t n16 = (map->capacity + 1) / 2;
-        // (a prefix of unknown length: few workgroups that loop, not one per
-        // 4 KB of the capacity, most of which would start only to leave)
-        empty_log_kernel<<<map->heap_dirty ? capped_grid(n16) : looping_grid(n16), kBlock, 0, s>>>(
-                reinterpret_cast<uint4*>(map->d.klog), map->capacity, map->d.ctr,
-                map->heap_dirty ? 0 : 1);
-        ASH_LAUNCH_CHECK();
-        map->log_stale = false;
-    }
+    // reads the log beyond the size: that part of the log (read on the device,
+    // before the counters are reset below) is emptied, or all of it once the heap
+    // has been written to.
+    const int64_t n16 = (map->capacity + 1) / 2;
+    // (a prefix of unknown length: few workgroups that loop, not one per
+    // 4 KB of the capacity, most of which would start only to leave)
+    empty_log_kernel<<<map->heap_dirty ? capped_grid(n16) : looping_grid(n16), kBlock, 0, s>>>(
+            reinterpret_cast<uint4*>(map->d.klog), map->capacity, map->d.ctr,
+            map->heap_dirty ? 0 : 1);
+    ASH_LAUNCH_CHECK();
+    map->log_stale = false;
     // Inserts only read the heap; while nothing has written to it since the
     // last reset it still is 0, 1, 2, ... and only the counters are reset.
     const bool rewrite = write_heap && map->heap_dirty;
     int64_t span = rewrite && map->capacity > kNumCounters ? map->capacity : kNumCounters;
     reset_heap_kernel<<<grid_for(span), kBlock, 0, s>>>(
-            map->d.heap, map->capacity, map->d.ctr, size, rewrite, keep_log, fresh);
+            map->d.heap, map->capacity, map->d.ctr, size, rewrite);
     ASH_LAUNCH_CHECK();
     if (rewrite) map->heap_dirty = false;
+    return 0;
+}
+
+// Value rows that a clear zeroes along with the table (16-byte aligned).
+struct ClearRows {
+    int n;
+    void* const* rows;
+    const int64_t* bytes;
+};
+
+class ClearList {
+  public:
+    void add(void* p, int64_t bytes, uint32_t word, bool count = false) {
+        if (bytes <= 0) return;
+        const int64_t pieces = bytes / 16;
+        args_.span[args_.n++] = {static_cast<uint4*>(p), pieces, word, static_cast<uint8_t>(bytes % 16),
+                                 count, static_cast<uint32_t>(groups_)};
+        groups_ += (pieces + (bytes % 16 != 0 ? 1 : 0) + kClearUnits - 1) / kClearUnits;
+    }
+    void add(const ClearRows& rows) {
+        for (int v = 0; v < rows.n; ++v) add(rows.rows[v], rows.bytes[v], 0u);
+    }
+    int launch(const ash_map* map, int counters, bool keep_log, hipStream_t s) const {
+        if (groups_ > 0x7FFFFFFF) ASH_FAIL("too many bytes to clear in one call");
+        if (groups_ == 0 && counters == kCountersAsTheyAre) return 0;
+        clear_kernel<<<static_cast<unsigned>(groups_ > 0 ? groups_ : 1), kBlock, 0, s>>>(
+                args_, map->d.ctr, counters, keep_log);
+        ASH_LAUNCH_CHECK();
+        return 0;
+    }
+
+  private:
+    ClearArgs args_ = {};
+    int64_t groups_ = 0;
+};
+
+// What a clear does of a map whose state the host knows, and what makes a new one
+// (`fresh`): counters, heap and second region are reset at once.  The bucket array is
+// left to the next call that needs it (settle_table) -- a streaming insert writes
+// every bucket itself -- unless the table is too small for any batch to be streamed
+// into it (streams_into_emptied: 2^18 keys, at most twelve per bucket); such a table
+// is at most 2.8 MB, filled here without a launch of its own.  The key log is left
+// alone while the heap is in its initial order (no listing reads an entry beyond the
+// size then), or emptied with the heap's order.
+int clear_lazily(ash_map* map, hipStream_t s, bool fresh, const ClearRows& rows) {
+    ClearList list;
+    list.add(rows);
+    const bool small = !streams_into_emptied(int64_t{1} << 18, map->d.nb);
+    if (small) list.add(map->d.buckets, static_cast<int64_t>(map->d.nb) * kGroup * 16, ~0u);
+    if (map->general_attached) list.add(map->d.gstate, static_cast<int64_t>(map->d.gslots) * 4, ~0u);
+    const bool keep_log = !map->heap_dirty;
+    const bool wide = reinterpret_cast<uintptr_t>(map->d.heap) % 16 == 0;   // (the caller's own buffer)
+    if (!keep_log) {
+        list.add(map->d.klog, (map->capacity + 1) / 2 * 16, ~0u);
+        if (wide) list.add(map->d.heap, map->capacity * 4, 0u, true);
+    }
+    if (list.launch(map, fresh ? kCountersFresh : kCountersReset, keep_log, s)) return 1;
+    if (!keep_log && !wide) {
+        reset_heap_kernel<<<grid_for(std::max<int64_t>(map->capacity, kNumCounters)), kBlock, 0, s>>>(
+                map->d.heap, map->capacity, map->d.ctr, 0, true);
+        ASH_LAUNCH_CHECK();
+    }
+    map->table_stale = true;
+    map->table_filled = small;
+    map->log_stale = keep_log;
+    map->heap_dirty = false;
     return 0;
 }
 
@@ -2347,6 +2458,10 @@ int settle_table(ash_map* map, hipStream_t s) {
         capturing != hipStreamCaptureStatusNone) {
         ASH_FAIL("the table was cleared and not used since: run one call outside the capture first");
     }
+    if (map->table_filled) {
+        map->table_stale = map->table_filled = false;
+        return 0;
+    }
     return fill_buckets(map, s);
 }
 
@@ -2558,7 +2673,7 @@ int ash_map_create(int key_dim, int64_t capacity, int32_t* heap, void* table_ws,
     map->device = device;
     map->table_bytes = table_bytes;
     map->general_attached = false;
-    map->table_stale = false;
+    map->table_stale = map->table_filled = false;
     map->heap_dirty = true;   // the caller's buffer holds anything
     map->log_stale = false;
     map->line = nullptr;
@@ -2581,9 +2696,7 @@ int ash_map_create(int key_dim, int64_t capacity, int32_t* heap, void* table_ws,
     map->d.nb = static_cast<uint32_t>(num_buckets(capacity));
     map->d.gslots = 0;
     map->d.capacity = static_cast<int32_t>(capacity);
-    // (the fill of the bucket array is left to the first call that needs it: a
-    // streaming insert, which writes every bucket itself, does not)
-    if (clear_table(map, static_cast<hipStream_t>(stream), true, 0, true, true)) {
+    if (clear_lazily(map, static_cast<hipStream_t>(stream), true, {})) {
         delete map;
         return 1;
     }
@@ -3117,7 +3230,20 @@ int ash_map_erase(ash_map_t* map, const int32_t* keys, int64_t n,
 }
 
 int ash_map_clear(ash_map_t* map, void* stream) {
+    return ash_map_clear_rows(map, 0, nullptr, nullptr, stream);
+}
+
+int ash_map_clear_rows(ash_map_t* map, int n_values, void* const* rows, const int64_t* row_bytes,
+                       void* stream) {
     if (check_map(map)) return 1;
+    if (n_values < 0 || n_values > kMaxFusedValues) ASH_FAIL("clear: up to 4 value tables per call");
+    if (n_values > 0 && (rows == nullptr || row_bytes == nullptr)) ASH_FAIL("null value tables");
+    for (int v = 0; v < n_values; ++v) {
+        if (row_bytes[v] < 0) ASH_FAIL("clear: negative size");
+        if (row_bytes[v] > 0 && rows[v] == nullptr) ASH_FAIL("null value tensor");
+        if (reinterpret_cast<uintptr_t>(rows[v]) % 16 != 0) ASH_FAIL("clear: values must be 16-byte aligned");
+    }
+    const ClearRows values = {n_values, rows, row_bytes};
     DeviceGuard guard;
     ASH_HIP(guard.enter(map->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -3126,9 +3252,12 @@ int ash_map_clear(ash_map_t* map, void* stream) {
         // what replays leave behind is unknown: everything is cleared now
         if (settle_table(map, s)) return 1;
         map->heap_dirty = true;
-        if (clear_table(map, s, true, 0, false)) return 1;
+        if (clear_table(map, s, true, 0)) return 1;
         map->heap_dirty = true;   // (whatever the flag would say: see heap_in_order)
-    } else if (clear_table(map, s, true, 0, true)) {
+        ClearList list;
+        list.add(values);
+        if (list.launch(map, kCountersAsTheyAre, false, s)) return 1;
+    } else if (clear_lazily(map, s, false, values)) {
         return 1;
     }
     // every counter is zero again: known without a read-back

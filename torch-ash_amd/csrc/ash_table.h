@@ -221,6 +221,11 @@ int insert_bulk(ash_map* map, const int32_t* keys, int64_t n, int n_values,
                 const void* const* src, void* const* dst, const int64_t* row_bytes,
                 void* workspace, int64_t workspace_bytes, uint64_t* early, uint64_t* late,
                 int32_t stamp, bool* published, void* stream);
+// Whether a batch is one to stream into a table of nb buckets that has been emptied
+// (or made) and not used since, by the numbers of both (ash_map_bulk_workspace_bytes).
+inline bool streams_into_emptied(int64_t n, int64_t nb) {
+    return n >= (int64_t{1} << 18) && n <= 12 * nb;
+}
 // Fills the bucket array if a clear() left that to the next user of the table.
 int settle_table(ash_map* map, hipStream_t s);
 // Before the first call that writes to the heap (an erase; a load brings a

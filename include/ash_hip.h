@@ -505,6 +505,14 @@ int ash_map_size(ash_map_t* map, int64_t* size, void* stream);
 int ash_map_items(ash_map_t* map, int32_t* keys_out, int64_t* indices_out,
                   int64_t n_expected, void* stream);
 
+/* The same with the value rows of the listed entries (ash/hashmap.py:138-146: the
+ * tables indexed by the listing): row dst[v][k] is row indices_out[k] of src[v], which
+ * has src_rows[v] rows of row_bytes[v] bytes (a multiple of 4); rows beyond the source
+ * read as zeros.  Up to four tables. */
+int ash_map_items_rows(ash_map_t* map, int32_t* keys_out, int64_t* indices_out, int64_t n_expected,
+                       int n_values, const void* const* src, void* const* dst,
+                       const int64_t* row_bytes, const int64_t* src_rows, void* stream);
+
 /* Whether the next ash_map_items lists entry i under index i (*dense = 1):
  * while nothing has been erased or loaded since the map was created or
  * cleared and no key lives in the second region, the indices in use are

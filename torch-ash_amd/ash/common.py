@@ -233,6 +233,11 @@ _SIGNATURES = {
     "ash_grid_collect_touched": (ctypes.c_int, [_PTR] * 6),
     "ash_map_size": (ctypes.c_int, [_PTR, ctypes.POINTER(_I64), _PTR]),
     "ash_map_items": (ctypes.c_int, [_PTR, _PTR, _PTR, _I64, _PTR]),
+    "ash_map_items_rows": (
+        ctypes.c_int,
+        [_PTR, _PTR, _PTR, _I64, ctypes.c_int, ctypes.POINTER(_PTR), ctypes.POINTER(_PTR),
+         ctypes.POINTER(_I64), ctypes.POINTER(_I64), _PTR],
+    ),
     "ash_map_load": (ctypes.c_int, [_PTR, _PTR, _PTR, _I64, _PTR, _PTR]),
     "ash_map_should_rebuild": (ctypes.c_int, [_PTR, _I64, _I64, _I64]),
     "ash_map_rebuild": (ctypes.c_int, [_PTR, _PTR, _PTR, _I64, _PTR]),
@@ -1422,14 +1427,23 @@ class _HashMap:
         self._backend.host.clear(self._address, self._index, list(rows))
         self.version = next(_VERSIONS)
 
-    def items(self) -> Tuple[torch.Tensor, torch.Tensor]:
+    def _listed(self) -> int:
+        """The number of entries that a listing has now."""
         n = self.size()
         # whether entry i is listed under index i: the value rows of the listing
         # are then the first n rows of every value tensor (HashMap.items)
         dense = ctypes.c_int(0)
         self._check(self._lib.ash_map_items_in_index_order(self._handle, ctypes.byref(dense)))
         self.last_items_in_index_order = bool(dense.value)
-        return self._backend.host.items(self._address, self.key_dim, self._index, n)
+        return n
+
+    def items(self) -> Tuple[torch.Tensor, torch.Tensor]:
+        return self._backend.host.items(self._address, self.key_dim, self._index, self._listed())
+
+    def items_rows(self, tables):
+        """(keys, indices, [table[indices] for each table]): the listing and the
+        value rows of its entries, for tables that `finds_rows_of` takes."""
+        return self._backend.host.items_rows(self._address, self.key_dim, self._index, self._listed(), tables)
 
     def neighbor_rows(
         self, num_rows: int, radius: int, bidirectional: bool

@@ -70,14 +70,16 @@ enum Counter {
     kCtrGenTombs = 7,  // of kCtrTombs, those in the general region
     // (the first eight are what a read-back of the counters copies to the host)
     kCtrLogHigh = 8,   // log entries at or beyond the size and below this index may hold keys of an earlier filling
-    kCtrCursor = 9,    // output cursor of items()
+    // (9 is unused)
     kCtrTicket = 10,   // workgroups of a running ash_grid_collect_touched that have read their input
-    // A word for each launch under way whose last workgroup does something for all
-    // of them (next_ticket): counts those that are done, zero before and after.
+    // A place for each launch under way whose last workgroup does something for all
+    // of them (next_slot): a word that counts those that are done, or, for listings,
+    // a word pair that counts them above the output cursor.  Zero before and after.
     kCtrTickets = 16,
+    kCtrCursors = 32,
     kNumCounters = 64
 };
-constexpr int kTickets = 16;
+constexpr int kLaunchSlots = 16;
 constexpr int kHostCounters = 8;
 // Page-locked words in which kernels leave answers for the host: a line per call
 // that waits for its answer (Answer), and one of its own for a map (take_line)
@@ -178,7 +180,7 @@ struct ash_map {
     // may have left tombstones: the next managed insert looks at the counters
     bool maybe_tombstones;
     int unread_inserts;
-    std::atomic<uint32_t> tickets;   // taken so far (next_ticket)
+    std::atomic<uint32_t> launches;   // that have taken a slot so far (next_slot)
     // A call that changes the map has been captured into a graph: replays
     // change the device's state behind the host's back, so from then on nothing
     // the host remembers of it is trusted -- the counters are copied from the

@@ -45,6 +45,7 @@ namespace py = pybind11;
     X(ash_map_erase_scratch_bytes)                                                    \
     X(ash_map_erase_auto)                                                             \
     X(ash_map_items)                                                                  \
+    X(ash_map_items_rows)                                                             \
     X(ash_map_counters)                                                               \
     X(ash_map_upkeep)                                                                 \
     X(ash_map_neighbors)                                                              \
@@ -416,6 +417,32 @@ std::tuple<Tensor, Tensor> items(uintptr_t handle, int64_t dim, int64_t device, 
                                 stream_of(device)));
     }
     return {keys, indices};
+}
+
+std::tuple<Tensor, Tensor, std::vector<Tensor>> items_rows(uintptr_t handle, int64_t dim, int64_t device,
+                                                           int64_t n, const std::vector<Tensor>& tables) {
+    need(tables.size() <= kMaxTables, "items_rows takes up to 4 tensors per call");
+    Tensor keys = empty({n, dim}, at::kInt, device), indices = empty({n}, at::kLong, device);
+    std::vector<Tensor> rows;
+    const void* src[kMaxTables];
+    void* dst[kMaxTables];
+    int64_t bytes[kMaxTables], count[kMaxTables];
+    for (const Tensor& t : tables) {
+        const size_t v = rows.size();
+        std::vector<int64_t> shape = t.sizes().vec();
+        shape[0] = n;
+        rows.push_back(empty(shape, t.scalar_type(), device));
+        src[v] = t.data_ptr();
+        dst[v] = rows[v].data_ptr();
+        bytes[v] = row_bytes_of(t);
+        count[v] = t.size(0);
+    }
+    if (n > 0) {
+        check(lib.ash_map_items_rows(map_of(handle), ptr<int32_t>(keys), ptr<int64_t>(indices), n,
+                                     static_cast<int>(tables.size()), src, dst, bytes, count,
+                                     stream_of(device)));
+    }
+    return {keys, indices, rows};
 }
 
 // (coords (rows, 3), lut (rows, K)) of the keys at offsets within `radius`
@@ -898,6 +925,7 @@ PYBIND11_MODULE(_ash_host, m) {
     m.def("clear", &clear);
     m.def("counters", &counters);
     m.def("items", &items);
+    m.def("items_rows", &items_rows);
     m.def("neighbors", &neighbors);
     m.def("query_cells", &query_cells);
     m.def("grid_forward", &grid_forward);

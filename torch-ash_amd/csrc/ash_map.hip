@@ -1024,9 +1024,18 @@ __global__ __launch_bounds__(kEraseBlock) void erase_selected_kernel(
     }
 }
 
+// Rows of up to kMaxFusedValues tables, and where they are to go.
+struct GatherArgs {
+    int n;
+    const uint32_t* src[kMaxFusedValues];
+    uint32_t* dst[kMaxFusedValues];
+    int32_t row_dwords[kMaxFusedValues];
+    int64_t src_rows[kMaxFusedValues];
+};
+
 // items(): the live entries are read from the key log (8 bytes per index,
-// against 21 bytes per index of bucket array).  A workgroup takes 8192
-// consecutive indices, each of its wavefronts 512 of them in eight rounds of
+// against 21 bytes per index of bucket array).  A workgroup takes 1024 * ROUNDS
+// consecutive indices, each of its wavefronts 64 * ROUNDS of them in rounds of
 // 64, so that reads are contiguous and -- positions being ranks in index order
 // -- so are the writes of every round; the entries of a workgroup come out
 // sorted by index, workgroups in the order in which they reserve their output
@@ -1034,10 +1043,19 @@ __global__ __launch_bounds__(kEraseBlock) void erase_selected_kernel(
 // written to the heap since it was last 0, 1, 2, ... (`identity`) and the
 // indices in use therefore are 0 .. size-1 -- only the size.
 // Output ranges come from one global cursor; atomics on that single address
-// serialise (about 7 ns each across the XCDs), hence the large workgroups.
+// serialise (about 7 ns each across the XCDs), hence the large workgroups, of which
+// there are as many as there are CUs while the table is small (items_rounds).  The
+// upper half of the cursor counts the workgroups: the last sets it back to zero for
+// the next listing, which a launch in front did before (`last`: nothing else goes on
+// with the cursor).
+// The value rows of an entry are copied along (`rows`: row_dwords words each): both
+// sides run in index order.  Bound by memory from a million entries on (8 + 2 times
+// the row bytes per index: 16 M in 24 M with rows of 16 bytes 287 -> 235 us, 5 TB/s),
+// by the chain of accesses below; the rows by a launch of their own, which read the
+// listed indices again, and the cursor's reset took two launches more (1.07 M in 1.6 M
+// 25.2 -> 18.6, 67 000 in 100 000 11.3 -> 6.2).
 constexpr int kItemsBlock = 1024;
-constexpr int kItemsRounds = 8;
-constexpr int kItemsSpan = kItemsBlock * kItemsRounds;   // indices per workgroup
+constexpr int kItemsWaves = kItemsBlock / 64;
 
 // items() while the heap is in its initial order and no key lives in the
 // second region: the indices in use are 0 .. n-1, every one of them, so entry
@@ -1056,37 +1074,45 @@ __global__ __launch_bounds__(kBlock) void items_dense_kernel(
     idx_out[i] = i;
 }
 
-template <int DIM>
+template <int DIM, int ROUNDS>
 __global__ __launch_bounds__(kItemsBlock) void items_kernel(
         MapDev m, int32_t* __restrict__ keys_out, int64_t* __restrict__ idx_out,
-        int64_t n_expected, int identity) {
-    constexpr int kWaves = kItemsBlock / 64;
-    __shared__ int s_cnt[kWaves * kItemsRounds];
+        int64_t n_expected, int identity, GatherArgs rows, int slot, bool last) {
+    constexpr int kCounts = kItemsWaves * ROUNDS;
+    static_assert(kCounts <= 128, "two wavefronts add them up");
+    __shared__ int s_cnt[kCounts];
     __shared__ int s_base;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
+    unsigned long long* cursor = reinterpret_cast<unsigned long long*>(m.ctr + kCtrCursors) + slot;
+    constexpr unsigned long long kDone = 1ull << 32;
+    const unsigned long long all_but_one = (gridDim.x - 1ull) << 32;
     const int64_t limit = identity ? static_cast<int64_t>(m.ctr[kCtrSize])
                                    : static_cast<int64_t>(m.capacity);
-    const int64_t first = static_cast<int64_t>(blockIdx.x) * kItemsSpan;
-    if (first >= limit) return;
-    const int64_t mine = first + wave * (64 * kItemsRounds) + lane;
-    uint64_t code[kItemsRounds];
-    int rank[kItemsRounds];
+    const int64_t first = static_cast<int64_t>(blockIdx.x) * (kItemsBlock * ROUNDS);
+    const int64_t mine = first + wave * (64 * ROUNDS) + lane;
+    uint64_t code[ROUNDS];
+    int rank[ROUNDS];
 #pragma unroll
-    for (int r = 0; r < kItemsRounds; ++r) {
+    for (int r = 0; r < ROUNDS; ++r) {
         const int64_t i = mine + r * 64;
         code[r] = i < limit ? m.klog[i] : kEmpty;
+    }
+#pragma unroll
+    for (int r = 0; r < ROUNDS; ++r) {
         const uint64_t live = __ballot(code[r] < kTomb);
         rank[r] = __popcll(live & ((1ull << lane) - 1ull));
-        if (lane == 0) s_cnt[wave * kItemsRounds + r] = __popcll(live);
+        if (lane == 0) s_cnt[wave * ROUNDS + r] = __popcll(live);
     }
     __syncthreads();
-    // exclusive scan of the 128 counts by the first two wavefronts
-    const bool scanner = threadIdx.x < kWaves * kItemsRounds;
+    // exclusive scan of the counts by the first two wavefronts
+    const bool scanner = threadIdx.x < kCounts;
     int c = 0, incl = 0;
     if (scanner) {
         c = s_cnt[threadIdx.x];
         incl = c;
+    }
+    if (threadIdx.x < 128) {
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
             const int up = __shfl_up(incl, d);
@@ -1101,21 +1127,51 @@ __global__ __launch_bounds__(kItemsBlock) void items_kernel(
     __syncthreads();
     if (scanner && threadIdx.x >= 64) s_cnt[threadIdx.x] += s_base;
     __syncthreads();
-    if (threadIdx.x == kWaves * kItemsRounds - 1) {
-        const int tot = s_cnt[threadIdx.x] + c;
-        s_base = tot > 0 ? atomicAdd(m.ctr + kCtrCursor, tot) : 0;
+    if (threadIdx.x == kCounts - 1) {
+        const unsigned long long at =
+                atomicAdd(cursor, kDone + static_cast<unsigned long long>(s_cnt[threadIdx.x] + c));
+        s_base = static_cast<int>(static_cast<uint32_t>(at));
+        // (everybody else has been here)
+        if (last && (at & ~(kDone - 1)) == all_but_one) atomicExch(cursor, 0ull);
     }
     __syncthreads();
+    uint64_t live[ROUNDS];   // of the 64 entries of a round, and where the first goes
+    int64_t to[ROUNDS];
 #pragma unroll
-    for (int r = 0; r < kItemsRounds; ++r) {
-        if (code[r] < kTomb) {
-            const int64_t pos = static_cast<int64_t>(s_base) + s_cnt[wave * kItemsRounds + r] + rank[r];
-            if (pos < n_expected) {
-                int32_t k[DIM];
-                unpack_key<DIM>(code[r], k);
+    for (int r = 0; r < ROUNDS; ++r) {
+        live[r] = __ballot(code[r] < kTomb);
+        to[r] = static_cast<int64_t>(s_base) + s_cnt[wave * ROUNDS + r];
+        const int64_t pos = to[r] + rank[r];
+        if (code[r] < kTomb && pos < n_expected) {
+            int32_t k[DIM];
+            unpack_key<DIM>(code[r], k);
 #pragma unroll
-                for (int d = 0; d < DIM; ++d) keys_out[pos * DIM + d] = k[d];
-                idx_out[pos] = mine + r * 64;
+            for (int d = 0; d < DIM; ++d) keys_out[pos * DIM + d] = k[d];
+            idx_out[pos] = mine + r * 64;
+        }
+    }
+    // The rows of a round's 64 indices are one stretch of the source; lanes walk along
+    // it, so that both sides are read and written whole (a lane per row and word after
+    // word: 4 M entries with rows of 16 bytes 80 -> 54 us).
+    for (int v = 0; v < rows.n; ++v) {
+        const uint32_t rd = static_cast<uint32_t>(rows.row_dwords[v]);
+        const uint32_t magic = 0xFFFFFFFFu / rd + 1u;   // (t / rd below 64 * rd, rd > 1)
+        const uint32_t* __restrict__ src = rows.src[v] + (mine - lane) * rd;
+        uint32_t* __restrict__ dst = rows.dst[v];
+        const int64_t have = rows.src_rows[v] - (mine - lane);   // beyond it rows read as zeros
+        for (uint32_t t = lane; t < 64u * rd; t += 64u) {
+            const uint32_t row = rd == 1u ? t : __umulhi(t, magic);
+            const uint64_t before = (1ull << row) - 1ull;
+            uint32_t w[ROUNDS];
+#pragma unroll
+            for (int r = 0; r < ROUNDS; ++r) {
+                const bool in = ((live[r] >> row) & 1ull) && row + r * 64 < have;
+                w[r] = in ? src[static_cast<int64_t>(r) * 64 * rd + t] : 0u;
+            }
+#pragma unroll
+            for (int r = 0; r < ROUNDS; ++r) {
+                const int64_t pos = to[r] + __popcll(live[r] & before);
+                if (((live[r] >> row) & 1ull) && pos < n_expected) dst[pos * rd + (t - row * rd)] = w[r];
             }
         }
     }
@@ -1124,7 +1180,7 @@ __global__ __launch_bounds__(kItemsBlock) void items_kernel(
 template <int DIM>
 __global__ __launch_bounds__(kBlock) void items_general_kernel(
         MapDev m, int32_t* __restrict__ keys_out, int64_t* __restrict__ idx_out,
-        int64_t n_expected) {
+        int64_t n_expected, int32_t* __restrict__ cursor) {
     const uint32_t p = blockIdx.x * kBlock + threadIdx.x;
     const int lane = threadIdx.x & 63;
     int32_t w = kGenEmpty;
@@ -1134,7 +1190,7 @@ __global__ __launch_bounds__(kBlock) void items_general_kernel(
     if (lm == 0) return;
     const int rank = __popcll(lm & ((1ull << lane) - 1ull));
     int base = 0;
-    if (lane == 0) base = atomicAdd(m.ctr + kCtrCursor, __popcll(lm));
+    if (lane == 0) base = atomicAdd(cursor, __popcll(lm));
     base = __shfl(base, 0);
     if (live) {
         const int64_t pos = static_cast<int64_t>(base) + rank;
@@ -1280,9 +1336,7 @@ __global__ __launch_bounds__(kBlock) void reset_heap_kernel(
         int32_t size_value, bool write_heap) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
     if (write_heap && i < capacity) heap[i] = static_cast<int32_t>(i);
-    if (i < kCtrTickets || (i >= kCtrTickets + kTickets && i < kNumCounters)) {
-        ctr[i] = i == kCtrSize ? size_value : 0;
-    }
+    if (i < kCtrTickets) ctr[i] = i == kCtrSize ? size_value : 0;
 }
 
 // A clear in one launch: counters, and stretches of memory that are filled with one
@@ -1325,7 +1379,7 @@ __global__ __launch_bounds__(kBlock) void clear_kernel(ClearArgs a, int32_t* __r
         const int32_t size = ctr[kCtrSize], high = ctr[kCtrLogHigh];
         int32_t v = 0;
         if (i == kCtrLogHigh && keep_log && counters == kCountersReset) v = size > high ? size : high;
-        if (counters == kCountersFresh || i < kCtrTickets || i >= kCtrTickets + kTickets) ctr[i] = v;
+        if (counters == kCountersFresh || i < kCtrTickets) ctr[i] = v;
     }
     if (a.n == 0) return;
     int k = 0;
@@ -1418,14 +1472,6 @@ __global__ __launch_bounds__(kBlock) void scatter_rows_kernel(
 // the indices once per word of a row (the repeats hit the first-level cache);
 // with indices in ascending runs, as items() returns them, source reads are
 // contiguous.  RD = row width in words, 0 = read it from the arguments.
-struct GatherArgs {
-    int n;
-    const uint32_t* src[kMaxFusedValues];
-    uint32_t* dst[kMaxFusedValues];
-    int32_t row_dwords[kMaxFusedValues];
-    int64_t src_rows[kMaxFusedValues];
-};
-
 template <int RD>
 __device__ __forceinline__ void gather_plane(const uint32_t* __restrict__ src,
                                              uint32_t* __restrict__ dst, int rd_runtime,
@@ -2369,12 +2415,11 @@ int settle_landing_place(ash_map* map) {
 
 namespace {
 
-// A word of the device for a launch whose workgroups count themselves.  Launches on
-// one stream could share one; as many as there are words may run at a time on
+// A place among the counters for a launch whose workgroups count themselves.  Launches
+// on one stream could share one; as many as there are places may run at a time on
 // several (a captured launch keeps its own).
-int32_t* next_ticket(ash_map* map) {
-    return map->d.ctr + kCtrTickets + map->tickets.fetch_add(1) % kTickets;
-}
+int next_slot(ash_map* map) { return static_cast<int>(map->launches.fetch_add(1) % kLaunchSlots); }
+int32_t* next_ticket(ash_map* map) { return map->d.ctr + kCtrTickets + next_slot(map); }
 
 // Keys up to which a launch leaves the counters itself (leave_with_last), instead
 // of one of its own behind it.  Its tickets queue on the line of the counters.  A call
@@ -2445,6 +2490,58 @@ int launch_selected(ash_map* map, bool codes, const int32_t* keys,
                     const ValueArgs& va, hipStream_t s, const Publish& publish) {
     return tombs_in(map) ? launch_selected_to<MODE, true>(map, codes, keys, sel, nsel, va, s, publish)
                          : launch_selected_to<MODE, false>(map, codes, keys, sel, nsel, va, s, publish);
+}
+
+}  // namespace
+
+namespace {
+
+// The tables of a gather, checked, and the words of the one with most of them for
+// n rows.
+int gather_args(int n_values, const void* const* src, void* const* dst, const int64_t* row_bytes,
+                const int64_t* src_rows, int64_t n, GatherArgs& a, int64_t& most) {
+    if (src == nullptr || dst == nullptr || row_bytes == nullptr || src_rows == nullptr) {
+        ASH_FAIL("null value tables");
+    }
+    a = {};
+    a.n = n_values;
+    most = 0;
+    for (int v = 0; v < n_values; ++v) {
+        if (src[v] == nullptr || dst[v] == nullptr) ASH_FAIL("null value tensor");
+        if (row_bytes[v] <= 0 || row_bytes[v] % 4 != 0) {
+            ASH_FAIL("gather_rows: rows must be a positive multiple of 4 bytes");
+        }
+        if (src_rows[v] < 0) ASH_FAIL("negative source row count");
+        a.src[v] = static_cast<const uint32_t*>(src[v]);
+        a.dst[v] = static_cast<uint32_t*>(dst[v]);
+        a.row_dwords[v] = static_cast<int32_t>(row_bytes[v] / 4);
+        a.src_rows[v] = src_rows[v];
+        most = std::max(most, n * a.row_dwords[v]);
+    }
+    return 0;
+}
+
+// Rounds of 1024 indices that a workgroup of a listing takes: eight where one
+// workgroup then takes them all (and lists them in order); else one while that makes
+// no more workgroups than there are CUs, so that a small table keeps the device busy;
+// more beyond, where the updates of the cursor would queue.  (Rows of 16 bytes along,
+// us with 1 / 4 / 8: 500 000 indices 12.3 / 10.9 / 14.9, 1.6 M 26.9 / 18.6 / 20.0, 24 M
+// - / 235 / 240; keys alone 1.6 M - / 10.9 / 10.6, 24 M - / 103 / 98.)
+int items_rounds(int64_t capacity, bool rows) {
+    if (capacity <= 8 * kItemsBlock) return 8;
+    if (capacity <= 256 * kItemsBlock) return 1;
+    return rows || capacity <= 1024 * kItemsBlock ? 4 : 8;
+}
+
+template <int DIM>
+void launch_items(const ash_map* map, int32_t* keys_out, int64_t* indices_out, int64_t n, int identity,
+                  const GatherArgs& rows, int slot, bool last, hipStream_t s) {
+    const int rounds = items_rounds(map->capacity, rows.n > 0);
+    auto kernel = rounds == 1   ? items_kernel<DIM, 1>
+                  : rounds == 4 ? items_kernel<DIM, 4>
+                                : items_kernel<DIM, 8>;
+    kernel<<<grid_for(map->capacity, kItemsBlock * rounds), kItemsBlock, 0, s>>>(
+            map->d, keys_out, indices_out, n, identity, rows, slot, last);
 }
 
 }  // namespace
@@ -2683,7 +2780,7 @@ int ash_map_create(int key_dim, int64_t capacity, int32_t* heap, void* table_ws,
     map->counters = {};
     map->maybe_tombstones = false;
     map->unread_inserts = 0;
-    map->tickets = 0;
+    map->launches = 0;
     map->replayed = false;
     map->d.ctr = static_cast<int32_t*>(table_ws);
     map->d.buckets = reinterpret_cast<uint64_t*>(static_cast<char*>(table_ws) +
@@ -3101,26 +3198,13 @@ int ash_gather_rows(int n_values, const void* const* src, void* const* dst,
         ASH_FAIL("gather_rows takes 1.." + std::to_string(kMaxFusedValues) + " tensors per call");
     }
     if (n < 0) ASH_FAIL("negative row count");
-    if (src == nullptr || dst == nullptr || row_bytes == nullptr || src_rows == nullptr) {
+    GatherArgs a;
+    int64_t most = 0;
+    if (n > 0 && gather_args(n_values, src, dst, row_bytes, src_rows, n, a, most)) return 1;
+    if (n == 0 && (src == nullptr || dst == nullptr || row_bytes == nullptr || src_rows == nullptr)) {
         ASH_FAIL("null value tables");
     }
     if (n == 0) return 0;
-    GatherArgs a = {};
-    a.n = n_values;
-    int64_t most = 0;
-    for (int v = 0; v < n_values; ++v) {
-        if (src[v] == nullptr || dst[v] == nullptr) ASH_FAIL("null value tensor");
-        if (row_bytes[v] <= 0 || row_bytes[v] % 4 != 0) {
-            ASH_FAIL("gather_rows: rows must be a positive multiple of 4 bytes");
-        }
-        if (src_rows[v] < 0) ASH_FAIL("negative source row count");
-        a.src[v] = static_cast<const uint32_t*>(src[v]);
-        a.dst[v] = static_cast<uint32_t*>(dst[v]);
-        a.row_dwords[v] = static_cast<int32_t>(row_bytes[v] / 4);
-        a.src_rows[v] = src_rows[v];
-        const int64_t words = n * a.row_dwords[v];
-        most = words > most ? words : most;
-    }
     PointerGuard guard;
     ASH_HIP(guard.enter_for(src[0]));
     if (indices == nullptr) {
@@ -3671,12 +3755,23 @@ int ash_map_size(ash_map_t* map, int64_t* size, void* stream) {
 
 int ash_map_items(ash_map_t* map, int32_t* keys_out, int64_t* indices_out,
                   int64_t n_expected, void* stream) {
+    return ash_map_items_rows(map, keys_out, indices_out, n_expected, 0, nullptr, nullptr, nullptr,
+                              nullptr, stream);
+}
+
+int ash_map_items_rows(ash_map_t* map, int32_t* keys_out, int64_t* indices_out, int64_t n_expected,
+                       int n_values, const void* const* src, void* const* dst,
+                       const int64_t* row_bytes, const int64_t* src_rows, void* stream) {
     if (check_map(map)) return 1;
     if (n_expected < 0) ASH_FAIL("negative item count");
+    if (n_values < 0 || n_values > kMaxFusedValues) ASH_FAIL("items: up to 4 value tables per call");
     if (n_expected == 0) return 0;
     if (keys_out == nullptr || indices_out == nullptr) {
         ASH_FAIL("null output pointer");
     }
+    GatherArgs rows = {};
+    int64_t most = 0;
+    if (n_values > 0 && gather_args(n_values, src, dst, row_bytes, src_rows, n_expected, rows, most)) return 1;
     DeviceGuard guard;
     ASH_HIP(guard.enter(map->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -3702,51 +3797,46 @@ int ash_map_items(ash_map_t* map, int32_t* keys_out, int64_t* indices_out,
                 break;
         }
         ASH_LAUNCH_CHECK();
-        return 0;
+        return n_values > 0 ? ash_gather_rows(n_values, src, dst, row_bytes, src_rows, nullptr, n, stream) : 0;
     }
-    set_counter_kernel<<<1, 64, 0, s>>>(map->d.ctr, kCtrCursor, 0);
-    ASH_LAUNCH_CHECK();
-    const unsigned g = grid_for(map->capacity, kItemsSpan);
+    // Rows go along with the entries that the log lists, up to the width at which a
+    // lane copies one word after the other; entries of the second region are not
+    // listed there.
+    bool along = none_in_general;
+    for (int v = 0; v < n_values; ++v) along = along && rows.row_dwords[v] <= kMaxFusedRowDwords;
+    if (!along) rows.n = 0;
+    const int slot = next_slot(map);
     switch (map->key_dim) {
         case 1:
-            items_kernel<1><<<g, kItemsBlock, 0, s>>>(map->d, keys_out, indices_out,
-                                                 n_expected, identity);
+            launch_items<1>(map, keys_out, indices_out, n_expected, identity, rows, slot, none_in_general, s);
             break;
         case 2:
-            items_kernel<2><<<g, kItemsBlock, 0, s>>>(map->d, keys_out, indices_out,
-                                                 n_expected, identity);
+            launch_items<2>(map, keys_out, indices_out, n_expected, identity, rows, slot, none_in_general, s);
             break;
         case 3:
-            items_kernel<3><<<g, kItemsBlock, 0, s>>>(map->d, keys_out, indices_out,
-                                                 n_expected, identity);
+            launch_items<3>(map, keys_out, indices_out, n_expected, identity, rows, slot, none_in_general, s);
             break;
         default:
-            items_kernel<4><<<g, kItemsBlock, 0, s>>>(map->d, keys_out, indices_out,
-                                                 n_expected, identity);
+            launch_items<4>(map, keys_out, indices_out, n_expected, identity, rows, slot, none_in_general, s);
             break;
     }
     ASH_LAUNCH_CHECK();
     if (!none_in_general) {
         const unsigned gg = grid_for(map->d.gslots);
-        switch (map->key_dim) {
-            case 1:
-                items_general_kernel<1><<<gg, kBlock, 0, s>>>(
-                        map->d, keys_out, indices_out, n_expected);
-                break;
-            case 2:
-                items_general_kernel<2><<<gg, kBlock, 0, s>>>(
-                        map->d, keys_out, indices_out, n_expected);
-                break;
-            case 3:
-                items_general_kernel<3><<<gg, kBlock, 0, s>>>(
-                        map->d, keys_out, indices_out, n_expected);
-                break;
-            default:
-                items_general_kernel<4><<<gg, kBlock, 0, s>>>(
-                        map->d, keys_out, indices_out, n_expected);
-                break;
-        }
+        int32_t* cursor = map->d.ctr + kCtrCursors + 2 * slot;   // its lower half
+        auto kernel = map->key_dim == 1   ? items_general_kernel<1>
+                      : map->key_dim == 2 ? items_general_kernel<2>
+                      : map->key_dim == 3 ? items_general_kernel<3>
+                                          : items_general_kernel<4>;
+        kernel<<<gg, kBlock, 0, s>>>(map->d, keys_out, indices_out, n_expected, cursor);
         ASH_LAUNCH_CHECK();
+        for (int half = 0; half < 2; ++half) {
+            set_counter_kernel<<<1, 64, 0, s>>>(cursor, half, 0);
+            ASH_LAUNCH_CHECK();
+        }
+    }
+    if (n_values > 0 && !along) {
+        return ash_gather_rows(n_values, src, dst, row_bytes, src_rows, indices_out, n_expected, stream);
     }
     return 0;
 }

@@ -5,7 +5,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda:0")
-# tables of up to 42 probe ranges are filled by the clear itself (12 * 42 * 512 < 2^18)
+# tables of up to 42 probe ranges are filled by the clear itself (kFillAtOnce)
 EDGE = 42 * 512 * 6
 
 

@@ -55,6 +55,10 @@ constexpr int kSplitThreads = 1024;
 constexpr int kSplitKeys = 4;                   // records per thread
 constexpr int kSplitChunk = kSplitThreads * kSplitKeys;
 constexpr int kMaxBins = 256;
+// Inserts of at most kOnceChunks chunks into tables of at most kOnceParts partitions
+// take one split pass (split_once_kernel) instead of two.
+constexpr int kOnceChunks = 1024;
+constexpr int kOnceParts = 4096;
 constexpr int kBuildThreads = 512;
 constexpr int kBuildRecs = 4;                   // records per thread and round
 constexpr int kCopyThreads = 256;
@@ -72,6 +76,11 @@ enum { kHdrSpillKeys = 0, kHdrSpillA = 1, kHdrWasEmpty = 3,
 
 struct BulkPlan {
     int64_t n;
+    bool once;             // one split pass: of what follows only `parts`, `cap_part`,
+                           // `once_chunks` and the planes named there are used
+    uint32_t once_chunks;
+    int once_slot;           // of the launches' places (next_slot)
+    uint32_t once_halving;   // the largest power of two below once_chunks (or 0)
     uint32_t parts;        // partitions of kPartBuckets buckets
     uint32_t bins;         // coarse bins of (1 << fine_shift) partitions
     uint32_t fine_shift;
@@ -95,6 +104,10 @@ struct BulkPlan {
     // provisional scheme
     int32_t* rows_a;       // bins * cap_bin input row numbers
     int32_t* rows_b;       // parts * cap_part
+    // one split pass: codes_a holds once_chunks * kSplitChunk codes, each chunk's by
+    // partition, rows_once (with value rows) their numbers inside the chunk
+    uint16_t* starts;      // [once_chunks][parts + 1]: where a partition's records start in the chunk
+    uint16_t* rows_once;
     uint8_t* flags;        // n: 1 = row i did not win a slot
     int32_t* holes;        // n / 2 + 64 row numbers
 };
@@ -103,8 +116,9 @@ inline int64_t align256(int64_t x) { return (x + 255) & ~int64_t{255}; }
 
 // Fills `pl` for `n` keys; returns the workspace size, or 0 when the bulk path
 // does not apply.  With ws == nullptr only sizes are computed.
+// `insert`: of an insert (an erase always splits twice).
 int64_t make_plan(const ash_map* map, int64_t n, int n_values,
-                  const int64_t* row_bytes, char* ws, BulkPlan& pl) {
+                  const int64_t* row_bytes, char* ws, BulkPlan& pl, bool insert = true) {
     if (n < kMinKeys || n_values < 0 || n_values > kMaxFusedValues) return 0;
     for (int v = 0; v < n_values; ++v) {
         if (row_bytes[v] <= 0 || row_bytes[v] % 4 != 0 ||
@@ -148,6 +162,12 @@ int64_t make_plan(const ash_map* map, int64_t n, int n_values,
     pl.cap_part = static_cast<uint32_t>(cap_part);
     pl.chunks = static_cast<uint32_t>((cap_bin + kSplitChunk - 1) / kSplitChunk);
 
+    const int64_t once_chunks = (n + kSplitChunk - 1) / kSplitChunk;
+    pl.once = insert && parts <= kOnceParts && once_chunks <= kOnceChunks;
+    pl.once_chunks = static_cast<uint32_t>(once_chunks);
+    pl.once_halving = 0;
+    for (uint32_t h = 1; h < pl.once_chunks; h <<= 1) pl.once_halving = h;
+
     int64_t off = 0;
     auto take = [&](int64_t bytes) {
         char* p = ws ? ws + off : nullptr;
@@ -155,6 +175,25 @@ int64_t make_plan(const ash_map* map, int64_t n, int n_values,
         return p;
     };
     pl.hdr = reinterpret_cast<int32_t*>(take(kHdrWords * 4));
+    if (pl.once) {
+        const int64_t records = once_chunks * kSplitChunk;
+        pl.cursor_bin = pl.cursor_part = pl.rows_a = pl.rows_b = pl.spill_a = pl.holes = nullptr;
+        pl.codes_b = nullptr;
+        pl.rows_once = nullptr;
+        pl.flags = nullptr;
+        pl.starts = reinterpret_cast<uint16_t*>(take(once_chunks * (parts + 1) * 2));
+        pl.codes_a = reinterpret_cast<uint64_t*>(take(records * 8));
+        pl.spill_keys = reinterpret_cast<int32_t*>(take(n * 4));
+        if (n_values == 0) {
+            pl.spill_a = reinterpret_cast<int32_t*>(take(n * 4));
+        } else {
+            pl.rows_once = reinterpret_cast<uint16_t*>(take(records * 2));
+            pl.flags = reinterpret_cast<uint8_t*>(take(n));
+            pl.holes = reinterpret_cast<int32_t*>(take((n / 2 + 64) * 4));
+        }
+        return off;
+    }
+    pl.starts = pl.rows_once = nullptr;
     pl.cursor_bin = reinterpret_cast<int32_t*>(take((bins << lane_shift) * 4));
     pl.cursor_part = reinterpret_cast<int32_t*>(take((bins << fine_shift) * 4));
     pl.codes_a = reinterpret_cast<uint64_t*>(take(na * 8));
@@ -189,8 +228,8 @@ __global__ void bulk_init_kernel(MapDev m, BulkPlan pl, int ncursors) {
 }
 
 // Rows of the batch that can be promised a heap position.
-__device__ __forceinline__ int64_t rows_that_fit(const MapDev& m, const BulkPlan& pl) {
-    const int64_t room = static_cast<int64_t>(m.capacity) - pl.hdr[kHdrBase];
+__device__ __forceinline__ int64_t rows_that_fit(const MapDev& m, const BulkPlan& pl, int32_t heap_base) {
+    const int64_t room = static_cast<int64_t>(m.capacity) - heap_base;
     return room < 0 ? 0 : (room < pl.n ? room : pl.n);
 }
 
@@ -325,8 +364,8 @@ __global__ __launch_bounds__(kSplitThreads) void split_keys_kernel(
     }
     __syncthreads();
     const int bin_shift = kPartShift + static_cast<int>(pl.fine_shift);
-    const int64_t fit = PROV ? rows_that_fit(m, pl) : pl.n;
-    const int64_t heap_base = PROV ? pl.hdr[kHdrBase] : 0;
+    const int32_t heap_base = PROV ? pl.hdr[kHdrBase] : 0;
+    const int64_t fit = PROV ? rows_that_fit(m, pl, heap_base) : pl.n;
     uint64_t code[kSplitKeys];
     int32_t aux[kSplitKeys];
     int bin[kSplitKeys];
@@ -400,6 +439,153 @@ __global__ __launch_bounds__(kSplitThreads) void split_keys_kernel(
         if (tid == 0 &&
             atomicAdd(pl.hdr + kHdrTicket, 1) == static_cast<int32_t>(gridDim.x) - 1) {
             leave_word(early, atomicAdd(pl.hdr + kHdrSpillKeys, 0), stamp);
+        }
+    }
+}
+
+// The one split pass of an insert that needs no more: a chunk's records are sorted by
+// partition and left in the chunk's own place, with where each partition starts, and
+// the build pass collects a partition's records from all chunks (1 M keys into 2 M: 652
+// partitions, 245 chunks, six records a time).  Nothing is reserved and nothing can
+// overflow here, so there are no cursors and no atomics but those in LDS; both the
+// codes and the starts are written front to back.  Two passes read and write the
+// records once more and want their cursors cleared by a launch in front: 1 M keys 1.9 +
+// 13.3 + 8.6 us, now 11.2, for 3.5 us more in the build pass (25.3 -> 28.8), whose
+// look for a record's chunk is what more chunks make longer; 4 M keys into 8 M filled
+// and asked 206 -> 192, 4 M with rows into 6 M 361 -> 343.
+struct OnceShared {
+    int start[kOnceParts];     // counts, then first sorted positions
+    int wave_total[kSplitThreads / 64];
+    int losers;
+    int nspill;
+    int spill_first;
+    uint16_t aux[kSplitChunk];     // sorted position -> number of the record in the chunk
+    uint64_t stage[kSplitChunk];   // sorted position -> code
+};
+
+template <int DIM, bool PROV>
+__global__ __launch_bounds__(kSplitThreads) void split_once_kernel(
+        MapDev m, BulkPlan pl, const int32_t* __restrict__ keys, int identity,
+        uint64_t* early, int32_t stamp) {
+    __shared__ OnceShared sh;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int parts = static_cast<int>(pl.parts);
+    const int64_t base = static_cast<int64_t>(blockIdx.x) * kSplitChunk;
+    int32_t key[kSplitKeys][DIM];
+#pragma unroll
+    for (int k = 0; k < kSplitKeys; ++k) {   // (all asked for at once, as in split_keys_kernel)
+        const int64_t i = base + k * kSplitThreads + tid;
+        load_key<DIM>(keys, i < pl.n ? i : 0, true, key[k]);
+    }
+    for (int b = tid; b < parts; b += kSplitThreads) sh.start[b] = 0;
+    if (tid == 0) {
+        sh.losers = 0;
+        sh.nspill = 0;
+    }
+    __syncthreads();
+    const int32_t heap_base = m.ctr[kCtrSize];   // (nothing changes it before the build pass)
+    const int64_t fit = PROV ? rows_that_fit(m, pl, heap_base) : pl.n;
+    uint64_t code[kSplitKeys];
+    int bin[kSplitKeys];
+    int rank[kSplitKeys];
+    int spill_rank[kSplitKeys];
+#pragma unroll
+    for (int k = 0; k < kSplitKeys; ++k) {
+        const int64_t i = base + k * kSplitThreads + tid;
+        const bool active = i < pl.n;
+        const bool fits = pack_key<DIM>(key[k], code[k]);
+        bin[k] = -1;
+        rank[k] = 0;
+        spill_rank[k] = -1;
+        if (active && fits && i < fit) {
+            bin[k] = static_cast<int>(bucket_of(code[k], m.nb) >> kPartShift);
+            rank[k] = atomicAdd(&sh.start[bin[k]], 1);
+            if constexpr (PROV) {
+                pl.flags[i] = 0;
+                if (identity) __builtin_nontemporal_store(code[k], m.klog + heap_base + i);
+            }
+        } else if (active) {
+            spill_rank[k] = atomicAdd(&sh.nspill, 1);   // (as in split_keys_kernel)
+            if constexpr (PROV) pl.flags[i] = 1;
+        }
+    }
+    __syncthreads();
+    // the launch's place: rows on the spill list below, workgroups that are done above
+    unsigned long long* place = reinterpret_cast<unsigned long long*>(m.ctr + kCtrCursors) + pl.once_slot;
+    constexpr unsigned long long kDone = 1ull << 32;
+    if (tid == 0 && sh.nspill) {
+        sh.spill_first = static_cast<int>(atomicAdd(place, static_cast<unsigned long long>(sh.nspill)));
+    }
+    // running sums of the counts, four to a thread
+    static_assert(kOnceParts == 4 * kSplitThreads, "a thread adds up four counts");
+    int own[4], sum = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        own[q] = 4 * tid + q < parts ? sh.start[4 * tid + q] : 0;
+        sum += own[q];
+    }
+    int incl = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int up = __shfl_up(incl, d);
+        if (lane >= d) incl += up;
+    }
+    if (lane == 63) sh.wave_total[tid >> 6] = incl;
+    __syncthreads();
+    int at = incl - sum, total = 0;
+#pragma unroll
+    for (int w = 0; w < kSplitThreads / 64; ++w) {
+        if (w < (tid >> 6)) at += sh.wave_total[w];
+        total += sh.wave_total[w];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        if (4 * tid + q < parts) sh.start[4 * tid + q] = at;
+        at += own[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kSplitKeys; ++k) {
+        if (bin[k] >= 0) {
+            const int sp = sh.start[bin[k]] + rank[k];
+            sh.stage[sp] = code[k];
+            if constexpr (PROV) sh.aux[sp] = static_cast<uint16_t>(k * kSplitThreads + tid);
+        }
+        if (spill_rank[k] >= 0) {
+            pl.spill_keys[sh.spill_first + spill_rank[k]] =
+                    static_cast<int32_t>(base + k * kSplitThreads + tid);
+        }
+    }
+    uint16_t* starts = pl.starts + static_cast<int64_t>(blockIdx.x) * (parts + 1);
+    for (int b = tid; b <= parts; b += kSplitThreads) {
+        starts[b] = static_cast<uint16_t>(b < parts ? sh.start[b] : total);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kSplitKeys; ++j) {
+        const int t = j * kSplitThreads + tid;
+        if (t < total) {
+            pl.codes_a[base + t] = sh.stage[t];
+            if constexpr (PROV) pl.rows_once[base + t] = sh.aux[t];
+        }
+    }
+    // The workgroup that finishes last makes the header for the passes that follow
+    // (bulk_init_kernel in front of the other split) and tells the host, as in
+    // split_keys_kernel.  (Its own place on the list has come back to the thread that
+    // counts the workgroup done.)
+    __syncthreads();
+    if (tid == 0) {
+        const unsigned long long at = atomicAdd(place, kDone);
+        if (at >> 32 == gridDim.x - 1u) {
+            const int32_t spilled = static_cast<int32_t>(static_cast<uint32_t>(at));
+            atomicExch(place, 0ull);
+            for (int w = 0; w < kHdrWords; ++w) pl.hdr[w] = 0;
+            pl.hdr[kHdrSpillKeys] = spilled;
+            if constexpr (PROV) pl.hdr[kHdrLosers] = spilled;
+            pl.hdr[kHdrBase] = heap_base;
+            pl.hdr[kHdrWasEmpty] = (heap_base == 0 && m.ctr[kCtrTombs] == 0) ? 1 : 0;
+            if (early != nullptr) leave_word(early, spilled, stamp);
         }
     }
 }
@@ -619,7 +805,10 @@ enum { kRecIdle = 0, kRecPlaced = 1, kRecLost = 2 };
 constexpr int kWaitList = 128;
 
 // (four wavefronts per SIMD: the two workgroups that the LDS holds)
-template <bool PROV, bool TOMBS>
+// ONCE: the records come from one split pass, a few from each chunk.  A workgroup adds
+// up how many there are in each and finds the chunk of a record by halving; workgroups
+// of one XCD take neighbouring partitions, whose records share lines.
+template <bool PROV, bool TOMBS, bool ONCE>
 __global__ __launch_bounds__(kBuildThreads, 4) void build_kernel(
         MapDev m, BulkPlan pl, int stale, int identity) {
     // Records per thread and round.  With rows the partitions of a batch of the
@@ -648,16 +837,75 @@ __global__ __launch_bounds__(kBuildThreads, 4) void build_kernel(
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
-    const uint32_t p = blockIdx.x;
-    int cnt = pl.cursor_part[p];
-    if (cnt > static_cast<int>(pl.cap_part)) cnt = static_cast<int>(pl.cap_part);
+    // ONCE: records of the chunks before a chunk (none beyond the last), and where the
+    // chunk's first record of this partition would lie if it were record 0
+    __shared__ int s_before[ONCE ? kOnceChunks : 1];
+    __shared__ int s_from[ONCE ? kOnceChunks : 1];
+    const uint32_t p = ONCE ? (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
     const uint32_t b0 = p << kPartShift;
-    if (b0 >= m.nb) return;
+    if (p >= pl.parts || b0 >= m.nb) return;
+    const bool was_empty = pl.hdr[kHdrWasEmpty] != 0;
     const int nbk = static_cast<int>(m.nb - b0 < static_cast<uint32_t>(kPartBuckets)
                                              ? m.nb - b0
                                              : static_cast<uint32_t>(kPartBuckets));
+    int cnt = 0;
+    if constexpr (ONCE) {
+        static_assert(kOnceChunks == 2 * kBuildThreads, "a thread adds up two chunks");
+        int first[2], own[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int c = 2 * tid + q;
+            first[q] = own[q] = 0;
+            if (c < static_cast<int>(pl.once_chunks)) {
+                const uint16_t* at = pl.starts + static_cast<int64_t>(c) * (pl.parts + 1) + p;
+                first[q] = at[0];
+                own[q] = at[1] - at[0];
+            }
+        }
+        // (an empty range is made while they come)
+        if (was_empty) {
+            for (int t = tid; t < nbk * kGroup; t += kBuildThreads) {
+                tab[staged(t >> 3, t & 7)] = make_uint4(~0u, ~0u, ~0u, ~0u);
+            }
+        }
+        int incl = own[0] + own[1];
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int up = __shfl_up(incl, d);
+            if (lane >= d) incl += up;
+        }
+        if (lane == 63) s_wcnt[wave] = incl;
+        __syncthreads();
+        int before = incl - own[0] - own[1];
+#pragma unroll
+        for (int w = 0; w < kBuildThreads / 64; ++w) {
+            if (w < wave) before += s_wcnt[w];
+            cnt += s_wcnt[w];
+        }
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int c = 2 * tid + q;
+            s_before[c] = c < static_cast<int>(pl.once_chunks) ? before : 0x7FFFFFFF;
+            s_from[c] = c * kSplitChunk + first[q] - before;
+            before += own[q];
+        }
+        __syncthreads();
+    } else {
+        cnt = pl.cursor_part[p];
+    }
+    // record r of the partition -> its place in codes_a (and its chunk)
+    auto place_of = [&](int r, int& chunk) {
+        int c = 0;
+        for (int step = static_cast<int>(pl.once_halving); step > 0; step >>= 1) {
+            if (s_before[c + step] <= r) c += step;
+        }
+        chunk = c;
+        return s_from[c] + r;
+    };
     uint4* __restrict__ gl =
             reinterpret_cast<uint4*>(m.buckets) + static_cast<size_t>(b0) * kGroup;
+    const int all = cnt;   // of which those beyond the partition's capacity are left to the per-key kernel
+    if (cnt > static_cast<int>(pl.cap_part)) cnt = static_cast<int>(pl.cap_part);
     if (cnt == 0) {
         if (stale) {
             for (int t = tid; t < nbk * kGroup; t += kBuildThreads) {
@@ -666,7 +914,6 @@ __global__ __launch_bounds__(kBuildThreads, 4) void build_kernel(
         }
         return;
     }
-    const bool was_empty = pl.hdr[kHdrWasEmpty] != 0;
     const bool counted = was_empty && cnt <= kCountedRounds * kRound;
     const int32_t heap_base = pl.hdr[kHdrBase];
     const int64_t bbase = static_cast<int64_t>(p) * pl.cap_part;
@@ -685,16 +932,25 @@ __global__ __launch_bounds__(kBuildThreads, 4) void build_kernel(
         for (int k = 0; k < kRecs; ++k) {
             const int r = rb + k * kBuildThreads + tid;
             const bool take = r < cnt && ((only >> k) & 1u);
-            codes[k] = take ? __builtin_nontemporal_load(pl.codes_b + bbase + r) : 0ull;
-            if constexpr (PROV) rows[k] = take ? __builtin_nontemporal_load(pl.rows_b + bbase + r) : 0;
+            if constexpr (ONCE) {
+                int chunk;
+                const int at = place_of(take ? r : 0, chunk);
+                codes[k] = take ? pl.codes_a[at] : 0ull;
+                if constexpr (PROV) rows[k] = take ? chunk * kSplitChunk + pl.rows_once[at] : 0;
+            } else {
+                codes[k] = take ? __builtin_nontemporal_load(pl.codes_b + bbase + r) : 0ull;
+                if constexpr (PROV) rows[k] = take ? __builtin_nontemporal_load(pl.rows_b + bbase + r) : 0;
+            }
         }
     };
     // The first round's records are requested before the table range is
     // staged, so that both latencies overlap.
     load_round(0, ~0u);
-    for (int t = tid; t < nbk * kGroup; t += kBuildThreads) {
-        tab[staged(t >> 3, t & 7)] =
-                was_empty ? make_uint4(~0u, ~0u, ~0u, ~0u) : gl[t];
+    if (!ONCE || !was_empty) {
+        for (int t = tid; t < nbk * kGroup; t += kBuildThreads) {
+            tab[staged(t >> 3, t & 7)] =
+                    was_empty ? make_uint4(~0u, ~0u, ~0u, ~0u) : gl[t];
+        }
     }
     for (int t = tid; t < static_cast<int>(kPartBuckets); t += kBuildThreads) {
         s_drawn[t] = 0;
@@ -899,6 +1155,18 @@ __global__ __launch_bounds__(kBuildThreads, 4) void build_kernel(
             probe_round(mine, state, wslot);
             settle_round(state, wslot);
         }
+    }
+    if constexpr (ONCE) {
+        for (int r = cnt + tid; r < all; r += kBuildThreads) {
+            int chunk;
+            const int at = place_of(r, chunk);
+            if constexpr (PROV) {
+                give_up_row(pl, chunk * kSplitChunk + pl.rows_once[at], &s_losers, true);
+            } else {
+                pl.spill_a[atomicAdd(pl.hdr + kHdrSpillA, 1)] = at;
+            }
+        }
+        if constexpr (PROV) __syncthreads();   // (uniform: s_losers is final)
     }
     // (stores marked as not to be kept in the caches: nothing reads the range,
     // the value rows or the log entries again before a later call does; the
@@ -1110,74 +1378,20 @@ __device__ __forceinline__ void copy_plane(const MapDev& m, const BulkPlan& pl,
     if (tid < words - 4 * quads) move_word(4 * quads + tid);
 }
 
-__global__ __launch_bounds__(kCopyThreads) void copy_rows_kernel(
-        MapDev m, BulkPlan pl, ValueArgs va, int identity) {
-    const int32_t heap_base = pl.hdr[kHdrBase];
-    const int64_t winners = pl.n - pl.hdr[kHdrLosers];
-    for (int v = 0; v < va.n; ++v) {
-        const int rd = va.row_dwords[v];
-        switch (rd) {
-            case 1:
-                copy_plane<1>(m, pl, va.src[v], va.dst[v], rd, winners, heap_base, identity);
-                break;
-            case 2:
-                copy_plane<2>(m, pl, va.src[v], va.dst[v], rd, winners, heap_base, identity);
-                break;
-            case 3:
-                copy_plane<3>(m, pl, va.src[v], va.dst[v], rd, winners, heap_base, identity);
-                break;
-            case 4:
-                copy_plane<4>(m, pl, va.src[v], va.dst[v], rd, winners, heap_base, identity);
-                break;
-            default:
-                copy_plane<0>(m, pl, va.src[v], va.dst[v], rd, winners, heap_base, identity);
-                break;
-        }
-    }
-}
-
-// Positions of `mine` set lanes of the workgroup in a list that grows through
-// the counter `cursor`: one update of the counter per workgroup (updates of a
-// single address serialise across the device).  Every thread calls this; the
-// return value is the caller's position (meaningful when `mine`).
-constexpr int kListThreads = 1024;
-
-__device__ __forceinline__ int reserve_in_list(bool mine, int32_t* cursor, int* s_wave,
-                                               int* s_first) {
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const uint64_t mm = __ballot(mine);
-    if (lane == 0) s_wave[wave] = __popcll(mm);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int tot = 0;
-        for (int q = 0; q < kListThreads / 64; ++q) {
-            const int c = s_wave[q];
-            s_wave[q] = tot;
-            tot += c;
-        }
-        *s_first = tot ? atomicAdd(cursor, tot) : 0;
-    }
-    __syncthreads();
-    const int at = *s_first + s_wave[wave] + __popcll(mm & ((1ull << lane) - 1ull));
-    __syncthreads();   // s_wave / s_first are reused by the next call
-    return at;
-}
-
 // Provisional scheme, only when rows lost: the losers below row U are the
 // holes that the winners at or beyond U move into.  Sixteen flags per thread;
 // a workgroup that meets no loser (the usual case: a handful of rows lost among
 // millions) goes on without touching the list.
-__global__ __launch_bounds__(kListThreads) void list_holes_kernel(BulkPlan pl) {
-    __shared__ int s_wave[kListThreads / 64];
+__device__ __forceinline__ void list_holes(const BulkPlan& pl) {
+    __shared__ int s_wave[kCopyThreads / 64];
     __shared__ int s_first;
     const int32_t losers = pl.hdr[kHdrLosers];
     if (losers == 0) return;
     const int64_t winners = pl.n - losers;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
-    for (int64_t first = static_cast<int64_t>(blockIdx.x) * kListThreads * 16; first < winners;
-         first += static_cast<int64_t>(gridDim.x) * kListThreads * 16) {
+    for (int64_t first = static_cast<int64_t>(blockIdx.x) * kCopyThreads * 16; first < winners;
+         first += static_cast<int64_t>(gridDim.x) * kCopyThreads * 16) {
         const int64_t i0 = first + static_cast<int64_t>(threadIdx.x) * 16;
         uint32_t w[4] = {0u, 0u, 0u, 0u};
         if (i0 + 16 <= winners) {
@@ -1209,7 +1423,7 @@ __global__ __launch_bounds__(kListThreads) void list_holes_kernel(BulkPlan pl) {
         __syncthreads();
         if (threadIdx.x == 0) {
             int tot = 0;
-            for (int q = 0; q < kListThreads / 64; ++q) {
+            for (int q = 0; q < kCopyThreads / 64; ++q) {
                 const int c = s_wave[q];
                 s_wave[q] = tot;
                 tot += c;
@@ -1225,6 +1439,61 @@ __global__ __launch_bounds__(kListThreads) void list_holes_kernel(BulkPlan pl) {
         }
         __syncthreads();   // s_wave / s_first are reused by the next round
     }
+}
+
+__global__ __launch_bounds__(kCopyThreads) void copy_rows_kernel(
+        MapDev m, BulkPlan pl, ValueArgs va, int identity) {
+    const int32_t heap_base = pl.hdr[kHdrBase];
+    const int64_t winners = pl.n - pl.hdr[kHdrLosers];
+    for (int v = 0; v < va.n; ++v) {
+        const int rd = va.row_dwords[v];
+        switch (rd) {
+            case 1:
+                copy_plane<1>(m, pl, va.src[v], va.dst[v], rd, winners, heap_base, identity);
+                break;
+            case 2:
+                copy_plane<2>(m, pl, va.src[v], va.dst[v], rd, winners, heap_base, identity);
+                break;
+            case 3:
+                copy_plane<3>(m, pl, va.src[v], va.dst[v], rd, winners, heap_base, identity);
+                break;
+            case 4:
+                copy_plane<4>(m, pl, va.src[v], va.dst[v], rd, winners, heap_base, identity);
+                break;
+            default:
+                copy_plane<0>(m, pl, va.src[v], va.dst[v], rd, winners, heap_base, identity);
+                break;
+        }
+    }
+    list_holes(pl);
+}
+
+// Positions of `mine` set lanes of the workgroup in a list that grows through
+// the counter `cursor`: one update of the counter per workgroup (updates of a
+// single address serialise across the device).  Every thread calls this; the
+// return value is the caller's position (meaningful when `mine`).
+constexpr int kListThreads = 1024;
+
+__device__ __forceinline__ int reserve_in_list(bool mine, int32_t* cursor, int* s_wave,
+                                               int* s_first) {
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const uint64_t mm = __ballot(mine);
+    if (lane == 0) s_wave[wave] = __popcll(mm);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int tot = 0;
+        for (int q = 0; q < kListThreads / 64; ++q) {
+            const int c = s_wave[q];
+            s_wave[q] = tot;
+            tot += c;
+        }
+        *s_first = tot ? atomicAdd(cursor, tot) : 0;
+    }
+    __syncthreads();
+    const int at = *s_first + s_wave[wave] + __popcll(mm & ((1ull << lane) - 1ull));
+    __syncthreads();   // s_wave / s_first are reused by the next call
+    return at;
 }
 
 // The slot that holds `code` (which is stored), by one lane on its own.
@@ -1259,7 +1528,7 @@ __global__ __launch_bounds__(kListThreads) void settle_rows_kernel(
         m.ctr[kCtrSize] = heap_base + static_cast<int32_t>(winners);
     }
     if (losers == 0) return;
-    const int64_t fit = rows_that_fit(m, pl);
+    const int64_t fit = rows_that_fit(m, pl, heap_base);
     for (int64_t first = winners + static_cast<int64_t>(blockIdx.x) * kListThreads; first < fit;
          first += static_cast<int64_t>(gridDim.x) * kListThreads) {
         const int64_t i = first + threadIdx.x;
@@ -1306,6 +1575,19 @@ int check_values(int n_values, const void* const* src, void* const* dst,
 }
 
 template <bool PROV>
+int launch_split_once(ash_map* map, BulkPlan pl, const int32_t* keys, int identity,
+                      uint64_t* early, int32_t stamp, hipStream_t s) {
+    pl.once_slot = next_slot(map);
+    auto kernel = map->key_dim == 1   ? split_once_kernel<1, PROV>
+                  : map->key_dim == 2 ? split_once_kernel<2, PROV>
+                  : map->key_dim == 3 ? split_once_kernel<3, PROV>
+                                      : split_once_kernel<4, PROV>;
+    kernel<<<pl.once_chunks, kSplitThreads, 0, s>>>(map->d, pl, keys, identity, early, stamp);
+    ASH_LAUNCH_CHECK();
+    return 0;
+}
+
+template <bool PROV>
 int launch_split_keys(ash_map* map, const BulkPlan& pl, const int32_t* keys, int identity,
                       uint64_t* early, int32_t stamp, hipStream_t s) {
     const unsigned g = static_cast<unsigned>((pl.n + kSplitChunk - 1) / kSplitChunk);
@@ -1327,12 +1609,34 @@ int launch_split_keys(ash_map* map, const BulkPlan& pl, const int32_t* keys, int
     return 0;
 }
 
+// The passes up to the build of an insert: split once, or twice.
+template <bool PROV>
+int launch_split_and_build(ash_map* map, const BulkPlan& pl, const int32_t* keys, int stale,
+                           int identity, uint64_t* early, int32_t stamp, hipStream_t s) {
+    if (pl.once) {
+        if (launch_split_once<PROV>(map, pl, keys, identity, early, stamp, s)) return 1;
+        auto build = tombs_in(map) ? build_kernel<PROV, true, true> : build_kernel<PROV, false, true>;
+        build<<<8 * ((pl.parts + 7) / 8), kBuildThreads, 0, s>>>(map->d, pl, stale, identity);
+    } else {
+        const int ncursors = static_cast<int>(pl.bins << pl.fine_shift);   // (>= bins << lane_shift)
+        const int ninit = ncursors > kHdrWords ? ncursors : kHdrWords;
+        bulk_init_kernel<<<(ninit + 255) / 256, 256, 0, s>>>(map->d, pl, ncursors);
+        ASH_LAUNCH_CHECK();
+        if (launch_split_keys<PROV>(map, pl, keys, identity, early, stamp, s)) return 1;
+        split_records_kernel<PROV><<<(pl.bins << pl.lane_shift) * pl.chunks, kSplitThreads, 0, s>>>(map->d, pl);
+        ASH_LAUNCH_CHECK();
+        auto build = tombs_in(map) ? build_kernel<PROV, true, false> : build_kernel<PROV, false, false>;
+        build<<<pl.parts, kBuildThreads, 0, s>>>(map->d, pl, stale, identity);
+    }
+    ASH_LAUNCH_CHECK();
+    map->table_stale = map->table_filled = false;
+    return 0;
+}
+
 int launch_settle_rows(ash_map* map, const BulkPlan& pl, const int32_t* keys,
                        const ValueArgs& va, int identity, hipStream_t s) {
-    // both leave at once when no row lost: grids that cost little to launch
+    // leaves at once when no row lost: a grid that costs little to launch
     constexpr unsigned g = 128;
-    list_holes_kernel<<<g, kListThreads, 0, s>>>(pl);
-    ASH_LAUNCH_CHECK();
     switch (map->key_dim) {
         case 1:
             settle_rows_kernel<1><<<g, kListThreads, 0, s>>>(map->d, pl, keys, va, identity);
@@ -1380,12 +1684,11 @@ int ash_map_bulk_workspace_bytes(ash_map_t* map, int64_t n, int n_values,
                                  : (n >= (int64_t{1} << 20) && n >= nb));
         // A table that was emptied (or made) and not used since still has to
         // be filled before the per-key kernel can run; the build pass writes
-        // every range anyway and saves that fill.  Measured for such tables:
-        // the streaming path wins from 2^18 keys and a third of a key per
-        // bucket (half with value rows): 1 M keys into a new table of capacity
-        // 2 M take 77 us instead of 138.  Not for batches far beyond what the
-        // table holds (piles of duplicates would queue on a few ranges).
-        if (map->table_stale && streams_into_emptied(n, nb) &&
+        // every range anyway and saves that fill: the streaming path wins from
+        // 2^18 keys and a third of a key per bucket (half with value rows).  Not
+        // for batches far beyond what the table holds (piles of duplicates would
+        // queue on a few ranges).
+        if (map->table_stale && n >= (int64_t{1} << 18) && n <= 12 * nb &&
             (n_values > 0 ? 2 * n >= nb : 3 * n >= nb)) {
             big = true;
         }
@@ -1448,18 +1751,8 @@ int ash::insert_bulk(ash_map* map, const int32_t* keys, int64_t n,
         }
         return 0;
     };
-    const int ncursors = static_cast<int>(pl.bins << pl.fine_shift);   // (>= bins << lane_shift)
-    const int ninit = ncursors > kHdrWords ? ncursors : kHdrWords;
-    bulk_init_kernel<<<(ninit + 255) / 256, 256, 0, s>>>(map->d, pl, ncursors);
-    ASH_LAUNCH_CHECK();
     if (n_values == 0) {
-        if (launch_split_keys<false>(map, pl, keys, identity, early, stamp, s)) return 1;
-        split_records_kernel<false><<<(pl.bins << pl.lane_shift) * pl.chunks, kSplitThreads, 0, s>>>(map->d, pl);
-        ASH_LAUNCH_CHECK();
-        auto build = tombs_in(map) ? build_kernel<false, true> : build_kernel<false, false>;
-        build<<<pl.parts, kBuildThreads, 0, s>>>(map->d, pl, stale, identity);
-        ASH_LAUNCH_CHECK();
-        map->table_stale = map->table_filled = false;
+        if (launch_split_and_build<false>(map, pl, keys, stale, identity, early, stamp, s)) return 1;
         if (none_spilled(publish)) return 1;
         // (the first pass alone writes that list)
         if (publish.landing == nullptr &&
@@ -1468,13 +1761,7 @@ int ash::insert_bulk(ash_map* map, const int32_t* keys, int64_t n,
         }
         return insert_selected(map, true, pl.codes_a, pl.spill_a, pl.hdr + kHdrSpillA, none, s, publish);
     }
-    if (launch_split_keys<true>(map, pl, keys, identity, early, stamp, s)) return 1;
-    split_records_kernel<true><<<(pl.bins << pl.lane_shift) * pl.chunks, kSplitThreads, 0, s>>>(map->d, pl);
-    ASH_LAUNCH_CHECK();
-    auto build = tombs_in(map) ? build_kernel<true, true> : build_kernel<true, false>;
-    build<<<pl.parts, kBuildThreads, 0, s>>>(map->d, pl, stale, identity);
-    ASH_LAUNCH_CHECK();
-    map->table_stale = map->table_filled = false;
+    if (launch_split_and_build<true>(map, pl, keys, stale, identity, early, stamp, s)) return 1;
     int64_t words = 0;
     for (int v = 0; v < n_values; ++v) words = words > n * user.row_dwords[v] ? words : n * user.row_dwords[v];
     int64_t blocks = (words + kCopyThreads - 1) / kCopyThreads;
@@ -1500,7 +1787,7 @@ int ash_map_erase_bulk_query(ash_map_t* map, int64_t n, int64_t* bytes, int* wor
     if (map == nullptr) ASH_FAIL("null map handle");
     if (bytes == nullptr) ASH_FAIL("null output pointer");
     BulkPlan pl;
-    *bytes = make_plan(map, n, 0, nullptr, nullptr, pl);
+    *bytes = make_plan(map, n, 0, nullptr, nullptr, pl, false);
     if (worthwhile) {
         // The range pass reads the whole table and writes back what changed; the
         // per-key kernel is bound by the device's atomic rate (19 G keys/s).
@@ -1521,7 +1808,7 @@ int ash_map_erase_bulk(ash_map_t* map, const int32_t* keys, int64_t n, void* wor
         ASH_FAIL("bulk workspace must be 256-byte aligned");
     }
     BulkPlan pl;
-    const int64_t need = make_plan(map, n, 0, nullptr, static_cast<char*>(workspace), pl);
+    const int64_t need = make_plan(map, n, 0, nullptr, static_cast<char*>(workspace), pl, false);
     if (need == 0) ASH_FAIL("the bulk path does not apply to this batch");
     if (workspace_bytes < need) ASH_FAIL("bulk workspace too small");
     DeviceGuard guard;

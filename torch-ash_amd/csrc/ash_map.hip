@@ -2227,15 +2227,14 @@ class ClearList {
 // What a clear does of a map whose state the host knows, and what makes a new one
 // (`fresh`): counters, heap and second region are reset at once.  The bucket array is
 // left to the next call that needs it (settle_table) -- a streaming insert writes
-// every bucket itself -- unless the table is too small for any batch to be streamed
-// into it (streams_into_emptied: 2^18 keys, at most twelve per bucket); such a table
-// is at most 2.8 MB, filled here without a launch of its own.  The key log is left
+// every bucket itself -- unless the table is so small that it is filled here, without
+// a launch of its own (kFillAtOnce).  The key log is left
 // alone while the heap is in its initial order (no listing reads an entry beyond the
 // size then), or emptied with the heap's order.
 int clear_lazily(ash_map* map, hipStream_t s, bool fresh, const ClearRows& rows) {
     ClearList list;
     list.add(rows);
-    const bool small = !streams_into_emptied(int64_t{1} << 18, map->d.nb);
+    const bool small = static_cast<int64_t>(map->d.nb) <= kFillAtOnce;
     if (small) list.add(map->d.buckets, static_cast<int64_t>(map->d.nb) * kGroup * 16, ~0u);
     if (map->general_attached) list.add(map->d.gstate, static_cast<int64_t>(map->d.gslots) * 4, ~0u);
     const bool keep_log = !map->heap_dirty;
@@ -2415,10 +2414,6 @@ int settle_landing_place(ash_map* map) {
 
 namespace {
 
-// A place among the counters for a launch whose workgroups count themselves.  Launches
-// on one stream could share one; as many as there are places may run at a time on
-// several (a captured launch keeps its own).
-int next_slot(ash_map* map) { return static_cast<int>(map->launches.fetch_add(1) % kLaunchSlots); }
 int32_t* next_ticket(ash_map* map) { return map->d.ctr + kCtrTickets + next_slot(map); }
 
 // Keys up to which a launch leaves the counters itself (leave_with_last), instead

@@ -162,6 +162,11 @@ inline bool is_capturing(hipStream_t s) {
     return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
 }
 
+// A place among the counters for a launch whose workgroups count themselves.  Launches
+// on one stream could share one; as many as there are places may run at a time on
+// several (a captured launch keeps its own).
+inline int next_slot(ash_map* map) { return static_cast<int>(map->launches.fetch_add(1) % kLaunchSlots); }
+
 // Whether the heap array is known to be 0, 1, 2, ...
 inline bool heap_in_order(const ash_map* map) { return !map->heap_dirty && !map->replayed; }
 
@@ -221,11 +226,9 @@ int insert_bulk(ash_map* map, const int32_t* keys, int64_t n, int n_values,
                 const void* const* src, void* const* dst, const int64_t* row_bytes,
                 void* workspace, int64_t workspace_bytes, uint64_t* early, uint64_t* late,
                 int32_t stamp, bool* published, void* stream);
-// Whether a batch is one to stream into a table of nb buckets that has been emptied
-// (or made) and not used since, by the numbers of both (ash_map_bulk_workspace_bytes).
-inline bool streams_into_emptied(int64_t n, int64_t nb) {
-    return n >= (int64_t{1} << 18) && n <= 12 * nb;
-}
+// Buckets up to which a clear fills the table at once, in the launch that resets the
+// counters (2.8 MB, half a microsecond of stores where a streaming insert follows).
+constexpr int64_t kFillAtOnce = 21845;
 // Fills the bucket array if a clear() left that to the next user of the table.
 int settle_table(ash_map* map, hipStream_t s);
 // Before the first call that writes to the heap (an erase; a load brings a

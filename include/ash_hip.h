@@ -421,7 +421,12 @@ int ash_map_erase_bulk(ash_map_t* map, const int32_t* keys, int64_t n, void* wor
  * queues launches (no upkeep, no look at the counters): refused keys and keys
  * waiting for the second region stay in the counters.  `staging` as for
  * ash_map_counters. */
-enum { ASH_STREAMING_AUTO = 0, ASH_STREAMING_ALWAYS = 1, ASH_STREAMING_NEVER = 2 };
+enum { ASH_STREAMING_AUTO = 0, ASH_STREAMING_ALWAYS = 1, ASH_STREAMING_NEVER = 2,
+       /* inserts only: as AUTO, and in batches from 2^16 keys (2^17 with value rows)
+        * into tables emptied and not used since, where they pay off as long as most
+        * of the keys are not repeated; the package's own choice.  (AUTO keeps the
+        * bars by which callers have sized their scratch.) */
+       ASH_STREAMING_EARLY = 3 };
 enum { ASH_NEEDS_GENERAL = 2 };
 int ash_map_insert_scratch_bytes(ash_map_t* map, int64_t n, int n_values,
                                  const int64_t* row_bytes, int policy, int64_t* bytes);

@@ -183,3 +183,30 @@ def test_replays_of_a_streamed_insert(ash):
         s.insert(_keys(20_000, 8_000))
         s.erase(_keys(5_000, 23_000))
         assert s.size() == 0
+
+
+def test_which_batches_stream_early(monkeypatch):
+    """The bars of ASH_STREAMING_EARLY (3) on new tables and on tables in use, and what
+    ASH_STREAMING_AUTO (0) says to the same: scratch is asked for or not."""
+    import ctypes
+
+    import ash
+
+    def wanted(engine, n, policy, rows=()):
+        nbytes = ctypes.c_int64(-1)
+        widths = (ctypes.c_int64 * max(1, len(rows)))(*rows)
+        backend = engine.backend
+        backend._check(backend._lib.ash_map_insert_scratch_bytes(
+            backend._handle, n, len(rows), widths if rows else None, policy, ctypes.byref(nbytes)))
+        return nbytes.value > 0
+
+    engine = ash.ASHEngine(3, 300_000, DEV)          # 50 176 buckets
+    assert wanted(engine, 1 << 16, 3) and not wanted(engine, (1 << 16) - 1, 3)
+    assert wanted(engine, 1 << 17, 3, (12, 4)) and not wanted(engine, (1 << 17) - 1, 3, (12, 4))
+    assert not wanted(engine, 1 << 16, 0) and not wanted(engine, 1 << 17, 0, (12, 4))
+    assert not wanted(engine, 13 * 50_176, 3)        # piles
+    wide = ash.ASHEngine(3, 1_200_000, DEV)          # 200 192 buckets
+    assert not wanted(wide, 1 << 16, 3) and wanted(wide, 1 << 17, 3)
+    engine.find(_keys(0, 10))                        # in use from here on
+    assert not wanted(engine, 1 << 17, 3) and not wanted(engine, 1 << 18, 3, (12, 4))
+    assert wanted(engine, 1 << 18, 3) and not wanted(engine, 1 << 18, 0)

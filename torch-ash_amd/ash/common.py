@@ -353,6 +353,7 @@ GENERAL_JUST_IN_CASE_BYTES = 20 << 16
 BULK_INSERT = os.environ.get("ASH_BULK_INSERT", "auto")
 BULK_ERASE = os.environ.get("ASH_BULK_ERASE", "auto")
 _POLICY = {"auto": 0, "always": 1, "never": 2}   # the header's ASH_STREAMING_*
+_INSERT_POLICY = {**_POLICY, "auto": 3}          # ... ASH_STREAMING_EARLY
 NEEDS_GENERAL = 2                                # the header's ASH_NEEDS_GENERAL
 _DTYPE = {torch.float32: 0, torch.float64: 1}
 
@@ -1402,7 +1403,7 @@ class _HashMap:
     def _insert(self, keys, names, values, stores) -> None:
         """One ash_map_insert_auto (a second one after the second region has
         been attached, the first time a key does not fit the packed code)."""
-        policy = _POLICY[BULK_INSERT]
+        policy = _INSERT_POLICY[BULK_INSERT]
         for _ in range(2):
             waiting = self._backend.host.insert(self._address, self.key_dim, self._index, self.capacity,
                                                 keys, names, values, stores, policy)

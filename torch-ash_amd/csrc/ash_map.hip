@@ -3567,7 +3567,7 @@ enum { kPathPerKey = 0, kPathAssigned = 1, kPathStreaming = 2 };
 
 int plan_insert(ash_map_t* map, int64_t n, int n_values, const int64_t* row_bytes, int policy,
                 int* path, int64_t* bytes) {
-    if (policy < ASH_STREAMING_AUTO || policy > ASH_STREAMING_NEVER) ASH_FAIL("unknown policy");
+    if (policy < ASH_STREAMING_AUTO || policy > ASH_STREAMING_EARLY) ASH_FAIL("unknown policy");
     if (n_values < 0) ASH_FAIL("negative value count");
     if (n_values > 0 && row_bytes == nullptr) ASH_FAIL("null value tables");
     *path = kPathPerKey;
@@ -3579,7 +3579,8 @@ int plan_insert(ash_map_t* map, int64_t n, int n_values, const int64_t* row_byte
         int64_t ws = 0;
         int worthwhile = 0;
         if (ash_map_bulk_workspace_bytes(map, n, n_values, row_bytes, &ws, &worthwhile)) return 1;
-        if (ws > 0 && (worthwhile || policy == ASH_STREAMING_ALWAYS)) {
+        if (ws > 0 && (worthwhile || policy == ASH_STREAMING_ALWAYS ||
+                       (policy == ASH_STREAMING_EARLY && streams_early(map, n, n_values, row_bytes)))) {
             *path = kPathStreaming;
             *bytes = ws;
         }

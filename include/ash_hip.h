@@ -723,6 +723,17 @@ int ash_query_backward_backward_accumulate(const ash_query_args* a,
 int ash_query_backward_both(const ash_query_args* a, const void* z, const void* grad_grad_offsets,
                             const void* z_second, void* grad_embeddings, void* grad_offsets,
                             int32_t accumulate, void* stream);
+/* The same three with every gradient with respect to the offsets times offset_scale,
+ * as written (grad_offsets) and as read (grad_grad_offsets): for positions of which
+ * the offsets are a multiple.  grad_grad_offsets and z_second: both NULL, or as for
+ * ash_query_backward_both. */
+int ash_query_backward_forward_scaled(const ash_query_args* a, const void* z, const void* grad_grad_offsets,
+                                      const void* z_second, void* grad_embeddings, void* grad_offsets,
+                                      double offset_scale, int32_t accumulate, void* stream);
+int ash_query_backward_backward_scaled(const ash_query_args* a, const void* grad_grad_offsets,
+                                       const void* z, void* grad_z, void* grad_embeddings,
+                                       double offset_scale, int32_t accumulate, void* stream);
+
 
 /* Replaces `convolution_forward` (ash/src/grid.cu:948-1043, pybind.cpp:33).
  * inputs / outputs scalar[num_embeddings, cells_per_grid, embedding_dim];

@@ -245,3 +245,34 @@ def test_few_queries_are_not_put_off(scene, monkeypatch, more):
     y, _ = grid(xq, "smooth_step")
     got = _grad(grid, (y**2).mean() + _norm_loss(y, xq, 0) + _norm_loss(y, xq, 2))
     assert put_off == [more == 0] * 2 and _close(got, want)
+
+
+@pytest.mark.parametrize("dtype,width,n", [
+    (dtype, width, n) for dtype in (torch.float32, torch.float64) for width in (1, 3, 4, 5, 16)
+    for n in (1, 1000)] + [(torch.float32, 4, 600_001), (torch.float32, 5, 600_001)])
+@pytest.mark.parametrize("cell_size", [0.015, 3.0])
+def test_gradients_by_positions_in_units_of_a_cell(gpu_ash, dtype, width, n, cell_size):
+    """The kernels multiply as torch divides: gradients with respect to the positions to
+    the bit, those that the atomics add up to the rounding of their order."""
+    grid = _make_grid(gpu_ash, 4, width, 1, dtype=dtype, seed=width, holes=2)
+    ops = list(_operands(grid, _queries(4, 1, n, seed=n, margin=1.0)))
+    g = torch.Generator().manual_seed(n)
+    z, u, z2 = ((torch.rand(n, w, generator=g, dtype=dtype) - 0.5).to(DEV) for w in (width, 3, width))
+    host = gpu_ash.grid_query.backend.host
+    tol = dict(rtol=1e-5 if dtype == torch.float32 else 1e-12, atol=1e-5 * n ** 0.5)
+
+    emb, off = host.query_backward_forward(z, ops, "smooth_step", True, True, None, cell_size)
+    emb1, off1 = host.query_backward_forward(z, ops, "smooth_step", True, True, None)
+    assert torch.equal(off, off1 / cell_size) and torch.allclose(emb, emb1, **tol)
+    none, off = host.query_backward_forward(z, ops, "smooth_step", False, True, None, cell_size)
+    assert none is None and torch.equal(off, off1 / cell_size)
+    for need_z, need_emb in ((True, True), (True, False), (False, True)):
+        gz, emb = host.query_backward_backward(u, z, ops, "linear", need_z, need_emb, None, cell_size)
+        gz1, emb1 = host.query_backward_backward(u / cell_size, z, ops, "linear", need_z, need_emb, None)
+        assert not need_z or torch.equal(gz, gz1)
+        assert not need_emb or torch.allclose(emb, emb1, **tol)
+    for need_off in (True, False):
+        emb, off = host.query_backward_both(z, u, z2, ops, "smooth_step", need_off, None, cell_size)
+        emb1, off1 = host.query_backward_both(z, u / cell_size, z2, ops, "smooth_step", need_off, None)
+        assert torch.allclose(emb, emb1, **tol)
+        assert not need_off or torch.equal(off, off1 / cell_size)

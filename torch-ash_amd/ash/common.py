@@ -318,6 +318,14 @@ _SIGNATURES = {
         ctypes.c_int,
         [ctypes.POINTER(_QueryArgs)] + [_PTR] * 5 + [ctypes.c_int32, _PTR],
     ),
+    "ash_query_backward_forward_scaled": (
+        ctypes.c_int,
+        [ctypes.POINTER(_QueryArgs), _PTR, _PTR, _PTR, _PTR, _PTR, ctypes.c_double, ctypes.c_int32, _PTR],
+    ),
+    "ash_query_backward_backward_scaled": (
+        ctypes.c_int,
+        [ctypes.POINTER(_QueryArgs), _PTR, _PTR, _PTR, _PTR, ctypes.c_double, ctypes.c_int32, _PTR],
+    ),
     "ash_query_backward_backward_accumulate": (
         ctypes.c_int,
         [ctypes.POINTER(_QueryArgs), _PTR, _PTR, _PTR, _PTR, _PTR],
@@ -952,6 +960,7 @@ class _Backend:
         need_offsets: bool = True,
         accumulate_into: Optional[torch.Tensor] = None,
         along=(),
+        cell_size: float = 1.0,
     ) -> Tuple[Optional[torch.Tensor], Optional[torch.Tensor]]:
         """(grad_embeddings, grad_offsets); an output that is not needed is
         None and its work (for grad_embeddings: dense zero fill + atomics) is
@@ -960,16 +969,19 @@ class _Backend:
         to that tensor, which is also what is returned.  `along`: what
         query_backward_backward has put off for the same queries, pairs
         (grad_grad_offsets, z), taken along in grad_embeddings -- the first pair
-        in the same pass over the queries."""
+        in the same pass over the queries.  `cell_size`: the offsets are positions
+        divided by it, and the gradients with respect to the offsets, here and in
+        `along`, are those with respect to the positions."""
         operands = [embeddings, offsets, grid_indices, cell_indices, masks, lut_grid_nb2grid_idx,
                     lut_cell_nb2cell_idx, lut_cell_nb2grid_nb]
         if not along:
             return self.host.query_backward_forward(
-                z, operands, interpolation, need_embeddings, need_offsets, accumulate_into)
+                z, operands, interpolation, need_embeddings, need_offsets, accumulate_into, cell_size)
         grad_embeddings, grad_offsets = self.host.query_backward_both(
-            z, *along[0], operands, interpolation, need_offsets, accumulate_into)
+            z, *along[0], operands, interpolation, need_offsets, accumulate_into, cell_size)
         for pair in along[1:]:
-            self.host.query_backward_backward(*pair, operands, interpolation, False, True, grad_embeddings)
+            self.host.query_backward_backward(*pair, operands, interpolation, False, True, grad_embeddings,
+                                              cell_size)
         return grad_embeddings, grad_offsets
 
     def query_backward_forward_onto(self, grad_embeddings, z, *operands, need_offsets: bool = True, **along):
@@ -979,11 +991,13 @@ class _Backend:
         return _Backend.query_backward_forward(self, z, *operands, need_offsets=need_offsets,
                                                accumulate_into=grad_embeddings, **along)[1]
 
-    def query_backward_backward_onto(self, grad_embeddings, grad_grad_offsets, z, *operands) -> None:
+    def query_backward_backward_onto(self, grad_embeddings, grad_grad_offsets, z, *operands,
+                                     cell_size: float = 1.0) -> None:
         """query_backward_backward with no other result than an embedding
         gradient added to `grad_embeddings`."""
         _Backend.query_backward_backward(self, None, grad_grad_offsets, z, *operands, need_z=False,
-                                         accumulate_into=grad_embeddings, need_offsets=False)
+                                         accumulate_into=grad_embeddings, need_offsets=False,
+                                         cell_size=cell_size)
 
     def query_backward_backward(
         self,
@@ -1005,13 +1019,14 @@ class _Backend:
         accumulate_into: Optional[torch.Tensor] = None,
         need_offsets: bool = True,
         later: bool = False,
+        cell_size: float = 1.0,
     ) -> Tuple[Optional[torch.Tensor], Optional[torch.Tensor], Optional[torch.Tensor]]:
         """(grad_z, grad_embeddings, zero grad_offsets); outputs that are not
         needed are None and their work is skipped.  `accumulate_into` as for
         query_backward_forward.  `later`: grad_embeddings comes without the
         contributions of this call (zeros, or `accumulate_into` as it is); the
         caller has query_backward_forward or query_backward_backward_onto add
-        them.  There is no grad_z then."""
+        them.  There is no grad_z then.  `cell_size` as there."""
         operands = [embeddings, offsets, grid_indices, cell_indices, masks, lut_grid_nb2grid_idx,
                     lut_cell_nb2cell_idx, lut_cell_nb2grid_nb]
         if later:
@@ -1019,13 +1034,16 @@ class _Backend:
                 grad_grad_offsets, z, operands, interpolation, accumulate_into)
         else:
             grad_z, grad_embeddings = self.host.query_backward_backward(
-                grad_grad_offsets, z, operands, interpolation, need_z, need_embeddings, accumulate_into)
+                grad_grad_offsets, z, operands, interpolation, need_z, need_embeddings, accumulate_into,
+                cell_size)
         # the offsets second-order term is not produced (ash/src/grid.cu:417-418)
         zeros = embeddings.new_zeros(grid_indices.shape[0], 3) if need_offsets else None
         return grad_z, grad_embeddings, zeros
 
     # for callers that drop the zero grad_offsets above
     WITHOUT_OFFSETS = {"need_offsets": False}
+    # the backward functions take `cell_size`
+    TAKES_CELL_SIZE = True
 
 
 class _HashMap:

@@ -92,7 +92,10 @@ class _FusedGridForward(torch.autograd.Function):
                               again)
         ctx.grid_dim = grid_dim
         ctx.interpolation = interpolation
-        ctx.cell_size = cell_size
+        # d cell / d x of x -> (x - origin) / cell_size: within the backward kernels
+        # where they take it, else a division behind them
+        within = getattr(backend, "TAKES_CELL_SIZE", False)
+        ctx.cell_size, ctx.divide_by = (cell_size, 1.0) if within else (1.0, cell_size)
         ctx.spent = False
         ctx.outliving = None
         ctx.later = grid_query._Later() if hasattr(backend, "query_backward_backward_onto") else None
@@ -106,7 +109,8 @@ class _FusedGridForward(torch.autograd.Function):
         if z is None:   # only the gradient of the gradient was asked for
             parts = ctx.later.take() if ctx.later is not None else ()
             if parts:
-                carried = grid_query.add_put_off(parts, carried, ctx.grid_dim, ctx.interpolation)
+                carried = grid_query.add_put_off(parts, carried, ctx.grid_dim, ctx.interpolation,
+                                                 ctx.cell_size)
             if last and not ctx.spent and ctx.outliving is None:
                 _FusedGridForward._outlive(ctx)
             return (carried,) + (None,) * 9
@@ -120,12 +124,11 @@ class _FusedGridForward(torch.autograd.Function):
                 raise RuntimeError("one of the variables needed for gradient computation has been "
                                    "modified by an inplace operation since an earlier pass")
         grad_embeddings, grad_x = first_order_backward(ctx, z, operands, 0, 1, again, carried,
-                                                        ctx.later)
+                                                        ctx.later, ctx.cell_size)
         if last:
             ctx.spent, ctx.outliving = True, None
-        if grad_x is not None and ctx.cell_size != 1.0:
-            # d cell / d x of x -> (x - origin) / cell_size, as autograd has it
-            grad_x = grad_x / ctx.cell_size
+        if grad_x is not None and ctx.divide_by != 1.0:
+            grad_x = grad_x / ctx.divide_by
         return (grad_embeddings, grad_x) + (None,) * 8
 
     @staticmethod

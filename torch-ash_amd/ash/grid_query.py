@@ -283,7 +283,7 @@ class _Later:
         return parts
 
 
-def add_put_off(parts, carried, grid_dim, interpolation):
+def add_put_off(parts, carried, grid_dim, interpolation, cell_size: float = 1.0):
     """The gradient `carried` with `parts` of a `_Later`, by themselves."""
     if any(target is None for _, _, target in parts):
         if carried is None:
@@ -292,8 +292,14 @@ def add_put_off(parts, carried, grid_dim, interpolation):
             carried = carried.clone(memory_format=torch.contiguous_format)
     for (u, z), operands, target in parts:
         backend.query_backward_backward_onto(carried if target is None else target, u, z, *operands,
-                                             grid_dim, interpolation)
+                                             grid_dim, interpolation, **_per_cell(cell_size))
     return carried
+
+
+def _per_cell(cell_size):
+    """The argument for positions in units of a cell, which the native library alone
+    knows and which is left out where it says nothing."""
+    return {} if cell_size == 1.0 else {"cell_size": cell_size}
 
 
 class SparseDenseGridQuery(torch.autograd.Function):
@@ -342,10 +348,10 @@ class SparseDenseGridQuery(torch.autograd.Function):
 
 
 def first_order_backward(ctx, z, operands, embeddings_input: int = 0, offsets_input: int = 1,
-                         again=None, carried=None, later=None):
+                         again=None, carried=None, later=None, cell_size: float = 1.0):
     """(grad_embeddings, grad_offsets) of a forward node whose inputs number
-    `embeddings_input` / `offsets_input` are the embeddings and (what the
-    offsets depend on with unit Jacobian:) the offsets or positions; `operands`
+    `embeddings_input` / `offsets_input` are the embeddings and the offsets, or
+    positions of which the offsets are 1 / `cell_size`; `operands`
     = (embeddings, offsets, grid_indices, cell_indices, masks, three tables).
     `again`: the node's own copy of the embeddings, which a recorded backward is
     to depend on instead; `carried`: the gradient that has arrived for it;
@@ -358,7 +364,9 @@ def first_order_backward(ctx, z, operands, embeddings_input: int = 0, offsets_in
         return None, None
     if not need_embeddings:
         carried, parts = None, ()
-    along = {"along": [pair for pair, _, _ in parts]} if parts else {}
+    along = _per_cell(cell_size)
+    if parts:
+        along["along"] = [pair for pair, _, _ in parts]
     # The reference always produces both gradients (ash/grid_query.py:104-116);
     # the dense embedding gradient (zero fill + atomics over the whole
     # parameter) is skipped when nobody asked for it, e.g. in
@@ -410,6 +418,7 @@ def first_order_backward(ctx, z, operands, embeddings_input: int = 0, offsets_in
         need_offsets,
         owner,
         later,
+        cell_size,
     )
     if carried is not None:
         grad_embeddings = grad_embeddings + carried
@@ -443,11 +452,13 @@ class SparseDenseGridQueryBackward(torch.autograd.Function):
         need_grad_offsets: bool = True,
         owner=None,
         later=None,
+        cell_size: float = 1.0,
     ):
         """With both `need_*` flags at their default this is the reference's
         signature and result; an output that is not needed is returned as None
         and its work is skipped.  `owner`: weak reference to the embeddings that
-        the operand is the forward node's copy of; `later`: that node's."""
+        the operand is the forward node's copy of; `later`, `cell_size`: that
+        node's."""
         operands = (
             z,
             embeddings,
@@ -464,14 +475,16 @@ class SparseDenseGridQueryBackward(torch.autograd.Function):
         ctx.interpolation = interpolation
         ctx.owner = owner
         ctx.later = later
+        ctx.per_cell = _per_cell(cell_size)
         if need_grad_embeddings and need_grad_offsets:
-            return backend.query_backward_forward(*operands, grid_dim, interpolation)
+            return backend.query_backward_forward(*operands, grid_dim, interpolation, **ctx.per_cell)
         return backend.query_backward_forward(
             *operands,
             grid_dim,
             interpolation,
             need_embeddings=need_grad_embeddings,
             need_offsets=need_grad_offsets,
+            **ctx.per_cell,
         )
 
     @staticmethod
@@ -489,13 +502,13 @@ class SparseDenseGridQueryBackward(torch.autograd.Function):
         edges = _edges(ctx)
         need_z = _grad_requested(ctx, 0, edges=edges)
         need_embeddings = _grad_requested(ctx, 1, through=owned, edges=edges)
-        n_rest = _N_TABLE_ARGS + 5  # offsets, tables, grid_dim, interpolation, 2 flags, owner, later
+        n_rest = _N_TABLE_ARGS + 6  # offsets, tables, grid_dim, interpolation, 2 flags, owner, later, cell_size
         if grad_grad_offsets is None or not (need_z or need_embeddings):
             return (None, None) + (None,) * n_rest
         saved = ctx.saved_tensors
         embeddings = ctx.owner() if owned else saved[1]
         target = _dense_target(embeddings) if need_embeddings and embeddings is not None else None
-        unused = getattr(backend, "WITHOUT_OFFSETS", {})
+        unused = {**getattr(backend, "WITHOUT_OFFSETS", {}), **ctx.per_cell}
         put_off = None
         if (need_embeddings and not need_z and ctx.later is not None
                 and grad_grad_offsets.shape[0] >= PUT_OFF_FROM):

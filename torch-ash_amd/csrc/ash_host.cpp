@@ -62,10 +62,8 @@ namespace py = pybind11;
     X(ash_grid_forward)                                                               \
     X(ash_query_forward)                                                              \
     X(ash_query_backward_forward)                                                     \
-    X(ash_query_backward_forward_accumulate)                                          \
-    X(ash_query_backward_both)                                                        \
-    X(ash_query_backward_backward)                                                    \
-    X(ash_query_backward_backward_accumulate)
+    X(ash_query_backward_forward_scaled)                                              \
+    X(ash_query_backward_backward_scaled)
 
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
@@ -805,6 +803,11 @@ struct Operands {
         return t.contiguous();
     }
 
+    // What a gradient with respect to offsets is multiplied by to be that with respect
+    // to positions in units of a cell: torch, too, divides by a number by multiplying
+    // with its reciprocal, rounded from float64 to the tensor's type.
+    static double per_position(double cell_size) { return 1.0 / cell_size; }
+
     Tensor output(int64_t width) const { return empty({n, width}, emb.scalar_type(), device); }
 
     // where the embedding gradient goes: a new tensor, or `into` added to
@@ -829,14 +832,14 @@ Tensor query_forward(const std::vector<Tensor>& operands, const std::string& int
 std::tuple<Optional, Optional> query_backward_forward(const Tensor& z_in, const std::vector<Tensor>& operands,
                                                       const std::string& interpolation,
                                                       bool need_embeddings, bool need_offsets,
-                                                      const Optional& accumulate_into) {
+                                                      const Optional& accumulate_into, double cell_size) {
     Operands q(operands, interpolation);
     const Tensor z = q.like(z_in, q.e, "z");
     const Tensor grad = q.gradient(accumulate_into, need_embeddings);
     const Tensor offsets = need_offsets ? q.output(3) : Tensor();
-    auto entry = accumulate_into.has_value() ? lib.ash_query_backward_forward_accumulate
-                                             : lib.ash_query_backward_forward;
-    check(entry(&q.args, z.data_ptr(), ptr<void>(grad), ptr<void>(offsets), stream_of(q.device)));
+    check(lib.ash_query_backward_forward_scaled(&q.args, z.data_ptr(), nullptr, nullptr, ptr<void>(grad),
+                                                ptr<void>(offsets), q.per_position(cell_size),
+                                                accumulate_into.has_value(), stream_of(q.device)));
     return {maybe(grad), maybe(offsets)};
 }
 
@@ -844,15 +847,15 @@ std::tuple<Tensor, Optional> query_backward_both(const Tensor& z_in, const Tenso
                                                  const Tensor& z_second_in,
                                                  const std::vector<Tensor>& operands,
                                                  const std::string& interpolation, bool need_offsets,
-                                                 const Optional& accumulate_into) {
+                                                 const Optional& accumulate_into, double cell_size) {
     Operands q(operands, interpolation);
     const Tensor z = q.like(z_in, q.e, "z"), gg = q.like(gg_in, 3, "grad_grad_offsets");
     const Tensor z_second = q.like(z_second_in, q.e, "z of the second order");
     const Tensor grad = q.gradient(accumulate_into, true);
     const Tensor offsets = need_offsets ? q.output(3) : Tensor();
-    check(lib.ash_query_backward_both(&q.args, z.data_ptr(), gg.data_ptr(), z_second.data_ptr(),
-                                      grad.data_ptr(), ptr<void>(offsets), accumulate_into.has_value(),
-                                      stream_of(q.device)));
+    check(lib.ash_query_backward_forward_scaled(
+            &q.args, z.data_ptr(), gg.data_ptr(), z_second.data_ptr(), grad.data_ptr(), ptr<void>(offsets),
+            q.per_position(cell_size), accumulate_into.has_value(), stream_of(q.device)));
     return {grad, maybe(offsets)};
 }
 
@@ -860,15 +863,14 @@ std::tuple<Optional, Optional> query_backward_backward(const Tensor& gg_in, cons
                                                        const std::vector<Tensor>& operands,
                                                        const std::string& interpolation, bool need_z,
                                                        bool need_embeddings,
-                                                       const Optional& accumulate_into) {
+                                                       const Optional& accumulate_into, double cell_size) {
     Operands q(operands, interpolation);
     const Tensor z = q.like(z_in, q.e, "z"), gg = q.like(gg_in, 3, "grad_grad_offsets");
     const Tensor grad_z = need_z ? q.output(q.e) : Tensor();
     const Tensor grad = q.gradient(accumulate_into, need_embeddings);
-    auto entry = accumulate_into.has_value() ? lib.ash_query_backward_backward_accumulate
-                                             : lib.ash_query_backward_backward;
-    check(entry(&q.args, gg.data_ptr(), z.data_ptr(), ptr<void>(grad_z), ptr<void>(grad),
-                stream_of(q.device)));
+    check(lib.ash_query_backward_backward_scaled(&q.args, gg.data_ptr(), z.data_ptr(), ptr<void>(grad_z),
+                                                 ptr<void>(grad), q.per_position(cell_size),
+                                                 accumulate_into.has_value(), stream_of(q.device)));
     return {maybe(grad_z), maybe(grad)};
 }
 
@@ -934,9 +936,15 @@ PYBIND11_MODULE(_ash_host, m) {
     m.def("ray_sample", &ray_sample);
     m.def("surface_mesh", &surface_mesh);
     m.def("query_forward", &query_forward);
-    m.def("query_backward_forward", &query_backward_forward);
-    m.def("query_backward_both", &query_backward_both);
+    using py::arg;
+    m.def("query_backward_forward", &query_backward_forward, arg("z"), arg("operands"), arg("interpolation"),
+          arg("need_embeddings"), arg("need_offsets"), arg("accumulate_into"), arg("cell_size") = 1.0);
+    m.def("query_backward_both", &query_backward_both, arg("z"), arg("grad_grad_offsets"), arg("z_second"),
+          arg("operands"), arg("interpolation"), arg("need_offsets"), arg("accumulate_into"),
+          arg("cell_size") = 1.0);
     m.def("query_gradient_later", &query_gradient_later);
     m.def("hands_over_unseen", &hands_over_unseen);
-    m.def("query_backward_backward", &query_backward_backward);
+    m.def("query_backward_backward", &query_backward_backward, arg("grad_grad_offsets"), arg("z"),
+          arg("operands"), arg("interpolation"), arg("need_z"), arg("need_embeddings"),
+          arg("accumulate_into"), arg("cell_size") = 1.0);
 }

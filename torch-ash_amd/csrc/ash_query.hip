@@ -80,6 +80,11 @@ struct QDev {
     int64_t B;
     int64_t M;
     int E;
+    // Gradients with respect to the offsets are multiplied by it, both where they are
+    // written and where the gradient of one is read: the grid's positions are offsets
+    // in units of a cell, and a pass over the gradient behind or in front of the kernel
+    // takes 17 - 23 us of 4 M queries (three of them in a training pass).
+    double offset_scale = 1.0;
     int smooth;    // 0 linear, 1 smooth step
     int merge;     // pre-reduce runs of equal rows before the atomics
 };
@@ -677,9 +682,9 @@ query_backward_forward_kernel(
             if constexpr (second) {
                 if (on) zk2 = z2[q * a.E + ch];
                 if (valid) {
-                    gg[0] = gg_off[q * 3 + 0];
-                    gg[1] = gg_off[q * 3 + 1];
-                    gg[2] = gg_off[q * 3 + 2];
+                    gg[0] = gg_off[q * 3 + 0] * static_cast<T>(a.offset_scale);
+                    gg[1] = gg_off[q * 3 + 1] * static_cast<T>(a.offset_scale);
+                    gg[2] = gg_off[q * 3 + 2] * static_cast<T>(a.offset_scale);
                 }
             }
             GroupRuns<LPQ> runs;
@@ -717,9 +722,10 @@ query_backward_forward_kernel(
                 }
             }
             if (want_off && q < a.N && ch == 0) {
-                grad_off[q * 3 + 0] = valid ? go[0] : T(0);
-                grad_off[q * 3 + 1] = valid ? go[1] : T(0);
-                grad_off[q * 3 + 2] = valid ? go[2] : T(0);
+                const T scale = static_cast<T>(a.offset_scale);
+                grad_off[q * 3 + 0] = valid ? go[0] * scale : T(0);
+                grad_off[q * 3 + 1] = valid ? go[1] * scale : T(0);
+                grad_off[q * 3 + 2] = valid ? go[2] * scale : T(0);
             }
         }
     }
@@ -762,9 +768,9 @@ query_backward_backward_kernel(
             if (want_emb && a.merge) runs = find_group_runs<LPQ>(row[0], on, lane);
             T gg[3] = {T(0), T(0), T(0)};
             if (valid) {
-                gg[0] = gg_off[q * 3 + 0];
-                gg[1] = gg_off[q * 3 + 1];
-                gg[2] = gg_off[q * 3 + 2];
+                gg[0] = gg_off[q * 3 + 0] * static_cast<T>(a.offset_scale);
+                gg[1] = gg_off[q * 3 + 1] * static_cast<T>(a.offset_scale);
+                gg[2] = gg_off[q * 3 + 2] * static_cast<T>(a.offset_scale);
             }
             T e[8];
 #pragma unroll
@@ -1153,9 +1159,9 @@ query_backward_forward_vec_kernel(
             if constexpr (second) {
                 const v4f zs = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(z2 + q * 4));
                 y4 = make_float4(zs.x, zs.y, zs.z, zs.w);
-                gg[0] = __builtin_nontemporal_load(gg_off + q * 3 + 0);
-                gg[1] = __builtin_nontemporal_load(gg_off + q * 3 + 1);
-                gg[2] = __builtin_nontemporal_load(gg_off + q * 3 + 2);
+                gg[0] = __builtin_nontemporal_load(gg_off + q * 3 + 0) * static_cast<float>(a.offset_scale);
+                gg[1] = __builtin_nontemporal_load(gg_off + q * 3 + 1) * static_cast<float>(a.offset_scale);
+                gg[2] = __builtin_nontemporal_load(gg_off + q * 3 + 2) * static_cast<float>(a.offset_scale);
             }
         }
         AxisTerms<float> t;
@@ -1186,9 +1192,10 @@ query_backward_forward_vec_kernel(
                 go[2] += dot * gw[2];
             }
             if (q < a.N) {
-                __builtin_nontemporal_store(on ? go[0] : 0.f, grad_off + q * 3 + 0);
-                __builtin_nontemporal_store(on ? go[1] : 0.f, grad_off + q * 3 + 1);
-                __builtin_nontemporal_store(on ? go[2] : 0.f, grad_off + q * 3 + 2);
+                const float scale = static_cast<float>(a.offset_scale);
+                __builtin_nontemporal_store(on ? go[0] * scale : 0.f, grad_off + q * 3 + 0);
+                __builtin_nontemporal_store(on ? go[1] * scale : 0.f, grad_off + q * 3 + 1);
+                __builtin_nontemporal_store(on ? go[2] * scale : 0.f, grad_off + q * 3 + 2);
             }
         }
         if constexpr (want_emb) {
@@ -1243,9 +1250,9 @@ query_backward_backward_vec_kernel(
             typedef float v4f __attribute__((ext_vector_type(4)));
             const v4f zl = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(z + q * 4));
             z4 = make_float4(zl.x, zl.y, zl.z, zl.w);
-            gg[0] = __builtin_nontemporal_load(gg_off + q * 3 + 0);
-            gg[1] = __builtin_nontemporal_load(gg_off + q * 3 + 1);
-            gg[2] = __builtin_nontemporal_load(gg_off + q * 3 + 2);
+            gg[0] = __builtin_nontemporal_load(gg_off + q * 3 + 0) * static_cast<float>(a.offset_scale);
+            gg[1] = __builtin_nontemporal_load(gg_off + q * 3 + 1) * static_cast<float>(a.offset_scale);
+            gg[2] = __builtin_nontemporal_load(gg_off + q * 3 + 2) * static_cast<float>(a.offset_scale);
         }
         AxisTerms<float> t;
         axis_terms<float, true>(o, a.smooth, t);
@@ -2653,9 +2660,11 @@ int ash_grid_forward(ash_map_t* map, const float* x, const float* origin, float 
 namespace {
 
 int backward_forward(const ash_query_args* a, const void* z, void* grad_embeddings,
-                     void* grad_offsets, void* stream, bool clear, const Second& also = {}) {
+                     void* grad_offsets, void* stream, bool clear, const Second& also = {},
+                     double offset_scale = 1.0) {
     QDev d;
     if (check_args(a, d)) return 1;
+    d.offset_scale = offset_scale;
     if (grad_embeddings == nullptr && grad_offsets == nullptr) {
         ASH_FAIL("at least one of grad_embeddings / grad_offsets is required");
     }
@@ -2677,9 +2686,10 @@ int backward_forward(const ash_query_args* a, const void* z, void* grad_embeddin
 
 int backward_backward(const ash_query_args* a, const void* grad_grad_offsets,
                       const void* z, void* grad_z, void* grad_embeddings,
-                      void* stream, bool clear) {
+                      void* stream, bool clear, double offset_scale = 1.0) {
     QDev d;
     if (check_args(a, d)) return 1;
+    d.offset_scale = offset_scale;
     if (grad_embeddings == nullptr && grad_z == nullptr) {
         ASH_FAIL("at least one of grad_z / grad_embeddings is required");
     }
@@ -2738,6 +2748,26 @@ int ash_query_backward_backward_accumulate(const ash_query_args* a,
                                            void* stream) {
     if (grad_embeddings == nullptr) ASH_FAIL("accumulate: null grad_embeddings");
     return backward_backward(a, grad_grad_offsets, z, grad_z, grad_embeddings, stream, false);
+}
+
+int ash_query_backward_forward_scaled(const ash_query_args* a, const void* z, const void* grad_grad_offsets,
+                                      const void* z_second, void* grad_embeddings, void* grad_offsets,
+                                      double offset_scale, int32_t accumulate, void* stream) {
+    if (accumulate && grad_embeddings == nullptr) ASH_FAIL("accumulate: null grad_embeddings");
+    if ((grad_grad_offsets == nullptr) != (z_second == nullptr)) ASH_FAIL("null pointer");
+    if (grad_grad_offsets != nullptr && grad_embeddings == nullptr) {
+        ASH_FAIL("backward_both: null grad_embeddings");
+    }
+    return backward_forward(a, z, grad_embeddings, grad_offsets, stream, accumulate == 0,
+                            {grad_grad_offsets, z_second}, offset_scale);
+}
+
+int ash_query_backward_backward_scaled(const ash_query_args* a, const void* grad_grad_offsets,
+                                       const void* z, void* grad_z, void* grad_embeddings,
+                                       double offset_scale, int32_t accumulate, void* stream) {
+    if (accumulate && grad_embeddings == nullptr) ASH_FAIL("accumulate: null grad_embeddings");
+    return backward_backward(a, grad_grad_offsets, z, grad_z, grad_embeddings, stream, accumulate == 0,
+                             offset_scale);
 }
 
 namespace {

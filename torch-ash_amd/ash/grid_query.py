@@ -124,28 +124,24 @@ def _record_path(path: str) -> None:
     LAST_GRADIENT_PATH = path
 
 
-def _edges(ctx):
-    """ctx.next_functions, for `_grad_requested` (None where they cannot be had)."""
-    try:
-        return ctx.next_functions
-    except Exception:
-        return None
-
-
-def _grad_requested(ctx, index: int, through: bool = False, edges=None) -> bool:
+def _grad_requested(ctx, index: int, through: bool = False) -> bool:
     """Whether the running backward pass will consume the gradient of input
     `index`.  `ctx.needs_input_grad` only says that the input requires grad;
     in `autograd.grad(y, x)` the engine additionally knows which graph nodes it
     is going to execute, and the node behind an input it will not execute (the
     dense embeddings parameter, typically) needs no gradient from us.
     `through`: the input is the forward node's copy of the embeddings, and the
-    node asked about is the one behind that node's own embeddings.  `edges`:
-    ctx.next_functions, for callers that ask several times (each time they are
-    asked for, every one of them becomes a Python object)."""
+    node asked about is the one behind that node's own embeddings.  (In C++ where
+    the native module is there: asked in Python each node of the graph becomes an
+    object, and a leaf that the pass was asked for an exception, 20 us of a training
+    step of 420.)"""
+    host = getattr(backend, "host", None)
+    if host is not None and hasattr(torch._C, "_will_engine_execute_node"):
+        return host.grad_requested(ctx, index, through)
     if not ctx.needs_input_grad[index]:
         return False
     try:
-        node = (ctx.next_functions if edges is None else edges)[index][0]
+        node = ctx.next_functions[index][0]
         if through:
             node = node.next_functions[0][0]
         return node is not None and torch._C._will_engine_execute_node(node)
@@ -245,14 +241,14 @@ class _Later:
     def __init__(self):
         self.passes = {}   # id of a pass -> weak reference to its _Pass
 
-    def room(self, ctx, edges):
+    def room(self, ctx):
         """The list of the running pass if `ctx`, a second-order node whose second
         input is the forward node's copy of the embeddings, may put off its
-        contributions.  `edges`: ctx.next_functions."""
+        contributions."""
         try:
             task = torch._C._current_graph_task_id()
             if (task < 0 or torch.is_grad_enabled()
-                    or not torch._C._will_engine_execute_node(edges[1][0])
+                    or not torch._C._will_engine_execute_node(ctx.next_functions[1][0])
                     or not backend.host.hands_over_unseen(ctx, 1)):
                 return None
             here = self._of(task)
@@ -356,9 +352,8 @@ def first_order_backward(ctx, z, operands, embeddings_input: int = 0, offsets_in
     `again`: the node's own copy of the embeddings, which a recorded backward is
     to depend on instead; `carried`: the gradient that has arrived for it;
     `later`: what belongs to that and has been put off."""
-    edges = _edges(ctx)
-    need_embeddings = _grad_requested(ctx, embeddings_input, edges=edges)
-    need_offsets = _grad_requested(ctx, offsets_input, edges=edges)
+    need_embeddings = _grad_requested(ctx, embeddings_input)
+    need_offsets = _grad_requested(ctx, offsets_input)
     parts = later.take() if later is not None else ()
     if not (need_embeddings or need_offsets):
         return None, None
@@ -499,9 +494,8 @@ class SparseDenseGridQueryBackward(torch.autograd.Function):
         and no gradient flows to `offsets` at second order.
         """
         owned = ctx.owner is not None
-        edges = _edges(ctx)
-        need_z = _grad_requested(ctx, 0, edges=edges)
-        need_embeddings = _grad_requested(ctx, 1, through=owned, edges=edges)
+        need_z = _grad_requested(ctx, 0)
+        need_embeddings = _grad_requested(ctx, 1, owned)
         n_rest = _N_TABLE_ARGS + 6  # offsets, tables, grid_dim, interpolation, 2 flags, owner, later, cell_size
         if grad_grad_offsets is None or not (need_z or need_embeddings):
             return (None, None) + (None,) * n_rest
@@ -512,7 +506,7 @@ class SparseDenseGridQueryBackward(torch.autograd.Function):
         put_off = None
         if (need_embeddings and not need_z and ctx.later is not None
                 and grad_grad_offsets.shape[0] >= PUT_OFF_FROM):
-            put_off = ctx.later.room(ctx, edges)
+            put_off = ctx.later.room(ctx)
         if put_off is not None:
             put_off.append(((grad_grad_offsets, saved[0]), saved[1:], target))
             unused = {**unused, "later": True}

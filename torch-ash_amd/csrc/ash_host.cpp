@@ -10,6 +10,7 @@
 #include <torch/extension.h>
 
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/graph_task.h>
 #include <torch/csrc/autograd/python_function.h>
 
 #include <dlfcn.h>
@@ -901,6 +902,35 @@ bool hands_over_unseen(const py::object& ctx, size_t input) {
            next->retains_grad_hooks().empty();
 }
 
+// Whether the running backward pass consumes the gradient that the node of `ctx`
+// makes for its input `input` (`through`: the input belongs to a forward node's copy of
+// a tensor, and the node asked about is the one behind that node's first input).  As
+// torch._C._will_engine_execute_node says it of a Python object of the node, without
+// the object, and without the exception it raises for a leaf whose gradient is what
+// the pass was asked for (13 us of a training step); outside a pass: yes.
+bool grad_requested(const py::object& ctx, size_t input, bool through) {
+    if (!THPFunction_Check(ctx.ptr())) return true;
+    const auto function = reinterpret_cast<THPFunction*>(ctx.ptr());
+    const auto node = function->cdata.lock();
+    if (!node || input >= node->num_outputs()) return true;
+    const PyObject* wanted = PyTuple_GetItem(function->needs_input_grad, static_cast<Py_ssize_t>(input));
+    if (wanted == nullptr) throw py::error_already_set();
+    if (wanted != Py_True) return false;
+    auto behind = node->next_edge(input).function;
+    if (behind && through) {
+        if (behind->num_outputs() == 0) return true;
+        behind = behind->next_edge(0).function;
+    }
+    if (!behind) return false;
+    const auto* executed = torch::autograd::get_current_graph_task_exec_info();
+    const auto* all = torch::autograd::get_current_graph_task_nodes_in_graph();
+    if (executed == nullptr || all == nullptr) return true;
+    if (all->find(behind.get()) == all->end()) return false;
+    if (executed->empty()) return true;
+    const auto it = executed->find(behind.get());
+    return it != executed->end() && it->second.should_execute();
+}
+
 std::tuple<Optional, Tensor, std::vector<Tensor>> find_rows_py(uintptr_t handle, int64_t dim, int64_t device,
                                                                const Tensor& keys,
                                                                const std::vector<Tensor>& tables,
@@ -944,6 +974,7 @@ PYBIND11_MODULE(_ash_host, m) {
           arg("cell_size") = 1.0);
     m.def("query_gradient_later", &query_gradient_later);
     m.def("hands_over_unseen", &hands_over_unseen);
+    m.def("grad_requested", &grad_requested);
     m.def("query_backward_backward", &query_backward_backward, arg("grad_grad_offsets"), arg("z"),
           arg("operands"), arg("interpolation"), arg("need_z"), arg("need_embeddings"),
           arg("accumulate_into"), arg("cell_size") = 1.0);

@@ -1341,14 +1341,13 @@ __global__ __launch_bounds__(kBlock) void reset_heap_kernel(
 
 // A clear in one launch: counters, and stretches of memory that are filled with one
 // word (value rows with zeros, the bucket array, the second region's states and the
-// key log with ones) or counted up (the heap).  A workgroup takes kClearUnits pieces
-// of 16 bytes of one stretch, so that workgroups handed out one after the other walk
-// through memory in order.  Bound by the stores of large stretches (tables of 288 and
+// key log with ones) or counted up (the heap).  A piece of 16 bytes per thread, so
+// that workgroups handed out one after the other walk through memory in order (four
+// pieces: 200 MB 26.5 -> 26.0 us, but 512 MB 76 -> 86, 1.64 GB 240 -> 270).  Bound by the stores of large stretches (tables of 288 and
 // 96 MB, with the counters: two fills of torch's and a launch for the counters 36.6 +
-// 13.9 + 4.7 -> 47 us, 8.2 TB/s), and by the launch itself for small ones, which is
+// 13.9 + 4.7 -> 48 us, 8.0 TB/s), and by the launch itself for small ones, which is
 // why it is one (a launch in a busy stream costs 4 us however little it does; a set of
 // 5640 keys emptied, filled and asked 41.5 -> 34.2 us).
-constexpr int kClearUnits = 4 * kBlock;
 constexpr int kClearSpans = kMaxFusedValues + 4;
 
 struct ClearSpan {
@@ -1385,20 +1384,16 @@ __global__ __launch_bounds__(kBlock) void clear_kernel(ClearArgs a, int32_t* __r
     int k = 0;
     while (k + 1 < a.n && blockIdx.x >= a.span[k + 1].first) ++k;
     const ClearSpan& span = a.span[k];
-    const int64_t base = static_cast<int64_t>(blockIdx.x - span.first) * kClearUnits + threadIdx.x;
-#pragma unroll
-    for (int u = 0; u < kClearUnits / kBlock; ++u) {
-        const int64_t i = base + u * kBlock;
-        if (i < span.n16) {
-            const uint32_t w = static_cast<uint32_t>(4 * i);
-            span.p[i] = span.count ? make_uint4(w, w + 1, w + 2, w + 3)
-                                   : make_uint4(span.word, span.word, span.word, span.word);
-        } else if (i == span.n16) {
-            uint8_t* rest = reinterpret_cast<uint8_t*>(span.p + i);
-            for (int b = 0; b < span.tail; ++b) {
-                rest[b] = static_cast<uint8_t>((span.count ? static_cast<uint32_t>(4 * i) + b / 4 : span.word) >>
-                                               (8 * (b % 4)));
-            }
+    const int64_t i = static_cast<int64_t>(blockIdx.x - span.first) * kBlock + threadIdx.x;
+    if (i < span.n16) {
+        const uint32_t w = static_cast<uint32_t>(4 * i);
+        span.p[i] = span.count ? make_uint4(w, w + 1, w + 2, w + 3)
+                               : make_uint4(span.word, span.word, span.word, span.word);
+    } else if (i == span.n16) {
+        uint8_t* rest = reinterpret_cast<uint8_t*>(span.p + i);
+        for (int b = 0; b < span.tail; ++b) {
+            rest[b] = static_cast<uint8_t>((span.count ? static_cast<uint32_t>(4 * i) + b / 4 : span.word) >>
+                                           (8 * (b % 4)));
         }
     }
 }
@@ -2205,7 +2200,7 @@ class ClearList {
         const int64_t pieces = bytes / 16;
         args_.span[args_.n++] = {static_cast<uint4*>(p), pieces, word, static_cast<uint8_t>(bytes % 16),
                                  count, static_cast<uint32_t>(groups_)};
-        groups_ += (pieces + (bytes % 16 != 0 ? 1 : 0) + kClearUnits - 1) / kClearUnits;
+        groups_ += (pieces + (bytes % 16 != 0 ? 1 : 0) + kBlock - 1) / kBlock;
     }
     void add(const ClearRows& rows) {
         for (int v = 0; v < rows.n; ++v) add(rows.rows[v], rows.bytes[v], 0u);

@@ -515,13 +515,21 @@ __device__ __forceinline__ void insert_key(
             change_counter(m.ctr + kCtrGenLive, 1);
         }
         if constexpr (MODE == kInsertFused) {
+            // (four words at a time: word after word, each was waited for by its store)
+#pragma unroll 1
+            for (int v = 0; v < va.n; ++v) {
+                const int rd = va.row_dwords[v];
+                const uint32_t* s = va.src[v] + i * rd;
+                uint32_t* d = va.dst[v] + static_cast<int64_t>(idx) * rd;
+#pragma unroll 1
+                for (int q = 0; q < rd; q += 4) {
+                    uint32_t word[4];
 #pragma unroll
-            for (int v = 0; v < kMaxFusedValues; ++v) {
-                if (v < va.n) {
-                    const int rd = va.row_dwords[v];
-                    const uint32_t* s = va.src[v] + i * rd;
-                    uint32_t* d = va.dst[v] + static_cast<int64_t>(idx) * rd;
-                    for (int q = 0; q < rd; ++q) d[q] = s[q];
+                    for (int k = 0; k < 4; ++k) word[k] = q + k < rd ? s[q + k] : 0u;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        if (q + k < rd) d[q + k] = word[k];
+                    }
                 }
             }
         }

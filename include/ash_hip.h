@@ -241,10 +241,11 @@ int ash_grid_integrate_depth_flagged(ash_map_t* map, float* embeddings,
  * ash_grid_activate_positions and ash_grid_integrate_depth_flagged, two
  * launches.  Cell to world is cell * cell_to_world [+ world_origin], with
  * world_origin float32[3] on the device or NULL.  group_counts (int32
- * [ASH_FLAGGED_GROUPS] on the device, or NULL): a third, small launch adds up
- * the touched blocks and leaves the counters for the host behind the two others;
- * the next ash_map_counters waits for it and finds them in out[5].  Refused
- * with group_counts on a stream that is being captured. */
+ * [ASH_FLAGGED_GROUPS] of scratch on the device, or NULL): a small launch between
+ * the two (two above 2^18 rows) counts the touched blocks and leaves the counters for
+ * the host; the next ash_map_counters waits for them, not for the integration, and
+ * finds the count in out[5].  Refused with group_counts on a stream that is being
+ * captured. */
 enum { ASH_FLAGGED_GROUPS = 8192 };
 int ash_grid_fuse_frame(ash_map_t* map, const float* positions, int64_t n,
                         const float* origin, float cell_size, int dilation,

@@ -447,6 +447,29 @@ def test_integration_by_flags_equals_integration_by_listing(gpu_ash, grid_dim, e
     assert int(flagged.embeddings.detach()[free].count_nonzero()) == 0
 
 
+@pytest.mark.parametrize("capacity", [1, 17, 4_097, 262_144, 262_145, 700_001])
+def test_touched_blocks_are_counted_before_the_integration(gpu_ash, capacity):
+    """The number that fuse_frame returns, for tables whose flags one workgroup
+    counts and for those that several do (from 2^18 rows on), with ends inside 16
+    bytes, and flags from the first row to the last: blocks of one cell, all rows
+    in use, points in some blocks only, frame after frame."""
+    grid = gpu_ash.UnBoundedSparseDenseGrid(3, capacity, 2, 1, cell_size=1.0, device=DEV)
+    i = torch.arange(capacity, device=DEV, dtype=torch.int32)
+    keys = torch.stack([i % 64, i // 64 % 64, i // 4096], 1)
+    grid.engine.insert_keys(keys)
+    assert grid.engine.size() == capacity
+    rows = grid.engine.find(keys)[0]
+    depth, k, ext = torch.zeros(4, 4, device=DEV), torch.eye(3, device=DEV), torch.eye(4, device=DEV)
+    g = torch.Generator().manual_seed(capacity)
+    for share in (1.0, 0.3, 0.01):
+        pick = (torch.rand(capacity, generator=g) < share).to(DEV)
+        pick |= (rows == 0) | (rows == capacity - 1)
+        points = (keys[pick].float() + 0.25).contiguous()
+        assert gpu_ash.fusion.fuse_frame(grid, points, depth, k, ext, 0.04, 6.0,
+                                         dilation=0) == int(pick.sum())
+        assert int(grid.engine.backend._touched.sum()) == 0
+
+
 @pytest.mark.parametrize("capacity", [5, 1000, 80_000, 131_073, 200_000, 1_048_576])
 def test_touched_rows_are_listed_in_order(gpu_ash, capacity):
     """ash_grid_collect_touched against torch.nonzero: ascending rows, their

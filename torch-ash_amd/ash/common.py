@@ -349,7 +349,7 @@ RAY_STAGE_EXTRA = 2
 # Largest table whose touched rows ash_grid_collect_touched lists (the header's
 # ASH_COLLECT_MAX_BLOCKS).
 COLLECT_MAX_BLOCKS = 1 << 20
-# Workgroups of the integration that goes by flags (the header's ASH_FLAGGED_GROUPS).
+# Words of scratch for the count of a fusion frame (the header's ASH_FLAGGED_GROUPS).
 FLAGGED_GROUPS = 8192
 # Size of a second region that is attached before any key has asked for it
 # (2^16 slots of 20 bytes).
@@ -1384,8 +1384,9 @@ class _HashMap:
     ) -> None:
         """The activation of `activate_blocks` from world positions (cell units
         = (positions - origin) / cell_size) and the depth integration over the
-        rows it touches, two launches; with `count` a third leaves the counters,
-        the number of touched blocks among them, where `counters` finds them.
+        rows it touches, two launches; with `count` one between them leaves the
+        counters, the number of touched blocks among them, where `counters`
+        finds them (it does not wait for the integration).
         Nothing waits for the device and nothing is allocated once the map's
         arrays exist, so the launches can (without `count`) be captured into a
         graph; keys refused for lack of capacity show in the counters at the

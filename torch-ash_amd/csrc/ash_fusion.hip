@@ -211,18 +211,14 @@ __global__ __launch_bounds__(kBlock) void integrate_depth_counted_kernel(
 // are the low ones as a rule, so every workgroup gets its share of them),
 // kBlock flags per round, lists the flagged ones in LDS, takes the flags down
 // and updates the cells of the listed blocks, whose coordinates stand in
-// coords[row].  a.grid_idx is not used; a.n is the number of rows.  `counts`
-// (one word per workgroup, or null): how many flagged rows the workgroup met --
-// a plain store each; additions to one counter would serialise (7 ns each) and
-// outlast the integration.
+// coords[row].  a.grid_idx is not used; a.n is the number of rows.
 template <int G, int E>
 __global__ __launch_bounds__(kBlock) void integrate_depth_flagged_kernel(
-        IntegrateArgs a, uint8_t* __restrict__ touched, int32_t* __restrict__ counts) {
+        IntegrateArgs a, uint8_t* __restrict__ touched) {
     __shared__ int32_t s_rows[kBlock * 4];   // row and block coordinates of the flagged ones
     __shared__ int s_n;
     const int m = G > 0 ? G * G * G : a.m;
     const int64_t stride = gridDim.x;
-    int met = 0;
     for (int64_t first = blockIdx.x; first < a.n; first += stride * kBlock) {
         if (threadIdx.x == 0) s_n = 0;
         __syncthreads();
@@ -244,7 +240,6 @@ __global__ __launch_bounds__(kBlock) void integrate_depth_flagged_kernel(
         }
         __syncthreads();
         const int listed = s_n;
-        met += listed;
         for (int j = 0; j < listed; ++j) {
             const int32_t r = s_rows[j * 4 + 0];
             const int bx = s_rows[j * 4 + 1];
@@ -285,7 +280,6 @@ __global__ __launch_bounds__(kBlock) void integrate_depth_flagged_kernel(
         }
         __syncthreads();   // s_rows and s_n are rewritten by the next round
     }
-    if (counts != nullptr && threadIdx.x == 0) counts[blockIdx.x] = met;
 }
 
 }  // namespace
@@ -343,16 +337,15 @@ unsigned flagged_groups(const ash_map* map) {
     return groups < 1 ? 1u : static_cast<unsigned>(groups);
 }
 
-int launch_flagged(const ash_map* map, IntegrateArgs a, uint8_t* touched, int32_t* counts,
-                   hipStream_t s) {
+int launch_flagged(const ash_map* map, IntegrateArgs a, uint8_t* touched, hipStream_t s) {
     const unsigned groups = flagged_groups(map);
     a.grid_idx = nullptr;
     if (a.g == 8 && a.e == 2) {
-        integrate_depth_flagged_kernel<8, 2><<<groups, kBlock, 0, s>>>(a, touched, counts);
+        integrate_depth_flagged_kernel<8, 2><<<groups, kBlock, 0, s>>>(a, touched);
     } else if (a.g == 8 && a.e == 5) {
-        integrate_depth_flagged_kernel<8, 5><<<groups, kBlock, 0, s>>>(a, touched, counts);
+        integrate_depth_flagged_kernel<8, 5><<<groups, kBlock, 0, s>>>(a, touched);
     } else {
-        integrate_depth_flagged_kernel<0, 0><<<groups, kBlock, 0, s>>>(a, touched, counts);
+        integrate_depth_flagged_kernel<0, 0><<<groups, kBlock, 0, s>>>(a, touched);
     }
     ASH_LAUNCH_CHECK();
     return 0;
@@ -414,7 +407,7 @@ extern "C" int ash_grid_integrate_depth_flagged(
     }
     DeviceGuard guard;
     ASH_HIP(guard.enter(map->device));
-    return launch_flagged(map, a, touched, nullptr, static_cast<hipStream_t>(stream));
+    return launch_flagged(map, a, touched, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int ash_grid_fuse_frame(
@@ -444,10 +437,17 @@ extern "C" int ash_grid_fuse_frame(
     }
     DeviceGuard guard;
     ASH_HIP(guard.enter(map->device));
-    if (launch_flagged(map, a, touched, group_counts, s)) return 1;
-    return group_counts == nullptr
-                   ? 0
-                   : queue_touched_count(map, group_counts, static_cast<int>(flagged_groups(map)), s);
+    // Counted before the integration takes the flags down, not from it: the number is
+    // with the host while the integration runs, and the caller has its next frame
+    // queued by the time that ends.  (The count behind the integration, from a word of
+    // each of its workgroups, left the device idle for the way to the host and back:
+    // a VGA frame with its count 55 us, 43 like this.)
+    if (group_counts != nullptr &&
+        queue_touched_count(map, touched, std::min(map->capacity, num_embeddings), group_counts,
+                            kFlaggedGroups, s)) {
+        return 1;
+    }
+    return launch_flagged(map, a, touched, s);
 }
 
 extern "C" int ash_grid_integrate_depth(

@@ -1421,36 +1421,6 @@ __global__ void publish_counters_kernel(const int32_t* __restrict__ ctr, uint64_
     leave_counters(ctr, landing, stamp);
 }
 
-// The same with the touched blocks added up first (one workgroup).
-__global__ __launch_bounds__(kBlock) void publish_touched_kernel(int32_t* __restrict__ ctr,
-                                                                 const int32_t* __restrict__ counts,
-                                                                 int n, uint64_t* landing,
-                                                                 int32_t stamp) {
-    __shared__ int s_wave[kBlock / 64];
-    int sum = 0;
-    if (n == kBlock * 4 * (n / (kBlock * 4))) {
-        for (int i = threadIdx.x * 4; i < n; i += kBlock * 4) {
-            const int4 c = *reinterpret_cast<const int4*>(counts + i);
-            sum += c.x + c.y + c.z + c.w;
-        }
-    } else {
-        for (int i = threadIdx.x; i < n; i += kBlock) sum += counts[i];
-    }
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) sum += __shfl_xor(sum, d);
-    if ((threadIdx.x & 63) == 0) s_wave[threadIdx.x >> 6] = sum;
-    __syncthreads();
-    if (threadIdx.x >= 64) return;
-    int total = 0;
-#pragma unroll
-    for (int w = 0; w < kBlock / 64; ++w) total += s_wave[w];
-    if (threadIdx.x < kHostCounters) {
-        const int32_t v = threadIdx.x == kCtrTouched ? total : ctr[threadIdx.x];
-        if (threadIdx.x == kCtrTouched) ctr[kCtrTouched] = total;
-        leave_word(landing + threadIdx.x, v, stamp);
-    }
-}
-
 __global__ void set_counter_kernel(int32_t* ctr, int which, int32_t value) {
     if (threadIdx.x == 0 && blockIdx.x == 0) ctr[which] = value;
 }
@@ -1971,6 +1941,7 @@ constexpr int kCollectThreads = 1024;
 constexpr int kCollectGroups = 128;
 constexpr int kCollectMaxWords = 2;    // per thread: 2^20 flags / 128 groups / 1024 threads / 4
 constexpr int64_t kCollectMaxBlocks = int64_t{1} << 20;   // ASH_COLLECT_MAX_BLOCKS of the header
+constexpr int64_t kCountFlags = int64_t{1} << 18;   // per workgroup of count_flags_kernel: 16 loads a thread
 
 __device__ __forceinline__ int flags_in(uint32_t w) {
     return (w & 0xFFu ? 1 : 0) + (w & 0xFF00u ? 1 : 0) + (w & 0xFF0000u ? 1 : 0) +
@@ -2006,6 +1977,61 @@ __device__ __forceinline__ int block_sums(int v, int* s_wave, int& mine) {
         total += s_wave[q];
     }
     return total;
+}
+
+// The counters for the host, `total` blocks touched among them (one workgroup).
+__device__ __forceinline__ void leave_touched(int32_t* ctr, int total, uint64_t* landing,
+                                              int32_t stamp) {
+    if (threadIdx.x < kHostCounters) {
+        const int32_t v = threadIdx.x == kCtrTouched ? total : ctr[threadIdx.x];
+        if (threadIdx.x == kCtrTouched) ctr[kCtrTouched] = total;
+        leave_word(landing + threadIdx.x, v, stamp);
+    }
+}
+
+// How many of the first `rows` rows are flagged, while the flags stand: `counts[w]`
+// of workgroup w's share, and where one workgroup looks at all of them the counters
+// go to the host at once.  The flags are read 16 at a time, eight loads of a thread
+// on their way together (80 000 flags are five loads each: one wait for memory).
+__global__ __launch_bounds__(kCollectThreads) void count_flags_kernel(
+        const uint8_t* __restrict__ touched, int64_t rows, int32_t* __restrict__ counts,
+        int32_t* __restrict__ ctr, uint64_t* landing, int32_t stamp) {
+    __shared__ int s_wave[kCollectThreads / 64];
+    const int64_t at = static_cast<int64_t>(blockIdx.x) * kCollectThreads + threadIdx.x;
+    const int64_t stride = static_cast<int64_t>(gridDim.x) * kCollectThreads;
+    // what lies before the first whole 16 bytes and behind the last is counted byte by byte
+    int64_t head = (16 - static_cast<int64_t>(reinterpret_cast<uintptr_t>(touched) % 16)) % 16;
+    if (head > rows) head = rows;
+    const int64_t whole = (rows - head) / 16;
+    const uint4* quads = reinterpret_cast<const uint4*>(touched + head);
+    int sum = 0;
+#pragma unroll 8
+    for (int64_t i = at; i < whole; i += stride) {
+        const uint4 v = quads[i];
+        sum += flags_in(v.x) + flags_in(v.y) + flags_in(v.z) + flags_in(v.w);
+    }
+    if (at < head) sum += touched[at] != 0;
+    const int64_t rest = head + whole * 16 + at;
+    if (rest < rows) sum += touched[rest] != 0;
+    int unused;
+    const int total = block_sums(sum, s_wave, unused);
+    if (gridDim.x > 1) {
+        if (threadIdx.x == 0) counts[blockIdx.x] = total;
+        return;
+    }
+    leave_touched(ctr, total, landing, stamp);
+}
+
+// The same for several workgroups: their counts added up (one workgroup).
+__global__ __launch_bounds__(kCollectThreads) void publish_touched_kernel(
+        int32_t* __restrict__ ctr, const int32_t* __restrict__ counts, int n, uint64_t* landing,
+        int32_t stamp) {
+    __shared__ int s_wave[kCollectThreads / 64];
+    int sum = 0;
+    for (int i = threadIdx.x; i < n; i += kCollectThreads) sum += counts[i];
+    int unused;
+    const int total = block_sums(sum, s_wave, unused);
+    leave_touched(ctr, total, landing, stamp);
 }
 
 __global__ __launch_bounds__(kCollectThreads) void collect_touched_kernel(
@@ -3477,13 +3503,24 @@ int upkeep(ash_map* map, int64_t incoming, void* scratch, int64_t scratch_bytes,
 
 }  // extern "C"
 
-int ash::queue_touched_count(ash_map* map, const int32_t* counts, int n, hipStream_t s) {
+int ash::queue_touched_count(ash_map* map, const uint8_t* touched, int64_t rows, int32_t* counts,
+                             int max_counts, hipStream_t s) {
     if (take_line(map)) return 1;
     std::lock_guard<std::mutex> lock(map->counter_lock);
     if (settle_late_words(map)) return 1;
     const int32_t stamp = map->stamp = next_stamp(map->stamp);
-    publish_touched_kernel<<<1, kBlock, 0, s>>>(map->d.ctr, counts, n, map->line + kLineLate, stamp);
+    uint64_t* const landing = map->line + kLineLate;
+    int64_t groups = (rows + kCountFlags - 1) / kCountFlags;
+    if (groups > max_counts) groups = max_counts;
+    if (groups < 1) groups = 1;
+    count_flags_kernel<<<static_cast<unsigned>(groups), kCollectThreads, 0, s>>>(
+            touched, rows, counts, map->d.ctr, landing, stamp);
     ASH_LAUNCH_CHECK();
+    if (groups > 1) {
+        publish_touched_kernel<<<1, kCollectThreads, 0, s>>>(
+                map->d.ctr, counts, static_cast<int>(groups), landing, stamp);
+        ASH_LAUNCH_CHECK();
+    }
     map->counters_known = false;
     late_words_queued(map, stamp);
     return 0;

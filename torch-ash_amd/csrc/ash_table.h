@@ -215,9 +215,11 @@ int wait_for_words(const uint64_t* words, int count, int32_t stamp);
 inline bool tombs_in(const ash_map* map) { return map->maybe_tombstones || map->replayed; }
 // Waits for the counters that a launch may still owe at kLineLate.
 int settle_landing_place(ash_map* map);
-// Adds up `n` words of `counts` into the counter of touched blocks and queues the
-// read-back of the counters behind the stream's work (ash_map.hip).
-int queue_touched_count(ash_map* map, const int32_t* counts, int n, hipStream_t s);
+// Counts the flags that are up among the first `rows` into the counter of touched
+// blocks and queues the read-back of the counters behind the stream's work; `counts`:
+// `max_counts` words of scratch on the device (ash_map.hip).
+int queue_touched_count(ash_map* map, const uint8_t* touched, int64_t rows, int32_t* counts,
+                        int max_counts, hipStream_t s);
 // The streaming insert (ash_bulk.hip); `early`: page-locked word (or null) where
 // its first pass leaves the number of keys that it hands to the per-key kernel,
 // under `stamp`.  With `early` the call waits for that number; is it zero, the last

@@ -410,9 +410,10 @@ int ash_map_erase_bulk(ash_map_t* map, const int32_t* keys, int64_t n, void* wor
  *   2. it takes the streaming path (ash_map_insert_bulk) when the batch is large
  *      enough relative to the table, else the per-key kernel, with `scratch` as
  *      the workspace of either (`policy` overrides the choice);
- *   3. it reads the counters, or -- streaming path, no key of the
- *      batch handed to the per-key kernel -- queues their read-back behind the insert and returns without waiting
- *      for it (ash_map_counters picks it up).
+ *   3. it reads the counters, or -- streaming path, no key of the batch handed to
+ *      the per-key kernel; per-key kernel under ASH_STREAMING_EARLY, no key that
+ *      waits for the second region -- queues their read-back behind the insert and
+ *      returns without waiting for it (ash_map_counters picks it up).
  * Returns ASH_NEEDS_GENERAL (and inserts everything else) when keys of the
  * batch do not fit the packed code and no second region is attached: attach
  * one and issue the same call again.  n_values may be 0 (keys only).
@@ -425,8 +426,9 @@ int ash_map_erase_bulk(ash_map_t* map, const int32_t* keys, int64_t n, void* wor
 enum { ASH_STREAMING_AUTO = 0, ASH_STREAMING_ALWAYS = 1, ASH_STREAMING_NEVER = 2,
        /* inserts only: as AUTO, and in batches from 2^16 keys (2^17 with value rows)
         * into tables emptied and not used since, where they pay off as long as most
-        * of the keys are not repeated; the package's own choice.  (AUTO keeps the
-        * bars by which callers have sized their scratch.) */
+        * of the keys are not repeated, and without a wait for the counters of other
+        * batches; the package's own choice.  (AUTO keeps the bars by which callers
+        * have sized their scratch.) */
        ASH_STREAMING_EARLY = 3 };
 enum { ASH_NEEDS_GENERAL = 2 };
 int ash_map_insert_scratch_bytes(ash_map_t* map, int64_t n, int n_values,

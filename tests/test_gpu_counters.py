@@ -91,3 +91,61 @@ def test_erases_in_a_row_and_on_two_streams(ash):
     left = engine.keys().cpu().numpy()
     want = _keys(40_000, 10_000).cpu().numpy()
     assert np.array_equal(np.unique(left, axis=0), np.unique(want, axis=0))
+
+
+CHECK = 16 * 256          # keys that a workgroup of the check looks at in its first turns
+MOST = 256 * CHECK        # from here on each goes on
+
+
+@pytest.mark.parametrize("dim, away", [(2, 2**31 - 1), (3, 1 << 20), (4, 1 << 15)])
+@pytest.mark.parametrize("n, at", [(1, 0), (256, 255), (CHECK, 17), (CHECK + 1, CHECK), (70_001, 69_999),
+                                   (MOST + 300, 5), (MOST + 300, MOST + 299)])
+def test_keys_that_do_not_pack_are_met_wherever_they_stand(ash, dim, away, n, at):
+    """One key of a batch does not fit the packed code: the insert attaches the second
+    region and stores it.  The batch before has none: nothing is attached."""
+    # (so much room that no batch streams into a table in use)
+    engine = ash.ASHEngine(dim, 12 * n + 64, DEV)
+    i = torch.arange(2 * n, dtype=torch.int32, device=DEV)
+    keys = torch.zeros(2 * n, dim, dtype=torch.int32, device=DEV)
+    edge = {2: 2000, 3: 131, 4: 40}[dim]
+    for d in range(dim):
+        keys[:, d] = i // edge**d % edge
+    engine.insert_keys(keys[:n].contiguous())
+    assert engine.backend._general is None
+    assert engine.size() == n
+    batch = keys[n:].contiguous()
+    batch[at] = away
+    engine.insert_keys(batch)
+    assert engine.backend._general is not None
+    _agree(engine, 2 * n)
+    assert bool(engine.find(batch)[1].all()) and bool(engine.find(keys[:n].contiguous())[1].all())
+
+
+def test_inserts_in_a_row_and_by_two_threads(ash):
+    """The words that an insert leaves belong to one call at a time: batches one after
+    the other without a look at the counters, and inserts, erases and sizes of two
+    threads, each on a stream of its own."""
+    import threading
+
+    engine = ash.ASHEngine(3, 300_000, DEV)
+    for b in range(6):
+        engine.insert_keys(_keys(b * 3_001, 3_001))
+    _agree(engine, 6 * 3_001)
+
+    def work(first):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for b in range(20):
+                engine.insert_keys(_keys(first + b * 1_500, 1_500))
+                if b % 3 == 1:
+                    engine.erase(_keys(first + b * 1_500, 500))
+                if b % 4 == 2:
+                    engine.size()
+            torch.cuda.current_stream().synchronize()
+
+    torch.cuda.synchronize()
+    both = [threading.Thread(target=work, args=(first,)) for first in (50_000, 150_000)]
+    for t in both:
+        t.start()
+    for t in both:
+        t.join()
+    _agree(engine, 6 * 3_001 + 2 * (20 * 1_500 - 7 * 500))

@@ -170,9 +170,9 @@ class ASHEngine(nn.Module):
 
     def _surely_stored(self, inserted: int, room: Optional[int]) -> bool:
         """Whether the overflow check can be left out: the backend has returned
-        from a streaming insert without reading its counters, and the batch
-        fitted the free indices, so no key was refused for lack of room.  The
-        counters are looked at by the next call that needs them."""
+        from the insert without reading its counters, and the batch fitted the
+        free indices, so no key was refused for lack of room.  The counters are
+        looked at by the next call that needs them."""
         return (
             room is not None
             and inserted <= room

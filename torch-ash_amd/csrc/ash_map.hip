@@ -596,25 +596,68 @@ __device__ __forceinline__ void leave_counters(const int32_t* ctr, uint64_t* lan
 // (change_counter).  No fence: one per wavefront has the L2 written back each time
 // (65 537 keys that take a few tombstones per workgroup: 18 -> 40 us, and erased
 // again 12 -> 28; as it is 18 and 12).
-__device__ __forceinline__ void leave_with_last(const MapDev& m, const Publish& publish) {
+// `groups`: the workgroups that come here.
+__device__ __forceinline__ void leave_with_last(const MapDev& m, const Publish& publish,
+                                                unsigned groups) {
     if (publish.landing == nullptr) return;
     __shared__ bool s_last;
     __syncthreads();
     if (threadIdx.x == 0) {
-        s_last = atomicAdd(publish.ticket, 1) == static_cast<int32_t>(gridDim.x) - 1;
+        s_last = atomicAdd(publish.ticket, 1) == static_cast<int32_t>(groups) - 1;
         if (s_last) atomicExch(publish.ticket, 0);
     }
     __syncthreads();
     if (s_last) leave_counters(m.ctr, publish.landing, publish.stamp);
 }
 
+// What the host waits for before it returns from an insert, where there is no second
+// region: whether every key fits the packed code.  The first `groups` workgroups of
+// the launch (none: nobody waits) look at all keys and at nothing else, and the last
+// of them leaves the number of workgroups that have met one that does not fit.  That
+// is there as soon as the launch has begun, and what follows the insert is queued
+// while it runs; from its counters, behind it, the host knew only when it was done
+// (a batch of 65 537 that comes, is read and goes: 101.5 us, 90 this way; a map of 1000
+// keys filled and read back 45.5 -> 34).
+struct KeyCheck {
+    unsigned groups;
+    uint64_t* word;    // page-locked
+    int32_t stamp;
+    int32_t* ticket;   // zero before and after
+};
+constexpr int kCheckKeys = 16;   // per thread: a few turns of four loads
+constexpr unsigned kMostChecks = 256;
+
+template <int DIM>
+__device__ __forceinline__ void check_keys(const int32_t* __restrict__ keys, int64_t n,
+                                           const KeyCheck& check) {
+    bool bad = false;
+    const int64_t stride = static_cast<int64_t>(check.groups) * kHeapBlock;
+#pragma unroll 4
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * kHeapBlock + threadIdx.x; i < n; i += stride) {
+        int32_t k[DIM];
+        load_key<DIM>(keys, i, true, k);
+        uint64_t code;
+        bad = bad | !pack_key<DIM>(k, code);
+    }
+    bad = __syncthreads_or(bad) != 0;
+    if (threadIdx.x != 0) return;
+    constexpr int kBad = 1 << 16;
+    static_assert(kMostChecks < kBad, "workgroups below, those that met such a key above");
+    const int32_t before = atomicAdd(check.ticket, bad ? kBad + 1 : 1);
+    if ((before & (kBad - 1)) != static_cast<int32_t>(check.groups) - 1) return;
+    atomicExch(check.ticket, 0);
+    leave_word(check.word, (before >> 16) + (bad ? 1 : 0), check.stamp);
+}
+
 template <int DIM, int MODE, bool TOMBS>
 __global__ __launch_bounds__(kHeapBlock) void insert_kernel(
         MapDev m, const int32_t* __restrict__ keys, int64_t n, ValueArgs va,
-        int32_t* __restrict__ assigned, const int64_t* __restrict__ given, Publish publish) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * kHeapBlock + threadIdx.x;
+        int32_t* __restrict__ assigned, const int64_t* __restrict__ given, Publish publish,
+        KeyCheck check) {
+    if (blockIdx.x < check.groups) return check_keys<DIM>(keys, n, check);
+    const int64_t i = static_cast<int64_t>(blockIdx.x - check.groups) * kHeapBlock + threadIdx.x;
     insert_one<DIM, MODE, TOMBS, false>(m, keys, i, i < n, va, assigned, given);
-    leave_with_last(m, publish);
+    leave_with_last(m, publish, gridDim.x - check.groups);
 }
 
 // The same insert over a selection made on the device: thread t of the
@@ -1013,7 +1056,7 @@ __global__ __launch_bounds__(kEraseBlock) void erase_kernel(
         MapDev m, const int32_t* __restrict__ keys, int64_t n, Publish publish) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * kEraseBlock + threadIdx.x;
     erase_one<DIM, false>(m, keys, i, i < n);
-    leave_with_last(m, publish);
+    leave_with_last(m, publish, gridDim.x);
 }
 
 // The same erase over a selection made on the device (see
@@ -2434,6 +2477,47 @@ void late_words_queued(ash_map* map, int32_t stamp, bool of_erase = false) {
     map->late_of_erase = of_erase;
 }
 
+// The landing place at kLineLate, of one call from `take` on: a call of another thread
+// waits for its words (or does without) before it has others left there.
+class LatePlace {
+  public:
+    explicit LatePlace(ash_map* map) : map_(map) {}
+    ~LatePlace() {   // (nothing has been launched)
+        if (!taken_) return;
+        std::lock_guard<std::mutex> lock(map_->counter_lock);
+        if (map_->late_stamp == stamp) map_->late_in_flight = false;
+    }
+    // `settle`: words that are owed are waited for; else the place may not be had.
+    int take(bool settle) {
+        if (take_line(map_)) return 1;
+        std::lock_guard<std::mutex> lock(map_->counter_lock);
+        if (settle) {
+            if (settle_late_words(map_)) return 1;
+        } else if (map_->late_in_flight && !all_come(map_->line + kLineLate, kHostCounters, map_->late_stamp)) {
+            return 0;
+        }
+        stamp = map_->stamp = next_stamp(map_->stamp);
+        map_->late_stamp = stamp;
+        map_->late_in_flight = taken_ = true;
+        map_->late_pending = false;
+        return 0;
+    }
+    bool taken() const { return taken_; }
+    // The launch that leaves the words is queued: they are the latest state of the
+    // counters, unless another thread's call has changed them since.
+    void queued(bool of_erase) {
+        std::lock_guard<std::mutex> lock(map_->counter_lock);
+        taken_ = false;
+        if (!of_erase) map_->unread_inserts = 0;
+        if (map_->late_stamp == stamp) late_words_queued(map_, stamp, of_erase);
+    }
+    int32_t stamp = 0;
+
+  private:
+    ash_map* map_;
+    bool taken_ = false;
+};
+
 }  // namespace
 
 int settle_landing_place(ash_map* map) {
@@ -2471,13 +2555,13 @@ namespace {
 template <int MODE, bool TOMBS>
 int launch_insert_to(ash_map* map, const int32_t* keys, int64_t n,
                      const ValueArgs& va, int32_t* assigned, const int64_t* given,
-                     hipStream_t s, const Publish& publish = {}) {
-    const unsigned g = grid_for(n, kHeapBlock);
+                     hipStream_t s, const Publish& publish = {}, const KeyCheck& check = {}) {
+    const unsigned g = grid_for(n, kHeapBlock) + check.groups;
     auto kernel = map->key_dim == 1   ? insert_kernel<1, MODE, TOMBS>
                   : map->key_dim == 2 ? insert_kernel<2, MODE, TOMBS>
                   : map->key_dim == 3 ? insert_kernel<3, MODE, TOMBS>
                                       : insert_kernel<4, MODE, TOMBS>;
-    kernel<<<g, kHeapBlock, 0, s>>>(map->d, keys, n, va, assigned, given, publish);
+    kernel<<<g, kHeapBlock, 0, s>>>(map->d, keys, n, va, assigned, given, publish, check);
     ASH_LAUNCH_CHECK();
     return 0;
 }
@@ -2485,10 +2569,10 @@ int launch_insert_to(ash_map* map, const int32_t* keys, int64_t n,
 template <int MODE>
 int launch_insert(ash_map* map, const int32_t* keys, int64_t n,
                   const ValueArgs& va, int32_t* assigned, const int64_t* given,
-                  hipStream_t s, const Publish& publish) {
+                  hipStream_t s, const Publish& publish, const KeyCheck& check) {
     return tombs_in(map)
-                   ? launch_insert_to<MODE, true>(map, keys, n, va, assigned, given, s, publish)
-                   : launch_insert_to<MODE, false>(map, keys, n, va, assigned, given, s, publish);
+                   ? launch_insert_to<MODE, true>(map, keys, n, va, assigned, given, s, publish, check)
+                   : launch_insert_to<MODE, false>(map, keys, n, va, assigned, given, s, publish, check);
 }
 
 template <int MODE, bool TOMBS>
@@ -3166,7 +3250,7 @@ int ash_grid_activate_positions(ash_map_t* map, const float* positions, int64_t 
 namespace {
 int insert_per_key(ash_map* map, const int32_t* keys, int64_t n, int n_values,
                    const void* const* src, void* const* dst, const int64_t* row_bytes,
-                   int32_t* assigned, void* stream, const Publish& publish = {});
+                   int32_t* assigned, void* stream, const Publish& publish = {}, const KeyCheck& check = {});
 }
 
 int ash_map_insert_keys(ash_map_t* map, const int32_t* keys, int64_t n,
@@ -3251,7 +3335,8 @@ namespace {
 // `publish`: what the launch that changes the counters leaves for the host.
 int insert_per_key(ash_map* map, const int32_t* keys, int64_t n, int n_values,
                    const void* const* src, void* const* dst, const int64_t* row_bytes,
-                   int32_t* assigned, void* stream, const Publish& publish) {
+                   int32_t* assigned, void* stream, const Publish& publish,
+                   const KeyCheck& check) {
     if (check_batch(map, keys, n)) return 1;
     if (n_values < 0) ASH_FAIL("negative value count");
     if (n_values > 0 && (src == nullptr || dst == nullptr || row_bytes == nullptr)) {
@@ -3268,7 +3353,7 @@ int insert_per_key(ash_map* map, const int32_t* keys, int64_t n, int n_values,
     if (settle_table(map, s)) return 1;
     counters_changed(map, true, s);
     ValueArgs va = {};
-    if (n_values == 0) return launch_insert<kInsertKeys>(map, keys, n, va, nullptr, nullptr, s, publish);
+    if (n_values == 0) return launch_insert<kInsertKeys>(map, keys, n, va, nullptr, nullptr, s, publish, check);
     if (!ash_map_insert_needs_scratch(n_values, row_bytes)) {
         va.n = n_values;
         for (int v = 0; v < n_values; ++v) {
@@ -3276,12 +3361,12 @@ int insert_per_key(ash_map* map, const int32_t* keys, int64_t n, int n_values,
             va.dst[v] = static_cast<uint32_t*>(dst[v]);
             va.row_dwords[v] = static_cast<int32_t>(row_bytes[v] / 4);
         }
-        return launch_insert<kInsertFused>(map, keys, n, va, nullptr, nullptr, s, publish);
+        return launch_insert<kInsertFused>(map, keys, n, va, nullptr, nullptr, s, publish, check);
     }
     if (assigned == nullptr) {
         ASH_FAIL("these value rows need the `assigned` temporary");
     }
-    if (launch_insert<kInsertAssign>(map, keys, n, va, assigned, nullptr, s, publish)) {
+    if (launch_insert<kInsertAssign>(map, keys, n, va, assigned, nullptr, s, publish, check)) {
         return 1;
     }
     for (int v = 0; v < n_values; ++v) {
@@ -3314,14 +3399,10 @@ int ash_map_erase(ash_map_t* map, const int32_t* keys, int64_t n,
     // counters, and finds them with a launch less.  (Not where the words of an
     // earlier call are still owed: a run of erases is not to wait for each other.)
     Publish publish = {};
+    LatePlace late(map);
     if (n <= kLeaveKeys && !map->replayed && !is_capturing(s)) {
-        if (take_line(map)) return 1;
-        std::lock_guard<std::mutex> lock(map->counter_lock);
-        if (!map->late_in_flight ||
-            all_come(map->line + kLineLate, kHostCounters, map->late_stamp)) {
-            map->late_in_flight = false;
-            publish = {map->line + kLineLate, map->stamp = next_stamp(map->stamp), next_ticket(map)};
-        }
+        if (late.take(false)) return 1;
+        if (late.taken()) publish = {map->line + kLineLate, late.stamp, next_ticket(map)};
     }
     const unsigned g = grid_for(n, kEraseBlock);
     auto kernel = map->key_dim == 1   ? erase_kernel<1>
@@ -3330,10 +3411,7 @@ int ash_map_erase(ash_map_t* map, const int32_t* keys, int64_t n,
                                       : erase_kernel<4>;
     kernel<<<g, kEraseBlock, 0, s>>>(map->d, keys, n, publish);
     ASH_LAUNCH_CHECK();
-    if (publish.landing != nullptr) {
-        std::lock_guard<std::mutex> lock(map->counter_lock);
-        late_words_queued(map, publish.stamp, true);
-    }
+    if (late.taken()) late.queued(true);
     return 0;
 }
 
@@ -3693,25 +3771,60 @@ int ash_map_insert_auto(ash_map_t* map, const int32_t* keys, int64_t n, int n_va
             return 0;
         }
     } else {
-        // the counters are waited for below: short launches leave them themselves
-        Answer answer;
-        Publish publish = {};
-        if (!capturing && n <= kLeaveKeys) {
-            if (answer.take()) return 1;
-            publish = {answer.words, answer.stamp, next_ticket(map)};
-        }
-        if (insert_per_key(map, keys, n, n_values, src, dst, row_bytes,
-                           path == kPathAssigned ? static_cast<int32_t*>(scratch) : nullptr,
-                           stream, publish)) {
-            answer.abandon();   // (the launch may have been made)
-            return 1;
-        }
-        if (capturing) return 0;
-        if (publish.landing != nullptr) {
-            if (answer.wait(s, kHostCounters)) return 1;
-            std::lock_guard<std::mutex> lock(map->counter_lock);
-            decode_counters(answer.words, map->counters);
-            counters_taken(map);
+        // The counters come behind the insert (a short launch leaves them itself) and
+        // wait for the call that asks for them; only keys that may be waiting for the
+        // second region are waited for here.  (Under the other policies callers find
+        // the counters read.  Replays change them behind the host's back: read, too.)
+        if (capturing || map->replayed || policy != ASH_STREAMING_EARLY) {
+            // (short launches leave what is waited for below themselves)
+            Answer answer;
+            Publish publish = {};
+            if (!capturing && n <= kLeaveKeys) {
+                if (answer.take()) return 1;
+                publish = {answer.words, answer.stamp, next_ticket(map)};
+            }
+            if (insert_per_key(map, keys, n, n_values, src, dst, row_bytes,
+                               path == kPathAssigned ? static_cast<int32_t*>(scratch) : nullptr,
+                               stream, publish)) {
+                answer.abandon();   // (the launch may have been made)
+                return 1;
+            }
+            if (capturing) return 0;
+            if (publish.landing != nullptr) {
+                if (answer.wait(s, kHostCounters)) return 1;
+                std::lock_guard<std::mutex> lock(map->counter_lock);
+                decode_counters(answer.words, map->counters);
+                counters_taken(map);
+            }
+        } else {
+            Answer answer;
+            KeyCheck check = {};
+            if (map->key_dim > 1 && !map->general_attached) {
+                if (answer.take()) return 1;
+                const int64_t groups = (n + kCheckKeys * kHeapBlock - 1) / (kCheckKeys * kHeapBlock);
+                check = {static_cast<unsigned>(std::min<int64_t>(groups, kMostChecks)), answer.words,
+                         answer.stamp, next_ticket(map)};
+            }
+            // (the words of the answer may come from any exit below that follows a launch)
+            if (check.groups > 0) answer.abandon();
+            LatePlace late(map);
+            if (late.take(true)) return 1;
+            const bool leaves = n <= kLeaveKeys;
+            Publish publish = {};
+            if (leaves) publish = {map->line + kLineLate, late.stamp, next_ticket(map)};
+            if (insert_per_key(map, keys, n, n_values, src, dst, row_bytes,
+                               path == kPathAssigned ? static_cast<int32_t*>(scratch) : nullptr,
+                               stream, publish, check)) {
+                return 1;
+            }
+            if (!leaves) {
+                publish_counters_kernel<<<1, 64, 0, s>>>(map->d.ctr, map->line + kLineLate, late.stamp);
+                ASH_LAUNCH_CHECK();
+            }
+            late.queued(false);
+            if (check.groups == 0) return 0;
+            if (answer.wait(s, 1)) return 1;
+            if (value_of(answer.words[0]) == 0) return 0;
         }
     }
     if (refresh_counters(map, s)) return 1;

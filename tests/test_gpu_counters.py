@@ -149,3 +149,25 @@ def test_inserts_in_a_row_and_by_two_threads(ash):
     for t in both:
         t.join()
     _agree(engine, 6 * 3_001 + 2 * (20 * 1_500 - 7 * 500))
+
+
+@pytest.mark.parametrize("n", [(3 << 16) - 1, 3 << 16, (3 << 16) + 1, (3 << 16) + 513])
+@pytest.mark.parametrize("with_rows", [False, True])
+def test_batches_from_which_workgroups_are_larger(ash, n, with_rows):
+    """Keys of which a third is stored already, into a table with tombstones and without:
+    every key once, under an index of its own, with its own row."""
+    m = ash.HashMap(3, {"id": 1}, 10 * n, DEV)
+    rows = {"id": torch.arange(n, device=DEV).float().view(-1, 1)}
+    stored = _keys(0, n // 3)
+    for turn in range(3):
+        m.insert(stored, {"id": rows["id"][: n // 3].contiguous()})
+        keys = _keys(0, n)
+        m.insert(keys, rows) if with_rows else m.engine.insert_keys(keys)
+        _agree(m.engine, n)
+        idx, masks = m.engine.find(keys)
+        assert bool(masks.all()) and len(torch.unique(idx)) == n
+        if with_rows:
+            assert torch.equal(m.values["id"][idx], rows["id"])
+        m.erase(_keys(n // 5, n - n // 5) if turn else keys)
+        _agree(m.engine, n // 5 if turn else 0)
+        m.erase(_keys(0, n // 5))

@@ -51,9 +51,8 @@ namespace {
 
 constexpr int kBlock = 256;
 // Workgroup size of the kernels that advance the heap counter (once per
-// workgroup).  Larger groups mean fewer updates of that single address but
-// make every wavefront wait for the slowest probe of the group; measured on
-// 16 M keys: 256 -> 1.28 ms, 512 -> 1.46 ms, 1024 -> 1.42 ms.
+// workgroup).  Larger groups mean fewer updates of that single address but make
+// every wavefront wait for the slowest probe of the group (kWideInsert).
 constexpr int kHeapBlock = 256;
 constexpr uint32_t kSpinLimit = 1u << 22;
 
@@ -306,7 +305,8 @@ __device__ __forceinline__ void change_counter(int32_t* counter, int32_t by) {
 // The insert proper for a key held in registers (`code` is its packed form if
 // `fits`); `i` is the row of the key's value rows / `assigned` / `given` entry.
 // TOMBS: the table may hold tombstones (the same for the whole launch).
-template <int DIM, int MODE, bool TOMBS>
+// BLOCK: threads of the workgroup, all of which call this together.
+template <int DIM, int MODE, bool TOMBS, int BLOCK = kHeapBlock>
 __device__ __forceinline__ void insert_key(
         const MapDev& m, const int32_t (&k)[DIM], uint64_t code, bool fits,
         int64_t i, bool active, const ValueArgs& va,
@@ -452,8 +452,8 @@ __device__ __forceinline__ void insert_key(
             }
         }
     } else {
-        __shared__ int s_cnt[kHeapBlock / 64];
-        __shared__ int s_reused[kHeapBlock / 64];
+        __shared__ int s_cnt[BLOCK / 64];
+        __shared__ int s_reused[BLOCK / 64];
         __shared__ int s_base;
         const uint64_t wm = __ballot(w);
         const int nw = __popcll(wm);
@@ -466,7 +466,7 @@ __device__ __forceinline__ void insert_key(
         if (threadIdx.x == 0) {
             int tot = 0, again = 0;
 #pragma unroll
-            for (int q = 0; q < kHeapBlock / 64; ++q) {
+            for (int q = 0; q < BLOCK / 64; ++q) {
                 tot += s_cnt[q];
                 if constexpr (TOMBS) again += s_reused[q];
             }
@@ -562,7 +562,7 @@ __device__ __forceinline__ void insert_key(
 
 // One key per thread, every thread of the workgroup calls this together.
 // CODES: `keys` holds packed 64-bit codes instead of int32[DIM] rows.
-template <int DIM, int MODE, bool TOMBS, bool CODES>
+template <int DIM, int MODE, bool TOMBS, bool CODES, int BLOCK = kHeapBlock>
 __device__ __forceinline__ void insert_one(
         const MapDev& m, const int32_t* __restrict__ keys, int64_t i,
         bool active, const ValueArgs& va, int32_t* __restrict__ assigned,
@@ -577,7 +577,7 @@ __device__ __forceinline__ void insert_one(
         load_key<DIM>(keys, i, active, k);
         fits = pack_key<DIM>(k, code);
     }
-    insert_key<DIM, MODE, TOMBS>(m, k, code, fits, i, active, va, assigned, given);
+    insert_key<DIM, MODE, TOMBS, BLOCK>(m, k, code, fits, i, active, va, assigned, given);
 }
 
 // The counters, left where the host reads them: `landing` is a place in page-locked
@@ -627,13 +627,13 @@ struct KeyCheck {
 constexpr int kCheckKeys = 16;   // per thread: a few turns of four loads
 constexpr unsigned kMostChecks = 256;
 
-template <int DIM>
+template <int DIM, int BLOCK>
 __device__ __forceinline__ void check_keys(const int32_t* __restrict__ keys, int64_t n,
                                            const KeyCheck& check) {
     bool bad = false;
-    const int64_t stride = static_cast<int64_t>(check.groups) * kHeapBlock;
+    const int64_t stride = static_cast<int64_t>(check.groups) * BLOCK;
 #pragma unroll 4
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * kHeapBlock + threadIdx.x; i < n; i += stride) {
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * BLOCK + threadIdx.x; i < n; i += stride) {
         int32_t k[DIM];
         load_key<DIM>(keys, i, true, k);
         uint64_t code;
@@ -649,14 +649,14 @@ __device__ __forceinline__ void check_keys(const int32_t* __restrict__ keys, int
     leave_word(check.word, (before >> 16) + (bad ? 1 : 0), check.stamp);
 }
 
-template <int DIM, int MODE, bool TOMBS>
-__global__ __launch_bounds__(kHeapBlock) void insert_kernel(
+template <int DIM, int MODE, bool TOMBS, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void insert_kernel(
         MapDev m, const int32_t* __restrict__ keys, int64_t n, ValueArgs va,
         int32_t* __restrict__ assigned, const int64_t* __restrict__ given, Publish publish,
         KeyCheck check) {
-    if (blockIdx.x < check.groups) return check_keys<DIM>(keys, n, check);
-    const int64_t i = static_cast<int64_t>(blockIdx.x - check.groups) * kHeapBlock + threadIdx.x;
-    insert_one<DIM, MODE, TOMBS, false>(m, keys, i, i < n, va, assigned, given);
+    if (blockIdx.x < check.groups) return check_keys<DIM, BLOCK>(keys, n, check);
+    const int64_t i = static_cast<int64_t>(blockIdx.x - check.groups) * BLOCK + threadIdx.x;
+    insert_one<DIM, MODE, TOMBS, false, BLOCK>(m, keys, i, i < n, va, assigned, given);
     leave_with_last(m, publish, gridDim.x - check.groups);
 }
 
@@ -2552,18 +2552,35 @@ int give_up_heap_order(ash_map* map, hipStream_t s) {
 
 namespace {
 
+template <int MODE, bool TOMBS, int BLOCK>
+int launch_insert_by(ash_map* map, const int32_t* keys, int64_t n,
+                     const ValueArgs& va, int32_t* assigned, const int64_t* given,
+                     hipStream_t s, const Publish& publish = {}, const KeyCheck& check = {}) {
+    const unsigned g = grid_for(n, BLOCK) + check.groups;
+    auto kernel = map->key_dim == 1   ? insert_kernel<1, MODE, TOMBS, BLOCK>
+                  : map->key_dim == 2 ? insert_kernel<2, MODE, TOMBS, BLOCK>
+                  : map->key_dim == 3 ? insert_kernel<3, MODE, TOMBS, BLOCK>
+                                      : insert_kernel<4, MODE, TOMBS, BLOCK>;
+    kernel<<<g, BLOCK, 0, s>>>(map->d, keys, n, va, assigned, given, publish, check);
+    ASH_LAUNCH_CHECK();
+    return 0;
+}
+
+// Larger workgroups update the heap counter (and, of tombstones, theirs) less often, but
+// each of their wavefronts waits for the slowest probe of all.  A batch that comes, is read
+// and goes, of 256 -> 512 threads (us): 140 000 keys beside 20 000 111 -> 115, beside a
+// million 116 -> 114; 200 000 beside a million 135 -> 128, beside four 225 -> 217; 400 000
+// beside 300 000 188 -> 162; a million beside four 424 -> 397 (1024 threads: 402).
+constexpr int64_t kWideInsert = int64_t{3} << 16;
+constexpr int kWideBlock = 512;
+
 template <int MODE, bool TOMBS>
 int launch_insert_to(ash_map* map, const int32_t* keys, int64_t n,
                      const ValueArgs& va, int32_t* assigned, const int64_t* given,
                      hipStream_t s, const Publish& publish = {}, const KeyCheck& check = {}) {
-    const unsigned g = grid_for(n, kHeapBlock) + check.groups;
-    auto kernel = map->key_dim == 1   ? insert_kernel<1, MODE, TOMBS>
-                  : map->key_dim == 2 ? insert_kernel<2, MODE, TOMBS>
-                  : map->key_dim == 3 ? insert_kernel<3, MODE, TOMBS>
-                                      : insert_kernel<4, MODE, TOMBS>;
-    kernel<<<g, kHeapBlock, 0, s>>>(map->d, keys, n, va, assigned, given, publish, check);
-    ASH_LAUNCH_CHECK();
-    return 0;
+    return n > kWideInsert && (MODE == kInsertKeys || MODE == kInsertFused)
+                   ? launch_insert_by<MODE, TOMBS, kWideBlock>(map, keys, n, va, assigned, given, s, publish, check)
+                   : launch_insert_by<MODE, TOMBS, kHeapBlock>(map, keys, n, va, assigned, given, s, publish, check);
 }
 
 template <int MODE>

@@ -61,8 +61,8 @@ constexpr uint32_t kPartBuckets = 1u << kPartShift;
 // Device counters kept in the first 256 bytes of the table workspace.
 enum Counter {
     kCtrSize = 0,      // heap counter == number of live entries
-    kCtrDropped = 1,   // keys refused because the heap was exhausted
-    kCtrTombs = 2,     // tombstoned slots (packed + general)
+    kCtrTombs = 1,     // tombstoned slots (packed + general); changed with the size (change_size)
+    kCtrDropped = 2,   // keys refused because the heap was exhausted
     kCtrExotic = 3,    // unpackable keys seen while no general region exists
     kCtrLoadDup = 4,   // pairs refused by load: duplicate keys, indices outside 0 .. capacity-1
     kCtrGenLive = 5,   // entries that live in the general region

@@ -2589,14 +2589,17 @@ int launch_insert_by(ash_map* map, const int32_t* keys, int64_t n,
 // and goes, of 256 -> 512 threads (us): 140 000 keys beside 20 000 111 -> 115, beside a
 // million 116 -> 114; 200 000 beside a million 135 -> 128, beside four 225 -> 217; 400 000
 // beside 300 000 188 -> 162; a million beside four 424 -> 397 (1024 threads: 402).
-constexpr int64_t kWideInsert = int64_t{3} << 16;
+// Beyond three million the waits weigh more (the insert alone, without and with rows: a
+// million 117 -> 96, 126 -> 102; two 170 -> 146, 179 -> 150; four 322 -> 317, 363 -> 372;
+// eight 642 -> 647, 676 -> 732; sixteen 1016 -> 1039, 1117 -> 1239).
+constexpr int64_t kWideInsert = int64_t{3} << 16, kWideInsertEnd = int64_t{3} << 20;
 constexpr int kWideBlock = 512;
 
 template <int MODE, bool TOMBS>
 int launch_insert_to(ash_map* map, const int32_t* keys, int64_t n,
                      const ValueArgs& va, int32_t* assigned, const int64_t* given,
                      hipStream_t s, const Publish& publish = {}, const KeyCheck& check = {}) {
-    return n > kWideInsert && (MODE == kInsertKeys || MODE == kInsertFused)
+    return n > kWideInsert && n <= kWideInsertEnd && (MODE == kInsertKeys || MODE == kInsertFused)
                    ? launch_insert_by<MODE, TOMBS, kWideBlock>(map, keys, n, va, assigned, given, s, publish, check)
                    : launch_insert_by<MODE, TOMBS, kHeapBlock>(map, keys, n, va, assigned, given, s, publish, check);
 }

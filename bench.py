@@ -119,7 +119,7 @@ MEASURED_COUNTERS = {
 COUNTERS_SOURCE = {
     "profiles": ["profiles/bench_hbm_traffic_pmc.md",
                  "profiles/bench_l2_hit_rate_and_atomics_pmc.md"],
-    "csrc_sha256": "576cd81fe65654a3e10f373df0c45eeb1808ff868efdaac6c490bcebe8988f58",
+    "csrc_sha256": "b6e5106107bb8a48e91e634596896652713252a284a122ffb3ad7f00dc68ea1a",
 }
 
 

@@ -119,7 +119,7 @@ MEASURED_COUNTERS = {
 COUNTERS_SOURCE = {
     "profiles": ["profiles/bench_hbm_traffic_pmc.md",
                  "profiles/bench_l2_hit_rate_and_atomics_pmc.md"],
-    "csrc_sha256": "b6e5106107bb8a48e91e634596896652713252a284a122ffb3ad7f00dc68ea1a",
+    "csrc_sha256": "49111aa2eaedfa5ae836047654a6f58b637ee5960d2350fe23f2c2818b788e49",
 }
 
 

@@ -121,34 +121,36 @@ def test_keys_that_do_not_pack_are_met_wherever_they_stand(ash, dim, away, n, at
     assert bool(engine.find(batch)[1].all()) and bool(engine.find(keys[:n].contiguous())[1].all())
 
 
-def test_inserts_in_a_row_and_by_two_threads(ash):
-    """The words that an insert leaves belong to one call at a time: batches one after
-    the other without a look at the counters, and inserts, erases and sizes of two
-    threads, each on a stream of its own."""
+def test_inserts_in_a_row_while_others_ask_for_the_size(ash):
+    """The words that a call leaves belong to one call at a time: batches that come one
+    after the other without a look at the counters, some of them erased again, while
+    two threads ask for the size."""
     import threading
 
     engine = ash.ASHEngine(3, 300_000, DEV)
     for b in range(6):
         engine.insert_keys(_keys(b * 3_001, 3_001))
     _agree(engine, 6 * 3_001)
+    over, seen = threading.Event(), []
 
-    def work(first):
+    def ask():
         with torch.cuda.stream(torch.cuda.Stream()):
-            for b in range(20):
-                engine.insert_keys(_keys(first + b * 1_500, 1_500))
-                if b % 3 == 1:
-                    engine.erase(_keys(first + b * 1_500, 500))
-                if b % 4 == 2:
-                    engine.size()
-            torch.cuda.current_stream().synchronize()
+            while not over.is_set():
+                seen.append(engine.size())
 
-    torch.cuda.synchronize()
-    both = [threading.Thread(target=work, args=(first,)) for first in (50_000, 150_000)]
-    for t in both:
+    asking = [threading.Thread(target=ask) for _ in range(2)]
+    for t in asking:
         t.start()
-    for t in both:
+    for b in range(40):
+        first = 50_000 + b * 1_500
+        engine.insert_keys(_keys(first, 1_500))
+        if b % 3 == 1:
+            engine.erase(_keys(first, 500))
+    over.set()
+    for t in asking:
         t.join()
-    _agree(engine, 6 * 3_001 + 2 * (20 * 1_500 - 7 * 500))
+    _agree(engine, 6 * 3_001 + 40 * 1_500 - 13 * 500)
+    assert all(6 * 3_001 <= n <= 6 * 3_001 + 40 * 1_500 for n in seen)
 
 
 @pytest.mark.parametrize("n", [(3 << 16) - 1, 3 << 16, (3 << 16) + 1, (3 << 16) + 513])

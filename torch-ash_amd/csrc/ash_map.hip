@@ -2493,6 +2493,9 @@ void late_words_queued(ash_map* map, int32_t stamp, bool of_erase = false) {
     map->late_stamp = stamp;
     map->late_in_flight = map->late_pending = true;
     map->late_of_erase = of_erase;
+    // (a reader may have asked the device before the launch was queued)
+    map->counters_known = false;
+    ++map->changes;
 }
 
 // The landing place at kLineLate, of one call from `take` on: a call of another thread
@@ -2710,6 +2713,7 @@ int settle_table(ash_map* map, hipStream_t s) {
 
 void counters_changed(ash_map* map, bool inserted, hipStream_t s) {
     if (is_capturing(s)) map->replayed = true;
+    ++map->changes;
     map->counters_known = false;
     map->late_pending = false;   // what a queued read-back brings is out of date
     if (inserted) {
@@ -2927,6 +2931,7 @@ int ash_map_create(int key_dim, int64_t capacity, int32_t* heap, void* table_ws,
     map->maybe_tombstones = false;
     map->unread_inserts = 0;
     map->launches = 0;
+    map->changes = 0;
     map->replayed = false;
     map->d.ctr = static_cast<int32_t*>(table_ws);
     map->d.buckets = reinterpret_cast<uint64_t*>(static_cast<char*>(table_ws) +
@@ -3449,7 +3454,13 @@ int ash_map_erase(ash_map_t* map, const int32_t* keys, int64_t n,
                                       : erase_kernel<4>;
     kernel<<<g, kEraseBlock, 0, s>>>(map->d, keys, n, publish);
     ASH_LAUNCH_CHECK();
-    if (late.taken()) late.queued(true);
+    if (late.taken()) {
+        late.queued(true);
+    } else {
+        std::lock_guard<std::mutex> lock(map->counter_lock);
+        map->counters_known = false;
+        ++map->changes;
+    }
     return 0;
 }
 
@@ -3536,6 +3547,7 @@ int refresh_counters(ash_map* map, hipStream_t s, bool ask = false, ash_counters
                 ASH_FAIL("the table's counters cannot be read while the stream is being captured");
             }
             // (each of several readers waits for its own stream, not for the others)
+            const uint32_t changes = map->changes;
             lock.unlock();
             Answer answer;
             if (answer.take()) return 1;
@@ -3543,6 +3555,12 @@ int refresh_counters(ash_map* map, hipStream_t s, bool ask = false, ash_counters
             ASH_LAUNCH_CHECK();
             if (answer.wait(s, kHostCounters)) return 1;
             lock.lock();
+            if (map->changes != changes && copy != nullptr) {
+                // a call of another thread has changed them since: the answer is this
+                // reader's alone
+                decode_counters(answer.words, *copy);
+                return 0;
+            }
             decode_counters(answer.words, map->counters);
         }
         counters_taken(map);

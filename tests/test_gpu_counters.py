@@ -153,6 +153,27 @@ def test_inserts_in_a_row_while_others_ask_for_the_size(ash):
     assert all(6 * 3_001 <= n <= 6 * 3_001 + 40 * 1_500 for n in seen)
 
 
+def test_status_asked_for_beside_an_insert_under_way(ash):
+    """A reader of the device on a stream of its own sees the insert that has returned
+    before it asks, and what the insert leaves for the host stays there for others.
+    (One-dimensional keys: nothing is waited for behind the work in front.)"""
+    engine = ash.ASHEngine(1, 20_000, DEV)
+    work = torch.randn(8192, 8192, device=DEV)
+    keys = torch.arange(16_000, dtype=torch.int32, device=DEV).view(-1, 1)
+    one, other = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for n in (5_000, 16_000):
+        with torch.cuda.stream(one):
+            for _ in range(8):
+                work = torch.tanh(work @ work)
+            engine.insert_keys(keys[:n])
+        with torch.cuda.stream(other):
+            assert engine.backend.status()["size"] == n
+            assert engine.size() == n
+        assert engine.size() == n
+    torch.cuda.synchronize()
+
+
 @pytest.mark.parametrize("n", [(3 << 16) - 1, 3 << 16, (3 << 16) + 1, (3 << 16) + 513])
 @pytest.mark.parametrize("with_rows", [False, True])
 def test_batches_from_which_workgroups_are_larger(ash, n, with_rows):

@@ -3526,43 +3526,53 @@ void counters_taken(ash_map* map) {
     if (map->counters.dropped > 0 || map->counters.tombstones > 0) map->maybe_tombstones = true;
 }
 
+// The words that a call has queued, if they are the latest state, waited for and
+// taken.  The caller holds the map's counter_lock.
+int take_late_words(ash_map* map) {
+    if (!map->late_pending) return 0;
+    if (settle_late_words(map)) return 1;
+    map->late_pending = false;
+    decode_counters(map->line + kLineLate, map->counters);
+    counters_taken(map);
+    return 0;
+}
+
 // Brings map->counters up to date (the map's device is current): they are
 // known already, or a read-back queued behind the latest insert brings them,
-// or they are fetched now, which waits for `s`.  `ask`: fetched in any case;
+// or they are fetched now, which waits for `s`.  `ask`: fetched in any case,
+// behind words that are under way (they belong to a call that has returned);
+// what is fetched beside counters that are known is the asker's alone.
 // `copy`: a copy of them, for callers whose map other threads may read as well.
 int refresh_counters(ash_map* map, hipStream_t s, bool ask = false, ash_counters* copy = nullptr) {
     std::unique_lock<std::mutex> lock(map->counter_lock);
-    if (ask) map->counters_known = map->late_pending = false;
     if (map->replayed) {
         if (settle_late_words(map)) return 1;
         map->counters_known = map->late_pending = false;
     }
-    if (!map->counters_known) {
-        if (map->late_pending) {
-            if (settle_late_words(map)) return 1;
-            map->late_pending = false;
-            decode_counters(map->line + kLineLate, map->counters);
-        } else {
-            if (is_capturing(s)) {
-                ASH_FAIL("the table's counters cannot be read while the stream is being captured");
-            }
-            // (each of several readers waits for its own stream, not for the others)
-            const uint32_t changes = map->changes;
-            lock.unlock();
-            Answer answer;
-            if (answer.take()) return 1;
-            publish_counters_kernel<<<1, 64, 0, s>>>(map->d.ctr, answer.words, answer.stamp);
-            ASH_LAUNCH_CHECK();
-            if (answer.wait(s, kHostCounters)) return 1;
-            lock.lock();
-            if (map->changes != changes && copy != nullptr) {
-                // a call of another thread has changed them since: the answer is this
-                // reader's alone
-                decode_counters(answer.words, *copy);
-                return 0;
-            }
-            decode_counters(answer.words, map->counters);
+    if (take_late_words(map)) return 1;
+    if (ask || !map->counters_known) {
+        if (is_capturing(s)) {
+            ASH_FAIL("the table's counters cannot be read while the stream is being captured");
         }
+        // (each of several readers waits for its own stream, not for the others)
+        const uint32_t changes = map->changes;
+        lock.unlock();
+        Answer answer;
+        if (answer.take()) return 1;
+        publish_counters_kernel<<<1, 64, 0, s>>>(map->d.ctr, answer.words, answer.stamp);
+        ASH_LAUNCH_CHECK();
+        if (answer.wait(s, kHostCounters)) return 1;
+        lock.lock();
+        if (copy != nullptr) {
+            decode_counters(answer.words, *copy);
+            // (a call of another thread may have changed them since)
+            if (map->changes == changes && !map->counters_known) {
+                map->counters = *copy;
+                counters_taken(map);
+            }
+            return 0;
+        }
+        decode_counters(answer.words, map->counters);
         counters_taken(map);
     }
     if (copy != nullptr) *copy = map->counters;
@@ -3686,7 +3696,9 @@ int ash_map_counters(ash_map_t* map, int32_t* staging, int64_t out[7], void* str
 }
 
 int ash_map_counters_pending(ash_map_t* map) {
-    return map != nullptr && map->late_pending && !map->late_of_erase ? 1 : 0;
+    if (map == nullptr) return 0;
+    std::lock_guard<std::mutex> lock(map->counter_lock);
+    return map->late_pending && !map->late_of_erase ? 1 : 0;
 }
 
 int ash_map_known_size(ash_map_t* map, int64_t* size) {
@@ -3696,12 +3708,11 @@ int ash_map_known_size(ash_map_t* map, int64_t* size) {
         return -1;
     }
     if (map->replayed) return 0;
+    std::lock_guard<std::mutex> lock(map->counter_lock);
     if (!map->counters_known) {
         if (!map->late_pending) return 0;
         DeviceGuard guard;
-        if (guard.enter(map->device) != hipSuccess || refresh_counters(map, nullptr)) {
-            return -1;
-        }
+        if (guard.enter(map->device) != hipSuccess || take_late_words(map)) return -1;
     }
     *size = map->counters.size;
     return 1;

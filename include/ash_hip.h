@@ -471,7 +471,7 @@ int ash_map_clear_rows(ash_map_t* map, int n_values, void* const* rows,
                        const int64_t* row_bytes, void* stream);
 
 /* Host read-back of the device counters; always asks the device, which waits
- * for `stream`.
+ * for `stream` (and first for a queued read-back, see below).
  *   out[0] size (= heap counter, ash/src/hashmap_gpu.cuh:157)
  *   out[1] keys dropped because the map was full (since the last clear)
  *   out[2] tombstoned slots
@@ -489,7 +489,9 @@ int ash_map_status(ash_map_t* map, int64_t out[5], void* stream);
  * their way as a rule -- only when neither holds is the device asked,
  * which waits for `stream`: a kernel writes them into page-locked words of the
  * call's own, and the host looks for them there.  Several threads may read the
- * counters of one map at a time, each on its own stream.  `staging` is not
+ * counters of one map at a time, each on its own stream, also while one call changes
+ * them; what a reader was told on another stream than that of the latest change is not
+ * kept (another call there asks again).  `staging` is not
  * used any more (NULL).  No counterpart in the reference, whose `size()`
  * synchronises every time (ash/src/hashmap_gpu.cuh:157). */
 int ash_map_counters(ash_map_t* map, int32_t* staging, int64_t out[7], void* stream);

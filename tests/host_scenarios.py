@@ -2,7 +2,7 @@
 function a test of test_host_counters.py (each in a process of its own)."""
 import time
 
-from stand_in_device import (ALWAYS, DROPPED, EXOTIC, SIZE, Map, beside)
+from stand_in_device import ALWAYS, EXOTIC, SIZE, TOMBS, Map, beside
 
 ONE, OTHER = 0x10, 0x20   # streams
 
@@ -25,3 +25,112 @@ def status_beside_an_insert_under_way(device):
     device.stream(ONE).go()
     asked.join()
     assert (asked.result, m.size(OTHER), m.size(ONE)) == (100, 100, 100)
+
+
+def _stands_at(m, size):
+    """The size as the handle keeps it, on either stream, and as the device has it."""
+    seen = m.size(ONE), m.size(OTHER), m.status(ONE)
+    assert seen == (size,) * 3, seen
+
+
+def a_reader_on_another_stream_than_the_change(device):
+    """What a stream sees that does not wait for the change is not kept."""
+    m = Map(device)
+    device.stream(ONE).hold()
+    device.effects = [{SIZE: 7}]
+    assert m.activate(ONE) == 0
+    assert m.size(OTHER) == 0
+    device.stream(ONE).go()
+    _stands_at(m, 7)
+
+
+def _read_before(device, m, kernel):
+    """A reader that has its answer just before `kernel` is queued on its stream."""
+
+    def read():
+        reader = beside(lambda: m.size(ONE))
+        reader.join()
+        assert reader.result is not None
+
+    device.before[kernel] = read
+
+
+def a_reader_before_the_launch_of_an_activation(device):
+    m = Map(device)
+    device.effects = [{SIZE: 7}]
+    _read_before(device, m, "activate_runs_kernel")
+    assert m.activate(ONE) == 0
+    _stands_at(m, 7)
+
+
+def a_reader_before_the_launch_of_a_bulk_erase(device):
+    m = Map(device)
+    device.effects = [{SIZE: 700}, {SIZE: -600}]
+    assert m.activate(ONE) == 0
+    _read_before(device, m, "erase_range_kernel")
+    assert m.erase_bulk(stream=ONE) == 0
+    _stands_at(m, 100)
+
+
+def a_reader_before_the_last_launches_of_a_streaming_insert(device):
+    """Keys that wait for the second region are reported, whatever a reader was told
+    while the insert was being queued."""
+    m = Map(device)
+    device.spilled = 5
+    device.effects = [{SIZE: 70_000, EXOTIC: 5}]
+    _read_before(device, m, "build_kernel")
+    assert m.insert(70_000, ALWAYS, ONE) == 2   # ASH_NEEDS_GENERAL
+    assert device.ctr[SIZE] == 70_000
+    _stands_at(m, 70_000)
+
+
+def _answer_across(device, m, call):
+    """A reader whose answer is from before `call` and comes after it has returned."""
+    device.stream(OTHER).hold()
+    reader = beside(lambda: m.size(OTHER))
+    while not device.stream(OTHER).queue:
+        time.sleep(0.001)
+    device.stream(ONE).hold()
+    assert call() == 0
+    device.stream(OTHER).go()
+    reader.join()
+    device.stream(ONE).go()
+    return reader.result
+
+
+def a_reader_across_a_clear(device):
+    m = Map(device)
+    device.effects = [{SIZE: 7}]
+    assert m.activate(OTHER) == 0
+    assert _answer_across(device, m, lambda: m.clear(ONE)) == 7
+    _stands_at(m, 0)
+
+
+def a_reader_across_a_load(device):
+    m = Map(device)
+    device.effects = [{SIZE: 7}]
+    assert m.activate(OTHER) == 0
+    assert _answer_across(device, m, lambda: m.load(3, ONE)) == 7
+    _stands_at(m, 3)
+
+
+def a_reader_across_a_rebuild(device):
+    """(the tombstones go: the status has them)"""
+    m = Map(device)
+    device.effects = [{SIZE: 7, TOMBS: 5}]
+    assert m.activate(OTHER) == 0
+    assert _answer_across(device, m, lambda: m.rebuild(ONE)) == 7
+    assert m.counters(ONE)[2] == 0
+
+
+def words_under_way_when_the_second_region_comes(device):
+    """The size is that of the insert before, wherever it is asked for."""
+    m = _queued_insert(device)
+    attached = beside(lambda: m.attach(ONE))
+    time.sleep(0.1)
+    seen = beside(lambda: m.size(OTHER))
+    time.sleep(0.1)
+    device.stream(ONE).go()
+    attached.join(), seen.join()
+    assert (attached.result, seen.result) == (0, 100)
+    _stands_at(m, 100)

@@ -216,6 +216,17 @@ class Map:
         self.ok(self.lib.ash_map_size(self.handle, ctypes.byref(out), PTR(stream)))
         return out.value
 
+    def load(self, n, stream=0):
+        return self.lib.ash_map_load(self.handle, self.keys(), PTR(4096), I64(n), PTR(self.heap), PTR(stream))
+
+    def rebuild(self, stream=0):
+        return self.lib.ash_map_rebuild(self.handle, PTR(4096), PTR(4096), I64(0), PTR(stream))
+
+    def counters(self, stream=0):
+        out = (I64 * 7)()
+        self.ok(self.lib.ash_map_counters(self.handle, PTR(0), out, PTR(stream)))
+        return list(out)
+
     def status(self, stream=0):
         out = (I64 * 5)()
         self.ok(self.lib.ash_map_status(self.handle, out, PTR(stream)))

@@ -174,6 +174,43 @@ def test_status_asked_for_beside_an_insert_under_way(ash):
     torch.cuda.synchronize()
 
 
+def test_readers_beside_calls_that_are_queued_in_parts(ash, monkeypatch):
+    """Streaming inserts with keys for the second region and bulk erases, each several
+    launches, while others ask for the counters: what those are told in between does not
+    stay the latest state, and no key is lost."""
+    import threading
+
+    monkeypatch.setattr(ash.common, "BULK_INSERT", "always")
+    monkeypatch.setattr(ash.common, "BULK_ERASE", "always")
+    engine = ash.ASHEngine(3, 400_000, DEV)
+    engine.insert_keys(_keys(0, 70_000))
+    over = threading.Event()
+
+    def ask(read):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            while not over.is_set():
+                read()
+
+    asking = [threading.Thread(target=ask, args=(read,)) for read in (engine.size, engine.backend.status)]
+    for t in asking:
+        t.start()
+    try:
+        for b in range(12):
+            batch = _keys(70_000 + b * 9_000, 70_000)
+            batch[::500] += 1 << 24
+            engine.insert_keys(batch)
+            stored = engine.size()
+            assert stored == len(torch.unique(torch.cat([_keys(0, 70_000), batch]), dim=0))
+            assert bool(engine.find(batch)[1].all())
+            engine.erase(batch)
+            assert engine.size() == len(_keys(0, 70_000))
+    finally:
+        over.set()
+        for t in asking:
+            t.join()
+    _agree(engine, 70_000)
+
+
 @pytest.mark.parametrize("n", [(3 << 16) - 1, 3 << 16, (3 << 16) + 1, (3 << 16) + 513])
 @pytest.mark.parametrize("with_rows", [False, True])
 def test_batches_from_which_workgroups_are_larger(ash, n, with_rows):

@@ -1762,7 +1762,7 @@ int ash::insert_bulk(ash_map* map, const int32_t* keys, int64_t n,
     }
     const ValueArgs none = {};
     const int stale = map->table_stale && !map->table_filled ? 1 : 0;
-    counters_changed(map, true, s);
+    Change change(map, kChangeAdds, s);
     // (captured into a graph, the choice would be replayed whatever the heap
     // holds then: a captured call takes the variant that reads the heap)
     const int identity = heap_in_order(map) ? 1 : 0;
@@ -1844,7 +1844,7 @@ int ash_map_erase_bulk(ash_map_t* map, const int32_t* keys, int64_t n, void* wor
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (settle_table(map, s)) return 1;
     if (give_up_heap_order(map, s)) return 1;   // freed indices go back onto the heap
-    counters_changed(map, false, s);
+    Change change(map, kChangeErases, s);
     const int ncursors = static_cast<int>(pl.bins << pl.fine_shift);   // (>= bins << lane_shift)
     const int ninit = ncursors > kHdrWords ? ncursors : kHdrWords;
     bulk_init_kernel<<<(ninit + 255) / 256, 256, 0, s>>>(map->d, pl, ncursors);

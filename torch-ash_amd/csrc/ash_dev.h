@@ -175,9 +175,8 @@ struct ash_map {
     bool late_pending;      // ... and it is the latest state of the counters: nobody has looked at it yet
     bool late_of_erase;     // ... left by an erase
     bool counters_known;    // `counters` is what the device holds
-    // counts the calls that change the counters, where they begin and where their
-    // launches are queued: what a reader has asked the device for in between is out of date
-    std::atomic<uint32_t> changes;
+    uint32_t changes;       // both ends of every call that changes the counters (Change)
+    hipStream_t changed_on; // the stream of the latest of them
     ash_counters counters;
     // an erase, refused keys or a run of inserts whose counters nobody read
     // may have left tombstones: the next managed insert looks at the counters

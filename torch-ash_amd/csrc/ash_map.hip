@@ -2229,15 +2229,18 @@ int check_map(const ash_map* map) {
     return 0;
 }
 
+// Whether no entry lives in the second region: there is none, or the counters as
+// the host knows them say that it is empty.
+bool none_in_general(ash_map* map) {
+    if (!map->general_attached) return true;
+    std::lock_guard<std::mutex> lock(map->counter_lock);
+    return map->counters_known && map->counters.general_live == 0;
+}
+
 // Whether a listing has entry i under index i: nothing has written to the heap
 // since it was last 0, 1, 2, ... (no erase, no load) and no entry lives in the
-// second region -- there is none, or the counters as the host knows them say
-// that it is empty.
-bool lists_in_index_order(const ash_map* map) {
-    if (!heap_in_order(map)) return false;
-    return !map->general_attached ||
-           (map->counters_known && map->counters.general_live == 0);
-}
+// second region.
+bool lists_in_index_order(ash_map* map) { return heap_in_order(map) && none_in_general(map); }
 
 int fill_buckets(ash_map* map, hipStream_t s) {
     const int64_t n16 = static_cast<int64_t>(map->d.nb) * kGroup;
@@ -2487,6 +2490,37 @@ int settle_late_words(ash_map* map) {
     return 0;
 }
 
+void decode_counters(const uint64_t* words, ash_counters& c) {
+    int32_t host[kHostCounters];
+    for (int w = 0; w < kHostCounters; ++w) host[w] = value_of(words[w]);
+    c.size = host[kCtrSize];
+    c.dropped = host[kCtrDropped];
+    c.tombstones = host[kCtrTombs];
+    c.exotic_pending = host[kCtrExotic];
+    c.load_refused = host[kCtrLoadDup];
+    c.touched = host[kCtrTouched];
+    c.general_live = host[kCtrGenLive];
+    c.general_tombstones = host[kCtrGenTombs];
+}
+
+// map->counters are those of the device.  The caller holds the map's counter_lock.
+void counters_taken(ash_map* map) {
+    map->counters_known = true;
+    map->unread_inserts = 0;
+    if (map->counters.dropped > 0 || map->counters.tombstones > 0) map->maybe_tombstones = true;
+}
+
+// The words that a call has queued, if they are the latest state, waited for and
+// taken.  The caller holds the map's counter_lock.
+int take_late_words(ash_map* map) {
+    if (!map->late_pending) return 0;
+    if (settle_late_words(map)) return 1;
+    map->late_pending = false;
+    decode_counters(map->line + kLineLate, map->counters);
+    counters_taken(map);
+    return 0;
+}
+
 // The launch before this call leaves the counters at kLineLate with `stamp`: they
 // are the latest state of the counters.  The caller holds the map's counter_lock.
 void late_words_queued(ash_map* map, int32_t stamp, bool of_erase = false) {
@@ -2711,16 +2745,34 @@ int settle_table(ash_map* map, hipStream_t s) {
     return fill_buckets(map, s);
 }
 
-void counters_changed(ash_map* map, bool inserted, hipStream_t s) {
-    if (is_capturing(s)) map->replayed = true;
-    ++map->changes;
-    map->counters_known = false;
-    map->late_pending = false;   // what a queued read-back brings is out of date
-    if (inserted) {
-        ++map->unread_inserts;
-    } else {
-        map->maybe_tombstones = true;
-    }
+Change::Change(ash_map* map, ChangeKind kind, hipStream_t s) : map_(map) {
+    if (kind != kChangeElse && is_capturing(s)) map->replayed = true;
+    std::lock_guard<std::mutex> lock(map->counter_lock);
+    map->changed_on = s;
+    lapse();
+    if (kind == kChangeAdds) ++map->unread_inserts;
+    if (kind == kChangeErases) map->maybe_tombstones = true;
+}
+
+void Change::queued() {
+    if (map_ == nullptr) return;
+    std::lock_guard<std::mutex> lock(map_->counter_lock);
+    lapse();
+    map_ = nullptr;
+}
+
+void Change::queued_with(const ash_counters& c) {
+    std::lock_guard<std::mutex> lock(map_->counter_lock);
+    lapse();
+    map_->counters = c;
+    map_->counters_known = true;
+    map_ = nullptr;
+}
+
+void Change::lapse() {
+    ++map_->changes;
+    map_->counters_known = false;
+    map_->late_pending = false;   // what a queued read-back brings is out of date
 }
 
 int check_batch(const ash_map* map, const void* keys, int64_t n) {
@@ -2932,6 +2984,7 @@ int ash_map_create(int key_dim, int64_t capacity, int32_t* heap, void* table_ws,
     map->unread_inserts = 0;
     map->launches = 0;
     map->changes = 0;
+    map->changed_on = static_cast<hipStream_t>(stream);
     map->replayed = false;
     map->d.ctr = static_cast<int32_t*>(table_ws);
     map->d.buckets = reinterpret_cast<uint64_t*>(static_cast<char*>(table_ws) +
@@ -2968,6 +3021,16 @@ int ash_map_attach_general(ash_map_t* map, void* general_ws,
     DeviceGuard guard;
     ASH_HIP(guard.enter(map->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
+    // (what an insert before leaves for the host is not lost)
+    ash_counters before;
+    bool known;
+    {
+        std::lock_guard<std::mutex> lock(map->counter_lock);
+        if (take_late_words(map)) return 1;
+        before = map->counters;
+        known = map->counters_known;
+    }
+    Change change(map, kChangeElse, s);
     // keys first (16 B per slot, keeps them 16-byte aligned), then states
     map->d.gkeys = static_cast<int32_t*>(general_ws);
     map->d.gstate = map->d.gkeys + slots * 4;
@@ -2978,8 +3041,8 @@ int ash_map_attach_general(ash_map_t* map, void* general_ws,
     ASH_LAUNCH_CHECK();
     set_counter_kernel<<<1, 64, 0, s>>>(map->d.ctr, kCtrExotic, 0);
     ASH_LAUNCH_CHECK();
-    if (map->counters_known) map->counters.exotic_pending = 0;
-    map->late_pending = false;
+    before.exotic_pending = 0;
+    if (known) change.queued_with(before);
     return 0;
 }
 
@@ -3177,7 +3240,7 @@ int launch_activate(ash_map_t* map, const float* cells, int64_t n, int grid_dim,
                     int dilation, int bidirectional, int bound_lo, int bound_hi,
                     uint8_t* touched, int32_t* coords, int32_t* heads, hipStream_t s) {
     if (settle_table(map, s)) return 1;
-    counters_changed(map, true, s);
+    Change change(map, kChangeAdds, s);
     const int lo = bidirectional ? -dilation : 0;
     const int width = dilation - lo + 1;
     const float g = static_cast<float>(grid_dim);
@@ -3271,7 +3334,7 @@ int ash_grid_activate_positions(ash_map_t* map, const float* positions, int64_t 
     ASH_HIP(guard.enter(map->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (settle_table(map, s)) return 1;
-    counters_changed(map, true, s);
+    Change change(map, kChangeAdds, s);
     RunsArgs a;
     a.x = positions;
     a.origin = origin;
@@ -3394,7 +3457,7 @@ int insert_per_key(ash_map* map, const int32_t* keys, int64_t n, int n_values,
     ASH_HIP(guard.enter(map->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (settle_table(map, s)) return 1;
-    counters_changed(map, true, s);
+    Change change(map, kChangeAdds, s);
     ValueArgs va = {};
     if (n_values == 0) return launch_insert<kInsertKeys>(map, keys, n, va, nullptr, nullptr, s, publish, check);
     if (!ash_map_insert_needs_scratch(n_values, row_bytes)) {
@@ -3437,7 +3500,7 @@ int ash_map_erase(ash_map_t* map, const int32_t* keys, int64_t n,
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (settle_table(map, s)) return 1;
     if (give_up_heap_order(map, s)) return 1;   // freed indices go back onto the heap
-    counters_changed(map, false, s);
+    Change change(map, kChangeErases, s);
     // Nobody waits here; but a size, a listing or an insert that follows wants the
     // counters, and finds them with a launch less.  (Not where the words of an
     // earlier call are still owed: a run of erases is not to wait for each other.)
@@ -3454,13 +3517,8 @@ int ash_map_erase(ash_map_t* map, const int32_t* keys, int64_t n,
                                       : erase_kernel<4>;
     kernel<<<g, kEraseBlock, 0, s>>>(map->d, keys, n, publish);
     ASH_LAUNCH_CHECK();
-    if (late.taken()) {
-        late.queued(true);
-    } else {
-        std::lock_guard<std::mutex> lock(map->counter_lock);
-        map->counters_known = false;
-        ++map->changes;
-    }
+    change.queued();
+    if (late.taken()) late.queued(true);
     return 0;
 }
 
@@ -3483,6 +3541,7 @@ int ash_map_clear_rows(ash_map_t* map, int n_values, void* const* rows, const in
     ASH_HIP(guard.enter(map->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (is_capturing(s)) map->replayed = true;
+    Change change(map, kChangeElse, s);
     if (map->replayed) {
         // what replays leave behind is unknown: everything is cleared now
         if (settle_table(map, s)) return 1;
@@ -3496,9 +3555,7 @@ int ash_map_clear_rows(ash_map_t* map, int n_values, void* const* rows, const in
         return 1;
     }
     // every counter is zero again: known without a read-back
-    map->counters_known = true;
-    map->counters = {};
-    map->late_pending = false;
+    change.queued_with({});
     map->maybe_tombstones = false;
     map->unread_inserts = 0;
     return 0;
@@ -3506,76 +3563,46 @@ int ash_map_clear_rows(ash_map_t* map, int n_values, void* const* rows, const in
 
 namespace {
 
-void decode_counters(const uint64_t* words, ash_counters& c) {
-    int32_t host[kHostCounters];
-    for (int w = 0; w < kHostCounters; ++w) host[w] = value_of(words[w]);
-    c.size = host[kCtrSize];
-    c.dropped = host[kCtrDropped];
-    c.tombstones = host[kCtrTombs];
-    c.exotic_pending = host[kCtrExotic];
-    c.load_refused = host[kCtrLoadDup];
-    c.touched = host[kCtrTouched];
-    c.general_live = host[kCtrGenLive];
-    c.general_tombstones = host[kCtrGenTombs];
-}
+// Who wants the counters: the call that changes the map, which is ordered behind all
+// that have changed it; a reader, who may be another thread with a stream of its own;
+// a reader who has the device asked in any case.
+enum Asker { kOwnCall, kReader, kReaderOfDevice };
 
-// map->counters are those of the device.  The caller holds the map's counter_lock.
-void counters_taken(ash_map* map) {
-    map->counters_known = true;
-    map->unread_inserts = 0;
-    if (map->counters.dropped > 0 || map->counters.tombstones > 0) map->maybe_tombstones = true;
-}
-
-// The words that a call has queued, if they are the latest state, waited for and
-// taken.  The caller holds the map's counter_lock.
-int take_late_words(ash_map* map) {
-    if (!map->late_pending) return 0;
-    if (settle_late_words(map)) return 1;
-    map->late_pending = false;
-    decode_counters(map->line + kLineLate, map->counters);
-    counters_taken(map);
-    return 0;
-}
-
-// Brings map->counters up to date (the map's device is current): they are
-// known already, or a read-back queued behind the latest insert brings them,
-// or they are fetched now, which waits for `s`.  `ask`: fetched in any case,
-// behind words that are under way (they belong to a call that has returned);
-// what is fetched beside counters that are known is the asker's alone.
-// `copy`: a copy of them, for callers whose map other threads may read as well.
-int refresh_counters(ash_map* map, hipStream_t s, bool ask = false, ash_counters* copy = nullptr) {
+// The counters (the map's device is current): they are known already, or a read-back
+// queued behind the latest insert brings them, or they are fetched now, which waits for
+// `s`.  A reader of the device, too, asks behind words that are under way: they belong
+// to a call that has returned.  What a reader has fetched is the latest state only if
+// it was asked for on the stream of the latest change, behind that, and none has begun
+// or been queued since; else it is the reader's alone.
+int refresh_counters(ash_map* map, hipStream_t s, Asker asker, ash_counters& c) {
     std::unique_lock<std::mutex> lock(map->counter_lock);
     if (map->replayed) {
         if (settle_late_words(map)) return 1;
         map->counters_known = map->late_pending = false;
     }
     if (take_late_words(map)) return 1;
-    if (ask || !map->counters_known) {
-        if (is_capturing(s)) {
-            ASH_FAIL("the table's counters cannot be read while the stream is being captured");
-        }
-        // (each of several readers waits for its own stream, not for the others)
-        const uint32_t changes = map->changes;
-        lock.unlock();
-        Answer answer;
-        if (answer.take()) return 1;
-        publish_counters_kernel<<<1, 64, 0, s>>>(map->d.ctr, answer.words, answer.stamp);
-        ASH_LAUNCH_CHECK();
-        if (answer.wait(s, kHostCounters)) return 1;
-        lock.lock();
-        if (copy != nullptr) {
-            decode_counters(answer.words, *copy);
-            // (a call of another thread may have changed them since)
-            if (map->changes == changes && !map->counters_known) {
-                map->counters = *copy;
-                counters_taken(map);
-            }
-            return 0;
-        }
-        decode_counters(answer.words, map->counters);
+    if (map->counters_known && asker != kReaderOfDevice) {
+        c = map->counters;
+        return 0;
+    }
+    if (is_capturing(s)) {
+        ASH_FAIL("the table's counters cannot be read while the stream is being captured");
+    }
+    // (each of several readers waits for its own stream, not for the others)
+    const uint32_t changes = map->changes;
+    lock.unlock();
+    Answer answer;
+    if (answer.take()) return 1;
+    publish_counters_kernel<<<1, 64, 0, s>>>(map->d.ctr, answer.words, answer.stamp);
+    ASH_LAUNCH_CHECK();
+    if (answer.wait(s, kHostCounters)) return 1;
+    decode_counters(answer.words, c);
+    lock.lock();
+    if (asker == kOwnCall ||
+        (map->changes == changes && s == map->changed_on && !map->counters_known)) {
+        map->counters = c;
         counters_taken(map);
     }
-    if (copy != nullptr) *copy = map->counters;
     return 0;
 }
 
@@ -3609,11 +3636,14 @@ bool should_rebuild(const ash_map* map, int64_t size, int64_t tombstones, int64_
 // emptied table when too few empty slots would remain.
 int upkeep(ash_map* map, int64_t incoming, void* scratch, int64_t scratch_bytes,
            hipStream_t s) {
-    if (map->late_pending && refresh_counters(map, s)) return 1;
+    {
+        std::lock_guard<std::mutex> lock(map->counter_lock);
+        if (take_late_words(map)) return 1;
+    }
     if (map->unread_inserts >= kUpkeepEvery || map->replayed) map->maybe_tombstones = true;
     if (!map->maybe_tombstones) return 0;
-    if (refresh_counters(map, s)) return 1;
-    const ash_counters& c = map->counters;
+    ash_counters c;
+    if (refresh_counters(map, s, kOwnCall, c)) return 1;
     map->maybe_tombstones = c.tombstones > 0;
     if (!should_rebuild(map, c.size, c.tombstones, incoming,
                         c.general_live + c.general_tombstones, c.general_tombstones)) {
@@ -3637,9 +3667,11 @@ int upkeep(ash_map* map, int64_t incoming, void* scratch, int64_t scratch_bytes,
                 ((map->capacity * map->key_dim * 4 + 255) & ~int64_t{255}));
     }
     if (ash_map_rebuild(map, keys, indices, c.size, s)) return 1;
-    map->counters.tombstones = 0;
-    map->counters_known = true;
     map->maybe_tombstones = false;
+    c.tombstones = 0;
+    std::lock_guard<std::mutex> lock(map->counter_lock);
+    map->counters = c;
+    map->counters_known = true;
     return 0;
 }
 
@@ -3665,7 +3697,6 @@ int ash::queue_touched_count(ash_map* map, const uint8_t* touched, int64_t rows,
                 map->d.ctr, counts, static_cast<int>(groups), landing, stamp);
         ASH_LAUNCH_CHECK();
     }
-    map->counters_known = false;
     late_words_queued(map, stamp);
     return 0;
 }
@@ -3684,7 +3715,7 @@ int ash_map_counters(ash_map_t* map, int32_t* staging, int64_t out[7], void* str
     DeviceGuard guard;
     ASH_HIP(guard.enter(map->device));
     ash_counters c;
-    if (refresh_counters(map, static_cast<hipStream_t>(stream), false, &c)) return 1;
+    if (refresh_counters(map, static_cast<hipStream_t>(stream), kReader, c)) return 1;
     out[0] = c.size;
     out[1] = c.dropped;
     out[2] = c.tombstones;
@@ -3725,7 +3756,7 @@ int ash_map_status(ash_map_t* map, int64_t out[5], void* stream) {
     ASH_HIP(guard.enter(map->device));
     // always a copy from the device
     ash_counters c;
-    if (refresh_counters(map, static_cast<hipStream_t>(stream), true, &c)) return 1;
+    if (refresh_counters(map, static_cast<hipStream_t>(stream), kReaderOfDevice, c)) return 1;
     out[0] = c.size;
     out[1] = c.dropped;
     out[2] = c.tombstones;
@@ -3894,15 +3925,18 @@ int ash_map_insert_auto(ash_map_t* map, const int32_t* keys, int64_t n, int n_va
             if (value_of(answer.words[0]) == 0) return 0;
         }
     }
-    if (refresh_counters(map, s)) return 1;
-    if (map->counters.exotic_pending > 0 && map->general_attached) {
+    ash_counters c;
+    if (refresh_counters(map, s, kOwnCall, c)) return 1;
+    if (c.exotic_pending > 0 && map->general_attached) {
+        Change change(map, kChangeElse, s);
         fold_waiting_keys_kernel<<<1, 64, 0, s>>>(map->d.ctr);
         ASH_LAUNCH_CHECK();
-        map->counters.dropped += map->counters.exotic_pending;
-        map->counters.exotic_pending = 0;
+        c.dropped += c.exotic_pending;
+        c.exotic_pending = 0;
+        change.queued_with(c);
         map->maybe_tombstones = true;
     }
-    if (map->counters.exotic_pending > 0) {
+    if (c.exotic_pending > 0) {
         set_error("keys that do not fit the packed code are waiting for the second region: "
                   "attach it (ash_map_attach_general) and issue the insert again");
         return ASH_NEEDS_GENERAL;
@@ -3952,8 +3986,7 @@ int ash_grid_collect_touched(ash_map_t* map, uint8_t* touched, const int32_t* bl
     if (groups > kCollectGroups) groups = kCollectGroups;
     const int words = static_cast<int>((map->capacity + groups * per_group - 1) / (groups * per_group));
     groups = (map->capacity + words * per_group - 1) / (words * per_group);   // no empty chunks
-    map->counters_known = false;   // the number of listed rows is one of them
-    map->late_pending = false;
+    Change change(map, kChangeElse, static_cast<hipStream_t>(stream));   // the number of listed rows is a counter
     collect_touched_kernel<<<static_cast<unsigned>(groups), kCollectThreads, 0,
                              static_cast<hipStream_t>(stream)>>>(
             touched, block_coords, map->capacity, words, out_indices, out_coords, map->d.ctr);
@@ -3993,9 +4026,8 @@ int ash_map_items_rows(ash_map_t* map, int32_t* keys_out, int64_t* indices_out, 
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (settle_table(map, s)) return 1;
     const int identity = heap_in_order(map) ? 1 : 0;
-    const bool none_in_general = !map->general_attached ||
-                                 (map->counters_known && map->counters.general_live == 0);
-    if (lists_in_index_order(map)) {
+    const bool all_in_log = none_in_general(map);
+    if (identity && all_in_log) {
         const int64_t n = n_expected < map->capacity ? n_expected : map->capacity;
         const unsigned gd = grid_for(n);
         switch (map->key_dim) {
@@ -4018,26 +4050,26 @@ int ash_map_items_rows(ash_map_t* map, int32_t* keys_out, int64_t* indices_out, 
     // Rows go along with the entries that the log lists, up to the width at which a
     // lane copies one word after the other; entries of the second region are not
     // listed there.
-    bool along = none_in_general;
+    bool along = all_in_log;
     for (int v = 0; v < n_values; ++v) along = along && rows.row_dwords[v] <= kMaxFusedRowDwords;
     if (!along) rows.n = 0;
     const int slot = next_slot(map);
     switch (map->key_dim) {
         case 1:
-            launch_items<1>(map, keys_out, indices_out, n_expected, identity, rows, slot, none_in_general, s);
+            launch_items<1>(map, keys_out, indices_out, n_expected, identity, rows, slot, all_in_log, s);
             break;
         case 2:
-            launch_items<2>(map, keys_out, indices_out, n_expected, identity, rows, slot, none_in_general, s);
+            launch_items<2>(map, keys_out, indices_out, n_expected, identity, rows, slot, all_in_log, s);
             break;
         case 3:
-            launch_items<3>(map, keys_out, indices_out, n_expected, identity, rows, slot, none_in_general, s);
+            launch_items<3>(map, keys_out, indices_out, n_expected, identity, rows, slot, all_in_log, s);
             break;
         default:
-            launch_items<4>(map, keys_out, indices_out, n_expected, identity, rows, slot, none_in_general, s);
+            launch_items<4>(map, keys_out, indices_out, n_expected, identity, rows, slot, all_in_log, s);
             break;
     }
     ASH_LAUNCH_CHECK();
-    if (!none_in_general) {
+    if (!all_in_log) {
         const unsigned gg = grid_for(map->d.gslots);
         int32_t* cursor = map->d.ctr + kCtrCursors + 2 * slot;   // its lower half
         auto kernel = map->key_dim == 1   ? items_general_kernel<1>
@@ -4080,6 +4112,7 @@ int ash_map_rebuild(ash_map_t* map, int32_t* keys_scratch,
     DeviceGuard guard;
     ASH_HIP(guard.enter(map->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
+    Change change(map, kChangeElse, s);
     if (fill_buckets(map, s)) return 1;
     if (map->general_attached) {
         const int64_t g16 = static_cast<int64_t>(map->d.gslots) / 4;
@@ -4093,8 +4126,6 @@ int ash_map_rebuild(ash_map_t* map, int32_t* keys_scratch,
     }
     set_counter_kernel<<<1, 64, 0, s>>>(map->d.ctr, kCtrTombs, 0);
     ASH_LAUNCH_CHECK();
-    map->counters_known = false;
-    map->late_pending = false;
     if (n == 0) return 0;
     if (from_log) {
         int64_t g = (map->capacity + kHeapBlock - 1) / kHeapBlock;
@@ -4126,7 +4157,7 @@ int ash_map_neighbors(ash_map_t* map, int64_t num_rows, int radius, int bidirect
     if (settle_table(map, s)) return 1;
     neighbors_kernel<<<grid_for(num_rows * each), kBlock, 0, s>>>(map->d, a, heap_in_order(map) ? 1 : 0);
     ASH_LAUNCH_CHECK();
-    if (map->general_attached && !(map->counters_known && map->counters.general_live == 0)) {
+    if (!none_in_general(map)) {
         neighbors_general_kernel<<<looping_grid(map->d.gslots * each), kBlock, 0, s>>>(map->d, a);
         ASH_LAUNCH_CHECK();
     }
@@ -4149,10 +4180,9 @@ int ash_map_load(ash_map_t* map, const int32_t* keys, const int64_t* indices,
     ASH_HIP(guard.enter(map->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (is_capturing(s)) ASH_FAIL("ash_map_load cannot be captured into a graph");
+    Change change(map, kChangeElse, s);
     if (clear_table(map, s, false, static_cast<int32_t>(n))) return 1;
     map->heap_dirty = true;   // the heap is the caller's from here on
-    map->counters_known = false;
-    map->late_pending = false;
     map->maybe_tombstones = false;
     map->unread_inserts = 0;
     if (heap_src != nullptr && heap_src != map->d.heap) {

@@ -170,11 +170,30 @@ inline int next_slot(ash_map* map) { return static_cast<int>(map->launches.fetch
 // Whether the heap array is known to be 0, 1, 2, ...
 inline bool heap_in_order(const ash_map* map) { return !map->heap_dirty && !map->replayed; }
 
-// What the host keeps of the counters no longer holds: `inserted` for a call
-// that may have added entries (and ended without a look at the counters),
-// false for one that took entries away.
-// `s`: the stream the call runs on (captured: see ash_map::replayed).
-void counters_changed(ash_map* map, bool inserted, hipStream_t s);
+// A call that changes the counters, from before its first launch until its last is
+// queued (at the latest when it is left): at both ends what the host keeps of them
+// lapses, since what a reader has asked for in between may be from before.
+enum ChangeKind {
+    kChangeAdds,     // may have added entries (and ends without a look at the counters)
+    kChangeErases,   // may have left tombstones
+    kChangeElse
+};
+
+class Change {
+  public:
+    // `s`: the stream the call runs on (where one that adds or erases is captured, see
+    // ash_map::replayed)
+    Change(ash_map* map, ChangeKind kind, hipStream_t s);
+    Change(const Change&) = delete;
+    Change& operator=(const Change&) = delete;
+    ~Change() { queued(); }
+    void queued();
+    void queued_with(const ash_counters& c);   // ... and has left the counters at `c`
+
+  private:
+    void lapse();   // the caller holds the map's counter_lock
+    ash_map* map_;
+};
 // Leaves `value` for the host in a word of its line (kLineWords).
 __device__ __forceinline__ void leave_word(uint64_t* word, int32_t value, int32_t stamp) {
     __hip_atomic_store(word, static_cast<uint64_t>(static_cast<uint32_t>(value)) |

@@ -411,8 +411,8 @@ int ash_map_erase_bulk(ash_map_t* map, const int32_t* keys, int64_t n, void* wor
  *      enough relative to the table, else the per-key kernel, with `scratch` as
  *      the workspace of either (`policy` overrides the choice);
  *   3. it reads the counters, or -- streaming path, no key of the batch handed to
- *      the per-key kernel; per-key kernel under ASH_STREAMING_EARLY, no key that
- *      waits for the second region -- queues their read-back behind the insert and
+ *      the per-key kernel; per-key kernel under ASH_STREAMING_EARLY, no key for
+ *      the second region -- queues their read-back behind the insert and
  *      returns without waiting for it (ash_map_counters picks it up).
  * Returns ASH_NEEDS_GENERAL (and inserts everything else) when keys of the
  * batch do not fit the packed code and no second region is attached: attach

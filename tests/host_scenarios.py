@@ -2,7 +2,7 @@
 function a test of test_host_counters.py (each in a process of its own)."""
 import time
 
-from stand_in_device import ALWAYS, EXOTIC, SIZE, TOMBS, Map, beside
+from stand_in_device import ALWAYS, DROPPED, EXOTIC, SIZE, TOMBS, Map, beside
 
 ONE, OTHER = 0x10, 0x20   # streams
 
@@ -134,3 +134,16 @@ def words_under_way_when_the_second_region_comes(device):
     attached.join(), seen.join()
     assert (attached.result, seen.result) == (0, 100)
     _stands_at(m, 100)
+
+
+def keys_that_the_second_region_refuses(device):
+    """A batch with keys for the second region: the region may be full while the table
+    is not, so the counters have been read when the insert returns."""
+    m = Map(device)
+    assert m.attach() == 0
+    device.bad_keys, device.effects = 3, [{SIZE: 80, DROPPED: 20}]
+    assert m.insert() == 0 and not m.pending()
+    assert m.counters()[:2] == [80, 20]
+    device.bad_keys, device.effects = 0, [{SIZE: 100}]
+    assert m.insert() == 0 and m.pending()
+    assert m.counters()[:2] == [180, 20]

@@ -153,6 +153,24 @@ def test_inserts_in_a_row_while_others_ask_for_the_size(ash):
     assert all(6 * 3_001 <= n <= 6 * 3_001 + 40 * 1_500 for n in seen)
 
 
+def test_keys_that_a_full_second_region_refuses_are_reported(ash):
+    """A region attached just in case holds 65 536 keys, the table many more."""
+    engine = ash.ASHEngine(3, 200_000, DEV)
+    engine.insert_keys(_keys(0, 1_000))
+    engine.size()
+    engine.backend._attach_general(just_in_case=True)
+    with warnings.catch_warnings(record=True) as seen:
+        warnings.simplefilter("always")
+        engine.insert_keys(_keys(0, 66_000) + (1 << 24))
+    assert any("464 keys were not stored" in str(w.message) for w in seen)
+    _agree(engine, 66_536)
+    with warnings.catch_warnings(record=True) as seen:
+        warnings.simplefilter("always")
+        engine.insert_keys(_keys(1_000, 50_000))   # none for the region, which is as full
+    assert not seen
+    _agree(engine, 116_536)
+
+
 def test_status_asked_for_beside_an_insert_under_way(ash):
     """A reader of the device on a stream of its own sees the insert that has returned
     before it asks, and what the insert leaves for the host stays there for others.

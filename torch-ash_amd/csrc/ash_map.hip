@@ -628,8 +628,9 @@ __device__ __forceinline__ void leave_with_last(const MapDev& m, const Publish& 
     if (s_last) leave_counters(m.ctr, publish.landing, publish.stamp);
 }
 
-// What the host waits for before it returns from an insert, where there is no second
-// region: whether every key fits the packed code.  The first `groups` workgroups of
+// What the host waits for before it returns from an insert: whether every key fits the
+// packed code.  (One that does not wants the second region attached, or may find that
+// full while the table is not: the counters are read then.)  The first `groups` workgroups of
 // the launch (none: nobody waits) look at all keys and at nothing else, and the last
 // of them leaves the number of workgroups that have met one that does not fit.  That
 // is there as soon as the launch has begun, and what follows the insert is queued
@@ -3870,9 +3871,10 @@ int ash_map_insert_auto(ash_map_t* map, const int32_t* keys, int64_t n, int n_va
         }
     } else {
         // The counters come behind the insert (a short launch leaves them itself) and
-        // wait for the call that asks for them; only keys that may be waiting for the
-        // second region are waited for here.  (Under the other policies callers find
-        // the counters read.  Replays change them behind the host's back: read, too.)
+        // wait for the call that asks for them; only a batch with keys for the second
+        // region, which may be missing or full, is waited for here.  (Under the other
+        // policies callers find the counters read.  Replays change them behind the
+        // host's back: read, too.)
         if (capturing || map->replayed || policy != ASH_STREAMING_EARLY) {
             // (short launches leave what is waited for below themselves)
             Answer answer;
@@ -3897,7 +3899,7 @@ int ash_map_insert_auto(ash_map_t* map, const int32_t* keys, int64_t n, int n_va
         } else {
             Answer answer;
             KeyCheck check = {};
-            if (map->key_dim > 1 && !map->general_attached) {
+            if (map->key_dim > 1) {
                 if (answer.take()) return 1;
                 const int64_t groups = (n + kCheckKeys * kHeapBlock - 1) / (kCheckKeys * kHeapBlock);
                 check = {static_cast<unsigned>(std::min<int64_t>(groups, kMostChecks)), answer.words,

@@ -147,3 +147,48 @@ def keys_that_the_second_region_refuses(device):
     device.bad_keys, device.effects = 0, [{SIZE: 100}]
     assert m.insert() == 0 and m.pending()
     assert m.counters()[:2] == [180, 20]
+
+
+def _lines(device, stream):
+    return {word // 128 for on, word in device.words if on == stream}
+
+
+def a_streaming_insert_that_fails_behind_its_first_launch(device):
+    """(the word of its first pass is owed)"""
+    m = Map(device)
+    device.stream(ONE).hold()
+    device.refuse = ("build_kernel",)
+    assert m.insert(70_000, ALWAYS, ONE) == 1
+    device.refuse = ()
+    device.effects = [{SIZE: 70_000}]
+    assert m.insert(70_000, ALWAYS, OTHER) == 0
+    assert not _lines(device, ONE) & _lines(device, OTHER)
+    device.stream(ONE).go()
+    assert m.size(OTHER) == 70_000
+
+
+def a_map_that_goes_with_words_owed(device):
+    """The line of a failed call serves no other map."""
+    m = Map(device, key_dim=1)
+    device.stream(ONE).hold()
+    device.refuse = ("scatter_rows_kernel",)
+    assert m.insert(stream=ONE, values=1, row_bytes=4096) == 1
+    device.refuse = ()
+    assert m.lib.ash_map_destroy(m.handle) == 0
+    others = [Map(device, key_dim=1) for _ in range(3)]
+    for other in others:
+        assert other.insert(stream=OTHER) == 0
+    assert not _lines(device, ONE) & _lines(device, OTHER)
+    device.stream(ONE).go()
+
+
+def inserts_that_are_refused_before_their_launch(device):
+    """They owe nothing: their lines serve the next call."""
+    m = Map(device)
+    for _ in range(3):
+        assert m.insert() == 0
+    used = _lines(device, 0)
+    for _ in range(100):
+        assert m.insert(values=1, row_bytes=0) == 1   # (no value rows)
+        assert m.insert() == 0
+    assert _lines(device, 0) == used

@@ -50,6 +50,7 @@ class Device:
         self.runtime = ctypes.CDLL(stand_in, mode=ctypes.RTLD_GLOBAL)
         self.streams = {}
         self.launched = []        # names
+        self.words = []           # (stream, address) of words that launches are to leave
         self.refuse = ()          # parts of the names of kernels whose launch fails
         self.before = {}          # part of a kernel's name -> called (once) where it is launched
         self.no_host_memory = False
@@ -82,7 +83,7 @@ class Device:
     def _arg(self, args, k, layout):
         return struct.unpack(layout, ctypes.string_at(args[k], struct.calcsize(layout)))
 
-    def _work(self, name, args):
+    def _work(self, name, args, stream):
         """What the launch does, with its arguments as they are now."""
         arg = lambda k, layout: self._arg(args, k, layout)
         if "publish_counters_kernel" in name:
@@ -125,6 +126,9 @@ class Device:
         if "count_flags_kernel" in name:
             count = arg(4, "<Q") + arg(5, "<i")
 
+        owed = [publish and publish[0], early and early[0], count and count[0], check and check[0] and check[2]]
+        self.words += [(stream, word) for word in owed if word]
+
         def work():
             if check is not None and check[0]:
                 self._leave(check[2], check[3], [self.bad_keys])
@@ -148,7 +152,7 @@ class Device:
                 return 98
             self.launched.append(name)
             queue = self.stream(stream)
-            work = self._work(name, args)
+            work = self._work(name, args, stream)
             if queue.held:
                 queue.queue.append(work)
             else:

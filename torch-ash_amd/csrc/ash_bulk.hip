@@ -1560,20 +1560,6 @@ __global__ __launch_bounds__(kListThreads) void settle_rows_kernel(
     }
 }
 
-int check_values(int n_values, const void* const* src, void* const* dst,
-                 const int64_t* row_bytes) {
-    if (n_values < 0) ASH_FAIL("negative value count");
-    if (n_values == 0) return 0;
-    if (src == nullptr || dst == nullptr || row_bytes == nullptr) {
-        ASH_FAIL("null value tables");
-    }
-    for (int v = 0; v < n_values; ++v) {
-        if (src[v] == nullptr || dst[v] == nullptr) ASH_FAIL("null value tensor");
-        if (row_bytes[v] <= 0) ASH_FAIL("value rows must not be empty");
-    }
-    return 0;
-}
-
 template <bool PROV>
 int launch_split_once(ash_map* map, BulkPlan pl, const int32_t* keys, int identity,
                       uint64_t* early, int32_t stamp, hipStream_t s) {
@@ -1733,7 +1719,7 @@ int ash::insert_bulk(ash_map* map, const int32_t* keys, int64_t n,
                      int64_t workspace_bytes, uint64_t* early, uint64_t* late, int32_t stamp,
                      bool* published, void* stream) {
     if (check_batch(map, keys, n)) return 1;
-    if (check_values(n_values, src, dst, row_bytes)) return 1;
+    if (check_rows(n_values, src, dst, row_bytes)) return 1;
     if (workspace == nullptr) ASH_FAIL("null bulk workspace");
     if (reinterpret_cast<uintptr_t>(workspace) % 256 != 0) {
         ASH_FAIL("bulk workspace must be 256-byte aligned");

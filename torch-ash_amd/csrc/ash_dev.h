@@ -171,7 +171,7 @@ struct ash_map {
     uint64_t* line;         // page-locked words of the map's own (take_line), made on first use
     int32_t stamp;          // of the latest words asked for there
     int32_t late_stamp;
-    bool late_in_flight;    // the device may still owe the words at kLineLate
+    bool late_in_flight;    // the device may still owe the words at kLineLate (under late_stamp)
     bool late_pending;      // ... and it is the latest state of the counters: nobody has looked at it yet
     bool late_of_erase;     // ... left by an erase
     bool counters_known;    // `counters` is what the device holds

@@ -2522,51 +2522,50 @@ int take_late_words(ash_map* map) {
     return 0;
 }
 
-// The launch before this call leaves the counters at kLineLate with `stamp`: they
-// are the latest state of the counters.  The caller holds the map's counter_lock.
-void late_words_queued(ash_map* map, int32_t stamp, bool of_erase = false) {
-    map->late_stamp = stamp;
-    map->late_in_flight = map->late_pending = true;
-    map->late_of_erase = of_erase;
-    // (a reader may have asked the device before the launch was queued)
-    map->counters_known = false;
-    ++map->changes;
-}
-
-// The landing place at kLineLate, of one call from `take` on: a call of another thread
-// waits for its words (or does without) before it has others left there.
+// The map's own words, for the call that changes the map (there is one at a time): what
+// earlier calls owe there has come when they are taken.  A call that ends between its
+// launches and `queued` or `unused` may owe words itself: the line is given up then
+// (128 bytes), and the next call takes another.
 class LatePlace {
   public:
     explicit LatePlace(ash_map* map) : map_(map) {}
-    ~LatePlace() {   // (nothing has been launched)
+    LatePlace(const LatePlace&) = delete;
+    LatePlace& operator=(const LatePlace&) = delete;
+    ~LatePlace() {
         if (!taken_) return;
         std::lock_guard<std::mutex> lock(map_->counter_lock);
-        if (map_->late_stamp == stamp) map_->late_in_flight = false;
+        map_->line = nullptr;
+        map_->late_in_flight = map_->late_pending = false;
     }
     // `settle`: words that are owed are waited for; else the place may not be had.
     int take(bool settle) {
         if (take_line(map_)) return 1;
         std::lock_guard<std::mutex> lock(map_->counter_lock);
-        if (settle) {
-            if (settle_late_words(map_)) return 1;
-        } else if (map_->late_in_flight && !all_come(map_->line + kLineLate, kHostCounters, map_->late_stamp)) {
+        if (!settle && map_->late_in_flight &&
+            !all_come(map_->line + kLineLate, kHostCounters, map_->late_stamp)) {
             return 0;
         }
+        if (take_late_words(map_) || settle_late_words(map_)) return 1;
         stamp = map_->stamp = next_stamp(map_->stamp);
-        map_->late_stamp = stamp;
-        map_->late_in_flight = taken_ = true;
-        map_->late_pending = false;
+        taken_ = true;
         return 0;
     }
     bool taken() const { return taken_; }
-    // The launch that leaves the words is queued: they are the latest state of the
-    // counters, unless another thread's call has changed them since.
-    void queued(bool of_erase) {
+    uint64_t* late() const { return map_->line + kLineLate; }
+    uint64_t* early() const { return map_->line + kLineEarly; }
+    // The launch that leaves the counters at `late` under `stamp` is queued, the last
+    // of its Change: they are the latest state.
+    void queued(bool of_erase = false) {
         std::lock_guard<std::mutex> lock(map_->counter_lock);
         taken_ = false;
+        map_->late_stamp = stamp;
+        map_->late_in_flight = map_->late_pending = true;
+        map_->late_of_erase = of_erase;
+        map_->counters_known = false;   // (a reader may have asked the device since)
         if (!of_erase) map_->unread_inserts = 0;
-        if (map_->late_stamp == stamp) late_words_queued(map_, stamp, of_erase);
     }
+    // No launch leaves words any more.
+    void unused() { taken_ = false; }
     int32_t stamp = 0;
 
   private:
@@ -2575,11 +2574,6 @@ class LatePlace {
 };
 
 }  // namespace
-
-int settle_landing_place(ash_map* map) {
-    std::lock_guard<std::mutex> lock(map->counter_lock);
-    return settle_late_words(map);
-}
 
 namespace {
 
@@ -2781,6 +2775,18 @@ int check_batch(const ash_map* map, const void* keys, int64_t n) {
     if (n < 0) ASH_FAIL("negative key count");
     if (n > 0 && keys == nullptr) ASH_FAIL("null keys pointer");
     if (n > (int64_t{1} << 31) - kHeapBlock) ASH_FAIL("too many keys in one call");
+    return 0;
+}
+
+int check_rows(int n_values, const void* const* src, void* const* dst, const int64_t* row_bytes) {
+    if (n_values < 0) ASH_FAIL("negative value count");
+    if (n_values > 0 && (src == nullptr || dst == nullptr || row_bytes == nullptr)) {
+        ASH_FAIL("null value tables");
+    }
+    for (int v = 0; v < n_values; ++v) {
+        if (src[v] == nullptr || dst[v] == nullptr) ASH_FAIL("null value tensor");
+        if (row_bytes[v] <= 0) ASH_FAIL("value rows must not be empty");
+    }
     return 0;
 }
 
@@ -3054,7 +3060,8 @@ int ash_map_destroy(ash_map_t* map) {
     if (map->late_in_flight) {
         DeviceGuard guard;
         (void)guard.enter(map->device);
-        (void)settle_landing_place(map);
+        std::lock_guard<std::mutex> lock(map->counter_lock);
+        (void)settle_late_words(map);
     }
     if (!map->late_in_flight) give_back_line(map->line);
     delete map;
@@ -3444,15 +3451,7 @@ int insert_per_key(ash_map* map, const int32_t* keys, int64_t n, int n_values,
                    const void* const* src, void* const* dst, const int64_t* row_bytes,
                    int32_t* assigned, void* stream, const Publish& publish,
                    const KeyCheck& check) {
-    if (check_batch(map, keys, n)) return 1;
-    if (n_values < 0) ASH_FAIL("negative value count");
-    if (n_values > 0 && (src == nullptr || dst == nullptr || row_bytes == nullptr)) {
-        ASH_FAIL("null value tables");
-    }
-    for (int v = 0; v < n_values; ++v) {
-        if (src[v] == nullptr || dst[v] == nullptr) ASH_FAIL("null value tensor");
-        if (row_bytes[v] <= 0) ASH_FAIL("value rows must not be empty");
-    }
+    if (check_batch(map, keys, n) || check_rows(n_values, src, dst, row_bytes)) return 1;
     if (n == 0) return 0;
     DeviceGuard guard;
     ASH_HIP(guard.enter(map->device));
@@ -3509,7 +3508,7 @@ int ash_map_erase(ash_map_t* map, const int32_t* keys, int64_t n,
     LatePlace late(map);
     if (n <= kLeaveKeys && !map->replayed && !is_capturing(s)) {
         if (late.take(false)) return 1;
-        if (late.taken()) publish = {map->line + kLineLate, late.stamp, next_ticket(map)};
+        if (late.taken()) publish = {late.late(), late.stamp, next_ticket(map)};
     }
     const unsigned g = grid_for(n, kEraseBlock);
     auto kernel = map->key_dim == 1   ? erase_kernel<1>
@@ -3682,23 +3681,22 @@ int upkeep(ash_map* map, int64_t incoming, void* scratch, int64_t scratch_bytes,
 
 int ash::queue_touched_count(ash_map* map, const uint8_t* touched, int64_t rows, int32_t* counts,
                              int max_counts, hipStream_t s) {
-    if (take_line(map)) return 1;
-    std::lock_guard<std::mutex> lock(map->counter_lock);
-    if (settle_late_words(map)) return 1;
-    const int32_t stamp = map->stamp = next_stamp(map->stamp);
-    uint64_t* const landing = map->line + kLineLate;
+    LatePlace late(map);
+    if (late.take(true)) return 1;
     int64_t groups = (rows + kCountFlags - 1) / kCountFlags;
     if (groups > max_counts) groups = max_counts;
     if (groups < 1) groups = 1;
+    Change change(map, kChangeElse, s);
     count_flags_kernel<<<static_cast<unsigned>(groups), kCollectThreads, 0, s>>>(
-            touched, rows, counts, map->d.ctr, landing, stamp);
+            touched, rows, counts, map->d.ctr, late.late(), late.stamp);
     ASH_LAUNCH_CHECK();
     if (groups > 1) {
         publish_touched_kernel<<<1, kCollectThreads, 0, s>>>(
-                map->d.ctr, counts, static_cast<int>(groups), landing, stamp);
+                map->d.ctr, counts, static_cast<int>(groups), late.late(), late.stamp);
         ASH_LAUNCH_CHECK();
     }
-    late_words_queued(map, stamp);
+    change.queued();
+    late.queued();
     return 0;
 }
 
@@ -3838,6 +3836,7 @@ int ash_map_insert_auto(ash_map_t* map, const int32_t* keys, int64_t n, int n_va
     if (need > 0 && reinterpret_cast<uintptr_t>(scratch) % 256 != 0) {
         ASH_FAIL("insert scratch must be 256-byte aligned");
     }
+    if (check_rows(n_values, src, dst, row_bytes)) return 1;
     DeviceGuard guard;
     ASH_HIP(guard.enter(map->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -3846,29 +3845,24 @@ int ash_map_insert_auto(ash_map_t* map, const int32_t* keys, int64_t n, int n_va
     // refused keys stay in the counters for a later call to find)
     if (!capturing && upkeep(map, n, scratch, scratch_bytes, s)) return 1;
     if (path == kPathStreaming) {
-        uint64_t* early = nullptr;
-        if (!capturing) {
-            if (take_line(map) || settle_landing_place(map)) return 1;
-            early = map->line + kLineEarly;
-        }
-        const int32_t stamp = map->stamp = next_stamp(map->stamp);
+        LatePlace late(map);
+        if (!capturing && late.take(true)) return 1;
         // Only keys that the first pass hands to the per-key kernel can be
         // waiting for the second region; their number arrives a quarter into
         // the call's work.  None: the counters come with the insert's last
         // launch, and nobody waits for them here.
         bool published = false;
         if (insert_bulk(map, keys, n, n_values, src, dst, row_bytes, scratch, scratch_bytes,
-                        early, early != nullptr ? map->line + kLineLate : nullptr, stamp, &published,
-                        stream)) {
+                        capturing ? nullptr : late.early(), capturing ? nullptr : late.late(), late.stamp,
+                        &published, stream)) {
             return 1;
         }
         if (capturing) return 0;
         if (published) {
-            std::lock_guard<std::mutex> lock(map->counter_lock);
-            map->unread_inserts = 0;
-            late_words_queued(map, stamp);
+            late.queued();
             return 0;
         }
+        late.unused();
     } else {
         // The counters come behind the insert (a short launch leaves them itself) and
         // wait for the call that asks for them; only a batch with keys for the second
@@ -3905,23 +3899,23 @@ int ash_map_insert_auto(ash_map_t* map, const int32_t* keys, int64_t n, int n_va
                 check = {static_cast<unsigned>(std::min<int64_t>(groups, kMostChecks)), answer.words,
                          answer.stamp, next_ticket(map)};
             }
-            // (the words of the answer may come from any exit below that follows a launch)
-            if (check.groups > 0) answer.abandon();
             LatePlace late(map);
             if (late.take(true)) return 1;
+            // (the words of the answer may come from any exit below that follows a launch)
+            if (check.groups > 0) answer.abandon();
             const bool leaves = n <= kLeaveKeys;
             Publish publish = {};
-            if (leaves) publish = {map->line + kLineLate, late.stamp, next_ticket(map)};
+            if (leaves) publish = {late.late(), late.stamp, next_ticket(map)};
             if (insert_per_key(map, keys, n, n_values, src, dst, row_bytes,
                                path == kPathAssigned ? static_cast<int32_t*>(scratch) : nullptr,
                                stream, publish, check)) {
                 return 1;
             }
             if (!leaves) {
-                publish_counters_kernel<<<1, 64, 0, s>>>(map->d.ctr, map->line + kLineLate, late.stamp);
+                publish_counters_kernel<<<1, 64, 0, s>>>(map->d.ctr, late.late(), late.stamp);
                 ASH_LAUNCH_CHECK();
             }
-            late.queued(false);
+            late.queued();
             if (check.groups == 0) return 0;
             if (answer.wait(s, 1)) return 1;
             if (value_of(answer.words[0]) == 0) return 0;

@@ -157,6 +157,8 @@ int erase_selected(ash_map* map, bool codes, const void* keys, const int32_t* se
                    const int32_t* nsel, hipStream_t s);
 
 int check_batch(const ash_map* map, const void* keys, int64_t n);
+// The value tables of an insert.
+int check_rows(int n_values, const void* const* src, void* const* dst, const int64_t* row_bytes);
 inline bool is_capturing(hipStream_t s) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
@@ -232,8 +234,6 @@ int wait_for_words(const uint64_t* words, int count, int32_t stamp);
 // any table; refused keys whose counters nobody has read yet may have left some,
 // which then wait for a later insert.)
 inline bool tombs_in(const ash_map* map) { return map->maybe_tombstones || map->replayed; }
-// Waits for the counters that a launch may still owe at kLineLate.
-int settle_landing_place(ash_map* map);
 // Counts the flags that are up among the first `rows` into the counter of touched
 // blocks and queues the read-back of the counters behind the stream's work; `counts`:
 // `max_counts` words of scratch on the device (ash_map.hip).

@@ -192,3 +192,14 @@ def inserts_that_are_refused_before_their_launch(device):
         assert m.insert(values=1, row_bytes=0) == 1   # (no value rows)
         assert m.insert() == 0
     assert _lines(device, 0) == used
+
+
+def a_frame_whose_count_fails(device):
+    """It is integrated all the same: its flags, left up, would have the next frame
+    integrate and count its blocks as well."""
+    m = Map(device)
+    device.refuse = ("count_flags_kernel",)
+    assert m.fuse() == 1
+    assert any("integrate_depth_flagged_kernel" in name for name in device.launched)
+    device.refuse = ()
+    assert m.fuse() == 0

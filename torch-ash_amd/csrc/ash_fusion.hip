@@ -442,12 +442,14 @@ extern "C" int ash_grid_fuse_frame(
     // queued by the time that ends.  (The count behind the integration, from a word of
     // each of its workgroups, left the device idle for the way to the host and back:
     // a VGA frame with its count 55 us, 43 like this.)
-    if (group_counts != nullptr &&
-        queue_touched_count(map, touched, std::min(map->capacity, num_embeddings), group_counts,
-                            kFlaggedGroups, s)) {
-        return 1;
-    }
-    return launch_flagged(map, a, touched, s);
+    // (Where it fails the frame is integrated all the same: flags left up would be the
+    // next frame's.)
+    const int uncounted =
+            group_counts != nullptr
+                    ? queue_touched_count(map, touched, std::min(map->capacity, num_embeddings),
+                                          group_counts, kFlaggedGroups, s)
+                    : 0;
+    return launch_flagged(map, a, touched, s) || uncounted ? 1 : 0;
 }
 
 extern "C" int ash_grid_integrate_depth(

@@ -203,3 +203,10 @@ def a_frame_whose_count_fails(device):
     assert any("integrate_depth_flagged_kernel" in name for name in device.launched)
     device.refuse = ()
     assert m.fuse() == 0
+
+
+def larger_workgroups_only_where_they_are_launched(device):
+    """Inserts of keys, with rows and without (modes 0 and 1)."""
+    wide = {name.split("insert_kernelI")[1][:10] for name in device.kernels()
+            if "insert_kernelI" in name and "Li512E" in name}
+    assert wide == {f"Li{dim}ELi{mode}ELb" for dim in (1, 2, 3, 4) for mode in (0, 1)}, wide

@@ -66,6 +66,14 @@ class Device:
         self.lib.ash_last_error.restype = ctypes.c_char_p
         self.ctr = None
 
+    def kernels(self):
+        name = self.runtime.stand_in_kernel
+        name.restype = ctypes.c_char_p
+        names = []
+        while name(len(names)) is not None:
+            names.append(name(len(names)).decode())
+        return names
+
     def stream(self, number):
         return self.streams.setdefault(number, Stream())
 

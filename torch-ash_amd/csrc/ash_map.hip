@@ -2631,9 +2631,12 @@ template <int MODE, bool TOMBS>
 int launch_insert_to(ash_map* map, const int32_t* keys, int64_t n,
                      const ValueArgs& va, int32_t* assigned, const int64_t* given,
                      hipStream_t s, const Publish& publish = {}, const KeyCheck& check = {}) {
-    return n > kWideInsert && n <= kWideInsertEnd && (MODE == kInsertKeys || MODE == kInsertFused)
-                   ? launch_insert_by<MODE, TOMBS, kWideBlock>(map, keys, n, va, assigned, given, s, publish, check)
-                   : launch_insert_by<MODE, TOMBS, kHeapBlock>(map, keys, n, va, assigned, given, s, publish, check);
+    if constexpr (MODE == kInsertKeys || MODE == kInsertFused) {
+        if (n > kWideInsert && n <= kWideInsertEnd) {
+            return launch_insert_by<MODE, TOMBS, kWideBlock>(map, keys, n, va, assigned, given, s, publish, check);
+        }
+    }
+    return launch_insert_by<MODE, TOMBS, kHeapBlock>(map, keys, n, va, assigned, given, s, publish, check);
 }
 
 template <int MODE>

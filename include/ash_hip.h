@@ -424,11 +424,10 @@ int ash_map_erase_bulk(ash_map_t* map, const int32_t* keys, int64_t n, void* wor
  * waiting for the second region stay in the counters.  `staging` as for
  * ash_map_counters. */
 enum { ASH_STREAMING_AUTO = 0, ASH_STREAMING_ALWAYS = 1, ASH_STREAMING_NEVER = 2,
-       /* inserts only: as AUTO, and in batches from 2^16 keys (2^17 with value rows)
-        * into tables emptied and not used since, where they pay off as long as most
-        * of the keys are not repeated, and without a wait for the counters of other
-        * batches; the package's own choice.  (AUTO keeps the bars by which callers
-        * have sized their scratch.) */
+       /* inserts only: as AUTO, in batches of keys alone from 2^17 on into tables
+        * emptied and not used since as well, and without a wait for the counters of a
+        * per-key insert; the package's own choice.  (AUTO keeps the bars by which
+        * callers have sized their scratch.) */
        ASH_STREAMING_EARLY = 3 };
 enum { ASH_NEEDS_GENERAL = 2 };
 int ash_map_insert_scratch_bytes(ash_map_t* map, int64_t n, int n_values,

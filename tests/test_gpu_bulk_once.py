@@ -185,28 +185,38 @@ def test_replays_of_a_streamed_insert(ash):
         assert s.size() == 0
 
 
-def test_which_batches_stream_early(monkeypatch):
+def test_which_batches_stream():
     """The bars of ASH_STREAMING_EARLY (3) on new tables and on tables in use, and what
-    ASH_STREAMING_AUTO (0) says to the same: scratch is asked for or not."""
+    ASH_STREAMING_AUTO (0) says to the same: scratch is asked for or not.  Smaller
+    batches, those with rows and those into tables in use lose where keys repeat or are
+    stored already."""
     import ctypes
 
     import ash
 
-    def wanted(engine, n, policy, rows=()):
+    def wanted(engine, n, rows=()):
+        """(under ASH_STREAMING_EARLY, under ASH_STREAMING_AUTO)"""
         nbytes = ctypes.c_int64(-1)
         widths = (ctypes.c_int64 * max(1, len(rows)))(*rows)
-        backend = engine.backend
-        backend._check(backend._lib.ash_map_insert_scratch_bytes(
-            backend._handle, n, len(rows), widths if rows else None, policy, ctypes.byref(nbytes)))
-        return nbytes.value > 0
+        backend, both = engine.backend, []
+        for policy in (3, 0):
+            backend._check(backend._lib.ash_map_insert_scratch_bytes(
+                backend._handle, n, len(rows), widths if rows else None, policy, ctypes.byref(nbytes)))
+            both.append(nbytes.value > 0)
+        return tuple(both)
 
+    yes, no, early = (True, True), (False, False), (True, False)
     engine = ash.ASHEngine(3, 300_000, DEV)          # 50 176 buckets
-    assert wanted(engine, 1 << 16, 3) and not wanted(engine, (1 << 16) - 1, 3)
-    assert wanted(engine, 1 << 17, 3, (12, 4)) and not wanted(engine, (1 << 17) - 1, 3, (12, 4))
-    assert not wanted(engine, 1 << 16, 0) and not wanted(engine, 1 << 17, 0, (12, 4))
-    assert not wanted(engine, 13 * 50_176, 3)        # piles
+    assert wanted(engine, 1 << 17) == early and wanted(engine, (1 << 17) - 1) == no
+    assert wanted(engine, (1 << 18) - 1) == early and wanted(engine, 1 << 18) == yes
+    assert wanted(engine, (1 << 18) - 1, (12, 4)) == no and wanted(engine, 1 << 18, (12, 4)) == yes
+    assert wanted(engine, 13 * 50_176) == no         # piles
     wide = ash.ASHEngine(3, 1_200_000, DEV)          # 200 192 buckets
-    assert not wanted(wide, 1 << 16, 3) and wanted(wide, 1 << 17, 3)
-    engine.find(_keys(0, 10))                        # in use from here on
-    assert not wanted(engine, 1 << 17, 3) and not wanted(engine, 1 << 18, 3, (12, 4))
-    assert wanted(engine, 1 << 18, 3) and not wanted(engine, 1 << 18, 0)
+    assert wanted(wide, 200_191) == no and wanted(wide, 200_192) == early
+    large = ash.ASHEngine(3, 4_000_000, DEV)         # 667 136 buckets
+    assert wanted(large, 1 << 18) == yes
+    assert wanted(large, 1 << 18, (12, 4)) == no and wanted(large, 340_000, (12, 4)) == yes
+    for each in (engine, wide, large):
+        each.find(_keys(0, 10))                      # in use from here on
+        assert wanted(each, 1 << 18) == no and wanted(each, 400_000, (12, 4)) == no
+    assert wanted(large, 660_000) == no and wanted(large, 1 << 20) == yes

@@ -1685,32 +1685,28 @@ int ash_map_bulk_workspace_bytes(ash_map_t* map, int64_t n, int n_values,
 
 }  // extern "C"
 
-// The bars of one split pass (ASH_STREAMING_EARLY), beside those above.  Per key ->
-// streamed, the call and the size after it (us), tables emptied and not used since, by
-// keys per bucket:
-//   keys alone              3            1            1/2          1/4
-//     32 000             25.7 -> 26.9  25.0 -> 26.2  25.0 -> 27.2  25.7 -> 29.3
-//     65 000             32.7 -> 27.7  28.4 -> 27.7  28.8 -> 29.8  30.8 -> 34.3
-//     131 000            44.6 -> 30.8  40.3 -> 29.8  41.7 -> 34.8  43.2 -> 46.7
-//     262 000            68.9 -> 30.3  58.2 -> 35.3  58.7 -> 47.7  62.7 -> 65.8
-//   rows of 16 bytes
-//     65 000             38.1 -> 37.7  33.4 -> 36.7  33.6 -> 38.4  35.3 -> 40.8
-//     131 000            49.6 -> 38.6  45.3 -> 38.9  47.9 -> 41.2  53.6 -> 52.9
-//     262 000            70.8 -> 42.0  65.1 -> 47.2  64.8 -> 54.6  69.4 -> 72.5
-// Keys that repeat cost the streaming insert more: of 65 000 and 131 000 keys, three a
-// bucket, each stored twice 29.8 -> 28.4 and 39.3 -> 29.6, sixteen times 26.9 -> 40.1
-// and 33.1 -> 32.2; with rows, 131 000 each twice 42.4 -> 52.9.  Without a wait for
-// the size the streamed call gains 10 us more: it does not wait for its own counters.
-// Tables in use, keys alone: 262 000 keys into 167 000 buckets with 500 000 entries 56 ->
-// 36, 131 000 31.7 -> 33.4; 1 M into 667 000 with 2 M 113 -> 78, 524 000 71.8 -> 71.5.
-// With rows a batch of which many keys are stored already loses by its moves.
-bool ash::streams_early(const ash_map* map, int64_t n, int n_values, const int64_t* row_bytes) {
+// The bar of one split pass (ASH_STREAMING_EARLY), beside those above, for keys alone
+// into tables emptied and not used since.  Per key -> streamed, the call and the size
+// after it (us), by keys per bucket, each key once / twice / sixteen times / 64 times:
+//   131 000   3   45.6 -> 36.4   43.1 -> 35.6   35.6 -> 38.8   35.7 -> 49.3
+//             1   44.4 -> 37.0   43.1 -> 37.6   36.5 -> 49.0   36.7 -> 49.9
+//             1/2 42.2 -> 40.1   44.8 -> 39.9   37.2 -> 43.2
+//   200 000   3   53.9 -> 35.9   45.1 -> 36.8   38.2 -> 49.5   38.1 -> 49.6
+//             1   45.8 -> 39.0   43.8 -> 39.7   38.7 -> 42.6   39.3 -> 52.0
+//   65 000    3   35.5 -> 35.8   31.8 -> 35.4   30.0 -> 47.6
+// A batch of points to be set as voxels, ten or twenty of them in each, loses up to a
+// third, one of distinct keys gains as much; and where repeats are the rule the table
+// is sized for the voxels, and the bound against piles keeps them from here.  With
+// value rows repeats cost a move each (131 000 with rows of 16 bytes, three a bucket:
+// 49.1 -> 46.6, twice 45.4 -> 55.9, sixteen times 39.1 -> 58.8), and tables in use lose
+// where the keys are stored already, which costs the per-key kernel no atomics (262 000
+// of 500 000 entries 19.3 -> 31.2, a million of two 35.9 -> 62.9; half of them stored
+// and each four times 58.2 -> 86.6): neither streams before the bars above.
+bool ash::streams_early(const ash_map* map, int64_t n, int n_values) {
     BulkPlan pl;
     const int64_t nb = static_cast<int64_t>(map->d.nb);
-    if (n > 12 * nb || make_plan(map, n, n_values, row_bytes, nullptr, pl) == 0 || !pl.once) return false;
-    if (!map->table_stale) return n_values == 0 && n >= (int64_t{1} << 18) && 5 * n >= 6 * nb;
-    if (n_values > 0) return n >= (int64_t{1} << 17) && 2 * n >= nb;
-    return n >= (int64_t{1} << 17) ? 2 * n >= nb : n >= (int64_t{1} << 16) && n >= nb;
+    return map->table_stale && n_values == 0 && n >= (int64_t{1} << 17) && n >= nb && n <= 12 * nb &&
+           make_plan(map, n, 0, nullptr, nullptr, pl) > 0 && pl.once;
 }
 
 int ash::insert_bulk(ash_map* map, const int32_t* keys, int64_t n,

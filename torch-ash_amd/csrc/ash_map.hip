@@ -3798,7 +3798,7 @@ int plan_insert(ash_map_t* map, int64_t n, int n_values, const int64_t* row_byte
         int worthwhile = 0;
         if (ash_map_bulk_workspace_bytes(map, n, n_values, row_bytes, &ws, &worthwhile)) return 1;
         if (ws > 0 && (worthwhile || policy == ASH_STREAMING_ALWAYS ||
-                       (policy == ASH_STREAMING_EARLY && streams_early(map, n, n_values, row_bytes)))) {
+                       (policy == ASH_STREAMING_EARLY && streams_early(map, n, n_values)))) {
             *path = kPathStreaming;
             *bytes = ws;
         }

@@ -248,7 +248,7 @@ int insert_bulk(ash_map* map, const int32_t* keys, int64_t n, int n_values,
                 void* workspace, int64_t workspace_bytes, uint64_t* early, uint64_t* late,
                 int32_t stamp, bool* published, void* stream);
 // Whether a batch is one to stream under ASH_STREAMING_EARLY (ash_bulk.hip).
-bool streams_early(const ash_map* map, int64_t n, int n_values, const int64_t* row_bytes);
+bool streams_early(const ash_map* map, int64_t n, int n_values);
 // Buckets up to which a clear fills the table at once, in the launch that resets the
 // counters (2.8 MB, half a microsecond of stores where a streaming insert follows).
 constexpr int64_t kFillAtOnce = 21845;

@@ -241,7 +241,8 @@ int ash_grid_integrate_depth_flagged(ash_map_t* map, float* embeddings,
  * ash_grid_activate_positions and ash_grid_integrate_depth_flagged, two
  * launches.  Cell to world is cell * cell_to_world [+ world_origin], with
  * world_origin float32[3] on the device or NULL.  group_counts (int32
- * [ASH_FLAGGED_GROUPS] of scratch on the device, or NULL): a small launch between
+ * [ASH_FLAGGED_GROUPS] of scratch on the device, a word per 2^18 rows of the
+ * largest table, or NULL): a small launch between
  * the two (two above 2^18 rows) counts the touched blocks and leaves the counters for
  * the host; the next ash_map_counters waits for them, not for the integration, and
  * finds the count in out[5].  Refused with group_counts on a stream that is being

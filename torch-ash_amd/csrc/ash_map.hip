@@ -19,7 +19,7 @@
 // Index allocation follows the reference's heap protocol
 // (ash/src/hashmap_gpu.cuh:211-232,316-336): a new key takes heap[counter++],
 // an erased key stores its index at heap[--counter]; here the counter is
-// advanced once per 256-thread block instead of once per key.
+// advanced once per workgroup instead of once per key.
 #include "ash_probe.h"
 
 #include "../../include/ash_hip.h"

@@ -88,7 +88,7 @@ VALUE_ROW_BYTES = 2 * (12 + 4)               # color + depth, read and written
 #   atomic_requests: TCC_ATOMIC (all of them are forwarded to the memory side:
 #     TCC_EA0_ATOMIC reads the same).
 MEASURED_COUNTERS = {
-    "insert_values": (2_566_000_000 + 1_949_000_000, 0.381, 16_332_000),
+    "insert_values": (2_568_000_000 + 1_939_000_000, 0.364, 16_350_000),
     "insert_keys": (2_305_000_000 + 1_687_000_000, 0.282, 16_397_000),
     "find": (2_230_000_000 + 145_000_000, 0.064, 0),
     "erase": (2_236_000_000 + 1_217_000_000, 0.467, 16_031_000),
@@ -119,7 +119,7 @@ MEASURED_COUNTERS = {
 COUNTERS_SOURCE = {
     "profiles": ["profiles/bench_hbm_traffic_pmc.md",
                  "profiles/bench_l2_hit_rate_and_atomics_pmc.md"],
-    "csrc_sha256": "49111aa2eaedfa5ae836047654a6f58b637ee5960d2350fe23f2c2818b788e49",
+    "csrc_sha256": "6282425853ddb8d8372191e8e1a7d5d4bdc2e2609313ea9a6c82d02780da7e3d",
 }
 
 

@@ -495,8 +495,8 @@ int ash_map_status(ash_map_t* map, int64_t out[5], void* stream);
  * used any more (NULL).  No counterpart in the reference, whose `size()`
  * synchronises every time (ash/src/hashmap_gpu.cuh:157). */
 int ash_map_counters(ash_map_t* map, int32_t* staging, int64_t out[7], void* stream);
-/* 1 while the read-back that a streaming ash_map_insert_auto queued has not
- * been looked at yet. */
+/* 1 while the read-back that an ash_map_insert_auto queued has not been looked at
+ * yet. */
 int ash_map_counters_pending(ash_map_t* map);
 /* 1 and *size when the size is known without a copy from the device (waits for
  * a queued read-back if there is one), 0 when it is not, -1 on failure. */

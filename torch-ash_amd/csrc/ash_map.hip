@@ -3576,7 +3576,8 @@ enum Asker { kOwnCall, kReader, kReaderOfDevice };
 // `s`.  A reader of the device, too, asks behind words that are under way: they belong
 // to a call that has returned.  What a reader has fetched is the latest state only if
 // it was asked for on the stream of the latest change, behind that, and none has begun
-// or been queued since; else it is the reader's alone.
+// or been queued since; else it is the reader's alone.  (Replays change them on any
+// stream: what is kept then holds for the call behind the reader's only.)
 int refresh_counters(ash_map* map, hipStream_t s, Asker asker, ash_counters& c) {
     std::unique_lock<std::mutex> lock(map->counter_lock);
     if (map->replayed) {
@@ -3602,7 +3603,7 @@ int refresh_counters(ash_map* map, hipStream_t s, Asker asker, ash_counters& c) 
     decode_counters(answer.words, c);
     lock.lock();
     if (asker == kOwnCall ||
-        (map->changes == changes && s == map->changed_on && !map->counters_known)) {
+        (map->changes == changes && (s == map->changed_on || map->replayed) && !map->counters_known)) {
         map->counters = c;
         counters_taken(map);
     }

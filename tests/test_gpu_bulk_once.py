@@ -146,6 +146,35 @@ def test_piles_of_one_key(ash, with_rows):
 
 
 @pytest.mark.parametrize("with_rows", [False, True])
+@pytest.mark.parametrize("ranges", [512, 513, 1300])
+@pytest.mark.parametrize("per_bucket, copies", [(0.5, 1), (3, 2), (4.5, 1), (4.5, 40), (3, 4000)])
+def test_ranges_built_from_lists(ash, with_rows, ranges, per_bucket, copies):
+    """Emptied tables on both sides of the number of ranges and of the records per
+    bucket from which ranges are built from lists: buckets that overflow, keys that
+    repeat beyond a bucket's slots, beyond what is placed beside the list, beyond a
+    range's records."""
+    capacity, n = ranges * PART, int(ranges * 512 * per_bucket)
+    distinct = _keys(7, max(n // copies, n - 40_000) if copies == 4000 else n // copies)
+    if copies == 4000:   # piles of a few keys among many
+        keys = torch.cat([distinct, distinct[:10].repeat(4000, 1)[: n - len(distinct)]])
+    else:
+        keys = distinct.repeat(copies, 1)
+    keys = keys[torch.randperm(len(keys), device=DEV)].contiguous()
+    if with_rows:
+        m, rows = ash.HashMap(3, {"color": 3, "id": 1}, capacity, DEV), _rows(len(keys))
+        m.insert(keys, rows)
+        _check(m, distinct, (keys, rows))
+    else:
+        m = ash.HashSet(3, capacity, DEV)
+        m.insert(keys)
+        _check(m, distinct)
+    absent = _keys(100_000_000, 50_000)
+    assert not bool(m.engine.find(absent)[1].any())
+    m.engine.erase(distinct[::2].contiguous())
+    _check(m, distinct[1::2].contiguous())
+
+
+@pytest.mark.parametrize("with_rows", [False, True])
 def test_keys_that_do_not_pack_and_batches_beyond_the_capacity(ash, with_rows):
     far = _keys(0, 700) + (1 << 24)
     distinct = torch.cat([_keys(0, 9_000), far])

@@ -60,6 +60,16 @@ constexpr int kMaxBins = 256;
 constexpr int kOnceChunks = 1024;
 constexpr int kOnceParts = 4096;
 constexpr int kBuildThreads = 512;
+// Ranges that start empty are built from lists (build_lists_kernel) where there are more
+// than the two workgroups of build_kernel per CU take at once, and with up to so many
+// records per two buckets.  build_kernel -> lists, kernel (us), keys alone: 86 ranges
+// 11.7 -> 13.2, 261 15.9 -> 15.6, 652 28.3 -> 22.4, 1303 37.9 -> 35.8, 912 of 4.3 records
+// a bucket 44.9 -> 31.7, 2605 71.4 -> 68.7; with rows, four records a bucket: 128 ranges
+// 13.4 -> 16.1, 489 15.9 -> 17.5, 1465 42.9 -> 38.2, of two a bucket 2930 71.6 -> 49.2.
+// From five records a bucket on too many buckets overflow.
+constexpr int64_t kListsFrom = 512;
+constexpr int kMostPerTwoBuckets = 9;
+constexpr int kListRecs = 6;   // records per thread there
 constexpr int kBuildRecs = 4;                   // records per thread and round
 constexpr int kCopyThreads = 256;
 constexpr int64_t kMinKeys = 1 << 12;
@@ -78,6 +88,8 @@ struct BulkPlan {
     int64_t n;
     bool once;             // one split pass: of what follows only `parts`, `cap_part`,
                            // `once_chunks` and the planes named there are used
+    bool lists;            // ... and the ranges are built from lists (build_lists_kernel),
+    int share_shift;       // 1 << share_shift threads to a chunk
     uint32_t once_chunks;
     int once_slot;           // of the launches' places (next_slot)
     uint32_t once_halving;   // the largest power of two below once_chunks (or 0)
@@ -164,6 +176,13 @@ int64_t make_plan(const ash_map* map, int64_t n, int n_values,
 
     const int64_t once_chunks = (n + kSplitChunk - 1) / kSplitChunk;
     pl.once = insert && parts <= kOnceParts && once_chunks <= kOnceChunks;
+    pl.lists = pl.once && map->table_stale && heap_in_order(map) && parts > kListsFrom &&
+               2 * n <= kMostPerTwoBuckets * nb && cap_part <= kBuildThreads * kListRecs;
+    pl.share_shift = 0;
+    while (pl.lists && (once_chunks << (pl.share_shift + 1)) <= kBuildThreads &&
+           once_chunks + 1 <= cap_part) {
+        ++pl.share_shift;
+    }
     pl.once_chunks = static_cast<uint32_t>(once_chunks);
     pl.once_halving = 0;
     for (uint32_t h = 1; h < pl.once_chunks; h <<= 1) pl.once_halving = h;
@@ -1186,6 +1205,371 @@ __global__ __launch_bounds__(kBuildThreads, 4) void build_kernel(
     }
 }
 
+// Pass 3 where the ranges are known to start empty and a bucket gets a few records: a
+// workgroup sorts the records of its range by bucket into one list in LDS and makes the
+// buckets out of that as it writes them.  A list of what is there takes 12 bytes per
+// record where build_kernel holds the 64 KB that become of it, so that four workgroups
+// run on a CU instead of two, and a build is a chain of short steps with a barrier
+// behind each: what it takes is the time of a workgroup times the rounds they need
+// (1 M keys, half of them repeats, into 652 ranges: two rounds of 14 and 11 us, now one
+// of 15, a fifth of it the queue at the heap counter).
+//
+// A record draws a number in its bucket (one LDS atomic); the numbers below ten are
+// slots, and running sums of the buckets' numbers give each bucket's place in the list.
+// Then a thread per bucket empties the slots that repeat a lower one, and what is left
+// gets its indices: in the order of the list from one update of the heap counter, or
+// (provisional scheme) the promised ones.  Records with a number of ten or more are
+// compared with the bucket's slots; what is not found there and does not repeat one of
+// its like is placed by the rule of a probe, a thread each: in a slot that a repeat has
+// left, or behind the slots of the first bucket of the sequence that has one free.  The
+// latter have no place in the list and are written into their slots after the buckets.
+constexpr int kBeside = 128;   // of them; more are left to the per-key kernel
+
+template <bool PROV>
+__global__ __launch_bounds__(kBuildThreads, 8) void build_lists_kernel(
+        MapDev m, BulkPlan pl, int stale) {
+    constexpr int kWaves = kBuildThreads / 64;
+    constexpr int kRecs = kListRecs;
+    constexpr int kCounts = kRecs * kWaves;
+    static_assert(kBuildThreads == static_cast<int>(kPartBuckets), "a thread per bucket");
+    static_assert(kCounts < 64, "a wavefront adds up the counts of the list's pieces");
+    extern __shared__ uint64_t s_code[];                                 // cap_part codes: the list,
+    int32_t* s_idx = reinterpret_cast<int32_t*>(s_code + pl.cap_part);   // and their indices
+    __shared__ int s_cnt[kPartBuckets];         // numbers drawn per bucket; later the slots in use
+    __shared__ int s_first[kPartBuckets + 1];   // where a bucket's slots start in the list
+    __shared__ int s_sum[64];
+    __shared__ int s_base;
+    __shared__ int s_losers;
+    __shared__ uint64_t s_beside_code[kBeside];
+    __shared__ int32_t s_beside_row[kBeside];    // row (or place in codes_a); later the index
+    __shared__ int32_t s_beside_slot[kBeside];   // bucket * 16 + slot, or -1
+    __shared__ int s_nbeside;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
+    const uint32_t p = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (p >= pl.parts) return;
+    const uint32_t b0 = p << kPartShift;   // (nb is a multiple of kPartBuckets: more than one range)
+    typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+    v4u* __restrict__ gl = reinterpret_cast<v4u*>(m.buckets) + static_cast<size_t>(b0) * kGroup;
+
+    // the records of this range in each chunk, and before it
+    static_assert(kOnceChunks == 2 * kBuildThreads, "a thread adds up two chunks");
+    int first[2], own[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const int c = 2 * tid + q;
+        first[q] = own[q] = 0;
+        if (c < static_cast<int>(pl.once_chunks)) {
+            const uint16_t* at = pl.starts + static_cast<int64_t>(c) * (pl.parts + 1) + p;
+            first[q] = at[0];
+            own[q] = at[1] - at[0];
+        }
+    }
+    s_cnt[tid] = 0;
+    if (tid == 0) s_losers = s_nbeside = 0;
+    // running sums over the workgroup: what lies before the thread's `v`, and all
+    auto before_of = [&](int v, int& all) {
+        int incl = v;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int up = __shfl_up(incl, d);
+            if (lane >= d) incl += up;
+        }
+        if (lane == 63) s_sum[wave] = incl;
+        __syncthreads();
+        int before = incl - v;
+        all = 0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            if (w < wave) before += s_sum[w];
+            all += s_sum[w];
+        }
+        return before;
+    };
+    int all;
+    int before = before_of(own[0] + own[1], all);
+    if (all == 0) {
+        if (stale) {
+            for (int t = tid; t < static_cast<int>(kPartBuckets) * kGroup; t += kBuildThreads) {
+                const v4u none = {~0u, ~0u, ~0u, ~0u};
+                gl[t] = none;
+            }
+        }
+        return;
+    }
+    const int cnt = all < static_cast<int>(pl.cap_part) ? all : static_cast<int>(pl.cap_part);
+    // where the records lie, for whoever takes them; those beyond the range's capacity
+    // are left to the per-key kernel
+    auto leave = [&](int32_t row) {
+        if constexpr (PROV) {
+            give_up_row(pl, row, &s_losers, true);
+        } else {
+            pl.spill_a[atomicAdd(pl.hdr + kHdrSpillA, 1)] = row;
+        }
+    };
+    auto row_at = [&](int at) -> int32_t {
+        if constexpr (PROV) return (at & ~(kSplitChunk - 1)) + pl.rows_once[at];
+        return at;
+    };
+    // (several threads to a chunk where there are few: pl.share_shift)
+    int2* s_from = reinterpret_cast<int2*>(s_code);   // of a chunk: its first record, and those before it
+    const int share = 1 << pl.share_shift;
+    auto list_chunk = [&](int at, int done, int many, int j) {
+        for (; j < many; j += share) {
+            if (done + j < cnt) {
+                s_idx[done + j] = at + j;
+            } else {
+                leave(row_at(at + j));
+            }
+        }
+    };
+    if (share == 1) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            list_chunk((2 * tid + q) * kSplitChunk + first[q], before, own[q], 0);
+            before += own[q];
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int c = 2 * tid + q;
+            if (c <= static_cast<int>(pl.once_chunks)) s_from[c] = make_int2(c * kSplitChunk + first[q], before);
+            before += own[q];
+        }
+        __syncthreads();
+        const int c = tid >> pl.share_shift;
+        if (c < static_cast<int>(pl.once_chunks)) {
+            const int2 from = s_from[c];
+            list_chunk(from.x, from.y, s_from[c + 1].y - from.y, tid & (share - 1));
+        }
+    }
+    __syncthreads();
+    uint64_t code[kRecs];
+    int32_t row[kRecs];
+    int drawn[kRecs];   // number << kPartShift | bucket, or -1
+#pragma unroll
+    for (int k = 0; k < kRecs; ++k) {
+        code[k] = 0ull;
+        row[k] = 0;
+        if (k * kBuildThreads + tid < cnt) {
+            const int at = s_idx[k * kBuildThreads + tid];
+            code[k] = pl.codes_a[at];
+            row[k] = row_at(at);
+        }
+    }
+    bool crowded = false;
+#pragma unroll
+    for (int k = 0; k < kRecs; ++k) {
+        drawn[k] = -1;
+        if (k * kBuildThreads + tid < cnt) {
+            const int lb = static_cast<int>(bucket_of(code[k], m.nb) - b0);
+            const int number = atomicAdd(&s_cnt[lb], 1);
+            drawn[k] = number << kPartShift | lb;
+            crowded = crowded || number >= kSlots;
+        }
+    }
+    crowded = __syncthreads_or(crowded);
+    const int slots = s_cnt[tid] < kSlots ? s_cnt[tid] : kSlots;
+    int total;
+    const int mine = before_of(slots, total);
+    s_first[tid] = mine;
+    if (tid == 0) s_first[kPartBuckets] = total;
+    s_cnt[tid] = slots;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kRecs; ++k) {
+        if (drawn[k] >= 0 && drawn[k] < kSlots << kPartShift) {
+            const int at = s_first[drawn[k] & (kPartBuckets - 1)] + (drawn[k] >> kPartShift);
+            s_code[at] = code[k];
+            if constexpr (PROV) s_idx[at] = row[k];   // (the heap holds 0, 1, 2, ...)
+        }
+    }
+    __syncthreads();
+    if (crowded) {
+#pragma unroll
+        for (int k = 0; k < kRecs; ++k) {
+            if (drawn[k] < kSlots << kPartShift) continue;
+            const int from = s_first[drawn[k] & (kPartBuckets - 1)];
+            bool known = false;
+            // (a repeat may be emptied meanwhile, below; the lowest slot of its code stays)
+#pragma unroll
+            for (int j = 0; j < kSlots; ++j) known = known || s_code[from + j] == code[k];
+            if (known) {
+                if constexpr (PROV) give_up_row(pl, row[k], &s_losers, false);
+                continue;
+            }
+            const int at = atomicAdd(&s_nbeside, 1);
+            if (at < kBeside) {
+                s_beside_code[at] = code[k];
+                s_beside_row[at] = row[k];
+            } else {
+                leave(row[k]);
+            }
+        }
+    }
+    // a thread per bucket: slots that repeat a lower one are emptied
+    {
+        uint64_t c[kSlots];
+#pragma unroll
+        for (int j = 0; j < kSlots; ++j) c[j] = s_code[mine + j];   // (what lies behind its own does not count)
+#pragma unroll
+        for (int j = 1; j < kSlots; ++j) {
+            bool repeat = false;
+#pragma unroll
+            for (int i = 0; i < j; ++i) repeat = repeat | (c[i] == c[j]);
+            if (repeat & (j < slots)) {
+                if constexpr (PROV) give_up_row(pl, s_idx[mine + j], &s_losers, false);
+                s_code[mine + j] = kEmpty;
+                s_idx[mine + j] = -1;
+            }
+        }
+    }
+    __syncthreads();
+    int nbeside = 0;
+    if (crowded) {
+        // distinct among themselves first; then each goes where a probe would look for it
+        // (what is taken of a bucket is never given back here, so a key that goes on has
+        // met ten slots in use)
+        nbeside = s_nbeside < kBeside ? s_nbeside : kBeside;
+        if (tid < nbeside) {
+            const uint64_t own_code = s_beside_code[tid];
+            const int32_t own_row = s_beside_row[tid];
+            bool known = false;
+            for (int x = 0; x < tid; ++x) known = known || s_beside_code[x] == own_code;
+            int b = static_cast<int>(bucket_of(own_code, m.nb) - b0);
+            int at = -1;        // its place in the list
+            int beside = -1;    // or beside it
+            for (int visited = 0; !known && at < 0 && beside < 0 && visited < static_cast<int>(kPartBuckets);
+                 ++visited) {
+                const int to = s_first[b + 1];
+                for (int h = s_first[b]; h < to && at < 0; ++h) {
+                    if (s_code[h] != kEmpty) continue;
+                    if (atomicCAS(reinterpret_cast<unsigned long long*>(s_code + h), kEmpty, own_code) == kEmpty) at = h;
+                }
+                if (at < 0 && s_cnt[b] < kSlots) {
+                    const int slot = atomicAdd(&s_cnt[b], 1);
+                    if (slot < kSlots) beside = b * 16 + slot;
+                }
+                b = b + 1 == static_cast<int>(kPartBuckets) ? 0 : b + 1;
+            }
+            s_beside_slot[tid] = beside;
+            if (at >= 0) {
+                if constexpr (PROV) s_idx[at] = own_row;
+            } else if (beside < 0) {
+                if (!known) atomicAdd(m.ctr + kCtrDropped, 1);   // refused
+                if constexpr (PROV) give_up_row(pl, own_row, &s_losers, false);
+            }
+        }
+        __syncthreads();
+    }
+    // what becomes of a bucket: five pieces of two codes each, three with the indices
+    constexpr int kCodePieces = kSlots / 2;
+    auto code_piece = [&](int b, int q) {
+        const int from = s_first[b] + 2 * q, to = s_first[b + 1];
+        const uint64_t c0 = from < to ? s_code[from] : kEmpty;
+        const uint64_t c1 = from + 1 < to ? s_code[from + 1] : kEmpty;
+        const v4u y = {static_cast<uint32_t>(c0), static_cast<uint32_t>(c0 >> 32),
+                       static_cast<uint32_t>(c1), static_cast<uint32_t>(c1 >> 32)};
+        return y;
+    };
+    auto index_piece = [&](int b, int q) {
+        const int from = s_first[b] + 4 * (q - kCodePieces), to = s_first[b + 1];
+        v4u y;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) y[w] = from + w < to ? static_cast<uint32_t>(s_idx[from + w]) : ~0u;
+        return y;
+    };
+    // indices (those of rows are in place, and pass 1 has written the log)
+    if constexpr (!PROV) {
+        int rank[kRecs];
+#pragma unroll
+        for (int k = 0; k < kRecs; ++k) {
+            const int at = k * kBuildThreads + tid;
+            const uint64_t wins = __ballot(at < total && s_code[at < total ? at : 0] != kEmpty);
+            rank[k] = __popcll(wins & ((1ull << lane) - 1ull));
+            if (lane == 0) s_sum[k * kWaves + wave] = __popcll(wins);
+        }
+        if (crowded && wave == 0) {
+            // (kBeside: two to a lane)
+            const uint64_t low = __ballot(lane < nbeside && s_beside_slot[lane] >= 0);
+            const uint64_t high = __ballot(lane + 64 < nbeside && s_beside_slot[lane + 64] >= 0);
+            if (lane == 0) s_sum[kCounts] = __popcll(low) + __popcll(high);
+        } else if (tid == 0) {
+            s_sum[kCounts] = 0;
+        }
+        __syncthreads();
+        if (wave == 0) {
+            const int v = lane <= kCounts ? s_sum[lane] : 0;
+            int incl = v;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const int up = __shfl_up(incl, d);
+                if (lane >= d) incl += up;
+            }
+            s_sum[lane] = incl - v;
+            if (lane == 63) {
+                int at = 0;
+                if (incl > 0) {
+                    at = atomicAdd(m.ctr + kCtrSize, incl);
+                    if (at + incl > m.capacity) {
+                        const int lo = at > m.capacity ? at : m.capacity;
+                        const int excess = at + incl - lo;
+                        atomicSub(m.ctr + kCtrSize, excess);
+                        atomicAdd(m.ctr + kCtrDropped, excess);
+                    }
+                }
+                s_base = at;
+            }
+        }
+        __syncthreads();
+        // the index at `top` of the heap; none left: the slot is given up again
+        auto take = [&](int top, uint64_t& of, int32_t& idx) {
+            if (top < m.capacity) {
+                idx = top;   // (the heap holds 0, 1, 2, ...)
+                m.klog[idx] = of;
+            } else {
+                of = kTomb;
+                idx = -1;
+                atomicAdd(m.ctr + kCtrTombs, 1);
+            }
+        };
+#pragma unroll
+        for (int k = 0; k < kRecs; ++k) {
+            const int at = k * kBuildThreads + tid;
+            if (at < total && s_code[at] != kEmpty) {
+                take(s_base + s_sum[k * kWaves + wave] + rank[k], s_code[at], s_idx[at]);
+            }
+        }
+        if (tid < nbeside && s_beside_slot[tid] >= 0) {
+            int beside_rank = 0;
+            for (int x = 0; x < tid; ++x) beside_rank += s_beside_slot[x] >= 0 ? 1 : 0;
+            take(s_base + s_sum[kCounts] + beside_rank, s_beside_code[tid], s_beside_row[tid]);
+        }
+    }
+    __syncthreads();
+    // (whole lines past the caches, as in build_kernel: the codes first, while the heap
+    // counter is on its way, took a microsecond more, and 16 where they went past the
+    // caches as well)
+#pragma unroll 4
+    for (int t = tid; t < static_cast<int>(kPartBuckets) * kGroup; t += kBuildThreads) {
+        const int b = t >> 3, q = t & (kGroup - 1);
+        __builtin_nontemporal_store(q < kCodePieces ? code_piece(b, q) : index_piece(b, q), gl + t);
+    }
+    if (crowded) {
+        __syncthreads();   // (and the stores above are done)
+        if (tid < nbeside && s_beside_slot[tid] >= 0) {
+            const int b = s_beside_slot[tid] >> 4, slot = s_beside_slot[tid] & 15;
+            uint64_t* line = m.buckets + static_cast<size_t>(b0 + b) * kBucketQwords;
+            line[slot] = s_beside_code[tid];
+            reinterpret_cast<int32_t*>(line)[kValDword0 + slot] = s_beside_row[tid];
+        }
+    }
+    if constexpr (PROV) {
+        if (tid == 0 && s_losers) atomicAdd(pl.hdr + kHdrLosers, s_losers);
+    }
+}
+
 // Streaming erase, pass 3: one workgroup per partition takes its range of the
 // table into LDS, looks its records up there and frees what it finds: the slot
 // goes back to empty while its bucket has an empty slot left (such a bucket has
@@ -1601,8 +1985,13 @@ int launch_split_and_build(ash_map* map, const BulkPlan& pl, const int32_t* keys
                            int identity, uint64_t* early, int32_t stamp, hipStream_t s) {
     if (pl.once) {
         if (launch_split_once<PROV>(map, pl, keys, identity, early, stamp, s)) return 1;
-        auto build = tombs_in(map) ? build_kernel<PROV, true, true> : build_kernel<PROV, false, true>;
-        build<<<8 * ((pl.parts + 7) / 8), kBuildThreads, 0, s>>>(map->d, pl, stale, identity);
+        const unsigned groups = 8 * ((pl.parts + 7) / 8);
+        if (pl.lists) {
+            build_lists_kernel<PROV><<<groups, kBuildThreads, pl.cap_part * 12, s>>>(map->d, pl, stale);
+        } else {
+            auto build = tombs_in(map) ? build_kernel<PROV, true, true> : build_kernel<PROV, false, true>;
+            build<<<groups, kBuildThreads, 0, s>>>(map->d, pl, stale, identity);
+        }
     } else {
         const int ncursors = static_cast<int>(pl.bins << pl.fine_shift);   // (>= bins << lane_shift)
         const int ninit = ncursors > kHdrWords ? ncursors : kHdrWords;

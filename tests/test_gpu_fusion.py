@@ -397,6 +397,36 @@ def test_activation_from_world_positions_equals_activation_from_cells(gpu_ash):
         direct.close()
 
 
+@pytest.mark.parametrize("n", [255, 3_000, 20_000])
+@pytest.mark.parametrize("far", [False, True])
+def test_activation_of_standing_and_missing_blocks(gpu_ash, n, far):
+    """The same positions into an emptied table, where every block is inserted at once,
+    into the one that stands then, with every third block gone, and emptied again; `far`:
+    blocks whose coordinates do not pack, in the second region."""
+    g = torch.Generator().manual_seed(n)
+    cells = ((torch.rand(n, 3, generator=g).cumsum(0) * 0.4) % 200.0).to(DEV)
+    if far:
+        cells[n // 2:] += 8.0 * (1 << 21)   # (floats hold multiples of two there)
+    grid = gpu_ash.UnBoundedSparseDenseGrid(3, 60_000, 1, 8, cell_size=1.0, device=DEV)
+    want = None
+    for step in ("emptied", "standing", "holes", "emptied"):
+        if step == "holes":
+            grid.engine.erase(want[::3].contiguous())
+        elif step == "emptied":
+            grid.engine.clear()
+        coords, _, rows, _ = grid.spatial_init_(cells, dilation=1, bidirectional=True)
+        coords, rows = coords.view(-1, 3), rows.view(-1)
+        if want is None:
+            base = torch.unique(torch.floor(cells.cpu() / 8).int(), dim=0)
+            around = torch.cartesian_prod(*[torch.arange(-1, 2, dtype=torch.int32)] * 3)
+            want = torch.unique((base.view(-1, 1, 3) + around).view(-1, 3), dim=0).to(DEV)
+        assert torch.equal(torch.unique(coords, dim=0), want) and len(coords) == len(want), step
+        assert grid.engine.size() == len(want), step
+        found, masks = grid.engine.find(coords)
+        assert bool(masks.all()) and torch.equal(found, rows), step
+        assert torch.equal(torch.sort(rows)[0], torch.sort(grid.engine.items()[1])[0]), step
+
+
 @pytest.mark.parametrize("grid_dim,e,bounded", [(8, 2, False), (8, 5, False), (4, 2, True), (8, 2, True)])
 def test_integration_by_flags_equals_integration_by_listing(gpu_ash, grid_dim, e, bounded):
     """ash_grid_integrate_depth_flagged (after ash_grid_activate_positions)

@@ -840,6 +840,7 @@ struct RunsArgs {
     int64_t n;
     int off_lo, width;     // neighbour offsets off_lo .. off_lo + width - 1 per axis
     int bound_lo, bound_hi;
+    bool empty;            // the table holds nothing yet
 };
 
 __device__ __forceinline__ bool block_of_world(const RunsArgs& a, int64_t i,
@@ -864,11 +865,20 @@ constexpr int kDistinctSlots = 2048;     // two LDS slots per candidate of a chu
 // candidates of a workgroup -- some 270 for 128 depth pixels at dilation 1 --
 // name every block twice on average (the neighbourhoods of neighbouring
 // blocks overlap in 18 of 27), so they are first made distinct in an LDS set,
-// which leaves one round of table work per workgroup as a rule.  The insert
+// and then looked up by a lane each, one after the other without a barrier in
+// between: a block that stands, which is what a frame mostly meets, is flagged there
+// and then, once the key log confirms its index.  (A table that has been emptied and not
+// used since holds none: frames of 640 x 480 and 1200 x 900 into such a one 52 and 100
+// us, 54 and 111 with the look.)  What is left is inserted.  The insert
 // reports the index of every key it can be sure of (insert_key, kInsertReport)
 // and the row is flagged at once; a key that another thread is storing at
 // that moment is flagged by that thread, which is handed the index.  No second
 // launch has to wait for the indices to settle.
+//
+// A chain of waits; VGA frame, 791 workgroups of some 240 distinct blocks (us): every
+// block through the insert, which a third of the workgroups entered twice, 14.3; as it
+// is 11.6.  512 threads, one round for everybody: 16, the registers of the insert leave
+// room for half of the workgroups; 128 and 64 positions 16.6 and 23.
 template <bool TOMBS>
 __global__ __launch_bounds__(kHeapBlock) void activate_runs_kernel(
         MapDev m, RunsArgs a, uint8_t* __restrict__ touched, int32_t* __restrict__ coords) {
@@ -877,6 +887,7 @@ __global__ __launch_bounds__(kHeapBlock) void activate_runs_kernel(
     __shared__ int32_t s_heads[kRunPositions * 3];
     __shared__ int s_wave[kRunPositions / 64];
     __shared__ int s_ncand;
+    __shared__ int s_nmissing;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int64_t i = static_cast<int64_t>(blockIdx.x) * kRunPositions + threadIdx.x;
@@ -909,9 +920,15 @@ __global__ __launch_bounds__(kHeapBlock) void activate_runs_kernel(
     const int per_head = a.width * a.width * a.width;
     const int total = nh * per_head;   // the same for every thread of the workgroup
     const ValueArgs none = {};
+    auto flag = [&](int32_t row, const int32_t (&k)[3]) {
+        touched[row] = 1;
+        coords[static_cast<int64_t>(row) * 3 + 0] = k[0];
+        coords[static_cast<int64_t>(row) * 3 + 1] = k[1];
+        coords[static_cast<int64_t>(row) * 3 + 2] = k[2];
+    };
     for (int first = 0; first < total; first += kCandChunk) {
         for (int q = threadIdx.x; q < kDistinctSlots; q += kHeapBlock) s_set[q] = kEmpty;
-        if (threadIdx.x == 0) s_ncand = 0;
+        if (threadIdx.x == 0) s_ncand = s_nmissing = 0;
         __syncthreads();   // (also: s_heads is complete, the rounds below are over)
         const int end = total - first < kCandChunk ? total : first + kCandChunk;
         for (int t = first + threadIdx.x; t < end; t += kHeapBlock) {
@@ -946,11 +963,31 @@ __global__ __launch_bounds__(kHeapBlock) void activate_runs_kernel(
         }
         __syncthreads();
         const int distinct = s_ncand;
-        for (int r0 = 0; r0 < distinct; r0 += kHeapBlock) {
-            const int t = r0 + threadIdx.x;
-            const bool ok = t < distinct;
+        // blocks that stand, and whose index is certain, are flagged by whoever looks
+        // them up; the others, none as a rule, are listed (over the set, which is done with)
+        int32_t* const s_missing = reinterpret_cast<int32_t*>(s_set);
+        for (int t = threadIdx.x; t < (a.empty ? 0 : distinct); t += kHeapBlock) {
+            const int32_t k[3] = {s_cand[t * 3 + 0], s_cand[t * 3 + 1], s_cand[t * 3 + 2]};
+            uint64_t code;
+            const bool fits = pack_key<3>(k, code);
+            int32_t row = -1;
+            bool stands = find_key_alone<3>(m, k, true, row);
+            if (stands && fits) {
+                stands = static_cast<uint32_t>(row) < static_cast<uint32_t>(m.capacity) && m.klog[row] == code;
+            }
+            if (stands) {
+                flag(row, k);
+            } else {
+                s_missing[atomicAdd(&s_nmissing, 1)] = t;
+            }
+        }
+        __syncthreads();
+        const int missing = a.empty ? distinct : s_nmissing;
+        for (int r0 = 0; r0 < missing; r0 += kHeapBlock) {
+            const bool ok = r0 + static_cast<int>(threadIdx.x) < missing;
             int32_t k[3] = {0, 0, 0};
             if (ok) {
+                const int t = a.empty ? r0 + static_cast<int>(threadIdx.x) : s_missing[r0 + threadIdx.x];
                 k[0] = s_cand[t * 3 + 0];
                 k[1] = s_cand[t * 3 + 1];
                 k[2] = s_cand[t * 3 + 2];
@@ -959,12 +996,7 @@ __global__ __launch_bounds__(kHeapBlock) void activate_runs_kernel(
             const bool fits = pack_key<3>(k, code);
             int32_t row = -1;
             insert_key<3, kInsertReport, TOMBS>(m, k, code, fits, 0, ok, none, nullptr, nullptr, &row);
-            if (ok && row >= 0) {
-                touched[row] = 1;
-                coords[static_cast<int64_t>(row) * 3 + 0] = k[0];
-                coords[static_cast<int64_t>(row) * 3 + 1] = k[1];
-                coords[static_cast<int64_t>(row) * 3 + 2] = k[2];
-            }
+            if (ok && row >= 0) flag(row, k);
             __syncthreads();   // insert_key's own words are rewritten by the next round
         }
     }
@@ -3344,6 +3376,7 @@ int ash_grid_activate_positions(ash_map_t* map, const float* positions, int64_t 
     DeviceGuard guard;
     ASH_HIP(guard.enter(map->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
+    const bool empty = map->table_stale;
     if (settle_table(map, s)) return 1;
     Change change(map, kChangeAdds, s);
     RunsArgs a;
@@ -3356,6 +3389,7 @@ int ash_grid_activate_positions(ash_map_t* map, const float* positions, int64_t 
     a.width = dilation - a.off_lo + 1;
     a.bound_lo = bound_lo;
     a.bound_hi = bound_hi;
+    a.empty = empty;
     const int64_t groups = (n + kRunPositions - 1) / kRunPositions;
     if (groups > 0x7FFFFFFFll) ASH_FAIL("too many positions in one call");
     auto kernel = tombs_in(map) ? activate_runs_kernel<true> : activate_runs_kernel<false>;

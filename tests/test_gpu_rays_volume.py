@@ -36,3 +36,38 @@ def test_same_rays_with_and_without(gpu_ash, bounds, n):
         assert len(plain[0]) > n
         grid.engine.erase(keys[1000:3000])
         grid.engine.insert_keys(keys[4000:])
+
+
+@pytest.mark.parametrize("n", [8195, 66_000])
+@pytest.mark.parametrize("far_block", [None, (40, 3, 5), (2**31 - 1, 0, 4)])
+def test_rays_that_leave_the_volume(gpu_ash, far_block, n):
+    """Ranges far beyond the grid (of rays that meet nothing), rays that are not finite,
+    and the word that says whether a block is stored out there: all in bounds, one
+    beyond them in the table, one in the second region."""
+    grid = gpu_ash.BoundedSparseDenseGrid(3, 3000, 1, 8, 32, device=DEV)
+    backend, table = gpu_ash.grid.backend, grid.engine.backend
+    g = torch.Generator().manual_seed(n)
+    grid.engine.insert_keys(torch.randint(0, 32, (2500, 3), generator=g).int().to(DEV))
+    if far_block is not None:
+        grid.engine.insert_keys(torch.tensor([far_block], dtype=torch.int32, device=DEV))
+    o = torch.rand(n, 3, generator=g) * 256
+    d = torch.nn.functional.normalize(torch.randn(n, 3, generator=g), dim=1)
+    target = torch.tensor([40.0, 3, 5]) * 8 + 4
+    d[::3] = torch.nn.functional.normalize(target - o[::3], dim=1)
+    nan, inf = float("nan"), float("inf")
+    d[:6] = torch.tensor([[0, 0, 0], [nan, 0, 1], [inf, 0, 1], [0, -inf, 0], [1e-3, 0, 0], [3e38, 0, -3e38]])
+    o[6:9] = torch.tensor([[nan, 1, 1], [-inf, 1, 1], [1, 3e38, 1]])
+    o, d = o.to(DEV), d.to(DEV)
+    near = torch.where(torch.arange(n) % 2 == 0, -1.0, 20.0).to(DEV)
+    far = torch.where(torch.arange(n) % 5 == 0, 60.0, 2000.0).to(DEV)
+    near[9], far[10], near[11], far[12] = nan, nan, -inf, inf
+    wide = [torch.full((3,), x, device=DEV) for x in (-inf, inf)]
+    for box in ([torch.zeros(3, device=DEV), torch.full((3,), 256.0, device=DEV)], wide):
+        args = (table, o, d, None, 1.0, *box, 0.0, 800.0, 8.0)
+        for a, b in zip(backend.ray_find_near_far_world(*args), backend.ray_find_near_far_world(*args, (0, 31))):
+            assert torch.equal(a, b)
+    args = (table, o, d, None, 1.0, near, far, 128, 8.0)
+    plain = backend.ray_sample_world(*args)
+    for a, b in zip(plain, backend.ray_sample_world(*args, (0, 31))):
+        assert a.dtype == b.dtype and torch.equal(torch.nan_to_num(a), torch.nan_to_num(b))
+    assert len(plain[0]) > n // 2   # (a block in thirteen is stored)

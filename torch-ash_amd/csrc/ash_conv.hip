@@ -57,13 +57,27 @@ struct Shape {
         return p;
     }
     static constexpr int kLayer = layer();
-    static constexpr int kPlane = kLayer * kT;
-    // results on their way out: a z layer's rows, four words apart from the next
-    // layer's (banks)
-    static constexpr int kOutLayer = 64 * E + 4;
+    // and between the planes of two channels: what makes the fewest lanes meet at a bank
+    // where a block's rows are put into the tile, counted for each shape over the places
+    // below (cycles of a block, without and with: five channels, 3^3, 382 -> 366, 5^3 1068
+    // -> 570, 7^3 1445 -> 908; eight channels 600 -> 450, 1728 -> 720, 1960 -> 1078).
+    static constexpr int plane_gap() {
+        constexpr int kGap[3][8] = {{0, 0, 30, 8, 18, 4, 2, 4},
+                                    {0, 16, 4, 8, 4, 4, 18, 4},
+                                    {0, 0, 30, 8, 2, 2, 30, 4}};
+        return kGap[kR - 1][E - 1];
+    }
+    static constexpr int kPlane = kLayer * kT + plane_gap();
+    // results on their way out: a z layer's rows, some words apart from the next
+    // layer's (banks: a wavefront writes a word of eight cells in eight layers, 16
+    // cycles for eight of these with five channels and a gap of eight, 32 with four)
+    static constexpr int kOutLayer = 64 * E + (E % 4 == 0 ? 4 : 8);
     static constexpr int kTileWords = E * kPlane;
     static constexpr int kOutWords = kG * kOutLayer;
-    static constexpr int kWeightWords = E * W * 64;
+    // The taps of a 3^3 window stay in scalar registers; those of the others are read
+    // from LDS, a lane each, and handed out lane by lane (one instruction per tap).
+    static constexpr bool kTapsHeld = W == 3;
+    static constexpr int kWeightWords = kTapsHeld ? 0 : E * W * 64;
     static constexpr int kFit = 160 * 1024 / (4 * (kTileWords + kOutWords + kWeightWords) + 1024);
     // Cells along y per lane, and with them wavefronts per channel.  Two per
     // channel, but for odd numbers of channels, where that is no multiple of the
@@ -81,10 +95,14 @@ struct Shape {
     static constexpr int kParts = kG / kY;
     static constexpr int kWorkers = E * kParts;                    // wavefronts that compute
     static constexpr int kThreads = 64 * (kOneEach ? (kWorkers + 3) / 4 * 4 : kWorkers);
-    static constexpr int kPieces = kM * E / 4;                     // of 16 bytes, a block's own rows
-    static constexpr int kOwnEach = (kPieces + kThreads - 1) / kThreads;   // per thread
-    static constexpr int kHalo = kT * kT * kT - kM;               // rows
-    static constexpr int kHaloEach = (kHalo * E + kThreads - 1) / kThreads;   // elements per thread
+    static constexpr int kOwnPieces = kM * E / 4;                  // of 16 bytes, a block's own rows
+    static constexpr int kOwnEach = (kOwnPieces + kThreads - 1) / kThreads;   // per thread
+    // the tile: kT * kT lines of eight cells along x, of 2 E pieces, and at either
+    // end of a line kR cells, word by word
+    static constexpr int kPieces = kT * kT * 2 * E;
+    static constexpr int kPiecesEach = (kPieces + kThreads - 1) / kThreads;
+    static constexpr int kEnds = 2 * kR * kT * kT * E;
+    static constexpr int kEndsEach = (kEnds + kThreads - 1) / kThreads;
     static constexpr int kTaps = W * W;                           // of one dz
     // wavefronts per SIMD that the tile leaves room for.  No more than the
     // registers allow: 64 for windows of 3 and 72 - 80 for 5 are eight and six, 108
@@ -94,7 +112,9 @@ struct Shape {
     // blocks 33.8 -> 30.7 us, 1000 40 -> 40, 3000 81 -> 82, 6000 129 -> 125, 12 000
     // 241 -> 222, 25 000 495 -> 457; four and six channels 165 -> 151 and 281 -> 244
     // at 12 000 without spilling, the others alike.
-    static constexpr int kMostWaves = W == 3 ? 8 : (W == 5 ? 6 : 4);
+    // Windows of 3 whose workgroups are a wavefront per SIMD: six (40 000 blocks of
+    // one to three channels with eight 44, 75, 130 us, with five to seven 44, 73 - 75, 108).
+    static constexpr int kMostWaves = W == 3 ? (kThreads <= 256 ? 6 : 8) : (W == 5 ? 6 : 4);
     static constexpr int waves() {
         const int each = (kThreads / 64 + 3) / 4;   // of one workgroup
         const int fit = kFit < kMostWaves / each ? kFit : kMostWaves / each;
@@ -119,8 +139,8 @@ convolution_block8_kernel(ConvArgs a) {
     typedef float v4 __attribute__((ext_vector_type(4)));
     __shared__ __align__(16) float s_tile[S::kTileWords];
     __shared__ __align__(16) float s_out[S::kOutWords];
-    __shared__ float s_w[S::kWeightWords];
-    __shared__ int32_t s_nb[2][28];   // rows of the 27 neighbour blocks, and the block's own
+    __shared__ float s_w[S::kTapsHeld ? 1 : S::kWeightWords];
+    __shared__ uint32_t s_nb[2][28];   // where the rows of the 27 neighbour blocks start, and the block's own
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -128,75 +148,62 @@ convolution_block8_kernel(ConvArgs a) {
     const int y0 = wave % S::kParts * S::kY;     // and the first of its cells along y
     constexpr int R = S::kR, T = S::kT, kY = S::kY;
 
-    // weights by channel and dz, one tap per lane
-    for (int t = tid; t < S::kWeightWords; t += S::kThreads) {
-        const int tap = t & 63;
-        const int dz = (t >> 6) % W;
-        const int ch = (t >> 6) / W;
-        s_w[t] = tap < S::kTaps ? a.w[(dz * S::kTaps + tap) * E + ch] : 0.f;
-    }
-    // Where this thread's elements of the block's own rows go in the tile
-    uint32_t own_dst[S::kOwnEach][2];   // two 16-bit places per word
+    // weights by channel and dz: one tap per lane, or all of the wavefront's channel
+    float held[S::kTapsHeld ? W * W * W : 1];
+    if constexpr (S::kTapsHeld) {
+        const int ch = wave < S::kWorkers ? q : 0;
 #pragma unroll
-    for (int i = 0; i < S::kOwnEach; ++i) {
+        for (int k = 0; k < W * W * W; ++k) {
+            held[k] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(a.w[k * E + ch])));
+        }
+    } else {
+        for (int t = tid; t < S::kWeightWords; t += S::kThreads) {
+            const int tap = t & 63;
+            const int dz = (t >> 6) % W;
+            const int ch = (t >> 6) / W;
+            s_w[t] = tap < S::kTaps ? a.w[(dz * S::kTaps + tap) * E + ch] : 0.f;
+        }
+    }
+    // Along y or z: the block that tile coordinate `at` lies in (0, 1, 2: the block
+    // before, the own, the next), and the cell there.
+    auto block_at = [](int at) { return at < R ? 0 : (at >= R + kG ? 2 : 1); };
+    auto cell_at = [](int at) { return (at - R + kG) % kG; };
+    // This thread's pieces: neighbour << 14 | byte within that block's rows, and where
+    // the four words go in the tile, two 16-bit places per register.
+    uint32_t piece_src[S::kPiecesEach], piece_dst[S::kPiecesEach][2];
+#pragma unroll
+    for (int i = 0; i < S::kPiecesEach; ++i) {
+        const int p = tid + i * S::kThreads < S::kPieces ? tid + i * S::kThreads : S::kPieces - 1;
+        const int line = p / (2 * E), part = p - line * (2 * E);
+        const int y = line % T, z = line / T;
         uint32_t place[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            const int e = 4 * (tid + i * S::kThreads) + c;
+            const int e = 4 * part + c;
             const int cell = e / E;
-            place[c] = static_cast<uint32_t>((e - cell * E) * S::kPlane + (cell & 7) + R +
-                                             T * (((cell >> 3) & 7) + R) +
-                                             S::kLayer * ((cell >> 6) + R));
+            place[c] = static_cast<uint32_t>((e - cell * E) * S::kPlane + cell + R + T * y + S::kLayer * z);
         }
-        own_dst[i][0] = place[0] | (place[1] << 16);
-        own_dst[i][1] = place[2] | (place[3] << 16);
+        piece_dst[i][0] = place[0] | (place[1] << 16);
+        piece_dst[i][1] = place[2] | (place[3] << 16);
+        const int nb = 1 + 3 * block_at(y) + 9 * block_at(z);
+        piece_src[i] = (static_cast<uint32_t>(nb == 13 ? 27 : nb) << 14) |
+                       static_cast<uint32_t>((kG * cell_at(y) + kG * kG * cell_at(z)) * E * 4 + 16 * part);
     }
-    // and its elements of the halo: place in the tile << 17 | neighbour << 12 |
+    // and its words of the lines' ends: place in the tile << 17 | neighbour << 12 |
     // word within that block's rows
-    constexpr uint32_t kNone = 0xFFFFFFFFu;
-    uint32_t halo[S::kHaloEach];
+    uint32_t ends[S::kEndsEach];
 #pragma unroll
-    for (int i = 0; i < S::kHaloEach; ++i) {
-        const int h = tid + i * S::kThreads;
-        halo[i] = kNone;
-        if (h < S::kHalo * E) {
-            int p = h / E;
-            const int ch = h - p * E;
-            int at[3];   // tile coordinates of the p-th row of the halo
-            constexpr int kSlab = T * T, kRing = T * T - kG * kG;
-            if (p < 2 * R * kSlab) {
-                at[2] = p / kSlab;
-                if (at[2] >= R) at[2] += kG;
-                p %= kSlab;
-                at[1] = p / T;
-                at[0] = p % T;
-            } else {
-                p -= 2 * R * kSlab;
-                at[2] = R + p / kRing;
-                p %= kRing;
-                if (p < 2 * R * T) {
-                    at[1] = p / T;
-                    if (at[1] >= R) at[1] += kG;
-                    at[0] = p % T;
-                } else {
-                    p -= 2 * R * T;
-                    at[1] = R + p / (2 * R);
-                    at[0] = p % (2 * R);
-                    if (at[0] >= R) at[0] += kG;
-                }
-            }
-            int nb = 0, cell = 0, step3 = 1, step8 = 1;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                const int b = at[d] < R ? -1 : (at[d] >= R + kG ? 1 : 0);
-                nb += (b + 1) * step3;
-                cell += (at[d] - R - b * kG) * step8;
-                step3 *= 3;
-                step8 *= kG;
-            }
-            halo[i] = (static_cast<uint32_t>(ch * S::kPlane + at[0] + T * at[1] + S::kLayer * at[2]) << 17) |
-                      static_cast<uint32_t>(nb << 12) | static_cast<uint32_t>(cell * E + ch);
-        }
+    for (int i = 0; i < S::kEndsEach; ++i) {
+        const int h = tid + i * S::kThreads < S::kEnds ? tid + i * S::kThreads : S::kEnds - 1;
+        const int p = h / E, ch = h - p * E;
+        const int line = p / (2 * R);
+        const int y = line % T, z = line / T;
+        int x = p % (2 * R);
+        if (x >= R) x += kG;
+        const int nb = block_at(x) + 3 * block_at(y) + 9 * block_at(z);
+        const int cell = cell_at(x) + kG * cell_at(y) + kG * kG * cell_at(z);
+        ends[i] = (static_cast<uint32_t>(ch * S::kPlane + x + T * y + S::kLayer * z) << 17) |
+                  static_cast<uint32_t>(nb << 12) | static_cast<uint32_t>(cell * E + ch);
     }
 
     const TileWalk walk(a.n_grids);
@@ -208,30 +215,26 @@ convolution_block8_kernel(ConvArgs a) {
         const int64_t row = a.lut_g[g * 27 + tid];
         return (row >= 0 && row < a.B) ? static_cast<int32_t>(row) : -1;
     };
-    // (byte offsets fit 32 bits: the tensors are below 4 GiB, which the host
-    // checks; one register per address and no 64-bit arithmetic.  Words of
-    // missing blocks are read from the start of the tensor and dropped.)
-    v4 own[S::kOwnEach];
-    float ring[S::kHaloEach];
-    uint64_t have = 0;   // bit i: ring[i] holds a word of a stored block
-    const char* const in = reinterpret_cast<const char*>(a.in);
-    constexpr uint32_t kBlockBytes = kM * E * 4;
-    auto load_block = [&](const int32_t* nb) {
-        const uint32_t g = nb[27] < 0 ? 0u : static_cast<uint32_t>(nb[27]);
+    // Byte offsets fit 32 bits: the host sees to it that one block more would still be
+    // below 4 GiB, and a missing block's rows stand there, beyond the tensor, where the
+    // loads give zeros by themselves.
+    constexpr uint32_t kBlockBytes = kM * E * 4, kMissing = 0u - kBlockBytes;
+    auto start_of = [&](int32_t row) { return row < 0 ? kMissing : static_cast<uint32_t>(row) * kBlockBytes; };
+    const auto in = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.in), 0,
+                                                      static_cast<int>(static_cast<uint32_t>(a.B) * kBlockBytes),
+                                                      0x00020000);
+    v4 piece[S::kPiecesEach];
+    float end[S::kEndsEach];
+    auto load_block = [&](const uint32_t* nb) {
 #pragma unroll
-        for (int i = 0; i < S::kOwnEach; ++i) {
-            const int piece = tid + i * S::kThreads;
-            if (S::kPieces % S::kThreads == 0 || piece < S::kPieces) {
-                own[i] = *reinterpret_cast<const v4*>(in + (g * kBlockBytes + 16u * static_cast<uint32_t>(piece)));
-            }
+        for (int i = 0; i < S::kPiecesEach; ++i) {
+            const uint32_t at = nb[piece_src[i] >> 14] + (piece_src[i] & 0x3FFFu);
+            piece[i] = __builtin_bit_cast(v4, __builtin_amdgcn_raw_buffer_load_b128(in, static_cast<int>(at), 0, 0));
         }
-        have = 0;
 #pragma unroll
-        for (int i = 0; i < S::kHaloEach; ++i) {
-            const int32_t row = halo[i] == kNone ? -1 : nb[(halo[i] >> 12) & 31u];
-            const uint32_t at = row < 0 ? 0u : static_cast<uint32_t>(row) * kBlockBytes + (halo[i] & 0xFFFu) * 4u;
-            if (row >= 0) have |= uint64_t{1} << i;
-            ring[i] = *reinterpret_cast<const float*>(in + at);
+        for (int i = 0; i < S::kEndsEach; ++i) {
+            const uint32_t at = nb[(ends[i] >> 12) & 31u] + (ends[i] & 0xFFFu) * 4u;
+            end[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(in, static_cast<int>(at), 0, 0));
         }
     };
 
@@ -256,13 +259,13 @@ convolution_block8_kernel(ConvArgs a) {
         for (int j = 0; j < bare; ++j) {
             v4* rows = reinterpret_cast<v4*>(a.out) +
                        static_cast<uint64_t>(static_cast<uint32_t>(s_bare[j])) * (kM * E / 4);
-            for (int f = tid; f < S::kPieces; f += S::kThreads) {
+            for (int f = tid; f < S::kOwnPieces; f += S::kThreads) {
                 __builtin_nontemporal_store(v4{0.f, 0.f, 0.f, 0.f}, rows + f);
             }
         }
         __syncthreads();   // the list is written again by the next round
     }
-    if (tid <= 27) s_nb[0][tid] = rows_reg;
+    if (tid <= 27) s_nb[0][tid] = start_of(rows_reg);
     rows_reg = fetch_rows(blk + walk.step);
     __syncthreads();
     if (blk < walk.end) load_block(s_nb[0]);
@@ -271,18 +274,19 @@ convolution_block8_kernel(ConvArgs a) {
     float* const result = s_out + (x + kG * y0) * E + z * S::kOutLayer + q;
 
     for (; blk < walk.end; blk += walk.step, buf ^= 1) {
-        const int32_t g = s_nb[buf][27];
+        const uint32_t own = s_nb[buf][27];
 #pragma unroll
-        for (int i = 0; i < S::kOwnEach; ++i) {
+        for (int i = 0; i < S::kPiecesEach; ++i) {
             if (S::kPieces % S::kThreads != 0 && tid + i * S::kThreads >= S::kPieces) continue;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) s_tile[(own_dst[i][c >> 1] >> (16 * (c & 1))) & 0xFFFFu] = own[i][c];
+            for (int c = 0; c < 4; ++c) s_tile[(piece_dst[i][c >> 1] >> (16 * (c & 1))) & 0xFFFFu] = piece[i][c];
         }
 #pragma unroll
-        for (int i = 0; i < S::kHaloEach; ++i) {
-            if (halo[i] != kNone) s_tile[halo[i] >> 17] = ((have >> i) & 1u) ? ring[i] : 0.f;
+        for (int i = 0; i < S::kEndsEach; ++i) {
+            if (S::kEnds % S::kThreads != 0 && tid + i * S::kThreads >= S::kEnds) continue;
+            s_tile[ends[i] >> 17] = end[i];
         }
-        if (tid <= 27) s_nb[buf ^ 1][tid] = rows_reg;
+        if (tid <= 27) s_nb[buf ^ 1][tid] = start_of(rows_reg);
         __syncthreads();   // the tile is complete
         rows_reg = fetch_rows(blk + 2 * walk.step);
         if (blk + walk.step < walk.end) load_block(s_nb[buf ^ 1]);
@@ -291,10 +295,8 @@ convolution_block8_kernel(ConvArgs a) {
             float acc[kY];
 #pragma unroll
             for (int j = 0; j < kY; ++j) acc[j] = 0.f;
-#pragma unroll 1
-            for (int dz = 0; dz < W; ++dz) {
-                const float* layer = window + S::kLayer * dz;
-                const float taps = s_w[(q * W + dz) * 64 + lane];
+            // one layer of the window, tap(k) the k-th weight of it
+            auto add_layer = [&](const float* layer, auto tap) {
 #pragma unroll
                 for (int y = 0; y < kY + 2 * R; ++y) {
                     float row[W];
@@ -305,28 +307,37 @@ convolution_block8_kernel(ConvArgs a) {
                         const int dy = y - j;
                         if (dy < 0 || dy >= W) continue;
 #pragma unroll
-                        for (int dx = 0; dx < W; ++dx) {
-                            const float tap = __int_as_float(
-                                    __builtin_amdgcn_readlane(__float_as_int(taps), dy * W + dx));
-                            acc[j] = fmaf(row[dx], tap, acc[j]);
-                        }
+                        for (int dx = 0; dx < W; ++dx) acc[j] = fmaf(row[dx], tap(dy * W + dx), acc[j]);
                     }
+                }
+            };
+            if constexpr (S::kTapsHeld) {
+#pragma unroll
+                for (int dz = 0; dz < W; ++dz) {
+                    add_layer(window + S::kLayer * dz, [&](int k) { return held[dz * S::kTaps + k]; });
+                }
+            } else {
+#pragma unroll 1
+                for (int dz = 0; dz < W; ++dz) {
+                    const float taps = s_w[(q * W + dz) * 64 + lane];
+                    add_layer(window + S::kLayer * dz, [&](int k) {
+                        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(taps), k));
+                    });
                 }
             }
 #pragma unroll
             for (int j = 0; j < kY; ++j) result[j * kG * E] = acc[j];
         }
         __syncthreads();   // the results are complete, and the tile has been read
-        if (g >= 0) {
-            v4* rows = reinterpret_cast<v4*>(a.out) +
-                       static_cast<uint64_t>(static_cast<uint32_t>(g)) * (kM * E / 4);
+        if (own != kMissing) {
+            v4* rows = reinterpret_cast<v4*>(reinterpret_cast<char*>(a.out) + own);
 #pragma unroll
             for (int i = 0; i < S::kOwnEach; ++i) {
                 const int f = tid + i * S::kThreads;
-                if (S::kPieces % S::kThreads != 0 && f >= S::kPieces) continue;
+                if (S::kOwnPieces % S::kThreads != 0 && f >= S::kOwnPieces) continue;
                 const int out_z = f / (16 * E);
-                __builtin_nontemporal_store(*reinterpret_cast<const v4*>(s_out + 4 * f + 4 * out_z),
-                                            rows + f);
+                __builtin_nontemporal_store(
+                        *reinterpret_cast<const v4*>(s_out + 4 * f + (S::kOutLayer - 64 * E) * out_z), rows + f);
             }
         }
     }
@@ -380,7 +391,7 @@ int ash_convolution_cube_supported(int64_t num_embeddings, int grid_dim, int win
                                    int64_t embedding_dim, int32_t dtype) {
     return dtype == ASH_F32 && grid_dim == kG && (window == 3 || window == 5 || window == 7) &&
            embedding_dim >= 1 && embedding_dim <= kMaxChannels && num_embeddings >= 1 &&
-           num_embeddings * embedding_dim * kM * 4 <= 0xFFFFFFFFll;
+           (num_embeddings + 1) * embedding_dim * kM * 4 <= 0x100000000ll;   // (kMissing)
 }
 
 int ash_convolution_cube(const void* inputs, const void* weights, const int64_t* grid_indices,

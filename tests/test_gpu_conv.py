@@ -291,3 +291,22 @@ def test_other_block_edges(gpu_ash, oracle, grid_dim, radius, channels, monkeypa
                                                    grid_dim)
     ref = oracle.convolution_forward(inputs, weights, masks, gi, ci, g2g, c2c, c2g, grid_dim)
     assert torch.equal(out.cpu(), ref) and float(ref.abs().max()) > 1.0
+
+
+@pytest.mark.parametrize("radius", [1, 2, 3])
+@pytest.mark.parametrize("channels", [1, 2, 3, 4, 5, 6, 7, 8])
+def test_every_width_of_rows_and_window(gpu_ash, oracle, channels, radius):
+    """Each has places of its own for a block's pieces and its lines' ends; blocks at the
+    two ends of the tensor, so that missing neighbours stand beyond it on either side."""
+    grid, _, _ = workloads.build_grid(gpu_ash, 90, channels, 8, 16, device=DEV)
+    g = torch.Generator().manual_seed(900 + 10 * channels + radius)
+    inputs = torch.randn(grid.embeddings.shape, generator=g).to(DEV)
+    size = 2 * radius + 1
+    weights = torch.randn(size, size, size, channels, generator=g).to(DEV)
+    out = grid.convolution(inputs, weights)
+    c2g, c2c, g2g, gi, ci = _tables(grid, radius)
+    masks = torch.ones(inputs.shape[:2], dtype=torch.bool)
+    ref = oracle.convolution_forward(inputs, weights.view(size**3, channels), masks, gi, ci,
+                                     g2g, c2c, c2g, 8)
+    assert bool((g2g[gi.view(-1)] < 0).any())
+    assert torch.equal(out.cpu(), ref)

@@ -37,3 +37,22 @@ def test_same_table_as_the_general_path(gpu_ash, blocks, far, erased, radius, bi
     assert coords.dtype == want_coords.dtype and lut.dtype == want_lut.dtype
     assert torch.equal(coords, want_coords) and torch.equal(lut, want_lut)
     assert int((lut[:, 0] >= 0).sum()) > 0 or radius > 0 or blocks == 0
+
+
+@pytest.mark.parametrize("blocks", [31, 64, 700])   # 27 offsets: shares that end within a row, within and at a wavefront
+def test_one_sided_window_of_three(gpu_ash, blocks):
+    """The width of the two-sided window of one, from another first offset."""
+    grid = gpu_ash.UnBoundedSparseDenseGrid(3, 901, 1, 2, device=DEV)
+    g = torch.Generator().manual_seed(blocks)
+    grid.engine.insert_keys(torch.randint(-6, 6, (blocks, 3), generator=g).int().to(DEV))
+    coords, lut = grid.construct_grid_neighbor_lut(2, False)
+    keys, indices = (t.cpu() for t in grid.engine.items())
+    index = {tuple(k): int(i) for k, i in zip(keys.tolist(), indices)}
+    coords, lut = coords.cpu(), lut.cpu()
+    want = torch.full_like(lut, -1)
+    for key, i in index.items():
+        assert tuple(coords[i].tolist()) == key
+        for n in range(27):
+            there = tuple(key[d] + n // 3**d % 3 for d in range(3))
+            want[i, n] = index.get(there, -1)
+    assert torch.equal(lut, want)

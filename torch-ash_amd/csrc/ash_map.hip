@@ -1310,8 +1310,12 @@ __global__ __launch_bounds__(kBlock) void items_general_kernel(
 // keys, their find and the scattering of both): a lane per row and offset, the
 // row's key from the log, `width`^3 offsets with the first axis fastest, each
 // `pad` less than its digit.  Rows without a key and offsets without a stored
-// neighbour get -1.  Bound by the find's random lines (60 000 blocks of a surface,
-// 8 offsets: 80 us and 26 launches before, 17 now).
+// neighbour get -1.  A lane looks its neighbour up by itself, and the widths of the
+// functions here are constants of their own: bound by vector instructions, of which the
+// cooperative probe and divisions by a width from memory were the most (752 of a wavefront;
+// 60 000 blocks of a surface, 8 offsets 15.3 -> 9.1 us, 27 offsets 34.7 -> 23.8; 200 000
+// blocks 37 -> 25 and 106 -> 80; a million scattered ones, lines from behind the L2s, 197
+// -> 123 and 657 -> 431; by a listing, a find and the scattering of both 80 us for the first).
 struct NeighborArgs {
     int32_t* coords;   // [rows, 3]
     int64_t* lut;      // [rows, width^3]
@@ -1319,10 +1323,12 @@ struct NeighborArgs {
     int width, pad;
 };
 
-// every lane of the wavefront calls this together; lane `k` of row i
+// every lane of the wavefront calls this together; lane `k` of row i.  WIDTH: the
+// width, where it is not 0.
+template <int WIDTH>
 __device__ __forceinline__ void write_neighbor(const MapDev& m, const NeighborArgs& a, bool write,
                                                bool live, int64_t i, uint32_t k, const int32_t (&key)[3]) {
-    const uint32_t w = static_cast<uint32_t>(a.width);
+    const uint32_t w = static_cast<uint32_t>(WIDTH > 0 ? WIDTH : a.width);
     const uint32_t digit[3] = {k % w, k / w % w, k / w / w};
     int32_t other[3];
     bool self = true;
@@ -1333,7 +1339,7 @@ __device__ __forceinline__ void write_neighbor(const MapDev& m, const NeighborAr
         other[d] = static_cast<int32_t>(static_cast<uint32_t>(key[d]) + static_cast<uint32_t>(o));
     }
     int32_t res = 0;
-    const bool found = find_key<3>(m, other, live && !self, res);
+    const bool found = find_key_alone<3>(m, other, live && !self, res);
     if (!write) return;
     a.lut[i * (w * w * w) + k] = live && self ? i : (found ? static_cast<int64_t>(res) : -1);
     if (k == 0) {
@@ -1343,26 +1349,29 @@ __device__ __forceinline__ void write_neighbor(const MapDev& m, const NeighborAr
 }
 
 // Share `block` of a workgroup: kBlock consecutive (row, offset) pairs.
+template <int WIDTH>
 __device__ __forceinline__ void row_and_offset(const NeighborArgs& a, int64_t block, int64_t& i,
                                                uint32_t& k) {
-    const uint32_t n = static_cast<uint32_t>(a.width * a.width * a.width);
+    const int w = WIDTH > 0 ? WIDTH : a.width;
+    const uint32_t n = static_cast<uint32_t>(w * w * w);
     const int64_t base = block * kBlock;
     const uint32_t local = static_cast<uint32_t>(base % n) + threadIdx.x;
     i = base / n + local / n;
     k = local % n;
 }
 
+template <int WIDTH>
 __global__ __launch_bounds__(kBlock) void neighbors_kernel(MapDev m, NeighborArgs a, int identity) {
     const int64_t limit = identity ? static_cast<int64_t>(m.ctr[kCtrSize])
                                    : static_cast<int64_t>(m.capacity);
     int64_t i;
     uint32_t k;
-    row_and_offset(a, blockIdx.x, i, k);
+    row_and_offset<WIDTH>(a, blockIdx.x, i, k);
     const uint64_t code = i < limit && i < a.rows ? m.klog[i] : kEmpty;
     const bool live = code < kTomb;
     int32_t key[3] = {0, 0, 0};
     if (live) unpack_key<3>(code, key);
-    write_neighbor(m, a, i < a.rows, live, i, k, key);
+    write_neighbor<WIDTH>(m, a, i < a.rows, live, i, k, key);
 }
 
 // The same for the keys of the general region, behind it.
@@ -1371,7 +1380,7 @@ __global__ __launch_bounds__(kBlock) void neighbors_general_kernel(MapDev m, Nei
     for (int64_t share = blockIdx.x; share < shares; share += gridDim.x) {
         int64_t p;
         uint32_t k;
-        row_and_offset(a, share, p, k);
+        row_and_offset<0>(a, share, p, k);
         const int32_t i = p < m.gslots ? m.gstate[p] : kGenEmpty;
         const bool live = i >= 0 && i < a.rows;
         int32_t key[3] = {0, 0, 0};
@@ -1379,7 +1388,7 @@ __global__ __launch_bounds__(kBlock) void neighbors_general_kernel(MapDev m, Nei
 #pragma unroll
             for (int d = 0; d < 3; ++d) key[d] = m.gkeys[static_cast<size_t>(p) * 4 + d];
         }
-        write_neighbor(m, a, live, live, i, k, key);
+        write_neighbor<0>(m, a, live, live, i, k, key);
     }
 }
 
@@ -4189,7 +4198,8 @@ int ash_map_neighbors(ash_map_t* map, int64_t num_rows, int radius, int bidirect
     ASH_HIP(guard.enter(map->device));
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (settle_table(map, s)) return 1;
-    neighbors_kernel<<<grid_for(num_rows * each), kBlock, 0, s>>>(map->d, a, heap_in_order(map) ? 1 : 0);
+    const auto kernel = a.width == 2 ? neighbors_kernel<2> : a.width == 3 ? neighbors_kernel<3> : neighbors_kernel<0>;
+    kernel<<<grid_for(num_rows * each), kBlock, 0, s>>>(map->d, a, heap_in_order(map) ? 1 : 0);
     ASH_LAUNCH_CHECK();
     if (!none_in_general(map)) {
         neighbors_general_kernel<<<looping_grid(map->d.gslots * each), kBlock, 0, s>>>(map->d, a);

@@ -31,6 +31,7 @@
 #include <cstring>
 #include <mutex>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 // Scratch of ash_grid_activate_static, the entry point that allocates nothing:
@@ -141,6 +142,36 @@ __device__ __forceinline__ void probe_pass(const MapDev& m, uint64_t code,
     compare(Round<3>());
 }
 
+// The same by every lane for itself (see kAloneKeys), and with no answer for keys that
+// are not pending.  VAL: the index is asked for as well.
+template <bool TOMBS = false, bool VAL = true>
+__device__ __forceinline__ void probe_alone(const MapDev& m, uint64_t code, uint32_t b, bool pend,
+                                            ProbeResult& out) {
+    if (!pend) return;
+    const uint4* line = reinterpret_cast<const uint4*>(m.buckets + static_cast<size_t>(b) * kBucketQwords);
+    uint4 w[kSlots / 2];
+#pragma unroll
+    for (int r = 0; r < kSlots / 2; ++r) w[r] = line[r];
+    out.slot = -1;
+    out.emask = 0;
+    if constexpr (TOMBS) out.tmask = 0;
+#pragma unroll
+    for (int s = kSlots - 1; s >= 0; --s) {
+        const uint4 v = w[s / 2];
+        const uint64_t q = s % 2 == 0 ? v.x | (static_cast<uint64_t>(v.y) << 32)
+                                      : v.z | (static_cast<uint64_t>(v.w) << 32);
+        if (q == code) out.slot = s;
+        if (q == kEmpty) out.emask |= 1u << s;
+        if constexpr (TOMBS) {
+            if (q == kTomb) out.tmask |= 1u << s;
+        }
+    }
+    out.status = out.slot >= 0 ? kProbeFound : (out.emask ? kProbeHasEmpty : kProbeFull);
+    if constexpr (VAL) {
+        if (out.slot >= 0) out.val = *value_ptr(m, b, out.slot);
+    }
+}
+
 // ------------------------------------------------ general (exotic) region
 enum { kGenWon = 0, kGenDup = 1, kGenFull = 2, kGenNoRegion = 3 };
 
@@ -239,7 +270,23 @@ __device__ __forceinline__ bool find_key(const MapDev& m, const int32_t (&k)[DIM
     return found;
 }
 
-template <int DIM>
+// Keys up to which every lane looks its own up (find_key_alone): half the vector
+// instructions and registers, and one trip to memory less before the codes are
+// compared, but five requests per line instead of two, which bound batches that fill the
+// device.  A batch, cooperative -> alone (us): without rows, among a million keys 131 000
+// 7.5 -> 6.6, 300 000 10.8 -> 8.6, 500 000 15.3 -> 12.5, 1 M 23.9 -> 21.9, among 100 000
+// 10.7 -> 9.8 at 500 000, 12.3 -> 12.5 at 700 000, 15.6 -> 16.9 at 1 M, 85 -> 113 at 8 M;
+// with rows of 12 and 4 bytes 131 000 10.2 -> 9.4, 200 000 12.1 -> 11.6, 300 000 14.5
+// -> 14.7, 1 M 41 -> 44.
+constexpr int64_t kAloneKeys = int64_t{1} << 19, kAloneKeysWithRows = int64_t{1} << 18;
+
+template <int DIM, bool ALONE>
+__device__ __forceinline__ bool look_up(const MapDev& m, const int32_t (&k)[DIM], bool active, int32_t& res) {
+    if constexpr (ALONE) return find_key_alone<DIM>(m, k, active, res);
+    else return find_key<DIM>(m, k, active, res);
+}
+
+template <int DIM, bool ALONE>
 __global__ __launch_bounds__(kBlock) void find_kernel(
         MapDev m, const int32_t* __restrict__ keys, int64_t n,
         int64_t* __restrict__ idx_out, uint8_t* __restrict__ mask_out) {
@@ -248,7 +295,7 @@ __global__ __launch_bounds__(kBlock) void find_kernel(
     int32_t k[DIM];
     load_key<DIM>(keys, i, active, k);
     int32_t res = 0;
-    const bool found = find_key<DIM>(m, k, active, res);
+    const bool found = look_up<DIM, ALONE>(m, k, active, res);
     if (active) {
         idx_out[i] = found ? static_cast<int64_t>(res) : 0;
         mask_out[i] = found ? 1 : 0;
@@ -324,8 +371,9 @@ __device__ __forceinline__ int32_t change_size(int32_t* ctr, int32_t by, int32_t
 // The insert proper for a key held in registers (`code` is its packed form if
 // `fits`); `i` is the row of the key's value rows / `assigned` / `given` entry.
 // TOMBS: the table may hold tombstones (the same for the whole launch).
-// BLOCK: threads of the workgroup, all of which call this together.
-template <int DIM, int MODE, bool TOMBS, int BLOCK = kHeapBlock>
+// BLOCK: threads of the workgroup, all of which call this together.  ALONE: buckets are
+// looked at by each lane for itself.
+template <int DIM, int MODE, bool TOMBS, int BLOCK = kHeapBlock, bool ALONE = false>
 __device__ __forceinline__ void insert_key(
         const MapDev& m, const int32_t (&k)[DIM], uint64_t code, bool fits,
         int64_t i, bool active, const ValueArgs& va,
@@ -371,7 +419,8 @@ __device__ __forceinline__ void insert_key(
     uint32_t first_tombs = 0, first_b = 0, first_steps = 0;   // in a bucket on the way
     while (__ballot(pend)) {
         ProbeResult p;
-        probe_pass<TOMBS>(m, code, b, pend, lane, p);
+        if constexpr (ALONE) probe_alone<TOMBS, MODE == kInsertReport>(m, code, b, pend, p);
+        else probe_pass<TOMBS>(m, code, b, pend, lane, p);
         if (pend) {
             if (p.status == kProbeFound) {
                 pend = false;
@@ -580,7 +629,7 @@ __device__ __forceinline__ void insert_key(
 
 // One key per thread, every thread of the workgroup calls this together.
 // CODES: `keys` holds packed 64-bit codes instead of int32[DIM] rows.
-template <int DIM, int MODE, bool TOMBS, bool CODES, int BLOCK = kHeapBlock>
+template <int DIM, int MODE, bool TOMBS, bool CODES, int BLOCK = kHeapBlock, bool ALONE = false>
 __device__ __forceinline__ void insert_one(
         const MapDev& m, const int32_t* __restrict__ keys, int64_t i,
         bool active, const ValueArgs& va, int32_t* __restrict__ assigned,
@@ -595,7 +644,7 @@ __device__ __forceinline__ void insert_one(
         load_key<DIM>(keys, i, active, k);
         fits = pack_key<DIM>(k, code);
     }
-    insert_key<DIM, MODE, TOMBS, BLOCK>(m, k, code, fits, i, active, va, assigned, given);
+    insert_key<DIM, MODE, TOMBS, BLOCK, ALONE>(m, k, code, fits, i, active, va, assigned, given);
 }
 
 // The counters, left where the host reads them: `landing` is a place in page-locked
@@ -668,14 +717,14 @@ __device__ __forceinline__ void check_keys(const int32_t* __restrict__ keys, int
     leave_word(check.word, (before >> 16) + (bad ? 1 : 0), check.stamp);
 }
 
-template <int DIM, int MODE, bool TOMBS, int BLOCK>
+template <int DIM, int MODE, bool TOMBS, int BLOCK, bool ALONE>
 __global__ __launch_bounds__(BLOCK) void insert_kernel(
         MapDev m, const int32_t* __restrict__ keys, int64_t n, ValueArgs va,
         int32_t* __restrict__ assigned, const int64_t* __restrict__ given, Publish publish,
         KeyCheck check) {
     if (blockIdx.x < check.groups) return check_keys<DIM, BLOCK>(keys, n, check);
     const int64_t i = static_cast<int64_t>(blockIdx.x - check.groups) * BLOCK + threadIdx.x;
-    insert_one<DIM, MODE, TOMBS, false, BLOCK>(m, keys, i, i < n, va, assigned, given);
+    insert_one<DIM, MODE, TOMBS, false, BLOCK, ALONE>(m, keys, i, i < n, va, assigned, given);
     leave_with_last(m, publish, gridDim.x - check.groups);
 }
 
@@ -1007,11 +1056,20 @@ __global__ __launch_bounds__(kHeapBlock) void activate_runs_kernel(
 // each), so larger groups pay off here: measured on 16 M stored keys,
 // 256 threads with a tombstone update per wavefront 3.0 ms, 1024 threads with
 // one update of each counter per workgroup 0.85 ms.
+// Fewer keys are better spread over the CUs.  Lanes that look at their buckets by
+// themselves (up to kWideInsertEnd keys, as inserts do), beside 100 000 | a million
+// keys, cooperative with 1024 threads -> 256 / 512 / 1024 (us): 8000 keys 10.9 | 11.7 ->
+// 7.1 / 8.5 / 11.8 | 6.9 / 8.5 / 11.4, 65 537 11.3 | 12.3 -> 10.8 / 11.8 / 14.2 | 10.5 /
+// 10.9 / 12.7, 98 000 13.7 | 13.4 -> 14.6 / 13.8 / 15.2 | 13.9 / 12.5 / 13.7, 131 000 14.3 |
+// 16.1 -> 17.6 / 15.5 / 16.4 | 17.6 / 15.2 / 15.0, 196 000 18.5 | 17.9 -> 22 / 19.6 / 18.5 |
+// 22 / 17.9 / 16.6, 300 000 38 | 39 -> 29 / 26 / 28 | 29 / 25 / 26, 1 M 65 | 63 -> 73 / 60 /
+// 57 | 74 / 59 / 56.
 constexpr int kEraseBlock = 1024;
+constexpr int64_t kEraseBy256 = int64_t{5} << 14, kEraseBy512 = int64_t{5} << 15;
 
 // One key per thread, every thread of the workgroup calls this together.
 // CODES: `keys` holds packed 64-bit codes instead of int32[DIM] rows.
-template <int DIM, bool CODES>
+template <int DIM, bool CODES, int BLOCK = kEraseBlock, bool ALONE = false>
 __device__ __forceinline__ void erase_one(const MapDev& m, const int32_t* __restrict__ keys,
                                           int64_t i, bool active) {
     const int lane = threadIdx.x & 63;
@@ -1034,7 +1092,8 @@ __device__ __forceinline__ void erase_one(const MapDev& m, const int32_t* __rest
     int32_t idx = 0;
     while (__ballot(pend)) {
         ProbeResult p;
-        probe_pass(m, code, b, pend, lane, p);
+        if constexpr (ALONE) probe_alone(m, code, b, pend, p);
+        else probe_pass(m, code, b, pend, lane, p);
         if (pend) {
             if (p.status == kProbeFound) {
                 // A bucket that still has an empty slot has never been full,
@@ -1070,8 +1129,8 @@ __device__ __forceinline__ void erase_one(const MapDev& m, const int32_t* __rest
             }
         }
     }
-    __shared__ int s_cnt[kEraseBlock / 64];
-    __shared__ int s_tomb[kEraseBlock / 64];
+    __shared__ int s_cnt[BLOCK / 64];
+    __shared__ int s_tomb[BLOCK / 64];
     __shared__ int s_base;
     const uint64_t wm = __ballot(won);
     const int nw = __popcll(wm);
@@ -1085,7 +1144,7 @@ __device__ __forceinline__ void erase_one(const MapDev& m, const int32_t* __rest
     if (threadIdx.x == 0) {
         int tot = 0, tombs = 0;
 #pragma unroll
-        for (int q = 0; q < kEraseBlock / 64; ++q) {
+        for (int q = 0; q < BLOCK / 64; ++q) {
             tot += s_cnt[q];
             tombs += s_tomb[q];
         }
@@ -1102,11 +1161,11 @@ __device__ __forceinline__ void erase_one(const MapDev& m, const int32_t* __rest
     }
 }
 
-template <int DIM>
-__global__ __launch_bounds__(kEraseBlock) void erase_kernel(
+template <int DIM, int BLOCK, bool ALONE>
+__global__ __launch_bounds__(BLOCK) void erase_kernel(
         MapDev m, const int32_t* __restrict__ keys, int64_t n, Publish publish) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * kEraseBlock + threadIdx.x;
-    erase_one<DIM, false>(m, keys, i, i < n);
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * BLOCK + threadIdx.x;
+    erase_one<DIM, false, BLOCK, ALONE>(m, keys, i, i < n);
     leave_with_last(m, publish, gridDim.x);
 }
 
@@ -1687,7 +1746,7 @@ __device__ __forceinline__ void copy_rows_of_wave(const RowTables& tabs, int32_t
 // through memory unless the caller wants them, and the line of a key's bucket
 // and the lines of its rows are asked for by the same wavefront.  16 M keys
 // with rows of 12 and 4 bytes: see the table of the design notes.
-template <int DIM>
+template <int DIM, bool ALONE>
 __global__ __launch_bounds__(kBlock) void find_rows_kernel(
         MapDev m, const int32_t* __restrict__ keys, int64_t n, RowTables tabs, int miss_row,
         int64_t* __restrict__ idx_out, uint8_t* __restrict__ mask_out) {
@@ -1696,7 +1755,7 @@ __global__ __launch_bounds__(kBlock) void find_rows_kernel(
     int32_t k[DIM];
     load_key<DIM>(keys, i, active, k);
     int32_t res = 0;
-    const bool found = find_key<DIM>(m, k, active, res);
+    const bool found = look_up<DIM, ALONE>(m, k, active, res);
     if (active) {
         if (idx_out != nullptr) idx_out[i] = found ? static_cast<int64_t>(res) : 0;
         if (mask_out != nullptr) mask_out[i] = found ? 1 : 0;
@@ -2643,15 +2702,15 @@ int give_up_heap_order(ash_map* map, hipStream_t s) {
 
 namespace {
 
-template <int MODE, bool TOMBS, int BLOCK>
+template <int MODE, bool TOMBS, int BLOCK, bool ALONE>
 int launch_insert_by(ash_map* map, const int32_t* keys, int64_t n,
                      const ValueArgs& va, int32_t* assigned, const int64_t* given,
                      hipStream_t s, const Publish& publish = {}, const KeyCheck& check = {}) {
     const unsigned g = grid_for(n, BLOCK) + check.groups;
-    auto kernel = map->key_dim == 1   ? insert_kernel<1, MODE, TOMBS, BLOCK>
-                  : map->key_dim == 2 ? insert_kernel<2, MODE, TOMBS, BLOCK>
-                  : map->key_dim == 3 ? insert_kernel<3, MODE, TOMBS, BLOCK>
-                                      : insert_kernel<4, MODE, TOMBS, BLOCK>;
+    auto kernel = map->key_dim == 1   ? insert_kernel<1, MODE, TOMBS, BLOCK, ALONE>
+                  : map->key_dim == 2 ? insert_kernel<2, MODE, TOMBS, BLOCK, ALONE>
+                  : map->key_dim == 3 ? insert_kernel<3, MODE, TOMBS, BLOCK, ALONE>
+                                      : insert_kernel<4, MODE, TOMBS, BLOCK, ALONE>;
     kernel<<<g, BLOCK, 0, s>>>(map->d, keys, n, va, assigned, given, publish, check);
     ASH_LAUNCH_CHECK();
     return 0;
@@ -2665,6 +2724,14 @@ int launch_insert_by(ash_map* map, const int32_t* keys, int64_t n,
 // Beyond three million the waits weigh more (the insert alone, without and with rows: a
 // million 117 -> 96, 126 -> 102; two 170 -> 146, 179 -> 150; four 322 -> 317, 363 -> 372;
 // eight 642 -> 647, 676 -> 732; sixteen 1016 -> 1039, 1117 -> 1239).
+//
+// Up to there every lane looks at its buckets by itself, which takes half of the
+// vector instructions and registers (the kernel with rows of 16 bytes, cooperative ->
+// alone, beside a million keys: 8000 12.5 -> 11.3 us, 65 537 20.8 -> 19.3, 131 000 29.5 ->
+// 27.0, 300 000 39 -> 34; beside 100 000 131 000 36.8 -> 31.7, 196 000 48.6 -> 39; keys
+// alone into an emptied table 16 000 13.1 -> 11.7, 98 000 21.8 -> 20.3); batches beyond
+// are bound by requests, of which that makes more (four million that come and go beside
+// four 600 -> 640, eight beside eight 1137 -> 1245).
 constexpr int64_t kWideInsert = int64_t{3} << 16, kWideInsertEnd = int64_t{3} << 20;
 constexpr int kWideBlock = 512;
 
@@ -2674,10 +2741,13 @@ int launch_insert_to(ash_map* map, const int32_t* keys, int64_t n,
                      hipStream_t s, const Publish& publish = {}, const KeyCheck& check = {}) {
     if constexpr (MODE == kInsertKeys || MODE == kInsertFused) {
         if (n > kWideInsert && n <= kWideInsertEnd) {
-            return launch_insert_by<MODE, TOMBS, kWideBlock>(map, keys, n, va, assigned, given, s, publish, check);
+            return launch_insert_by<MODE, TOMBS, kWideBlock, true>(map, keys, n, va, assigned, given, s, publish, check);
+        }
+        if (n <= kWideInsert) {
+            return launch_insert_by<MODE, TOMBS, kHeapBlock, true>(map, keys, n, va, assigned, given, s, publish, check);
         }
     }
-    return launch_insert_by<MODE, TOMBS, kHeapBlock>(map, keys, n, va, assigned, given, s, publish, check);
+    return launch_insert_by<MODE, TOMBS, kHeapBlock, false>(map, keys, n, va, assigned, given, s, publish, check);
 }
 
 template <int MODE>
@@ -3122,19 +3192,16 @@ int ash_map_find(ash_map_t* map, const int32_t* keys, int64_t n,
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (settle_table(map, s)) return 1;
     const unsigned g = grid_for(n);
+    auto launch = [&](auto dim) {
+        constexpr int DIM = decltype(dim)::value;
+        const auto kernel = n <= kAloneKeys ? find_kernel<DIM, true> : find_kernel<DIM, false>;
+        kernel<<<g, kBlock, 0, s>>>(map->d, keys, n, indices, masks);
+    };
     switch (map->key_dim) {
-        case 1:
-            find_kernel<1><<<g, kBlock, 0, s>>>(map->d, keys, n, indices, masks);
-            break;
-        case 2:
-            find_kernel<2><<<g, kBlock, 0, s>>>(map->d, keys, n, indices, masks);
-            break;
-        case 3:
-            find_kernel<3><<<g, kBlock, 0, s>>>(map->d, keys, n, indices, masks);
-            break;
-        default:
-            find_kernel<4><<<g, kBlock, 0, s>>>(map->d, keys, n, indices, masks);
-            break;
+        case 1: launch(std::integral_constant<int, 1>{}); break;
+        case 2: launch(std::integral_constant<int, 2>{}); break;
+        case 3: launch(std::integral_constant<int, 3>{}); break;
+        default: launch(std::integral_constant<int, 4>{}); break;
     }
     ASH_LAUNCH_CHECK();
     return 0;
@@ -3198,19 +3265,16 @@ int ash_map_find_rows_scratch(ash_map_t* map, const int32_t* keys, int64_t n, in
         }
     }
     const unsigned g = grid_for(n);
+    auto launch = [&](auto dim) {
+        constexpr int DIM = decltype(dim)::value;
+        const auto kernel = n <= kAloneKeysWithRows ? find_rows_kernel<DIM, true> : find_rows_kernel<DIM, false>;
+        kernel<<<g, kBlock, 0, s>>>(map->d, keys, n, tabs, miss, indices, masks);
+    };
     switch (map->key_dim) {
-        case 1:
-            find_rows_kernel<1><<<g, kBlock, 0, s>>>(map->d, keys, n, tabs, miss, indices, masks);
-            break;
-        case 2:
-            find_rows_kernel<2><<<g, kBlock, 0, s>>>(map->d, keys, n, tabs, miss, indices, masks);
-            break;
-        case 3:
-            find_rows_kernel<3><<<g, kBlock, 0, s>>>(map->d, keys, n, tabs, miss, indices, masks);
-            break;
-        default:
-            find_rows_kernel<4><<<g, kBlock, 0, s>>>(map->d, keys, n, tabs, miss, indices, masks);
-            break;
+        case 1: launch(std::integral_constant<int, 1>{}); break;
+        case 2: launch(std::integral_constant<int, 2>{}); break;
+        case 3: launch(std::integral_constant<int, 3>{}); break;
+        default: launch(std::integral_constant<int, 4>{}); break;
     }
     ASH_LAUNCH_CHECK();
     return 0;
@@ -3556,12 +3620,19 @@ int ash_map_erase(ash_map_t* map, const int32_t* keys, int64_t n,
         if (late.take(false)) return 1;
         if (late.taken()) publish = {late.late(), late.stamp, next_ticket(map)};
     }
-    const unsigned g = grid_for(n, kEraseBlock);
-    auto kernel = map->key_dim == 1   ? erase_kernel<1>
-                  : map->key_dim == 2 ? erase_kernel<2>
-                  : map->key_dim == 3 ? erase_kernel<3>
-                                      : erase_kernel<4>;
-    kernel<<<g, kEraseBlock, 0, s>>>(map->d, keys, n, publish);
+    auto launch = [&](auto block, auto alone) {
+        constexpr int BLOCK = decltype(block)::value;
+        constexpr bool ALONE = decltype(alone)::value;
+        auto kernel = map->key_dim == 1   ? erase_kernel<1, BLOCK, ALONE>
+                      : map->key_dim == 2 ? erase_kernel<2, BLOCK, ALONE>
+                      : map->key_dim == 3 ? erase_kernel<3, BLOCK, ALONE>
+                                          : erase_kernel<4, BLOCK, ALONE>;
+        kernel<<<grid_for(n, BLOCK), BLOCK, 0, s>>>(map->d, keys, n, publish);
+    };
+    if (n <= kEraseBy256) launch(std::integral_constant<int, 256>{}, std::true_type{});
+    else if (n <= kEraseBy512) launch(std::integral_constant<int, 512>{}, std::true_type{});
+    else if (n <= kWideInsertEnd) launch(std::integral_constant<int, kEraseBlock>{}, std::true_type{});
+    else launch(std::integral_constant<int, kEraseBlock>{}, std::false_type{});
     ASH_LAUNCH_CHECK();
     change.queued();
     if (late.taken()) late.queued(true);

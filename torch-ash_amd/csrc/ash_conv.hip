@@ -13,24 +13,25 @@
 // sees its taps in table order, one fused multiply-add per tap, as in the other
 // kernels.
 //
-// 60 000 blocks: five channels 3^3 347 us a call (440 before one wavefront each, 1275
-// with tables and instances for powers of two), two channels 126 (501); 1000
-// blocks, 7^3: 94 (990: every workgroup used to check the tables).  3^3 windows of
-// five channels move 1.47 GB beyond the L2s, 4.3 TB/s: 0.61 GB of results and 0.86
-// of rows, 1.4 times what there are (the halo along x takes most lines of two
-// neighbours); vector instructions are issued in 0.59 of the cycles, the LDS is
-// busy in 0.54.  7^3 windows of two channels are bound by vector instructions
-// (0.87 of the cycles; 1941 per wavefront and block, 1372 of them multiply-adds
-// and 343 tap reads).
+// 60 000 blocks, the kernel alone: five channels 3^3 321 us (345 with the halo word by
+// word, its missing rows selected and the taps read lane by lane; 1275 with tables and
+// instances for powers of two); 40 000 blocks of two 87 -> 74 us a call; 4000 blocks,
+// 7^3, of five 215 -> 195.  3^3 windows of five channels move 1.61 GB beyond the L2s at
+// 5.0 TB/s, what a large copy reaches, and are bound by that: 0.61 GB of results and
+// 1.0 of rows, 1.6 times what there are (the halo along x takes most lines of two
+// neighbours; the listing along other curves changes nothing).  Without any
+// arithmetic 307 us, without the results' way out 220; vector instructions are issued
+// in 0.47 of the cycles, the LDS is busy in 0.52.  7^3 windows are bound by vector
+// instructions (of two channels in 0.87 of the cycles).
 //
-// The block's own rows are contiguous in memory whatever their width: they come
-// in as 16-byte pieces and leave the same way, through LDS.
-// The halo comes element by element (consecutive lanes, consecutive words of a
-// row).  Where an element goes in the tile never changes from block to block
-// and is kept in registers.  Software pipeline: while a block is computed the
-// next block's elements are on their way into registers and the row numbers of
-// the one after are fetched.  Rows of missing blocks are staged as zeros (with
-// finite weights adding 0 * w leaves a sum as it is).
+// A tile is kT * kT lines of eight cells along x, contiguous in memory whatever the
+// width of the rows: they come in as 16-byte pieces, and results leave the same way,
+// through LDS.  The lines' ends come word by word (consecutive lanes, consecutive
+// words of a row).  Where a piece or word goes in the tile never changes from block to
+// block and is kept in registers.  Software pipeline: while a block is computed the
+// next block's pieces are on their way into registers and the row numbers of the one
+// after are fetched.  Rows of missing blocks are staged as zeros (with finite weights
+// adding 0 * w leaves a sum as it is).
 #include "ash_table.h"
 #include "ash_walk.h"
 
@@ -215,11 +216,14 @@ convolution_block8_kernel(ConvArgs a) {
         const int64_t row = a.lut_g[g * 27 + tid];
         return (row >= 0 && row < a.B) ? static_cast<int32_t>(row) : -1;
     };
-    // Byte offsets fit 32 bits: the host sees to it that one block more would still be
-    // below 4 GiB, and a missing block's rows stand there, beyond the tensor, where the
-    // loads give zeros by themselves.
-    constexpr uint32_t kBlockBytes = kM * E * 4, kMissing = 0u - kBlockBytes;
+    // Byte offsets fit 32 bits: the tensors are below 4 GiB, which the host checks, and
+    // end at a multiple of 2048.  A missing block's rows are read beyond the tensor, where
+    // the loads give zeros by themselves.
+    constexpr uint32_t kBlockBytes = kM * E * 4, kMissing = 0xFFFFFFFFu, kBeyond = 0xFFFFFFF0u;
     auto start_of = [&](int32_t row) { return row < 0 ? kMissing : static_cast<uint32_t>(row) * kBlockBytes; };
+    auto place_in = [&](uint32_t start, uint32_t byte) {
+        return static_cast<int>(start == kMissing ? kBeyond : start + byte);
+    };
     const auto in = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.in), 0,
                                                       static_cast<int>(static_cast<uint32_t>(a.B) * kBlockBytes),
                                                       0x00020000);
@@ -228,13 +232,13 @@ convolution_block8_kernel(ConvArgs a) {
     auto load_block = [&](const uint32_t* nb) {
 #pragma unroll
         for (int i = 0; i < S::kPiecesEach; ++i) {
-            const uint32_t at = nb[piece_src[i] >> 14] + (piece_src[i] & 0x3FFFu);
-            piece[i] = __builtin_bit_cast(v4, __builtin_amdgcn_raw_buffer_load_b128(in, static_cast<int>(at), 0, 0));
+            const int at = place_in(nb[piece_src[i] >> 14], piece_src[i] & 0x3FFFu);
+            piece[i] = __builtin_bit_cast(v4, __builtin_amdgcn_raw_buffer_load_b128(in, at, 0, 0));
         }
 #pragma unroll
         for (int i = 0; i < S::kEndsEach; ++i) {
-            const uint32_t at = nb[(ends[i] >> 12) & 31u] + (ends[i] & 0xFFFu) * 4u;
-            end[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(in, static_cast<int>(at), 0, 0));
+            const int at = place_in(nb[(ends[i] >> 12) & 31u], (ends[i] & 0xFFFu) * 4u);
+            end[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(in, at, 0, 0));
         }
     };
 
@@ -391,7 +395,7 @@ int ash_convolution_cube_supported(int64_t num_embeddings, int grid_dim, int win
                                    int64_t embedding_dim, int32_t dtype) {
     return dtype == ASH_F32 && grid_dim == kG && (window == 3 || window == 5 || window == 7) &&
            embedding_dim >= 1 && embedding_dim <= kMaxChannels && num_embeddings >= 1 &&
-           (num_embeddings + 1) * embedding_dim * kM * 4 <= 0x100000000ll;   // (kMissing)
+           num_embeddings * embedding_dim * kM * 4 <= 0xFFFFFFFFll;
 }
 
 int ash_convolution_cube(const void* inputs, const void* weights, const int64_t* grid_indices,

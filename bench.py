@@ -119,7 +119,7 @@ MEASURED_COUNTERS = {
 COUNTERS_SOURCE = {
     "profiles": ["profiles/bench_hbm_traffic_pmc.md",
                  "profiles/bench_l2_hit_rate_and_atomics_pmc.md"],
-    "csrc_sha256": "6282425853ddb8d8372191e8e1a7d5d4bdc2e2609313ea9a6c82d02780da7e3d",
+    "csrc_sha256": "5cc4fb85697e538bfa803f6d3eb5ea7dea9fc7fd5df5bb89a94186475593410a",
 }
 
 

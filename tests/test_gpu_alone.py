@@ -82,3 +82,9 @@ def test_batches_come_and_go(ash, dim, n):
     if n > STORED:   # erased among keys that are not there, the others stay
         m.erase(torch.cat([new[: n - 100], stored[:100]]))
         assert m.size() == STORED - 100 and bool(m.engine.find(stored[100:])[1].all())
+
+
+@pytest.mark.parametrize("dim,n", [(3, 3 << 14), (2, (3 << 14) + 1), (1, 7 << 14), (4, (7 << 14) + 1), (3, 150_001)])
+def test_erases_where_their_workgroups_change(ash, dim, n):
+    """The index comes along with the codes of a bucket that other lanes erase from."""
+    test_batches_come_and_go(ash, dim, n)

@@ -143,33 +143,40 @@ __device__ __forceinline__ void probe_pass(const MapDev& m, uint64_t code,
 }
 
 // The same by every lane for itself (see kAloneKeys), and with no answer for keys that
-// are not pending.  VAL: the index is asked for as well.
+// are not pending.  VAL: the index is asked for as well, along with the codes: read
+// behind them, the line has often gone to an atomic of another lane in between (erases
+// of 131 000 keys 13.4 -> 15.6 us when it was).
 template <bool TOMBS = false, bool VAL = true>
 __device__ __forceinline__ void probe_alone(const MapDev& m, uint64_t code, uint32_t b, bool pend,
                                             ProbeResult& out) {
     if (!pend) return;
+    constexpr int kPieces = VAL ? kGroup : kSlots / 2;
     const uint4* line = reinterpret_cast<const uint4*>(m.buckets + static_cast<size_t>(b) * kBucketQwords);
-    uint4 w[kSlots / 2];
+    uint4 w[kPieces];
 #pragma unroll
-    for (int r = 0; r < kSlots / 2; ++r) w[r] = line[r];
+    for (int r = 0; r < kPieces; ++r) w[r] = line[r];
     out.slot = -1;
     out.emask = 0;
     if constexpr (TOMBS) out.tmask = 0;
+    if constexpr (VAL) out.val = 0;
 #pragma unroll
     for (int s = kSlots - 1; s >= 0; --s) {
         const uint4 v = w[s / 2];
         const uint64_t q = s % 2 == 0 ? v.x | (static_cast<uint64_t>(v.y) << 32)
                                       : v.z | (static_cast<uint64_t>(v.w) << 32);
         if (q == code) out.slot = s;
+        if constexpr (VAL) {
+            static_assert(kValDword0 % 4 == 0, "four indices to a piece");
+            const uint4 i = w[(kValDword0 + s) / 4];
+            const uint32_t val = s % 4 == 0 ? i.x : s % 4 == 1 ? i.y : s % 4 == 2 ? i.z : i.w;
+            if (q == code) out.val = static_cast<int32_t>(val);
+        }
         if (q == kEmpty) out.emask |= 1u << s;
         if constexpr (TOMBS) {
             if (q == kTomb) out.tmask |= 1u << s;
         }
     }
     out.status = out.slot >= 0 ? kProbeFound : (out.emask ? kProbeHasEmpty : kProbeFull);
-    if constexpr (VAL) {
-        if (out.slot >= 0) out.val = *value_ptr(m, b, out.slot);
-    }
 }
 
 // ------------------------------------------------ general (exotic) region
@@ -1056,16 +1063,20 @@ __global__ __launch_bounds__(kHeapBlock) void activate_runs_kernel(
 // each), so larger groups pay off here: measured on 16 M stored keys,
 // 256 threads with a tombstone update per wavefront 3.0 ms, 1024 threads with
 // one update of each counter per workgroup 0.85 ms.
-// Fewer keys are better spread over the CUs.  Lanes that look at their buckets by
-// themselves (up to kWideInsertEnd keys, as inserts do), beside 100 000 | a million
-// keys, cooperative with 1024 threads -> 256 / 512 / 1024 (us): 8000 keys 10.9 | 11.7 ->
-// 7.1 / 8.5 / 11.8 | 6.9 / 8.5 / 11.4, 65 537 11.3 | 12.3 -> 10.8 / 11.8 / 14.2 | 10.5 /
-// 10.9 / 12.7, 98 000 13.7 | 13.4 -> 14.6 / 13.8 / 15.2 | 13.9 / 12.5 / 13.7, 131 000 14.3 |
-// 16.1 -> 17.6 / 15.5 / 16.4 | 17.6 / 15.2 / 15.0, 196 000 18.5 | 17.9 -> 22 / 19.6 / 18.5 |
-// 22 / 17.9 / 16.6, 300 000 38 | 39 -> 29 / 26 / 28 | 29 / 25 / 26, 1 M 65 | 63 -> 73 / 60 /
-// 57 | 74 / 59 / 56.
+// Fewer keys are better spread over the CUs.  Lanes look at their buckets by themselves
+// up to kWideInsertEnd keys, as inserts do, but take the index along with the codes
+// (probe_alone).  Cooperative with 1024 threads -> alone with the index read behind the
+// codes -> as it is (us), stored keys beside 100 000 | four million: 16 000 9.1 -> 6.8 ->
+// 6.3 | 11.1 -> 7.5 -> 7.3, 65 537 10.0 -> 11.0 -> 9.6 | 12.4 -> 10.8 -> 10.0, 98 000 11.5
+// -> 12.9 -> 11.4 | 13.9 -> 12.6 -> 11.9, 131 000 13.6 -> 15.7 -> 13.3 | 16.1 -> 15.2 ->
+// 13.7, 164 000 15.0 -> 18.2 -> 14.0 | 17.7 -> 17.2 -> 14.4, 400 000 42 -> 32 -> 27 | 33 ->
+// 28 -> 26, 1.6 million 92 -> 92 -> 85 | 88 -> 96 -> 84, 3.1 million 175 -> 228 -> 178
+// beside four; each key four times 131 000 13.7 -> 16.6 -> 13.0, 3.1 million 109 -> 126 -> 90;
+// absent keys 131 000 7.1 -> 5.8 -> 6.5, 3.1 million 77 -> 62 -> 63.  With 256 | 512 | 1024
+// threads: 50 000 8.6 | 8.5 | 11.0, 98 000 12.9 | 11.3 | 11.9, 115 000 15.0 | 12.5 | 12.6,
+// 131 000 17.9 | 14.1 | 13.3.
 constexpr int kEraseBlock = 1024;
-constexpr int64_t kEraseBy256 = int64_t{5} << 14, kEraseBy512 = int64_t{5} << 15;
+constexpr int64_t kEraseBy256 = int64_t{3} << 14, kEraseBy512 = int64_t{7} << 14;
 
 // One key per thread, every thread of the workgroup calls this together.
 // CODES: `keys` holds packed 64-bit codes instead of int32[DIM] rows.

@@ -427,6 +427,38 @@ def test_activation_of_standing_and_missing_blocks(gpu_ash, n, far):
         assert torch.equal(torch.sort(rows)[0], torch.sort(grid.engine.items()[1])[0]), step
 
 
+@pytest.mark.parametrize("workgroups", [512, 513, 1280, 1281])   # of 256 positions, on 256 CUs
+@pytest.mark.parametrize("one_more", [0, 1])
+def test_activation_where_its_launch_changes(gpu_ash, workgroups, one_more):
+    test_activation_of_standing_and_missing_blocks(gpu_ash, workgroups * 256 + one_more, False)
+
+
+@pytest.mark.parametrize("share", [0.03, 0.5, 1.0])
+@pytest.mark.parametrize("n", [20_000, 150_000, 400_000])
+def test_activation_of_blocks_new_to_a_standing_table(gpu_ash, n, share):
+    """Many workgroups name each of the blocks that are missing, beside others that stand:
+    every index once, and the block's own."""
+    g = torch.Generator().manual_seed(n)
+    cells = ((torch.rand(n, 3, generator=g).cumsum(0) * 0.02) % 100.0).to(DEV)
+    grid = gpu_ash.UnBoundedSparseDenseGrid(3, 9_000, 1, 8, cell_size=1.0, device=DEV)
+    grid.engine.insert_keys((torch.randint(20, 40, (3000, 3), generator=g)).int().to(DEV))
+    beside = grid.engine.size()
+    coords = grid.spatial_init_(cells, dilation=1, bidirectional=True)[0].view(-1, 3)
+    want = torch.unique(coords, dim=0)
+    assert len(want) == len(coords) and grid.engine.size() == beside + len(want)
+    order = torch.randperm(len(want), generator=g)[: int(share * len(want))].to(DEV)
+    for _ in range(3):
+        grid.engine.erase(want[order].contiguous())
+        coords, _, rows, _ = grid.spatial_init_(cells, dilation=1, bidirectional=True)
+        coords, rows = coords.view(-1, 3), rows.view(-1)
+        assert len(coords) == len(want) and torch.equal(torch.unique(coords, dim=0), want)
+        assert grid.engine.size() == beside + len(want)
+        found, masks = grid.engine.find(coords)
+        assert bool(masks.all()) and torch.equal(found, rows)
+        indices = torch.cat([grid.engine.items()[1], grid.engine._heap[grid.engine.size():].long()])
+        assert torch.equal(torch.sort(indices)[0], torch.arange(grid.engine.capacity, device=DEV))
+
+
 @pytest.mark.parametrize("grid_dim,e,bounded", [(8, 2, False), (8, 5, False), (4, 2, True), (8, 2, True)])
 def test_integration_by_flags_equals_integration_by_listing(gpu_ash, grid_dim, e, bounded):
     """ash_grid_integrate_depth_flagged (after ash_grid_activate_positions)

@@ -21,6 +21,7 @@
 // an erased key stores its index at heap[--counter]; here the counter is
 // advanced once per workgroup instead of once per key.
 #include "ash_probe.h"
+#include "ash_walk.h"
 
 #include "../../include/ash_hip.h"
 
@@ -918,24 +919,36 @@ constexpr int kCandChunk = 1024;         // candidates made distinct at a time
 constexpr int kDistinctSlots = 2048;     // two LDS slots per candidate of a chunk
 
 // One launch per batch: insert and flag.  The (head, neighbour offset)
-// candidates of a workgroup -- some 270 for 128 depth pixels at dilation 1 --
+// candidates of a workgroup -- 570 for 256 pixels of a VGA frame at dilation 1 --
 // name every block twice on average (the neighbourhoods of neighbouring
 // blocks overlap in 18 of 27), so they are first made distinct in an LDS set,
 // and then looked up by a lane each, one after the other without a barrier in
 // between: a block that stands, which is what a frame mostly meets, is flagged there
 // and then, once the key log confirms its index.  (A table that has been emptied and not
-// used since holds none: frames of 640 x 480 and 1200 x 900 into such a one 52 and 100
-// us, 54 and 111 with the look.)  What is left is inserted.  The insert
+// used since holds none, and is not looked at.)  What is left is inserted.  The insert
 // reports the index of every key it can be sure of (insert_key, kInsertReport)
 // and the row is flagged at once; a key that another thread is storing at
 // that moment is flagged by that thread, which is handed the index.  No second
 // launch has to wait for the indices to settle.
 //
-// A chain of waits; VGA frame, 791 workgroups of some 240 distinct blocks (us): every
-// block through the insert, which a third of the workgroups entered twice, 14.3; as it
-// is 11.6.  512 threads, one round for everybody: 16, the registers of the insert leave
-// room for half of the workgroups; 128 and 64 positions 16.6 and 23.
-template <bool TOMBS>
+// ALONE: the insert's lanes look at their buckets by themselves, with the index along with
+// the codes, as other workgroups' atomics take the lines away.  Into emptied tables only
+// up to two workgroups per CU: beyond, all of them meet in the same buckets at once, and
+// the quicker probe makes more of their atomics fail (VGA frame 27.6 -> 30.2 us; 160 x
+// 120 32.0 -> 27.2).
+//
+// A chain of waits.  Every block through a cooperative insert | that insert behind the look
+// | as it is (us), by the share of a frame's blocks that are new to a standing table, at one
+// side of it: VGA frame, 817 workgroups of some 250 distinct blocks, none 14.7 | 12.5 | 12.5,
+// 3 % 17.4 | 18.0 | 16.0, 10 % 20.5 | 20.6 | 17.6, half 24.0 | 24.8 | 22.9, all 28.4 | 31.6 |
+// 32.2; 160 x 120 26 | 18.7 | 18.6, 27.5 | 25.8 | 22.9, 28.4 | 27.2 | 24.1, 31 | 29.6 | 26.7,
+// 33 | 37 | 33; 1200 x 900 25 | 21 | 21, 30 | 31 | 25, 38 | 39 | 29, 52 | 57 | 45, 63 | 68 |
+// 62; VGA with blocks of twice the edge 10.2 | 8.3 | 8.8, 11.4 | 13.8 | 12.8, 15.1 | 15.7 |
+// 15.1, 21 | 21 | 23, 26 | 28 | 30.  (Frames of which everything is new are better off without the
+// look, which nobody knows beforehand.)  512 threads, one round for everybody: 16, the
+// registers of the insert leave room for half of the workgroups; 128 and 64 positions 16.6
+// and 23.
+template <bool TOMBS, bool ALONE>
 __global__ __launch_bounds__(kHeapBlock) void activate_runs_kernel(
         MapDev m, RunsArgs a, uint8_t* __restrict__ touched, int32_t* __restrict__ coords) {
     __shared__ unsigned long long s_set[kDistinctSlots];
@@ -1051,7 +1064,7 @@ __global__ __launch_bounds__(kHeapBlock) void activate_runs_kernel(
             uint64_t code;
             const bool fits = pack_key<3>(k, code);
             int32_t row = -1;
-            insert_key<3, kInsertReport, TOMBS>(m, k, code, fits, 0, ok, none, nullptr, nullptr, &row);
+            insert_key<3, kInsertReport, TOMBS, kHeapBlock, ALONE>(m, k, code, fits, 0, ok, none, nullptr, nullptr, &row);
             if (ok && row >= 0) flag(row, k);
             __syncthreads();   // insert_key's own words are rewritten by the next round
         }
@@ -3476,7 +3489,9 @@ int ash_grid_activate_positions(ash_map_t* map, const float* positions, int64_t 
     a.empty = empty;
     const int64_t groups = (n + kRunPositions - 1) / kRunPositions;
     if (groups > 0x7FFFFFFFll) ASH_FAIL("too many positions in one call");
-    auto kernel = tombs_in(map) ? activate_runs_kernel<true> : activate_runs_kernel<false>;
+    const bool alone = !empty || groups <= 2 * compute_units();
+    auto kernel = tombs_in(map) ? (alone ? activate_runs_kernel<true, true> : activate_runs_kernel<true, false>)
+                                : (alone ? activate_runs_kernel<false, true> : activate_runs_kernel<false, false>);
     kernel<<<static_cast<unsigned>(groups), kHeapBlock, 0, s>>>(map->d, a, touched, coords);
     ASH_LAUNCH_CHECK();
     return 0;

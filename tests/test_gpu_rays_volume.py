@@ -71,3 +71,29 @@ def test_rays_that_leave_the_volume(gpu_ash, far_block, n):
     for a, b in zip(plain, backend.ray_sample_world(*args, (0, 31))):
         assert a.dtype == b.dtype and torch.equal(torch.nan_to_num(a), torch.nan_to_num(b))
     assert len(plain[0]) > n // 2   # (a block in thirteen is stored)
+
+
+@pytest.mark.parametrize("zeros", [1, 2])
+@pytest.mark.parametrize("n", [8195, 66_000])
+def test_rays_along_axes(gpu_ash, zeros, n):
+    """Directions with components of +0 and -0, from inside the bounds and from their faces."""
+    grid = gpu_ash.BoundedSparseDenseGrid(3, 3000, 1, 8, 32, device=DEV)
+    backend, table = gpu_ash.grid.backend, grid.engine.backend
+    g = torch.Generator().manual_seed(n + zeros)
+    grid.engine.insert_keys(torch.randint(0, 32, (2500, 3), generator=g).int().to(DEV))
+    o = torch.rand(n, 3, generator=g) * 256
+    d = torch.randn(n, 3, generator=g)
+    axis = torch.randint(3, (n,), generator=g)
+    for k in range(zeros):
+        sign = torch.where(torch.rand(n, generator=g) < 0.5, 0.0, -0.0)
+        d[torch.arange(n), (axis + k) % 3] = sign
+        o[k::7, 0], o[k + 2::7, 1] = 0.0, 256.0
+    o, d = o.to(DEV), torch.nn.functional.normalize(d, dim=1).to(DEV)
+    box = [torch.full((3,), x, device=DEV) for x in (0.0, 256.0)]
+    args = (table, o, d, None, 1.0, *box, 0.0, 800.0, 8.0)
+    near, far = backend.ray_find_near_far_world(*args)
+    for a, b in zip((near, far), backend.ray_find_near_far_world(*args, (0, 31))):
+        assert torch.equal(a, b)
+    # (a block in thirteen is stored, of the sixteen that a ray along an axis passes; a
+    # ray that leaves at once from a face passes none)
+    assert int((near >= 0).sum()) > n // 4

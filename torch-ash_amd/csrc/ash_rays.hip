@@ -292,7 +292,9 @@ __global__ __launch_bounds__(kBlock) void ray_near_far_kernel(
 // before it are then only looked up, without the box.
 //
 // Bound by vector instructions (410 of a wavefront): with the box asked at every step
-// 22.4 us for 32 768 rays across 200 000 blocks, 15.5 with the end found first.
+// 22.4 us for 32 768 rays across 200 000 blocks, 15.5 with the end found first; of rays with
+// one component of zero 20.5 and 14.4 (16.3 where such a component sent the first guess to
+// the ray's start).
 struct RaySteps {
     int most;         // whose parameter lies below t_max
     float per_step;   // about 1 / step, for the first guess
@@ -354,7 +356,10 @@ __global__ __launch_bounds__(kBlock) void ray_near_far_pairs_kernel(
         float at = t_max;
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            at = fminf(at, ((d[a] > 0.f ? hi[a] : lo[a]) - o[a]) * __builtin_amdgcn_rcpf(d[a]));
+            // (by the sign bit: a component of +0 or -0 gives +infinity, and 0 * infinity,
+            // which is no number, does not count)
+            const float side = __float_as_int(d[a]) >= 0 ? hi[a] : lo[a];
+            at = fminf(at, (side - o[a]) * __builtin_amdgcn_rcpf(d[a]));
         }
         const float guess = fminf(fmaxf((at - t_min) * steps.per_step - 16.f, 0.f), static_cast<float>(steps.most));
         const int base = static_cast<int>(guess);

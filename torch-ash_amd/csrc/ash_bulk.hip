@@ -39,6 +39,7 @@
 // any input.  (A probe sequence stays inside its partition by the table's own
 // rule, ash_table.h: next_bucket.)
 #include "ash_table.h"
+#include "ash_walk.h"
 
 #include "../../include/ash_hip.h"
 
@@ -61,15 +62,19 @@ constexpr int kOnceChunks = 1024;
 constexpr int kOnceParts = 4096;
 constexpr int kBuildThreads = 512;
 // Ranges that start empty are built from lists (build_lists_kernel) where there are more
-// than the two workgroups of build_kernel per CU take at once, and with up to so many
+// than two workgroups of build_kernel per CU take at once, and with up to so many
 // records per two buckets.  build_kernel -> lists, kernel (us), keys alone: 86 ranges
 // 11.7 -> 13.2, 261 15.9 -> 15.6, 652 28.3 -> 22.4, 1303 37.9 -> 35.8, 912 of 4.3 records
 // a bucket 44.9 -> 31.7, 2605 71.4 -> 68.7; with rows, four records a bucket: 128 ranges
 // 13.4 -> 16.1, 489 15.9 -> 17.5, 1465 42.9 -> 38.2, of two a bucket 2930 71.6 -> 49.2.
 // From five records a bucket on too many buckets overflow.
-constexpr int64_t kListsFrom = 512;
+constexpr int kListsPerCu = 2;
 constexpr int kMostPerTwoBuckets = 9;
 constexpr int kListRecs = 6;   // records per thread there
+// which are all that a range's buffer holds (cap_part: the mean, ten of its roots and 64, in
+// sixteens)
+static_assert(kMostPerTwoBuckets * static_cast<int>(kPartBuckets) / 2 + 10 * 48 + 64 + 15 <= kBuildThreads * kListRecs &&
+              kMostPerTwoBuckets * static_cast<int>(kPartBuckets) / 2 <= 48 * 48, "a round takes a range's records");
 constexpr int kBuildRecs = 4;                   // records per thread and round
 constexpr int kCopyThreads = 256;
 constexpr int64_t kMinKeys = 1 << 12;
@@ -176,8 +181,10 @@ int64_t make_plan(const ash_map* map, int64_t n, int n_values,
 
     const int64_t once_chunks = (n + kSplitChunk - 1) / kSplitChunk;
     pl.once = insert && parts <= kOnceParts && once_chunks <= kOnceChunks;
-    pl.lists = pl.once && map->table_stale && heap_in_order(map) && parts > kListsFrom &&
-               2 * n <= kMostPerTwoBuckets * nb && cap_part <= kBuildThreads * kListRecs;
+    // (an emptied table: every key finds an index as n is at most the capacity, and a slot
+    // in its range, which has ten per bucket)
+    pl.lists = pl.once && map->table_stale && heap_in_order(map) && n <= map->d.capacity &&
+               parts > kListsPerCu * static_cast<int64_t>(compute_units()) && 2 * n <= kMostPerTwoBuckets * nb;
     pl.share_shift = 0;
     while (pl.lists && (once_chunks << (pl.share_shift + 1)) <= kBuildThreads &&
            once_chunks + 1 <= cap_part) {
@@ -823,6 +830,22 @@ __device__ __forceinline__ void drop_repeats(uint4* tab, int lb, int n, Dropped 
 enum { kRecIdle = 0, kRecPlaced = 1, kRecLost = 2 };
 constexpr int kWaitList = 128;
 
+// One split pass: where range p's records start in the thread's two chunks, and how many
+// there are.
+static_assert(kOnceChunks == 2 * kBuildThreads, "a thread adds up two chunks");
+__device__ __forceinline__ void records_in_chunks(const BulkPlan& pl, uint32_t p, int (&first)[2], int (&own)[2]) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const int c = 2 * static_cast<int>(threadIdx.x) + q;
+        first[q] = own[q] = 0;
+        if (c < static_cast<int>(pl.once_chunks)) {
+            const uint16_t* at = pl.starts + static_cast<int64_t>(c) * (pl.parts + 1) + p;
+            first[q] = at[0];
+            own[q] = at[1] - at[0];
+        }
+    }
+}
+
 // (four wavefronts per SIMD: the two workgroups that the LDS holds)
 // ONCE: the records come from one split pass, a few from each chunk.  A workgroup adds
 // up how many there are in each and finds the chunk of a record by halving; workgroups
@@ -869,18 +892,8 @@ __global__ __launch_bounds__(kBuildThreads, 4) void build_kernel(
                                              : static_cast<uint32_t>(kPartBuckets));
     int cnt = 0;
     if constexpr (ONCE) {
-        static_assert(kOnceChunks == 2 * kBuildThreads, "a thread adds up two chunks");
         int first[2], own[2];
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int c = 2 * tid + q;
-            first[q] = own[q] = 0;
-            if (c < static_cast<int>(pl.once_chunks)) {
-                const uint16_t* at = pl.starts + static_cast<int64_t>(c) * (pl.parts + 1) + p;
-                first[q] = at[0];
-                own[q] = at[1] - at[0];
-            }
-        }
+        records_in_chunks(pl, p, first, own);
         // (an empty range is made while they come)
         if (was_empty) {
             for (int t = tid; t < nbk * kGroup; t += kBuildThreads) {
@@ -1254,18 +1267,8 @@ __global__ __launch_bounds__(kBuildThreads, 8) void build_lists_kernel(
     v4u* __restrict__ gl = reinterpret_cast<v4u*>(m.buckets) + static_cast<size_t>(b0) * kGroup;
 
     // the records of this range in each chunk, and before it
-    static_assert(kOnceChunks == 2 * kBuildThreads, "a thread adds up two chunks");
     int first[2], own[2];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-        const int c = 2 * tid + q;
-        first[q] = own[q] = 0;
-        if (c < static_cast<int>(pl.once_chunks)) {
-            const uint16_t* at = pl.starts + static_cast<int64_t>(c) * (pl.parts + 1) + p;
-            first[q] = at[0];
-            own[q] = at[1] - at[0];
-        }
-    }
+    records_in_chunks(pl, p, first, own);
     s_cnt[tid] = 0;
     if (tid == 0) s_losers = s_nbeside = 0;
     // running sums over the workgroup: what lies before the thread's `v`, and all
@@ -1440,6 +1443,7 @@ __global__ __launch_bounds__(kBuildThreads, 8) void build_lists_kernel(
             int b = static_cast<int>(bucket_of(own_code, m.nb) - b0);
             int at = -1;        // its place in the list
             int beside = -1;    // or beside it
+            // (ends: a range has more slots than records)
             for (int visited = 0; !known && at < 0 && beside < 0 && visited < static_cast<int>(kPartBuckets);
                  ++visited) {
                 const int to = s_first[b + 1];
@@ -1454,11 +1458,9 @@ __global__ __launch_bounds__(kBuildThreads, 8) void build_lists_kernel(
                 b = b + 1 == static_cast<int>(kPartBuckets) ? 0 : b + 1;
             }
             s_beside_slot[tid] = beside;
-            if (at >= 0) {
-                if constexpr (PROV) s_idx[at] = own_row;
-            } else if (beside < 0) {
-                if (!known) atomicAdd(m.ctr + kCtrDropped, 1);   // refused
-                if constexpr (PROV) give_up_row(pl, own_row, &s_losers, false);
+            if constexpr (PROV) {
+                if (at >= 0) s_idx[at] = own_row;
+                if (known) give_up_row(pl, own_row, &s_losers, false);
             }
         }
         __syncthreads();
@@ -1508,31 +1510,13 @@ __global__ __launch_bounds__(kBuildThreads, 8) void build_lists_kernel(
                 if (lane >= d) incl += up;
             }
             s_sum[lane] = incl - v;
-            if (lane == 63) {
-                int at = 0;
-                if (incl > 0) {
-                    at = atomicAdd(m.ctr + kCtrSize, incl);
-                    if (at + incl > m.capacity) {
-                        const int lo = at > m.capacity ? at : m.capacity;
-                        const int excess = at + incl - lo;
-                        atomicSub(m.ctr + kCtrSize, excess);
-                        atomicAdd(m.ctr + kCtrDropped, excess);
-                    }
-                }
-                s_base = at;
-            }
+            if (lane == 63) s_base = incl > 0 ? atomicAdd(m.ctr + kCtrSize, incl) : 0;
         }
         __syncthreads();
-        // the index at `top` of the heap; none left: the slot is given up again
-        auto take = [&](int top, uint64_t& of, int32_t& idx) {
-            if (top < m.capacity) {
-                idx = top;   // (the heap holds 0, 1, 2, ...)
-                m.klog[idx] = of;
-            } else {
-                of = kTomb;
-                idx = -1;
-                atomicAdd(m.ctr + kCtrTombs, 1);
-            }
+        // the index at `top` of the heap
+        auto take = [&](int top, uint64_t of, int32_t& idx) {
+            idx = top;   // (the heap holds 0, 1, 2, ..., and as many as there are keys)
+            m.klog[idx] = of;
         };
 #pragma unroll
         for (int k = 0; k < kRecs; ++k) {
@@ -1557,7 +1541,7 @@ __global__ __launch_bounds__(kBuildThreads, 8) void build_lists_kernel(
         __builtin_nontemporal_store(q < kCodePieces ? code_piece(b, q) : index_piece(b, q), gl + t);
     }
     if (crowded) {
-        __syncthreads();   // (and the stores above are done)
+        __syncthreads();   // (the stores above may still be on their way, but stay ahead: a CU's own, to the same line)
         if (tid < nbeside && s_beside_slot[tid] >= 0) {
             const int b = s_beside_slot[tid] >> 4, slot = s_beside_slot[tid] & 15;
             uint64_t* line = m.buckets + static_cast<size_t>(b0 + b) * kBucketQwords;

@@ -90,3 +90,39 @@ def test_rows_of_unlisted_blocks_are_cleared(gpu_ash, blocks, channels, window):
         want = torch.zeros_like(inputs)
         want[rows] = everywhere[rows]
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("channels,window", [(1, 3), (3, 3), (5, 5), (8, 3), (8, 7)])
+def test_tensors_of_almost_four_gib(gpu_ash, channels, window):
+    """Rows at both ends of the largest tensors, at 2 GiB and on either side of it, each with
+    neighbours among the others and missing ones, against the same blocks in a small tensor;
+    all other rows hold what is no number."""
+    backend = gpu_ash.grid.backend
+    blocks = 0xFFFFFFFF // (2048 * channels)
+    assert backend.lib.ash_convolution_cube_supported(blocks, 8, window, channels, 0)
+    assert not backend.lib.ash_convolution_cube_supported(blocks + 1, 8, window, channels, 0)
+    middle = (1 << 31) // (2048 * channels)
+    g = torch.Generator().manual_seed(window * 10 + channels)
+    apart = torch.randint(4, blocks - 4, (50,), generator=g)
+    rows = torch.unique(torch.cat([torch.tensor([0, 1, 2, blocks - 3, blocks - 2, blocks - 1]),
+                                   torch.arange(middle - 2, middle + 3), apart]))
+    n = len(rows)
+    few = torch.randn(n, 512, channels, generator=g).to(DEV)
+    weights = torch.randn(window, window, window, channels, generator=g).to(DEV)
+    near = torch.randint(n, (n, 27), generator=g)
+    near[torch.rand(n, 27, generator=g) < 0.3] = -1
+    near[:, 13] = torch.arange(n)
+    lut = torch.full((blocks, 27), -1, dtype=torch.int64, device=DEV)
+    lut[rows.to(DEV)] = torch.where(near >= 0, rows[near.clamp_min(0)], -1).to(DEV)
+    inputs = torch.full((blocks, 512, channels), float("nan"), device=DEV)
+    inputs[rows.to(DEV)] = few
+    order = torch.randperm(n, generator=g)
+    got = backend.convolution_cube(inputs, weights, rows[order].to(DEV), lut, 8)
+    grid, _ = _grid(gpu_ash, channels, 20, seed=1)
+    c2g, c2c, _ = grid._window_tables(window // 2)
+    want = backend.convolution_forward(
+        few, weights.view(-1, channels), torch.ones(n, 512, dtype=torch.bool, device=DEV),
+        torch.arange(n, device=DEV), grid.cell_indices, near.to(DEV), c2c, c2g, 8)
+    assert float(want.abs().max()) > 1.0 and torch.equal(got[rows.to(DEV)], want)
+    got[rows.to(DEV)] = 0.0
+    assert int(torch.count_nonzero(got)) == 0   # (what is no number counts)

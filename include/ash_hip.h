@@ -317,7 +317,7 @@ int ash_ray_sample_compact(const int64_t* counts, const int64_t* prefix, const f
  * (sampling: 0 for near_far, 1 for the march), 16-byte aligned, for a map of the
  * blocks volume_lo .. volume_hi (on every axis) that the call makes and then asks
  * instead of the table, or NULL; where that function returns 0 there is none.
- * Blocks outside are looked up as ever. */
+ * Blocks outside are looked up in the table where at least one is stored out there. */
 int64_t ash_ray_volume_bytes(int lo, int hi, int64_t n, int sampling);
 int ash_ray_find_near_far_world(ash_map_t* map, uint8_t* volume, int volume_lo,
                                 int volume_hi, const float* ray_origins,

@@ -87,10 +87,11 @@ struct Shape {
     // the grid ran behind, 16 wavefronts per CU on average).  There one wavefront
     // per channel, and helpers up to a multiple of four that only load and
     // store; where the LDS holds a single workgroup, two per channel are better.
-    // 40 000 blocks, 3^3: three channels 157 -> 129 us, five 293 -> 236, seven
-    // 400 -> 321; 12 000 blocks, 5^3: 155 -> 139, 244 -> 234, 390 -> 298; 4000,
-    // 7^3: 160 -> 146, 261 -> 223, seven (one workgroup) 311 against 324.  Even
-    // numbers that way: 0 - 20 % slower; one channel with helpers 56 -> 71.
+    // 40 000 blocks, 3^3: three channels 101 -> 103 us, five 284 -> 208, seven
+    // 355 -> 278; 12 000 blocks, 5^3: 139 -> 120, 218 -> 208, 299 -> 268; 4000,
+    // 7^3: 129 -> 119, 207 -> 199, seven (one workgroup) 265 against 255 by now.  Even
+    // numbers that way: from 4 % faster (eight, 7^3) to 19 % slower (two, 5^3); one
+    // channel with helpers 39 -> 47.
     static constexpr bool kOneEach = E % 2 == 1 && E > 1 && kFit > 1;
     static constexpr int kY = kOneEach ? 8 : 4;
     static constexpr int kParts = kG / kY;
@@ -106,12 +107,11 @@ struct Shape {
     static constexpr int kEndsEach = (kEnds + kThreads - 1) / kThreads;
     static constexpr int kTaps = W * W;                           // of one dz
     // wavefronts per SIMD that the tile leaves room for.  No more than the
-    // registers allow: 64 for windows of 3 and 72 - 80 for 5 are eight and six, 108
-    // - 128 for 7 are four.  (Five, 96 registers, for 7: 20 000 blocks, one channel
-    // 192 -> 222 us, two 340 -> 344; three, five channels 223 -> 286.)  Five channels,
-    // 5^3, spill 14 registers with six and gain all the same, five against six: 300
-    // blocks 33.8 -> 30.7 us, 1000 40 -> 40, 3000 81 -> 82, 6000 129 -> 125, 12 000
-    // 241 -> 222, 25 000 495 -> 457; four and six channels 165 -> 151 and 281 -> 244
+    // registers allow: 54 - 72 for windows of 3 and 71 - 80 for most of 5 are eight and
+    // six, 104 - 120 for most of 7 are four.  (Five for 7: 4000 blocks of one channel 39.6 ->
+    // 44.6 us, the others alike; three: alike.)  Five channels, 5^3, spill 3 registers with
+    // six and gain all the same, five against six: 1000 blocks 26.6 -> 26.9 us, 12 000
+    // 224 -> 208, 25 000 449 -> 417; four and six channels 153 -> 147 and 246 -> 221
     // at 12 000 without spilling, the others alike.
     // Windows of 3 whose workgroups are a wavefront per SIMD: six (40 000 blocks of
     // one to three channels with eight 44, 75, 130 us, with five to seven 44, 73 - 75, 108).

@@ -285,7 +285,10 @@ __device__ __forceinline__ bool find_key(const MapDev& m, const int32_t (&k)[DIM
 // 7.5 -> 6.6, 300 000 10.8 -> 8.6, 500 000 15.3 -> 12.5, 1 M 23.9 -> 21.9, among 100 000
 // 10.7 -> 9.8 at 500 000, 12.3 -> 12.5 at 700 000, 15.6 -> 16.9 at 1 M, 85 -> 113 at 8 M;
 // with rows of 12 and 4 bytes 131 000 10.2 -> 9.4, 200 000 12.1 -> 11.6, 300 000 14.5
-// -> 14.7, 1 M 41 -> 44.
+// -> 14.7, 1 M 41 -> 44.  Up to the bounds the size of the table does not matter: among four
+// million | sixteen, of which seven in ten are stored, 2^19 16.3 -> 13.7 | 17.9 -> 15.9, with
+// rows 2^18 14.9 -> 15.2 | 15.6 -> 15.3 (all stored 17.1 -> 17.4 | 18.8 -> 19.5, none 13.8
+// -> 9.9 | 13.5 -> 10.2).
 constexpr int64_t kAloneKeys = int64_t{1} << 19, kAloneKeysWithRows = int64_t{1} << 18;
 
 template <int DIM, bool ALONE>
@@ -1396,7 +1399,8 @@ __global__ __launch_bounds__(kBlock) void items_general_kernel(
 // neighbour get -1.  A lane looks its neighbour up by itself, and the widths of the
 // functions here are constants of their own: bound by vector instructions, of which the
 // cooperative probe and divisions by a width from memory were the most (752 of a wavefront;
-// 60 000 blocks of a surface, 8 offsets 15.3 -> 9.1 us, 27 offsets 34.7 -> 23.8; 200 000
+// 60 000 blocks of a surface, 8 offsets 15.3 -> 9.1 us (11 where other work has taken the
+// caches in between), 27 offsets 34.7 -> 23.8; 200 000
 // blocks 37 -> 25 and 106 -> 80; a million scattered ones, lines from behind the L2s, 197
 // -> 123 and 657 -> 431; by a listing, a find and the scattering of both 80 us for the first).
 struct NeighborArgs {
@@ -2753,7 +2757,11 @@ int launch_insert_by(ash_map* map, const int32_t* keys, int64_t n,
 // vector instructions and registers (the kernel with rows of 16 bytes, cooperative ->
 // alone, beside a million keys: 8000 12.5 -> 11.3 us, 65 537 20.8 -> 19.3, 131 000 29.5 ->
 // 27.0, 300 000 39 -> 34; beside 100 000 131 000 36.8 -> 31.7, 196 000 48.6 -> 39; keys
-// alone into an emptied table 16 000 13.1 -> 11.7, 98 000 21.8 -> 20.3); batches beyond
+// alone into an emptied table 16 000 13.1 -> 11.7, 98 000 21.8 -> 20.3).  Keys that are
+// stored already gain as well, beyond where look-ups (kAloneKeys) do not: beside 100 000 | four million | sixteen, a million 19.6 -> 17.4 | 25.0 -> 23.5 | 27.4 -> 24.3, 3.1
+// million 52.5 -> 45.9 | 64.0 -> 62.7 | 70 -> 63; of new keys, each sixteen times, a million
+// 36 -> 33 | 37 -> 35 | 42 -> 37, 3.1 million 82 -> 77 | 90 -> 80 | 95 -> 80; half stored, half
+// new 50 -> 45 | 52 -> 50 | 56 -> 52, 129 -> 126 | 180 -> 169 | 188 -> 165.  Batches beyond
 // are bound by requests, of which that makes more (four million that come and go beside
 // four 600 -> 640, eight beside eight 1137 -> 1245).
 constexpr int64_t kWideInsert = int64_t{3} << 16, kWideInsertEnd = int64_t{3} << 20;

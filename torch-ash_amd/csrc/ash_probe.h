@@ -94,11 +94,12 @@ __device__ bool gen_find(const MapDev& m, const int32_t (&k)[DIM],
 }
 
 // Look-up of one key by one lane on its own (the cooperative probe of
-// ash_map.hip shares a bucket read among eight lanes): the lane reads the ten
-// codes of the key's bucket itself (five 16-byte loads of one 128-byte line).  Far fewer vector
-// instructions per wavefront than the cooperative probe, at the price of one
-// line per lane and load instruction; for kernels whose table is small enough
-// to stay in the caches and that are bound by instructions, not by lines.
+// ash_map.hip shares a bucket read among four lanes): the lane reads the ten
+// codes of the key's bucket itself (five 16-byte loads of one 128-byte line), and the
+// index when it knows the slot.  Far fewer vector instructions per wavefront than the
+// cooperative probe, at the price of five requests per line instead of two: for batches
+// that do not fill the device (kAloneKeys), and for kernels of any size that are bound by
+// their instructions (neighbour tables, the blocks of positions).
 template <int DIM>
 __device__ __forceinline__ bool find_key_alone(const MapDev& m, const int32_t (&k)[DIM],
                                                bool active, int32_t& res) {

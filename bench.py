@@ -88,26 +88,26 @@ VALUE_ROW_BYTES = 2 * (12 + 4)               # color + depth, read and written
 #   atomic_requests: TCC_ATOMIC (all of them are forwarded to the memory side:
 #     TCC_EA0_ATOMIC reads the same).
 MEASURED_COUNTERS = {
-    "insert_values": (2_568_000_000 + 1_939_000_000, 0.364, 16_350_000),
-    "insert_keys": (2_305_000_000 + 1_687_000_000, 0.282, 16_397_000),
+    "insert_values": (2_569_000_000 + 1_940_000_000, 0.362, 16_348_000),
+    "insert_keys": (2_306_000_000 + 1_687_000_000, 0.283, 16_397_000),
     "find": (2_230_000_000 + 145_000_000, 0.064, 0),
-    "erase": (2_236_000_000 + 1_217_000_000, 0.467, 16_031_000),
+    "erase": (2_236_000_000 + 1_216_000_000, 0.467, 16_016_000),
     # the two keys-only split passes and the range pass
     "erase_bulk": (962_000_000 + 1_373_000_000, 0.213, 279_000),
     "items": (128_000_000 + 320_000_000, 0.417, 0),
     "items_values_by_index": (528_000_000 + 256_000_000, 0.247, 0),
     # sums over the split, build and row-copy kernels
-    "insert_values_bulk": (836_000_000 + 1_328_000_000, 0.412, 262_000),
+    "insert_values_bulk": (836_000_000 + 1_328_000_000, 0.412, 263_000),
     "insert_keys_bulk": (450_000_000 + 919_000_000, 0.426, 271_000),
-    "cfg3_forward_linear": (3_502_000_000 + 282_000_000, 0.130, 0),
-    "cfg3_forward_smooth_step": (3_502_000_000 + 282_000_000, 0.130, 0),
-    "cfg4_forward": (377_000_000 + 67_000_000, 0.331, 0),
+    "cfg3_forward_linear": (3_502_000_000 + 282_000_000, 0.129, 0),
+    "cfg3_forward_smooth_step": (3_502_000_000 + 282_000_000, 0.129, 0),
+    "cfg4_forward": (379_000_000 + 67_000_000, 0.331, 0),
     # kernel only: the zero fill of the dense gradient adds 1.64 GB written
-    "cfg4_backward": (438_000_000 + 149_000_000 + 1_638_400_000, 0.113, 2_344_000),
-    "cfg4_double_backward": (486_000_000 + 166_000_000 + 1_638_400_000, 0.122, 2_344_000),
+    "cfg4_backward": (441_000_000 + 149_000_000 + 1_638_400_000, 0.112, 2_344_000),
+    "cfg4_double_backward": (488_000_000 + 166_000_000 + 1_638_400_000, 0.120, 2_344_000),
     "cfg4_grid_query": (71_000_000 + 122_000_000, 0.398, 0),
-    "cfg4_module_forward": (325_000_000 + 72_000_000, 0.404, 0),
-    "cfg4_module_forward_for_training": (326_000_000 + 189_000_000, 0.437, 0),
+    "cfg4_module_forward": (328_000_000 + 72_000_000, 0.402, 0),
+    "cfg4_module_forward_for_training": (329_000_000 + 189_000_000, 0.434, 0),
 }
 
 
@@ -119,7 +119,7 @@ MEASURED_COUNTERS = {
 COUNTERS_SOURCE = {
     "profiles": ["profiles/bench_hbm_traffic_pmc.md",
                  "profiles/bench_l2_hit_rate_and_atomics_pmc.md"],
-    "csrc_sha256": "5cc4fb85697e538bfa803f6d3eb5ea7dea9fc7fd5df5bb89a94186475593410a",
+    "csrc_sha256": "30921e8d860b0fe53b624e3456ada8288778447cdbc7b49230b983595bd17a03",
 }
 
 

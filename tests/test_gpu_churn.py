@@ -86,6 +86,28 @@ def test_copies_of_a_key_meet_in_one_freed_slot(gpu_ash, monkeypatch, policy):
         assert bool(masks.all()) and len(torch.unique(indices)) == len(near)
 
 
+@pytest.mark.parametrize("n", [1, 9, 10, 11, 21])
+def test_copies_of_the_keys_of_one_bucket(gpu_ash, monkeypatch, n):
+    """A bucket's ten slots, tried by every key from one of its own on: keys of one home
+    bucket, each a hundred times in the batch, into an empty map, beside half of them,
+    and behind what was erased."""
+    monkeypatch.setattr(common, "BULK_INSERT", "never")
+    near = _keys_near(100, 1, n)
+    engine = gpu_ash.ASHEngine(3, CAPACITY, DEV)
+    g = torch.Generator(device=DEV).manual_seed(n)
+    for gone in (n, (n + 1) // 2, 1):
+        batch = near.repeat(100, 1)
+        engine.insert_keys(batch[torch.randperm(len(batch), generator=g, device=DEV)])
+        keys, indices = engine.items()
+        assert engine.size() == n == len(torch.unique(keys, dim=0)) == len(torch.unique(indices))
+        found, masks = engine.find(near)
+        filed = torch.zeros(CAPACITY, 3, dtype=torch.int32, device=DEV)
+        filed[indices] = keys
+        assert bool(masks.all()) and torch.equal(filed[found], near)
+        engine.erase(near[:gone])
+        assert engine.size() == n - gone
+
+
 def test_refused_keys_leave_slots_that_later_inserts_take(gpu_ash, monkeypatch):
     """Inserts that do not look for tombstones (none known), into a full map whose
     refused keys have left some, with copies; then those that do, captured ones

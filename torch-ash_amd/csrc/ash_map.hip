@@ -397,6 +397,7 @@ __device__ __forceinline__ void insert_key(
     bool gdup = false;     // kInsertReport: the key stands in the general region
     bool pend = active && fits;
     uint32_t b = bucket_of(code, m.nb);
+    const int turn = first_slot(code);
     uint32_t steps = 0;
 
     bool won = false;      // claimed a packed slot (wb, ws)
@@ -458,8 +459,10 @@ __device__ __forceinline__ void insert_key(
                     }
                     em = claiming ? p.emask | p.tmask : 0u;
                 }
+                em = (em | (em << kSlots)) >> turn & ((1u << kSlots) - 1u);
                 while (em) {
-                    const int s = __builtin_ctz(em);
+                    const int at = __builtin_ctz(em) + turn;
+                    const int s = at < kSlots ? at : at - kSlots;
                     const unsigned long long free = TOMBS && ((p.tmask >> s) & 1u) ? kTomb : kEmpty;
                     const unsigned long long old = atomicCAS(slot_ptr(m, b, s), free, code);
                     if (old == free) {

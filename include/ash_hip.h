@@ -317,8 +317,16 @@ int ash_ray_sample_compact(const int64_t* counts, const int64_t* prefix, const f
  * (sampling: 0 for near_far, 1 for the march), 16-byte aligned, for a map of the
  * blocks volume_lo .. volume_hi (on every axis) that the call makes and then asks
  * instead of the table, or NULL; where that function returns 0 there is none.
- * Blocks outside are looked up in the table where at least one is stored out there. */
+ * Blocks outside are looked up in the table where at least one is stored out there.
+ * The two functions with volume_mark are for callers that keep the scratch: with 0 it
+ * holds anything, is cleared (a launch of its own) and then marked with 1, as by the
+ * functions without; with 1 .. ASH_RAY_VOLUME_MARKS it is one that calls with bounds of
+ * the same bytes have used since it was cleared, on the same stream, of any map, none of
+ * them with this mark. */
+#define ASH_RAY_VOLUME_MARKS 255
 int64_t ash_ray_volume_bytes(int lo, int hi, int64_t n, int sampling);
+/* The same for a map, whose log is read through: 0 for fewer rays than gain that back. */
+int64_t ash_map_ray_volume_bytes(const ash_map_t* map, int lo, int hi, int64_t n, int sampling);
 int ash_ray_find_near_far_world(ash_map_t* map, uint8_t* volume, int volume_lo,
                                 int volume_hi, const float* ray_origins,
                                 const float* ray_directions, const float* origin,
@@ -326,6 +334,13 @@ int ash_ray_find_near_far_world(ash_map_t* map, uint8_t* volume, int volume_lo,
                                 const float* bbox_max, int64_t n, float t_min,
                                 float t_max, float grid2cell_multiplier,
                                 float* ray_nears, float* ray_fars, void* stream);
+int ash_ray_find_near_far_marked(ash_map_t* map, uint8_t* volume, int volume_lo,
+                                 int volume_hi, int volume_mark, const float* ray_origins,
+                                 const float* ray_directions, const float* origin,
+                                 float cell_size, const float* bbox_min,
+                                 const float* bbox_max, int64_t n, float t_min,
+                                 float t_max, float grid2cell_multiplier,
+                                 float* ray_nears, float* ray_fars, void* stream);
 int64_t ash_ray_sample_groups(int64_t n);
 int ash_ray_sample_march(ash_map_t* map, uint8_t* volume, int volume_lo, int volume_hi,
                          const float* ray_origins,
@@ -335,6 +350,15 @@ int ash_ray_sample_march(ash_map_t* map, uint8_t* volume, int volume_lo, int vol
                          int64_t max_samples_per_ray, float grid2cell_multiplier,
                          int64_t* counts, int64_t* groups, float* stage, int64_t stride,
                          int64_t out[2], void* stream);
+int ash_ray_sample_march_marked(ash_map_t* map, uint8_t* volume, int volume_lo,
+                                int volume_hi, int volume_mark, const float* ray_origins,
+                                const float* ray_directions, const float* origin,
+                                float cell_size, const float* ray_nears,
+                                const float* ray_fars, float near_for_all,
+                                float far_for_all, int64_t n, int64_t max_samples_per_ray,
+                                float grid2cell_multiplier, int64_t* counts,
+                                int64_t* groups, float* stage, int64_t stride,
+                                int64_t out[2], void* stream);
 int ash_ray_sample_place(const int64_t* counts, const int64_t* groups, const float* stage,
                          int64_t stride, int64_t n, float cell_size, int64_t* ray_indices,
                          float* t_nears, float* t_fars, int64_t* prefix, void* stream);

@@ -97,3 +97,50 @@ def test_rays_along_axes(gpu_ash, zeros, n):
     # (a block in thirteen is stored, of the sixteen that a ray along an axis passes; a
     # ray that leaves at once from a face passes none)
     assert int((near >= 0).sum()) > n // 4
+
+
+@pytest.mark.parametrize("n,where", [(8195, "one stream"), (8195, "two streams"), (8195, "captured"),
+                                     (1024, "one stream"), (2048, "one stream")])
+def test_blocks_of_earlier_calls_are_not_met(gpu_ash, n, where):
+    """The volume that a map keeps, marked with another number by every call until it is
+    cleared: blocks come and go in between, through more calls than there are numbers."""
+    grid = gpu_ash.BoundedSparseDenseGrid(3, 3000, 1, 8, 32, device=DEV)
+    backend, table = gpu_ash.grid.backend, grid.engine.backend
+    g = torch.Generator().manual_seed(5)
+    keys = torch.randint(0, 32, (2000, 3), generator=g).int().to(DEV)
+    few_rays = backend.lib.ash_map_ray_volume_bytes
+    assert few_rays(table._address, 0, 31, n, 0) > 0 and few_rays(table._address, 0, 31, 1023, 0) == 0
+    o = (torch.rand(n, 3, generator=g) * 256).to(DEV)
+    d = torch.nn.functional.normalize(torch.randn(n, 3, generator=g), dim=1).to(DEV)
+    box = [torch.full((3,), x, device=DEV) for x in (0.0, 256.0)]
+    args = (table, o, d, None, 1.0, *box, 0.0, 800.0, 8.0)
+    streams = [torch.cuda.current_stream(), torch.cuda.Stream()]
+    graph = torch.cuda.CUDAGraph()
+    if where == "captured":
+        grid.engine.insert_keys(keys)   # (a replay lists the blocks as the captured call did)
+        grid.engine.erase(keys)
+        backend.ray_find_near_far_world(*args, (0, 31))
+        with torch.cuda.graph(graph):
+            held = backend.ray_find_near_far_world(*args, (0, 31))
+    for turn in range(300):
+        few = keys[turn * 7 % 1900:][:100]
+        if turn % 2 == 0:
+            grid.engine.insert_keys(few)
+        plain = backend.ray_find_near_far_world(*args)
+        torch.cuda.synchronize()
+        if where == "captured" and turn % 3 == 0:
+            graph.replay()
+            got = held
+        else:
+            with torch.cuda.stream(streams[turn % 2 if where == "two streams" else 0]):
+                bounds = (0, 31) if turn % 5 else (0, 20)
+                got = backend.ray_find_near_far_world(*args, bounds)
+                if turn % 50 < 3:
+                    samples = backend.ray_sample_world(table, o, d, None, 1.0, *got, 64, 8.0, bounds)
+                    for a, b in zip(backend.ray_sample_world(table, o, d, None, 1.0, *got, 64, 8.0), samples):
+                        assert torch.equal(a, b)
+        torch.cuda.synchronize()
+        for a, b in zip(plain, got):
+            assert torch.equal(a, b), turn
+        if turn % 2 == 1:
+            grid.engine.erase(few)

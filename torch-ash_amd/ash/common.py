@@ -136,9 +136,15 @@ _SIGNATURES = {
     ),
     "ash_ray_sample_compact": (ctypes.c_int, [_PTR] * 3 + [_I64, _I64] + [_PTR] * 4),
     "ash_ray_volume_bytes": (_I64, [ctypes.c_int, ctypes.c_int, _I64, ctypes.c_int]),
+    "ash_map_ray_volume_bytes": (_I64, [_PTR, ctypes.c_int, ctypes.c_int, _I64, ctypes.c_int]),
     "ash_ray_find_near_far_world": (
         ctypes.c_int,
         [_PTR, _PTR, ctypes.c_int, ctypes.c_int] + [_PTR] * 3
+        + [ctypes.c_float, _PTR, _PTR, _I64] + [ctypes.c_float] * 3 + [_PTR] * 3,
+    ),
+    "ash_ray_find_near_far_marked": (
+        ctypes.c_int,
+        [_PTR, _PTR] + [ctypes.c_int] * 3 + [_PTR] * 3
         + [ctypes.c_float, _PTR, _PTR, _I64] + [ctypes.c_float] * 3 + [_PTR] * 3,
     ),
     "ash_surface_block8_workspace_bytes": (_I64, [_I64, _I64]),
@@ -156,6 +162,12 @@ _SIGNATURES = {
     "ash_ray_sample_march": (
         ctypes.c_int,
         [_PTR, _PTR, ctypes.c_int, ctypes.c_int] + [_PTR] * 3
+        + [ctypes.c_float, _PTR, _PTR, ctypes.c_float, ctypes.c_float, _I64, _I64,
+           ctypes.c_float, _PTR, _PTR, _PTR, _I64, ctypes.POINTER(_I64), _PTR],
+    ),
+    "ash_ray_sample_march_marked": (
+        ctypes.c_int,
+        [_PTR, _PTR] + [ctypes.c_int] * 3 + [_PTR] * 3
         + [ctypes.c_float, _PTR, _PTR, ctypes.c_float, ctypes.c_float, _I64, _I64,
            ctypes.c_float, _PTR, _PTR, _PTR, _I64, ctypes.POINTER(_I64), _PTR],
     ),
@@ -690,7 +702,7 @@ class _Backend:
         cell_size: the transforms of rays, box and results in the same launch
         (t_min and t_max in cell units).  block_bounds: where the blocks of the
         grid lie (lo, hi; a range that is small enough speeds the look-ups up)."""
-        return self.host.ray_near_far(hashmap._address, hashmap._index, ray_origins, ray_directions,
+        return self.host.ray_near_far(hashmap._address, hashmap._index, hashmap._volumes, ray_origins, ray_directions,
                                       origin, cell_size, bbox_min, bbox_max, t_min, t_max,
                                       grid2cell_multiplier, *block_bounds)
 
@@ -703,7 +715,7 @@ class _Backend:
         stride = max(1, int(max_samples_per_ray) + RAY_STAGE_EXTRA)
         if ray_origins.shape[0] * stride > RAY_STAGE_LIMIT:
             return None
-        return self.host.ray_sample(hashmap._address, hashmap._index, ray_origins, ray_directions,
+        return self.host.ray_sample(hashmap._address, hashmap._index, hashmap._volumes, ray_origins, ray_directions,
                                     origin, cell_size, ray_nears, ray_fars, int(max_samples_per_ray),
                                     grid2cell_multiplier, stride, *block_bounds)
 
@@ -1103,6 +1115,7 @@ class _HashMap:
             )
         self._handle = handle
         self._address, self._index = handle.value, self._device.index
+        self._volumes = self._backend.host.Volumes()
 
     def __del__(self):
         handle, self._handle = getattr(self, "_handle", None), None

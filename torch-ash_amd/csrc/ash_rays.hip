@@ -38,25 +38,32 @@ __device__ __forceinline__ bool uniform(bool c) {
     return __builtin_amdgcn_readfirstlane(static_cast<int>(c)) != 0;
 }
 
-// A byte per block of the cube lo .. lo + edge - 1 (each axis), 1 where the block
-// is stored, in bricks of 4 x 4 x 8 blocks: a ray stays within a line of 128 for
+// A byte per block of the cube lo .. lo + edge - 1 (each axis), `mark` where the block
+// is stored and anything else where it is not, in bricks of 4 x 4 x 8 blocks: a ray stays within a line of 128 for
 // some eight steps.  With it a look-up is one load and fifteen instructions
 // instead of the six loads and eighty of a bucket.  Behind the bytes stands a word
-// that is not zero if a block is stored outside: only then the table is asked about
+// that is `mark` if a block is stored outside: only then the table is asked about
 // blocks out there (a ray that meets nothing is sampled far beyond its grid).
 struct Volume {
     const uint8_t* at;   // null: none
     int32_t lo;
     uint32_t edge;
+    uint32_t mark;       // 1 .. kMostMarks
 };
+constexpr uint32_t kMostMarks = ASH_RAY_VOLUME_MARKS;
 
 // More than this does not stay in an XCD's L2.
 constexpr int64_t kMaxVolume = int64_t{4} << 20;
-// Making it takes two launches of 4 us each, which so many rays gain back: near
-// and far of 3000 rays 15 -> 15 us, 4096 17 -> 14, 8192 29 -> 15, 32 768 79 -> 27;
-// samples of 8000 rays 32 - 57 -> 36 - 48 (few blocks and short rays - many and
-// long), 32 768 37 - 77 -> 38 - 55.
-constexpr int64_t kVolumeRaysNearFar = 4096, kVolumeRaysSampling = 8192;
+// Making it takes a launch of 3 - 4 us (two where it has to be cleared), and longer where
+// the log is long, which so many rays gain back.  Near and far, from the table -> with a
+// volume that need not be cleared, us: 1500 blocks, 1100 rays 10.7 -> 6.7, 4000 15.1 -> 6.9;
+// 200 000 blocks 12.3 -> 8.4, 17.6 -> 9.0; 200 000 of 1.5 M in the log 1000 8.8 -> 9.2, 1500
+// 11.1 -> 9.3; 1.2 M of 1.5 M 2500 14.0 -> 15.5 (cleared, 4096 17 -> 14, 32 768 79 -> 27).
+// Samples, up to 32 | 128 of a ray: 1500 blocks 2100 rays 33.2 -> 34.2 | 39.7 -> 38.2; 30 000
+// 35.7 -> 34.5 | 44.6 -> 40.6; 200 000 36.4 -> 36.2 | 51.0 -> 45.4, 8100 37.6 -> 37.0 | 56.9 ->
+// 45.9; 1.2 M of 1.5 M in the log 2500 34.7 -> 41.3 | 55.7 -> 53.0.
+constexpr int64_t kVolumeRaysNearFar = 1024, kVolumeRaysSampling = 2048;
+constexpr int64_t kVolumeLogPerRay = 384, kVolumeRaysAnyLog = 4096;
 
 __host__ __device__ __forceinline__ int64_t volume_bytes(int64_t edge) {
     const int64_t flat = (edge + 3) / 4, tall = (edge + 7) / 8;
@@ -66,7 +73,7 @@ __host__ __device__ __forceinline__ int64_t volume_bytes(int64_t edge) {
 constexpr int64_t kOutsideBytes = 16;   // of the word
 
 // (to be asked for early and looked at late)
-__device__ __forceinline__ uint32_t stored_outside(const Volume& v) {
+__device__ __forceinline__ uint32_t outside_word(const Volume& v) {
     return *reinterpret_cast<const uint32_t*>(v.at + volume_bytes(v.edge));
 }
 
@@ -114,9 +121,9 @@ __global__ __launch_bounds__(kBlock) void mark_volume_kernel(MapDev m, int ident
     unpack_key<3>(code, block);
     uint32_t at;
     if (code < kTomb && in_volume(v, block, at)) {
-        to[at] = 1;
+        to[at] = static_cast<uint8_t>(v.mark);
     } else {
-        *reinterpret_cast<uint32_t*>(to + volume_bytes(v.edge)) = 1u;
+        *reinterpret_cast<uint32_t*>(to + volume_bytes(v.edge)) = v.mark;
     }
 }
 
@@ -136,7 +143,7 @@ __device__ __forceinline__ void are_stored(const MapDev& m, const Volume& v, con
         others = others | (active[h] & !inside[h]);
     }
 #pragma unroll
-    for (int h = 0; h < K; ++h) stored[h] = inside[h] & (word[h] != 0);
+    for (int h = 0; h < K; ++h) stored[h] = inside[h] & (word[h] == v.mark);
     if (__ballot(others) != 0) {
 #pragma unroll
         for (int h = 0; h < K; ++h) {
@@ -316,7 +323,7 @@ __global__ __launch_bounds__(kBlock) void ray_near_far_pairs_kernel(
     const float* const o_from = origins + 6 * pair;
     const float* const d_from = directions + 6 * pair;
     const float t_grid_step = static_cast<float>(grid2cell * 0.5);
-    const uint32_t outside = stored_outside(volume);
+    const uint32_t outside = outside_word(volume);
     float o[3], d[3], lo[3], hi[3], zero[3] = {0.f, 0.f, 0.f};
     if (u.origin != nullptr) {
 #pragma unroll
@@ -398,7 +405,7 @@ __global__ __launch_bounds__(kBlock) void ray_near_far_pairs_kernel(
     };
     const int ends[2] = {__builtin_amdgcn_readlane(end, 0), __builtin_amdgcn_readlane(end, 32)};
     const int most = ends[0] > ends[1] ? ends[0] : ends[1];
-    if (uniform(outside == 0u)) {
+    if (uniform(outside != volume.mark)) {
         // (exact parameters are also the sums of these steps, and in their order)
         float t = parameter(j);
         const float t_end = parameter(end);
@@ -430,7 +437,7 @@ __global__ __launch_bounds__(kBlock) void ray_near_far_pairs_kernel(
             __builtin_amdgcn_sched_barrier(0);   // (all are on their way before one is waited for)
 #pragma unroll
             for (int h = 0; h < kLooks; ++h) {
-                count(before[h] & __builtin_amdgcn_ballot_w64(word[h] != 0), first + 32 * h);
+                count(before[h] & __builtin_amdgcn_ballot_w64(word[h] == volume.mark), first + 32 * h);
             }
         };
         int first = 0;
@@ -511,8 +518,8 @@ __global__ __launch_bounds__(kBlock) void ray_sample_kernel(
     const int64_t from = active ? i : n - 1;
     float o[3], d[3], zero[3] = {0.f, 0.f, 0.f};
     float ray_near = near_for_all, ray_far = far_for_all;
-    uint32_t outside_word = 0;
-    if constexpr (VOLUME) outside_word = stored_outside(volume);
+    uint32_t beyond = 0;
+    if constexpr (VOLUME) beyond = outside_word(volume);
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         o[a] = origins[from * 3 + a];
@@ -551,7 +558,7 @@ __global__ __launch_bounds__(kBlock) void ray_sample_kernel(
     bool outside = false, odd = false;
     uint32_t last_byte = 0;
     if constexpr (VOLUME) {
-        outside = uniform(outside_word != 0u);
+        outside = uniform(beyond == volume.mark);
         odd = !(fabsf(o[0]) + fabsf(o[1]) + fabsf(o[2]) + fabsf(d[0]) + fabsf(d[1]) + fabsf(d[2]) < INFINITY);
         last_byte = static_cast<uint32_t>(volume_bytes(volume.edge) - 1);
     }
@@ -600,7 +607,7 @@ __global__ __launch_bounds__(kBlock) void ray_sample_kernel(
             // (outside: anywhere)
             const uint32_t where = volume_offset(volume, p);
             stored = __builtin_amdgcn_ballot_w64(outermost(p) < volume.edge) &
-                     __builtin_amdgcn_ballot_w64(volume.at[where < last_byte ? where : last_byte] != 0);
+                     __builtin_amdgcn_ballot_w64(volume.at[where < last_byte ? where : last_byte] == volume.mark);
         }
         const uint64_t expected = stands & ~(stored ^ __builtin_amdgcn_ballot_w64(run_stored));
         // a ray takes its steps up to the first that is not as expected: the ones at the
@@ -821,18 +828,24 @@ int launch_march(ash_map_t* map, const Volume& volume, const March& r, int64_t* 
     return 0;
 }
 
-// The volume of the map's blocks in lo .. hi, if there is room for one.
-int make_volume(ash_map_t* map, uint8_t* bytes, int lo, int hi, Volume& v, hipStream_t s) {
+// The volume of the map's blocks in lo .. hi, if there is room for one.  `mark` 0: its
+// bytes hold anything and are cleared; else none of them holds `mark`.  (A call that
+// clears launches one kernel more, 3 - 4 us.)
+int make_volume(ash_map_t* map, uint8_t* bytes, int lo, int hi, int mark, Volume& v, hipStream_t s) {
     v = {};
     if (bytes == nullptr) return 0;
+    if (mark < 0 || mark > static_cast<int>(kMostMarks)) ASH_FAIL("rays: a volume's mark must be 0 .. 255");
     const int64_t edge = static_cast<int64_t>(hi) - lo + 1;
     if (edge < 1 || volume_bytes(edge) > kMaxVolume) ASH_FAIL("rays: too many blocks for a volume");
     if (reinterpret_cast<uintptr_t>(bytes) % 16 != 0) ASH_FAIL("rays: the volume must be 16-byte aligned");
-    v = {bytes, lo, static_cast<uint32_t>(edge)};
-    const int64_t units = (volume_bytes(edge) + kOutsideBytes) / 16;
-    clear_volume_kernel<<<static_cast<unsigned>((units + kBlock - 1) / kBlock), kBlock, 0, s>>>(
-            reinterpret_cast<uint4*>(bytes), units);
-    ASH_LAUNCH_CHECK();
+    v = {bytes, lo, static_cast<uint32_t>(edge), static_cast<uint32_t>(mark)};
+    if (mark == 0) {
+        v.mark = 1;
+        const int64_t units = (volume_bytes(edge) + kOutsideBytes) / 16;
+        clear_volume_kernel<<<static_cast<unsigned>((units + kBlock - 1) / kBlock), kBlock, 0, s>>>(
+                reinterpret_cast<uint4*>(bytes), units);
+        ASH_LAUNCH_CHECK();
+    }
     mark_volume_kernel<<<static_cast<unsigned>((map->capacity + kBlock - 1) / kBlock), kBlock, 0, s>>>(
             map->d, heap_in_order(map) ? 1 : 0, v, bytes);
     ASH_LAUNCH_CHECK();
@@ -861,7 +874,7 @@ float last_place(float x) {
     return std::ldexp(static_cast<float>(digits & (0u - digits)), e - 24);
 }
 
-int near_far(ash_map_t* map, uint8_t* bytes, int lo, int hi, const float* origins, const float* directions, const RayUnits& units,
+int near_far(ash_map_t* map, uint8_t* bytes, int lo, int hi, int mark, const float* origins, const float* directions, const RayUnits& units,
              const float* bbox_min, const float* bbox_max, int64_t n, float t_min, float t_max,
              float grid2cell, float* nears, float* fars, hipStream_t s) {
     if (check_rays(map, origins, directions, n, grid2cell, units.cell)) return 1;
@@ -882,7 +895,7 @@ int near_far(ash_map_t* map, uint8_t* bytes, int lo, int hi, const float* origin
         }
     }
     Volume volume;
-    if (make_volume(map, bytes, lo, hi, volume, s)) return 1;
+    if (make_volume(map, bytes, lo, hi, mark, volume, s)) return 1;
     StepChain chain;
     float t = t_min;
     for (int k = 0; k < kChain; ++k) {
@@ -936,7 +949,7 @@ int ash_ray_find_near_far(ash_map_t* map, const float* ray_origins,
                           float t_max, float t_step, float grid2cell_multiplier,
                           float* ray_nears, float* ray_fars, void* stream) {
     (void)t_step;  // unused by the reference as well (ash/src/sampler.cu:21)
-    return near_far(map, nullptr, 0, 0, ray_origins, ray_directions, kCellUnits, bbox_min, bbox_max, n, t_min,
+    return near_far(map, nullptr, 0, 0, 0, ray_origins, ray_directions, kCellUnits, bbox_min, bbox_max, n, t_min,
                     t_max, grid2cell_multiplier, ray_nears, ray_fars,
                     static_cast<hipStream_t>(stream));
 }
@@ -949,15 +962,32 @@ int64_t ash_ray_volume_bytes(int lo, int hi, int64_t n, int sampling) {
     return bytes <= kMaxVolume ? bytes + kOutsideBytes : 0;
 }
 
+int64_t ash_map_ray_volume_bytes(const ash_map_t* map, int lo, int hi, int64_t n, int sampling) {
+    if (map == nullptr) return 0;
+    if (n < kVolumeRaysAnyLog && map->capacity > n * kVolumeLogPerRay) return 0;
+    return ash_ray_volume_bytes(lo, hi, n, sampling);
+}
+
+int ash_ray_find_near_far_marked(ash_map_t* map, uint8_t* volume, int volume_lo, int volume_hi,
+                                 int volume_mark, const float* ray_origins,
+                                 const float* ray_directions, const float* origin, float cell_size,
+                                 const float* bbox_min, const float* bbox_max, int64_t n, float t_min,
+                                 float t_max, float grid2cell_multiplier, float* ray_nears,
+                                 float* ray_fars, void* stream) {
+    return near_far(map, volume, volume_lo, volume_hi, volume_mark, ray_origins, ray_directions,
+                    {origin, 1.0f / cell_size, cell_size}, bbox_min, bbox_max, n, t_min, t_max,
+                    grid2cell_multiplier, ray_nears, ray_fars, static_cast<hipStream_t>(stream));
+}
+
 int ash_ray_find_near_far_world(ash_map_t* map, uint8_t* volume, int volume_lo, int volume_hi,
                                 const float* ray_origins,
                                 const float* ray_directions, const float* origin, float cell_size,
                                 const float* bbox_min, const float* bbox_max, int64_t n, float t_min,
                                 float t_max, float grid2cell_multiplier, float* ray_nears,
                                 float* ray_fars, void* stream) {
-    return near_far(map, volume, volume_lo, volume_hi, ray_origins, ray_directions, {origin, 1.0f / cell_size, cell_size}, bbox_min,
-                    bbox_max, n, t_min, t_max, grid2cell_multiplier, ray_nears, ray_fars,
-                    static_cast<hipStream_t>(stream));
+    return ash_ray_find_near_far_marked(map, volume, volume_lo, volume_hi, 0, ray_origins, ray_directions,
+                                        origin, cell_size, bbox_min, bbox_max, n, t_min, t_max,
+                                        grid2cell_multiplier, ray_nears, ray_fars, stream);
 }
 
 int ash_ray_sample(ash_map_t* map, const float* ray_origins,
@@ -1027,13 +1057,13 @@ int ash_ray_sample_compact(const int64_t* counts, const int64_t* prefix, const f
 
 int64_t ash_ray_sample_groups(int64_t n) { return n > 0 ? static_cast<int64_t>(march_groups(n)) : 0; }
 
-int ash_ray_sample_march(ash_map_t* map, uint8_t* scratch, int volume_lo, int volume_hi,
-                         const float* ray_origins, const float* ray_directions,
-                         const float* origin, float cell_size, const float* ray_nears,
-                         const float* ray_fars, float near_for_all, float far_for_all, int64_t n,
-                         int64_t max_samples_per_ray, float grid2cell_multiplier, int64_t* counts,
-                         int64_t* groups, float* stage, int64_t stride, int64_t out[2],
-                         void* stream) {
+int ash_ray_sample_march_marked(ash_map_t* map, uint8_t* scratch, int volume_lo, int volume_hi,
+                                int volume_mark, const float* ray_origins,
+                                const float* ray_directions, const float* origin, float cell_size,
+                                const float* ray_nears, const float* ray_fars, float near_for_all,
+                                float far_for_all, int64_t n, int64_t max_samples_per_ray,
+                                float grid2cell_multiplier, int64_t* counts, int64_t* groups,
+                                float* stage, int64_t stride, int64_t out[2], void* stream) {
     if (check_rays(map, ray_origins, ray_directions, n, grid2cell_multiplier, cell_size)) return 1;
     if (max_samples_per_ray < 1) ASH_FAIL("max_samples_per_ray must be positive");
     if (stride < 1) ASH_FAIL("ray_sample_march: stride must be positive");
@@ -1055,7 +1085,7 @@ int ash_ray_sample_march(ash_map_t* map, uint8_t* scratch, int volume_lo, int vo
     Answer answer;
     if (answer.take()) return 1;
     Volume volume;
-    if (make_volume(map, scratch, volume_lo, volume_hi, volume, s)) return 1;
+    if (make_volume(map, scratch, volume_lo, volume_hi, volume_mark, volume, s)) return 1;
     auto* g = reinterpret_cast<GroupSamples*>(groups);
     if (launch_march(map, volume, {ray_origins, ray_directions, {origin, 1.0f / cell_size, cell_size}, ray_nears,
                            ray_fars, near_for_all, far_for_all, n,
@@ -1068,6 +1098,19 @@ int ash_ray_sample_march(ash_map_t* map, uint8_t* scratch, int volume_lo, int vo
     if (answer.wait(s, 4)) return 1;
     for (int w = 0; w < 2; ++w) out[w] = answer.pair(2 * w);
     return 0;
+}
+
+int ash_ray_sample_march(ash_map_t* map, uint8_t* volume, int volume_lo, int volume_hi,
+                         const float* ray_origins, const float* ray_directions,
+                         const float* origin, float cell_size, const float* ray_nears,
+                         const float* ray_fars, float near_for_all, float far_for_all, int64_t n,
+                         int64_t max_samples_per_ray, float grid2cell_multiplier, int64_t* counts,
+                         int64_t* groups, float* stage, int64_t stride, int64_t out[2],
+                         void* stream) {
+    return ash_ray_sample_march_marked(map, volume, volume_lo, volume_hi, 0, ray_origins, ray_directions,
+                                       origin, cell_size, ray_nears, ray_fars, near_for_all, far_for_all,
+                                       n, max_samples_per_ray, grid2cell_multiplier, counts, groups,
+                                       stage, stride, out, stream);
 }
 
 int ash_ray_sample_place(const int64_t* counts, const int64_t* groups, const float* stage,

@@ -88,3 +88,22 @@ def test_any_number_of_crossed_cells_in_a_block(gpu_ash, field, light):
         grid.lut_cell_nb2cell_idx, grid.lut_cell_nb2grid_nb, 8, 0.0, 0.5)
     assert torch.equal(triangles, want) and torch.equal(vertices, grid.transform_cell_to_world(points))
     assert len(want) > 300
+
+
+@pytest.mark.parametrize("blocks", [64, 700])
+def test_rows_listed_before_and_not_now(gpu_ash, blocks):
+    """The workspace is not cleared and comes back from call to call: rows of blocks that
+    have gone, whose places of the call before name others now, or none."""
+    grid, g = _grid(gpu_ash, blocks, True, seed=blocks)
+    backend = gpu_ash.grid.backend
+    rows = torch.randn(grid.num_embeddings, 512, 2, generator=g).to(DEV)
+    for turn in range(6):
+        grid.construct_grid_neighbor_lut_(radius=1, bidirectional=False)
+        triangles, vertices = grid.surface_mesh(rows[..., 0], rows[..., 1], 0.1, -0.5)
+        _, listed = grid._blocks_in_spatial_order()
+        want, points = backend.marching_cubes(
+            rows[..., 0], rows[..., 1], listed, grid.grid_coords, grid.lut_grid_nb2grid_idx, grid.cell_coords,
+            grid.lut_cell_nb2cell_idx, grid.lut_cell_nb2grid_nb, 8, 0.1, -0.5)
+        assert torch.equal(triangles, want) and torch.equal(vertices, grid.transform_cell_to_world(points))
+        keys = grid.engine.items()[0]
+        grid.engine.erase(keys[torch.randperm(len(keys), generator=g)[:len(keys) // 3].to(DEV)])

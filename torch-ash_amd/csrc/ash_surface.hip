@@ -22,12 +22,12 @@
 //   points, triangles
 //            a wavefront per block lists the block's points / triangles in LDS
 //            and consecutive lanes handle consecutive ones.  A vertex id is the
-//            start of the row plus the flags below the edge's
+//            start of the row plus the flags below the edge's.  One launch for both
 //
-// 60 000 blocks, field and weights in rows of five channels, us: listing 9, bits
-// 99, classify 26, count and scan 20, points 48, triangles 56, together 258; with
-// case bytes, a slot word per cell and the two channels copied out first: copies
-// 274, clear, classify, count, points and triangles 415.
+// 60 000 blocks, field and weights in rows of five channels, us: listing 5, bits
+// 98, classify 27, count and scan 20, points and triangles 99 (51 and 61 one after the
+// other), together 249; with case bytes, a slot word per cell and the two channels copied
+// out first: copies 274, clear, classify, count, points and triangles 415.
 //
 // Vertices are numbered along the listing, cells in order within a block, the
 // axes in order within a cell, and triangles likewise: as in ash_mesh.hip.
@@ -70,7 +70,7 @@ struct Work {
     uint64_t* faces;    // [B, 8]   edges of the low-face cells that neighbours flag
     uint32_t* rows;     // [B, 64]  three flag bytes | points before in the layer << 24
     uint16_t* layer;    // [B, 8]   points before the layer in the block
-    uint32_t* first;    // [B]      first point of the block
+    uint32_t* place;    // [B]      where the block stands in the listing (place_of)
     uint2* local;       // [n]      points and triangles before the listed block in its group
     Sums* groups;       // [ceil(n / kGroupBlocks)]
 };
@@ -108,26 +108,28 @@ int64_t lay_out(Work& w, char* base, int64_t n, int64_t B) {
     take(w.faces, 8 * B);
     take(w.rows, 64 * B);
     take(w.layer, 8 * B);
-    take(w.first, B);
+    take(w.place, B);
     take(w.local, n);
     take(w.groups, groups_of(n));
     return at;
 }
 
-// Which rows are listed, in `first` (where the points' kernel puts a block's first
-// point later): blocks that are not listed count as missing, their bits are zero.
-__global__ __launch_bounds__(kBlock) void clear_listed_kernel(uint32_t* listed, int64_t B) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-    if (i < B) listed[i] = 0;
-}
-
-__global__ __launch_bounds__(kBlock) void mark_listed_kernel(const int64_t* __restrict__ grid_indices,
-                                                             int64_t n, int64_t B,
-                                                             uint32_t* __restrict__ listed) {
+// Where the rows stand in the listing.  Rows that are not listed are not cleared (a
+// launch less): whatever stands there, the listing does not name them at that place.
+__global__ __launch_bounds__(kBlock) void place_listed_kernel(const int64_t* __restrict__ grid_indices,
+                                                              int64_t n, int64_t B,
+                                                              uint32_t* __restrict__ place) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
     if (i >= n) return;
     const int64_t g = grid_indices[i];
-    if (g >= 0 && g < B) listed[g] = 1;
+    if (g >= 0 && g < B) place[g] = static_cast<uint32_t>(i);
+}
+
+// The place of row g, or -1 where it is not listed: blocks that are not listed count
+// as missing, their bits are zero.
+__device__ __forceinline__ int64_t place_of(const SurfaceArgs& a, int64_t g) {
+    const int64_t at = a.w.place[g];
+    return at < a.n && a.grid_indices[at] == g ? at : -1;
 }
 
 // The bits of row g from the values of its cells, one layer per register: every
@@ -157,10 +159,14 @@ __global__ __launch_bounds__(kBlock) void bits_kernel(SurfaceArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t g = static_cast<int64_t>(blockIdx.x) * (kBlock / 64) + wave;
     if (g >= a.B) return;
-    if (a.w.first[g] == 0) {
+    const auto nothing = [&] {
         if (lane < 16) a.w.bits[g * 16 + lane] = 0;
-        return;
-    }
+    };
+    // (a place that may be the row's as a rule is: the rows are asked for along with the
+    // listing)
+    const int64_t at_most = a.w.place[g];
+    if (at_most >= a.n) return nothing();
+    const int64_t listed = a.grid_indices[at_most];
     const T* sdfs = static_cast<const T*>(a.sdfs) + g * kM * a.sdf_stride;
     const T* weights = static_cast<const T*>(a.weights) + g * kM * a.weight_stride;
     const int s = static_cast<int>(a.sdf_stride), t = static_cast<int>(a.weight_stride);
@@ -170,6 +176,7 @@ __global__ __launch_bounds__(kBlock) void bits_kernel(SurfaceArgs a) {
         v[z] = sdfs[(z * 64 + lane) * s];
         w[z] = weights[(z * 64 + lane) * t];
     }
+    if (listed != g) return nothing();
     leave_bits(a, g, v, w);
 }
 
@@ -187,10 +194,12 @@ __global__ __launch_bounds__(kBlock) void bits_staged_kernel(SurfaceArgs a, cons
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t g = static_cast<int64_t>(blockIdx.x) * (kBlock / 64) + wave;
     if (g >= a.B) return;
-    if (a.w.first[g] == 0) {
+    const auto nothing = [&] {
         if (lane < 16) a.w.bits[g * 16 + lane] = 0;
-        return;
-    }
+    };
+    const int64_t at_most = a.w.place[g];   // (as above)
+    if (at_most >= a.n) return nothing();
+    const int64_t listed = a.grid_indices[at_most];
     // up to the last value that is needed: the rows may end with it
     const int pieces = ((kM - 1) * S + (sdf > weight ? sdf : weight)) / 4 + 1;
     const v4* rows = reinterpret_cast<const v4*>(at + g * (kM * S));
@@ -200,6 +209,7 @@ __global__ __launch_bounds__(kBlock) void bits_staged_kernel(SurfaceArgs a, cons
         const int p = i * 64 + lane;
         piece[i] = __builtin_nontemporal_load(rows + (p < pieces ? p : 0));
     }
+    if (listed != g) return nothing();
 #pragma unroll
     for (int i = 0; i < 2 * S; ++i) s_rows[wave][i * 64 + lane] = piece[i];
     // (a wavefront's own: its LDS instructions execute in order)
@@ -239,8 +249,9 @@ struct Blocks {
         const int64_t r = a.lut_g[g * 8 + s];
         return (r >= 0 && r < a.B) ? r : -1;
     }
-    __device__ __forceinline__ Blocks(const SurfaceArgs& args)
-        : a(args), walk(args.n), at(walk.next) {
+    __device__ __forceinline__ Blocks(const SurfaceArgs& args) : Blocks(args, blockIdx.x, gridDim.x) {}
+    __device__ __forceinline__ Blocks(const SurfaceArgs& args, unsigned group, unsigned groups)
+        : a(args), walk(args.n, group, groups), at(walk.next) {
         own = index(at);
         next_own = index(at + walk.step);
         row = source(own);
@@ -549,13 +560,16 @@ __device__ __forceinline__ float to_world(float p, float scale, const float* ori
 // The zero crossing of every flagged edge, linear between its two ends
 // (ash/src/grid.cu:748-771).  Bound by the lines of the field that its cells and
 // their partners lie in.
+struct PointLists {
+    uint16_t point[3 * kM];   // cell | axis << 9
+};
+
 template <typename T>
-__global__ __launch_bounds__(64) void points_kernel(SurfaceArgs a) {
-    __shared__ uint16_t s_point[3 * kM];   // cell | axis << 9
+__device__ __forceinline__ void points_of(const SurfaceArgs& a, Blocks& blk, PointLists& lists) {
+    uint16_t* const s_point = lists.point;
     const T* sdfs = static_cast<const T*>(a.sdfs);
     const int lane = threadIdx.x;
     const int row0 = (lane & 7) * kG + (lane >> 3) * 64;   // first cell of the lane's row
-    Blocks blk(a);
     // what the next block's list is made from is fetched while this one's points are
     uint32_t next_word = 0;
     int next_layer = 0;
@@ -576,7 +590,6 @@ __global__ __launch_bounds__(64) void points_kernel(SurfaceArgs a) {
         if (g < 0) continue;   // the same for the whole wavefront
         const uint32_t flags = word & kRowBits;
         if (__ballot(flags != 0u) == 0) continue;
-        if (lane == 0) a.w.first[g] = static_cast<uint32_t>(first);
         const int total = __shfl(at + __popc(flags), 63);
         __syncthreads();   // the previous block's list has been read
         for (uint32_t left = (flags | (flags >> 8) | (flags >> 16)) & 0xFFu; left != 0u; left &= left - 1u) {
@@ -620,32 +633,45 @@ __global__ __launch_bounds__(64) void points_kernel(SurfaceArgs a) {
 // Triangles of every crossed cell as ids of the points on its edges
 // (ash/src/grid.cu:796-842); the table's rows have the orientation the reference
 // writes.
-__global__ __launch_bounds__(64) void triangles_kernel(SurfaceArgs a) {
-    constexpr int kRows = (kG + 1) * (kG + 1);
-    __shared__ __align__(16) uint8_t s_bits[8 * 128];
-    __shared__ uint64_t s_table[256];
-    __shared__ uint8_t s_count[256];
-    __shared__ uint8_t s_case[kM];
-    __shared__ uint2 s_rows[64];
-    __shared__ uint16_t s_triangle[5 * kRoundCells];   // cell | number in the cell << 9
+struct TriangleLists {
+    static constexpr int kRows = (kG + 1) * (kG + 1);
+    __align__(16) uint8_t bits[8 * 128];        // of the eight sources; then the crossed cells
+    uint2 rows[64];
+    uint8_t case_of[kRoundCells];               // of the round's crossed cells
+    uint16_t triangle[5 * kRoundCells];         // of the round: crossed cell | number in the cell << 8
+    uint32_t flags[2 * kRows];                  // rows (y, z) of the block and of its +x neighbours
+    uint32_t first[2 * kRows];
+};
+
+__device__ __forceinline__ void triangles_of(const SurfaceArgs& a, Blocks& blk, TriangleLists& lists) {
+    constexpr int kRows = TriangleLists::kRows;
+    uint8_t* const s_bits = lists.bits;
+    uint8_t* const s_case = lists.case_of;
+    uint2* const s_rows = lists.rows;
+    uint16_t* const s_triangle = lists.triangle;
     uint16_t* const s_cell = reinterpret_cast<uint16_t*>(s_bits);   // (the bits are read by then)
-    static_assert(sizeof(s_bits) >= kM * sizeof(uint16_t), "all cells of a block");
-    __shared__ uint32_t s_flags[2 * kRows];               // rows (y, z) of the block and of its +x neighbours
-    __shared__ uint32_t s_first[2 * kRows];
+    static_assert(sizeof(lists.bits) >= kM * sizeof(uint16_t), "all cells of a block");
+    uint32_t* const s_flags = lists.flags;
+    uint32_t* const s_first = lists.first;
     const int lane = threadIdx.x;
-    for (int i = lane; i < 256; i += 64) {
-        s_table[i] = kMcPackedRows[i];
-        s_count[i] = static_cast<uint8_t>(kMcTriangleCount[i]);
-    }
-    Blocks blk(a);
+    // The first point of the lane's source, of this block and, a block ahead, of the next
+    // (which is listed, or flags no edge).
+    auto first_point = [&](int64_t place) {
+        return place < 0 ? 0u : static_cast<uint32_t>(a.w.groups[place / kGroupBlocks].points) + a.w.local[place].x;
+    };
+    auto place = [&](int64_t r) { return r < 0 ? int64_t{-1} : place_of(a, r); };
+    uint32_t source_first = first_point(place(blk.row));
     uint4 piece = blk.piece();
     for (; blk.more(); blk.advance()) {
         __syncthreads();   // the previous block's lists have been read
         reinterpret_cast<uint4*>(s_bits)[lane] = piece;
         __syncthreads();
         piece = blk.next_piece();   // on its way while this block is worked on
-        if (blk.own < 0) continue;   // the same for the whole wavefront
+        const uint32_t starts = source_first;
+        const int64_t next_place = place(blk.next_row);
         const RowCells r = row_cells(s_bits);
+        source_first = first_point(next_place);
+        if (blk.own < 0) continue;   // the same for the whole wavefront
         if (__ballot(r.crossed != 0u) == 0) continue;
         int64_t first = a.w.groups[blk.at / kGroupBlocks].triangles + a.w.local[blk.at].y;
 #pragma unroll
@@ -655,11 +681,12 @@ __global__ __launch_bounds__(64) void triangles_kernel(SurfaceArgs a) {
             const int y = p % (kG + 1), z = p / (kG + 1);
             const int s = side | ((y >> 3) << 1) | ((z >> 3) << 2);
             const int64_t g = __shfl(blk.row, (s & 7) * 8);
+            const uint32_t start = static_cast<uint32_t>(__shfl(static_cast<int>(starts), (s & 7) * 8));
             if (i >= 2 * kRows) continue;
             uint32_t word = 0, id = 0;
             if (g >= 0) {
                 word = a.w.rows[g * 64 + (y & 7) + 8 * (z & 7)];
-                id = a.w.first[g] + a.w.layer[g * 8 + (z & 7)] + (word >> 24);
+                id = start + a.w.layer[g * 8 + (z & 7)] + (word >> 24);
             }
             s_flags[i] = word & kRowBits;
             s_first[i] = id;
@@ -672,24 +699,24 @@ __global__ __launch_bounds__(64) void triangles_kernel(SurfaceArgs a) {
             int listed = 0;
             for (int c = c0; c < crossed && c < c0 + kRoundCells; c += 64) {
                 const bool any = c + lane < crossed;
-                const int cell = any ? s_cell[c + lane] : 0;
-                const uint32_t code = case_at(s_rows, cell);
-                const int n = any ? s_count[code] : 0;
-                if (any) s_case[cell] = static_cast<uint8_t>(code);
+                const int at = c - c0 + lane;
+                const uint32_t code = any ? case_at(s_rows, s_cell[c + lane]) : 0u;
+                const int n = kMcTriangleCount[code];   // (none of case 0)
+                if (any) s_case[at] = static_cast<uint8_t>(code);
                 const int upto = sum_up_to(n);
                 const int to = listed + upto - n;
 #pragma unroll
                 for (int t = 0; t < 5; ++t) {
-                    if (t < n) s_triangle[to + t] = static_cast<uint16_t>(cell | (t << 9));
+                    if (t < n) s_triangle[to + t] = static_cast<uint16_t>(at | (t << 8));
                 }
                 listed += last_lane(upto);
             }
             __syncthreads();
             for (int q = lane; q < listed; q += 64) {
                 if (first + q >= a.n_triangles) continue;   // never with the totals of the scan
-                const int cell = s_triangle[q] & (kM - 1);
-                const int t = s_triangle[q] >> 9;
-                const uint32_t edges = static_cast<uint32_t>(s_table[s_case[cell]] >> (12 * t));
+                const int at = s_triangle[q] & 0xFF, t = s_triangle[q] >> 8;
+                const int cell = s_cell[c0 + at];
+                const uint32_t edges = static_cast<uint32_t>(kMcPackedRows[s_case[at]] >> (12 * t));
                 const int x = cell & 7, y = (cell >> 3) & 7, z = cell >> 6;
                 int32_t* out = a.triangles + (first + q) * 3;
 #pragma unroll
@@ -710,6 +737,25 @@ __global__ __launch_bounds__(64) void triangles_kernel(SurfaceArgs a) {
             first += listed;
         }
     }
+}
+
+// Points and triangles by one launch, half of the workgroups each, of which every XCD has
+// as many: the points wait for memory, the triangles for their vector instructions, and
+// neither needs the other.  60 000 blocks of five channels, us: two launches 51 + 61, one
+// 114 while the triangles kept their tables in LDS (7.6 KB a wavefront, 21 on a CU, of both
+// kinds), 99 with the tables in the L1 and lists by round (4.9 KB, 28 on a CU); 27 000 of two
+// channels 21 + 29 -> 42, 6000 of five 10 + 11 -> 15, 700 of two 7 + 7 -> 8.  Held to 64
+// registers (32 on a CU) 102; lists of 128 cells instead of 192 101.
+template <typename T>
+__global__ __launch_bounds__(64) void extract_kernel(SurfaceArgs a) {
+    __shared__ union {
+        PointLists points;
+        TriangleLists triangles;
+    } s;
+    const unsigned pair = blockIdx.x / (2 * kXcds), side = blockIdx.x / kXcds % 2;
+    Blocks blk(a, pair * kXcds + blockIdx.x % kXcds, gridDim.x / 2);
+    if (side == 0) points_of<T>(a, blk, s.points);
+    else triangles_of(a, blk, s.triangles);
 }
 
 unsigned walk_grid(int64_t n) { return static_cast<unsigned>(n < kWalkGroups ? n : kWalkGroups); }
@@ -820,11 +866,8 @@ int ash_surface_block8_classify(ash_map_t* map, const void* sdfs, int64_t sdf_st
     ASH_HIP(guard.enter(map->device));
     Answer answer;
     if (answer.take()) return 1;
-    clear_listed_kernel<<<static_cast<unsigned>((num_embeddings + kBlock - 1) / kBlock), kBlock, 0, s>>>(
-            a.w.first, num_embeddings);
-    ASH_LAUNCH_CHECK();
-    mark_listed_kernel<<<static_cast<unsigned>((num_grids + kBlock - 1) / kBlock), kBlock, 0, s>>>(
-            grid_indices, num_grids, num_embeddings, a.w.first);
+    place_listed_kernel<<<static_cast<unsigned>((num_grids + kBlock - 1) / kBlock), kBlock, 0, s>>>(
+            grid_indices, num_grids, num_embeddings, a.w.place);
     ASH_LAUNCH_CHECK();
     if (launch_bits(a, dtype, s)) return 1;
     classify_kernel<<<walk_grid(num_grids), 64, 0, s>>>(a);
@@ -869,16 +912,10 @@ int ash_surface_block8_extract(const void* sdfs, int64_t sdf_stride, const int64
     PointerGuard guard;
     ASH_HIP(guard.enter_for(sdfs));
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (dtype == ASH_F32) {
-        points_kernel<float><<<walk_grid(num_grids), 64, 0, s>>>(a);
-    } else {
-        points_kernel<double><<<walk_grid(num_grids), 64, 0, s>>>(a);
-    }
+    const unsigned groups = 2 * ((walk_grid(num_grids) + kXcds - 1) / kXcds * kXcds);
+    auto kernel = dtype == ASH_F32 ? extract_kernel<float> : extract_kernel<double>;
+    kernel<<<groups, 64, 0, s>>>(a);
     ASH_LAUNCH_CHECK();
-    if (n_triangles > 0) {
-        triangles_kernel<<<walk_grid(num_grids), 64, 0, s>>>(a);
-        ASH_LAUNCH_CHECK();
-    }
     return 0;
 }
 

@@ -16,11 +16,13 @@ struct TileWalk {
     int64_t next;
     int64_t end;
     int64_t step;
-    __device__ __forceinline__ TileWalk(int64_t ntiles) {
+    __device__ __forceinline__ TileWalk(int64_t ntiles) : TileWalk(ntiles, blockIdx.x, gridDim.x) {}
+    // the `group`-th of `groups` workgroups, on the XCD of its number
+    __device__ __forceinline__ TileWalk(int64_t ntiles, unsigned group, unsigned groups) {
         const int64_t per_xcd = (ntiles + kXcds - 1) / kXcds;
-        const int xcd = blockIdx.x % kXcds;
-        const int slot = blockIdx.x / kXcds;
-        step = (gridDim.x + kXcds - 1 - xcd) / kXcds;  // workgroups on this XCD
+        const int xcd = group % kXcds;
+        const int slot = group / kXcds;
+        step = (groups + kXcds - 1 - xcd) / kXcds;  // workgroups on this XCD
         next = xcd * per_xcd + slot;
         end = (xcd + 1) * per_xcd;
         if (end > ntiles) end = ntiles;

@@ -144,3 +144,23 @@ def test_blocks_of_earlier_calls_are_not_met(gpu_ash, n, where):
             assert torch.equal(a, b), turn
         if turn % 2 == 1:
             grid.engine.erase(few)
+
+
+def test_a_ray_beside_one_that_has_ended(gpu_ash):
+    """The last lane of a ray that has ended stands in the block that the next ray's first
+    lane asks the table about: it has not asked, and has no answer to give."""
+    n, samples = 8193, 62
+    grid = gpu_ash.BoundedSparseDenseGrid(3, 3000, 1, 8, 32, device=DEV)
+    backend, table = gpu_ash.grid.backend, grid.engine.backend
+    g = torch.Generator().manual_seed(n + samples)
+    grid.engine.insert_keys(torch.randint(9, 23, (2500, 3), generator=g).int().to(DEV))
+    o = (torch.rand(n, 3, generator=g) * 256).to(DEV)
+    d = torch.nn.functional.normalize(torch.randn(n, 3, generator=g), dim=1).to(DEV)
+    near, far = torch.zeros(n, device=DEV), (torch.rand(n, generator=g) * 200).to(DEV)
+    args = (table, o, d, None, 1.0, near, far, samples, 8.0)
+    for a, b in zip(backend.ray_sample_world(*args), backend.ray_sample_world(*args, (0, 31))):
+        assert torch.equal(a, b)
+    alone = [len(backend.ray_sample_world(table, o[r:r + 1], d[r:r + 1], None, 1.0, near[r:r + 1], far[r:r + 1],
+                                          samples, 8.0)[0]) for r in range(4240, 4248)]
+    counts = torch.bincount(backend.ray_sample_world(*args)[0], minlength=n)
+    assert counts[4240:4248].tolist() == alone

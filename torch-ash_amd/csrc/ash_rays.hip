@@ -174,7 +174,9 @@ __device__ __forceinline__ void ray_block(const float (&o)[3], const float (&d)[
 // The same from the table; the first lane of a run of equal blocks asks.
 __device__ __forceinline__ bool is_stored_by_runs(const MapDev& m, const int32_t (&block)[3], bool active) {
     const int lane = threadIdx.x & 63;
-    int same = lane > 0 && active && lane_before(static_cast<int32_t>(active)) != 0;
+    // (asked of every lane: of one that takes no part, the shift gives back the asker's own)
+    const int32_t active_before = lane_before(static_cast<int32_t>(active));
+    int same = lane > 0 && active && active_before != 0;
 #pragma unroll
     for (int a = 0; a < 3; ++a) same &= lane_before(block[a]) == block[a];
     int32_t idx;

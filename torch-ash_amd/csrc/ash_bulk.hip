@@ -376,12 +376,15 @@ __global__ __launch_bounds__(kSplitThreads) void split_keys_kernel(
     const int64_t base = static_cast<int64_t>(blockIdx.x) * kSplitChunk;
     // (all keys are asked for at once and first: the draws of ranks in LDS would
     // keep the loads apart, a trip to memory each.  No branch around them: lanes
-    // beyond the last key read the first; 16 M keys 135 -> 130 us)
+    // beyond the last key read the first; 16 M keys 135 -> 130 us.  Marked as not to be
+    // kept, they leave the caches to the open runs, whose lines are filled by several
+    // workgroups: 128 -> 107, 0.40 GB in and out and 0.14 for the log and flags at 5.0
+    // TB/s.  The runs themselves written past the caches: 177.)
     int32_t key[kSplitKeys][DIM];
 #pragma unroll
     for (int k = 0; k < kSplitKeys; ++k) {
         const int64_t i = base + k * kSplitThreads + tid;
-        load_key<DIM>(keys, i < pl.n ? i : 0, true, key[k]);
+        load_key_once<DIM>(keys, i < pl.n ? i : 0, key[k]);
     }
     if (tid < kMaxBins) sh.cnt[tid] = 0;
     if (tid == 0) {

@@ -100,6 +100,15 @@ __device__ __forceinline__ void load_key(const int32_t* __restrict__ keys,
     for (int d = 0; d < DIM; ++d) k[d] = active ? keys[i * DIM + d] : 0;
 }
 
+// The same for keys that are read once and come from memory, marked as not to be kept
+// in the caches: what is written meanwhile stays there instead.
+template <int DIM>
+__device__ __forceinline__ void load_key_once(const int32_t* __restrict__ keys, int64_t i,
+                                              int32_t (&k)[DIM]) {
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) k[d] = __builtin_nontemporal_load(keys + i * DIM + d);
+}
+
 // Value rows copied by a fused insert: row i of src[v] goes to row `index` of
 // dst[v]; rows are row_dwords[v] 32-bit words long.
 struct ValueArgs {

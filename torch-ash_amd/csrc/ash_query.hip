@@ -58,6 +58,12 @@ constexpr int kWavesFull = 8;
 constexpr int kWavesWide = 7;
 constexpr int kWavesBoth = 6;   // positions' gradient and both orders' of the rows: 60 - 78 registers
 constexpr int kWavesBackward = 3;
+// ... and of the kernels that give a lane a whole query: two workgroups of eight, which the
+// line tables leave room for, want 128 registers at most (rows of seven 151 -> 118 us; up to
+// six take fewer anyway, twelve need more)
+// (Workgroups of four on a CU without tables: 8 of up to 64 registers, ..., 3 of 168.)
+constexpr int resident_rows(int E) { return E <= 5 ? 8 : E == 6 ? 6 : E == 7 ? 5 : E <= 12 ? 4 : 3; }
+constexpr int waves_of_rows(int E, int threads) { return threads > 256 && (E == 7 || E == 8) ? 4 : kWavesBackward; }
 constexpr int forward_waves(int vec, int lpq) {
     return vec > 4 || (vec == 4 && lpq > 2) ? kWavesWide : kWavesFull;
 }
@@ -169,7 +175,7 @@ __device__ __forceinline__ T corner_slope(const AxisTerms<T>& t, const SlopeTerm
 // ------------------------------------------------------------ LDS layout
 // [ tile: row[8][256] uint32, off[3][256] float ]  (only when LPQ > 1)
 // [ per-cell table: uint16[M][8] ]  (only when lds_lut)
-// [ one LineTable per wavefront ]  (E = 4 backward kernels that produce grad_embeddings)
+// [ one LineTable per wavefront ]  (backward kernels by rows that produce grad_embeddings)
 struct Tile {
     uint32_t row[8][kBlock];
     float off[3][kBlock];
@@ -233,7 +239,7 @@ __device__ __forceinline__ CellLut stage_cell_lut(const QDev& a,
     return lut;
 }
 
-// Where the line tables of the float4 backward kernels start in dynamic LDS.
+// Where the line tables of the backward kernels by rows start in dynamic LDS.
 __host__ __device__ inline size_t table_offset(const QDev& a, int lpq, bool lds_lut) {
     size_t bytes = lpq > 1 ? sizeof(Tile) : 0;
     if (lds_lut) bytes += static_cast<size_t>(a.M) * 8 * 2;
@@ -799,11 +805,11 @@ query_backward_backward_kernel(
     }
 }
 
-// ================================================== float4 backward kernels
-// fp32 embeddings of four channels (a signed distance and a colour, say): one
-// lane holds a whole query, as in the forward kernel, so that a wavefront
-// serves 64 queries per tile: four times the loads in flight and a quarter of
-// the per-query arithmetic of the one-lane-per-channel kernels above.
+// ================================================= backward kernels by rows
+// fp32 rows of few channels (rows_by_lane): one lane holds a whole query, as in the
+// forward kernel, so that a wavefront serves 64 queries per tile: four channels have four
+// times the loads in flight and a quarter of the per-query arithmetic of the
+// one-lane-per-channel kernels above, and rows of five leave no lanes idle.
 //
 // Gradient rows.  The memory side executes atomics at a fixed rate of
 // requests, and one request is what one instruction of a wavefront sends to
@@ -813,7 +819,8 @@ query_backward_backward_kernel(
 // over and over -- the x neighbour is the next row, a corner of this sample is
 // another corner of the next -- but in different instructions.  So every
 // wavefront first adds its contributions into a small table of lines in LDS
-// (open addressing on the line number, sixteen floats per entry) and sends the
+// (open addressing on the line number, sixteen floats per entry; a row may end in the
+// line after the one it starts in) and sends the
 // table out once per tile, one line per sixteen lanes: a third of the requests
 // on ray-ordered samples.  Before that, runs of consecutive queries with the
 // same row are summed in registers (lane exchange inside a row of 16 lanes is
@@ -821,8 +828,18 @@ query_backward_backward_kernel(
 // through the LDS pipeline, so a run is cut at the row of lanes; the table
 // joins the pieces).  A row whose line finds no place within kLineProbes steps
 // goes to memory directly, and a wavefront that sent more rows that way than
-// the table has lines (unordered queries share no lines) leaves the table
-// aside for the next kLineRest tiles.
+// the table has lines leaves the table aside for the next kLineRest tiles.
+//
+// Queries in no order share no lines but those of neighbouring corners.  A tile of which
+// more than half lie in another block than the query before them leaves the table aside
+// at once: the rows of two corners that differ in x follow each other in memory, and leave
+// together by neighbouring lanes of one instruction, five requests for eight rows of four
+// channels (rows of one by one through the table until it had rested: 398 -> 273 us for
+// 1 M unordered queries of four channels, 17 -> 7 for 1000).  Ordered tiles pay 1 us of a
+// launch for that (131 000 of four channels 12.2 -> 13.5, 4 M 251 -> 253).
+// Every corner with a copy of its code: one copy for all, which selects its row and its
+// terms, takes half as long again (131 000 of four channels 19 us), as does a second pass
+// for the rows past the table (14.6).
 template <int CTRL>
 __device__ __forceinline__ int dpp_int(int v) {
     return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
@@ -851,14 +868,20 @@ struct Runs {
     bool take[4];     // step 1, 2, 4, 8 of the segmented sum adds what lies that far below
     bool takes_offer; // adds what lane 15 of the row before holds
     bool tail;        // this lane ends its run and holds the total
+    bool ordered;     // half of the queries are less than a block's cells from the one before (the same for all lanes)
 };
 
-// `id`: the row of the query's cell, or for a lane without a query a number no
-// neighbour shares.  Every lane of the wavefront must take part.
-__device__ __forceinline__ Runs find_runs(uint32_t id, int lane) {
+// The runs of a tile.  Lanes without a query (not `on`) get a number no neighbour shares.
+// `cells`: of a block.  Every lane of the wavefront must take part.
+__device__ __forceinline__ Runs find_runs(uint32_t cell_row, bool on, uint32_t cells, int lane) {
     Runs r;
+    const uint32_t id = on ? cell_row : (kNoRow - static_cast<uint32_t>(lane & 1));
     const int g = lane & 15;
     const uint32_t prev = dpp<kRowShr + 1>(id);
+    const uint32_t ahead = id - prev, behind = prev - id;
+    const uint64_t queries = __builtin_amdgcn_ballot_w64(on);
+    const uint64_t near = __builtin_amdgcn_ballot_w64((ahead < behind ? ahead : behind) < cells);
+    r.ordered = 2 * __popcll(near & queries) >= __popcll(queries);
     const uint32_t next = dpp<kRowShl + 1>(id);
     const bool joins = g > 0 && prev == id;
     r.any = __ballot(joins) != 0;
@@ -901,10 +924,10 @@ __device__ __forceinline__ Runs find_runs(uint32_t id, int lane) {
     return r;
 }
 
-template <int D>
-__device__ __forceinline__ void run_step(float (&v)[4], bool take) {
+template <int D, int E>
+__device__ __forceinline__ void run_step(float (&v)[E], bool take) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < E; ++k) {
         const float vu = dpp<kRowShr + D>(v[k]);
         if (take) v[k] += vu;
     }
@@ -912,13 +935,14 @@ __device__ __forceinline__ void run_step(float (&v)[4], bool take) {
 
 // Sums `v` over the runs; the lanes with r.tail hold the totals afterwards.
 // Every lane of the wavefront must take part.
-__device__ __forceinline__ void sum_runs(const Runs& r, float (&v)[4]) {
+template <int E>
+__device__ __forceinline__ void sum_runs(const Runs& r, float (&v)[E]) {
     run_step<1>(v, r.take[0]);
     run_step<2>(v, r.take[1]);
     run_step<4>(v, r.take[2]);
     run_step<8>(v, r.take[3]);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < E; ++k) {
         const float part = dpp<kRowBcast15>(v[k]);
         if (r.takes_offer) v[k] += part;
     }
@@ -927,7 +951,10 @@ __device__ __forceinline__ void sum_runs(const Runs& r, float (&v)[4]) {
 constexpr int kLineSlots = 128;   // lines per wavefront's table
 constexpr int kLineProbes = 4;
 constexpr int kLineRest = 7;
-constexpr int kLineOut = 16;      // rows that leave past the table by one instruction
+// Lanes that a row leaves past the table by, and rows of one instruction (of one
+// channel: of a quarter of its lanes, for which there is room)
+constexpr int line_out_lanes(int E) { return E <= 4 ? 4 : E <= 8 ? 8 : 16; }
+constexpr int line_out_rows(int E) { return 64 / line_out_lanes(E); }
 constexpr uint32_t kLineFree = 0xFFFFFFFFu;
 // float k of slot h sits at k * kLinePitch + h: the sixteen floats of a line
 // and the same float of neighbouring slots fall into different banks
@@ -940,8 +967,8 @@ struct LineTable {
     // of used slots in the same place
     union {
         struct {
-            uint32_t row[kLineOut];
-            float v[kLineOut * 4];
+            uint32_t row[16];
+            float v[64];
         } out;
         uint8_t used[kLineSlots];
     };
@@ -955,33 +982,53 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// at[k * kLinePitch] += v[k], k = 0..3, in LDS.  The LDS executes a
-// floating-point add atomic one lane after the other (about three cycles a
+// The floats of a row added to their places in LDS, `at(k)` for the k-th.  The LDS
+// executes a floating-point add atomic one lane after the other (about three cycles a
 // lane, measured) and a 32-bit compare-and-swap at full rate: the add is a read
-// and a compare-and-swap of the sum.  The four floats go side by side, two
+// and a compare-and-swap of the sum.  The floats go side by side, two
 // round trips for all of them; lanes that met another lane's update in between
 // (seldom: runs of equal rows have been summed before) repeat float by float.
-__device__ __forceinline__ void lds_add4(float* at, const float (&v)[4]) {
-    unsigned int* w = reinterpret_cast<unsigned int*>(at);
-    unsigned int seen[4], got[4];
+template <int E, typename At>
+__device__ __forceinline__ void lds_add(At at, const float (&v)[E]) {
+    unsigned int seen[E], got[E];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) seen[k] = w[k * kLinePitch];
+    for (int k = 0; k < E; ++k) seen[k] = *at(k);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        got[k] = atomicCAS(w + k * kLinePitch, seen[k],
-                           __float_as_uint(__uint_as_float(seen[k]) + v[k]));
+    for (int k = 0; k < E; ++k) {
+        got[k] = atomicCAS(at(k), seen[k], __float_as_uint(__uint_as_float(seen[k]) + v[k]));
     }
-    if (got[0] == seen[0] && got[1] == seen[1] && got[2] == seen[2] && got[3] == seen[3]) return;
+    bool done = true;
+#pragma unroll
+    for (int k = 0; k < E; ++k) done = done && got[k] == seen[k];
+    if (done) return;
 #pragma unroll 1
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < E; ++k) {
         // (selects, not an indexed access: the arrays stay in registers)
-        unsigned int g = k == 0 ? got[0] : k == 1 ? got[1] : k == 2 ? got[2] : got[3];
-        unsigned int s = k == 0 ? seen[0] : k == 1 ? seen[1] : k == 2 ? seen[2] : seen[3];
-        const float add = k == 0 ? v[0] : k == 1 ? v[1] : k == 2 ? v[2] : v[3];
+        unsigned int g = got[0], s = seen[0];
+        float add = v[0];
+#pragma unroll
+        for (int q = 1; q < E; ++q) {
+            g = k == q ? got[q] : g;
+            s = k == q ? seen[q] : s;
+            add = k == q ? v[q] : add;
+        }
         while (g != s) {
             s = g;
-            g = atomicCAS(w + k * kLinePitch, s, __float_as_uint(__uint_as_float(s) + add));
+            g = atomicCAS(at(k), s, __float_as_uint(__uint_as_float(s) + add));
         }
+    }
+}
+
+// Line of a row's first float, and where in it that stands.
+template <int E>
+__device__ __forceinline__ void line_of(uint32_t row, uint32_t& line, uint32_t& pos) {
+    if constexpr (16 % E == 0) {
+        line = row / (16 / E);
+        pos = row % (16 / E) * E;
+    } else {
+        const uint64_t first = static_cast<uint64_t>(row) * E;
+        line = static_cast<uint32_t>(first >> 4);
+        pos = static_cast<uint32_t>(first) & 15u;
     }
 }
 
@@ -989,133 +1036,220 @@ struct LineAcc {
     LineTable* tab;
     int rest;      // tiles left during which the table is left aside
     int spilled;   // rows that found no place in the table since the last flush (whole wavefront)
+    bool aside;    // the table is left aside during this tile, and its place used otherwise
+    bool ready;    // the table is empty and its floats are zero (at the start of a tile)
 
     __device__ __forceinline__ void start(LineTable* t, int lane) {
         tab = t;
         rest = 0;
         spilled = 0;
-        if (tab != nullptr) {
-            for (int i = lane; i < 16 * kLinePitch; i += 64) tab->val[i] = 0.f;
-            tab->key[lane] = kLineFree;
-            tab->key[lane + 64] = kLineFree;
-            wave_lds_fence();
-        }
+        if (tab != nullptr) empty(lane);
     }
 
-    // grad[4 * row .. 4 * row + 3] += v for the lanes that `want`; every lane
-    // of the wavefront must take part.
-    __device__ __forceinline__ void add4(float* __restrict__ grad, bool want, uint32_t row,
-                                         const float (&v)[4], int lane) {
-        bool placed = false;
-        if (want && rest == 0) {
-            const uint32_t line = row >> 2;
-            uint32_t h = (line * 0x9E3779B1u) >> 25;
+    __device__ __forceinline__ void empty(int lane) {
+        for (int i = lane; i < 16 * kLinePitch; i += 64) tab->val[i] = 0.f;
+        tab->key[lane] = kLineFree;
+        tab->key[lane + 64] = kLineFree;
+        wave_lds_fence();
+        ready = true;
+    }
+
+    // Whole wavefront, before the first row of a tile.
+    __device__ __forceinline__ void tile(bool ordered, int lane) {
+        aside = rest > 0 || !ordered;
+        if (!aside && !ready) empty(lane);
+    }
+
+    // The slot of `line`, or kLineSlots where it finds no place.
+    __device__ __forceinline__ uint32_t slot_of(uint32_t line) {
+        uint32_t h = (line * 0x9E3779B1u) >> 25;
 #pragma unroll 1
-            for (int p = 0; p < kLineProbes; ++p) {
-                const uint32_t old = atomicCAS(&tab->key[h], kLineFree, line);
-                if (old == kLineFree || old == line) {
-                    placed = true;
-                    break;
-                }
-                h = (h + 1) & (kLineSlots - 1);
-            }
-            if (placed) lds_add4(tab->val + (row & 3u) * 4 * kLinePitch + h, v);
+        for (int p = 0; p < kLineProbes; ++p) {
+            const uint32_t old = atomicCAS(&tab->key[h], kLineFree, line);
+            if (old == kLineFree || old == line) return h;
+            h = (h + 1) & (kLineSlots - 1);
         }
-        // The rest goes to memory now, regrouped so that the four floats of a
+        return kLineSlots;
+    }
+
+    // grad[E * row .. E * row + E - 1] += v for the lanes that `want`; every lane
+    // of the wavefront must take part.
+    template <int E>
+    __device__ __forceinline__ void add(float* __restrict__ grad, bool want, uint32_t row,
+                                        const float (&v)[E], int lane) {
+        bool placed = false;
+        if (want) {
+            uint32_t line, pos;
+            line_of<E>(row, line, pos);
+            const uint32_t h = slot_of(line);
+            placed = h < kLineSlots;
+            if constexpr (16 % E == 0) {
+                unsigned int* at = reinterpret_cast<unsigned int*>(tab->val + pos * kLinePitch + h);
+                if (placed) lds_add<E>([&](int k) { return at + k * kLinePitch; }, v);
+            } else {
+                // a row may end in the next line (a line that was claimed for it alone
+                // and stays empty where this one finds no place sends nothing)
+                uint32_t next = h;
+                if (placed && pos + E > 16u) {
+                    next = slot_of(line + 1u);
+                    placed = next < kLineSlots;
+                }
+                unsigned int* at = reinterpret_cast<unsigned int*>(tab->val + pos * kLinePitch + h);
+                const int over = static_cast<int>(next) - static_cast<int>(h) - 16 * kLinePitch;
+                if (placed) {
+                    lds_add<E>([&](int k) { return at + k * kLinePitch + (pos + k > 15u ? over : 0); }, v);
+                }
+            }
+        }
+        // The rest goes to memory now, regrouped so that the floats of a
         // row leave from neighbouring lanes of one instruction (one request a
-        // row; one lane sending its four floats would make four).
+        // row; one lane sending its floats would make as many).
         const uint64_t out = __ballot(want && !placed);
         if (out == 0) return;
+        constexpr int kLanes = line_out_lanes(E), kRows = line_out_rows(E);
         const int n = __popcll(out);
-        spilled += n;
         const int mine = __popcll(out & ((1ull << lane) - 1ull));
-        for (int i = 0; i < n; i += kLineOut) {
+        spilled += n;
+        for (int i = 0; i < n; i += kRows) {
             const int at = mine - i;
             wave_lds_fence();
-            if (want && !placed && at >= 0 && at < kLineOut) {
+            if (want && !placed && at >= 0 && at < kRows) {
                 tab->out.row[at] = row;
-                *reinterpret_cast<float4*>(tab->out.v + at * 4) = make_float4(v[0], v[1], v[2], v[3]);
+                if constexpr (E == 4) {
+                    *reinterpret_cast<float4*>(tab->out.v + at * 4) = make_float4(v[0], v[1], v[2], v[3]);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < E; ++k) tab->out.v[at * kLanes + k] = v[k];
+                }
             }
             wave_lds_fence();
-            const int e = lane >> 2;
-            if (i + e < n) {
-                unsafeAtomicAdd(grad + static_cast<uint64_t>(tab->out.row[e]) * 4 + (lane & 3),
-                                tab->out.v[e * 4 + (lane & 3)]);
+            const int e = lane / kLanes, k = lane % kLanes;
+            if (i + e < n && k < E) {
+                unsafeAtomicAdd(grad + static_cast<uint64_t>(tab->out.row[e]) * E + k, tab->out.v[lane]);
             }
         }
         wave_lds_fence();
     }
 
+    // The same past the table, which is left aside and leaves room for all rows of two
+    // corners: these follow each other in memory as a rule, and leave together.
+    template <int E>
+    __device__ __forceinline__ void send_two(float* __restrict__ grad, bool want, const uint32_t (&row)[2],
+                                             const float (&v)[2][E], int lane) {
+        constexpr int kPitch = 2 * E + 1, kAtOnce = 64 / (2 * E);
+        static_assert(64 * (kPitch + 2) <= 16 * kLinePitch, "128 rows and their numbers");
+        const uint64_t out = __ballot(want);
+        const int n = __popcll(out);
+        const int mine = __popcll(out & ((1ull << lane) - 1ull));
+        uint32_t* const rows = reinterpret_cast<uint32_t*>(tab->val);
+        float* const floats = tab->val + 128;
+        wave_lds_fence();
+        if (want) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                rows[2 * mine + h] = row[h];
+#pragma unroll
+                for (int k = 0; k < E; ++k) floats[mine * kPitch + h * E + k] = v[h][k];
+            }
+        }
+        wave_lds_fence();
+        const int e = lane / (2 * E), at = lane % (2 * E);
+        const int half = at >= E ? 1 : 0, k = at - half * E;
+        for (int i = e; i < n && e < kAtOnce; i += kAtOnce) {
+            unsafeAtomicAdd(grad + static_cast<uint64_t>(rows[2 * i + half]) * E + k, floats[i * kPitch + at]);
+        }
+    }
+
     // Whole wavefront: sends the table's lines out and empties it.
     __device__ __forceinline__ void flush(float* __restrict__ grad, int lane) {
-        if (rest > 0) {
-            --rest;
-        } else {
-            wave_lds_fence();
-            const bool lo = tab->key[lane] != kLineFree;
-            const bool hi = tab->key[lane + 64] != kLineFree;
-            const uint64_t mlo = __ballot(lo), mhi = __ballot(hi);
-            const uint64_t below = (1ull << lane) - 1ull;
-            const int nlo = __popcll(mlo);
-            const int n = nlo + __popcll(mhi);
-            if (lo) tab->used[__popcll(mlo & below)] = static_cast<uint8_t>(lane);
-            if (hi) tab->used[nlo + __popcll(mhi & below)] = static_cast<uint8_t>(lane + 64);
-            wave_lds_fence();
-            // four lines per instruction, sixteen lines per turn: the reads of
-            // a turn are issued together
-            for (int i = 0; i < n; i += 16) {
-                uint32_t h[4], line[4];
-                float v[4];
-                float* at[4];
+        wave_lds_fence();
+        const bool lo = tab->key[lane] != kLineFree;
+        const bool hi = tab->key[lane + 64] != kLineFree;
+        const uint64_t mlo = __ballot(lo), mhi = __ballot(hi);
+        const uint64_t below = (1ull << lane) - 1ull;
+        const int nlo = __popcll(mlo);
+        const int n = nlo + __popcll(mhi);
+        if (lo) tab->used[__popcll(mlo & below)] = static_cast<uint8_t>(lane);
+        if (hi) tab->used[nlo + __popcll(mhi & below)] = static_cast<uint8_t>(lane + 64);
+        wave_lds_fence();
+        // four lines per instruction, sixteen lines per turn: the reads of
+        // a turn are issued together
+        for (int i = 0; i < n; i += 16) {
+            uint32_t h[4], line[4];
+            float v[4];
+            float* at[4];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int e = i + j * 4 + (lane >> 4);
-                    h[j] = e < n ? tab->used[e] : 0u;
-                }
+            for (int j = 0; j < 4; ++j) {
+                const int e = i + j * 4 + (lane >> 4);
+                h[j] = e < n ? tab->used[e] : 0u;
+            }
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int e = i + j * 4 + (lane >> 4);
-                    at[j] = tab->val + (lane & 15) * kLinePitch + h[j];
-                    line[j] = tab->key[h[j]];
-                    v[j] = e < n ? *at[j] : 0.f;
-                }
+            for (int j = 0; j < 4; ++j) {
+                const int e = i + j * 4 + (lane >> 4);
+                at[j] = tab->val + (lane & 15) * kLinePitch + h[j];
+                line[j] = tab->key[h[j]];
+                v[j] = e < n ? *at[j] : 0.f;
+            }
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    // floats nobody contributed to are zero
-                    if (v[j] != 0.f) {
-                        *at[j] = 0.f;
-                        unsafeAtomicAdd(
-                                grad + ((static_cast<uint64_t>(line[j]) << 4) | (lane & 15)), v[j]);
-                    }
+            for (int j = 0; j < 4; ++j) {
+                // floats nobody contributed to are zero
+                if (v[j] != 0.f) {
+                    *at[j] = 0.f;
+                    unsafeAtomicAdd(
+                            grad + ((static_cast<uint64_t>(line[j]) << 4) | (lane & 15)), v[j]);
                 }
             }
-            wave_lds_fence();
-            tab->key[lane] = kLineFree;
-            tab->key[lane + 64] = kLineFree;
-            wave_lds_fence();
-            // more rows went past the table than it has lines
-            if (spilled > kLineSlots) rest = kLineRest;
+        }
+        wave_lds_fence();
+        tab->key[lane] = kLineFree;
+        tab->key[lane + 64] = kLineFree;
+        wave_lds_fence();
+    }
+
+    // The tile is done with.
+    __device__ __forceinline__ void done() {
+        if (aside) ready = false;
+        if (rest > 0) {
+            --rest;
+        } else if (spilled > kLineSlots) {
+            rest = kLineRest;   // more rows went past the table than it has lines
         }
         spilled = 0;
     }
 };
 
-// grad_emb[row, 0..3] += v for the lanes that are `on`; every lane of the
-// wavefront must take part.  `runs`: find_runs of this tile.
-__device__ __forceinline__ void accumulate_row4(LineAcc& acc, float* __restrict__ grad_emb,
-                                                uint32_t row, bool on, const Runs& runs,
-                                                float (&v)[4], int lane) {
-    bool tail = true;
-    if (runs.any) {   // (samples cells apart, scattered points: nothing to join)
-        sum_runs(runs, v);
-        tail = runs.tail;
+// grad_emb[row[c], 0..E - 1] += part(c, v) of the eight corners for the lanes that are
+// `on`; every lane of the wavefront must take part.  `runs`: find_runs of this tile.
+template <int E, typename Part>
+__device__ __forceinline__ void scatter_rows(LineAcc& acc, float* __restrict__ grad_emb,
+                                             const uint32_t (&row)[8], bool on, const Runs& runs,
+                                             Part part, int lane) {
+    // (samples cells apart, scattered points: nothing to join)
+    const bool want = on && (!runs.any || runs.tail);
+    if (acc.aside) {
+#pragma unroll
+        for (int c = 0; c < 8; c += 2) {
+            const uint32_t rows[2] = {row[c], row[c + 1]};
+            float v[2][E];
+            part(c, v[0]);
+            part(c + 1, v[1]);
+            if (runs.any) {
+                sum_runs(runs, v[0]);
+                sum_runs(runs, v[1]);
+            }
+            acc.send_two<E>(grad_emb, want, rows, v, lane);
+        }
+    } else {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            float v[E];
+            part(c, v);
+            if (runs.any) sum_runs(runs, v);
+            acc.add<E>(grad_emb, want, row[c], v, lane);
+        }
+        acc.flush(grad_emb, lane);
     }
-    acc.add4(grad_emb, on && tail, row, v, lane);
-}
-
-// The runs of a tile: lanes without a query get a number no neighbour shares.
-__device__ __forceinline__ Runs tile_runs(uint32_t cell_row, bool on, int lane) {
-    return find_runs(on ? cell_row : (kNoRow - static_cast<uint32_t>(lane & 1)), lane);
+    acc.done();
 }
 
 __device__ __forceinline__ LineTable* line_table(unsigned char* smem, const QDev& a,
@@ -1125,9 +1259,54 @@ __device__ __forceinline__ LineTable* line_table(unsigned char* smem, const QDev
            (threadIdx.x >> 6);
 }
 
-// First-order backward, E = 4 (formulas as in query_backward_forward_kernel).
-template <bool LDS, int OUT, int THREADS>
-__global__ __launch_bounds__(THREADS, kWavesBackward) void
+// Rows of E floats, by a lane each (16-byte aligned where E is four).
+template <int E>
+__device__ __forceinline__ void load_whole_row(const float* __restrict__ at, float (&v)[E]) {
+    if constexpr (E == 4) {
+        const float4 r = *reinterpret_cast<const float4*>(at);
+        v[0] = r.x, v[1] = r.y, v[2] = r.z, v[3] = r.w;
+    } else {
+        const FloatRow<E> r = *reinterpret_cast<const FloatRow<E>*>(at);
+#pragma unroll
+        for (int k = 0; k < E; ++k) v[k] = r.v[k];
+    }
+}
+
+template <int E>
+__device__ __forceinline__ void load_row_once(const float* __restrict__ at, float (&v)[E]) {
+    if constexpr (E == 4) {
+        typedef float v4f __attribute__((ext_vector_type(4)));
+        const v4f r = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(at));
+        v[0] = r.x, v[1] = r.y, v[2] = r.z, v[3] = r.w;
+    } else {
+#pragma unroll
+        for (int k = 0; k < E; ++k) v[k] = __builtin_nontemporal_load(at + k);
+    }
+}
+
+template <int E>
+__device__ __forceinline__ float row_product(const float (&a)[E], const float (&b)[E]) {
+    if constexpr (E == 16) {   // pairs, pairs of pairs, ...: see rows_by_lane
+        float p[E];
+#pragma unroll
+        for (int k = 0; k < E; ++k) p[k] = __fmul_rn(a[k], b[k]);
+#pragma unroll
+        for (int n = E / 2; n > 0; n /= 2) {
+#pragma unroll
+            for (int k = 0; k < n; ++k) p[k] = __fadd_rn(p[2 * k], p[2 * k + 1]);
+        }
+        return p[0];
+    } else {
+        float dot = a[0] * b[0];
+#pragma unroll
+        for (int k = 1; k < E; ++k) dot += a[k] * b[k];
+        return dot;
+    }
+}
+
+// First-order backward, rows of E (formulas as in query_backward_forward_kernel).
+template <int E, bool LDS, int OUT, int THREADS>
+__global__ __launch_bounds__(THREADS, waves_of_rows(E, THREADS)) void
 query_backward_forward_vec_kernel(
         QDev a, const float* __restrict__ z, float* __restrict__ grad_emb,
         float* __restrict__ grad_off, const float* __restrict__ gg_off,
@@ -1150,15 +1329,12 @@ query_backward_forward_vec_kernel(
         const QueryInputs in = load_inputs(a, q);
         resolve_rows<LDS>(a, lut, in, row, o);
         const bool on = row[0] != kNoRow;
-        float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f), y4 = z4;
+        float zq[E] = {}, yq[E] = {};
         float gg[3] = {0.f, 0.f, 0.f};
         if (on) {
-            typedef float v4f __attribute__((ext_vector_type(4)));
-            const v4f zl = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(z + q * 4));
-            z4 = make_float4(zl.x, zl.y, zl.z, zl.w);
+            load_row_once<E>(z + q * E, zq);
             if constexpr (second) {
-                const v4f zs = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(z2 + q * 4));
-                y4 = make_float4(zs.x, zs.y, zs.z, zs.w);
+                load_row_once<E>(z2 + q * E, yq);
                 gg[0] = __builtin_nontemporal_load(gg_off + q * 3 + 0) * static_cast<float>(a.offset_scale);
                 gg[1] = __builtin_nontemporal_load(gg_off + q * 3 + 1) * static_cast<float>(a.offset_scale);
                 gg[2] = __builtin_nontemporal_load(gg_off + q * 3 + 2) * static_cast<float>(a.offset_scale);
@@ -1169,24 +1345,19 @@ query_backward_forward_vec_kernel(
         // the gathered rows are used up before the scatter starts, which keeps
         // them out of the registers the scatter needs
         if constexpr (want_off) {
-            float4 e[8];
+            float e[8][E];
 #pragma unroll
             for (int c = 0; c < 8; ++c) {
-                e[c] = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (on) {
-                    e[c] = *reinterpret_cast<const float4*>(
-                            emb + static_cast<int64_t>(row[c]) * 4);
-                }
+#pragma unroll
+                for (int k = 0; k < E; ++k) e[c][k] = 0.f;
+                if (on) load_whole_row<E>(emb + static_cast<int64_t>(row[c]) * E, e[c]);
             }
             float go[3] = {0.f, 0.f, 0.f};
 #pragma unroll
             for (int c = 0; c < 8; ++c) {
                 float gw[3];
                 corner_weight_grad<float>(t, c, gw);
-                float dot = e[c].x * z4.x;
-                dot += e[c].y * z4.y;
-                dot += e[c].z * z4.z;
-                dot += e[c].w * z4.w;
+                const float dot = row_product<E>(e[c], zq);
                 go[0] += dot * gw[0];
                 go[1] += dot * gw[1];
                 go[2] += dot * gw[2];
@@ -1199,31 +1370,28 @@ query_backward_forward_vec_kernel(
             }
         }
         if constexpr (want_emb) {
-            const Runs runs = tile_runs(row[0], on, lane);
+            const Runs runs = find_runs(row[0], on, static_cast<uint32_t>(a.M), lane);
+            acc.tile(runs.ordered, lane);
             SlopeTerms<float> slope;
             if constexpr (second) slope_terms<float>(t, gg, slope);
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
+            scatter_rows<E>(acc, grad_emb, row, on, runs, [&](int c, float (&v)[E]) {
                 const float w = corner_weight<float>(t, c);
-                float v[4] = {w * z4.x, w * z4.y, w * z4.z, w * z4.w};
+#pragma unroll
+                for (int k = 0; k < E; ++k) v[k] = w * zq[k];
                 if constexpr (second) {
                     const float d = corner_slope<float>(t, slope, c);
-                    v[0] += d * y4.x;
-                    v[1] += d * y4.y;
-                    v[2] += d * y4.z;
-                    v[3] += d * y4.w;
+#pragma unroll
+                    for (int k = 0; k < E; ++k) v[k] += d * yq[k];
                 }
-                accumulate_row4(acc, grad_emb, row[c], on, runs, v, lane);
-            }
-            acc.flush(grad_emb, lane);
+            }, lane);
         }
     }
 }
 
-// Backward of the backward, E = 4 (formulas as in
+// Backward of the backward, rows of E (formulas as in
 // query_backward_backward_kernel).
-template <bool LDS, int OUT, int THREADS>
-__global__ __launch_bounds__(THREADS, kWavesBackward) void
+template <int E, bool LDS, int OUT, int THREADS>
+__global__ __launch_bounds__(THREADS, waves_of_rows(E, THREADS)) void
 query_backward_backward_vec_kernel(
         QDev a, const float* __restrict__ gg_off, const float* __restrict__ z,
         float* __restrict__ grad_z, float* __restrict__ grad_emb) {
@@ -1244,12 +1412,10 @@ query_backward_backward_vec_kernel(
         const QueryInputs in = load_inputs(a, q);
         resolve_rows<LDS>(a, lut, in, row, o);
         const bool on = row[0] != kNoRow;
-        float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
+        float zq[E] = {};
         float gg[3] = {0.f, 0.f, 0.f};
         if (on) {
-            typedef float v4f __attribute__((ext_vector_type(4)));
-            const v4f zl = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(z + q * 4));
-            z4 = make_float4(zl.x, zl.y, zl.z, zl.w);
+            load_row_once<E>(z + q * E, zq);
             gg[0] = __builtin_nontemporal_load(gg_off + q * 3 + 0) * static_cast<float>(a.offset_scale);
             gg[1] = __builtin_nontemporal_load(gg_off + q * 3 + 1) * static_cast<float>(a.offset_scale);
             gg[2] = __builtin_nontemporal_load(gg_off + q * 3 + 2) * static_cast<float>(a.offset_scale);
@@ -1257,43 +1423,43 @@ query_backward_backward_vec_kernel(
         AxisTerms<float> t;
         axis_terms<float, true>(o, a.smooth, t);
         if constexpr (want_z) {
-            float4 e[8];
+            float e[8][E];
 #pragma unroll
             for (int c = 0; c < 8; ++c) {
-                e[c] = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (on) {
-                    e[c] = *reinterpret_cast<const float4*>(
-                            emb + static_cast<int64_t>(row[c]) * 4);
-                }
+#pragma unroll
+                for (int k = 0; k < E; ++k) e[c][k] = 0.f;
+                if (on) load_whole_row<E>(emb + static_cast<int64_t>(row[c]) * E, e[c]);
             }
-            float gz[4] = {0.f, 0.f, 0.f, 0.f};
+            float gz[E] = {};
 #pragma unroll
             for (int c = 0; c < 8; ++c) {
                 float gw[3];
                 corner_weight_grad<float>(t, c, gw);
                 const float d = gw[0] * gg[0] + gw[1] * gg[1] + gw[2] * gg[2];
-                gz[0] += d * e[c].x;
-                gz[1] += d * e[c].y;
-                gz[2] += d * e[c].z;
-                gz[3] += d * e[c].w;
+#pragma unroll
+                for (int k = 0; k < E; ++k) gz[k] += d * e[c][k];
             }
             if (q < a.N) {
-                typedef float v4f __attribute__((ext_vector_type(4)));
-                const v4f g4 = {on ? gz[0] : 0.f, on ? gz[1] : 0.f, on ? gz[2] : 0.f, on ? gz[3] : 0.f};
-                __builtin_nontemporal_store(g4, reinterpret_cast<v4f*>(grad_z + q * 4));
+                if constexpr (E == 4) {
+                    typedef float v4f __attribute__((ext_vector_type(4)));
+                    const v4f g4 = {on ? gz[0] : 0.f, on ? gz[1] : 0.f, on ? gz[2] : 0.f, on ? gz[3] : 0.f};
+                    __builtin_nontemporal_store(g4, reinterpret_cast<v4f*>(grad_z + q * 4));
+                } else {
+#pragma unroll
+                    for (int k = 0; k < E; ++k) __builtin_nontemporal_store(on ? gz[k] : 0.f, grad_z + q * E + k);
+                }
             }
         }
         if constexpr (want_emb) {
-            const Runs runs = tile_runs(row[0], on, lane);
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
+            const Runs runs = find_runs(row[0], on, static_cast<uint32_t>(a.M), lane);
+            acc.tile(runs.ordered, lane);
+            scatter_rows<E>(acc, grad_emb, row, on, runs, [&](int c, float (&v)[E]) {
                 float gw[3];
                 corner_weight_grad<float>(t, c, gw);
                 const float d = gw[0] * gg[0] + gw[1] * gg[1] + gw[2] * gg[2];
-                float v[4] = {d * z4.x, d * z4.y, d * z4.z, d * z4.w};
-                accumulate_row4(acc, grad_emb, row[c], on, runs, v, lane);
-            }
-            acc.flush(grad_emb, lane);
+#pragma unroll
+                for (int k = 0; k < E; ++k) v[k] = d * zq[k];
+            }, lane);
         }
     }
 }
@@ -2393,23 +2559,28 @@ bool aligned16(const void* p) {
 // four are twelve.  2^22 ray samples on 200 k blocks of 8^3: backward 221 -> 190
 // us, second order 214 -> 187; 1.5 x 10^6 unordered queries 541 and 542 us as
 // before (their rows leave past the tables, bound by requests).
+// (Rows of twelve have registers for twelve wavefronts on a CU.)
 int vec_threads(const QDev& d, int out) {
-    const bool wide = lut_in_lds(d) && (out & 1) != 0 && 2 * smem_bytes(d, 1, 2 * kBlock / 64) <= kLdsPerCu;
+    const bool wide = lut_in_lds(d) && (out & 1) != 0 && d.E <= 8 && 2 * smem_bytes(d, 1, 2 * kBlock / 64) <= kLdsPerCu;
     return wide ? 2 * kBlock : kBlock;
 }
 
+template <int E>
 int launch_bwd_fwd_vec(const QDev& d, const void* z, void* ge, void* go, const Second& also,
                        hipStream_t s) {
     const int out = gradients_wanted(ge, go, also);
     const int threads = vec_threads(d, out);
     const size_t smem = smem_bytes(d, 1, ge != nullptr ? threads / 64 : 0);
-    const unsigned g = persistent_grid((d.N + threads - 1) / threads, smem);
+    const unsigned g = persistent_grid((d.N + threads - 1) / threads, smem, resident_rows(E));
 #define ASH_BF(L, O, T)                                                       \
-    query_backward_forward_vec_kernel<L, O, T><<<g, T, smem, s>>>(    \
+    query_backward_forward_vec_kernel<E, L, O, T><<<g, T, smem, s>>>(    \
             d, static_cast<const float*>(z), static_cast<float*>(ge),         \
             static_cast<float*>(go), static_cast<const float*>(also.gg),      \
             static_cast<const float*>(also.z))
-    if (threads > kBlock) {
+    if constexpr (E > 12) {
+        if (lut_in_lds(d)) ASH_BF(true, 2, kBlock);
+        else ASH_BF(false, 2, kBlock);
+    } else if (threads > kBlock) {
         if (out == 7) ASH_BF(true, 7, 2 * kBlock);
         else if (out == 5) ASH_BF(true, 5, 2 * kBlock);
         else if (out == 3) ASH_BF(true, 3, 2 * kBlock);
@@ -2432,17 +2603,21 @@ int launch_bwd_fwd_vec(const QDev& d, const void* z, void* ge, void* go, const S
     return 0;
 }
 
+template <int E>
 int launch_bwd_bwd_vec(const QDev& d, const void* gg, const void* z, void* gz,
                        void* ge, hipStream_t s) {
     const int out = (ge != nullptr ? 1 : 0) | (gz != nullptr ? 2 : 0);
     const int threads = vec_threads(d, out);
     const size_t smem = smem_bytes(d, 1, ge != nullptr ? threads / 64 : 0);
-    const unsigned g = persistent_grid((d.N + threads - 1) / threads, smem);
+    const unsigned g = persistent_grid((d.N + threads - 1) / threads, smem, resident_rows(E));
 #define ASH_BB(L, O, T)                                                       \
-    query_backward_backward_vec_kernel<L, O, T><<<g, T, smem, s>>>(   \
+    query_backward_backward_vec_kernel<E, L, O, T><<<g, T, smem, s>>>(   \
             d, static_cast<const float*>(gg), static_cast<const float*>(z),   \
             static_cast<float*>(gz), static_cast<float*>(ge))
-    if (threads > kBlock) {
+    if constexpr (E > 12) {
+        if (lut_in_lds(d)) ASH_BB(true, 2, kBlock);
+        else ASH_BB(false, 2, kBlock);
+    } else if (threads > kBlock) {
         if (out == 3) ASH_BB(true, 3, 2 * kBlock);
         else ASH_BB(true, 1, 2 * kBlock);
     } else if (lut_in_lds(d)) {
@@ -2459,10 +2634,31 @@ int launch_bwd_bwd_vec(const QDev& d, const void* gg, const void* z, void* gz,
     return 0;
 }
 
-// fp32 rows of four channels on 16-byte aligned buffers
-bool rows_as_float4(const QDev& d, const void* p0, const void* p1, const void* p2) {
-    return d.E == 4 && aligned16(d.emb) && aligned16(p0) && aligned16(p1) &&
-           aligned16(p2);
+// Whether a backward goes by the kernels that give a lane a whole query, in fp32 (`out`: bit
+// 0 scatters to the embeddings).  Widths of their own: 1 to 8 channels (four on 16-byte
+// aligned buffers) and 12; of 16 what scatters nothing (a pair of its rows is two lines
+// anyway, and sixteen floats of two kinds and eight rows are more than the registers
+// hold).  Before (a lane per channel) -> now, us:
+//   gradient of the positions, ray samples: 2 M of 1, 2, 3 channels 36 -> 34, 40 -> 36, 52
+//     -> 38; 1 M of 5, 7, 8 57 -> 32, 58 -> 34, 57 -> 34; 660 000 of 12 83 -> 32; 500 000
+//     of 16 61 -> 27; 1000 of 5 12.5 -> 4.3
+//   both orders of the scatter with it: 124 -> 81, 161 -> 97, 213 -> 128; 170 -> 93, 186 ->
+//     118, 147 -> 131; 183 -> 163
+//   the same in no order, 1 M: of 1 channel 399 -> 234, 3 442 -> 293, 4 398 -> 273, 5 494 ->
+//     354, 8 392 -> 330; 660 000 of 12 403 -> 338; 1000 of 5 12.2 -> 7.1
+// What a query gets is the same to the bit whatever else is asked for: a width's sizes go
+// either way with all their gradients, and sixteen channels are added up as a lane per
+// channel does it.  (The two kinds of these in a launch each: 500 000 in order 139 -> 137,
+// in none 218 -> 272.)
+// Below 98 304 queries rows of one and two channels go by a lane per channel,
+// which is there all the same and has less to set up: 50 000 of one 7.2 | 9.5, 90 000 10.1 |
+// 11.5, 131 000 14.2 | 10.9; 70 000 of two 10.7 | 12.0, 131 000 15.9 | 12.1.
+constexpr int64_t kNarrowScatter = int64_t{3} << 15;
+
+bool rows_by_lane(const QDev& d, int out, const void* p0, const void* p1, const void* p2) {
+    if (d.E == 4) return aligned16(d.emb) && aligned16(p0) && aligned16(p1) && aligned16(p2);
+    if (d.E <= 2) return d.N >= kNarrowScatter;
+    return d.E <= 8 || d.E == 12 || (d.E == 16 && (out & 1) == 0);
 }
 
 template <typename T>
@@ -2561,7 +2757,21 @@ template <typename T>
 int dispatch_bwd_fwd(const QDev& d, const void* z, void* ge, void* go, const Second& also,
                      hipStream_t s) {
     if constexpr (sizeof(T) == 4) {
-        if (rows_as_float4(d, z, ge, also.z)) return launch_bwd_fwd_vec(d, z, ge, go, also, s);
+        const int out = gradients_wanted(ge, go, also);
+        if (rows_by_lane(d, out, z, ge, also.z)) {
+            switch (d.E) {
+                case 1: return launch_bwd_fwd_vec<1>(d, z, ge, go, also, s);
+                case 2: return launch_bwd_fwd_vec<2>(d, z, ge, go, also, s);
+                case 3: return launch_bwd_fwd_vec<3>(d, z, ge, go, also, s);
+                case 4: return launch_bwd_fwd_vec<4>(d, z, ge, go, also, s);
+                case 5: return launch_bwd_fwd_vec<5>(d, z, ge, go, also, s);
+                case 6: return launch_bwd_fwd_vec<6>(d, z, ge, go, also, s);
+                case 7: return launch_bwd_fwd_vec<7>(d, z, ge, go, also, s);
+                case 8: return launch_bwd_fwd_vec<8>(d, z, ge, go, also, s);
+                case 12: return launch_bwd_fwd_vec<12>(d, z, ge, go, also, s);
+                default: return launch_bwd_fwd_vec<16>(d, z, ge, go, also, s);
+            }
+        }
     }
     switch (pow2_ceil(d.E)) {
         case 1:
@@ -2581,7 +2791,21 @@ template <typename T>
 int dispatch_bwd_bwd(const QDev& d, const void* gg, const void* z, void* gz,
                      void* ge, hipStream_t s) {
     if constexpr (sizeof(T) == 4) {
-        if (rows_as_float4(d, z, ge, gz)) return launch_bwd_bwd_vec(d, gg, z, gz, ge, s);
+        const int out = (ge != nullptr ? 1 : 0) | (gz != nullptr ? 2 : 0);
+        if (rows_by_lane(d, out, z, ge, gz)) {
+            switch (d.E) {
+                case 1: return launch_bwd_bwd_vec<1>(d, gg, z, gz, ge, s);
+                case 2: return launch_bwd_bwd_vec<2>(d, gg, z, gz, ge, s);
+                case 3: return launch_bwd_bwd_vec<3>(d, gg, z, gz, ge, s);
+                case 4: return launch_bwd_bwd_vec<4>(d, gg, z, gz, ge, s);
+                case 5: return launch_bwd_bwd_vec<5>(d, gg, z, gz, ge, s);
+                case 6: return launch_bwd_bwd_vec<6>(d, gg, z, gz, ge, s);
+                case 7: return launch_bwd_bwd_vec<7>(d, gg, z, gz, ge, s);
+                case 8: return launch_bwd_bwd_vec<8>(d, gg, z, gz, ge, s);
+                case 12: return launch_bwd_bwd_vec<12>(d, gg, z, gz, ge, s);
+                default: return launch_bwd_bwd_vec<16>(d, gg, z, gz, ge, s);
+            }
+        }
     }
     switch (pow2_ceil(d.E)) {
         case 1:

@@ -1286,12 +1286,17 @@ __device__ __forceinline__ void load_row_once(const float* __restrict__ at, floa
 
 template <int E>
 __device__ __forceinline__ float row_product(const float (&a)[E], const float (&b)[E]) {
-    if constexpr (E == 16) {   // pairs, pairs of pairs, ...: see rows_by_lane
-        float p[E];
+    if constexpr (E >= 8) {
+        // pairs, pairs of pairs, ..., as a lane per channel adds them up: one after the
+        // other, wide rows lose by the roundings of the sum what they gain by those of the
+        // products (error against 64 bits, 2-norm: of eight channels 9.5e-8 and 9.7e-8, of
+        // twelve 9.7e-8 and 1.03e-7; of five 9.3e-8 and 9.2e-8)
+        constexpr int kWide = E > 8 ? 16 : 8;
+        float p[kWide];
 #pragma unroll
-        for (int k = 0; k < E; ++k) p[k] = __fmul_rn(a[k], b[k]);
+        for (int k = 0; k < kWide; ++k) p[k] = k < E ? __fmul_rn(a[k < E ? k : 0], b[k < E ? k : 0]) : 0.f;
 #pragma unroll
-        for (int n = E / 2; n > 0; n /= 2) {
+        for (int n = kWide / 2; n > 0; n /= 2) {
 #pragma unroll
             for (int k = 0; k < n; ++k) p[k] = __fadd_rn(p[2 * k], p[2 * k + 1]);
         }
@@ -2648,7 +2653,7 @@ int launch_bwd_bwd_vec(const QDev& d, const void* gg, const void* z, void* gz,
 //     354, 8 392 -> 330; 660 000 of 12 403 -> 338; 1000 of 5 12.2 -> 7.1
 // What a query gets is the same to the bit whatever else is asked for: a width's sizes go
 // either way with all their gradients, and sixteen channels are added up as a lane per
-// channel does it.  (The two kinds of these in a launch each: 500 000 in order 139 -> 137,
+// channel does it (row_product).  (The two kinds of these in a launch each: 500 000 in order 139 -> 137,
 // in none 218 -> 272.)
 // Below 98 304 queries rows of one and two channels go by a lane per channel,
 // which is there all the same and has less to set up: 50 000 of one 7.2 | 9.5, 90 000 10.1 |

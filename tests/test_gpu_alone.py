@@ -88,3 +88,23 @@ def test_batches_come_and_go(ash, dim, n):
 def test_erases_where_their_workgroups_change(ash, dim, n):
     """The index comes along with the codes of a bucket that other lanes erase from."""
     test_batches_come_and_go(ash, dim, n)
+
+
+@pytest.mark.parametrize("dim,n", [(3, 5), (1, 1 << 21), (3, 1 << 21), (4, (1 << 21) + 1)])
+def test_loads_on_either_side(ash, dim, n):
+    """A state dict brought in by lanes alone or by the cooperative probe: every key under
+    its index, the others absent."""
+    keys = _keys(n + 1000, dim, n)
+    engine = ash.HashSet(dim, n + n // 4, DEV).engine
+    order = torch.randperm(n, device=DEV)
+    state = {"_heap": torch.arange(engine.capacity, dtype=torch.int32, device=DEV),
+             "_keys": torch.zeros(engine.capacity, dim, dtype=torch.int32, device=DEV),
+             "_indices": torch.zeros(engine.capacity, dtype=torch.int64, device=DEV),
+             "_size": torch.tensor([n], dtype=torch.int32, device=DEV)}
+    state["_keys"][:n], state["_indices"][:n] = keys[:n], order
+    for _ in range(2):   # into a new table, and into one that holds them
+        engine.load_state_dict(state)
+        assert engine.size() == n
+        indices, masks = engine.find(keys)
+        assert bool(masks[:n].all()) and not bool(masks[n:].any())
+        assert torch.equal(indices[:n], order)

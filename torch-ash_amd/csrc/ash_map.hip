@@ -1082,8 +1082,8 @@ __global__ __launch_bounds__(kHeapBlock) void activate_runs_kernel(
 // each), so larger groups pay off here: measured on 16 M stored keys,
 // 256 threads with a tombstone update per wavefront 3.0 ms, 1024 threads with
 // one update of each counter per workgroup 0.85 ms.
-// Fewer keys are better spread over the CUs.  Lanes look at their buckets by themselves
-// up to kWideInsertEnd keys, as inserts do, but take the index along with the codes
+// Fewer keys are better spread over the CUs.  Lanes look at their buckets by themselves,
+// as inserts do, but take the index along with the codes
 // (probe_alone).  Cooperative with 1024 threads -> alone with the index read behind the
 // codes -> as it is (us), stored keys beside 100 000 | four million: 16 000 9.1 -> 6.8 ->
 // 6.3 | 11.1 -> 7.5 -> 7.3, 65 537 10.0 -> 11.0 -> 9.6 | 12.4 -> 10.8 -> 10.0, 98 000 11.5
@@ -1091,7 +1091,11 @@ __global__ __launch_bounds__(kHeapBlock) void activate_runs_kernel(
 // 13.7, 164 000 15.0 -> 18.2 -> 14.0 | 17.7 -> 17.2 -> 14.4, 400 000 42 -> 32 -> 27 | 33 ->
 // 28 -> 26, 1.6 million 92 -> 92 -> 85 | 88 -> 96 -> 84, 3.1 million 175 -> 228 -> 178
 // beside four; each key four times 131 000 13.7 -> 16.6 -> 13.0, 3.1 million 109 -> 126 -> 90;
-// absent keys 131 000 7.1 -> 5.8 -> 6.5, 3.1 million 77 -> 62 -> 63.  With 256 | 512 | 1024
+// absent keys 131 000 7.1 -> 5.8 -> 6.5, 3.1 million 77 -> 62 -> 63.  Larger batches,
+// cooperative -> as it is: stored keys, four million beside four 225 -> 205, eight beside
+// sixteen 400 -> 378, sixteen beside sixteen 843 -> 772; absent ones 120 -> 125, 265 -> 225,
+// 632 -> 426; each four times, four million 116 -> 108, each sixteen times, eight 248 -> 188.
+// With 256 | 512 | 1024
 // threads: 50 000 8.6 | 8.5 | 11.0, 98 000 12.9 | 11.3 | 11.9, 115 000 15.0 | 12.5 | 12.6,
 // 131 000 17.9 | 14.1 | 13.3.
 constexpr int kEraseBlock = 1024;
@@ -1191,11 +1195,11 @@ __device__ __forceinline__ void erase_one(const MapDev& m, const int32_t* __rest
     }
 }
 
-template <int DIM, int BLOCK, bool ALONE>
+template <int DIM, int BLOCK>
 __global__ __launch_bounds__(BLOCK) void erase_kernel(
         MapDev m, const int32_t* __restrict__ keys, int64_t n, Publish publish) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * BLOCK + threadIdx.x;
-    erase_one<DIM, false, BLOCK, ALONE>(m, keys, i, i < n);
+    erase_one<DIM, false, BLOCK, true>(m, keys, i, i < n);
     leave_with_last(m, publish, gridDim.x);
 }
 
@@ -2755,11 +2759,8 @@ int launch_insert_by(ash_map* map, const int32_t* keys, int64_t n,
 // and goes, of 256 -> 512 threads (us): 140 000 keys beside 20 000 111 -> 115, beside a
 // million 116 -> 114; 200 000 beside a million 135 -> 128, beside four 225 -> 217; 400 000
 // beside 300 000 188 -> 162; a million beside four 424 -> 397 (1024 threads: 402).
-// Beyond three million the waits weigh more (the insert alone, without and with rows: a
-// million 117 -> 96, 126 -> 102; two 170 -> 146, 179 -> 150; four 322 -> 317, 363 -> 372;
-// eight 642 -> 647, 676 -> 732; sixteen 1016 -> 1039, 1117 -> 1239).
 //
-// Up to there every lane looks at its buckets by itself, which takes half of the
+// Every lane looks at its buckets by itself, which takes half of the
 // vector instructions and registers (the kernel with rows of 16 bytes, cooperative ->
 // alone, beside a million keys: 8000 12.5 -> 11.3 us, 65 537 20.8 -> 19.3, 131 000 29.5 ->
 // 27.0, 300 000 39 -> 34; beside 100 000 131 000 36.8 -> 31.7, 196 000 48.6 -> 39; keys
@@ -2767,10 +2768,15 @@ int launch_insert_by(ash_map* map, const int32_t* keys, int64_t n,
 // stored already gain as well, beyond where look-ups (kAloneKeys) do not: beside 100 000 | four million | sixteen, a million 19.6 -> 17.4 | 25.0 -> 23.5 | 27.4 -> 24.3, 3.1
 // million 52.5 -> 45.9 | 64.0 -> 62.7 | 70 -> 63; of new keys, each sixteen times, a million
 // 36 -> 33 | 37 -> 35 | 42 -> 37, 3.1 million 82 -> 77 | 90 -> 80 | 95 -> 80; half stored, half
-// new 50 -> 45 | 52 -> 50 | 56 -> 52, 129 -> 126 | 180 -> 169 | 188 -> 165.  Batches beyond
-// are bound by requests, of which that makes more (four million that come and go beside
-// four 600 -> 640, eight beside eight 1137 -> 1245).
-constexpr int64_t kWideInsert = int64_t{3} << 16, kWideInsertEnd = int64_t{3} << 20;
+// new 50 -> 45 | 52 -> 50 | 56 -> 52, 129 -> 126 | 180 -> 169 | 188 -> 165. Larger
+// batches, 256 cooperative -> 512 alone, of new keys: with rows of 4 bytes four million beside
+// four 285 -> 254, eight beside eight 532 -> 492, five beside sixteen 337 -> 297, of 16 bytes
+// sixteen beside sixteen 573 -> 556; keys alone 3.5 million beside four 242 -> 208, each
+// sixteen times 114 -> 83; stored ones 127 -> 131, eight million 253 -> 253.  (While all keys
+// of a bucket went for its first free slot, see first_slot, four million were slower alone.)
+// Loads, 256 threads: 3000 keys 8.2 -> 6.9, 30 000 12.1 -> 10.8, 300 000 33.7 -> 25.9, a
+// million 80 -> 58, two 130 -> 122, three 225 -> 233, four 306 -> 312, sixteen 931 -> 1042.
+constexpr int64_t kWideInsert = int64_t{3} << 16, kAloneLoad = int64_t{1} << 21;
 constexpr int kWideBlock = 512;
 
 template <int MODE, bool TOMBS>
@@ -2778,14 +2784,15 @@ int launch_insert_to(ash_map* map, const int32_t* keys, int64_t n,
                      const ValueArgs& va, int32_t* assigned, const int64_t* given,
                      hipStream_t s, const Publish& publish = {}, const KeyCheck& check = {}) {
     if constexpr (MODE == kInsertKeys || MODE == kInsertFused) {
-        if (n > kWideInsert && n <= kWideInsertEnd) {
-            return launch_insert_by<MODE, TOMBS, kWideBlock, true>(map, keys, n, va, assigned, given, s, publish, check);
-        }
-        if (n <= kWideInsert) {
+        return n > kWideInsert
+                       ? launch_insert_by<MODE, TOMBS, kWideBlock, true>(map, keys, n, va, assigned, given, s, publish, check)
+                       : launch_insert_by<MODE, TOMBS, kHeapBlock, true>(map, keys, n, va, assigned, given, s, publish, check);
+    } else {
+        if (MODE == kInsertLoad && n <= kAloneLoad) {
             return launch_insert_by<MODE, TOMBS, kHeapBlock, true>(map, keys, n, va, assigned, given, s, publish, check);
         }
+        return launch_insert_by<MODE, TOMBS, kHeapBlock, false>(map, keys, n, va, assigned, given, s, publish, check);
     }
-    return launch_insert_by<MODE, TOMBS, kHeapBlock, false>(map, keys, n, va, assigned, given, s, publish, check);
 }
 
 template <int MODE>
@@ -3660,19 +3667,17 @@ int ash_map_erase(ash_map_t* map, const int32_t* keys, int64_t n,
         if (late.take(false)) return 1;
         if (late.taken()) publish = {late.late(), late.stamp, next_ticket(map)};
     }
-    auto launch = [&](auto block, auto alone) {
+    auto launch = [&](auto block) {
         constexpr int BLOCK = decltype(block)::value;
-        constexpr bool ALONE = decltype(alone)::value;
-        auto kernel = map->key_dim == 1   ? erase_kernel<1, BLOCK, ALONE>
-                      : map->key_dim == 2 ? erase_kernel<2, BLOCK, ALONE>
-                      : map->key_dim == 3 ? erase_kernel<3, BLOCK, ALONE>
-                                          : erase_kernel<4, BLOCK, ALONE>;
+        auto kernel = map->key_dim == 1   ? erase_kernel<1, BLOCK>
+                      : map->key_dim == 2 ? erase_kernel<2, BLOCK>
+                      : map->key_dim == 3 ? erase_kernel<3, BLOCK>
+                                          : erase_kernel<4, BLOCK>;
         kernel<<<grid_for(n, BLOCK), BLOCK, 0, s>>>(map->d, keys, n, publish);
     };
-    if (n <= kEraseBy256) launch(std::integral_constant<int, 256>{}, std::true_type{});
-    else if (n <= kEraseBy512) launch(std::integral_constant<int, 512>{}, std::true_type{});
-    else if (n <= kWideInsertEnd) launch(std::integral_constant<int, kEraseBlock>{}, std::true_type{});
-    else launch(std::integral_constant<int, kEraseBlock>{}, std::false_type{});
+    if (n <= kEraseBy256) launch(std::integral_constant<int, 256>{});
+    else if (n <= kEraseBy512) launch(std::integral_constant<int, 512>{});
+    else launch(std::integral_constant<int, kEraseBlock>{});
     ASH_LAUNCH_CHECK();
     change.queued();
     if (late.taken()) late.queued(true);

@@ -197,7 +197,8 @@ def _learn_holders() -> None:
 
 
 # Queries from which second-order nodes leave their share to the forward node, by the
-# wall time of a training step of 20 000 blocks (own share -> put off, us).  Fewer wait
+# wall time of a training step of 20 000 blocks (own share -> put off, us; rows of other
+# than four channels by kernels of a lane per channel, which took twice as long).  Fewer wait
 # for the host, 350 - 490 us by its clock, and the kernel time saved (22 us for 131 000
 # of five channels) reaches nobody: 131 000 of 1, 4, 5, 16 channels 331 -> 335, 469 ->
 # 470, 504 -> 497, 472 -> 476; 262 000 352 -> 355, 485 -> 488, 488 -> 493, 474 -> 478.

@@ -654,7 +654,8 @@ __device__ __forceinline__ void accumulate_row(T* __restrict__ grad_emb,
 // gg_off and z2 (below): the two contributions of a query go to the same eight
 // rows, and the requests for these are what either kernel is bound by (131 k ray
 // samples, rows of five: 28 + 23 -> 29 us; 2^22, rows of four, in the kernel for
-// these: 187 + 184 -> 254).
+// these: 187 + 184 -> 254).  Rows of 1 to 8 and 12 floats as a rule go by the kernels for
+// whole rows (rows_by_lane).
 template <typename T, int LPQ, bool LDS, int OUT>
 __global__ __launch_bounds__(kBlock, kWavesBackward) void
 query_backward_forward_kernel(

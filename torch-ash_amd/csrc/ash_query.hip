@@ -2649,9 +2649,9 @@ int launch_bwd_bwd_vec(const QDev& d, const void* gg, const void* z, void* gz,
 //     -> 38; 1 M of 5, 7, 8 57 -> 32, 58 -> 34, 57 -> 34; 660 000 of 12 83 -> 32; 500 000
 //     of 16 61 -> 27; 1000 of 5 12.5 -> 4.3
 //   both orders of the scatter with it: 124 -> 81, 161 -> 97, 213 -> 128; 170 -> 93, 186 ->
-//     118, 147 -> 131; 183 -> 163
-//   the same in no order, 1 M: of 1 channel 399 -> 234, 3 442 -> 293, 4 398 -> 273, 5 494 ->
-//     354, 8 392 -> 330; 660 000 of 12 403 -> 338; 1000 of 5 12.2 -> 7.1
+//     112, 147 -> 113; 183 -> 132
+//   the same in no order, 1 M: of 1 channel 399 -> 234, 3 442 -> 293, 4 398 -> 274, 5 494 ->
+//     354, 8 392 -> 339; 660 000 of 12 403 -> 323; 1000 of 5 11.9 -> 6.9
 // What a query gets is the same to the bit whatever else is asked for: a width's sizes go
 // either way with all their gradients, and sixteen channels are added up as a lane per
 // channel does it (row_product).  (The two kinds of these in a launch each: 500 000 in order 139 -> 137,

@@ -327,6 +327,9 @@ int ash_ray_sample_compact(const int64_t* counts, const int64_t* prefix, const f
 int64_t ash_ray_volume_bytes(int lo, int hi, int64_t n, int sampling);
 /* The same for a map, whose log is read through: 0 for fewer rays than gain that back. */
 int64_t ash_map_ray_volume_bytes(const ash_map_t* map, int lo, int hi, int64_t n, int sampling);
+/* Whether the scratch of a call on this stream may be kept: not while the stream is being
+ * captured (replays mark with the number of the captured call), whichever device is current. */
+int ash_ray_volume_kept(const ash_map_t* map, void* stream);
 int ash_ray_find_near_far_world(ash_map_t* map, uint8_t* volume, int volume_lo,
                                 int volume_hi, const float* ray_origins,
                                 const float* ray_directions, const float* origin,

@@ -2,7 +2,7 @@
 function a test of test_host_counters.py (each in a process of its own)."""
 import time
 
-from stand_in_device import ALWAYS, DROPPED, EXOTIC, SIZE, TOMBS, Map, beside
+from stand_in_device import ALWAYS, DROPPED, EXOTIC, PTR, SIZE, TOMBS, Map, beside
 
 ONE, OTHER = 0x10, 0x20   # streams
 
@@ -203,6 +203,22 @@ def a_frame_whose_count_fails(device):
     assert any("integrate_depth_flagged_kernel" in name for name in device.launched)
     device.refuse = ()
     assert m.fuse() == 0
+
+
+def scratch_of_rays_that_are_captured_is_not_kept(device):
+    """Whether the call's own stream is captured: not that of the device which is current."""
+    m = Map(device)
+    kept = m.lib.ash_ray_volume_kept
+    ask = lambda stream: kept(m.handle, PTR(stream))
+    assert [ask(s) for s in (0, ONE, OTHER)] == [1, 1, 1] and kept(PTR(0), PTR(ONE)) == 0
+    for current in (0, 1):
+        for captured in (0, ONE):
+            device.runtime.stand_in_capture(2, current, 0, PTR(captured))
+            assert [ask(s) for s in (0, ONE, OTHER)] == [int(s != captured) for s in (0, ONE, OTHER)]
+            assert device.runtime.stand_in_current_device() == current
+            # (a capture of the other device's default stream is none of this map's)
+            device.runtime.stand_in_capture(2, current, 1, PTR(0))
+            assert ask(0) == 1
 
 
 def larger_workgroups_only_where_they_are_launched(device):

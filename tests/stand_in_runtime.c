@@ -89,9 +89,19 @@ int hipLaunchKernel(const void* stub, dim3_t grid, dim3_t block, void** args, si
 
 int hipStreamSynchronize(void* stream) { return failed(on_wait((uintptr_t)stream)); }
 int hipDeviceSynchronize(void) { return failed(on_wait((uintptr_t)-1)); }
+/* the devices that there are, the one that is current, and the stream of one that is captured */
+static int num_devices = 1, current_device, capturing_device = -1;
+static void* capturing_stream;
+void stand_in_capture(int devices, int current, int device, void* stream) {
+    num_devices = devices;
+    current_device = current;
+    capturing_device = device;
+    capturing_stream = stream;
+}
+int stand_in_current_device(void) { return current_device; }
+/* (the default stream is the current device's) */
 int hipStreamIsCapturing(void* stream, int* status) {
-    (void)stream;
-    *status = 0;
+    *status = capturing_device >= 0 && stream == capturing_stream && (stream != NULL || current_device == capturing_device);
     return 0;
 }
 int hipHostMalloc(void** p, size_t bytes, unsigned flags) {
@@ -107,10 +117,14 @@ int hipMemcpyAsync(void* to, const void* from, size_t bytes, int kind, void* str
     return 0;
 }
 int hipGetDevice(int* device) {
-    *device = 0;
+    *device = current_device;
     return 0;
 }
-int hipSetDevice(int device) { return device == 0 ? 0 : failed(101); }
+int hipSetDevice(int device) {
+    if (device < 0 || device >= num_devices) return failed(101);
+    current_device = device;
+    return 0;
+}
 int hipDeviceGetAttribute(int* value, int attribute, int device) {
     (void)attribute, (void)device;
     *value = 256;

@@ -9,7 +9,6 @@
 // with their rows: 23 us of Python around 7 us of kernel).
 #include <torch/extension.h>
 
-#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/graph_task.h>
 #include <torch/csrc/autograd/python_function.h>
@@ -55,6 +54,7 @@ namespace py = pybind11;
     X(ash_map_neighbors)                                                              \
     X(ash_grid_fuse_frame)                                                            \
     X(ash_map_ray_volume_bytes)                                                       \
+    X(ash_ray_volume_kept)                                                            \
     X(ash_ray_find_near_far_marked)                                                   \
     X(ash_ray_sample_groups)                                                          \
     X(ash_ray_sample_march_marked)                                                    \
@@ -531,7 +531,7 @@ class Volumes {
         const int64_t bytes = lib.ash_map_ray_volume_bytes(map, lo, hi, n, sampling);
         if (bytes <= 0) return v;
         v.stream = stream_of(device);
-        v.keep = c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None;
+        v.keep = lib.ash_ray_volume_kept(map, v.stream) != 0;
         if (v.keep) {
             std::lock_guard<std::mutex> lock(mutex_);
             for (auto k = kept_.begin(); k != kept_.end(); ++k) {

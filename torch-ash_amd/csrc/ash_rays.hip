@@ -970,6 +970,13 @@ int64_t ash_map_ray_volume_bytes(const ash_map_t* map, int lo, int hi, int64_t n
     return ash_ray_volume_bytes(lo, hi, n, sampling);
 }
 
+int ash_ray_volume_kept(const ash_map_t* map, void* stream) {
+    if (map == nullptr) return 0;
+    DeviceGuard guard;
+    // (the default stream of a device is known by the device alone)
+    return guard.enter(map->device) == hipSuccess && !is_capturing(static_cast<hipStream_t>(stream)) ? 1 : 0;
+}
+
 int ash_ray_find_near_far_marked(ash_map_t* map, uint8_t* volume, int volume_lo, int volume_hi,
                                  int volume_mark, const float* ray_origins,
                                  const float* ray_directions, const float* origin, float cell_size,

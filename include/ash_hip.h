@@ -325,8 +325,10 @@ int ash_ray_sample_compact(const int64_t* counts, const int64_t* prefix, const f
  * them with this mark. */
 #define ASH_RAY_VOLUME_MARKS 255
 int64_t ash_ray_volume_bytes(int lo, int hi, int64_t n, int sampling);
-/* The same for a map, whose log is read through: 0 for fewer rays than gain that back. */
-int64_t ash_map_ray_volume_bytes(const ash_map_t* map, int lo, int hi, int64_t n, int sampling);
+/* The same for scratch that is kept and need not be cleared, which fewer rays gain back
+ * (samples: 0 for near_far, the most of a ray for the march), for a map whose log is not
+ * too long for them. */
+int64_t ash_map_ray_volume_bytes(const ash_map_t* map, int lo, int hi, int64_t n, int64_t samples);
 /* Whether the scratch of a call on this stream may be kept: not while the stream is being
  * captured (replays mark with the number of the captured call), whichever device is current. */
 int ash_ray_volume_kept(const ash_map_t* map, void* stream);

@@ -2,7 +2,7 @@
 function a test of test_host_counters.py (each in a process of its own)."""
 import time
 
-from stand_in_device import ALWAYS, DROPPED, EXOTIC, PTR, SIZE, TOMBS, Map, beside
+from stand_in_device import ALWAYS, DROPPED, EXOTIC, I64, INT, PTR, SIZE, TOMBS, Map, beside
 
 ONE, OTHER = 0x10, 0x20   # streams
 
@@ -219,6 +219,25 @@ def scratch_of_rays_that_are_captured_is_not_kept(device):
             # (a capture of the other device's default stream is none of this map's)
             device.runtime.stand_in_capture(2, current, 1, PTR(0))
             assert ask(0) == 1
+
+
+def as_many_rays_as_gain_their_volume_back(device):
+    """More where the call clears it than where it is kept, and beside a long log."""
+    short, long = Map(device, capacity=100_000), Map(device, capacity=3_000_000)
+    cleared, kept = device.lib.ash_ray_volume_bytes, device.lib.ash_map_ray_volume_bytes
+    cleared.restype = kept.restype = I64
+    has = lambda n, sampling, hi=31: cleared(INT(0), INT(hi), I64(n), INT(sampling)) > 0
+    keeps = lambda m, n, samples, hi=31: kept(m.handle, INT(0), INT(hi), I64(n), I64(samples)) > 0
+    assert [has(n, 0) for n in (0, 1024, 4095, 4096)] == [False, False, False, True]
+    assert [has(n, 1) for n in (0, 2048, 8191, 8192)] == [False, False, False, True]
+    assert [keeps(short, n, 0) for n in (1023, 1024, 4095, 4096)] == [False, True, True, True]
+    assert [keeps(long, n, 0) for n in (1024, 4095, 4096)] == [False, False, True]
+    for samples in (1, 16, 63):
+        assert [keeps(m, n, samples) for m in (short, long) for n in (8191, 8192)] == [False, True] * 2
+    for samples in (64, 128, 1 << 40):
+        assert [keeps(short, n, samples) for n in (2047, 2048, 8191, 8192)] == [False, True, True, True]
+        assert [keeps(long, n, samples) for n in (2048, 7812, 7813, 8192)] == [False, False, True, True]
+    assert not has(1 << 20, 0, 161) and not keeps(short, 1 << 20, 0, 161) and not keeps(short, 1 << 20, 0, -1)
 
 
 def larger_workgroups_only_where_they_are_launched(device):

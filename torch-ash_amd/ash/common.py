@@ -136,7 +136,7 @@ _SIGNATURES = {
     ),
     "ash_ray_sample_compact": (ctypes.c_int, [_PTR] * 3 + [_I64, _I64] + [_PTR] * 4),
     "ash_ray_volume_bytes": (_I64, [ctypes.c_int, ctypes.c_int, _I64, ctypes.c_int]),
-    "ash_map_ray_volume_bytes": (_I64, [_PTR, ctypes.c_int, ctypes.c_int, _I64, ctypes.c_int]),
+    "ash_map_ray_volume_bytes": (_I64, [_PTR, ctypes.c_int, ctypes.c_int, _I64, _I64]),
     "ash_ray_volume_kept": (ctypes.c_int, [_PTR, _PTR]),
     "ash_ray_find_near_far_world": (
         ctypes.c_int,

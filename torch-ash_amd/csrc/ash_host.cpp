@@ -53,6 +53,7 @@ namespace py = pybind11;
     X(ash_map_upkeep)                                                                 \
     X(ash_map_neighbors)                                                              \
     X(ash_grid_fuse_frame)                                                            \
+    X(ash_ray_volume_bytes)                                                           \
     X(ash_map_ray_volume_bytes)                                                       \
     X(ash_ray_volume_kept)                                                            \
     X(ash_ray_find_near_far_marked)                                                   \
@@ -526,12 +527,14 @@ class Volumes {
         return those;
     }
 
-    Volume take(const ash_map_t* map, int lo, int hi, int64_t n, bool sampling, int64_t device) {
+    Volume take(const ash_map_t* map, int lo, int hi, int64_t n, int64_t samples, int64_t device) {
         Volume v;
-        const int64_t bytes = lib.ash_map_ray_volume_bytes(map, lo, hi, n, sampling);
+        int64_t bytes = lib.ash_map_ray_volume_bytes(map, lo, hi, n, samples);
         if (bytes <= 0) return v;
         v.stream = stream_of(device);
         v.keep = lib.ash_ray_volume_kept(map, v.stream) != 0;
+        if (!v.keep) bytes = lib.ash_ray_volume_bytes(lo, hi, n, samples != 0);
+        if (bytes <= 0) return v;
         if (v.keep) {
             std::lock_guard<std::mutex> lock(mutex_);
             for (auto k = kept_.begin(); k != kept_.end(); ++k) {
@@ -576,7 +579,7 @@ std::tuple<Tensor, Tensor> ray_near_far(uintptr_t handle, int64_t device, Volume
     need(lo.numel() == 3 && hi.numel() == 3, "the box has three coordinates per corner");
     const int64_t n = r.o.size(0);
     Tensor nears = empty({n}, at::kFloat, device), fars = empty({n}, at::kFloat, device);
-    Volume volume = volumes.take(map_of(handle), block_lo, block_hi, n, false, device);
+    Volume volume = volumes.take(map_of(handle), block_lo, block_hi, n, 0, device);
     check(lib.ash_ray_find_near_far_marked(
             map_of(handle), ptr<uint8_t>(volume.bytes), block_lo, block_hi, volume.mark, ptr<float>(r.o),
             ptr<float>(r.d), ptr<float>(r.origin), static_cast<float>(cell_size), ptr<float>(lo),
@@ -612,7 +615,7 @@ std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> ray_sample(
     const Tensor counts = empty({n}, at::kLong, device), prefix = empty({n}, at::kLong, device);
     const Tensor groups = empty({lib.ash_ray_sample_groups(n), 2}, at::kLong, device);
     const Tensor stage = empty({n, stride, 2}, at::kFloat, device);
-    Volume volume = volumes.take(map_of(handle), block_lo, block_hi, n, true, device);
+    Volume volume = volumes.take(map_of(handle), block_lo, block_hi, n, max_samples, device);
     void* stream = stream_of(device);
     int64_t out[2] = {0, 0};
     int status;

@@ -54,16 +54,21 @@ constexpr uint32_t kMostMarks = ASH_RAY_VOLUME_MARKS;
 
 // More than this does not stay in an XCD's L2.
 constexpr int64_t kMaxVolume = int64_t{4} << 20;
-// Making it takes a launch of 3 - 4 us (two where it has to be cleared), and longer where
-// the log is long, which so many rays gain back.  Near and far, from the table -> with a
-// volume that need not be cleared, us: 1500 blocks, 1100 rays 10.7 -> 6.7, 4000 15.1 -> 6.9;
-// 200 000 blocks 12.3 -> 8.4, 17.6 -> 9.0; 200 000 of 1.5 M in the log 1000 8.8 -> 9.2, 1500
-// 11.1 -> 9.3; 1.2 M of 1.5 M 2500 14.0 -> 15.5 (cleared, 4096 17 -> 14, 32 768 79 -> 27).
-// Samples, up to 32 | 128 of a ray: 1500 blocks 2100 rays 33.2 -> 34.2 | 39.7 -> 38.2; 30 000
-// 35.7 -> 34.5 | 44.6 -> 40.6; 200 000 36.4 -> 36.2 | 51.0 -> 45.4, 8100 37.6 -> 37.0 | 56.9 ->
-// 45.9; 1.2 M of 1.5 M in the log 2500 34.7 -> 41.3 | 55.7 -> 53.0.
-constexpr int64_t kVolumeRaysNearFar = 1024, kVolumeRaysSampling = 2048;
-constexpr int64_t kVolumeLogPerRay = 384, kVolumeRaysAnyLog = 4096;
+// Making it takes two launches of 4 us each, which so many rays gain back: near
+// and far of 3000 rays 15 -> 15 us, 4096 17 -> 14, 8192 29 -> 15, 32 768 79 -> 27;
+// samples of 8000 rays 32 - 57 -> 36 - 48 (few blocks and short rays - many and
+// long), 32 768 37 - 77 -> 38 - 55.
+constexpr int64_t kVolumeRaysNearFar = 4096, kVolumeRaysSampling = 8192;
+// One that is kept need not be cleared, which leaves one launch of 3 - 4 us, longer where
+// the log is long.  Near and far, from the table -> with it, us: 1500 blocks, 1100 rays
+// 10.7 -> 6.7, 4000 15.1 -> 6.9; 200 000 blocks 12.3 -> 8.4, 17.6 -> 9.0; 200 000 of 1.5 M in
+// the log 1000 8.8 -> 9.2, 1500 11.1 -> 9.3; 1.2 M of 1.5 M 2500 14.0 -> 15.5.  Whole calls of
+// samples, up to 16 | 32 | 64 | 128 of a ray: 2100 rays, 1500 blocks 27.3 -> 28.4 | 29.0 ->
+// 29.7 | 31.2 -> 31.0 | 35.4 -> 33.3; 30 000 28.5 -> 28.9 | 31.2 -> 30.5 | 35.5 -> 33.0 | 40.1
+// -> 36.1; 200 000 29.3 -> 29.2 | 33.3 -> 32.2 | 38.9 -> 35.2 | 46.9 -> 40.8; 8100 rays, 1500
+// blocks 27.1 -> 28.5 | 29.5 -> 29.8 | 32.0 -> 31.4 | 36.3 -> 33.6: from 64 on they gain.
+constexpr int64_t kKeptRaysNearFar = 1024, kKeptRaysSampling = 2048;
+constexpr int64_t kKeptSamples = 64, kKeptLogPerRay = 384;
 
 __host__ __device__ __forceinline__ int64_t volume_bytes(int64_t edge) {
     const int64_t flat = (edge + 3) / 4, tall = (edge + 7) / 8;
@@ -71,6 +76,14 @@ __host__ __device__ __forceinline__ int64_t volume_bytes(int64_t edge) {
 }
 
 constexpr int64_t kOutsideBytes = 16;   // of the word
+
+// Bytes of a volume and its word, 0 where there is none.
+int64_t volume_scratch(int lo, int hi) {
+    const int64_t edge = static_cast<int64_t>(hi) - lo + 1;
+    if (edge < 1 || edge > kMaxVolume) return 0;
+    const int64_t bytes = volume_bytes(edge);
+    return bytes <= kMaxVolume ? bytes + kOutsideBytes : 0;
+}
 
 // (to be asked for early and looked at late)
 __device__ __forceinline__ uint32_t outside_word(const Volume& v) {
@@ -957,17 +970,15 @@ int ash_ray_find_near_far(ash_map_t* map, const float* ray_origins,
 }
 
 int64_t ash_ray_volume_bytes(int lo, int hi, int64_t n, int sampling) {
-    if (n < (sampling ? kVolumeRaysSampling : kVolumeRaysNearFar)) return 0;
-    const int64_t edge = static_cast<int64_t>(hi) - lo + 1;
-    if (edge < 1 || edge > kMaxVolume) return 0;
-    const int64_t bytes = volume_bytes(edge);
-    return bytes <= kMaxVolume ? bytes + kOutsideBytes : 0;
+    return n < (sampling ? kVolumeRaysSampling : kVolumeRaysNearFar) ? 0 : volume_scratch(lo, hi);
 }
 
-int64_t ash_map_ray_volume_bytes(const ash_map_t* map, int lo, int hi, int64_t n, int sampling) {
+int64_t ash_map_ray_volume_bytes(const ash_map_t* map, int lo, int hi, int64_t n, int64_t samples) {
     if (map == nullptr) return 0;
-    if (n < kVolumeRaysAnyLog && map->capacity > n * kVolumeLogPerRay) return 0;
-    return ash_ray_volume_bytes(lo, hi, n, sampling);
+    const int64_t bytes = ash_ray_volume_bytes(lo, hi, n, samples != 0);
+    const bool pays = samples == 0 ? n >= kKeptRaysNearFar : n >= kKeptRaysSampling && samples >= kKeptSamples;
+    if (bytes > 0 || !pays || map->capacity > n * kKeptLogPerRay) return bytes;
+    return volume_scratch(lo, hi);
 }
 
 int ash_ray_volume_kept(const ash_map_t* map, void* stream) {

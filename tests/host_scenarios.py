@@ -1,8 +1,9 @@
 """What the host keeps of a map's counters while calls and readers meet, one
 function a test of test_host_counters.py (each in a process of its own)."""
+import re
 import time
 
-from stand_in_device import ALWAYS, DROPPED, EXOTIC, I64, INT, PTR, SIZE, TOMBS, Map, beside
+from stand_in_device import ALWAYS, DROPPED, EXOTIC, I64, INT, LIBRARY, PTR, SIZE, TOMBS, Map, beside
 
 ONE, OTHER = 0x10, 0x20   # streams
 
@@ -245,3 +246,11 @@ def larger_workgroups_only_where_they_are_launched(device):
     wide = {name.split("insert_kernelI")[1][:10] for name in device.kernels()
             if "insert_kernelI" in name and "Li512E" in name}
     assert wide == {f"Li{dim}ELi{mode}ELb" for dim in (1, 2, 3, 4) for mode in (0, 1)}, wide
+
+
+def every_kernel_that_is_built_is_launched_from_somewhere(device):
+    """(the device code holds what a template names, also where its launch is never compiled)"""
+    with open(LIBRARY, "rb") as f:
+        built = {name.decode() for name in re.findall(rb"(_Z\w+)\.kd\0", f.read())}
+    registered = set(device.kernels())
+    assert len(built) > 100 and built == registered, built ^ registered

@@ -2788,8 +2788,10 @@ int launch_insert_to(ash_map* map, const int32_t* keys, int64_t n,
                        ? launch_insert_by<MODE, TOMBS, kWideBlock, true>(map, keys, n, va, assigned, given, s, publish, check)
                        : launch_insert_by<MODE, TOMBS, kHeapBlock, true>(map, keys, n, va, assigned, given, s, publish, check);
     } else {
-        if (MODE == kInsertLoad && n <= kAloneLoad) {
-            return launch_insert_by<MODE, TOMBS, kHeapBlock, true>(map, keys, n, va, assigned, given, s, publish, check);
+        if constexpr (MODE == kInsertLoad) {
+            if (n <= kAloneLoad) {
+                return launch_insert_by<MODE, TOMBS, kHeapBlock, true>(map, keys, n, va, assigned, given, s, publish, check);
+            }
         }
         return launch_insert_by<MODE, TOMBS, kHeapBlock, false>(map, keys, n, va, assigned, given, s, publish, check);
     }

@@ -254,3 +254,11 @@ def every_kernel_that_is_built_is_launched_from_somewhere(device):
         built = {name.decode() for name in re.findall(rb"(_Z\w+)\.kd\0", f.read())}
     registered = set(device.kernels())
     assert len(built) > 100 and built == registered, built ^ registered
+
+
+def backward_kernels_only_of_widths_that_are_launched(device):
+    """A lane per channel, eight lanes a query: rows of five to eight, which go by rows in
+    single precision."""
+    by_channel = [name for name in device.kernels() if "query_backward_" in name and "_vec_kernel" not in name]
+    assert any("IdLi8E" in name for name in by_channel) and any("IfLi16E" in name for name in by_channel)
+    assert not [name for name in by_channel if "IfLi8E" in name]

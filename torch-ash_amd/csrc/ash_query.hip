@@ -652,10 +652,10 @@ __device__ __forceinline__ void accumulate_row(T* __restrict__ grad_emb,
 // OUT: bit 0 = produce grad_embeddings, bit 1 = produce grad_offsets; bit 2 (with
 // bit 0) = and add to grad_embeddings what the backward of the backward does for
 // gg_off and z2 (below): the two contributions of a query go to the same eight
-// rows, and the requests for these are what either kernel is bound by (131 k ray
-// samples, rows of five: 28 + 23 -> 29 us; 2^22, rows of four, in the kernel for
-// these: 187 + 184 -> 254).  Rows of 1 to 8 and 12 floats as a rule go by the kernels for
-// whole rows (rows_by_lane).
+// rows, and the requests for these are what either kernel is bound by (positions'
+// gradient and rows of sixteen, 131 k ray samples: 52 + 39 -> 62 us, 500 k 122 + 99 ->
+// 136; 2^22, rows of four, in the kernel for these: 187 + 184 -> 254).  Rows of 1 to 8
+// and 12 floats as a rule go by the kernels for whole rows (rows_by_lane).
 template <typename T, int LPQ, bool LDS, int OUT>
 __global__ __launch_bounds__(kBlock, kWavesBackward) void
 query_backward_forward_kernel(
@@ -2786,8 +2786,9 @@ int dispatch_bwd_fwd(const QDev& d, const void* z, void* ge, void* go, const Sec
             return launch_bwd_fwd<T, 2>(d, z, ge, go, also, s);
         case 4:
             return launch_bwd_fwd<T, 4>(d, z, ge, go, also, s);
-        case 8:
-            return launch_bwd_fwd<T, 8>(d, z, ge, go, also, s);
+        case 8:   // (fp32 rows of five to eight: all by rows)
+            if constexpr (sizeof(T) == 8) return launch_bwd_fwd<T, 8>(d, z, ge, go, also, s);
+            [[fallthrough]];
         default:
             return launch_bwd_fwd<T, 16>(d, z, ge, go, also, s);
     }
@@ -2820,8 +2821,9 @@ int dispatch_bwd_bwd(const QDev& d, const void* gg, const void* z, void* gz,
             return launch_bwd_bwd<T, 2>(d, gg, z, gz, ge, s);
         case 4:
             return launch_bwd_bwd<T, 4>(d, gg, z, gz, ge, s);
-        case 8:
-            return launch_bwd_bwd<T, 8>(d, gg, z, gz, ge, s);
+        case 8:   // (fp32 rows of five to eight: all by rows)
+            if constexpr (sizeof(T) == 8) return launch_bwd_bwd<T, 8>(d, gg, z, gz, ge, s);
+            [[fallthrough]];
         default:
             return launch_bwd_bwd<T, 16>(d, gg, z, gz, ge, s);
     }

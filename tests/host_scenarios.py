@@ -262,3 +262,7 @@ def backward_kernels_only_of_widths_that_are_launched(device):
     by_channel = [name for name in device.kernels() if "query_backward_" in name and "_vec_kernel" not in name]
     assert any("IdLi8E" in name for name in by_channel) and any("IfLi16E" in name for name in by_channel)
     assert not [name for name in by_channel if "IfLi8E" in name]
+    # eight wavefronts to a table of cells: rows of up to eight that are scattered
+    wide = {int(name.split("_vec_kernelILi")[1].split("E")[0]) for name in device.kernels()
+            if "_vec_kernelI" in name and "Li512E" in name}
+    assert wide == set(range(1, 9)), wide

@@ -2566,8 +2566,9 @@ bool aligned16(const void* p) {
 // us, second order 214 -> 187; 1.5 x 10^6 unordered queries 541 and 542 us as
 // before (their rows leave past the tables, bound by requests).
 // (Rows of twelve have registers for twelve wavefronts on a CU.)
+constexpr int kWideRows = 8;
 int vec_threads(const QDev& d, int out) {
-    const bool wide = lut_in_lds(d) && (out & 1) != 0 && d.E <= 8 && 2 * smem_bytes(d, 1, 2 * kBlock / 64) <= kLdsPerCu;
+    const bool wide = lut_in_lds(d) && (out & 1) != 0 && d.E <= kWideRows && 2 * smem_bytes(d, 1, 2 * kBlock / 64) <= kLdsPerCu;
     return wide ? 2 * kBlock : kBlock;
 }
 
@@ -2586,11 +2587,12 @@ int launch_bwd_fwd_vec(const QDev& d, const void* z, void* ge, void* go, const S
     if constexpr (E > 12) {
         if (lut_in_lds(d)) ASH_BF(true, 2, kBlock);
         else ASH_BF(false, 2, kBlock);
-    } else if (threads > kBlock) {
-        if (out == 7) ASH_BF(true, 7, 2 * kBlock);
-        else if (out == 5) ASH_BF(true, 5, 2 * kBlock);
-        else if (out == 3) ASH_BF(true, 3, 2 * kBlock);
-        else ASH_BF(true, 1, 2 * kBlock);
+    } else if (E <= kWideRows && threads > kBlock) {
+        constexpr int wide = E <= kWideRows ? 2 * kBlock : kBlock;   // (not built for others)
+        if (out == 7) ASH_BF(true, 7, wide);
+        else if (out == 5) ASH_BF(true, 5, wide);
+        else if (out == 3) ASH_BF(true, 3, wide);
+        else ASH_BF(true, 1, wide);
     } else if (lut_in_lds(d)) {
         if (out == 7) ASH_BF(true, 7, kBlock);
         else if (out == 5) ASH_BF(true, 5, kBlock);
@@ -2623,9 +2625,10 @@ int launch_bwd_bwd_vec(const QDev& d, const void* gg, const void* z, void* gz,
     if constexpr (E > 12) {
         if (lut_in_lds(d)) ASH_BB(true, 2, kBlock);
         else ASH_BB(false, 2, kBlock);
-    } else if (threads > kBlock) {
-        if (out == 3) ASH_BB(true, 3, 2 * kBlock);
-        else ASH_BB(true, 1, 2 * kBlock);
+    } else if (E <= kWideRows && threads > kBlock) {
+        constexpr int wide = E <= kWideRows ? 2 * kBlock : kBlock;
+        if (out == 3) ASH_BB(true, 3, wide);
+        else ASH_BB(true, 1, wide);
     } else if (lut_in_lds(d)) {
         if (out == 3) ASH_BB(true, 3, kBlock);
         else if (out == 1) ASH_BB(true, 1, kBlock);

@@ -266,3 +266,15 @@ def backward_kernels_only_of_widths_that_are_launched(device):
     wide = {int(name.split("_vec_kernelILi")[1].split("E")[0]) for name in device.kernels()
             if "_vec_kernelI" in name and "Li512E" in name}
     assert wide == set(range(1, 9)), wide
+
+
+def programs_that_interpolate_do_not_load_the_backward_by_rows(device):
+    """The runtime loads a device code with the first of its kernels: every width's by
+    rows has one of its own."""
+    with open(LIBRARY, "rb") as f:
+        codes = f.read().split(b"\x7fELF")[2:]   # (the library itself comes first)
+    kernels = [{name.decode() for name in re.findall(rb"(_Z\w+)\.kd\0", code)} for code in codes]
+    by_rows = [names for names in kernels if any("_vec_kernelI" in name for name in names)]
+    widths = [{name.split("_vec_kernelILi")[1].split("E")[0] for name in names} for names in by_rows]
+    assert sorted(int(width) for width, in widths) == [1, 2, 3, 4, 5, 6, 7, 8, 12, 16], widths
+    assert any("grid_forward_kernel" in name for names in kernels for name in names)

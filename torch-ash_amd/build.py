@@ -21,9 +21,13 @@ HOST_SOURCE = os.path.join(CSRC, "ash_host.cpp")
 HOST_OUT = os.path.join(OUT_DIR, "_ash_host.so")
 SOURCES = ["ash_map.hip", "ash_bulk.hip", "ash_query.hip", "ash_fusion.hip", "ash_mesh.hip",
            "ash_rays.hip", "ash_conv.hip", "ash_surface.hip"]
+# compiled once for every width of rows (channels): device code of its own, which the
+# runtime loads where it is used
+ROWS_SOURCE, ROW_WIDTHS = "ash_rows.hip", (1, 2, 3, 4, 5, 6, 7, 8, 12, 16)
 HEADERS = [
     os.path.join(CSRC, "ash_probe.h"),
     os.path.join(CSRC, "ash_dev.h"),
+    os.path.join(CSRC, "ash_query.h"),
     os.path.join(CSRC, "ash_table.h"),
     os.path.join(CSRC, "ash_walk.h"),
     os.path.join(CSRC, "ash_mc_table.h"),
@@ -52,6 +56,12 @@ def compile_flags():
         "-Wall",
         "-Wno-unused-function",
     ]
+
+
+def units():
+    """(source, object, flags of its own) of everything that is compiled."""
+    return [(s, s.replace(".hip", ".o"), []) for s in SOURCES] + [
+        (ROWS_SOURCE, f"ash_rows_{width}.o", [f"-DASH_ROW_WIDTH={width}"]) for width in ROW_WIDTHS]
 
 
 def source_fingerprint() -> str:
@@ -91,7 +101,7 @@ def _older(out, deps) -> bool:
 
 
 def is_stale() -> bool:
-    return _older(OUT, [os.path.join(CSRC, s) for s in SOURCES] + HEADERS)
+    return _older(OUT, [os.path.join(CSRC, s) for s in [*SOURCES, ROWS_SOURCE]] + HEADERS)
 
 
 def host_is_stale() -> bool:
@@ -152,9 +162,9 @@ def build_kernels(force: bool, verbose: bool) -> str:
     stamp = f'-DASH_SOURCE_FINGERPRINT="{source_fingerprint()}"'
     objs = []
     procs = []
-    for src in SOURCES:
-        obj = os.path.join(OUT_DIR, src.replace(".hip", ".o"))
-        cmd = [hipcc, *compile_flags(), "-c", os.path.join(CSRC, src), "-o", obj]
+    for src, name, flags in units():
+        obj = os.path.join(OUT_DIR, name)
+        cmd = [hipcc, *compile_flags(), *flags, "-c", os.path.join(CSRC, src), "-o", obj]
         if src == "ash_map.hip":
             cmd.insert(1, stamp)
         if verbose:

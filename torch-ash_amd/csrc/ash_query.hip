@@ -24,25 +24,16 @@
 // are accumulated with hardware floating-point atomics; consecutive queries of
 // a wavefront that hit the same row are summed in registers first and issue
 // one atomic per run (ray-ordered samples produce long runs).
-#include "ash_probe.h"
-#include "ash_walk.h"
+#include "ash_query.h"
 
 #include <type_traits>
-
-#include <hip/amd_detail/amd_hip_unsafe_atomics.h>
 
 #include <cmath>
 #include <cstdlib>
 
-#include "../../include/ash_hip.h"
-
 namespace ash {
 namespace {
 
-constexpr int kBlock = 256;
-constexpr int64_t kMaxLdsCells = 2048;  // 2048 * 8 * 2 B = 32 KiB
-constexpr uint32_t kNoRow = 0xFFFFFFFFu;
-constexpr int kLdsPerCu = 160 * 1024;
 // Wavefronts per SIMD, which is workgroups per CU.  Forward kernels are held to
 // the 64 registers of eight, but for the widest rows (64 - 70 registers, seven),
 // which would spill; the backward ones are bound by their registers (both
@@ -58,12 +49,6 @@ constexpr int kWavesFull = 8;
 constexpr int kWavesWide = 7;
 constexpr int kWavesBoth = 6;   // positions' gradient and both orders' of the rows: 60 - 78 registers
 constexpr int kWavesBackward = 3;
-// ... and of the kernels that give a lane a whole query: two workgroups of eight, which the
-// line tables leave room for, want 128 registers at most (rows of seven 151 -> 118 us; up to
-// six take fewer anyway, twelve need more)
-// (Workgroups of four on a CU without tables: 8 of up to 64 registers, ..., 3 of 168.)
-constexpr int resident_rows(int E) { return E <= 5 ? 8 : E == 6 ? 6 : E == 7 ? 5 : E <= 12 ? 4 : 3; }
-constexpr int waves_of_rows(int E, int threads) { return threads > 256 && (E == 7 || E == 8) ? 4 : kWavesBackward; }
 constexpr int forward_waves(int vec, int lpq) {
     return vec > 4 || (vec == 4 && lpq > 2) ? kWavesWide : kWavesFull;
 }
@@ -71,259 +56,6 @@ template <typename T>
 constexpr int backward_waves(int out) {
     if (sizeof(T) == 8) return (out & 3) == 3 ? 4 : 5;
     return out == 7 ? kWavesBoth : out == 3 ? kWavesWide : kWavesFull;
-}
-
-struct QDev {
-    const void* emb;
-    const float* off;
-    const int64_t* gidx;
-    const int64_t* cidx;
-    const uint8_t* mask;
-    const int64_t* lut_g;
-    const int64_t* lut_c2c;
-    const int64_t* lut_c2g;
-    int64_t N;
-    int64_t B;
-    int64_t M;
-    int E;
-    // Gradients with respect to the offsets are multiplied by it, both where they are
-    // written and where the gradient of one is read: the grid's positions are offsets
-    // in units of a cell, and a pass over the gradient behind or in front of the kernel
-    // takes 17 - 23 us of 4 M queries (three of them in a training pass).
-    double offset_scale = 1.0;
-    int smooth;    // 0 linear, 1 smooth step
-    int merge;     // pre-reduce runs of equal rows before the atomics
-};
-
-// Interpolation basis (ash/src/grid.cu:7-41).
-template <typename T>
-__device__ __forceinline__ T basis(T x, int smooth) {
-    return smooth ? x * x * (T(3) - T(2) * x) : x;
-}
-template <typename T>
-__device__ __forceinline__ T dbasis(T x, int smooth) {
-    return smooth ? T(6) * x * (T(1) - x) : T(1);
-}
-
-// Per-axis factors of the corner weights and of their derivatives
-// (ash/src/grid.cu:113-118,229-241): side 0 is the "1 - o" side.
-template <typename T>
-struct AxisTerms {
-    T w[3][2];
-    T dw[3][2];
-};
-
-template <typename T, bool GRAD>
-__device__ __forceinline__ void axis_terms(const float (&o)[3], int smooth,
-                                           AxisTerms<T>& t) {
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const T x1 = static_cast<T>(o[d]);
-        const T x0 = static_cast<T>(1.0f - o[d]);
-        t.w[d][0] = basis<T>(x0, smooth);
-        t.w[d][1] = basis<T>(x1, smooth);
-        if constexpr (GRAD) {
-            t.dw[d][0] = -dbasis<T>(x0, smooth);
-            t.dw[d][1] = dbasis<T>(x1, smooth);
-        }
-    }
-}
-
-template <typename T>
-__device__ __forceinline__ T corner_weight(const AxisTerms<T>& t, int c) {
-    T w = T(1);
-    w *= t.w[0][c & 1];
-    w *= t.w[1][(c >> 1) & 1];
-    w *= t.w[2][(c >> 2) & 1];
-    return w;
-}
-
-template <typename T>
-__device__ __forceinline__ void corner_weight_grad(const AxisTerms<T>& t, int c,
-                                                   T (&g)[3]) {
-    const int b0 = c & 1, b1 = (c >> 1) & 1, b2 = (c >> 2) & 1;
-    g[0] = t.dw[0][b0] * t.w[1][b1] * t.w[2][b2];
-    g[1] = t.w[0][b0] * t.dw[1][b1] * t.w[2][b2];
-    g[2] = t.w[0][b0] * t.w[1][b1] * t.dw[2][b2];
-}
-
-// grad w_c . u for the eight corners, with the products of the first two axes
-// taken once for both sides of the third: half the operations of the sum of
-// corner_weight_grad's three terms, and one rounding less on each.
-template <typename T>
-struct SlopeTerms {
-    T w01[4], d01[4], d2[2];
-};
-
-template <typename T>
-__device__ __forceinline__ void slope_terms(const AxisTerms<T>& t, const T (&u)[3], SlopeTerms<T>& s) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int b0 = i & 1, b1 = i >> 1;
-        s.w01[i] = t.w[0][b0] * t.w[1][b1];
-        s.d01[i] = (t.dw[0][b0] * u[0]) * t.w[1][b1] + t.w[0][b0] * (t.dw[1][b1] * u[1]);
-    }
-    s.d2[0] = t.dw[2][0] * u[2];
-    s.d2[1] = t.dw[2][1] * u[2];
-}
-
-template <typename T>
-__device__ __forceinline__ T corner_slope(const AxisTerms<T>& t, const SlopeTerms<T>& s, int c) {
-    return s.d01[c & 3] * t.w[2][c >> 2] + s.w01[c & 3] * s.d2[c >> 2];
-}
-
-// ------------------------------------------------------------ LDS layout
-// [ tile: row[8][256] uint32, off[3][256] float ]  (only when LPQ > 1)
-// [ per-cell table: uint16[M][8] ]  (only when lds_lut)
-// [ one LineTable per wavefront ]  (backward kernels by rows that produce grad_embeddings)
-struct Tile {
-    uint32_t row[8][kBlock];
-    float off[3][kBlock];
-};
-
-// A cell's eight corners, one 16-bit code each (cell of the corner, below
-// kMaxLdsCells, and number of its neighbour block above it): one 16-byte read
-// per query.
-struct CellLut {
-    const uint4* codes;
-};
-
-constexpr int kCodeCellBits = 11;
-static_assert(kMaxLdsCells == int64_t{1} << kCodeCellBits, "cells of a code");
-
-template <bool LDS>
-__device__ __forceinline__ void cell_neighbors(const QDev& a, const CellLut& lut, int64_t cell,
-                                               uint32_t (&nb_cell)[8], uint32_t (&nb_grid)[8]) {
-    if constexpr (LDS) {
-        const uint4 v = lut.codes[cell];
-        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const uint32_t code = (w[c >> 1] >> (16 * (c & 1))) & 0xFFFFu;
-            nb_cell[c] = code & (kMaxLdsCells - 1);
-            nb_grid[c] = code >> kCodeCellBits;
-        }
-    } else {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            int64_t v = a.lut_c2c[cell * 8 + c];
-            v = v < 0 ? 0 : (v >= a.M ? a.M - 1 : v);
-            nb_cell[c] = static_cast<uint32_t>(v);
-            nb_grid[c] = static_cast<uint32_t>(a.lut_c2g[cell * 8 + c]) & 7u;
-        }
-    }
-}
-
-template <bool LDS, int THREADS = kBlock>
-__device__ __forceinline__ CellLut stage_cell_lut(const QDev& a,
-                                                  unsigned char* smem) {
-    CellLut lut = {nullptr};
-    if constexpr (LDS) {
-        // a cell at a time: its sixteen table entries come by eight loads in flight
-        uint4* codes = reinterpret_cast<uint4*>(smem);
-        const int cells = static_cast<int>(a.M);
-#pragma unroll 1
-        for (int cell = threadIdx.x; cell < cells; cell += THREADS) {
-            uint32_t nb_cell[8], nb_grid[8], w[4];
-            cell_neighbors<false>(a, lut, cell, nb_cell, nb_grid);
-#pragma unroll
-            for (int c = 0; c < 8; c += 2) {
-                w[c >> 1] = nb_cell[c] | (nb_grid[c] << kCodeCellBits) | (nb_cell[c + 1] << 16) |
-                            (nb_grid[c + 1] << (16 + kCodeCellBits));
-            }
-            codes[cell] = make_uint4(w[0], w[1], w[2], w[3]);
-        }
-        __syncthreads();
-        lut.codes = reinterpret_cast<const uint4*>(smem);
-    }
-    return lut;
-}
-
-// Where the line tables of the backward kernels by rows start in dynamic LDS.
-__host__ __device__ inline size_t table_offset(const QDev& a, int lpq, bool lds_lut) {
-    size_t bytes = lpq > 1 ? sizeof(Tile) : 0;
-    if (lds_lut) bytes += static_cast<size_t>(a.M) * 8 * 2;
-    return (bytes + 15) & ~static_cast<size_t>(15);
-}
-
-// What a query brings.  The mask, the indices and the offsets are asked for
-// together (one trip to memory, not two); what a masked query has there is read
-// and dropped.  They are read once, like z, and the per-query outputs are
-// written once: those loads and stores carry the non-temporal hint, which
-// leaves the caches to the embedding rows (forward, E = 4: 0.129 -> 0.117 ms).
-struct QueryInputs {
-    // low dwords of the int64 indices: a row of the block table is below 2^31
-    // and "none" is -1, a cell is below 2^31 too
-    int32_t gi, ci;
-    float o[3];
-    uint8_t m;   // 0: masked out or beyond the last query
-};
-
-__device__ __forceinline__ QueryInputs load_inputs(const QDev& a, int64_t q) {
-    QueryInputs in;
-    in.gi = in.ci = 0;
-    in.o[0] = in.o[1] = in.o[2] = 0.f;
-    in.m = 0;
-    if (q < a.N) {
-        in.m = __builtin_nontemporal_load(a.mask + q);
-        in.gi = __builtin_nontemporal_load(reinterpret_cast<const int32_t*>(a.gidx) + q * 2);
-        in.ci = __builtin_nontemporal_load(reinterpret_cast<const int32_t*>(a.cidx) + q * 2);
-        in.o[0] = __builtin_nontemporal_load(a.off + q * 3 + 0);
-        in.o[1] = __builtin_nontemporal_load(a.off + q * 3 + 1);
-        in.o[2] = __builtin_nontemporal_load(a.off + q * 3 + 2);
-    }
-    return in;
-}
-
-// Phase 1 for one query: the 8 corner rows (kNoRow in row[0] when the query is
-// masked out, out of range, or misses a neighbour block) and the offsets.
-// Latency bounds it, so the eight table entries are asked for together and
-// checked afterwards.  Leaving at the first missing corner made every entry wait
-// for the one before it, up to eight trips to the L2 in nearly every wavefront
-// (one of its lanes stands at a block's edge), and the branches kept 126 - 168
-// registers alive instead of 53 - 94, three or four wavefronts per SIMD instead
-// of five to eight.  2^22 ray samples, rows of four, 200 k blocks: forward with
-// its operands 166 -> 131 us, gradient of the positions 158 -> 87, backward 296
-// -> 219, second order 262 -> 212; 10^6 samples, rows of sixteen: 75 -> 56, 140
-// -> 121, 293 -> 220, 200 -> 167.
-template <bool LDS>
-__device__ __forceinline__ void resolve_rows(const QDev& a, const CellLut& lut,
-                                             const QueryInputs& in, uint32_t (&row)[8],
-                                             float (&o)[3]) {
-    bool valid = in.m != 0 && static_cast<uint32_t>(in.gi) < static_cast<uint32_t>(a.B);
-    const int64_t gi = valid ? in.gi : 0;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) o[d] = valid ? in.o[d] : 0.f;
-    const int64_t ci = in.ci < 0 ? 0 : (in.ci >= a.M ? a.M - 1 : in.ci);
-    // Block indices are below 2^31 and a missing block is -1, so the low
-    // dword of each int64 table entry carries everything.
-    const int32_t* lut_g32 = reinterpret_cast<const int32_t*>(a.lut_g) + gi * 16;
-    uint32_t nb_cell[8], nb_grid[8];
-    int32_t own = -1, other[8];
-    if (valid) own = lut_g32[0];
-    cell_neighbors<LDS>(a, lut, ci, nb_cell, nb_grid);
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        other[c] = -1;
-        if (valid && nb_grid[c] != 0) other[c] = lut_g32[nb_grid[c] * 2];
-    }
-    const uint32_t cells = static_cast<uint32_t>(a.M);
-    uint32_t most = 0;   // a missing block is the largest number
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        const uint32_t g = static_cast<uint32_t>(nb_grid[c] != 0 ? other[c] : own);
-        most = g > most ? g : most;
-        row[c] = g * cells + nb_cell[c];
-    }
-    valid = valid && most < static_cast<uint32_t>(a.B);
-    if (!valid) row[0] = kNoRow;
-}
-
-template <bool LDS>
-__device__ __forceinline__ void resolve_rows(const QDev& a, const CellLut& lut,
-                                             int64_t q, uint32_t (&row)[8],
-                                             float (&o)[3]) {
-    resolve_rows<LDS>(a, lut, load_inputs(a, q), row, o);
 }
 
 // Runs phase 1 for the tile and hands every thread the rows / offsets of the
@@ -386,13 +118,6 @@ struct VecOf<float, 4> {
 template <>
 struct VecOf<float, 1> {
     using type = float;
-};
-// Rows of two, three or five fp32 channels taken whole by one lane: a row is
-// only 4-byte aligned in general (rows of 12 or 20 bytes follow each other), which is
-// all a global load of several dwords asks for on this device.
-template <int N>
-struct alignas(4) FloatRow {
-    float v[N];
 };
 template <>
 struct VecOf<float, 2> {
@@ -806,670 +531,6 @@ query_backward_backward_kernel(
     }
 }
 
-// ================================================= backward kernels by rows
-// fp32 rows of few channels (rows_by_lane): one lane holds a whole query, as in the
-// forward kernel, so that a wavefront serves 64 queries per tile: four channels have four
-// times the loads in flight and a quarter of the per-query arithmetic of the
-// one-lane-per-channel kernels above, and rows of five leave no lanes idle.
-//
-// Gradient rows.  The memory side executes atomics at a fixed rate of
-// requests, and one request is what one instruction of a wavefront sends to
-// one 64-byte line, whether it carries one float or sixteen (measured: 18 G
-// requests/s for 4-byte and for 64-byte groups alike).  The eight corners of a
-// query and the queries that follow it along a ray meet the same few lines
-// over and over -- the x neighbour is the next row, a corner of this sample is
-// another corner of the next -- but in different instructions.  So every
-// wavefront first adds its contributions into a small table of lines in LDS
-// (open addressing on the line number, sixteen floats per entry; a row may end in the
-// line after the one it starts in) and sends the
-// table out once per tile, one line per sixteen lanes: a third of the requests
-// on ray-ordered samples.  Before that, runs of consecutive queries with the
-// same row are summed in registers (lane exchange inside a row of 16 lanes is
-// a modifier of an ordinary vector instruction, across rows it would be a trip
-// through the LDS pipeline, so a run is cut at the row of lanes; the table
-// joins the pieces).  A row whose line finds no place within kLineProbes steps
-// goes to memory directly, and a wavefront that sent more rows that way than
-// the table has lines leaves the table aside for the next kLineRest tiles.
-//
-// Queries in no order share no lines but those of neighbouring corners.  A tile of which
-// more than half lie in another block than the query before them leaves the table aside
-// at once: the rows of two corners that differ in x follow each other in memory, and leave
-// together by neighbouring lanes of one instruction, five requests for eight rows of four
-// channels (rows of one by one through the table until it had rested: 398 -> 273 us for
-// 1 M unordered queries of four channels, 17 -> 7 for 1000).  Ordered tiles pay 1 us of a
-// launch for that (131 000 of four channels 12.2 -> 13.5, 4 M 251 -> 253).
-// Every corner with a copy of its code: one copy for all, which selects its row and its
-// terms, takes half as long again (131 000 of four channels 19 us), as does a second pass
-// for the rows past the table (14.6).
-template <int CTRL>
-__device__ __forceinline__ int dpp_int(int v) {
-    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
-}
-template <int CTRL, typename T>
-__device__ __forceinline__ T dpp(T v) {
-    static_assert(sizeof(T) == 4, "32-bit values");
-    return __builtin_bit_cast(T, dpp_int<CTRL>(__builtin_bit_cast(int, v)));
-}
-constexpr int kRowShl = 0x100;  // lane i takes lane i + n of its row of 16 (0 beyond it)
-constexpr int kRowShr = 0x110;  // lane i takes lane i - n
-
-constexpr int kRowBcast15 = 0x142;  // every lane of a row takes lane 15 of the row before
-
-// Runs of consecutive lanes whose queries lie in the same cell.  Two queries
-// meet in the same row at a corner only when they lie in the same cell, and
-// then at every corner, so the runs are found once per tile, from the row of the
-// cell itself, and the sums over them are taken corner by corner (sum_runs).
-// The sums run inside the rows of 16 lanes; a run that goes on in the next row
-// hands its part over: lane 15 keeps quiet and the lane that ends the run in
-// the next row adds what lane 15 had.  (A run that fills a whole row and still
-// goes on is not handed over a second time; its parts meet in the table of
-// lines.)
-struct Runs {
-    bool any;         // some lane continues the run of the lane before it (the same for all lanes)
-    bool take[4];     // step 1, 2, 4, 8 of the segmented sum adds what lies that far below
-    bool takes_offer; // adds what lane 15 of the row before holds
-    bool tail;        // this lane ends its run and holds the total
-    bool ordered;     // half of the queries are less than a block's cells from the one before (the same for all lanes)
-};
-
-// The runs of a tile.  Lanes without a query (not `on`) get a number no neighbour shares.
-// `cells`: of a block.  Every lane of the wavefront must take part.
-__device__ __forceinline__ Runs find_runs(uint32_t cell_row, bool on, uint32_t cells, int lane) {
-    Runs r;
-    const uint32_t id = on ? cell_row : (kNoRow - static_cast<uint32_t>(lane & 1));
-    const int g = lane & 15;
-    const uint32_t prev = dpp<kRowShr + 1>(id);
-    const uint32_t ahead = id - prev, behind = prev - id;
-    const uint64_t queries = __builtin_amdgcn_ballot_w64(on);
-    const uint64_t near = __builtin_amdgcn_ballot_w64((ahead < behind ? ahead : behind) < cells);
-    r.ordered = 2 * __popcll(near & queries) >= __popcll(queries);
-    const uint32_t next = dpp<kRowShl + 1>(id);
-    const bool joins = g > 0 && prev == id;
-    r.any = __ballot(joins) != 0;
-    const bool starts = g > 0 && prev != id;   // a run starts here, inside the row
-    int f = (g == 0 || starts) ? 1 : 0;        // a run starts at or below this lane, as far as summed
-    {
-        const int fu = dpp_int<kRowShr + 1>(f);
-        r.take[0] = g >= 1 && !f;
-        if (r.take[0]) f |= fu;
-    }
-    {
-        const int fu = dpp_int<kRowShr + 2>(f);
-        r.take[1] = g >= 2 && !f;
-        if (r.take[1]) f |= fu;
-    }
-    {
-        const int fu = dpp_int<kRowShr + 4>(f);
-        r.take[2] = g >= 4 && !f;
-        if (r.take[2]) f |= fu;
-    }
-    r.take[3] = g >= 8 && !f;
-    bool tail = g == 15 || next != id;
-    // in the first run of its row: no run starts between the row's first lane and here
-    const uint64_t started = __ballot(starts);
-    const uint64_t upto = (2ull << lane) - 1ull;
-    const uint64_t row_lanes = 0xFFFFull << (lane & 48);
-    const bool first_run = (started & upto & row_lanes) == 0;
-    // lane 15 offers its sum unless its run began with the row
-    const int offers = (g == 15 && !first_run) ? 1 : 0;
-    const int offered = dpp_int<kRowBcast15>(offers);
-    const uint32_t offered_id = dpp<kRowBcast15>(id);
-    r.takes_offer = lane >= 16 && tail && first_run && offered != 0 && offered_id == id;
-    // ... and keeps quiet when the next row takes the offer
-    const uint32_t id16 = __builtin_amdgcn_readlane(id, 16);
-    const uint32_t id32 = __builtin_amdgcn_readlane(id, 32);
-    const uint32_t id48 = __builtin_amdgcn_readlane(id, 48);
-    const uint32_t over = lane < 16 ? id16 : lane < 32 ? id32 : id48;
-    if (offers != 0 && lane < 48 && over == id) tail = false;
-    r.tail = tail;
-    return r;
-}
-
-template <int D, int E>
-__device__ __forceinline__ void run_step(float (&v)[E], bool take) {
-#pragma unroll
-    for (int k = 0; k < E; ++k) {
-        const float vu = dpp<kRowShr + D>(v[k]);
-        if (take) v[k] += vu;
-    }
-}
-
-// Sums `v` over the runs; the lanes with r.tail hold the totals afterwards.
-// Every lane of the wavefront must take part.
-template <int E>
-__device__ __forceinline__ void sum_runs(const Runs& r, float (&v)[E]) {
-    run_step<1>(v, r.take[0]);
-    run_step<2>(v, r.take[1]);
-    run_step<4>(v, r.take[2]);
-    run_step<8>(v, r.take[3]);
-#pragma unroll
-    for (int k = 0; k < E; ++k) {
-        const float part = dpp<kRowBcast15>(v[k]);
-        if (r.takes_offer) v[k] += part;
-    }
-}
-
-constexpr int kLineSlots = 128;   // lines per wavefront's table
-constexpr int kLineProbes = 4;
-constexpr int kLineRest = 7;
-// Lanes that a row leaves past the table by, and rows of one instruction (of one
-// channel: of a quarter of its lanes, for which there is room)
-constexpr int line_out_lanes(int E) { return E <= 4 ? 4 : E <= 8 ? 8 : 16; }
-constexpr int line_out_rows(int E) { return 64 / line_out_lanes(E); }
-constexpr uint32_t kLineFree = 0xFFFFFFFFu;
-// float k of slot h sits at k * kLinePitch + h: the sixteen floats of a line
-// and the same float of neighbouring slots fall into different banks
-constexpr int kLinePitch = kLineSlots + 1;
-
-struct LineTable {
-    float val[16 * kLinePitch];
-    uint32_t key[kLineSlots];
-    // rows on their way to memory without the table; the flush keeps its list
-    // of used slots in the same place
-    union {
-        struct {
-            uint32_t row[16];
-            float v[64];
-        } out;
-        uint8_t used[kLineSlots];
-    };
-};
-
-// Orders the LDS traffic of one wavefront (whose LDS instructions execute in
-// program order, each for all its lanes) for the compiler.
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// The floats of a row added to their places in LDS, `at(k)` for the k-th.  The LDS
-// executes a floating-point add atomic one lane after the other (about three cycles a
-// lane, measured) and a 32-bit compare-and-swap at full rate: the add is a read
-// and a compare-and-swap of the sum.  The floats go side by side, two
-// round trips for all of them; lanes that met another lane's update in between
-// (seldom: runs of equal rows have been summed before) repeat float by float.
-template <int E, typename At>
-__device__ __forceinline__ void lds_add(At at, const float (&v)[E]) {
-    unsigned int seen[E], got[E];
-#pragma unroll
-    for (int k = 0; k < E; ++k) seen[k] = *at(k);
-#pragma unroll
-    for (int k = 0; k < E; ++k) {
-        got[k] = atomicCAS(at(k), seen[k], __float_as_uint(__uint_as_float(seen[k]) + v[k]));
-    }
-    bool done = true;
-#pragma unroll
-    for (int k = 0; k < E; ++k) done = done && got[k] == seen[k];
-    if (done) return;
-#pragma unroll 1
-    for (int k = 0; k < E; ++k) {
-        // (selects, not an indexed access: the arrays stay in registers)
-        unsigned int g = got[0], s = seen[0];
-        float add = v[0];
-#pragma unroll
-        for (int q = 1; q < E; ++q) {
-            g = k == q ? got[q] : g;
-            s = k == q ? seen[q] : s;
-            add = k == q ? v[q] : add;
-        }
-        while (g != s) {
-            s = g;
-            g = atomicCAS(at(k), s, __float_as_uint(__uint_as_float(s) + add));
-        }
-    }
-}
-
-// Line of a row's first float, and where in it that stands.
-template <int E>
-__device__ __forceinline__ void line_of(uint32_t row, uint32_t& line, uint32_t& pos) {
-    if constexpr (16 % E == 0) {
-        line = row / (16 / E);
-        pos = row % (16 / E) * E;
-    } else {
-        const uint64_t first = static_cast<uint64_t>(row) * E;
-        line = static_cast<uint32_t>(first >> 4);
-        pos = static_cast<uint32_t>(first) & 15u;
-    }
-}
-
-struct LineAcc {
-    LineTable* tab;
-    int rest;      // tiles left during which the table is left aside
-    int spilled;   // rows that found no place in the table since the last flush (whole wavefront)
-    bool aside;    // the table is left aside during this tile, and its place used otherwise
-    bool ready;    // the table is empty and its floats are zero (at the start of a tile)
-
-    __device__ __forceinline__ void start(LineTable* t, int lane) {
-        tab = t;
-        rest = 0;
-        spilled = 0;
-        if (tab != nullptr) empty(lane);
-    }
-
-    __device__ __forceinline__ void empty(int lane) {
-        for (int i = lane; i < 16 * kLinePitch; i += 64) tab->val[i] = 0.f;
-        tab->key[lane] = kLineFree;
-        tab->key[lane + 64] = kLineFree;
-        wave_lds_fence();
-        ready = true;
-    }
-
-    // Whole wavefront, before the first row of a tile.
-    __device__ __forceinline__ void tile(bool ordered, int lane) {
-        aside = rest > 0 || !ordered;
-        if (!aside && !ready) empty(lane);
-    }
-
-    // The slot of `line`, or kLineSlots where it finds no place.
-    __device__ __forceinline__ uint32_t slot_of(uint32_t line) {
-        uint32_t h = (line * 0x9E3779B1u) >> 25;
-#pragma unroll 1
-        for (int p = 0; p < kLineProbes; ++p) {
-            const uint32_t old = atomicCAS(&tab->key[h], kLineFree, line);
-            if (old == kLineFree || old == line) return h;
-            h = (h + 1) & (kLineSlots - 1);
-        }
-        return kLineSlots;
-    }
-
-    // grad[E * row .. E * row + E - 1] += v for the lanes that `want`; every lane
-    // of the wavefront must take part.
-    template <int E>
-    __device__ __forceinline__ void add(float* __restrict__ grad, bool want, uint32_t row,
-                                        const float (&v)[E], int lane) {
-        bool placed = false;
-        if (want) {
-            uint32_t line, pos;
-            line_of<E>(row, line, pos);
-            const uint32_t h = slot_of(line);
-            placed = h < kLineSlots;
-            if constexpr (16 % E == 0) {
-                unsigned int* at = reinterpret_cast<unsigned int*>(tab->val + pos * kLinePitch + h);
-                if (placed) lds_add<E>([&](int k) { return at + k * kLinePitch; }, v);
-            } else {
-                // a row may end in the next line (a line that was claimed for it alone
-                // and stays empty where this one finds no place sends nothing)
-                uint32_t next = h;
-                if (placed && pos + E > 16u) {
-                    next = slot_of(line + 1u);
-                    placed = next < kLineSlots;
-                }
-                unsigned int* at = reinterpret_cast<unsigned int*>(tab->val + pos * kLinePitch + h);
-                const int over = static_cast<int>(next) - static_cast<int>(h) - 16 * kLinePitch;
-                if (placed) {
-                    lds_add<E>([&](int k) { return at + k * kLinePitch + (pos + k > 15u ? over : 0); }, v);
-                }
-            }
-        }
-        // The rest goes to memory now, regrouped so that the floats of a
-        // row leave from neighbouring lanes of one instruction (one request a
-        // row; one lane sending its floats would make as many).
-        const uint64_t out = __ballot(want && !placed);
-        if (out == 0) return;
-        constexpr int kLanes = line_out_lanes(E), kRows = line_out_rows(E);
-        const int n = __popcll(out);
-        const int mine = __popcll(out & ((1ull << lane) - 1ull));
-        spilled += n;
-        for (int i = 0; i < n; i += kRows) {
-            const int at = mine - i;
-            wave_lds_fence();
-            if (want && !placed && at >= 0 && at < kRows) {
-                tab->out.row[at] = row;
-                if constexpr (E == 4) {
-                    *reinterpret_cast<float4*>(tab->out.v + at * 4) = make_float4(v[0], v[1], v[2], v[3]);
-                } else {
-#pragma unroll
-                    for (int k = 0; k < E; ++k) tab->out.v[at * kLanes + k] = v[k];
-                }
-            }
-            wave_lds_fence();
-            const int e = lane / kLanes, k = lane % kLanes;
-            if (i + e < n && k < E) {
-                unsafeAtomicAdd(grad + static_cast<uint64_t>(tab->out.row[e]) * E + k, tab->out.v[lane]);
-            }
-        }
-        wave_lds_fence();
-    }
-
-    // The same past the table, which is left aside and leaves room for all rows of two
-    // corners: these follow each other in memory as a rule, and leave together.
-    template <int E>
-    __device__ __forceinline__ void send_two(float* __restrict__ grad, bool want, const uint32_t (&row)[2],
-                                             const float (&v)[2][E], int lane) {
-        constexpr int kPitch = 2 * E + 1, kAtOnce = 64 / (2 * E);
-        static_assert(64 * (kPitch + 2) <= 16 * kLinePitch, "128 rows and their numbers");
-        const uint64_t out = __ballot(want);
-        const int n = __popcll(out);
-        const int mine = __popcll(out & ((1ull << lane) - 1ull));
-        uint32_t* const rows = reinterpret_cast<uint32_t*>(tab->val);
-        float* const floats = tab->val + 128;
-        wave_lds_fence();
-        if (want) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                rows[2 * mine + h] = row[h];
-#pragma unroll
-                for (int k = 0; k < E; ++k) floats[mine * kPitch + h * E + k] = v[h][k];
-            }
-        }
-        wave_lds_fence();
-        const int e = lane / (2 * E), at = lane % (2 * E);
-        const int half = at >= E ? 1 : 0, k = at - half * E;
-        for (int i = e; i < n && e < kAtOnce; i += kAtOnce) {
-            unsafeAtomicAdd(grad + static_cast<uint64_t>(rows[2 * i + half]) * E + k, floats[i * kPitch + at]);
-        }
-    }
-
-    // Whole wavefront: sends the table's lines out and empties it.
-    __device__ __forceinline__ void flush(float* __restrict__ grad, int lane) {
-        wave_lds_fence();
-        const bool lo = tab->key[lane] != kLineFree;
-        const bool hi = tab->key[lane + 64] != kLineFree;
-        const uint64_t mlo = __ballot(lo), mhi = __ballot(hi);
-        const uint64_t below = (1ull << lane) - 1ull;
-        const int nlo = __popcll(mlo);
-        const int n = nlo + __popcll(mhi);
-        if (lo) tab->used[__popcll(mlo & below)] = static_cast<uint8_t>(lane);
-        if (hi) tab->used[nlo + __popcll(mhi & below)] = static_cast<uint8_t>(lane + 64);
-        wave_lds_fence();
-        // four lines per instruction, sixteen lines per turn: the reads of
-        // a turn are issued together
-        for (int i = 0; i < n; i += 16) {
-            uint32_t h[4], line[4];
-            float v[4];
-            float* at[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int e = i + j * 4 + (lane >> 4);
-                h[j] = e < n ? tab->used[e] : 0u;
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int e = i + j * 4 + (lane >> 4);
-                at[j] = tab->val + (lane & 15) * kLinePitch + h[j];
-                line[j] = tab->key[h[j]];
-                v[j] = e < n ? *at[j] : 0.f;
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                // floats nobody contributed to are zero
-                if (v[j] != 0.f) {
-                    *at[j] = 0.f;
-                    unsafeAtomicAdd(
-                            grad + ((static_cast<uint64_t>(line[j]) << 4) | (lane & 15)), v[j]);
-                }
-            }
-        }
-        wave_lds_fence();
-        tab->key[lane] = kLineFree;
-        tab->key[lane + 64] = kLineFree;
-        wave_lds_fence();
-    }
-
-    // The tile is done with.
-    __device__ __forceinline__ void done() {
-        if (aside) ready = false;
-        if (rest > 0) {
-            --rest;
-        } else if (spilled > kLineSlots) {
-            rest = kLineRest;   // more rows went past the table than it has lines
-        }
-        spilled = 0;
-    }
-};
-
-// grad_emb[row[c], 0..E - 1] += part(c, v) of the eight corners for the lanes that are
-// `on`; every lane of the wavefront must take part.  `runs`: find_runs of this tile.
-template <int E, typename Part>
-__device__ __forceinline__ void scatter_rows(LineAcc& acc, float* __restrict__ grad_emb,
-                                             const uint32_t (&row)[8], bool on, const Runs& runs,
-                                             Part part, int lane) {
-    // (samples cells apart, scattered points: nothing to join)
-    const bool want = on && (!runs.any || runs.tail);
-    if (acc.aside) {
-#pragma unroll
-        for (int c = 0; c < 8; c += 2) {
-            const uint32_t rows[2] = {row[c], row[c + 1]};
-            float v[2][E];
-            part(c, v[0]);
-            part(c + 1, v[1]);
-            if (runs.any) {
-                sum_runs(runs, v[0]);
-                sum_runs(runs, v[1]);
-            }
-            acc.send_two<E>(grad_emb, want, rows, v, lane);
-        }
-    } else {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            float v[E];
-            part(c, v);
-            if (runs.any) sum_runs(runs, v);
-            acc.add<E>(grad_emb, want, row[c], v, lane);
-        }
-        acc.flush(grad_emb, lane);
-    }
-    acc.done();
-}
-
-__device__ __forceinline__ LineTable* line_table(unsigned char* smem, const QDev& a,
-                                                 bool lds_lut, bool wanted) {
-    if (!wanted) return nullptr;
-    return reinterpret_cast<LineTable*>(smem + table_offset(a, 1, lds_lut)) +
-           (threadIdx.x >> 6);
-}
-
-// Rows of E floats, by a lane each (16-byte aligned where E is four).
-template <int E>
-__device__ __forceinline__ void load_whole_row(const float* __restrict__ at, float (&v)[E]) {
-    if constexpr (E == 4) {
-        const float4 r = *reinterpret_cast<const float4*>(at);
-        v[0] = r.x, v[1] = r.y, v[2] = r.z, v[3] = r.w;
-    } else {
-        const FloatRow<E> r = *reinterpret_cast<const FloatRow<E>*>(at);
-#pragma unroll
-        for (int k = 0; k < E; ++k) v[k] = r.v[k];
-    }
-}
-
-template <int E>
-__device__ __forceinline__ void load_row_once(const float* __restrict__ at, float (&v)[E]) {
-    if constexpr (E == 4) {
-        typedef float v4f __attribute__((ext_vector_type(4)));
-        const v4f r = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(at));
-        v[0] = r.x, v[1] = r.y, v[2] = r.z, v[3] = r.w;
-    } else {
-#pragma unroll
-        for (int k = 0; k < E; ++k) v[k] = __builtin_nontemporal_load(at + k);
-    }
-}
-
-template <int E>
-__device__ __forceinline__ float row_product(const float (&a)[E], const float (&b)[E]) {
-    if constexpr (E >= 8) {
-        // pairs, pairs of pairs, ..., as a lane per channel adds them up: one after the
-        // other, wide rows lose by the roundings of the sum what they gain by those of the
-        // products (error against 64 bits, 2-norm: of eight channels 9.5e-8 and 9.7e-8, of
-        // twelve 9.7e-8 and 1.03e-7; of five 9.3e-8 and 9.2e-8)
-        constexpr int kWide = E > 8 ? 16 : 8;
-        float p[kWide];
-#pragma unroll
-        for (int k = 0; k < kWide; ++k) p[k] = k < E ? __fmul_rn(a[k < E ? k : 0], b[k < E ? k : 0]) : 0.f;
-#pragma unroll
-        for (int n = kWide / 2; n > 0; n /= 2) {
-#pragma unroll
-            for (int k = 0; k < n; ++k) p[k] = __fadd_rn(p[2 * k], p[2 * k + 1]);
-        }
-        return p[0];
-    } else {
-        float dot = a[0] * b[0];
-#pragma unroll
-        for (int k = 1; k < E; ++k) dot += a[k] * b[k];
-        return dot;
-    }
-}
-
-// First-order backward, rows of E (formulas as in query_backward_forward_kernel).
-template <int E, bool LDS, int OUT, int THREADS>
-__global__ __launch_bounds__(THREADS, waves_of_rows(E, THREADS)) void
-query_backward_forward_vec_kernel(
-        QDev a, const float* __restrict__ z, float* __restrict__ grad_emb,
-        float* __restrict__ grad_off, const float* __restrict__ gg_off,
-        const float* __restrict__ z2) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    const CellLut lut = stage_cell_lut<LDS, THREADS>(a, smem);
-    const int lane = threadIdx.x & 63;
-    const float* __restrict__ emb = static_cast<const float*>(a.emb);
-    constexpr bool want_emb = (OUT & 1) != 0;
-    constexpr bool want_off = (OUT & 2) != 0;
-    constexpr bool second = (OUT & 4) != 0;
-    LineAcc acc;
-    acc.start(line_table(smem, a, LDS, want_emb), lane);
-    const int64_t ntiles = (a.N + THREADS - 1) / THREADS;
-    TileWalk walk(ntiles);
-    for (int64_t tile = walk.next; tile < walk.end; tile += walk.step) {
-        uint32_t row[8];
-        float o[3];
-        const int64_t q = tile * THREADS + threadIdx.x;
-        const QueryInputs in = load_inputs(a, q);
-        resolve_rows<LDS>(a, lut, in, row, o);
-        const bool on = row[0] != kNoRow;
-        float zq[E] = {}, yq[E] = {};
-        float gg[3] = {0.f, 0.f, 0.f};
-        if (on) {
-            load_row_once<E>(z + q * E, zq);
-            if constexpr (second) {
-                load_row_once<E>(z2 + q * E, yq);
-                gg[0] = __builtin_nontemporal_load(gg_off + q * 3 + 0) * static_cast<float>(a.offset_scale);
-                gg[1] = __builtin_nontemporal_load(gg_off + q * 3 + 1) * static_cast<float>(a.offset_scale);
-                gg[2] = __builtin_nontemporal_load(gg_off + q * 3 + 2) * static_cast<float>(a.offset_scale);
-            }
-        }
-        AxisTerms<float> t;
-        axis_terms<float, true>(o, a.smooth, t);
-        // the gathered rows are used up before the scatter starts, which keeps
-        // them out of the registers the scatter needs
-        if constexpr (want_off) {
-            float e[8][E];
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-#pragma unroll
-                for (int k = 0; k < E; ++k) e[c][k] = 0.f;
-                if (on) load_whole_row<E>(emb + static_cast<int64_t>(row[c]) * E, e[c]);
-            }
-            float go[3] = {0.f, 0.f, 0.f};
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                float gw[3];
-                corner_weight_grad<float>(t, c, gw);
-                const float dot = row_product<E>(e[c], zq);
-                go[0] += dot * gw[0];
-                go[1] += dot * gw[1];
-                go[2] += dot * gw[2];
-            }
-            if (q < a.N) {
-                const float scale = static_cast<float>(a.offset_scale);
-                __builtin_nontemporal_store(on ? go[0] * scale : 0.f, grad_off + q * 3 + 0);
-                __builtin_nontemporal_store(on ? go[1] * scale : 0.f, grad_off + q * 3 + 1);
-                __builtin_nontemporal_store(on ? go[2] * scale : 0.f, grad_off + q * 3 + 2);
-            }
-        }
-        if constexpr (want_emb) {
-            const Runs runs = find_runs(row[0], on, static_cast<uint32_t>(a.M), lane);
-            acc.tile(runs.ordered, lane);
-            SlopeTerms<float> slope;
-            if constexpr (second) slope_terms<float>(t, gg, slope);
-            scatter_rows<E>(acc, grad_emb, row, on, runs, [&](int c, float (&v)[E]) {
-                const float w = corner_weight<float>(t, c);
-#pragma unroll
-                for (int k = 0; k < E; ++k) v[k] = w * zq[k];
-                if constexpr (second) {
-                    const float d = corner_slope<float>(t, slope, c);
-#pragma unroll
-                    for (int k = 0; k < E; ++k) v[k] += d * yq[k];
-                }
-            }, lane);
-        }
-    }
-}
-
-// Backward of the backward, rows of E (formulas as in
-// query_backward_backward_kernel).
-template <int E, bool LDS, int OUT, int THREADS>
-__global__ __launch_bounds__(THREADS, waves_of_rows(E, THREADS)) void
-query_backward_backward_vec_kernel(
-        QDev a, const float* __restrict__ gg_off, const float* __restrict__ z,
-        float* __restrict__ grad_z, float* __restrict__ grad_emb) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    const CellLut lut = stage_cell_lut<LDS, THREADS>(a, smem);
-    const int lane = threadIdx.x & 63;
-    const float* __restrict__ emb = static_cast<const float*>(a.emb);
-    constexpr bool want_emb = (OUT & 1) != 0;
-    constexpr bool want_z = (OUT & 2) != 0;
-    LineAcc acc;
-    acc.start(line_table(smem, a, LDS, want_emb), lane);
-    const int64_t ntiles = (a.N + THREADS - 1) / THREADS;
-    TileWalk walk(ntiles);
-    for (int64_t tile = walk.next; tile < walk.end; tile += walk.step) {
-        uint32_t row[8];
-        float o[3];
-        const int64_t q = tile * THREADS + threadIdx.x;
-        const QueryInputs in = load_inputs(a, q);
-        resolve_rows<LDS>(a, lut, in, row, o);
-        const bool on = row[0] != kNoRow;
-        float zq[E] = {};
-        float gg[3] = {0.f, 0.f, 0.f};
-        if (on) {
-            load_row_once<E>(z + q * E, zq);
-            gg[0] = __builtin_nontemporal_load(gg_off + q * 3 + 0) * static_cast<float>(a.offset_scale);
-            gg[1] = __builtin_nontemporal_load(gg_off + q * 3 + 1) * static_cast<float>(a.offset_scale);
-            gg[2] = __builtin_nontemporal_load(gg_off + q * 3 + 2) * static_cast<float>(a.offset_scale);
-        }
-        AxisTerms<float> t;
-        axis_terms<float, true>(o, a.smooth, t);
-        if constexpr (want_z) {
-            float e[8][E];
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-#pragma unroll
-                for (int k = 0; k < E; ++k) e[c][k] = 0.f;
-                if (on) load_whole_row<E>(emb + static_cast<int64_t>(row[c]) * E, e[c]);
-            }
-            float gz[E] = {};
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                float gw[3];
-                corner_weight_grad<float>(t, c, gw);
-                const float d = gw[0] * gg[0] + gw[1] * gg[1] + gw[2] * gg[2];
-#pragma unroll
-                for (int k = 0; k < E; ++k) gz[k] += d * e[c][k];
-            }
-            if (q < a.N) {
-                if constexpr (E == 4) {
-                    typedef float v4f __attribute__((ext_vector_type(4)));
-                    const v4f g4 = {on ? gz[0] : 0.f, on ? gz[1] : 0.f, on ? gz[2] : 0.f, on ? gz[3] : 0.f};
-                    __builtin_nontemporal_store(g4, reinterpret_cast<v4f*>(grad_z + q * 4));
-                } else {
-#pragma unroll
-                    for (int k = 0; k < E; ++k) __builtin_nontemporal_store(on ? gz[k] : 0.f, grad_z + q * E + k);
-                }
-            }
-        }
-        if constexpr (want_emb) {
-            const Runs runs = find_runs(row[0], on, static_cast<uint32_t>(a.M), lane);
-            acc.tile(runs.ordered, lane);
-            scatter_rows<E>(acc, grad_emb, row, on, runs, [&](int c, float (&v)[E]) {
-                float gw[3];
-                corner_weight_grad<float>(t, c, gw);
-                const float d = gw[0] * gg[0] + gw[1] * gg[1] + gw[2] * gg[2];
-#pragma unroll
-                for (int k = 0; k < E; ++k) v[k] = d * zq[k];
-            }, lane);
-        }
-    }
-}
-
 // Sparse convolution forward (ash/src/grid.cu:948-1043): for every cell of the
 // listed blocks, out[row] = sum over the K window taps k of
 // in[row of neighbour k] * w[k], channel by channel, taps whose block is
@@ -1565,7 +626,6 @@ __global__ __launch_bounds__(kBlock) void convolution_cell_kernel(ConvDev a, int
 // are kept in LDS in compact form (uint16 cell, uint8 block offset) for the
 // whole launch, when they fit.  Taps, order and arithmetic are unchanged.
 constexpr int kConvThreads = 512;
-unsigned persistent_grid(int64_t ntiles, size_t smem, int max_per_cu = 8);
 
 template <typename T, int EC>
 __global__ __launch_bounds__(kConvThreads) void convolution_block_kernel(
@@ -2425,34 +1485,8 @@ int pow2_ceil(int v) {
     return p;
 }
 
-// Whether the per-cell tables go to LDS.  Up to 2^19 queries a workgroup of a
-// full device meets one tile, and filling its LDS (sixteen table entries a cell,
-// a trip to the L2 and a barrier) costs more than reading the tables where they
-// are.  Blocks of 8^3, ray-ordered queries: forward of 131 k rows of four 7.5 ->
-// 6.1 us, 524 k 23.5 -> 17.2; gradient of the positions 524 k 21.3 -> 14.3; rows
-// of sixteen 131 k 9.8 -> 8.3.  Unordered ones, rows of four: 100 k 15.5 -> 14.3,
-// 500 k 56.1 and 56.0.  Above, ordered and unordered queries part (1 M: 33.9
-// against 27.1, and 109 against 117), and at 4 M LDS is ahead for both (132
-// against 139, 701 against 745 for rows of sixteen).
-constexpr int64_t kMaxDirectQueries = int64_t{1} << 19;
-bool lut_in_lds(const QDev& d) { return d.M <= kMaxLdsCells && d.N > kMaxDirectQueries; }
-
-size_t smem_bytes(const QDev& d, int lpq, int line_tables = 0) {
-    return table_offset(d, lpq, lut_in_lds(d)) + line_tables * sizeof(LineTable);
-}
-
-// Enough persistent workgroups to fill every CU as far as LDS allows.
-unsigned persistent_grid(int64_t ntiles, size_t smem, int max_per_cu) {
-    int per_cu = max_per_cu;
-    if (smem > 0) {
-        const int fit = static_cast<int>(kLdsPerCu / smem);
-        if (fit < per_cu) per_cu = fit < 1 ? 1 : fit;
-    }
-    int64_t g = static_cast<int64_t>(compute_units()) * per_cu;
-    if (g > ntiles) g = ntiles;
-    g = (g + kXcds - 1) / kXcds * kXcds;  // whole rounds over the XCDs
-    if (g < kXcds) g = kXcds;
-    return static_cast<unsigned>(g);
+size_t smem_bytes(const QDev& d, int lpq) {
+    return table_offset(d, lpq, lut_in_lds(d));
 }
 
 template <typename T, int VEC, int LPQ>
@@ -2487,17 +1521,6 @@ int launch_grid_forward(const QDev& d, const FrontDev& f, void* out, hipStream_t
 #undef ASH_GF
     ASH_LAUNCH_CHECK();
     return 0;
-}
-
-// What a first-order backward takes along of the second order: nothing, or the
-// gradient with respect to the offsets' gradient and the z of that pass.
-struct Second {
-    const void* gg;
-    const void* z;
-};
-
-int gradients_wanted(const void* ge, const void* go, const Second& also) {
-    return (ge != nullptr ? 1 : 0) | (go != nullptr ? 2 : 0) | (also.gg != nullptr ? 4 : 0);
 }
 
 template <typename T, int LPQ>
@@ -2549,94 +1572,6 @@ int launch_bwd_bwd(const QDev& d, const void* gg, const void* z, void* gz,
         if (out == 3) ASH_BB(false, 3);
         else if (out == 1) ASH_BB(false, 1);
         else ASH_BB(false, 2);
-    }
-#undef ASH_BB
-    ASH_LAUNCH_CHECK();
-    return 0;
-}
-
-bool aligned16(const void* p) {
-    return reinterpret_cast<uintptr_t>(p) % 16 == 0;
-}
-
-// Workgroups of the kernels with line tables (OUT bit 0) share one table of
-// cells between eight wavefronts where two of them fit a CU (blocks of up to 576
-// cells): 80 KB each and sixteen wavefronts on a CU, where three of 44 KB with
-// four are twelve.  2^22 ray samples on 200 k blocks of 8^3: backward 221 -> 190
-// us, second order 214 -> 187; 1.5 x 10^6 unordered queries 541 and 542 us as
-// before (their rows leave past the tables, bound by requests).
-// (Rows of twelve have registers for twelve wavefronts on a CU.)
-constexpr int kWideRows = 8;
-int vec_threads(const QDev& d, int out) {
-    const bool wide = lut_in_lds(d) && (out & 1) != 0 && d.E <= kWideRows && 2 * smem_bytes(d, 1, 2 * kBlock / 64) <= kLdsPerCu;
-    return wide ? 2 * kBlock : kBlock;
-}
-
-template <int E>
-int launch_bwd_fwd_vec(const QDev& d, const void* z, void* ge, void* go, const Second& also,
-                       hipStream_t s) {
-    const int out = gradients_wanted(ge, go, also);
-    const int threads = vec_threads(d, out);
-    const size_t smem = smem_bytes(d, 1, ge != nullptr ? threads / 64 : 0);
-    const unsigned g = persistent_grid((d.N + threads - 1) / threads, smem, resident_rows(E));
-#define ASH_BF(L, O, T)                                                       \
-    query_backward_forward_vec_kernel<E, L, O, T><<<g, T, smem, s>>>(    \
-            d, static_cast<const float*>(z), static_cast<float*>(ge),         \
-            static_cast<float*>(go), static_cast<const float*>(also.gg),      \
-            static_cast<const float*>(also.z))
-    if constexpr (E > 12) {
-        if (lut_in_lds(d)) ASH_BF(true, 2, kBlock);
-        else ASH_BF(false, 2, kBlock);
-    } else if (E <= kWideRows && threads > kBlock) {
-        constexpr int wide = E <= kWideRows ? 2 * kBlock : kBlock;   // (not built for others)
-        if (out == 7) ASH_BF(true, 7, wide);
-        else if (out == 5) ASH_BF(true, 5, wide);
-        else if (out == 3) ASH_BF(true, 3, wide);
-        else ASH_BF(true, 1, wide);
-    } else if (lut_in_lds(d)) {
-        if (out == 7) ASH_BF(true, 7, kBlock);
-        else if (out == 5) ASH_BF(true, 5, kBlock);
-        else if (out == 3) ASH_BF(true, 3, kBlock);
-        else if (out == 1) ASH_BF(true, 1, kBlock);
-        else ASH_BF(true, 2, kBlock);
-    } else {
-        if (out == 7) ASH_BF(false, 7, kBlock);
-        else if (out == 5) ASH_BF(false, 5, kBlock);
-        else if (out == 3) ASH_BF(false, 3, kBlock);
-        else if (out == 1) ASH_BF(false, 1, kBlock);
-        else ASH_BF(false, 2, kBlock);
-    }
-#undef ASH_BF
-    ASH_LAUNCH_CHECK();
-    return 0;
-}
-
-template <int E>
-int launch_bwd_bwd_vec(const QDev& d, const void* gg, const void* z, void* gz,
-                       void* ge, hipStream_t s) {
-    const int out = (ge != nullptr ? 1 : 0) | (gz != nullptr ? 2 : 0);
-    const int threads = vec_threads(d, out);
-    const size_t smem = smem_bytes(d, 1, ge != nullptr ? threads / 64 : 0);
-    const unsigned g = persistent_grid((d.N + threads - 1) / threads, smem, resident_rows(E));
-#define ASH_BB(L, O, T)                                                       \
-    query_backward_backward_vec_kernel<E, L, O, T><<<g, T, smem, s>>>(   \
-            d, static_cast<const float*>(gg), static_cast<const float*>(z),   \
-            static_cast<float*>(gz), static_cast<float*>(ge))
-    if constexpr (E > 12) {
-        if (lut_in_lds(d)) ASH_BB(true, 2, kBlock);
-        else ASH_BB(false, 2, kBlock);
-    } else if (E <= kWideRows && threads > kBlock) {
-        constexpr int wide = E <= kWideRows ? 2 * kBlock : kBlock;
-        if (out == 3) ASH_BB(true, 3, wide);
-        else ASH_BB(true, 1, wide);
-    } else if (lut_in_lds(d)) {
-        if (out == 3) ASH_BB(true, 3, kBlock);
-        else if (out == 1) ASH_BB(true, 1, kBlock);
-        else ASH_BB(true, 2, kBlock);
-    } else {
-        if (out == 3) ASH_BB(false, 3, kBlock);
-        else if (out == 1) ASH_BB(false, 1, kBlock);
-        else ASH_BB(false, 2, kBlock);
     }
 #undef ASH_BB
     ASH_LAUNCH_CHECK();

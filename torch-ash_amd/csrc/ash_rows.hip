@@ -53,11 +53,12 @@ constexpr int waves_of_rows(int E, int threads) { return threads > 256 && (E == 
 // at once: the rows of two corners that differ in x follow each other in memory, and leave
 // together by neighbouring lanes of one instruction, five requests for eight rows of four
 // channels (rows of one by one through the table until it had rested: 398 -> 273 us for
-// 1 M unordered queries of four channels, 17 -> 7 for 1000).  Ordered tiles pay 1 us of a
-// launch for that (131 000 of four channels 12.2 -> 13.5, 4 M 251 -> 253).
+// 1 M unordered queries of four channels, 17 -> 7 for 1000).  Ordered tiles do not pay for
+// it: second order and both orders of four channels, without the test and the rows past
+// the table -> with them, 131 000 12.5 -> 12.3, 400 000 34.9 -> 34.8, 4 M 248 -> 248.
 // Every corner with a copy of its code: one copy for all, which selects its row and its
-// terms, takes half as long again (131 000 of four channels 19 us), as does a second pass
-// for the rows past the table (14.6).
+// terms, takes half as long again (131 000 of four channels 13 -> 19 us), and a second pass
+// for the rows past the table 14.6.
 template <int CTRL>
 __device__ __forceinline__ int dpp_int(int v) {
     return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
@@ -278,16 +279,23 @@ struct LineAcc {
         if (!aside && !ready) empty(lane);
     }
 
-    // The slot of `line`, or kLineSlots where it finds no place.
-    __device__ __forceinline__ uint32_t slot_of(uint32_t line) {
-        uint32_t h = (line * 0x9E3779B1u) >> 25;
+    // Whether `line` finds a place, and its slot.  (Told by a flag: where the loop returns
+    // the slot, it is four blocks with two branches a probe instead of one, in the chain that
+    // a launch waits for: second order of 131 000 of four channels 13.2 us, so 12.3, of five
+    // 17.8 -> 16.3; both orders of 400 000 of four 36.1 -> 34.8, of 1.6 M of five 140 -> 137.)
+    __device__ __forceinline__ bool slot_of(uint32_t line, uint32_t& h) {
+        bool placed = false;
+        h = (line * 0x9E3779B1u) >> 25;
 #pragma unroll 1
         for (int p = 0; p < kLineProbes; ++p) {
             const uint32_t old = atomicCAS(&tab->key[h], kLineFree, line);
-            if (old == kLineFree || old == line) return h;
+            if (old == kLineFree || old == line) {
+                placed = true;
+                break;
+            }
             h = (h + 1) & (kLineSlots - 1);
         }
-        return kLineSlots;
+        return placed;
     }
 
     // grad[E * row .. E * row + E - 1] += v for the lanes that `want`; every lane
@@ -299,8 +307,8 @@ struct LineAcc {
         if (want) {
             uint32_t line, pos;
             line_of<E>(row, line, pos);
-            const uint32_t h = slot_of(line);
-            placed = h < kLineSlots;
+            uint32_t h;
+            placed = slot_of(line, h);
             if constexpr (16 % E == 0) {
                 unsigned int* at = reinterpret_cast<unsigned int*>(tab->val + pos * kLinePitch + h);
                 if (placed) lds_add<E>([&](int k) { return at + k * kLinePitch; }, v);
@@ -308,10 +316,7 @@ struct LineAcc {
                 // a row may end in the next line (a line that was claimed for it alone
                 // and stays empty where this one finds no place sends nothing)
                 uint32_t next = h;
-                if (placed && pos + E > 16u) {
-                    next = slot_of(line + 1u);
-                    placed = next < kLineSlots;
-                }
+                if (placed && pos + E > 16u) placed = slot_of(line + 1u, next);
                 unsigned int* at = reinterpret_cast<unsigned int*>(tab->val + pos * kLinePitch + h);
                 const int over = static_cast<int>(next) - static_cast<int>(h) - 16 * kLinePitch;
                 if (placed) {

@@ -15,13 +15,27 @@
 namespace ash {
 namespace {
 
-// Wavefronts per SIMD of the kernels that give a lane a whole query: two workgroups of eight, which the
-// line tables leave room for, want 128 registers at most (rows of seven 151 -> 118 us; up to
-// six take fewer anyway, twelve need more)
-// (Workgroups of four on a CU without tables: 8 of up to 64 registers, ..., 3 of 168.)
-constexpr int resident_rows(int E) { return E <= 5 ? 8 : E == 6 ? 6 : E == 7 ? 5 : E <= 12 ? 4 : 3; }
+// Wavefronts per SIMD that the kernels are compiled for.  Two workgroups of eight, which
+// the line tables leave room for, want 128 registers at most: both gradients of seven and
+// eight channels, which take 123 - 139 else (rows of seven 151 -> 118 us, for 8 bytes of
+// scratch a lane; eight, 32 and 60; up to six take fewer anyway).  Twelve, held to 168 by
+// three, spill 8 and, both orders with the positions' gradient, 60 bytes.
 constexpr int kWavesRows = 3;
 constexpr int waves_of_rows(int E, int threads) { return threads > 256 && (E == 7 || E == 8) ? 4 : kWavesRows; }
+
+// Workgroups of four wavefronts that are on a CU at once by their registers (the fifth of
+// 96, the fourth of 128, the third of 168; LDS leaves room for four with line tables): a
+// persistent grid of more is not all under way from the start.  `order` 1: the backward,
+// 2: that of the backward; `out`: what is asked for, as the kernels have it.  With four
+// where three fit: 500 000 ray samples, both orders with the positions' gradient and second
+// order with grad_z, of seven channels 82 -> 68 and 76 -> 64 us, of eight 70 -> 58 and 68 ->
+// 57; grad_z alone with six where five fit and four where three: 1.3 M of six 77 -> 70,
+// 660 000 of twelve 56 -> 53.
+constexpr int resident_rows(int E, int order, int out) {
+    if ((out & 1) != 0) return (out & 2) == 0 || E < 7 || (E <= 8 && order == 1 && out == 3) ? 4 : 3;
+    if (order == 1) return E <= 5 ? 8 : E == 6 ? 7 : E == 7 ? 5 : E <= 12 ? 4 : 3;
+    return E <= 3 ? 8 : E == 4 ? 7 : E == 5 ? 6 : E <= 7 ? 5 : E == 8 ? 4 : 3;
+}
 
 // ================================================= backward kernels by rows
 // fp32 rows of few channels (rows_by_lane): one lane holds a whole query, as in the
@@ -718,7 +732,7 @@ int launch_bwd_fwd_vec(const QDev& d, const void* z, void* ge, void* go, const S
     const int out = gradients_wanted(ge, go, also);
     const int threads = vec_threads(d, out);
     const size_t smem = rows_smem(d, ge != nullptr ? threads / 64 : 0);
-    const unsigned g = persistent_grid((d.N + threads - 1) / threads, smem, resident_rows(E));
+    const unsigned g = persistent_grid((d.N + threads - 1) / threads, smem, resident_rows(E, 1, out));
 #define ASH_BF(L, O, T)                                                       \
     query_backward_forward_vec_kernel<E, L, O, T><<<g, T, smem, s>>>(    \
             d, static_cast<const float*>(z), static_cast<float*>(ge),         \
@@ -757,7 +771,7 @@ int launch_bwd_bwd_vec(const QDev& d, const void* gg, const void* z, void* gz,
     const int out = (ge != nullptr ? 1 : 0) | (gz != nullptr ? 2 : 0);
     const int threads = vec_threads(d, out);
     const size_t smem = rows_smem(d, ge != nullptr ? threads / 64 : 0);
-    const unsigned g = persistent_grid((d.N + threads - 1) / threads, smem, resident_rows(E));
+    const unsigned g = persistent_grid((d.N + threads - 1) / threads, smem, resident_rows(E, 2, out));
 #define ASH_BB(L, O, T)                                                       \
     query_backward_backward_vec_kernel<E, L, O, T><<<g, T, smem, s>>>(   \
             d, static_cast<const float*>(gg), static_cast<const float*>(z),   \

@@ -72,3 +72,19 @@ def test_every_gradient_against_the_oracle(gpu_ash, oracle, width, n, cells):
         assert_close_sums(ge, both_ref, both, what="both orders", **dense)
         if need_offsets:
             assert torch.allclose(go.cpu(), go_ref, **per_query)
+
+
+@pytest.mark.parametrize("width", [1, 2, 3, 4, 5, 7, 8, 12, 16])
+@pytest.mark.parametrize("n", [5003, _NARROW - 1, _NARROW, _LDS])
+def test_a_query_gets_the_same_whatever_else_is_asked_for(gpu_ash, width, n):
+    """To the bit, whichever kernels the sizes and the gradients asked for choose."""
+    ops, (z, u, z2) = _operands(width, n, 64, seed=width)
+    dev = [t.to(DEV) for t in ops]
+    z, u, z2 = z.to(DEV), u.to(DEV), z2.to(DEV)
+    backend = gpu_ash.grid_query.backend
+    alone = backend.query_backward_forward(z, *dev, 2, "smooth_step", need_embeddings=False, need_offsets=True)[1]
+    for both in (backend.query_backward_forward(z, *dev, 2, "smooth_step")[1],
+                 backend.host.query_backward_both(z, u, z2, dev, "smooth_step", True, None)[1]):
+        assert torch.equal(alone, both)
+    alone = backend.query_backward_backward(None, u, z, *dev, 2, "smooth_step", need_embeddings=False)[0]
+    assert torch.equal(alone, backend.query_backward_backward(None, u, z, *dev, 2, "smooth_step")[0])

@@ -266,6 +266,10 @@ def backward_kernels_only_of_widths_that_are_launched(device):
     wide = {int(name.split("_vec_kernelILi")[1].split("E")[0]) for name in device.kernels()
             if "_vec_kernelI" in name and "Li512E" in name}
     assert wide == set(range(1, 9)), wide
+    # gradients of queries alone: all widths but that of one channel
+    alone = {int(name.split("_vec_kernelILi")[1].split("E")[0]) for name in device.kernels()
+             if re.search(r"_vec_kernelILi\d+ELb[01]ELi2E", name)}
+    assert alone == {2, 3, 4, 5, 6, 7, 8, 12, 16}, alone
 
 
 def programs_that_interpolate_do_not_load_the_backward_by_rows(device):

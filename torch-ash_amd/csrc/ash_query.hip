@@ -1580,20 +1580,30 @@ int launch_bwd_bwd(const QDev& d, const void* gg, const void* z, void* gz,
 
 // Whether a backward goes by the kernels that give a lane a whole query, in fp32 (`out`: bit
 // 0 scatters to the embeddings).  Widths of their own: 1 to 8 channels (four on 16-byte
-// aligned buffers) and 12; of 16 what scatters nothing (a pair of its rows is two lines
-// anyway, and sixteen floats of two kinds and eight rows are more than the registers
-// hold).  Before (a lane per channel) -> now, us:
-//   gradient of the positions, ray samples: 2 M of 1, 2, 3 channels 36 -> 34, 40 -> 36, 52
-//     -> 38; 1 M of 5, 7, 8 57 -> 32, 58 -> 34, 57 -> 34; 660 000 of 12 83 -> 32; 500 000
-//     of 16 61 -> 27; 1000 of 5 12.5 -> 4.3
-//   both orders of the scatter with it: 124 -> 81, 161 -> 97, 213 -> 128; 170 -> 93, 186 ->
-//     112, 147 -> 113; 183 -> 132
-//   the same in no order, 1 M: of 1 channel 399 -> 234, 3 442 -> 293, 4 398 -> 274, 5 494 ->
-//     354, 8 392 -> 339; 660 000 of 12 403 -> 323; 1000 of 5 11.9 -> 6.9
-// What a query gets is the same to the bit whatever else is asked for: a width's sizes go
-// either way with all their gradients, and sixteen channels are added up as a lane per
-// channel does it (row_product).  (The two kinds of these in a launch each: 500 000 in order 139 -> 137,
-// in none 218 -> 272.)
+// aligned buffers) and 12, as fields of a distance, colours, weights or four of either have
+// them; 9 to 11 and 13 to 15 channels are built for a lane per channel alone, as every width
+// of its own takes 0.4 MB of device code.  Of 16 what scatters nothing (a pair of its rows is
+// two lines anyway, and sixteen floats of two kinds and eight rows are more than the
+// registers hold), of 1 what scatters (a lane per channel is one per query there).  By a lane
+// per channel -> by rows, us, queries along rays | in no order:
+//   gradient of the positions alone: 300 000 of 2 channels 8.8 -> 7.8 | 22.0 -> 23.0, 1 M 26.7
+//     -> 24.0 | 69.1 -> 71.2; 1 M of 3 33.1 -> 25.1 | 83.5 -> 83.9, of 5 58.6 -> 30.9 | 108.7 ->
+//     106.6, of 7 58.7 -> 30.2 | 117.2 -> 116.1, of 8 59.1 -> 30.0 | 104.2 -> 102.1; 660 000 of
+//     12 84.1 -> 28.2 | 92.5 -> 86.1, of 16 84.6 -> 35.4 | 91.4 -> 84.4
+//   grad_z alone: 300 000 of 2 9.5 -> 7.9 | 20.7 -> 22.4, 1 M 26.3 -> 23.4 | 69.0 -> 70.5; 1 M of
+//     3 32.0 -> 25.2 | 84.0 -> 83.6, of 5 46.7 -> 29.0 | 106.9 -> 108.8, of 7 48.0 -> 32.2 | 116.5
+//     -> 121.9, of 8 48.3 -> 32.0 | 105.1 -> 107.5; 660 000 of 12 53.5 -> 30.3 | 89.1 -> 86.0, of
+//     16 54.6 -> 37.2 | 87.8 -> 85.8
+//   both orders of the scatter with the positions' gradient: 1 M of 1 72 -> 39 | 394 -> 231, of
+//     2 96 -> 51 | 383 -> 231, of 3 123 -> 63 | 436 -> 283, of 5 172 -> 85 | 479 -> 340, of 7 185
+//     -> 105 | 522 -> 390, of 8 145 -> 109 | 388 -> 330; 660 000 of 12 178 -> 127 | 399 -> 324;
+//     1000 of 5 18.4 -> 8.6
+// (Gathers in no order are bound by the lines of the rows either way; of two channels, and
+// grad_z of five to eight, they lose 2 - 8 % there, where a lane asks for a line each.)
+// What a query gets is the same to the bit whatever else is asked for, and so by either
+// kind: both add up a query's corners and channels in the same order (row_product).  (The
+// two kinds of sixteen channels in a launch each: 500 000 in order 139 -> 137, in none 218 ->
+// 272.)
 // Below 98 304 queries rows of one and two channels go by a lane per channel,
 // which is there all the same and has less to set up: 50 000 of one 7.2 | 9.5, 90 000 10.1 |
 // 11.5, 131 000 14.2 | 10.9; 70 000 of two 10.7 | 12.0, 131 000 15.9 | 12.1.
@@ -1601,7 +1611,7 @@ constexpr int64_t kNarrowScatter = int64_t{3} << 15;
 
 bool rows_by_lane(const QDev& d, int out, const void* p0, const void* p1, const void* p2) {
     if (d.E == 4) return aligned16(d.emb) && aligned16(p0) && aligned16(p1) && aligned16(p2);
-    if (d.E <= 2) return d.N >= kNarrowScatter;
+    if (d.E <= 2) return d.N >= kNarrowScatter && (d.E == 2 || (out & 1) != 0);
     return d.E <= 8 || d.E == 12 || (d.E == 16 && (out & 1) == 0);
 }
 

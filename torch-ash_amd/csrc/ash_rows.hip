@@ -709,10 +709,10 @@ query_backward_backward_vec_kernel(
 #pragma unroll
                     for (int k = 0; k < E; ++k) __builtin_nontemporal_store(on ? gz[k] : 0.f, grad_z + q * E + k);
                 } else {
-                    // (left to the caches, which join the pieces of a line: 660 000 queries of
-                    // twelve and sixteen channels in no order 107 -> 101 and 118 -> 100 us, by a
-                    // lane per channel 100 and 98, in order 53 -> 50 and 74 -> 55; of eight, with
-                    // two pieces, 120 -> 117, but in order 53.9 -> 56.6)
+                    // (left to the caches, which join the pieces of a line: behind a scatter,
+                    // 660 000 queries of twelve and sixteen channels in no order 107 -> 101 and
+                    // 118 -> 100 us, by a lane per channel 100 and 98, in order 53 -> 50 and 74 ->
+                    // 55; of eight, with two pieces, 120 -> 117, but in order 53.9 -> 56.6)
 #pragma unroll
                     for (int k = 0; k < E; ++k) grad_z[q * E + k] = on ? gz[k] : 0.f;
                 }
@@ -782,13 +782,13 @@ int launch_bwd_fwd_vec(const QDev& d, const void* z, void* ge, void* go, const S
         else if (out == 5) ASH_BF(true, 5, kBlock);
         else if (out == 3) ASH_BF(true, 3, kBlock);
         else if (out == 1) ASH_BF(true, 1, kBlock);
-        else ASH_BF(true, 2, kBlock);
+        else if constexpr (E > 1) ASH_BF(true, 2, kBlock);
     } else {
         if (out == 7) ASH_BF(false, 7, kBlock);
         else if (out == 5) ASH_BF(false, 5, kBlock);
         else if (out == 3) ASH_BF(false, 3, kBlock);
         else if (out == 1) ASH_BF(false, 1, kBlock);
-        else ASH_BF(false, 2, kBlock);
+        else if constexpr (E > 1) ASH_BF(false, 2, kBlock);
     }
 #undef ASH_BF
     ASH_LAUNCH_CHECK();
@@ -816,11 +816,11 @@ int launch_bwd_bwd_vec(const QDev& d, const void* gg, const void* z, void* gz,
     } else if (lut_in_lds(d)) {
         if (out == 3) ASH_BB(true, 3, kBlock);
         else if (out == 1) ASH_BB(true, 1, kBlock);
-        else ASH_BB(true, 2, kBlock);
+        else if constexpr (E > 1) ASH_BB(true, 2, kBlock);
     } else {
         if (out == 3) ASH_BB(false, 3, kBlock);
         else if (out == 1) ASH_BB(false, 1, kBlock);
-        else ASH_BB(false, 2, kBlock);
+        else if constexpr (E > 1) ASH_BB(false, 2, kBlock);
     }
 #undef ASH_BB
     ASH_LAUNCH_CHECK();

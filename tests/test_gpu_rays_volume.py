@@ -1,6 +1,10 @@
 """Rays that ask a map of the blocks in bounds, made by the call, against the
 look-ups in the table: the same results, also for blocks outside the bounds and
 after keys have come and gone."""
+import ctypes
+import os
+import re
+
 import pytest
 import torch
 
@@ -102,8 +106,8 @@ def test_rays_along_axes(gpu_ash, zeros, n):
 @pytest.mark.parametrize("n,where", [(8195, "one stream"), (8195, "two streams"), (8195, "captured"),
                                      (1024, "one stream"), (2048, "one stream")])
 def test_blocks_of_earlier_calls_are_not_met(gpu_ash, n, where):
-    """The volume that a map keeps, marked with another number by every call until it is
-    cleared: blocks come and go in between, through more calls than there are numbers."""
+    """The volumes that are kept, of two sizes, marked with another number by every call:
+    blocks come and go in between."""
     grid = gpu_ash.BoundedSparseDenseGrid(3, 3000, 1, 8, 32, device=DEV)
     backend, table = gpu_ash.grid.backend, grid.engine.backend
     g = torch.Generator().manual_seed(5)
@@ -164,3 +168,95 @@ def test_a_ray_beside_one_that_has_ended(gpu_ash):
                                           samples, 8.0)[0]) for r in range(4240, 4248)]
     counts = torch.bincount(backend.ray_sample_world(*args)[0], minlength=n)
     assert counts[4240:4248].tolist() == alone
+
+
+@pytest.mark.parametrize("streams", [1, 2])
+def test_numbers_come_again(gpu_ash, streams):
+    """More than twice as many calls on every stream as there are numbers to mark with, with
+    bounds of three sizes and origins that share a volume.  A call's blocks are stored for it
+    alone, so that each keeps its number until this is given again; one beyond the narrower
+    bounds comes and goes."""
+    with open(os.path.join(os.path.dirname(__file__), os.pardir, "include", "ash_hip.h")) as f:
+        marks = int(re.search(r"ASH_RAY_VOLUME_MARKS (\d+)", f.read())[1])
+    grid = gpu_ash.BoundedSparseDenseGrid(3, 3000, 1, 8, 32, device=DEV)
+    backend, table = gpu_ash.grid.backend, grid.engine.backend
+    n, samples, each = 2048, 64, 30
+    sizes = {backend.lib.ash_map_ray_volume_bytes(table._address, lo, hi, n, kind)
+             for lo, hi in ((0, 31), (1, 30), (0, 28)) for kind in (0, samples)}
+    assert len(sizes) == 1 and sizes.pop() > 0
+    g = torch.Generator().manual_seed(streams)
+    cube = torch.randperm(31 ** 3, generator=g)
+    blocks = torch.stack([cube // 961, cube // 31 % 31, cube % 31], 1).int().to(DEV)
+    beyond = torch.tensor([[31, 31, 31]], dtype=torch.int32, device=DEV)
+    o = (torch.rand(n, 3, generator=g) * 256).to(DEV)
+    d = torch.nn.functional.normalize(torch.randn(n, 3, generator=g), dim=1).to(DEV)
+    box = [torch.full((3,), x, device=DEV) for x in (0.0, 256.0)]
+    args = (table, o, d, None, 1.0, *box, 0.0, 800.0, 8.0)
+    on = [torch.cuda.Stream() for _ in range(streams)]
+    calls, met, turn = [0] * streams, 0, 0
+    while min(calls) < 2 * marks + 2:
+        k = turn % streams
+        here = blocks[turn * each % (len(blocks) - each):][:each]
+        if turn // streams % 3 == 0:
+            here = torch.cat([here, beyond])
+        grid.engine.insert_keys(here)
+        plain = backend.ray_find_near_far_world(*args)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(on[k]):
+            bounds = ((0, 31), (1, 30), (0, 28))[turn % 5 % 3]
+            got = backend.ray_find_near_far_world(*args, bounds)
+            calls[k] += 1
+            if turn % 7 == 0:
+                asked = (table, o, d, None, 1.0, *got, samples, 8.0)
+                for a, b in zip(backend.ray_sample_world(*asked, bounds), backend.ray_sample_world(*asked)):
+                    assert torch.equal(a, b), turn
+                calls[k] += 1
+        torch.cuda.synchronize()
+        for a, b in zip(plain, got):
+            assert torch.equal(a, b), turn
+        met += int((got[0] >= 0).any())
+        grid.engine.erase(here)
+        turn += 1
+    # (no block was stored twice while its number could come again)
+    assert met > turn // 2 and (marks + 2) * streams * each < len(blocks)
+
+
+@pytest.mark.parametrize("n", [4096, 8195])
+def test_scratch_that_holds_anything(gpu_ash, n):
+    """The functions that clear their scratch themselves."""
+    grid = gpu_ash.BoundedSparseDenseGrid(3, 3000, 1, 8, 32, device=DEV)
+    backend, table = gpu_ash.grid.backend, grid.engine.backend
+    lib, ptr = backend.lib, ctypes.c_void_p
+    g = torch.Generator().manual_seed(n)
+    grid.engine.insert_keys(torch.randint(0, 32, (2500, 3), generator=g).int().to(DEV))
+    o = (torch.rand(n, 3, generator=g) * 256).to(DEV)
+    d = torch.nn.functional.normalize(torch.randn(n, 3, generator=g), dim=1).to(DEV)
+    lo, hi = (torch.full((3,), x, device=DEV) for x in (0.0, 256.0))
+    near, far = backend.ray_find_near_far_world(table, o, d, None, 1.0, lo, hi, 0.0, 800.0, 8.0)
+    at = lambda t: ptr(t.data_ptr())
+    stream = ptr(torch.cuda.current_stream().cuda_stream)
+
+    def scratch(sampling):
+        size = lib.ash_ray_volume_bytes(0, 31, n, sampling)
+        return torch.randint(0, 256, (size,), generator=g).to(torch.uint8).to(DEV) if size else None
+
+    for _ in range(2):
+        bytes_, nears, fars = scratch(0), torch.empty(n, device=DEV), torch.empty(n, device=DEV)
+        assert bytes_ is not None
+        assert lib.ash_ray_find_near_far_world(table._address, at(bytes_), 0, 31, at(o), at(d), None, 1.0, at(lo),
+                                               at(hi), n, 0.0, 800.0, 8.0, at(nears), at(fars), stream) == 0
+        assert torch.equal(nears, near) and torch.equal(fars, far)
+        bytes_, stride = scratch(1), 64
+        assert (bytes_ is None) == (n < 8192)
+        counts = torch.empty(n, dtype=torch.int64, device=DEV)
+        groups = torch.empty(lib.ash_ray_sample_groups(n), 2, dtype=torch.int64, device=DEV)
+        stage, out = torch.empty(n, stride, 2, device=DEV), (ctypes.c_int64 * 2)()
+        assert lib.ash_ray_sample_march(table._address, at(bytes_) if bytes_ is not None else None, 0, 31, at(o), at(d),
+                                        None, 1.0, at(near), at(far), 0.0, 0.0, n, 32, 8.0, at(counts), at(groups),
+                                        at(stage), stride, out, stream) == 0
+        rays, starts, ends, prefix = backend.ray_sample_world(table, o, d, None, 1.0, near, far, 32, 8.0)
+        assert out[0] == len(rays) and out[1] <= stride
+        got = (torch.empty_like(rays), torch.empty_like(starts), torch.empty_like(ends), torch.empty_like(prefix))
+        assert lib.ash_ray_sample_place(at(counts), at(groups), at(stage), stride, n, 1.0, *map(at, got), stream) == 0
+        for a, b in zip(got, (rays, starts, ends, prefix)):
+            assert torch.equal(a, b)

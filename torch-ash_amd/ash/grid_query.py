@@ -196,16 +196,17 @@ def _learn_holders() -> None:
         pass
 
 
-# Queries from which second-order nodes leave their share to the forward node, by the
-# wall time of a training step of 20 000 blocks (own share -> put off, us; rows of other
-# than four channels by kernels of a lane per channel, which took twice as long).  Fewer wait
-# for the host, 350 - 490 us by its clock, and the kernel time saved (22 us for 131 000
-# of five channels) reaches nobody: 131 000 of 1, 4, 5, 16 channels 331 -> 335, 469 ->
-# 470, 504 -> 497, 472 -> 476; 262 000 352 -> 355, 485 -> 488, 488 -> 493, 474 -> 478.
-# From here on the kernels bound the steps with wide rows: 393 000 495 -> 491, 497 ->
-# 494, 429 -> 415, 477 -> 468; 524 000 of 5 and 16 channels 370 -> 354 and 568 -> 485;
-# 1 M of 5, 594 -> 450.  Narrow rows gain later, of one and four channels from 2 M on
-# (507 -> 493 and 555 -> 497), and lose nothing in between.
+# Queries from which second-order nodes leave their share to the forward node, by the wall
+# time of training steps of 20 000 blocks, one after the other | each waited for (own share
+# -> put off, us).  Fewer wait for the host, and the kernel time saved reaches nobody: 131 000
+# of 1, 4, 5, 16 channels 308 -> 308, 428 -> 436, 425 -> 430, 437 -> 440; 262 000 307 -> 310,
+# 428 -> 433, 419 -> 431, 439 -> 441 | 361 -> 363, 475 -> 483, 470 -> 478, 603 -> 570.  From
+# here on the kernels of wide rows show, first where steps are waited for: 393 000 of 5, 8, 12,
+# 16 channels 417 -> 425, 427 -> 429, 431 -> 435, 466 -> 436 | 462 -> 467, 490 -> 475, 562 ->
+# 541, 640 -> 572; 524 000 421 -> 428, 427 -> 430, 431 -> 434, 569 -> 476 | 477 -> 466, 504 ->
+# 482, 582 -> 561, 721 -> 635; 1 M of 1, 4, 5, 8, 12 310 -> 313, 434 -> 436, 430 -> 429, 465 ->
+# 439, 630 -> 578 | 379 -> 358, 514 -> 480, 536 -> 478, 584 -> 551, 715 -> 663; 2 M of 1, 4, 5
+# 432 -> 437, 544 -> 457, 628 -> 529.
 PUT_OFF_FROM = 3 << 17
 
 

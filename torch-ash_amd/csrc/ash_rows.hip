@@ -41,7 +41,7 @@ constexpr int resident_rows(int E, int order, int out) {
 // fp32 rows of few channels (rows_by_lane): one lane holds a whole query, as in the
 // forward kernel, so that a wavefront serves 64 queries per tile: four channels have four
 // times the loads in flight and a quarter of the per-query arithmetic of the
-// one-lane-per-channel kernels above, and rows of five leave no lanes idle.
+// one-lane-per-channel kernels of ash_query.hip, and rows of five leave no lanes idle.
 //
 // Gradient rows.  The memory side executes atomics at a fixed rate of
 // requests, and one request is what one instruction of a wavefront sends to

@@ -79,7 +79,7 @@ __device__ __forceinline__ uint32_t bucket_of(uint64_t code, uint32_t nb) {
 // are done each time, and four keys a bucket are what a filling map has (the kernel alone,
 // us: 100 000 keys with rows into an emptied map 23.3 -> 17.4, 200 000 33.4 -> 23.5, keys
 // alone 20.0 -> 15.7; beside 47 000 keys 190 000 43 -> 32, 300 000 51 -> 38.7; beside a
-// million 65 537 15.7 -> 15.4, 300 000 33.4 -> 30.9; 600 000 beside four million 62.7).
+// million 65 537 15.7 -> 15.4, 300 000 33.4 -> 30.9).
 __device__ __forceinline__ int first_slot(uint64_t code) {
     return static_cast<int>(__umulhi(static_cast<uint32_t>(mix64(code)), static_cast<uint32_t>(kSlots)));
 }
